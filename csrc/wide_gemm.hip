@@ -206,7 +206,9 @@ __device__ inline void wide_epilogue(frag_cd (&acc)[FA][FB], const Params& p, in
 //
 // Software pipeline (one barrier per stage, every wave's stage is the same mix of work):
 //   top of step i:  s_waitcnt vmcnt((NS - 2) G)   this wave's pieces of stage i+1 have landed
-//                   s_barrier                     ... and everybody's; all reads of stage i are done
+//                   s_waitcnt lgkmcnt(0)          its reads of stage i have been answered (without this a slow read, as beside
+//                                                 another kernel on the CU, could meet the DMA below)
+//                   s_barrier                     ... and everybody's
 //                   LDS-DMA of stage i+NS   -> buffer i % NS (free: stage i sits in registers)
 //                   fragment reads of stage i+1 -> register set (i+1) & 1   } interleaved
 //                   MFMAs on register set i & 1 (stage i)                   }
@@ -384,8 +386,8 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_kernel(const Params p)
 #define WG_STEP(CUR, NXT, I)                                                                                                 \
   do {                                                                                                                      \
     const int i_ = (I);                                                                                                     \
-    if constexpr ((NS - 2) * G == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                       \
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * G) : "memory");                                                \
+    if constexpr ((NS - 2) * G == 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");                            \
+    else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * G) : "memory");                                     \
     __builtin_amdgcn_s_barrier();                                                                                           \
     unsigned char* dst_ = smem + (i_ % NS) * STAGE;                                                                         \
     const unsigned char* src_ = smem + ((i_ + 1) % NS) * STAGE;                                                             \
@@ -577,8 +579,8 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_rs_kernel(const Params
 #define RS_STEP(CUR, NXT, I)                                                                                          \
   do {                                                                                                               \
     const int i_ = (I);                                                                                              \
-    if (w_role) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSW - 2) * GA) : "memory");                                \
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSX - 2) * GX) : "memory");                                       \
+    if (w_role) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NSW - 2) * GA) : "memory");                     \
+    else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NSX - 2) * GX) : "memory");                            \
     __builtin_amdgcn_s_barrier();                                                                                    \
     const unsigned char* sa_ = a_ring + ba * A_BYTES;                                                                \
     const unsigned char* sx_ = x_ring + bx * X_BYTES;                                                                \

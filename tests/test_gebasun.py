@@ -450,6 +450,23 @@ def test_replayed_graphs_equal_eager_steps(models, name):
 
 
 @pytest.mark.gpu
+def test_experts_on_a_second_stream_change_nothing():
+    """Experts beside the mixer share compute units with its kernels; every product must be the one computed alone, bit for bit."""
+    cfg = gebasun.stack("two-streams", 512, 2048, "SMSM", 16, 4, 128, 4096, 0, 64, 32, 64, 128, 1, 16, 4, 1408, 2816)
+    eng = LLMEngine(EngineConfig(model=cfg.name, device="cuda:0", max_num_seqs=2, max_batched_tokens=1536, max_model_len=1600, num_blocks=110, use_graphs=False, logit_rows=1536),
+                    weights=registry.random_weights(cfg, "cuda:0", torch.bfloat16, seed=3))
+    seq = eng.make_sequence(tokens(1536, 512, 1))  # (whole buckets: padding rows hold anything)
+    batch = eng.scheduler.schedule_given([(seq, 1536, list(range(1536)))])
+    aside = eng.runner.aside
+    assert aside is not None
+    eng.runner.aside = None
+    alone = eng.runner.execute(batch)[1].clone()
+    eng.runner.aside = aside
+    for _ in range(6):
+        assert torch.equal(eng.runner.execute(batch)[1], alone)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 def test_long_contexts(models, dtype):
     """More than 2000 tokens of context, beside a short request, in prompts and in decode steps (graphs) that share the windows' keys out."""
