@@ -1,4 +1,4 @@
-// Shared by the experts' kernels (csrc/experts.hip) and the tiled GEMM's grouped form (csrc/wide_gemm.hip).
+// Shared by the experts' kernels (csrc/experts.hip, csrc/panel_gemm.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -1,5 +1,5 @@
 // Mixture of experts for gfx950: routing, the grouping of (token, choice) pairs by expert, and the experts' products for few rows (the
-// products for many rows are the tiled GEMM's grouped form, csrc/wide_gemm.hip).
+// products for many rows: csrc/panel_gemm.hip).
 //
 // A pair p = token * top + choice; expert_of[p] is its expert (-1: the row is padding and chooses nobody), weight_of[p] its weight.  Matrices
 // of all experts are stacked; in bf16 in MFMA fragment order [N / 16][K / 32][64][8], an expert's first tile at expert * N / 16.  Gate and up
@@ -148,7 +148,8 @@ __global__ __launch_bounds__(1024) void route_kernel(const T* __restrict__ h, co
   a.weight_of[t * a.top + lane] = ok ? score(mine) * a.scale : 0.f;
 }
 
-// ---- grouping for many rows: pairs in the order of their experts, cut into tiles of at most `bm` pairs.  One workgroup.
+// ---- grouping for many rows: pairs in the order of their experts, an expert's in equal tiles of at most `bm` pairs (whole 32s: what the products
+// go by).  One workgroup.
 __global__ __launch_bounds__(1024) void group_pairs_kernel(const int* __restrict__ expert_of, int n_pairs, int E, int bm, GroupedRows g) {
   __shared__ int cnt[1024], off[1024], tiles[1024];
   const int e = threadIdx.x;
@@ -171,11 +172,12 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(const int* __restrict
     __syncthreads();
   }
   const int first = off[e] - mine, tile0 = tiles[e] - my_tiles;
+  const int per = my_tiles > 1 ? ((mine + my_tiles - 1) / my_tiles + 31) / 32 * 32 : mine;
   for (int i = 0; i < my_tiles; ++i) {
     if (tile0 + i >= g.max_tiles) break;
     g.tile_expert[tile0 + i] = e;
-    g.tile_first[tile0 + i] = first + i * bm;
-    g.tile_rows[tile0 + i] = mine - i * bm < bm ? mine - i * bm : bm;
+    g.tile_first[tile0 + i] = first + i * per;
+    g.tile_rows[tile0 + i] = mine - i * per < per ? mine - i * per : per;
   }
   if (e == 1023) g.n_tiles[0] = tiles[e] < g.max_tiles ? tiles[e] : g.max_tiles;
   cnt[e] = first;
@@ -367,7 +369,7 @@ int kve_route(const void* h, int f32, long long ldh, const void* w, const float*
 }
 
 int kve_group(const int* expert_of, int n_pairs, int E, int bm, int* order, int* tiles, int max_tiles, int* n_tiles, hipStream_t s) {
-  if (n_pairs <= 0 || E <= 0 || E > 1024 || bm <= 0 || max_tiles < n_pairs / bm + (E < n_pairs ? E : n_pairs)) return -1;
+  if (n_pairs <= 0 || E <= 0 || E > 1024 || bm <= 0 || (bm & 31) || max_tiles < n_pairs / bm + (E < n_pairs ? E : n_pairs)) return -1;
   const GroupedRows g{order, tiles, tiles + max_tiles, tiles + 2 * max_tiles, n_tiles, max_tiles, 1};
   hipLaunchKernelGGL(group_pairs_kernel, dim3(1), dim3(1024), 0, s, expert_of, n_pairs, E, bm, g);
   return (int)hipGetLastError();

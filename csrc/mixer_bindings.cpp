@@ -80,8 +80,8 @@ int kve_route(const void* h, int f32, long long ldh, const void* w, const float*
               hipStream_t s);
 int kve_group(const int* expert_of, int n_pairs, int E, int bm, int* order, int* tiles, int max_tiles, int* n_tiles, hipStream_t s);
 int kve_rows(const void* w, const void* x, void* y, int f32, int mode, const int* expert_of, int n_pairs, int top, int E, int N, int K, long long ldx, long long ldy, float limit, float slope, float shift, hipStream_t s);
-int kv_wide_gemm_grouped(const void* Wp, const void* x, void* out, int N, int K, long long ldx, long long ldy, int mode, float limit, float slope, float shift, int bm, int* order, int* tiles, int max_tiles, int* n_tiles,
-                         int row_div, hipStream_t stream);
+int kv_expert_panels(const void* Wp, const void* x, void* y, int N, int K, long long ldx, long long ldy, long long x_rows, int mode, float limit, float slope, float shift, int* order, int* tiles, int max_tiles, int* n_tiles,
+                     int row_div, hipStream_t stream);
 int kvm_norm_rope_write(const void* proj, int f32, void* q, void* k_cache, void* v_cache, long long ldp, int q_off, int k_off, int v_off, const float* bias, const float* q_norm,
                         const float* k_norm, const int* positions, const int* slots, const float* cos_t, const float* sin_t, int rot_dims, int T, int nh, int nkv, int dim, int vdim,
                         int dkp, int dvp, int block_size, float eps, hipStream_t s);
@@ -505,7 +505,8 @@ std::vector<Tensor> route(Tensor h, Tensor router, Tensor correction, Tensor slo
 
 // The chosen experts' outputs, one row per pair: [T * top, K of gate_up].  gate_up [E, 2 ffp, K] (gated) or [E, ffp, K] (squared relu), down [E, K, ffp].  tile: rows per tile of the
 // grouped products (64, 128 or 256), 0: the few-row kernels (bf16: at most 128 tokens).
-Tensor expert_outputs(Tensor h, Tensor idx, Tensor gate_up, Tensor down, bool gated, double limit, double slope, double shift, int64_t tile) {
+// grouped: the pairs are sorted by expert and multiplied in tiles (many rows, bf16); else workgroups look their expert's rows up themselves
+Tensor expert_outputs(Tensor h, Tensor idx, Tensor gate_up, Tensor down, bool gated, double limit, double slope, double shift, bool grouped) {
   const bool f = is_f32(h);
   const int64_t T = h.size(0), top = idx.size(1), P = T * top, E = gate_up.size(0), N = gate_up.size(1), K = gate_up.size(2), ffp = gated ? N / 2 : N;
   const int mode = gated ? 1 : 2;
@@ -515,21 +516,26 @@ Tensor expert_outputs(Tensor h, Tensor idx, Tensor gate_up, Tensor down, bool ga
   rows2d(h, h.scalar_type(), T, K, "experts: rows");
   const int* ip = i32p(idx, P, "choices");
   Tensor act = at::empty({P, ffp}, h.options()), y = at::empty({P, K}, h.options());
-  if (tile == 0) {
+  if (!grouped) {
     check(kve_rows(gate_up.data_ptr(), h.data_ptr(), act.data_ptr(), f, mode, ip, (int)P, (int)top, (int)E, (int)N, (int)K, h.stride(0), ffp, (float)limit, (float)slope, (float)shift, stream()), "expert gate / up");
     check(kve_rows(down.data_ptr(), act.data_ptr(), y.data_ptr(), f, 0, ip, (int)P, (int)top, (int)E, (int)K, (int)ffp, ffp, K, (float)limit, (float)slope, (float)shift, stream()), "expert down");
     return y;
   }
-  TORCH_CHECK(!f && (tile == 64 || tile == 128 || tile == 256), "experts: tiles of 64, 128 or 256 rows, bf16");
-  const int64_t max_tiles = P / tile + std::min(E, P);
-  Tensor ws = at::empty({P + 3 * max_tiles + 1}, idx.options());
-  int* order = (int*)ws.data_ptr();
-  int* tiles = order + P;
-  int* n_tiles = tiles + 3 * max_tiles;
-  check(kve_group(ip, (int)P, (int)E, (int)tile, order, tiles, (int)max_tiles, n_tiles, stream()), "expert grouping");
-  check(kv_wide_gemm_grouped(gate_up.data_ptr(), h.data_ptr(), act.data_ptr(), (int)N, (int)K, h.stride(0), ffp, mode, (float)limit, (float)slope, (float)shift, (int)tile, order, tiles, (int)max_tiles, n_tiles, (int)top, stream()),
-        "grouped gate / up");
-  check(kv_wide_gemm_grouped(down.data_ptr(), act.data_ptr(), y.data_ptr(), (int)K, (int)ffp, ffp, K, 0, (float)limit, (float)slope, (float)shift, (int)tile, order, tiles, (int)max_tiles, n_tiles, 1, stream()), "grouped down");
+  TORCH_CHECK(!f, "experts: grouped rows are bf16");
+  // (as many tokens at a time as 32-bit offsets reach)
+  const int64_t most = std::max<int64_t>(1, ((1ll << 31) - 1) / (2 * std::max(h.stride(0), top * ffp)) - 1);
+  for (int64_t t0 = 0; t0 < T; t0 += most) {
+    const int64_t n = std::min(most, T - t0), pairs = n * top, max_tiles = pairs / 256 + std::min(E, pairs);
+    Tensor ws = at::empty({pairs + 3 * max_tiles + 1}, idx.options());
+    int* order = (int*)ws.data_ptr();
+    int* tiles = order + pairs;
+    int* n_tiles = tiles + 3 * max_tiles;
+    auto rows = [&](const Tensor& x, int64_t row) { return (char*)x.data_ptr() + row * x.stride(0) * 2; };
+    check(kve_group(ip + t0 * top, (int)pairs, (int)E, 256, order, tiles, (int)max_tiles, n_tiles, stream()), "expert grouping");
+    check(kv_expert_panels(gate_up.data_ptr(), rows(h, t0), rows(act, t0 * top), (int)N, (int)K, h.stride(0), ffp, n, mode, (float)limit, (float)slope, (float)shift, order, tiles, (int)max_tiles, n_tiles, (int)top, stream()),
+          "grouped gate / up");
+    check(kv_expert_panels(down.data_ptr(), rows(act, t0 * top), rows(y, t0 * top), (int)K, (int)ffp, ffp, K, pairs, 0, (float)limit, (float)slope, (float)shift, order, tiles, (int)max_tiles, n_tiles, 1, stream()), "grouped down");
+  }
   return y;
 }
 

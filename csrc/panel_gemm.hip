@@ -1,0 +1,274 @@
+// Tiled products of a mixture of experts for many rows on gfx950: the (token, choice) pairs that chose an expert, up to 256 a tile, times the
+// expert's matrix, y[pair] = W[expert] x[row of the pair].
+//
+// What bounds it is the matrices: every expert's is read once (1.2 GB for 64 of 2304 x 4096), for some 100 to 300 rows, so bytes and matrix
+// work take about as long.  Hence:
+//  * A workgroup is a panel of 256 features x the tile's rows; each of its 8 waves owns 32 features and all rows.  Weights (fragment order
+//    [N/16][K/32][64][8]) go straight to registers, no byte twice, 3 stages of 64 columns ahead (96 KiB of them in flight per CU: through
+//    LDS there was room for 48), the rows to LDS by LDS-DMA, as far ahead, in a ring of 4 stages; all waves read all rows from there.
+//    They are read past the caches' reuse (nobody else wants them) and every workgroup starts at another column and goes round: panels lie a
+//    power of two apart, and in step they would all ask the same memory channels.  (293 -> 262 us; either alone 278 and 292.)
+//  * Work follows the rows that exist, in steps of 32: 2 x NF products per 64 columns and feature tile, NF = rows / 16 rounded up to an even
+//    number, one loop for each NF.  All waves have the same share, whatever the number.
+//  * LDS-DMA and loads are buffer instructions: the offset of a stage is scalar, and the compiler counts them exactly in front of a use (beside
+//    the FLAT form it waits for everything in flight).
+//  * Stores are 16 bytes a lane, gathered from the two feature tiles (and, gated, two row tiles) by lane swaps.
+// Measured, 64 experts of 2304 x 4096 with 187 rows each: 282 us; the tile of 256 x 256 through LDS (all 256 rows multiplied) 338 us.  64 rows: 246
+// against 311 us.
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+#include <type_traits>
+
+#include "experts.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 frag_ab;
+typedef __attribute__((ext_vector_type(4))) float frag_cd;
+typedef __attribute__((ext_vector_type(4))) unsigned int raw16;
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+
+enum Mode { PLAIN = 0, GATED = 1, SQUARED = 2 };
+
+constexpr int ROWS = 256, FEATURES = 256;  // of a tile
+constexpr int AHEAD = 3, RING = AHEAD + 1;  // stages of 64 columns
+constexpr int STAGE = ROWS * 128;           // bytes of a stage's rows
+
+struct PanelArgs {
+  const unsigned char* w; const __bf16* x; unsigned short* y;
+  int N, K; long long ldx, ldy;
+  int n_panels;
+  unsigned int x_bytes;
+  ExpertGate gate;
+  GroupedRows groups;
+};
+
+__device__ inline unsigned int f2bf(float f) {
+  unsigned int u = __float_as_uint(f);
+  if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40;
+  return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+__device__ inline uint2 pack4(frag_cd v) { return make_uint2(f2bf(v[0]) | f2bf(v[1]) << 16, f2bf(v[2]) | f2bf(v[3]) << 16); }
+
+__device__ inline rsrc_t buffer_of(const void* p, unsigned int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00027000); }
+constexpr int NON_TEMPORAL = 2;
+__device__ inline raw16 load16(rsrc_t r, int lane_off, int off) { return __builtin_bit_cast(raw16, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, NON_TEMPORAL)); }
+// one LDS-DMA piece: lane l's 16 bytes land at lds + 16 l
+__device__ inline void dma16(rsrc_t r, int lane_off, int off, void* lds) { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, lane_off, off, 0, 0); }
+
+// The 8-row piece of a stage that slot i of a wave copies; where there are fewer pieces than slots a piece is copied twice (the same bytes), so
+// that every wave has the same number in flight.
+__device__ inline int piece_of(int wave, int i, int pieces) {
+  const int p = wave + 8 * i;
+  return p < pieces ? p : i > 0 ? p - 8 : p % pieces;
+}
+
+// acc[i][j] += the wave's feature tile i x rows 16 j .. of NF row tiles (a multiple of two), over n stages of 64 columns
+template <int NF>
+__device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int start, int wave, int lane) {
+  constexpr int PX = (2 * NF + 7) / 8, OPS = 4 + PX;  // pieces of x and memory operations per wave and stage
+  constexpr int F = 2 * NF, NB = F / 4;               // row fragments of a stage (two k-steps), in batches of four
+  const int r = lane & 15, q = lane >> 4;
+  int xdst[PX];
+#pragma unroll
+  for (int i = 0; i < PX; ++i) xdst[i] = piece_of(wave, i, 2 * NF) * 1024;
+  // rows of 128 bytes whose 16-byte chunks are swizzled by (row >> 1) & 7: a fragment read touches 16 distinct chunks per 16 lanes
+  const int xo[2] = {r * 128 + ((q ^ (r >> 1)) << 4), r * 128 + (((4 + q) ^ (r >> 1)) << 4)};
+  raw16 w[AHEAD][2][2];
+  frag_ab b[2][4];
+  auto read = [&](int set, const unsigned char* img, int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int f = 4 * t + e;
+      b[set][e] = *reinterpret_cast<const frag_ab*>(img + xo[f / NF] + f % NF * 2048);
+    }
+  };
+  auto column = [&](int s) __attribute__((always_inline)) {  // of stage s (behind the end the last one is fetched again)
+    const int c = (s < n ? s : n - 1) + start;
+    return c < n ? c : c - n;
+  };
+  // memory operations behind batch t: pieces of x spread over the stage, weights where those they replace have been multiplied
+  auto fetch = [&](int t, int u, int st, unsigned char* dst) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < PX; ++i)
+      if (t == i * NB / PX) dma16(xr, xsrc[i], st * 128, dst + xdst[i]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (t == (k == 0 ? (NF - 1) / 4 : NB - 1)) {
+        w[u][k][0] = load16(wr, w0, st * 2048 + k * 1024);
+        w[u][k][1] = load16(wr, w1, st * 2048 + k * 1024);
+      }
+  };
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s)
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      fetch(t, s, column(s), ring + s * STAGE);
+      __builtin_amdgcn_sched_barrier(0);  // (in the order of the loop: what is in flight at its top is the same on both ways in)
+    }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * OPS) : "memory");
+  __builtin_amdgcn_s_barrier();
+  read(0, ring, 0);
+  int slot = 0;
+  // The barrier at the top of stage s: everybody's pieces of stage s + 1 have landed, and everybody has multiplied stage s - 1, whose place
+  // stage s + AHEAD takes.  (Reads still in flight there are of stage s.)
+  auto stage = [&](auto uc, int s) __attribute__((always_inline)) {
+    constexpr int u = decltype(uc)::value;
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 2) * OPS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    const int next = slot + 1 == RING ? 0 : slot + 1;
+    const unsigned char* cur = ring + slot * STAGE;
+    const unsigned char* nxt = ring + next * STAGE;
+    unsigned char* dst = ring + (slot == 0 ? RING - 1 : slot - 1) * STAGE;
+    const int sa = column(s + AHEAD);
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      const int set = (u * NB + t) & 1;
+      read(set ^ 1, t + 1 < NB ? cur : nxt, t + 1 < NB ? t + 1 : 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int f = 4 * t + e, k = f / NF, j = f % NF;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][k][i]), b[set][e], acc[i][j], 0, 0, 0);
+      }
+      fetch(t, u, sa, dst);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    slot = next;
+  };
+  static_assert(AHEAD == 3, "the unrolled loop and its tail");
+  int s = 0;
+  for (; s + 3 <= n; s += 3) {
+    stage(std::integral_constant<int, 0>{}, s);
+    stage(std::integral_constant<int, 1>{}, s + 1);
+    stage(std::integral_constant<int, 2>{}, s + 2);
+    if constexpr (NB & 1) {  // (an odd number of batches: the sets have swapped)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { const frag_ab v = b[0][e]; b[0][e] = b[1][e]; b[1][e] = v; }
+    }
+  }
+  if (s < n) stage(std::integral_constant<int, 0>{}, s);
+  if (s + 1 < n) stage(std::integral_constant<int, 1>{}, s + 1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
+}
+
+template <int MODE>
+__global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  // blockIdx -> (tile, panel): of those that exist, each XCD has a contiguous range, panels fastest (a tile's panels share its rows through that L2)
+  const int nwg = p.groups.n_tiles[0] * p.n_panels;
+  int id = blockIdx.x;
+  {
+    const int xcd = id & 7, qd = nwg >> 3, rm = nwg & 7;
+    if ((id >> 3) >= qd + (xcd < rm ? 1 : 0)) return;
+    id = (xcd < rm ? xcd * (qd + 1) : rm * (qd + 1) + (xcd - rm) * qd) + (id >> 3);
+  }
+  const int tile = id / p.n_panels, panel = id % p.n_panels;
+  const int* row_of = p.groups.order + p.groups.tile_first[tile];
+  const int rows = p.groups.tile_rows[tile];
+  const int nf = (rows + 31) / 32 * 2, nks = p.K / 32;
+  // the expert's panel; past the last feature reads give zeros
+  const int tiles = p.N / 16 - panel * (FEATURES / 16) < FEATURES / 16 ? p.N / 16 - panel * (FEATURES / 16) : FEATURES / 16;
+  const rsrc_t wr = buffer_of(p.w + ((long long)p.groups.tile_expert[tile] * (p.N / 16) + panel * (FEATURES / 16)) * nks * 1024, (unsigned int)tiles * nks * 1024);
+  const int w0 = 2 * wave * nks * 1024 + lane * 16, w1 = w0 + nks * 1024;
+  const rsrc_t xr = buffer_of(p.x, p.x_bytes);
+  int xsrc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 8 * piece_of(wave, i, 2 * nf) + (lane >> 3);
+    const int pair = row_of[row < rows ? row : rows - 1];  // (rows past the end read the last one; nobody stores what becomes of them)
+    xsrc[i] = (int)((unsigned int)(pair / p.groups.row_div) * (unsigned int)(p.ldx * 2)) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+  }
+  frag_cd acc[2][16];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
+  const int n = p.K / 64, start = id * 5 % n;
+  switch (nf) {
+    case 16: multiply<16>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 14: multiply<14>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 12: multiply<12>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 10: multiply<10>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 8: multiply<8>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 6: multiply<6>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 4: multiply<4>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    default: multiply<2>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+  }
+  // acc[i][j][e]: feature 16 i + 4 q + e of the wave's 32, row 16 j + r
+  const int f0 = panel * FEATURES + wave * 32;
+  if (f0 >= p.N) return;
+#pragma unroll
+  for (int j = 0; j < 16; j += 2) {
+    if (16 * j >= rows) break;
+    uint2 v[2][2];  // [row tile][half]: halves are feature tiles, or (gated) one half of the lanes has one and the other the other
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      frag_cd a = acc[0][j + t], b = acc[1][j + t];
+      if constexpr (MODE == GATED) {  // a tile is 8 gate rows and their 8 up rows: the upper half of the lanes takes the other tile's
+        frag_cd o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const auto gu = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[e]), __float_as_uint(b[e]), false, false);
+          o[e] = expert_gate(__uint_as_float(gu[0]), __uint_as_float(gu[1]), p.gate);
+        }
+        v[0][t] = pack4(o);
+      } else {
+        if constexpr (MODE == SQUARED) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { a[e] = fmaxf(a[e], 0.f); b[e] = fmaxf(b[e], 0.f); a[e] *= a[e]; b[e] *= b[e]; }
+        }
+        v[t][0] = pack4(a);
+        v[t][1] = pack4(b);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < (MODE == GATED ? 1 : 2); ++t) {
+      // sixteen lanes each: 0 the first half's (4 + 4 features), 1 the second's, 2 and 3 those eight features further
+      const auto lo = __builtin_amdgcn_permlane16_swap(v[t][0].x, v[t][1].x, false, false), hi = __builtin_amdgcn_permlane16_swap(v[t][0].y, v[t][1].y, false, false);
+      const raw16 o = {lo[0], hi[0], lo[1], hi[1]};
+      const int row = 16 * (j + (MODE == GATED ? q & 1 : t)) + r;
+      const int f = MODE == GATED ? f0 / 2 + 8 * (q >> 1) : f0 + 16 * (q & 1) + 8 * (q >> 1);
+      if (row < rows) *reinterpret_cast<raw16*>(p.y + (long long)row_of[row] * p.ldy + f) = o;
+    }
+  }
+}
+
+template <int MODE>
+int launch(const PanelArgs& a, hipStream_t s) {
+  constexpr int LDS = RING * STAGE;
+  const auto kern = expert_panel_kernel<MODE>;
+  static const hipError_t lds_ok = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (lds_ok != hipSuccess) return -2;
+  hipLaunchKernelGGL(kern, dim3(a.groups.max_tiles * a.n_panels), dim3(512), LDS, s, a);
+  return (int)hipGetLastError();
+}
+
+}  // namespace
+
+extern "C" {
+
+// Wp holds the packed matrices [N, K] of all experts, one behind the other; row i of the tiled rows (kve_group, at most 256 a tile) is pair order[i],
+// x's row is pair / row_div, y's row the pair.  mode 1: bf16 y[pairs, N / 2] with the experts' gate; 2: bf16 max(y, 0)^2 [pairs, N]; 0: bf16 y[pairs, N].
+// N % 32 == 0, K % 64 == 0, rows of x and y of whole 16-byte pieces; x_rows rows of x must lie within 2 GiB (offsets are 32-bit).
+int kv_expert_panels(const void* Wp, const void* x, void* y, int N, int K, long long ldx, long long ldy, long long x_rows, int mode, float limit, float slope, float shift, int* order, int* tiles, int max_tiles, int* n_tiles,
+                     int row_div, hipStream_t stream) {
+  if (N <= 0 || K <= 0 || (N & 31) || (K & 63) || K > (1 << 21) || (ldx & 7) || (ldy & 7) || max_tiles <= 0 || row_div <= 0 || x_rows <= 0 || mode < PLAIN || mode > SQUARED) return -1;
+  const long long bytes = ((x_rows - 1) * ldx + K) * 2;
+  if (bytes >= (1ll << 31) || ldx < K) return -1;
+  PanelArgs a;
+  a.w = (const unsigned char*)Wp; a.x = (const __bf16*)x; a.y = (unsigned short*)y;
+  a.N = N; a.K = K; a.ldx = ldx; a.ldy = ldy;
+  a.n_panels = (N + FEATURES - 1) / FEATURES;
+  a.x_bytes = (unsigned int)bytes;
+  a.gate = ExpertGate{limit, slope, shift};
+  a.groups = GroupedRows{order, tiles, tiles + max_tiles, tiles + 2 * max_tiles, n_tiles, max_tiles, row_div};
+  return mode == GATED ? launch<GATED>(a, stream) : mode == SQUARED ? launch<SQUARED>(a, stream) : launch<PLAIN>(a, stream);
+}
+
+}  // extern "C"

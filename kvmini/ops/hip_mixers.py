@@ -1,5 +1,5 @@
 """Sequence mixers and experts on the hand-written gfx950 kernels (``csrc/mixer_kernels.hip``, ``chunk_attention.hip``,
-``delta_rule.hip``, ``latent_attention.hip``, ``retention.hip``, ``state_space.hip``, ``experts.hip``, the grouped form of ``wide_gemm.hip``); call surface of :mod:`kvmini.ops.torch_mixers`."""
+``delta_rule.hip``, ``latent_attention.hip``, ``retention.hip``, ``state_space.hip``, ``experts.hip``, ``panel_gemm.hip``); call surface of :mod:`kvmini.ops.torch_mixers`."""
 
 from __future__ import annotations
 
@@ -268,14 +268,6 @@ def latent_plan(rows: int, heads: int, dvp: int, window: int, long: bool) -> Tup
 EXPERT_FEW_ROWS = 128  # up to as many tokens, workgroups look up their experts' rows themselves; beyond, rows are grouped into tiles
 
 
-def expert_tile(tokens: int, top: int, experts: int) -> int:
-    """Rows per tile of the grouped products: what an expert's rows (somewhat more than the mean) fill best.  A tile loads its operands
-    once for all its rows, so per row the small ones cost more."""
-    mean = tokens * top / experts
-    rows = mean + 2.0 * mean ** 0.5
-    return min((256, 128, 64), key=lambda t: -(-rows // t) * t * (1.0 + 76.0 / t))
-
-
 def shared_expert(m: MoeSpec, w: MoeWeights, h: torch.Tensor) -> Any:
     from .hip_ops import linear, linear_relu2, linear_swiglu
 
@@ -292,8 +284,7 @@ def experts(m: MoeSpec, w: MoeWeights, h: torch.Tensor, st: Step, shared: bool =
     gate_row = m.shared_ff > 0 and m.shared_gate
     idx, wt, gate = C.route(h, w.router, w.correction, st.slots, m.top, ("sigmoid", "softmax", "chosen").index(m.scores), m.scale, gate_row, w.bias)
     t = h.shape[0]
-    tile = 0 if h.dtype != torch.bfloat16 or t <= EXPERT_FEW_ROWS else expert_tile(t, m.top, m.experts)
-    rows = C.expert_outputs(h, idx, w.gate_up, w.down, m.gated, *m.glu, tile)
+    rows = C.expert_outputs(h, idx, w.gate_up, w.down, m.gated, *m.glu, h.dtype == torch.bfloat16 and t > EXPERT_FEW_ROWS)
     out = ExpertRows(rows, wt, None, gate if gate_row else None)
     return with_shared(out, m, w, h) if shared else out
 

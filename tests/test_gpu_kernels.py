@@ -2546,3 +2546,35 @@ def test_mxfp4_weights_times_fp8_activations_matches_fp32_matmul_of_the_quantise
     err = (y.float() - ref).abs().max().item()
     tol = 1.2e-2 * ref.abs().max().item() + 1e-2
     assert y.shape == ref.shape and err <= tol, (err, tol)
+
+
+@pytest.mark.parametrize("ff,width,gated", [(64, 64, True), (128, 128, False), (192, 320, True), (384, 256, False), (1408, 512, True)])
+def test_expert_panels_at_every_number_of_rows(C, ff, width, gated):
+    """Experts chosen by 0, 1, 2, ... rows: every number of row tiles, several tiles of one expert, panels cut short, few and many stages of columns."""
+    from kvmini.ops.hip_mixers import layout
+
+    counts = [0, 1, 15, 16, 17, 32, 33, 64, 65, 97, 129, 160, 161, 192, 193, 224, 225, 255, 256, 257, 300, 513]
+    torch.manual_seed(width + ff)
+    expert = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
+    t = expert.numel()
+    expert = expert[torch.randperm(t)].to(_dev())
+    expert[7] = -1  # a padding row
+    lay = layout(torch.bfloat16)
+    n = 2 * ff if gated else ff
+    up = (torch.randn(len(counts), n, width, device=_dev()) / width ** 0.5).bfloat16()
+    down = (torch.randn(len(counts), width, ff, device=_dev()) / ff ** 0.5).bfloat16()
+    x = torch.randn(t, width + 64, device=_dev()).bfloat16()[:, :width]  # (rows further apart than they are long)
+    y = C.expert_outputs(x, expert.int().view(-1, 1), lay.experts(up), lay.experts(down), gated, math.inf, 1.0, 0.0, True).float()
+    for e in range(len(counts)):
+        at = (expert == e).nonzero().view(-1)
+        if not len(at):
+            continue
+        h = x[at].float() @ up[e].float().T
+        if gated:  # rows in eights: gate, up, gate, ...
+            g, u = h.view(len(at), -1, 2, 8).unbind(2)
+            h = (torch.nn.functional.silu(g) * u).reshape(len(at), ff)
+        else:
+            h = torch.relu(h) ** 2
+        want = h.bfloat16().float() @ down[e].float().T
+        # bf16 rounding of the hidden row (2^-9 relative each, ff independent terms) and of the result
+        assert ((y[at] - want).norm(dim=1) / want.norm(dim=1)).max().item() < 1e-2, (e, counts[e])
