@@ -13,11 +13,12 @@
 //                        sub-histograms live in LDS (4 waves x 2048 bins x 4 B = 32 KiB of
 //                        the CU's 160 KiB) and are updated with LDS atomics; one global
 //                        atomic per non-empty bin per workgroup flushes them.
-//   kv_radix_hist/scan  exact order statistics by MSD radix select on order-preserving
+//   kv_select_quantiles  exact order statistics by MSD radix select on order-preserving
 //                        integer keys: 11-bit digits, i.e. the same 2048-bin LDS histogram,
 //                        restricted to samples whose higher digits match the prefix of a
-//                        target rank; a single-workgroup scan kernel turns the bin counts
-//                        into the next prefix.  Up to 8 ranks are tracked at once (floor and
+//                        target rank; the last workgroup of a pass turns the bin counts
+//                        into the next prefix (kv_radix_pass_*: a launch of its own, for samples
+//                        spread over ranks).  Up to 8 ranks are tracked at once (floor and
 //                        ceil rank of p50/p95/p99), so three quantiles of 10^8 doubles cost 6
 //                        streaming passes and no sort.  The result is bit-exact: the CPU
 //                        interpolates between the two selected samples exactly like
@@ -200,170 +201,329 @@ struct RadixState {
   int slot[KV_MAX_RANKS];                   // rank -> index into uniq
   int n_uniq;
   int n_ranks;
+  unsigned long long count;                 // samples
 };
 
-template <typename T>
-__global__ __launch_bounds__(KV_THREADS) void radix_hist_kernel(const T* __restrict__ x, long long n, long long row_stride,
-                                                                const RadixState* __restrict__ st, unsigned int* __restrict__ hist,
-                                                                int shift, int digit_bits, int first_pass) {
-  // first pass: one prefix (empty) -> per-wave private sub-histograms; later passes: one
-  // workgroup-shared histogram per distinct prefix.
-  __shared__ unsigned int lds[KV_MAX_RANKS * KV_BINS];  // 64 KiB
+// Ranks from quantile levels: pos = p*(n-1), ranks floor(pos) and ceil(pos) — the definition of analyze.py:75-81.
+struct Levels { double p[KV_MAX_RANKS / 2]; int n; };
+__device__ inline unsigned long long rank_of(const Levels& lv, int r, unsigned long long n) {
+  double p = lv.p[r >> 1];
+  p = p < 0.0 ? 0.0 : (p > 1.0 ? 1.0 : p);
+  const double pos = p * (double)(n - 1);
+  return (unsigned long long)((r & 1) ? ceil(pos) : floor(pos));
+}
+
+// A pass counts the 11-bit digits behind each distinct prefix.  Latencies are clustered (a first digit is a quarter of an octave, and most
+// of a wave's 64 samples share it), so what bounds a pass is LDS atomics that meet on one address: a workgroup of 16 waves keeps the histogram
+// 16 times (fewer times when there are more prefixes), bin by bin next to each other, and a lane uses copy lane % 16 — at most 4 lanes
+// of an instruction meet, in different banks.  One global atomic per non-empty bin and workgroup adds it up, so there are few workgroups,
+// one a CU.  3 x 4 M floats: 27 us a pass, picking included, where one histogram a wave with ballot aggregation took 48 and picking 14 more.
+constexpr int SEL_THREADS = 1024;
+constexpr int SEL_WORDS = 16 * KV_BINS;  // LDS words of the copies: 128 KiB
+constexpr int PER = KV_MAX_RANKS * KV_BINS / SEL_THREADS;  // bins per thread, of all prefixes
+constexpr int SEL_ROW = KV_BINS + KV_BINS / 32;  // LDS words of a summed histogram, 33 per 32 bins (a lane's 32 bins then start in a bank of their own)
+
+// (clearing and summing the copies takes a few us: a few thousand samples meet seldom enough in fewer)
+__device__ inline int log2_copies(int prefixes, long long n) {
+  const int room = prefixes <= 1 ? 4 : prefixes == 2 ? 3 : prefixes <= 4 ? 2 : 1, wanted = n <= 2048 ? 0 : n <= 8192 ? 2 : 4;
+  return room < wanted ? room : wanted;
+}
+
+// counts the digits of the samples first, first + stride, ... (in 16-byte pieces) of a row into h[prefix][bin][copy]; MOST: at least U prefixes
+// (0: the first pass, which has none)
+template <typename T, int MOST>
+__device__ void count_digits(const T* __restrict__ row, long long n, long long first, long long stride, unsigned int* h, const unsigned long long* uniq, int U, int shift, int digit_bits) {
   using KT = typename KeyOf<T>::type;
-  const int tid = threadIdx.x, wave = tid >> 6;
-  const int m = blockIdx.y;
-  const RadixState* s = st + m;
-  const int U = first_pass ? 1 : s->n_uniq;
-  const int nclear = first_pass ? KV_WAVES * KV_BINS : U * KV_BINS;
-  for (int i = tid; i < nclear; i += KV_THREADS) lds[i] = 0;
-  KT pre[KV_MAX_RANKS];
-#pragma unroll
-  for (int u = 0; u < KV_MAX_RANKS; ++u) pre[u] = (KT)(u < U && !first_pass ? (s->uniq[u] >> (64 - KeyOf<T>::bits)) : 0);
-  __syncthreads();
-
-  const T* row = x + (long long)m * row_stride;
-  const KT dmask = (KT)((1u << digit_bits) - 1u);
-  // bits above the current digit
-  const int hi_shift = shift + digit_bits;
   constexpr int VEC = 16 / sizeof(T);
-  struct alignas(16) Pack { T v[VEC]; };
-  const long long nvec = n / VEC;
-  const long long stride = (long long)gridDim.x * KV_THREADS;
-  const bool aligned = (((uintptr_t)row) & 15) == 0;
-
+  const int cl = log2_copies(U, n), copy = threadIdx.x & ((1 << cl) - 1);
+  const KT dmask = (KT)((1u << digit_bits) - 1u);
+  const int hi_shift = shift + digit_bits;  // bits above the current digit
+  KT pre[MOST > 0 ? MOST : 1] = {};
+#pragma unroll
+  for (int u = 0; u < MOST; ++u) pre[u] = (KT)((KT)(uniq[u < U ? u : 0] >> (64 - KeyOf<T>::bits)) >> hi_shift);  // (unused ones repeat the first)
   auto visit = [&](T v) {
-    if (v == v) {
-      KT key = KeyOf<T>::key(v);
-      unsigned int d = (unsigned int)((key >> shift) & dmask);
-      if (first_pass) {
-        hist_add(lds + wave * KV_BINS, d);
-      } else {
-        KT hi = hi_shift >= KeyOf<T>::bits ? (KT)0 : (KT)(key >> hi_shift);
+    if (!(v == v)) return;
+    const KT key = KeyOf<T>::key(v);
+    int bin = (int)((key >> shift) & dmask);
+    if constexpr (MOST > 0) {
+      const KT hi = (KT)(key >> hi_shift);
+      int at = -1;
 #pragma unroll
-        for (int u = 0; u < KV_MAX_RANKS; ++u)
-          if (u < U && hi == (hi_shift >= KeyOf<T>::bits ? (KT)0 : (KT)(pre[u] >> hi_shift))) hist_add(lds + u * KV_BINS, d);
-      }
+      for (int u = MOST - 1; u >= 0; --u) at = hi == pre[u] ? u : at;
+      if (at < 0) return;
+      bin += at * KV_BINS;
     }
+    atomicAdd(&h[(bin << cl) + copy], 1u);
   };
-  if (aligned) {
-    const Pack* pv = reinterpret_cast<const Pack*>(row);
-    long long i = (long long)blockIdx.x * KV_THREADS + tid;
-    for (; i + 3 * stride < nvec; i += 4 * stride) {  // four loads in flight per lane
-      const Pack p0 = pv[i], p1 = pv[i + stride], p2 = pv[i + 2 * stride], p3 = pv[i + 3 * stride];
+  struct alignas(16) Pack { T v[VEC]; };
+  // (rows need not start at a multiple of 16 bytes: the samples in front of the first whole piece and behind the last go one by one)
+  long long head = (VEC - (long long)((uintptr_t)row / sizeof(T)) % VEC) % VEC;
+  head = head < n ? head : n;
+  const Pack* pv = reinterpret_cast<const Pack*>(row + head);
+  const long long nvec = (n - head) / VEC, tail = head + nvec * VEC;
+  auto visit_pack = [&](const Pack& p) {
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) visit(p0.v[j]);
+    for (int j = 0; j < VEC; ++j) visit(p.v[j]);
+  };
+  constexpr int AHEAD = 4;  // loads in flight per lane while the ones before are counted
+  Pack p[AHEAD];
+  long long i = first;
+  if (i + (AHEAD - 1) * stride < nvec) {
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) visit(p1.v[j]);
+    for (int k = 0; k < AHEAD; ++k) p[k] = pv[i + k * stride];
+    for (;;) {
+      i += AHEAD * stride;
+      const bool more = i + (AHEAD - 1) * stride < nvec;
+      Pack q[AHEAD];
+      if (more) {
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) visit(p2.v[j]);
+        for (int k = 0; k < AHEAD; ++k) q[k] = pv[i + k * stride];
+      }
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) visit(p3.v[j]);
-    }
-    for (; i < nvec; i += stride) {
-      Pack p = pv[i];
+      for (int k = 0; k < AHEAD; ++k) visit_pack(p[k]);
+      if (!more) break;
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) visit(p.v[j]);
+      for (int k = 0; k < AHEAD; ++k) p[k] = q[k];
     }
   }
-  for (long long i = (aligned ? nvec * VEC : 0) + (long long)blockIdx.x * KV_THREADS + tid; i < n; i += stride) visit(row[i]);
-  __syncthreads();
+  for (; i < nvec; i += stride) visit_pack(pv[i]);
+  if (first < head) visit(row[first]);
+  if (tail + first < n) visit(row[tail + first]);
+}
 
+// the copies of bin i (counted over all prefixes)
+__device__ inline unsigned int sum_copies(const unsigned int* h, int i, int cl) {
+  if (cl < 2) return cl == 0 ? h[i] : h[2 * i] + h[2 * i + 1];
+  unsigned int c = 0;
+  for (int k = 0; k < 1 << cl; k += 4) {
+    const uint4 v = *reinterpret_cast<const uint4*>(h + (i << cl) + k);
+    c += v.x + v.y + v.z + v.w;
+  }
+  return c;
+}
+
+// The whole workgroup: every rank picks the bin that holds it, appends the digit to its prefix and keeps its rank inside; then the distinct
+// prefixes.  A wave per rank.  sums: LDS, [prefix][SEL_ROW].  `levels` (first pass): the ranks follow from the number of samples counted.
+__device__ void pick_digits(RadixState* s, const unsigned int* sums, int shift, bool first_pass, const Levels* levels) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int R = levels ? 2 * levels->n : s->n_ranks;
+  if (wave < R) {
+    const unsigned int* p = sums + (first_pass ? 0 : s->slot[wave]) * SEL_ROW + lane * 33;
+    unsigned int t[32];
+    unsigned long long local = 0;
+#pragma unroll
+    for (int j = 0; j < 32; ++j) t[j] = p[j];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) local += t[j];
+    unsigned long long upto = local;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const unsigned long long v = __shfl_up(upto, o, 64);
+      if (lane >= o) upto += v;
+    }
+    const unsigned long long total = __shfl(upto, 63, 64);
+    const unsigned long long k = levels ? (total ? rank_of(*levels, wave, total) : 0) : s->k[wave];
+    unsigned long long run = upto - local;
+    if (k >= run && k < upto) {
+      int bin = 0;
+      unsigned long long below = 0;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) {
+        if (k >= run && k < run + t[j]) { bin = lane * 32 + j; below = run; }
+        run += t[j];
+      }
+      s->prefix[wave] |= (unsigned long long)bin << shift;
+      s->k[wave] = k - below;
+    }
+    if (levels && wave == 0 && lane == 0) s->count = total;
+  }
+  __syncthreads();
+  if (wave == 0) {  // a lane per rank: the first rank with the same prefix, and how many such firsts there are in front of it
+    const unsigned long long mine = s->prefix[lane < KV_MAX_RANKS ? lane : 0];
+    int first = lane;
+#pragma unroll
+    for (int r = KV_MAX_RANKS - 1; r >= 0; --r) {
+      const unsigned long long other = __shfl(mine, r, 64);
+      if (r < R && other == mine) first = r;
+    }
+    const unsigned long long firsts = __ballot(lane < R && first == lane);
+    if (lane < R) {
+      const int at = __popcll(firsts & ((1ull << first) - 1));
+      s->slot[lane] = at;
+      if (first == lane) s->uniq[at] = mine;
+    }
+    if (lane == 0) {
+      s->n_uniq = __popcll(firsts);
+      s->n_ranks = R;
+    }
+  }
+  __syncthreads();
+}
+
+// What a selection leaves per metric: the keys of the ranks (left-aligned in 64 bits) and the number of samples.
+constexpr int SEL_OUT = KV_MAX_RANKS + 1;
+
+__device__ inline void copy_state(RadixState* to, const RadixState* from) {
+  static_assert(sizeof(RadixState) % 4 == 0 && sizeof(RadixState) / 4 <= SEL_THREADS, "a word per thread");
+  if (threadIdx.x < sizeof(RadixState) / 4) reinterpret_cast<unsigned int*>(to)[threadIdx.x] = reinterpret_cast<const unsigned int*>(from)[threadIdx.x];
+}
+__device__ inline void clear_state(RadixState* s) {
+  if (threadIdx.x < sizeof(RadixState) / 4) reinterpret_cast<unsigned int*>(s)[threadIdx.x] = 0;
+}
+
+// a pass's workgroup: its samples' digits in h, counted
+template <typename T>
+__device__ void count_pass(const T* row, long long n, int part, int parts, unsigned int* h, const RadixState* s, int U, int shift, int digit_bits, bool first_pass) {
+  for (int i = threadIdx.x; i < U * KV_BINS << log2_copies(U, n); i += SEL_THREADS) h[i] = 0;
+  __syncthreads();
+  const long long first = (long long)part * SEL_THREADS + threadIdx.x, stride = (long long)parts * SEL_THREADS;
+  if (first_pass) count_digits<T, 0>(row, n, first, stride, h, s->uniq, U, shift, digit_bits);
+  else if (U <= 1) count_digits<T, 1>(row, n, first, stride, h, s->uniq, U, shift, digit_bits);
+  else if (U <= 4) count_digits<T, 4>(row, n, first, stride, h, s->uniq, U, shift, digit_bits);
+  else count_digits<T, KV_MAX_RANKS>(row, n, first, stride, h, s->uniq, U, shift, digit_bits);
+  __syncthreads();
+}
+
+// One pass: grid (workgroups, metrics).  PICK: the last workgroup of a metric to finish picks the digits (`done` counts them, and is zero again
+// behind it) and clears the histogram for the next pass; with out also what the selection leaves.
+template <typename T, bool PICK>
+__global__ __launch_bounds__(SEL_THREADS) void select_pass_kernel(const T* __restrict__ x, long long n, long long row_stride, RadixState* st, unsigned int* hist, int shift, int digit_bits, bool first_pass,
+                                                                  Levels levels, unsigned int* done, unsigned long long* out) {
+  extern __shared__ __attribute__((aligned(16))) unsigned int h[];
+  __shared__ RadixState s;
+  __shared__ bool last;
+  const int tid = threadIdx.x, m = blockIdx.y;
+  copy_state(&s, st + m);
+  __syncthreads();
+  const int U = first_pass ? 1 : s.n_uniq, cl = log2_copies(U, n);
+  count_pass<T>(x + (long long)m * row_stride, n, blockIdx.x, gridDim.x, h, &s, U, shift, digit_bits, first_pass);
   unsigned int* gh = hist + (long long)m * KV_MAX_RANKS * KV_BINS;
-  if (first_pass) {
-    for (int b = tid; b < KV_BINS; b += KV_THREADS) {
-      unsigned int c = lds[b] + lds[KV_BINS + b] + lds[2 * KV_BINS + b] + lds[3 * KV_BINS + b];
-      if (c) atomicAdd(&gh[b], c);
+  for (int i = tid; i < U * KV_BINS; i += SEL_THREADS) {
+    const unsigned int c = sum_copies(h, i, cl);
+    if (c) atomicAdd(&gh[i], c);
+  }
+  if constexpr (PICK) {
+    __syncthreads();
+    if (tid == 0) {  // (one fence a workgroup: each one writes an XCD's L2 back, from every wave they took 80 us a pass)
+      __threadfence();
+      last = atomicAdd(&done[m], 1u) == gridDim.x - 1;
     }
-  } else {
-    for (int i = tid; i < U * KV_BINS; i += KV_THREADS) {
-      unsigned int c = lds[i];
-      if (c) atomicAdd(&gh[i], c);
+    __syncthreads();
+    if (!last) return;
+    unsigned int c[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j)  // (all on their way at once)
+      c[j] = tid + j * SEL_THREADS < U * KV_BINS ? __hip_atomic_load(&gh[tid + j * SEL_THREADS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int i = tid + j * SEL_THREADS;
+      if (i >= U * KV_BINS) break;
+      h[i + (i >> 5)] = c[j];
+      gh[i] = 0;
     }
+    if (tid == 0) done[m] = 0;
+    __syncthreads();
+    pick_digits(&s, h, shift + 64 - KeyOf<T>::bits, first_pass, first_pass ? &levels : nullptr);
+    copy_state(st + m, &s);
+    if (out && tid < SEL_OUT) out[(long long)m * SEL_OUT + tid] = tid < KV_MAX_RANKS ? s.prefix[tid] : s.count;
   }
 }
 
-// Ranks from quantile levels, on the device (no host round trip between the streaming
-// pass that counts the non-NaN samples and the selection): pos = p*(n-1), ranks floor(pos)
-// and ceil(pos) — the definition of analyze.py:75-81.
+// Up to 1024 samples (a run's requests): a thread per sample counts how many come in front of it.  A workgroup per metric.
+template <typename T>
+__global__ __launch_bounds__(SEL_THREADS) void select_by_rank_kernel(const T* __restrict__ x, int n, long long row_stride, Levels levels, unsigned long long* out) {
+  __shared__ __attribute__((aligned(16))) unsigned long long keys[SEL_THREADS + 1];
+  const int tid = threadIdx.x, m = blockIdx.x;
+  const T v = tid < n ? x[(long long)m * row_stride + tid] : (T)0;
+  const bool on = tid < n && v == v;
+  const unsigned long long key = (unsigned long long)KeyOf<T>::key(v) << (64 - KeyOf<T>::bits);
+  const int count = __syncthreads_count(on);
+  keys[tid] = on ? key : ~0ull;  // (no sample's key: that one is a NaN's)
+  if (tid == 0) keys[SEL_THREADS] = ~0ull;
+  __syncthreads();
+  int before = 0;
+  const int pairs = (tid & ~63) < n ? n : 0;  // (waves without a sample need not count)
+#pragma unroll 4
+  for (int j = 0; j < pairs; j += 2) {
+    const ulonglong2 k = *reinterpret_cast<const ulonglong2*>(&keys[j]);
+    before += (k.x < key || (k.x == key && j < tid) ? 1 : 0) + (k.y < key || (k.y == key && j + 1 < tid) ? 1 : 0);
+  }
+  unsigned long long* o = out + (long long)m * SEL_OUT;
+  if (tid == 0) o[KV_MAX_RANKS] = (unsigned long long)count;
+  if (on)
+    for (int r = 0; r < 2 * levels.n; ++r)
+      if (rank_of(levels, r, (unsigned long long)count) == (unsigned long long)before) o[r] = key;
+}
+
+// Few samples: all passes in one launch, a workgroup per metric.
+template <typename T>
+__global__ __launch_bounds__(SEL_THREADS) void select_few_kernel(const T* __restrict__ x, long long n, long long row_stride, Levels levels, unsigned long long* out) {
+  extern __shared__ __attribute__((aligned(16))) unsigned int h[];
+  __shared__ RadixState s;
+  const int tid = threadIdx.x, m = blockIdx.x;
+  clear_state(&s);
+  __syncthreads();
+  for (int top = KeyOf<T>::bits; top > 0;) {
+    const bool first = top == KeyOf<T>::bits;
+    const int digit_bits = top >= 11 ? 11 : top, U = first ? 1 : s.n_uniq, cl = log2_copies(U, n);
+    top -= digit_bits;
+    count_pass<T>(x + (long long)m * row_stride, n, 0, 1, h, &s, U, top, digit_bits, first);
+    unsigned int c[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int i = tid + j * SEL_THREADS;
+      c[j] = i < U * KV_BINS ? sum_copies(h, i, cl) : 0;
+    }
+    __syncthreads();  // (the sums lie where the copies were)
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int i = tid + j * SEL_THREADS;
+      if (i < U * KV_BINS) h[i + (i >> 5)] = c[j];
+    }
+    __syncthreads();
+    pick_digits(&s, h, top + 64 - KeyOf<T>::bits, first, first ? &levels : nullptr);
+  }
+  if (tid < SEL_OUT) out[(long long)m * SEL_OUT + tid] = tid < KV_MAX_RANKS ? s.prefix[tid] : s.count;
+}
+
+// clears a selection's state, histograms and counters (a kernel, not a memset: callers may capture it)
+__global__ __launch_bounds__(SEL_THREADS) void select_clear_kernel(unsigned int* words, int n) {
+  const int i = blockIdx.x * SEL_THREADS + threadIdx.x;
+  if (i < n) words[i] = 0;
+}
+
+// Samples spread over ranks: the digits of the summed histograms.  Grid: metrics.
+__global__ __launch_bounds__(SEL_THREADS) void select_scan_kernel(RadixState* st, unsigned int* hist, int shift, bool first_pass) {
+  extern __shared__ __attribute__((aligned(16))) unsigned int h[];
+  __shared__ RadixState s;
+  const int tid = threadIdx.x, m = blockIdx.x;
+  copy_state(&s, st + m);
+  unsigned int* gh = hist + (long long)m * KV_MAX_RANKS * KV_BINS;
+  for (int i = tid; i < KV_MAX_RANKS * KV_BINS; i += SEL_THREADS) {
+    h[i + (i >> 5)] = gh[i];
+    gh[i] = 0;
+  }
+  __syncthreads();
+  pick_digits(&s, h, shift, first_pass, nullptr);
+  copy_state(st + m, &s);
+}
+
+// ... and the ranks of the samples they have together (device array of levels, the count as the streaming state holds it)
 __global__ void radix_init_kernel(const StreamState* __restrict__ stream, RadixState* __restrict__ st, const double* __restrict__ ps, int n_ps) {
   const int m = blockIdx.x;
   if (threadIdx.x != 0) return;
   RadixState* s = st + m;
-  unsigned long long n = stream[m].count;
-  int r = 0;
-  if (n > 0) {
-    for (int i = 0; i < n_ps && r + 1 < KV_MAX_RANKS; ++i) {
-      double p = ps[i];
-      p = p < 0.0 ? 0.0 : (p > 1.0 ? 1.0 : p);
-      double pos = p * (double)(n - 1);
-      s->prefix[r] = 0; s->k[r] = (unsigned long long)floor(pos); ++r;
-      s->prefix[r] = 0; s->k[r] = (unsigned long long)ceil(pos); ++r;
-    }
+  Levels lv{};
+  lv.n = n_ps;
+  for (int i = 0; i < n_ps && i < KV_MAX_RANKS / 2; ++i) lv.p[i] = ps[i];
+  s->count = stream[m].count;
+  const int r = s->count ? 2 * lv.n : 0;
+  for (int i = 0; i < KV_MAX_RANKS; ++i) {
+    s->prefix[i] = 0; s->uniq[i] = 0; s->slot[i] = 0;
+    s->k[i] = i < r ? rank_of(lv, i, s->count) : 0;
   }
-  for (int i = r; i < KV_MAX_RANKS; ++i) { s->prefix[i] = 0; s->k[i] = 0; }
-  for (int i = 0; i < KV_MAX_RANKS; ++i) { s->uniq[i] = 0; s->slot[i] = 0; }
   s->n_uniq = r ? 1 : 0;
   s->n_ranks = r;
-}
-
-// One workgroup per metric: prefix-scan each rank's histogram, pick the bin that holds
-// rank k, append the digit to the prefix, subtract the counts below it, rebuild the
-// distinct-prefix list, and clear the histograms for the next pass.
-__global__ __launch_bounds__(KV_THREADS) void radix_scan_kernel(RadixState* __restrict__ st, unsigned int* __restrict__ hist, int shift, int first_pass) {
-  __shared__ unsigned long long part[KV_THREADS];
-  __shared__ int sel_bin;
-  __shared__ unsigned long long sel_below;
-  const int tid = threadIdx.x;
-  const int m = blockIdx.x;
-  RadixState* s = st + m;
-  unsigned int* gh = hist + (long long)m * KV_MAX_RANKS * KV_BINS;
-  const int R = s->n_ranks;
-  constexpr int PER = KV_BINS / KV_THREADS;  // 8 bins per thread
-
-  for (int r = 0; r < R; ++r) {
-    const unsigned int* h = gh + (first_pass ? 0 : s->slot[r]) * KV_BINS;
-    unsigned long long k = s->k[r];
-    unsigned int c[PER];
-    unsigned long long local = 0;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) { c[j] = h[tid * PER + j]; local += c[j]; }
-    part[tid] = local;
-    __syncthreads();
-    // inclusive scan over the 256 partial sums (Hillis-Steele in LDS)
-    for (int o = 1; o < KV_THREADS; o <<= 1) {
-      unsigned long long v = tid >= o ? part[tid - o] : 0;
-      __syncthreads();
-      part[tid] += v;
-      __syncthreads();
-    }
-    unsigned long long before = part[tid] - local;  // samples in bins below this thread's
-    if (k >= before && k < before + local) {
-      unsigned long long run = before;
-#pragma unroll
-      for (int j = 0; j < PER; ++j) {
-        if (k >= run && k < run + c[j]) { sel_bin = tid * PER + j; sel_below = run; }
-        run += c[j];
-      }
-    }
-    __syncthreads();
-    if (tid == 0) {
-      s->prefix[r] |= ((unsigned long long)sel_bin) << shift;
-      s->k[r] = k - sel_below;
-    }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    int nu = 0;
-    for (int r = 0; r < R; ++r) {
-      int f = -1;
-      for (int u = 0; u < nu; ++u) if (s->uniq[u] == s->prefix[r]) f = u;
-      if (f < 0) { s->uniq[nu] = s->prefix[r]; f = nu++; }
-      s->slot[r] = f;
-    }
-    s->n_uniq = nu;
-  }
-  __syncthreads();
-  for (int i = tid; i < KV_MAX_RANKS * KV_BINS; i += KV_THREADS) gh[i] = 0;
 }
 
 // ---------------------------------------------------------------------------------
@@ -482,6 +642,58 @@ __global__ __launch_bounds__(256) void gap_commit_kernel(const long long* __rest
   atomicMax(&last_t[req], t);
 }
 
+// Up to SEL_FEW samples a row one workgroup per row makes all passes, beyond a launch per pass (and one that clears) spreads them.  The line lies where
+// whole calls take as long: 3 x 32768 floats 59 us in the one form, one sample more a row 63 in the other; 5000 take 43, 100000 65.
+constexpr long long SEL_FEW = 32768;
+
+long long select_work_bytes(int n_metrics) { return (long long)n_metrics * (sizeof(RadixState) + KV_MAX_RANKS * KV_BINS * 4 + 8); }
+
+void radix_pass_geometry(int dtype, int pass, int* shift, int* digit_bits) {
+  int top = dtype == 0 ? 32 : 64;
+  for (int i = 0;; ++i) {
+    const int db = top >= 11 ? 11 : top;
+    if (i == pass) { *shift = top - db; *digit_bits = db; return; }
+    top -= db;
+  }
+}
+
+// LDS above 64 KiB has to be asked for, once per kernel
+template <typename K>
+bool big_lds(K kernel) { return hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SEL_WORDS * 4) == hipSuccess; }
+
+// workgroups per row: one a CU, each with at least 32 KiB of samples
+int select_parts(long long n, int n_metrics, int dtype) {
+  const long long want = (n * (dtype == 0 ? 4 : 8) + 32767) / 32768, most = n_metrics < 256 ? 256 / n_metrics : 1;
+  return (int)(want < 1 ? 1 : want < most ? want : most);
+}
+
+template <typename T>
+int select(const T* x, long long n, long long row_stride, int n_metrics, int dtype, const Levels& lv, void* work, unsigned long long* out, hipStream_t stream) {
+  static const bool ok = big_lds(select_few_kernel<T>) && big_lds(select_pass_kernel<T, true>);
+  if (!ok) return -2;
+  if (n <= SEL_THREADS) {
+    hipLaunchKernelGGL(select_by_rank_kernel<T>, dim3(n_metrics), dim3(SEL_THREADS), 0, stream, x, (int)n, row_stride, lv, out);
+    return (int)hipGetLastError();
+  }
+  if (n <= SEL_FEW) {
+    hipLaunchKernelGGL(select_few_kernel<T>, dim3(n_metrics), dim3(SEL_THREADS), SEL_WORDS * 4, stream, x, n, row_stride, lv, out);
+    return (int)hipGetLastError();
+  }
+  RadixState* st = (RadixState*)work;
+  unsigned int* hist = (unsigned int*)(st + n_metrics);
+  unsigned int* done = hist + (long long)n_metrics * KV_MAX_RANKS * KV_BINS;
+  const int words = (int)(select_work_bytes(n_metrics) / 4);
+  hipLaunchKernelGGL(select_clear_kernel, dim3((words + SEL_THREADS - 1) / SEL_THREADS), dim3(SEL_THREADS), 0, stream, (unsigned int*)work, words);
+  const dim3 grid(select_parts(n, n_metrics, dtype), n_metrics);
+  const int passes = (dtype == 0 ? 3 : 6);
+  for (int p = 0; p < passes; ++p) {
+    int shift = 0, digit_bits = 0;
+    radix_pass_geometry(dtype, p, &shift, &digit_bits);
+    hipLaunchKernelGGL((select_pass_kernel<T, true>), grid, dim3(SEL_THREADS), SEL_WORDS * 4, stream, x, n, row_stride, st, hist, shift, digit_bits, p == 0, lv, done, p == passes - 1 ? out : nullptr);
+  }
+  return (int)hipGetLastError();
+}
+
 }  // namespace
 
 extern "C" {
@@ -521,28 +733,18 @@ int kv_radix_init(const void* stream_state, void* st, const double* ps, int n_ps
   return (int)hipGetLastError();
 }
 
-// Runs every radix pass.  ``st`` must be initialised by the caller (prefix = 0, k = target
-// rank, n_ranks), ``hist`` is [n_metrics][8][2048] zeros.  On return st->prefix[r]
-// holds the order-preserving key of rank r (left-aligned in 64 bits).
-int kv_radix_select(const void* x, long long n, long long row_stride, int n_metrics, int dtype, void* st, unsigned int* hist, hipStream_t stream) {
-  if (n <= 0 || n_metrics <= 0) return 0;
-  const int key_bits = dtype == 0 ? 32 : 64;
-  dim3 grid(grid_x(n, 16), n_metrics);
-  int top = key_bits;
-  int first = 1;
-  while (top > 0) {
-    int digit_bits = top >= 11 ? 11 : top;
-    int shift = top - digit_bits;
-    if (dtype == 0)
-      hipLaunchKernelGGL(radix_hist_kernel<float>, grid, dim3(KV_THREADS), 0, stream, (const float*)x, n, row_stride, (const RadixState*)st, hist, shift, digit_bits, first);
-    else
-      hipLaunchKernelGGL(radix_hist_kernel<double>, grid, dim3(KV_THREADS), 0, stream, (const double*)x, n, row_stride, (const RadixState*)st, hist, shift, digit_bits, first);
-    // prefixes are kept left-aligned in 64 bits for both dtypes
-    hipLaunchKernelGGL(radix_scan_kernel, dim3(n_metrics), dim3(KV_THREADS), 0, stream, (RadixState*)st, hist, shift + (64 - key_bits), first);
-    first = 0;
-    top = shift;
-  }
-  return (int)hipGetLastError();
+// Selection of the order statistics around n_ps <= 4 quantile levels of every row of x, in scratch memory `work` (kv_select_work_bytes; nothing
+// in it needs to be set).  out: [n_metrics][9], the order-preserving keys of the floor and ceil ranks (left-aligned in 64 bits) and the count.
+long long kv_select_work_bytes(int n_metrics) { return select_work_bytes(n_metrics); }
+
+int kv_radix_num_passes(int dtype) { return dtype == 0 ? 3 : 6; }
+
+int kv_select_quantiles(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const double* ps, int n_ps, void* work, unsigned long long* out, hipStream_t stream) {
+  if (n <= 0 || n_metrics <= 0 || n_metrics > 65535 || n_ps < 1 || n_ps > KV_MAX_RANKS / 2) return -1;
+  Levels lv{};
+  lv.n = n_ps;
+  for (int i = 0; i < n_ps; ++i) lv.p[i] = ps[i];
+  return dtype == 0 ? select((const float*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream) : select((const double*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream);
 }
 
 // The same selection one pass at a time, for samples spread over several ranks: every rank runs
@@ -550,27 +752,18 @@ int kv_radix_select(const void* x, long long n, long long row_stride, int n_metr
 // [n_metrics][8][2048] counts per pass), and every rank runs pass_scan on the summed counts — the
 // selection state stays identical everywhere and ends at the exact order statistics of the union.
 // The state must have been initialised from the GLOBAL sample count.
-int kv_radix_num_passes(int dtype) { return dtype == 0 ? 3 : 6; }
-
-static void radix_pass_geometry(int dtype, int pass, int* shift, int* digit_bits) {
-  int top = dtype == 0 ? 32 : 64;
-  for (int i = 0;; ++i) {
-    const int db = top >= 11 ? 11 : top;
-    if (i == pass) { *shift = top - db; *digit_bits = db; return; }
-    top -= db;
-  }
-}
-
-int kv_radix_pass_hist(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const void* st, unsigned int* hist, int pass, hipStream_t stream) {
+int kv_radix_pass_hist(const void* x, long long n, long long row_stride, int n_metrics, int dtype, void* st, unsigned int* hist, int pass, hipStream_t stream) {
   if (n_metrics <= 0 || pass < 0 || pass >= kv_radix_num_passes(dtype)) return -1;
   if (n <= 0) return 0;  // a rank without samples contributes zeros
   int shift = 0, digit_bits = 0;
   radix_pass_geometry(dtype, pass, &shift, &digit_bits);
-  dim3 grid(grid_x(n, 16), n_metrics);
+  const dim3 grid(select_parts(n, n_metrics, dtype), n_metrics);
+  static const bool ok = big_lds(select_pass_kernel<float, false>) && big_lds(select_pass_kernel<double, false>);
+  if (!ok) return -2;
   if (dtype == 0)
-    hipLaunchKernelGGL(radix_hist_kernel<float>, grid, dim3(KV_THREADS), 0, stream, (const float*)x, n, row_stride, (const RadixState*)st, hist, shift, digit_bits, pass == 0 ? 1 : 0);
+    hipLaunchKernelGGL((select_pass_kernel<float, false>), grid, dim3(SEL_THREADS), SEL_WORDS * 4, stream, (const float*)x, n, row_stride, (RadixState*)st, hist, shift, digit_bits, pass == 0, Levels{}, nullptr, nullptr);
   else
-    hipLaunchKernelGGL(radix_hist_kernel<double>, grid, dim3(KV_THREADS), 0, stream, (const double*)x, n, row_stride, (const RadixState*)st, hist, shift, digit_bits, pass == 0 ? 1 : 0);
+    hipLaunchKernelGGL((select_pass_kernel<double, false>), grid, dim3(SEL_THREADS), SEL_WORDS * 4, stream, (const double*)x, n, row_stride, (RadixState*)st, hist, shift, digit_bits, pass == 0, Levels{}, nullptr, nullptr);
   return (int)hipGetLastError();
 }
 
@@ -579,7 +772,9 @@ int kv_radix_pass_scan(void* st, unsigned int* hist, int n_metrics, int dtype, i
   int shift = 0, digit_bits = 0;
   radix_pass_geometry(dtype, pass, &shift, &digit_bits);
   const int key_bits = dtype == 0 ? 32 : 64;
-  hipLaunchKernelGGL(radix_scan_kernel, dim3(n_metrics), dim3(KV_THREADS), 0, stream, (RadixState*)st, hist, shift + (64 - key_bits), pass == 0 ? 1 : 0);
+  static const bool ok = big_lds(select_scan_kernel);
+  if (!ok) return -2;
+  hipLaunchKernelGGL(select_scan_kernel, dim3(n_metrics), dim3(SEL_THREADS), KV_MAX_RANKS * SEL_ROW * 4, stream, (RadixState*)st, hist, shift + (64 - key_bits), pass == 0);
   return (int)hipGetLastError();
 }
 

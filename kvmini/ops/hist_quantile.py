@@ -91,32 +91,26 @@ def batched_quantiles(samples: Any, ps: Sequence[float] = (0.5, 0.95, 0.99), ret
         x = x.contiguous()
     if x.dim() == 1:
         x = x.unsqueeze(0)
-    m, n = x.shape
+    m = x.shape[0]
     is_double = x.dtype == torch.float64
-    dev = x.device
-    state, hist = _new_stream_state(m, dev)
-    C.stream_hist(x, n, hist, state, LO_LOG2, HI_LOG2)
-    rstate = torch.zeros(m * C.radix_state_bytes(), dtype=torch.uint8, device=dev)
-    rhist = torch.zeros((m, 8, BINS), dtype=torch.int32, device=dev)
-    ps_dev = torch.tensor(list(ps), dtype=torch.float64, device=dev)
-    C.radix_select(x, n, state, ps_dev, rstate, rhist)
-    rs = rstate.cpu().numpy()
-    stats = _decode_stream_state(state.cpu().numpy(), m, is_double)
-    rb = C.radix_state_bytes()
+    found = C.select_quantiles(x, [float(p) for p in ps]).numpy().view(np.uint64).tolist()
     out = np.full((m, len(ps)), np.nan, dtype=np.float64)
     for i in range(m):
-        cnt = stats[i]["count"]
+        *keys, cnt = found[i]
         if cnt == 0:
             continue
-        prefixes = struct.unpack("<8Q", rs[i * rb : i * rb + 64].tobytes())
         for j, p in enumerate(ps):
             p = max(0.0, min(float(p), 1.0))
             pos = p * (cnt - 1)
             lo = math.floor(pos)
-            v_lo = _key_to_value(prefixes[2 * j], is_double)
-            v_hi = _key_to_value(prefixes[2 * j + 1], is_double)
+            v_lo = _key_to_value(keys[2 * j], is_double)
+            v_hi = _key_to_value(keys[2 * j + 1], is_double)
             out[i, j] = v_lo if cnt == 1 or lo == math.ceil(pos) else v_lo + (pos - lo) * (v_hi - v_lo)
-    return (out, stats) if return_stats else out
+    if not return_stats:
+        return out
+    state, hist = _new_stream_state(m, x.device)
+    C.stream_hist(x, x.shape[1], hist, state, LO_LOG2, HI_LOG2)
+    return out, _decode_stream_state(state.cpu().numpy(), m, is_double)
 
 
 def _float_keys(x: np.ndarray) -> np.ndarray:
@@ -136,7 +130,7 @@ def distributed_quantiles(samples: Any, ps: Sequence[float], dist: Any, group: A
     sum the histograms (one all-reduce of 8 x 2048 counts per pass: 3 passes for float32, 6 for
     float64) and every rank walks the summed counts — so the selection state is the same
     everywhere and ends at the order statistics of the union.  NaN = missing.  On a GPU the
-    passes are ``radix_hist_kernel`` / ``radix_scan_kernel`` (csrc/hist_quantile.hip) and the
+    passes are ``select_pass_kernel`` / ``select_scan_kernel`` (csrc/hist_quantile.hip) and the
     all-reduce is RCCL's; on the host the same protocol runs in numpy (CPU rehearsals, tests).
     Every rank returns the same list; all NaN when no rank has a sample."""
     torch = _torch()

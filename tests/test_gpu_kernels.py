@@ -151,6 +151,35 @@ def test_quantiles_batched_ragged_and_degenerate():
     assert stats[1]["min"] == mat[1, :1234].min() and stats[1]["max"] == mat[1, :1234].max()
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m,n", [(1, 3), (3, 511), (4, 1023), (2, 1024), (3, 1025), (1, 8193), (3, 32767), (2, 32768), (3, 32769), (4, 99991), (1, 400003)])
+def test_quantiles_at_every_form_of_the_selection(m, n, dtype):
+    """Sizes on both sides of every change of form, rows that do not start at whole 16 bytes, ties, infinities, both zeros, missing rows; and the
+    passes one by one, as ranks that hold a part each make them."""
+    from kvmini.analysis.quantiles import percentiles
+    from kvmini.ops import hist_quantile as hq
+
+    rng = np.random.default_rng(n + m)
+    x = (12 * np.exp(rng.normal(size=(m, n)))).astype(dtype)
+    x[rng.random((m, n)) < 0.05] = np.nan
+    x[0, :: 7] *= -1
+    x[-1, :: 3] = 8.0
+    x[0, 0], x[0, 1], x[0, 2] = 0.0, -0.0, np.inf
+    if m > 2:
+        x[1] = np.nan
+    d = torch.from_numpy(x).to(_dev())
+    for ps in ((0.5, 0.95, 0.99), (0.0, 0.25, 0.999, 1.0)):
+        got = hq.batched_quantiles(d, ps)
+        for i in range(m):
+            want = np.full(len(ps), np.nan) if np.isnan(x[i]).all() else np.asarray(percentiles(x[i].astype(np.float64), ps, engine="numpy"))
+            assert np.array_equal(got[i], want, equal_nan=True), (ps, i, got[i], want)
+
+    class OneRank:  # (what torch.distributed does for a group of one)
+        all_reduce = staticmethod(lambda t, group=None: None)
+
+    assert np.array_equal(hq.distributed_quantiles(x[0], (0.5, 0.95, 0.99), OneRank, device=_dev()), hq.batched_quantiles(d[:1], (0.5, 0.95, 0.99))[0])
+
+
 def test_equal_width_histogram_matches_cpu():
     from kvmini.analysis.histograms import compute_histogram
     from kvmini.ops import hist_quantile as hq
