@@ -114,9 +114,9 @@ __device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1
   int slot = 0;
   // The barrier at the top of stage s: everybody's pieces of stage s + 1 have landed, and everybody has multiplied stage s - 1, whose place
   // stage s + AHEAD takes.  (Reads still in flight there are of stage s.)
-  auto stage = [&](auto uc, int s) __attribute__((always_inline)) {
+  auto stage = [&](auto uc, auto more, int s) __attribute__((always_inline)) {
     constexpr int u = decltype(uc)::value;
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 2) * OPS) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((more ? AHEAD - 2 : AHEAD - 2 - u) * OPS) : "memory");
     __builtin_amdgcn_s_barrier();
     const int next = slot + 1 == RING ? 0 : slot + 1;
     const unsigned char* cur = ring + slot * STAGE;
@@ -134,7 +134,7 @@ __device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1
 #pragma unroll
         for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][k][i]), b[set][e], acc[i][j], 0, 0, 0);
       }
-      fetch(t, u, sa, dst);
+      if constexpr (more) fetch(t, u, sa, dst);
       __builtin_amdgcn_sched_barrier(0);
     }
     slot = next;
@@ -142,16 +142,17 @@ __device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1
   static_assert(AHEAD == 3, "the unrolled loop and its tail");
   int s = 0;
   for (; s + 3 <= n; s += 3) {
-    stage(std::integral_constant<int, 0>{}, s);
-    stage(std::integral_constant<int, 1>{}, s + 1);
-    stage(std::integral_constant<int, 2>{}, s + 2);
+    stage(std::integral_constant<int, 0>{}, std::true_type{}, s);
+    stage(std::integral_constant<int, 1>{}, std::true_type{}, s + 1);
+    stage(std::integral_constant<int, 2>{}, std::true_type{}, s + 2);
     if constexpr (NB & 1) {  // (an odd number of batches: the sets have swapped)
 #pragma unroll
       for (int e = 0; e < 4; ++e) { const frag_ab v = b[0][e]; b[0][e] = b[1][e]; b[1][e] = v; }
     }
   }
-  if (s < n) stage(std::integral_constant<int, 0>{}, s);
-  if (s + 1 < n) stage(std::integral_constant<int, 1>{}, s + 1);
+  // (the last stages fetch nothing: the compiler would drop loads of weights that no stage multiplies, and the counts be wrong)
+  if (s < n) stage(std::integral_constant<int, 0>{}, std::false_type{}, s);
+  if (s + 1 < n) stage(std::integral_constant<int, 1>{}, std::false_type{}, s + 1);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
 }
 
