@@ -190,7 +190,8 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  const int n = p.K / 64, start = id * 5 % n;
+  // (the column a workgroup starts at is its expert's and panel's: which of the expert's tiles a row falls into changes from run to run, its sums must not)
+  const int n = p.K / 64, start = (p.groups.tile_expert[tile] * p.n_panels + panel) * 5 % n;
   switch (nf) {
     case 16: multiply<16>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
     case 14: multiply<14>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
