@@ -1,24 +1,28 @@
-// Tiled products of a mixture of experts for many rows on gfx950: the (token, choice) pairs that chose an expert, up to 256 a tile, times the
-// expert's matrix, y[pair] = W[expert] x[row of the pair].
-//
-// What bounds it is the matrices: every expert's is read once (1.2 GB for 64 of 2304 x 4096), for some 100 to 300 rows, so bytes and matrix
-// work take about as long.  Hence:
-//  * A workgroup is a panel of 256 features x the tile's rows; each of its 8 waves owns 32 features and all rows.  Weights (fragment order
-//    [N/16][K/32][64][8]) go straight to registers, no byte twice, 3 stages of 64 columns ahead (96 KiB of them in flight per CU: through
-//    LDS there was room for 48), the rows to LDS by LDS-DMA, as far ahead, in a ring of 4 stages; all waves read all rows from there.
-//    They are read past the caches' reuse (nobody else wants them) and every workgroup starts at another column and goes round: panels lie a
-//    power of two apart, and in step they would all ask the same memory channels.  (293 -> 262 us; either alone 278 and 292.)
+// Products by panels of 256 features on gfx950, for one matrix of many outputs and for a mixture of experts with many rows.
+//  * A workgroup is a panel x up to 256 rows; each of its 8 waves owns 32 features and all rows.  Weights (fragment order [N/16][K/32][64][8]) go
+//    straight to registers, no byte twice, 3 to 6 stages of 64 columns ahead (96 KiB of them in flight per CU: through LDS there was room for
+//    48), the rows to LDS by LDS-DMA, as far ahead, in a ring; all waves read all rows from there.
+//  * The barrier of a stage stands before its last batch, where the first read of the next stage is issued, not at its top: what is fetched has a
+//    stage longer to come (2048 x 28672 x 4096: 390 -> 373 us).
 //  * Work follows the rows that exist, in steps of 32: 2 x NF products per 64 columns and feature tile, NF = rows / 16 rounded up to an even
 //    number, one loop for each NF.  All waves have the same share, whatever the number.
 //  * LDS-DMA and loads are buffer instructions: the offset of a stage is scalar, and the compiler counts them exactly in front of a use (beside
 //    the FLAT form it waits for everything in flight).
 //  * Stores are 16 bytes a lane, gathered from the two feature tiles (and, gated, two row tiles) by lane swaps.
-// Measured, 64 experts of 2304 x 4096 with 187 rows each: 282 us; the tile of 256 x 256 through LDS (all 256 rows multiplied) 338 us.  64 rows: 246
+// Four waves of 64 features each, which read the LDS half as often, are slower (464 against 395 us): with one wave per SIMD nothing multiplies
+// while it issues memory operations.
+//
+// Experts (the (token, choice) pairs that chose one, up to 256 a tile, y[pair] = W[expert] x[row of the pair]) are bound by the matrices: every one is
+// read once (1.2 GB for 64 of 2304 x 4096) for some 100 to 300 rows, so bytes and matrix work take about as long.  They are read past the
+// caches' reuse (nobody else wants them) and every workgroup starts at another column and goes round: panels lie a power of two apart, and in step
+// they would all ask the same memory channels.  (293 -> 262 us; either alone 278 and 292.)
+// Measured, 64 experts of 2304 x 4096 with 187 rows each: 282 us; a tile of 256 x 256 through LDS (all 256 rows multiplied) 338 us.  64 rows: 246
 // against 311 us.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <type_traits>
+#include <utility>
 
 #include "experts.h"
 
@@ -33,8 +37,9 @@ typedef __amdgpu_buffer_rsrc_t rsrc_t;
 enum Mode { PLAIN = 0, GATED = 1, SQUARED = 2 };
 
 constexpr int ROWS = 256, FEATURES = 256;  // of a tile
-constexpr int AHEAD = 3, RING = AHEAD + 1;  // stages of 64 columns
-constexpr int STAGE = ROWS * 128;           // bytes of a stage's rows
+constexpr int RING_BYTES = 144 * 1024;
+// stages of 64 columns in flight, and one more in the ring: as many as registers (16 of weights a stage) and LDS (2 KiB of rows per row tile) hold
+constexpr int ahead(int nf) { return nf > 14 ? 3 : nf > 12 ? 4 : nf > 10 ? 5 : 6; }
 
 struct PanelArgs {
   const unsigned char* w; const __bf16* x; unsigned short* y;
@@ -53,8 +58,9 @@ __device__ inline unsigned int f2bf(float f) {
 __device__ inline uint2 pack4(frag_cd v) { return make_uint2(f2bf(v[0]) | f2bf(v[1]) << 16, f2bf(v[2]) | f2bf(v[3]) << 16); }
 
 __device__ inline rsrc_t buffer_of(const void* p, unsigned int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00027000); }
-constexpr int NON_TEMPORAL = 2;
-__device__ inline raw16 load16(rsrc_t r, int lane_off, int off) { return __builtin_bit_cast(raw16, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, NON_TEMPORAL)); }
+enum Caching { REUSED = 0, ONCE = 2 };  // of a load: ONCE is past the caches' reuse
+template <int CACHING>
+__device__ inline raw16 load16(rsrc_t r, int lane_off, int off) { return __builtin_bit_cast(raw16, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, CACHING)); }
 // one LDS-DMA piece: lane l's 16 bytes land at lds + 16 l
 __device__ inline void dma16(rsrc_t r, int lane_off, int off, void* lds) { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, lane_off, off, 0, 0); }
 
@@ -65,9 +71,14 @@ __device__ inline int piece_of(int wave, int i, int pieces) {
   return p < pieces ? p : i > 0 ? p - 8 : p % pieces;
 }
 
+template <class F, int... U>
+__device__ __attribute__((always_inline)) inline void each(const F& f, std::integer_sequence<int, U...>) { (f(std::integral_constant<int, U>{}), ...); }
+
 // acc[i][j] += the wave's feature tile i x rows 16 j .. of NF row tiles (a multiple of two), over n stages of 64 columns
-template <int NF>
-__device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int start, int wave, int lane) {
+template <int NF, int CACHING>
+__device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int start, int wave, int lane) {
+  constexpr int AHEAD = ahead(NF), RING = AHEAD + 1, STAGE = NF * 2048;
+  static_assert(RING * STAGE <= RING_BYTES, "ring");
   constexpr int PX = (2 * NF + 7) / 8, OPS = 4 + PX;  // pieces of x and memory operations per wave and stage
   constexpr int F = 2 * NF, NB = F / 4;               // row fragments of a stage (two k-steps), in batches of four
   const int r = lane & 15, q = lane >> 4;
@@ -97,8 +108,8 @@ __device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1
 #pragma unroll
     for (int k = 0; k < 2; ++k)
       if (t == (k == 0 ? (NF - 1) / 4 : NB - 1)) {
-        w[u][k][0] = load16(wr, w0, st * 2048 + k * 1024);
-        w[u][k][1] = load16(wr, w1, st * 2048 + k * 1024);
+        w[u][k][0] = load16<CACHING>(wr, w0, st * 2048 + k * 1024);
+        w[u][k][1] = load16<CACHING>(wr, w1, st * 2048 + k * 1024);
       }
   };
 #pragma unroll
@@ -112,12 +123,15 @@ __device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1
   __builtin_amdgcn_s_barrier();
   read(0, ring, 0);
   int slot = 0;
-  // The barrier at the top of stage s: everybody's pieces of stage s + 1 have landed, and everybody has multiplied stage s - 1, whose place
-  // stage s + AHEAD takes.  (Reads still in flight there are of stage s.)
+  // The barrier before the last batch of stage s: everybody's pieces of stage s + 1, read from there on, have landed, and everybody's reads of stage s,
+  // whose place stage s + RING takes, are answered.
+  constexpr int BEFORE = [] {  // memory operations of a stage in front of its last batch
+    int c = (NF - 1) / 4 < NB - 1 ? 2 : 0;
+    for (int i = 0; i < PX; ++i) c += i * NB / PX < NB - 1;
+    return c;
+  }();
   auto stage = [&](auto uc, auto more, int s) __attribute__((always_inline)) {
     constexpr int u = decltype(uc)::value;
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((more ? AHEAD - 2 : AHEAD - 2 - u) * OPS) : "memory");
-    __builtin_amdgcn_s_barrier();
     const int next = slot + 1 == RING ? 0 : slot + 1;
     const unsigned char* cur = ring + slot * STAGE;
     const unsigned char* nxt = ring + next * STAGE;
@@ -126,6 +140,10 @@ __device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1
 #pragma unroll
     for (int t = 0; t < NB; ++t) {
       const int set = (u * NB + t) & 1;
+      if (t == NB - 1) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(more ? (AHEAD - 2) * OPS + BEFORE : (AHEAD - 2 - u) * OPS) : "memory");
+        __builtin_amdgcn_s_barrier();
+      }
       read(set ^ 1, t + 1 < NB ? cur : nxt, t + 1 < NB ? t + 1 : 0);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -139,35 +157,94 @@ __device__ inline void multiply(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1
     }
     slot = next;
   };
-  static_assert(AHEAD == 3, "the unrolled loop and its tail");
   int s = 0;
-  for (; s + 3 <= n; s += 3) {
-    stage(std::integral_constant<int, 0>{}, std::true_type{}, s);
-    stage(std::integral_constant<int, 1>{}, std::true_type{}, s + 1);
-    stage(std::integral_constant<int, 2>{}, std::true_type{}, s + 2);
-    if constexpr (NB & 1) {  // (an odd number of batches: the sets have swapped)
+  for (; s + AHEAD <= n; s += AHEAD) {
+    each([&](auto uc) __attribute__((always_inline)) { stage(uc, std::true_type{}, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD>{});
+    if constexpr ((AHEAD * NB) & 1) {  // (an odd number of batches: the sets have swapped)
 #pragma unroll
       for (int e = 0; e < 4; ++e) { const frag_ab v = b[0][e]; b[0][e] = b[1][e]; b[1][e] = v; }
     }
   }
   // (the last stages fetch nothing: the compiler would drop loads of weights that no stage multiplies, and the counts be wrong)
-  if (s < n) stage(std::integral_constant<int, 0>{}, std::false_type{}, s);
-  if (s + 1 < n) stage(std::integral_constant<int, 1>{}, std::false_type{}, s + 1);
+  each([&](auto uc) __attribute__((always_inline)) { if (s + decltype(uc)::value < n) stage(uc, std::false_type{}, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD - 1>{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
+}
+
+template <int CACHING>
+__device__ __attribute__((always_inline)) inline void multiply(int nf, frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int start, int wave, int lane) {
+  switch (nf) {
+    case 16: multiply_rows<16, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 14: multiply_rows<14, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 12: multiply_rows<12, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 10: multiply_rows<10, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 8: multiply_rows<8, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 6: multiply_rows<6, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 4: multiply_rows<4, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    default: multiply_rows<2, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+  }
+}
+
+// What a wave stores of its 32 features from f0 on.  acc[i][j][e]: feature 16 i + 4 q + e, row 16 j + r, to be multiplied by scale(j); gate(g, u) of a
+// gated product; out(row): the row's outputs.
+template <int MODE, class Scale, class Gate, class Out>
+__device__ __attribute__((always_inline)) inline void store_rows(frag_cd (&acc)[2][16], int rows, int f0, int lane, Scale scale, Gate gate, Out out) {
+  const int r = lane & 15, q = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < 16; j += 2) {
+    if (16 * j >= rows) break;
+    uint2 v[2][2];  // [row tile][half]: halves are feature tiles, or (gated) one half of the lanes has one and the other the other
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      frag_cd a = acc[0][j + t], b = acc[1][j + t];
+      const float by = scale(j + t);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { a[e] *= by; b[e] *= by; }
+      if constexpr (MODE == GATED) {  // a tile is 8 gate rows and their 8 up rows: the upper half of the lanes takes the other tile's
+        frag_cd o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const auto gu = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[e]), __float_as_uint(b[e]), false, false);
+          o[e] = gate(__uint_as_float(gu[0]), __uint_as_float(gu[1]));
+        }
+        v[0][t] = pack4(o);
+      } else {
+        if constexpr (MODE == SQUARED) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { a[e] = fmaxf(a[e], 0.f); b[e] = fmaxf(b[e], 0.f); a[e] *= a[e]; b[e] *= b[e]; }
+        }
+        v[t][0] = pack4(a);
+        v[t][1] = pack4(b);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < (MODE == GATED ? 1 : 2); ++t) {
+      // sixteen lanes each: 0 the first half's (4 + 4 features), 1 the second's, 2 and 3 those eight features further
+      const auto lo = __builtin_amdgcn_permlane16_swap(v[t][0].x, v[t][1].x, false, false), hi = __builtin_amdgcn_permlane16_swap(v[t][0].y, v[t][1].y, false, false);
+      const raw16 o = {lo[0], hi[0], lo[1], hi[1]};
+      const int row = 16 * (j + (MODE == GATED ? q & 1 : t)) + r;
+      const int f = MODE == GATED ? f0 / 2 + 8 * (q >> 1) : f0 + 16 * (q & 1) + 8 * (q >> 1);
+      if (row < rows) *reinterpret_cast<raw16*>(out(row) + f) = o;
+    }
+  }
+}
+
+// i of 0 .. n - 1, as workgroups come, to an index such that each XCD (i % 8) has a contiguous range
+__device__ inline int xcd_range(int i, int n) {
+  const int xcd = i & 7, qd = n >> 3, rm = n & 7;
+  return (xcd < rm ? xcd * (qd + 1) : rm * (qd + 1) + (xcd - rm) * qd) + (i >> 3);
 }
 
 template <int MODE>
 __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = lane & 15, q = lane >> 4;
   // blockIdx -> (tile, panel): of those that exist, each XCD has a contiguous range, panels fastest (a tile's panels share its rows through that L2)
   const int nwg = p.groups.n_tiles[0] * p.n_panels;
   int id = blockIdx.x;
   {
     const int xcd = id & 7, qd = nwg >> 3, rm = nwg & 7;
     if ((id >> 3) >= qd + (xcd < rm ? 1 : 0)) return;
-    id = (xcd < rm ? xcd * (qd + 1) : rm * (qd + 1) + (xcd - rm) * qd) + (id >> 3);
+    id = xcd_range(id, nwg);
   }
   const int tile = id / p.n_panels, panel = id % p.n_panels;
   const int* row_of = p.groups.order + p.groups.tile_first[tile];
@@ -192,62 +269,78 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
   // (the column a workgroup starts at is its expert's and panel's: which of the expert's tiles a row falls into changes from run to run, its sums must not)
   const int n = p.K / 64, start = (p.groups.tile_expert[tile] * p.n_panels + panel) * 5 % n;
-  switch (nf) {
-    case 16: multiply<16>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 14: multiply<14>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 12: multiply<12>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 10: multiply<10>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 8: multiply<8>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 6: multiply<6>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 4: multiply<4>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    default: multiply<2>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-  }
-  // acc[i][j][e]: feature 16 i + 4 q + e of the wave's 32, row 16 j + r
+  multiply<ONCE>(nf, acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane);
   const int f0 = panel * FEATURES + wave * 32;
   if (f0 >= p.N) return;
-#pragma unroll
-  for (int j = 0; j < 16; j += 2) {
-    if (16 * j >= rows) break;
-    uint2 v[2][2];  // [row tile][half]: halves are feature tiles, or (gated) one half of the lanes has one and the other the other
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      frag_cd a = acc[0][j + t], b = acc[1][j + t];
-      if constexpr (MODE == GATED) {  // a tile is 8 gate rows and their 8 up rows: the upper half of the lanes takes the other tile's
-        frag_cd o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const auto gu = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[e]), __float_as_uint(b[e]), false, false);
-          o[e] = expert_gate(__uint_as_float(gu[0]), __uint_as_float(gu[1]), p.gate);
-        }
-        v[0][t] = pack4(o);
-      } else {
-        if constexpr (MODE == SQUARED) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) { a[e] = fmaxf(a[e], 0.f); b[e] = fmaxf(b[e], 0.f); a[e] *= a[e]; b[e] *= b[e]; }
-        }
-        v[t][0] = pack4(a);
-        v[t][1] = pack4(b);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < (MODE == GATED ? 1 : 2); ++t) {
-      // sixteen lanes each: 0 the first half's (4 + 4 features), 1 the second's, 2 and 3 those eight features further
-      const auto lo = __builtin_amdgcn_permlane16_swap(v[t][0].x, v[t][1].x, false, false), hi = __builtin_amdgcn_permlane16_swap(v[t][0].y, v[t][1].y, false, false);
-      const raw16 o = {lo[0], hi[0], lo[1], hi[1]};
-      const int row = 16 * (j + (MODE == GATED ? q & 1 : t)) + r;
-      const int f = MODE == GATED ? f0 / 2 + 8 * (q >> 1) : f0 + 16 * (q & 1) + 8 * (q >> 1);
-      if (row < rows) *reinterpret_cast<raw16*>(p.y + (long long)row_of[row] * p.ldy + f) = o;
-    }
-  }
+  store_rows<MODE>(acc, rows, f0, lane, [](int) { return 1.f; }, [&](float g, float u) { return expert_gate(g, u, p.gate); },
+                   [&](int row) { return p.y + (long long)row_of[row] * p.ldy; });
 }
 
+// ---- one matrix for all rows -----------------------------------------------------------------------------------------
+// y[M, N] = x[M, K] W[N, K]^T, the matrix multiplied by panels of 256 features x `height` rows: workgroups of one matrix share what they read through
+// the L2, panels in order, a panel's tiles next to one another.  The height is free in steps of 32, so that panels x tiles fill the CUs in whole rounds;
+// the panels of a last round may have another.  Bound by the matrix cores and the power they draw (2048 x 28672 x 4096 of zeros takes 308 us, of random
+// numbers 373) and by some 8 us per round outside the K loop.  Against tiles of up to 256 x 256 with both operands through LDS, 2048 rows:
+// 28672 x 4096 416 -> 358 us (1.34 PFLOP/s), 9216 x 4096 161 -> 129, 16384 x 2048 130 -> 111, 4096 x 14336 196 -> 190, 5632 x 2048 53 -> 44.
+struct DenseArgs {
+  const unsigned char* w; const __bf16* x; unsigned short* y;
+  int M, N, K; long long ldx, ldy;
+  int height[2], tiles[2];  // of a tile, and tiles per panel: of the first `panels`, and of those behind them
+  int panels;
+  const float* row_ss; int ss_parts; float inv_k, eps; int gelu;
+};
+
 template <int MODE>
-int launch(const PanelArgs& a, hipStream_t s) {
-  constexpr int LDS = RING * STAGE;
-  const auto kern = expert_panel_kernel<MODE>;
-  static const hipError_t lds_ok = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+__global__ __launch_bounds__(512) void dense_panel_kernel(const DenseArgs p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+  float* const row_scale = reinterpret_cast<float*>(ring + RING_BYTES);  // [ROWS]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int first = p.panels * p.tiles[0];
+  const bool behind = (int)blockIdx.x >= first;
+  const int id = behind ? xcd_range(blockIdx.x - first, gridDim.x - first) : xcd_range(blockIdx.x, first);
+  const int height = p.height[behind], tiles = p.tiles[behind];
+  const int panel = (behind ? p.panels : 0) + id / tiles, m0 = id % tiles * height;
+  const int rows = p.M - m0 < height ? p.M - m0 : height;
+  const int nf = (rows + 31) / 32 * 2, nks = p.K / 32;
+  if (p.row_ss != nullptr) {
+    const int i = threadIdx.x < rows ? threadIdx.x : rows - 1;
+    float ss = 0.f;
+    for (int k = 0; k < p.ss_parts; ++k) ss += p.row_ss[(long long)(m0 + i) * p.ss_parts + k];
+    if (threadIdx.x < ROWS) row_scale[threadIdx.x] = rsqrtf(ss * p.inv_k + p.eps);
+  }
+  const int have = p.N / 16 - panel * (FEATURES / 16) < FEATURES / 16 ? p.N / 16 - panel * (FEATURES / 16) : FEATURES / 16;  // feature tiles; past them reads give zeros
+  const rsrc_t wr = buffer_of(p.w + (long long)panel * (FEATURES / 16) * nks * 1024, (unsigned int)have * nks * 1024);
+  const int w0 = 2 * wave * nks * 1024 + lane * 16, w1 = w0 + nks * 1024;
+  const rsrc_t xr = buffer_of(p.x + m0 * p.ldx, (unsigned int)(((rows - 1) * p.ldx + p.K) * 2));
+  int xsrc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 8 * piece_of(wave, i, 2 * nf) + (lane >> 3);
+    xsrc[i] = (row < rows ? row : rows - 1) * (int)(p.ldx * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+  }
+  frag_cd acc[2][16];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
+  multiply<REUSED>(nf, acc, wr, w0, w1, xr, xsrc, ring, p.K / 64, 0, wave, lane);
+  if (p.row_ss != nullptr) __syncthreads();
+  const int f0 = panel * FEATURES + wave * 32;
+  if (f0 >= p.N) return;
+  store_rows<MODE>(acc, rows, f0, lane, [&](int j) { return p.row_ss != nullptr ? row_scale[16 * j + (lane & 15)] : 1.f; },
+                   [&](float g, float u) {  // silu(z) = z sigmoid(z); gelu_tanh(z) = z sigmoid(2 sqrt(2 / pi) (z + 0.044715 z^3))
+                     const float z = p.gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
+                     return g / (1.f + __expf(-z)) * u;
+                   },
+                   [&](int row) { return p.y + (m0 + row) * p.ldy; });
+}
+
+template <auto KERNEL, class Args>
+int launch(const Args& a, int grid, hipStream_t s) {
+  constexpr int LDS = RING_BYTES + ROWS * 4;
+  static const hipError_t lds_ok = hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (lds_ok != hipSuccess) return -2;
-  hipLaunchKernelGGL(kern, dim3(a.groups.max_tiles * a.n_panels), dim3(512), LDS, s, a);
+  hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(512), LDS, s, a);
   return (int)hipGetLastError();
 }
 
@@ -270,7 +363,36 @@ int kv_expert_panels(const void* Wp, const void* x, void* y, int N, int K, long 
   a.x_bytes = (unsigned int)bytes;
   a.gate = ExpertGate{limit, slope, shift};
   a.groups = GroupedRows{order, tiles, tiles + max_tiles, tiles + 2 * max_tiles, n_tiles, max_tiles, row_div};
-  return mode == GATED ? launch<GATED>(a, stream) : mode == SQUARED ? launch<SQUARED>(a, stream) : launch<PLAIN>(a, stream);
+  const int grid = max_tiles * a.n_panels;
+  return mode == GATED ? launch<expert_panel_kernel<GATED>>(a, grid, stream) : mode == SQUARED ? launch<expert_panel_kernel<SQUARED>>(a, grid, stream) : launch<expert_panel_kernel<PLAIN>>(a, grid, stream);
+}
+
+// Wp: one packed matrix [N, K]; epi 0: bf16 y[M, N], 2: the gated y[M, N / 2] with silu, 4: with gelu (tanh form), 5: max(y, 0)^2 [M, N].  The first
+// `panels` of the ceil(N / 256) panels are cut into tiles of `height` rows, those behind them of `height_behind` (multiples of 32 up to 256).  row_ss
+// (or null): fp32 [M][ss_parts] whose sums over K are the rows' mean squares; products are divided by the root of that.
+// N % 32 == 0, K % 64 == 0, rows of x and y of whole 16-byte pieces that start at such; 256 rows of x must lie within 2 GiB.
+int kv_dense_panels(const void* Wp, const void* x, void* y, int M, int N, int K, long long ldx, long long ldy, int epi, int height, int panels, int height_behind, const float* row_ss, int ss_parts, float eps,
+                    hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || (N & 31) || (K & 63) || K > (1 << 21) || (ldx & 7) || (ldy & 7) || ldx < K || ldx >= (1 << 22) || ((uintptr_t)x & 15) || ((uintptr_t)y & 15)) return -1;
+  const int all = (N + FEATURES - 1) / FEATURES;
+  for (int h : {height, height_behind})
+    if (h <= 0 || h > ROWS || (h & 31)) return -1;
+  if (panels < 0 || panels > all) return -1;
+  DenseArgs a;
+  a.w = (const unsigned char*)Wp; a.x = (const __bf16*)x; a.y = (unsigned short*)y;
+  a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldy = ldy;
+  a.height[0] = height; a.height[1] = height_behind;
+  a.tiles[0] = (M + height - 1) / height; a.tiles[1] = (M + height_behind - 1) / height_behind;
+  a.panels = panels;
+  a.row_ss = row_ss; a.ss_parts = ss_parts; a.inv_k = 1.f / (float)K; a.eps = eps; a.gelu = epi == 4;
+  const long long grid = (long long)panels * a.tiles[0] + (long long)(all - panels) * a.tiles[1];
+  if (grid > 0x7fffffffll) return -1;
+  switch (epi) {
+    case 0: return launch<dense_panel_kernel<PLAIN>>(a, (int)grid, stream);
+    case 2: case 4: return launch<dense_panel_kernel<GATED>>(a, (int)grid, stream);
+    case 5: return launch<dense_panel_kernel<SQUARED>>(a, (int)grid, stream);
+  }
+  return -1;
 }
 
 }  // extern "C"

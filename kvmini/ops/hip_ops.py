@@ -301,12 +301,11 @@ def _plan_slabs(n_pad: int, k: int, m: int = 32, group_cols: int = 256) -> Tuple
 
 
 # Tiled (wide) GEMM: (token tile, feature tile, pipeline variant) -> measured microseconds per
-# 64-wide K step of one workgroup with every CU busy (Llama-3-8B shapes, 1 x MI355X).  Per FLOP
-# 256 x 256 and 256 x 128 are alike (~1.28 PFLOP/s with every CU busy); the smaller tiles trade
-# efficiency for more workgroups; 256 x 224 and 256 x 192 exist for feature counts whose
-# 256-wide tiles leave a ragged last round over the 256 CUs (28672 = 128 x 224: 1024 tiles at
-# 2048 rows instead of 896; 6144 = 32 x 192: 256 tiles instead of 192).
-_WIDE_TILES_BF16 = (((256, 256, 1), 1.68), ((256, 224, 1), 1.615), ((256, 192, 0), 1.36), ((256, 128, 0), 0.84), ((128, 256, 0), 0.87), ((128, 128, 0), 0.62), ((256, 64, 0), 0.65))
+# 64-wide K step of one workgroup with every CU busy (Llama-3-8B shapes, 1 x MI355X).  The smaller
+# tiles trade efficiency for more workgroups; 256 x 224 and 256 x 192 (FP8 weights) exist for feature
+# counts whose 256-wide tiles leave a ragged last round over the 256 CUs.  bf16 weights come here
+# only with few outputs (_plan_panels).
+_WIDE_TILES_BF16 = (((256, 128, 0), 0.84), ((128, 256, 0), 0.87), ((128, 128, 0), 0.62), ((256, 64, 0), 0.65))
 _WIDE_TILES_FP8 = (((256, 256, 0), 1.9), ((256, 224, 0), 1.85), ((256, 192, 0), 1.55), ((256, 128, 0), 0.84), ((128, 256, 0), 0.87), ((128, 128, 0), 0.62))
 # The 128-wide tiles move 1.5 x the operand bytes per MAC of the 256-wide ones from L2 into LDS; on
 # grids of many rounds that traffic shows: + this many microseconds per step and round
@@ -369,6 +368,43 @@ def _plan_wide(m: int, n_pad: int, k: int, fp8: int, may_split: bool) -> Tuple[i
     return best[1]
 
 
+PANEL_HEIGHTS = (256, 224, 192, 160, 128, 96)  # rows of a tile (64 and 32: the panels' weights are then read more often than they are multiplied)
+
+
+@functools.lru_cache(maxsize=None)
+def _plan_panels(m: int, n: int, k: int) -> Optional[Tuple[int, int, int]]:
+    """How bf16 weights of many outputs are multiplied by panels of 256 features (``csrc/panel_gemm.hip``): (rows of a tile,
+    panels cut like that, rows of the tiles of the panels behind them), or None for the tiled GEMM above.
+
+    None up to one round of 128 x 128 tiles: there what counts is that all CUs have work, and a panel's tile is at least twice as wide
+    (measured on MI355X, us, this tiled GEMM and panels: 2048 rows x 2048 x 8192 77 and 89, 512 x 6144 x 4096 41 and 45, 256 x 4096 x 4096
+    40 and 45; beyond, 144 x 28672 x 4096 74 and 59, 1024 x 9216 x 4096 81 and 65, 2048 x 4096 x 14336 196 and 190, 2048 x 28672 x 4096 416 and 373).
+
+    The heights are those of the least modelled time: rounds over the CUs, each 8 us outside the K loop and 0.1 + 0.005 us per row in each
+    64 columns, less what CUs that stay empty in a last round leave to the others in power and bandwidth (0.7 of their share).  Fitted on ten
+    matrices at 144 to 4096 rows (5 % standard deviation); what it picks is within 1 % of the best height on all but one.  Two heights were 0.99
+    to 1.12 times as fast as the best single one, 1.035 in the mean over 16 sizes (2048 x 28672 x 4096: 372 -> 358 us); with 96 rows behind
+    whole rounds it was 0.97 over six others, so that is left out."""
+    cus = _num_cus()
+    if -(-m // 128) * -(-n // 128) <= cus:
+        return None
+    panels = -(-n // 256)
+
+    def time(count: int, height: int) -> float:
+        tiles = count * -(-m // height)
+        rounds, last = -(-tiles // cus), tiles % cus
+        empty = 1.0 - last / cus if last else 0.0
+        return rounds * (8.0 + k / 64 * (0.1 + 0.005 * height)) - k / 64 * 0.7 * empty * height / 256
+
+    best = min((time(panels, h), (h, panels, h)) for h in PANEL_HEIGHTS)
+    for h in PANEL_HEIGHTS:  # whole rounds of one height, the panels left over of another
+        per = -(-m // h)
+        whole = panels * per // cus * cus // per
+        if 0 < whole < panels:
+            best = min(best, min((time(whole, h) + time(panels - whole, rest), (h, whole, rest)) for rest in PANEL_HEIGHTS[:-1] if rest != h))
+    return best[1]
+
+
 def _wide(w: Union[PackedLinear, "_ExpandedView"], h: Union[torch.Tensor, "Normed"], epi: int, allow_slabs: bool) -> Union[torch.Tensor, "Partial"]:
     """More than 128 token rows: the tiled MFMA kernel on the packed weights."""
     C = native()
@@ -391,6 +427,12 @@ def _wide(w: Union[PackedLinear, "_ExpandedView"], h: Union[torch.Tensor, "Norme
         C.wide_gemm_fp8a(w.wp, w.n_pad, w.k, x8, a_scale, out, epi, bm, bn, variant, 1, sps, ss, eps, w.wscale, True)
         n_true = w.n // 2 if epi in GATED else w.n
         return out if n_true == n_out else out[:, :n_true]
+    cut = _plan_panels(m, w.n_pad, w.k) if w.wscale is None and x.data_ptr() % 16 == 0 and w.k <= x.stride(0) < 1 << 22 else None
+    if cut is not None:
+        out = torch.empty((m, w.n_pad // 2 if epi in GATED else w.n_pad), dtype=torch.bfloat16, device=x.device)
+        C.dense_panels(w.wp, w.n_pad, w.k, x, out, epi, *cut, ss, eps)
+        n_true = w.n // 2 if epi in GATED else w.n
+        return out if n_true == out.shape[1] else out[:, :n_true]
     bm, bn, variant, splits, sps = _plan_wide(m, w.n_pad, w.k, int(w.wscale is not None), may_split)
     if splits > 1:
         out = torch.empty((splits, m, w.n_pad), dtype=torch.float32, device=x.device)

@@ -1290,6 +1290,56 @@ def test_tiled_gemm_every_tile_and_pipeline_shape(C, tile, variant):
     assert (sl.sum(0) - ref).abs().max().item() <= 1e-4 * ref.abs().max().item()
 
 
+@pytest.mark.parametrize("M,N,K,cut", [
+    (1, 32, 64, (32, 1, 32)), (129, 96, 64, (256, 0, 96)), (255, 256, 128, (256, 1, 256)), (300, 544, 192, (64, 2, 224)), (257, 448, 320, (160, 1, 32)),
+    (1000, 288, 384, (192, 2, 256)), (513, 1024, 448, (128, 3, 96)), (448, 512, 832, (224, 1, 192)),
+])
+def test_dense_panels_of_every_height(C, M, N, K, cut):
+    """Panels of 256 features by tiles of 32 to 256 rows: ragged last tiles and panels, all counts of stages modulo those in flight, two heights in a
+    call, rows at a stride, each epilogue with and without the row scale.  Rounding to bf16 is within 2^-9 of the value (2^-8 with the
+    gates' exponential); the fp32 sums, K <= 832 of them in some 30 steps of 32 products each, within 2^-20 of the sum of magnitudes."""
+    torch.manual_seed(M)
+    x = torch.randn(M, K + 16, device="cuda").bfloat16()[:, 8 : 8 + K]
+    W = (torch.randn(N, K, device="cuda") * 0.1).bfloat16()
+    wp = C.pack_weight(W)
+    ss = torch.rand(M, 3, device="cuda") * K
+    scale = torch.rsqrt(ss.double().sum(1, keepdim=True) / K + 1e-5)
+    y, size = x.double() @ W.double().T, x.double().abs() @ W.double().abs().T
+    for rows in (None, ss):
+        by = scale if rows is not None else torch.ones_like(scale)
+        v, e = y * by, size * by * 2.0**-20
+        g, u, ge, ue = v.view(M, -1, 2, 8)[:, :, 0].flatten(1), v.view(M, -1, 2, 8)[:, :, 1].flatten(1), e.view(M, -1, 2, 8)[:, :, 0].flatten(1), e.view(M, -1, 2, 8)[:, :, 1].flatten(1)
+        silu, gelu, relu = torch.nn.functional.silu(g), torch.nn.functional.gelu(g, approximate="tanh"), v.clamp(min=0)
+        for epi, want, err in ((0, v, e), (2, silu * u, 1.2 * ge * u.abs() + silu.abs() * ue), (4, gelu * u, 1.2 * ge * u.abs() + gelu.abs() * ue), (5, relu**2, 2 * relu * e + e * e)):
+            out = torch.full((M + 1, want.shape[1]), 7.0, device="cuda", dtype=torch.bfloat16)
+            C.dense_panels(wp, N, K, x, out[:M], epi, *cut, rows, 1e-5)
+            assert ((out[:M].double() - want).abs() <= 2.0**-8 * want.abs() + err + 1e-30).all(), (epi, rows is not None)
+            assert (out[M] == 7).all()
+
+
+def test_matrices_of_many_outputs_go_by_panels():
+    """The op layer's rule: up to one round of 128 x 128 tiles the tiled kernel, beyond it panels whose cut covers all of them; the same rows either way."""
+    from kvmini.ops import hip_ops as ops
+
+    cus = ops._num_cus()
+    assert ops._plan_panels(128, 128 * cus, 256) is None
+    for m, n, k in ((129, 128 * cus, 256), (2048, 28672, 4096), (1500, 23040, 4096), (2048, 4096, 14336)):
+        height, panels, behind = ops._plan_panels(m, n, k)
+        assert height in ops.PANEL_HEIGHTS and behind in ops.PANEL_HEIGHTS and 0 < panels <= -(-n // 256)
+    torch.manual_seed(1)
+    n, k = 128 * cus + 64, 256
+    x = torch.randn(200, k, device="cuda").bfloat16()
+    w = (torch.randn(n, k, device="cuda") * 0.1).bfloat16()
+    pw = ops.PackedLinear(w)
+    assert ops._plan_panels(200, n, k) is not None
+    ref = x.double() @ w.double().T
+    wide = torch.cat((x, x), 1)[:, :k]  # (rows at a stride)
+    for rows in (x, wide):
+        got = ops.linear(rows, pw)
+        assert got.shape == (200, n)
+        assert ((got.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2.0**-20 * (x.double().abs() @ w.double().abs().T)).all()
+
+
 @pytest.mark.parametrize("bn,variant", [(224, 0), (224, 1), (224, 3), (192, 0), (192, 1), (192, 3)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_tiled_gemm_224_and_192_feature_tiles(C, bn, variant, fp8):
