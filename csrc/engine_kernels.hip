@@ -1922,13 +1922,32 @@ __global__ __launch_bounds__(256) void prefill_split_combine_kernel(const float*
 // the cache by later steps (rounded to e4m3, in stored units), so this kernel and the two-kernel
 // path agree.
 //
-// SPLIT (long contexts on small grids): gridDim.z workgroups share one (token, kv head); each walks
-// a contiguous range of the sequence's KV blocks (at least SPLIT_MIN_BLOCKS each: short contexts
-// use fewer workgroups, the rest exit at once), leaves its partial (max, sum, unnormalised output)
+// SPLIT (long contexts on small grids): several workgroups (at most n_z) share one (token, kv head); each walks
+// a contiguous range of the sequence's KV blocks, leaves its partial (max, sum, unnormalised output)
 // in a workspace, and the last one to arrive merges them — a 128k-token sequence decoded alone is
 // then streamed by up to 32 x nkv workgroups instead of nkv.  Every workgroup repeats phase A
 // (a few KB of slabs); only split 0 writes the cache and folds in the token's own key / value.
+// A range is at least the launch's blocks divided by the workgroups that are resident at once, and at least SPLIT_MIN_BLOCKS: a workgroup
+// costs some 10 us besides its blocks, so a second round of them, or short ranges, cost more than they spread.  The grid
+// holds the workgroups that can have work, not all (token, share) pairs: an idle one holds a CU's registers for a microsecond.
+// Measured, 16 rows of 8 kv heads and 4 heads each, ranges of 16 blocks from a grid of 32 shares per pair -> these: 16 x 4096 tokens 174 -> 59 us (e4m3 163 -> 38),
+// 16 x 1024 46 -> 23, 4 x 16384 82 -> 60, 2 x 32768 (14 rows of padding) 68 -> 59, 1 x 2000 15.6 -> 14.1, 1 x 100 10.8 -> 11.3.
 constexpr int SPLIT_MIN_BLOCKS = 16;
+constexpr int SPLIT_WAVES = 2048;  // 256 CUs of 8 waves with up to 256 registers
+// running sum over the lanes
+__device__ inline int wave_running_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // from 1, 2, 4, 8 lanes in front in the row
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, true);  // from the end of the row in front, of the half in front
+  return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, true);
+}
+// workgroups per kv head: each row has one, and what the ranges allow in addition fits the resident waves
+inline dim3 split_grid(int n_z, int n_rows, int nkv, int waves) {
+  const long long a = (long long)n_z * n_rows, b = SPLIT_WAVES / ((long long)waves * nkv) + n_rows;
+  return dim3((unsigned)(a < b ? a : b), nkv);
+}
 
 // all-reduce over the four lane quarters (lanes l, l ^ 16, l ^ 32, l ^ 48) with the two gfx950 row / half swaps
 __device__ inline float quarters_max(float v) {
@@ -1962,7 +1981,7 @@ __device__ inline float quarters_sum(float v) {
 // matrix form would need the block transposed).  With an e4m3 cache this halves the vector work per block, which
 // is what bounds that kernel (the bf16 cache is bound by the KV stream already).
 template <int REP, int NWAVE, bool KV8, bool SPLIT, bool ATTN = false, bool MF = false>
-__device__ __forceinline__ void decode_attention_body(const int bx, const int by, const int bz, const int gdx, const float* __restrict__ slabs, int n_slabs, long long slab_stride,
+__device__ __forceinline__ void decode_attention_body(const int bx, const int by, const int n_z, const int n_rows, const float* __restrict__ slabs, int n_slabs, long long slab_stride,
                                                                      const int* __restrict__ positions, const float* __restrict__ cos_t,
                                                                      const float* __restrict__ sin_t, void* __restrict__ k_cache,
                                                                      void* __restrict__ v_cache, const int* __restrict__ slot_mapping,
@@ -1991,22 +2010,44 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   __shared__ float p_lds[NWAVE][REP][BS];
   __shared__ float m_lds[NWAVE][REP], l_lds[NWAVE][REP];
   __shared__ float o_lds[NWAVE][4][REP][HD];  // [wave][token group]: partial outputs, summed in the merge
-  // SPLIT: grid = (splits, kv heads, tokens) — consecutive workgroup ids (which the dispatcher
-  // deals round-robin to the 8 XCDs) are the splits of one pair, so that a lone long sequence
-  // is streamed by every XCD; with the token index fastest, a 16-row step whose only live row
-  // is row 0 would put all its workgroups on one XCD.
-  const int t = ATTN ? row_list[bz] : SPLIT ? bz : bx, g = by;
-  const int n_z = SPLIT ? gdx : 1;
-  if constexpr (ATTN) {
-    if (t < 0) return;
-  }
   // wave index in a scalar register: block-table reads become scalar loads (see paged_attention_kernel)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int ctx = ctx_lens[t];
+  const int g = by;
+  int t = bx, listed = bx, z = 0, eff = 1, ctx;
+  if constexpr (SPLIT) {
+    // Which (row, share of its blocks) is workgroup bx of this kv head's?  Every wave reads all lengths, the shares follow from them.
+    auto length = [&](int i) __attribute__((always_inline)) {  // (-1: not in use)
+      const int r = i >= n_rows ? -1 : ATTN ? row_list[i] : i;
+      return r < 0 ? -1 : ctx_lens[r];
+    };
+    auto blocks = [&](int c) __attribute__((always_inline)) { return c > !ATTN ? (c - !ATTN + BS - 1) / BS : 0; };
+    const int c0 = length(lane);
+    int total = blocks(c0);
+    for (int i = lane + 64; i < n_rows; i += 64) total += blocks(length(i));
+    total = __builtin_amdgcn_readlane(wave_running_sum(total), 63);
+    const int fair = (int)(((long long)total * nkv * NWAVE + SPLIT_WAVES - 1) / SPLIT_WAVES), share = max(fair, SPLIT_MIN_BLOCKS);
+    const int up = fair < SPLIT_MIN_BLOCKS ? SPLIT_MIN_BLOCKS - 1 : 0;  // (rounded up where all of them are resident all the same)
+    int left = bx, base = 0;
+    for (;; base += 64) {
+      if (base >= n_rows) return;
+      const int c = base ? length(base + lane) : c0, e = c < 0 ? 0 : max(1, min(n_z, (blocks(c) + up) / share));
+      const int sum = wave_running_sum(e);
+      const unsigned long long past = __builtin_amdgcn_ballot_w64(sum > left);
+      if (past != 0) {
+        const int l = __builtin_ctzll(past);
+        listed = base + l;
+        ctx = __builtin_amdgcn_readlane(c, l);
+        eff = __builtin_amdgcn_readlane(e, l);
+        z = left - (__builtin_amdgcn_readlane(sum, l) - eff);
+        break;
+      }
+      left -= __builtin_amdgcn_readlane(sum, 63);
+    }
+    t = ATTN ? row_list[listed] : listed;
+  } else {
+    ctx = ctx_lens[t];
+  }
   unsigned short* orow = out + (long long)t * nh * HD + (long long)g * REP * HD;
-  // the split index is rotated by the pair index: when short contexts leave only split 0 at work,
-  // the working workgroups of consecutive pairs still sit on different XCDs
-  const int z = SPLIT ? (int)((bx + (unsigned)(t * nkv + g)) % (unsigned)n_z) : 0;
   if (ctx <= 0) {  // padding token: no KV write (slot -1), zero output
     if (z == 0)
       for (int i = tid; i < REP * HD; i += NT) orow[i] = 0;
@@ -2017,11 +2058,8 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   const int prev = ATTN ? ctx : ctx - 1;
   const int* bt = block_tables + (long long)tok_seq[t] * max_blocks_per_seq;
   const int all_blocks = (prev + BS - 1) / BS;
-  int eff = 1, b0 = 0, n_blocks = all_blocks;  // this workgroup walks blocks [b0, n_blocks)
+  int b0 = 0, n_blocks = all_blocks;  // this workgroup walks blocks [b0, n_blocks)
   if constexpr (SPLIT) {
-    eff = (all_blocks + SPLIT_MIN_BLOCKS - 1) / SPLIT_MIN_BLOCKS;
-    eff = eff < 1 ? 1 : (eff > n_z ? n_z : eff);
-    if (z >= eff) return;
     const int per = (all_blocks + eff - 1) / eff;
     b0 = z * per;
     n_blocks = b0 + per < all_blocks ? b0 + per : all_blocks;
@@ -2319,7 +2357,7 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   }
   __syncthreads();
   const bool direct = !SPLIT || eff == 1;
-  const int wt = ATTN ? bz : t;  // workspace entries go by grid row (listed rows may be any token rows of a wide step)
+  const int wt = listed;  // workspace entries go by grid row (listed rows may be any token rows of a wide step)
   const long long pbase = SPLIT ? ((long long)(wt * nkv + g) * n_z) : 0;  // this (token, kv head)'s first partial
   for (int i = tid; i < REP * HD; i += NT) {
     const int h = i / HD, d = i % HD;
@@ -2412,7 +2450,7 @@ __global__ __launch_bounds__(64 * NWAVE) void decode_attention_fused_kernel(cons
                                                                      const float* __restrict__ row_ss, int ss_parts, float inv_h, float eps,
                                                                      float scale_log2e, const float* __restrict__ kv_scale,
                                                                      float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ counters,
-                                                                     PrefetchPlan pf, const unsigned short* __restrict__ q_in = nullptr,
+                                                                     PrefetchPlan pf, int n_z, int n_rows, const unsigned short* __restrict__ q_in = nullptr,
                                                                      long long q_row_stride = 0, const int* __restrict__ row_list = nullptr) {
   if constexpr (!SPLIT) {
     // grid rows past the kv heads: weight prefetch for the output projection (see prefetch_role).
@@ -2424,7 +2462,7 @@ __global__ __launch_bounds__(64 * NWAVE) void decode_attention_fused_kernel(cons
       return;
     }
   }
-  decode_attention_body<REP, NWAVE, KV8, SPLIT, ATTN, MF>((int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.x, slabs, n_slabs, slab_stride, positions, cos_t, sin_t,
+  decode_attention_body<REP, NWAVE, KV8, SPLIT, ATTN, MF>((int)blockIdx.x, (int)blockIdx.y, n_z, n_rows, slabs, n_slabs, slab_stride, positions, cos_t, sin_t,
                                                       k_cache, v_cache, slot_mapping, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, out, nh, nkv, row_ss,
                                                       ss_parts, inv_h, eps, scale_log2e, kv_scale, part_o, part_ml, counters, q_in, q_row_stride, row_list);
 }
@@ -2862,7 +2900,7 @@ __global__ __launch_bounds__(512) void decode_layers_kernel(const DlParams p) {
       const float* kvs = KV8 ? p.kv_scale + (long long)li * p.kv_scale_stride : nullptr;
       const int n_items = T * p.nkv;
       for (int item = wg; item < n_items; item += G) {
-        decode_attention_body<REP, 8, KV8, false, false>(item / p.nkv, item % p.nkv, 0, 1, p.qkv_slabs, p.qkv.splits, (long long)T * qkv_w, p.positions, p.cos_t, p.sin_t,
+        decode_attention_body<REP, 8, KV8, false, false>(item / p.nkv, item % p.nkv, 1, T, p.qkv_slabs, p.qkv.splits, (long long)T * qkv_w, p.positions, p.cos_t, p.sin_t,
                                                          L.k_cache, L.v_cache, p.slot_mapping, p.block_tables, p.max_blocks_per_seq, p.tok_seq, p.ctx_lens,
                                                          p.attn_out, p.nh, p.nkv, ssin, parts, inv_h, p.eps, p.scale_log2e, kvs, nullptr, nullptr, nullptr, nullptr,
                                                          0, nullptr);
@@ -3196,7 +3234,7 @@ int kv_decode_attention_fused(const float* slabs, int n_slabs, long long slab_st
   dim3 grid(T, nkv), block(64 * waves);
   PrefetchPlan plan{};
   if (n_split > 1) {
-    grid = dim3(n_split, nkv, T);  // splits fastest: see the kernel
+    grid = split_grid(n_split, T, nkv, waves);
   } else if (pf_base != nullptr && pf != nullptr) {  // (long-context steps are bound by the KV stream themselves: no prefetch beside the split variant)
     if (make_prefetch_plan(pf_base, pf, pf_sink, &plan) != 0) return -1;
     grid.y += (plan.wgs + T - 1) / T;
@@ -3204,11 +3242,11 @@ int kv_decode_attention_fused(const float* slabs, int n_slabs, long long slab_st
 #define KV_LAUNCH_S(R, W, K8, SP)                                                                                                                        \
   hipLaunchKernelGGL((decode_attention_fused_kernel<R, W, K8, SP>), grid, block, 0, stream, slabs, n_slabs, slab_stride, positions, cos_t, sin_t, k_cache, \
                      v_cache, slot_mapping, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, (unsigned short*)out, nh, nkv, row_ss, ss_parts,        \
-                     inv_h, eps, sl, kv_scale, part_o, part_ml, counters, plan)
+                     inv_h, eps, sl, kv_scale, part_o, part_ml, counters, plan, n_split, T)
 #define KV_LAUNCH_MF(R, W, K8)                                                                                                                            \
   hipLaunchKernelGGL((decode_attention_fused_kernel<R, W, K8, true, false, true>), grid, block, 0, stream, slabs, n_slabs, slab_stride, positions, cos_t, sin_t, \
                      k_cache, v_cache, slot_mapping, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, (unsigned short*)out, nh, nkv, row_ss, ss_parts,      \
-                     inv_h, eps, sl, kv_scale, part_o, part_ml, counters, plan)
+                     inv_h, eps, sl, kv_scale, part_o, part_ml, counters, plan, n_split, T)
 #define KV_LAUNCH_K(R, W, K8)       \
   if (n_split > 1) {                \
     KV_LAUNCH_S(R, W, K8, true);    \
@@ -3218,7 +3256,7 @@ int kv_decode_attention_fused(const float* slabs, int n_slabs, long long slab_st
 #define KV_LAUNCH_MF1(R, W, K8)                                                                                                                           \
   hipLaunchKernelGGL((decode_attention_fused_kernel<R, W, K8, false, false, true>), grid, block, 0, stream, slabs, n_slabs, slab_stride, positions, cos_t, sin_t, \
                      k_cache, v_cache, slot_mapping, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, (unsigned short*)out, nh, nkv, row_ss, ss_parts,      \
-                     inv_h, eps, sl, kv_scale, part_o, part_ml, counters, plan)
+                     inv_h, eps, sl, kv_scale, part_o, part_ml, counters, plan, n_split, T)
 #define KV_LAUNCH_KM(R, W, K8)                        \
   if (n_split > 1 && g_attention_mfma) {              \
     KV_LAUNCH_MF(R, W, K8);                           \
@@ -3285,18 +3323,18 @@ int kv_split_decode_attention(const void* q, long long q_row_stride, const void*
   const int rep = nh / nkv;
   const float sl = scale * 1.4426950408889634f;
   if (rep > 4) waves = 4;
-  const dim3 grid(n_split, nkv, n_rows), block(64 * waves);
+  const dim3 grid = split_grid(n_split, n_rows, nkv, waves), block(64 * waves);
   const PrefetchPlan plan{};
 #define KV_LAUNCH_S(R, W, K8)                                                                                                                                  \
   hipLaunchKernelGGL((decode_attention_fused_kernel<R, W, K8, true, true>), grid, block, 0, stream, (const float*)nullptr, 0, 0LL, (const int*)nullptr,        \
                      (const float*)nullptr, (const float*)nullptr, const_cast<void*>(k_cache), const_cast<void*>(v_cache), (const int*)nullptr, block_tables, \
                      max_blocks_per_seq, tok_seq, ctx_lens, (unsigned short*)out, nh, nkv, (const float*)nullptr, 0, 0.f, 0.f, sl, kv_scale, part_o, part_ml,   \
-                     counters, plan, (const unsigned short*)q, q_row_stride, row_list)
+                     counters, plan, n_split, n_rows, (const unsigned short*)q, q_row_stride, row_list)
 #define KV_LAUNCH_MF(R, W, K8)                                                                                                                                 \
   hipLaunchKernelGGL((decode_attention_fused_kernel<R, W, K8, true, true, true>), grid, block, 0, stream, (const float*)nullptr, 0, 0LL, (const int*)nullptr,  \
                      (const float*)nullptr, (const float*)nullptr, const_cast<void*>(k_cache), const_cast<void*>(v_cache), (const int*)nullptr, block_tables, \
                      max_blocks_per_seq, tok_seq, ctx_lens, (unsigned short*)out, nh, nkv, (const float*)nullptr, 0, 0.f, 0.f, sl, kv_scale, part_o, part_ml,   \
-                     counters, plan, (const unsigned short*)q, q_row_stride, row_list)
+                     counters, plan, n_split, n_rows, (const unsigned short*)q, q_row_stride, row_list)
 #define KV_LAUNCH_X(R, W, K8)                             \
   if (g_attention_mfma) { KV_LAUNCH_MF(R, W, K8); }       \
   else { KV_LAUNCH_S(R, W, K8); }

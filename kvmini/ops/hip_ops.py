@@ -966,17 +966,14 @@ _split_ws: Dict[Any, torch.Tensor] = {}
 
 
 def decode_attention_splits(tokens: int, n_kv_heads: int) -> int:
-    """Workgroups per (token, kv head) for a decode step of ``tokens`` rows (padding rows count:
-    they are part of the captured grid and exit at once)."""
+    """Workgroups per (token, kv head), at most, for a decode step of ``tokens`` rows (padding rows
+    count).  How many of them a row gets the kernel finds from the lengths of all rows."""
     forced = int(os.environ.get("KVMINI_DECODE_SPLITS", "0"))
     if forced > 0:
         return forced
     pairs = tokens * n_kv_heads
     if pairs > SPLIT_KV_MAX_PAIRS:
         return 1
-    # (16 workgroups per CU's worth of pairs: the rows of a 16-row bucket that are padding, or short, leave at once,
-    # and a lone 128k-token sequence in such a step is then streamed by 256 workgroups instead of 128:
-    # 4.83 against 5.91 ms per step with the e4m3 cache, 6.09 against 6.50 with bf16)
     return max(1, min(SPLIT_KV_MAX, 16 * _num_cus() // pairs))
 
 

@@ -1860,6 +1860,36 @@ def test_split_kv_decode_attention_matches_the_unsplit_kernel(rep, kv8):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,longest", [(1, 4000), (63, 300), (64, 1100), (65, 1100), (127, 1500)])
+def test_split_kv_shares_cover_every_row_once(rows, longest):
+    """Ranges of the launch's fair share and of the least one, rows on both sides of a wave's width, padding rows in between: each row's blocks are
+    walked exactly once and each token is written, as by one workgroup per pair (both round the same sums to bf16: within two roundings, 2^-7 of the
+    largest value)."""
+    from kvmini.models.llama import LlamaConfig, rope_tables
+    from kvmini.ops import hip_ops
+
+    torch.manual_seed(rows)
+    dev, nkv, rep, hd, bs = _dev(), 1, 4, 128, 16
+    ctx = torch.tensor([longest - (131 * i) % (longest - 5) if i % 5 != 3 else 0 for i in range(rows)], device=dev, dtype=torch.int32)
+    per = -(-longest // bs)
+    cos, sin = rope_tables(LlamaConfig(head_dim=hd), longest, dev)
+    pos = (ctx - 1).clamp(min=0)
+    bt = torch.randperm(rows * per, device=dev).view(rows, per).int()
+    slots = torch.where(ctx > 0, bt[torch.arange(rows, device=dev), (pos // bs).long()] * bs + pos % bs, -1).int()
+    part = hip_ops.Partial(torch.randn(2, rows, (rep + 2) * hd, device=dev) * 0.4, torch.rand(rows, 1, device=dev) * 512 + 1.0, 1e-5, 512)
+    k, v = (torch.randn(rows * per, nkv, bs, hd, device=dev).bfloat16() for _ in range(2))
+    seq = torch.arange(rows, device=dev, dtype=torch.int32)
+    got = []
+    for n_split in (1, 5, 32):
+        kc, vc = k.clone(), v.clone()
+        got.append((hip_ops.rope_attention_fused(part, pos, cos, sin, kc, vc, slots, bt, seq, ctx, rep, hd**-0.5, n_split=n_split), kc, vc))
+    for out, kc, vc in got[1:]:
+        assert torch.equal(kc, got[0][1]) and torch.equal(vc, got[0][2])
+        assert (out.float() - got[0][0].float()).abs().max() <= 2.0**-7 * got[0][0].float().abs().max()
+        assert not out[ctx == 0].any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kv", ["auto", "fp8"])
 def test_engine_long_context_decode_takes_the_split_kv_graph_and_matches_eager(kv):
     """A 3000-token sequence decoded alone: the engine replays the split-KV variant of the
