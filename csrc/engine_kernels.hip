@@ -224,6 +224,27 @@ struct PAStage {
 };
 template <>
 struct PAStage<128, true> : KVStage<true> {};
+// what a wave of the fused decode kernel holds of a block: 16-byte pieces, a key over four lanes, a value row over HD / 8
+template <bool KV8, int HD>
+struct KVStageOf {
+  struct type {
+    static constexpr int NP = HD / 32;
+    bf16x8 k[NP], v[NP];
+    __device__ inline void load(const void* k_cache, const void* v_cache, long long blk, int key, int chunk, int tg, int dv) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) k[i] = kv_load8<KV8>(k_cache, blk + key * HD + chunk * (HD / 4) + i * 8);
+#pragma unroll
+      for (int i = 0; i < NP; ++i) v[i] = kv_load8<KV8>(v_cache, blk + dv * 8 + (tg + 512 / HD * i) * HD);
+    }
+    __device__ inline void unpack(bf16x8 (&kk)[NP], bf16x8 (&vv)[NP], int dv) const {
+      (void)dv;
+#pragma unroll
+      for (int i = 0; i < NP; ++i) { kk[i] = k[i]; vv[i] = v[i]; }
+    }
+  };
+};
+template <bool KV8>
+struct KVStageOf<KV8, 128> { using type = KVStage<KV8>; };
 // 8 values -> e4m3 bytes of v * inv_scale, clamped to the format's range (+-448)
 __device__ inline uint2 fp8_pack8(bf16x8 v, float inv_scale) {
   float f[8];
@@ -1980,7 +2001,7 @@ __device__ inline float quarters_sum(float v) {
 // every lane by v_readlane.  P . V stays on the vector ALU in packed fp32 pairs (V rows are head-dim-major: the
 // matrix form would need the block transposed).  With an e4m3 cache this halves the vector work per block, which
 // is what bounds that kernel (the bf16 cache is bound by the KV stream already).
-template <int REP, int NWAVE, bool KV8, bool SPLIT, bool ATTN = false, bool MF = false>
+template <int REP, int NWAVE, bool KV8, bool SPLIT, bool ATTN = false, bool MF = false, int HD = 128>
 __device__ __forceinline__ void decode_attention_body(const int bx, const int by, const int n_z, const int n_rows, const float* __restrict__ slabs, int n_slabs, long long slab_stride,
                                                                      const int* __restrict__ positions, const float* __restrict__ cos_t,
                                                                      const float* __restrict__ sin_t, void* __restrict__ k_cache,
@@ -1993,7 +2014,12 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
                                                                      float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ counters,
                                                                      const unsigned short* __restrict__ q_in,
                                                                      long long q_row_stride, const int* __restrict__ row_list) {
-  constexpr int HD = 128, BS = 16, HALF = 64, NT = 64 * NWAVE;
+  static_assert(HD == 64 || (HD == 128), "head width");
+  static_assert(HD == 128 || !MF, "the matrix form is of heads of 128");
+  constexpr int BS = 16, HALF = HD / 2, NT = 64 * NWAVE;
+  constexpr int NP = HD / 32;      // 16-byte pieces of K and of V per lane and block
+  constexpr int DV = HD / 8;       // lanes that share a value row (8 dims each) ...
+  constexpr int TG = 64 / DV;      // ... and rows read at a time
   static_assert(!ATTN || SPLIT, "the attention-only form exists in the split layout");
   float inv_ks = 1.f, inv_vs = 1.f, v_scale = 1.f;
   if constexpr (KV8) {
@@ -2009,7 +2035,7 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   __shared__ __attribute__((aligned(16))) unsigned short xb_lds[REP + 1][HD];
   __shared__ float p_lds[NWAVE][REP][BS];
   __shared__ float m_lds[NWAVE][REP], l_lds[NWAVE][REP];
-  __shared__ float o_lds[NWAVE][4][REP][HD];  // [wave][token group]: partial outputs, summed in the merge
+  __shared__ float o_lds[NWAVE][TG][REP][HD];  // [wave][token group]: partial outputs, summed in the merge
   // wave index in a scalar register: block-table reads become scalar loads (see paged_attention_kernel)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = by;
@@ -2066,23 +2092,24 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   }
   static_assert(!MF || REP <= 16, "one head per lane column");
   const int qk_tok = MF ? (lane & 15) : (lane >> 2), qk_c = MF ? (lane >> 4) : (lane & 3);
-  const int pv_tg = lane >> 4, pv_dv = lane & 15;
-  KVStage<KV8> st_cur, st_nxt;  // this wave's first block and the one after: two blocks (16 KB of bf16) per wave in flight at any time
+  const int pv_tg = lane / DV, pv_dv = lane % DV;
+  using Stage = typename KVStageOf<KV8, HD>::type;
+  Stage st_cur, st_nxt;  // this wave's first block and the one after: two blocks (16 KB of bf16) per wave in flight at any time
   if (b0 + wave < n_blocks) st_cur.load(k_cache, v_cache, ((long long)bt[b0 + wave] * nkv + g) * BS * HD, qk_tok, qk_c, pv_tg, pv_dv);
   if (b0 + wave + NWAVE < n_blocks) st_nxt.load(k_cache, v_cache, ((long long)bt[b0 + wave + NWAVE] * nkv + g) * BS * HD, qk_tok, qk_c, pv_tg, pv_dv);
   if constexpr (ATTN) {
     for (int pc = tid; pc < REP * (HD / 8); pc += NT) {
-      const int h = pc >> 4, d0 = (pc & 15) << 3;
+      const int h = pc / DV, d0 = pc % DV * 8;
       *reinterpret_cast<bf16x8*>(&xb_lds[h][d0]) = *reinterpret_cast<const bf16x8*>(q_in + (long long)t * q_row_stride + (long long)(g * REP + h) * HD + d0);
     }
   } else {
   // likewise the RoPE table row of this token (needed in A.2)
-  constexpr int ROT = (REP + 1) * 8;  // (q heads + k) x 8 pieces of 8 dims and their partners
+  constexpr int RP = HALF / 8, ROT = (REP + 1) * RP;  // (q heads + k) x pieces of 8 dims and their partners
   const int pos = positions[t];
   const int slot = slot_mapping[t];
   f32x4 csr[2], snr[2];
   if (tid < ROT) {
-    const int d0 = (tid & 7) << 3;
+    const int d0 = tid % RP * 8;
     const f32x4* cp = reinterpret_cast<const f32x4*>(cos_t + (long long)pos * HALF + d0);
     const f32x4* sp = reinterpret_cast<const f32x4*>(sin_t + (long long)pos * HALF + d0);
     csr[0] = cp[0]; csr[1] = cp[1]; snr[0] = sp[0]; snr[1] = sp[1];
@@ -2095,10 +2122,10 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
     if (row_ss != nullptr) rs = rsqrtf(row_ss_total(row_ss + (long long)t * ss_parts, ss_parts, lane) * inv_h + eps);
     const int width = (nh + 2 * nkv) * HD;
     const float* row0 = slabs + (long long)t * width;
-    constexpr int PIECES = (REP + 2) * (HD / 4);  // q heads, then k, then v; 32 pieces per row
+    constexpr int PIECES = (REP + 2) * (HD / 4);  // q heads, then k, then v
     constexpr int MAX_S = 16;
     for (int pc = tid; pc < PIECES; pc += NT) {
-      const int r = pc >> 5, c4 = (pc & 31) << 2;
+      const int r = pc / (HD / 4), c4 = pc % (HD / 4) * 4;
       const int col = (r < REP ? (g * REP + r) * HD : r == REP ? (nh + g) * HD : (nh + nkv + g) * HD) + c4;
       f32x4 v[MAX_S];
 #pragma unroll
@@ -2116,11 +2143,11 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   // ---- phase A.2: RoPE on q and k (pairs d, d + 64), cache write of k and v
   {
     const long long cache_row = (slot >= 0 && z == 0) ? (((long long)(slot / BS) * nkv + g) * BS + slot % BS) * HD : -1;
-    static_assert(ROT + 16 <= 256, "one task per thread");
+    static_assert(ROT + DV <= 256, "one task per thread");
     {
       const int task = tid;
       if (task < ROT) {
-        const int hsel = task >> 3, d0 = (task & 7) << 3;
+        const int hsel = task / RP, d0 = task % RP * 8;
         bf16x8 oa, ob;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -2135,7 +2162,7 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
         }
         *reinterpret_cast<bf16x8*>(&xb_lds[hsel][d0]) = oa;
         *reinterpret_cast<bf16x8*>(&xb_lds[hsel][HALF + d0]) = ob;
-      } else if (task < ROT + 16 && (cache_row >= 0 || KV8)) {
+      } else if (task < ROT + DV && (cache_row >= 0 || KV8)) {
         const int d0 = (task - ROT) << 3;
         bf16x8 ov;
 #pragma unroll
@@ -2155,13 +2182,13 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   // v_dot2_f32_bf16: half the multiply instructions, no bf16 -> fp32 unpacking of K, and a
   // register footprint that lets 8 waves per workgroup (2 per SIMD) run without spilling
   const int tail_c = lane & 3;  // dim chunk of the lane in the quad layout (the token's own key below)
-  bf16x2 qp[REP][16];
+  bf16x2 qp[REP][HD / 8];
   auto load_qp = [&]() {
 #pragma unroll
     for (int h = 0; h < REP; ++h)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const bf16x2x4 qw = __builtin_bit_cast(bf16x2x4, *reinterpret_cast<const bf16x8*>(&xb_lds[h][tail_c * 32 + v * 8]));
+      for (int v = 0; v < NP; ++v) {
+        const bf16x2x4 qw = __builtin_bit_cast(bf16x2x4, *reinterpret_cast<const bf16x8*>(&xb_lds[h][tail_c * (HD / 4) + v * 8]));
 #pragma unroll
         for (int j = 0; j < 4; ++j) qp[h][v * 4 + j] = qw.p[j];
       }
@@ -2262,16 +2289,16 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   for (int b = b0 + wave; b < n_blocks; b += NWAVE) {
     // this block's K / V and the next one's are in registers or on their way (loaded before
     // phase A, or by earlier iterations); start the loads of the block after those
-    KVStage<KV8> st_far;
+    Stage st_far;
     if (b + 2 * NWAVE < n_blocks) st_far.load(k_cache, v_cache, ((long long)bt[b + 2 * NWAVE] * nkv + g) * BS * HD, qk_tok, qk_c, pv_tg, pv_dv);
-    bf16x8 kv[4], vv[4];
+    bf16x8 kv[NP], vv[NP];
     st_cur.unpack(kv, vv, pv_dv);
     float s[REP];
 #pragma unroll
     for (int h = 0; h < REP; ++h) {
       float d = 0.f;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
+      for (int v = 0; v < NP; ++v) {
         const bf16x2x4 kw = __builtin_bit_cast(bf16x2x4, kv[v]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) d = __builtin_amdgcn_fdot2_f32_bf16(qp[h][v * 4 + j], kw.p[j], d, false);
@@ -2304,8 +2331,8 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tok = pv_tg + 4 * i;
+    for (int i = 0; i < NP; ++i) {
+      const int tok = pv_tg + TG * i;
 #pragma unroll
       for (int h = 0; h < REP; ++h) {
         const float p = p_lds[wave][h][tok];
@@ -2320,10 +2347,10 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   // ---- the token's own key / value (wave 0 of split 0; one token group adds the value)
   if (!ATTN && wave == 0 && z == 0) {
     if constexpr (MF) load_qp();
-    bf16x2 kp2[16];
+    bf16x2 kp2[HD / 8];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const bf16x2x4 kw = __builtin_bit_cast(bf16x2x4, *reinterpret_cast<const bf16x8*>(&xb_lds[REP][tail_c * 32 + v * 8]));
+    for (int v = 0; v < NP; ++v) {
+      const bf16x2x4 kw = __builtin_bit_cast(bf16x2x4, *reinterpret_cast<const bf16x8*>(&xb_lds[REP][tail_c * (HD / 4) + v * 8]));
 #pragma unroll
       for (int j = 0; j < 4; ++j) kp2[v * 4 + j] = kw.p[j];
     }
@@ -2331,7 +2358,7 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
     for (int h = 0; h < REP; ++h) {
       float d = 0.f;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) d = __builtin_amdgcn_fdot2_f32_bf16(qp[h][j], kp2[j], d, false);
+      for (int j = 0; j < HD / 8; ++j) d = __builtin_amdgcn_fdot2_f32_bf16(qp[h][j], kp2[j], d, false);
       d += dpp_f32<0xB1>(d);
       d += dpp_f32<0x4E>(d);
       d *= scale_log2e;
@@ -2368,7 +2395,10 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
 #pragma unroll
     for (int w = 0; w < NWAVE; ++w) {
       const float c = __builtin_amdgcn_exp2f(m_lds[w][h] - m);
-      num += (o_lds[w][0][h][d] + o_lds[w][1][h][d] + o_lds[w][2][h][d] + o_lds[w][3][h][d]) * c;
+      float o = 0.f;
+#pragma unroll
+      for (int k = 0; k < TG; ++k) o += o_lds[w][k][h][d];
+      num += o * c;
       den += l_lds[w][h] * c;
     }
     if (direct) {
@@ -2439,7 +2469,7 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
 // The kernel: one workgroup per (token, kv head[, split]) of the launch grid; grid rows past the kv
 // heads of an unsplit launch are weight-prefetch workgroups (see prefetch_role).  The same body runs
 // as the attention phase of the persistent decode kernel below, one (token, kv head) at a time.
-template <int REP, int NWAVE, bool KV8, bool SPLIT, bool ATTN = false, bool MF = false>
+template <int REP, int NWAVE, bool KV8, bool SPLIT, bool ATTN = false, bool MF = false, int HD = 128>
 __global__ __launch_bounds__(64 * NWAVE) void decode_attention_fused_kernel(const float* __restrict__ slabs, int n_slabs, long long slab_stride,
                                                                      const int* __restrict__ positions, const float* __restrict__ cos_t,
                                                                      const float* __restrict__ sin_t, void* __restrict__ k_cache,
@@ -2462,7 +2492,7 @@ __global__ __launch_bounds__(64 * NWAVE) void decode_attention_fused_kernel(cons
       return;
     }
   }
-  decode_attention_body<REP, NWAVE, KV8, SPLIT, ATTN, MF>((int)blockIdx.x, (int)blockIdx.y, n_z, n_rows, slabs, n_slabs, slab_stride, positions, cos_t, sin_t,
+  decode_attention_body<REP, NWAVE, KV8, SPLIT, ATTN, MF, HD>((int)blockIdx.x, (int)blockIdx.y, n_z, n_rows, slabs, n_slabs, slab_stride, positions, cos_t, sin_t,
                                                       k_cache, v_cache, slot_mapping, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, out, nh, nkv, row_ss,
                                                       ss_parts, inv_h, eps, scale_log2e, kv_scale, part_o, part_ml, counters, q_in, q_row_stride, row_list);
 }
@@ -2513,13 +2543,39 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const unsigned short* __re
 // before it had read that id back), feed[i] = 0 selects tokens[i].  One workgroup per row,
 // 16 bytes per thread per trip; ids outside [0, V) read row 0.
 __global__ __launch_bounds__(256) void embed_fed_kernel(const unsigned short* __restrict__ table, const int* __restrict__ tokens, const int* __restrict__ feed,
-                                                        const long long* __restrict__ prev_ids, int n_prev, unsigned short* __restrict__ out, int H, int V) {
-  const int i = blockIdx.x;
+                                                        const long long* __restrict__ prev_ids, int n_prev, unsigned short* __restrict__ out, int H, int V, float* __restrict__ ss_part) {
+  const int i = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, parts = (H + 511) / 512;
   const int f = feed[i];
   long long tok = (f > 0 && f <= n_prev) ? prev_ids[f - 1] : (long long)tokens[i];
   if (tok < 0 || tok >= V) tok = 0;
   const bf16x8* src = reinterpret_cast<const bf16x8*>(table + tok * H);
   bf16x8* dst = reinterpret_cast<bf16x8*>(out + (long long)i * H);
+  // the first residual stream: with ss_part, the sums of squares of its segments of 512 columns, as residual_reduce_kernel takes them
+  for (int p = wave; p < parts; p += 4) {
+    const int c = p * 64 + lane;
+    float ss = 0.f;
+    if (c < (H >> 3)) {
+      const bf16x8 v = src[c];
+      dst[c] = v;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss += bf2f(v[j]) * bf2f(v[j]);
+    }
+    if (ss_part != nullptr) {
+      ss = wave_sum(ss);
+      if (lane == 0) ss_part[(long long)i * parts + p] = ss;
+    }
+  }
+}
+
+// rows idx[i] of x (bf16, H columns) and of its sums of squares (fp32, `parts`; none: null), in one launch.  One workgroup per row.
+__global__ __launch_bounds__(256) void select_rows_kernel(const unsigned short* __restrict__ x, long long ldx, const float* __restrict__ ss, int parts, const int* __restrict__ idx, int T,
+                                                          unsigned short* __restrict__ out, float* __restrict__ out_ss, int H) {
+  const int i = blockIdx.x, r = idx[i];
+  if (r < 0 || r >= T) return;
+  const bf16x8* src = reinterpret_cast<const bf16x8*>(x + r * ldx);
+  bf16x8* dst = reinterpret_cast<bf16x8*>(out + (long long)i * H);
+  if (ss != nullptr)
+    for (int p = threadIdx.x; p < parts; p += 256) out_ss[(long long)i * parts + p] = ss[(long long)r * parts + p];
   for (int c = threadIdx.x; c < (H >> 3); c += 256) dst[c] = src[c];
 }
 
@@ -3225,7 +3281,7 @@ int kv_decode_attention_fused(const float* slabs, int n_slabs, long long slab_st
                               int waves, const float* kv_scale, int n_split, float* part_o, float* part_ml, int* counters, const void* pf_base,
                               const long long* pf, unsigned int* pf_sink, hipStream_t stream) {
   if (T <= 0) return 0;
-  if (hd != 128 || block_size != 16 || nh % nkv || n_slabs < 1 || n_slabs > 16 || (waves != 4 && waves != 8)) return -1;
+  if ((hd != 128 && hd != 64) || block_size != 16 || nh % nkv || n_slabs < 1 || n_slabs > 16 || (waves != 4 && waves != 8)) return -1;
   if (n_split < 1 || n_split > 64 || (n_split > 1 && (!part_o || !part_ml || !counters))) return -1;
   const int rep = nh / nkv;
   const float sl = scale * 1.4426950408889634f;
@@ -3289,6 +3345,38 @@ int kv_decode_attention_fused(const float* slabs, int n_slabs, long long slab_st
   } else {                \
     KV_LAUNCH_W(R, 4);    \
   }
+#define KV_LAUNCH_64(R, W, K8, SP)                                                                                                                       \
+  hipLaunchKernelGGL((decode_attention_fused_kernel<R, W, K8, SP, false, false, 64>), grid, block, 0, stream, slabs, n_slabs, slab_stride, positions, cos_t, sin_t, k_cache, \
+                     v_cache, slot_mapping, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, (unsigned short*)out, nh, nkv, row_ss, ss_parts,        \
+                     inv_h, eps, sl, kv_scale, part_o, part_ml, counters, plan, n_split, T)
+#define KV_LAUNCH_64K(R, W)                                                                    \
+  if (n_split > 1) {                                                                           \
+    if (kv_scale) { KV_LAUNCH_64(R, W, true, true); } else { KV_LAUNCH_64(R, W, false, true); } \
+  } else {                                                                                     \
+    if (kv_scale) { KV_LAUNCH_64(R, W, true, false); } else { KV_LAUNCH_64(R, W, false, false); } \
+  }
+#define KV_LAUNCH_64W(R)                      \
+  if (waves == 8) {                           \
+    KV_LAUNCH_64K(R, ((R) <= 4 ? 8 : 4));     \
+  } else {                                    \
+    KV_LAUNCH_64K(R, 4);                      \
+  }
+  if (hd == 64) {
+    switch (rep) {
+      case 1: KV_LAUNCH_64W(1); break;
+      case 2: KV_LAUNCH_64W(2); break;
+      case 3: KV_LAUNCH_64W(3); break;
+      case 4: KV_LAUNCH_64W(4); break;
+      case 6: KV_LAUNCH_64W(6); break;
+      case 7: KV_LAUNCH_64W(7); break;
+      case 8: KV_LAUNCH_64W(8); break;
+      default: return -1;
+    }
+    return (int)hipGetLastError();
+  }
+#undef KV_LAUNCH_64W
+#undef KV_LAUNCH_64K
+#undef KV_LAUNCH_64
   switch (rep) {
     case 1: KV_LAUNCH(1); break;
     case 2: KV_LAUNCH(2); break;
@@ -3388,10 +3476,19 @@ int kv_argmax(const void* logits, long long row_stride, int S, int V, long long*
   return (int)hipGetLastError();
 }
 
-int kv_embed_fed(const void* table, const int* tokens, const int* feed, const long long* prev_ids, int n_prev, void* out, int T, int H, int V, hipStream_t stream) {
+// ss_part (or null): fp32 [T][ceil(H / 512)], the sums of squares of each row's segments
+int kv_embed_fed(const void* table, const int* tokens, const int* feed, const long long* prev_ids, int n_prev, void* out, int T, int H, int V, float* ss_part, hipStream_t stream) {
   if (T <= 0) return 0;
   if (H % 8) return -1;
-  hipLaunchKernelGGL(embed_fed_kernel, dim3(T), dim3(256), 0, stream, (const unsigned short*)table, tokens, feed, prev_ids, n_prev, (unsigned short*)out, H, V);
+  hipLaunchKernelGGL(embed_fed_kernel, dim3(T), dim3(256), 0, stream, (const unsigned short*)table, tokens, feed, prev_ids, n_prev, (unsigned short*)out, H, V, ss_part);
+  return (int)hipGetLastError();
+}
+
+// out[i] = x[idx[i]] of [T, H] (bf16, rows of whole 16-byte pieces) for n rows, and out_ss[i] = ss[idx[i]] of [T, parts] (ss null: none); rows outside x are left
+int kv_select_rows(const void* x, long long ldx, const float* ss, int parts, const int* idx, int n, int T, void* out, float* out_ss, int H, hipStream_t stream) {
+  if (n <= 0) return 0;
+  if (T <= 0 || H <= 0 || (H & 7) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)out & 15) || (ss != nullptr && (parts < 1 || out_ss == nullptr))) return -1;
+  hipLaunchKernelGGL(select_rows_kernel, dim3(n), dim3(256), 0, stream, (const unsigned short*)x, ldx, ss, parts, idx, T, (unsigned short*)out, out_ss, H);
   return (int)hipGetLastError();
 }
 

@@ -31,7 +31,7 @@ from .runner import ModelRunner, select_ops
 
 
 class HybridRunner(ModelRunner):
-    SPLIT_MAX_ROWS = 32
+    SPLIT_KV_MIN_CTX, SPLIT_MAX_ROWS = 2048, 32
     QUERY_BLOCK = 32  # queries per work item of the prompt attention kernel
     LATENT_BLOCK = 128  # the same for latent attention
     CHUNK = 64  # tokens per work item of the retention and state-space kernels
@@ -291,7 +291,7 @@ class HybridRunner(ModelRunner):
             if observed:
                 self._after_layer(ri, x)
                 xb = mx.stream_norm(x, jn, fin, eps, width, dt)
-        hs = torch.index_select(xb, 0, self._dev("sample_idx", t_pad)[: self.sample_rows(t_pad)])
+        hs = mx.select_rows(xb, self._dev("sample_idx", t_pad)[: self.sample_rows(t_pad)])
         logits = ops.linear(hs, w.lm_head)
         if cfg.logit_softcap:
             mx.softcap(logits, cfg.logit_softcap)

@@ -355,8 +355,10 @@ class ModelRunner:
     # one launch).
     DECODE_FUSED_MAX_ROWS_KV8 = int(os.environ.get("KVMINI_DECODE_FUSED_MAX_ROWS_KV8", "32"))
     # contexts from this many tokens on take the split-KV variant of a decode-only step (when the
-    # step's shape has one: few rows); below it the extra workgroups only cost launch time
-    SPLIT_KV_MIN_CTX = 2048
+    # step's shape has one: few rows); below it the extra workgroups only cost launch time.  Measured on MI355X, us a layer, 16 rows of 8 kv
+    # heads of 4, one workgroup and shares: one row in use 500 tokens 14.9 and 14.5, 1000 21.9 and 13.9, 2000 35.0 and 14.3; all 16 500 16.1
+    # and 17.9, 1000 23.2 and 23.7, 1400 31.1 and 28.0.
+    SPLIT_KV_MIN_CTX = 1024
     # steps that also carry prompt chunks: at most this many decode tokens, the longest context
     # from DEC_SPLIT_MIN_CTX tokens on (such steps capture their graph on demand, see _variant_graph)
     DEC_SPLIT_ROWS = 16  # from ~64 consecutive decode rows on the per-token kernel fills the chip as well (measured equal)
@@ -409,20 +411,23 @@ class ModelRunner:
             p = plan(wt, t_pad, site) if plan is not None else None
             return {"prefetch": p} if p is not None else {}
 
-        x = ops.embed_tokens(w.embed, tokens, self._dev("feed", t_pad), self.out_ids)
+        ahead = pf(w.layers[0].wqkv, "qkv")
+        first = getattr(ops, "embed_residual", None)  # the embedding is the first residual stream: its sums of squares come with it
+        start = first(w.embed, tokens, self._dev("feed", t_pad), self.out_ids, cfg.rms_eps) if first is not None and not ahead else None
+        x = ops.embed_tokens(w.embed, tokens, self._dev("feed", t_pad), self.out_ids) if start is None else None
         if decode_only == 1 and self.decode_layers is not None and t_pad <= 64:
             # plain decoding step: every layer in one persistent launch (phases separated by device-wide
             # barriers instead of kernel boundaries, weight chunks in flight across them)
-            h, residual = self._add_rmsnorm(x, None, w.layers[0].attn_norm, False)
+            h, residual = start if start is not None else self._add_rmsnorm(x, None, w.layers[0].attn_norm, False)
             self.decode_layers.run(residual, h.ss, positions, self.cos, self.sin, slots, bt, tok_seq, ctx, cfg.rms_eps, self.scale)
             hs = ops.select_rows(h, sample_idx[: self.sample_rows(t_pad)])
             logits = ops.linear(hs, w.lm_head)
             self.out_ids[: logits.shape[0]].copy_(ops.greedy_sample(logits))
             return logits
         side = self._side_stream if (decode_only == 1 and plan is not None and hasattr(ops, "prefetch_weight")) else None
-        residual = None  # the first residual add is a copy
+        # the first residual add is a copy; h: set when the residual stream and its sums are there already (embedding, fused epilogue)
+        h, residual = start if start is not None else (None, None)
         pending_reduce = False  # x is a row-parallel projection's partial output that still has to be summed over the TP ranks
-        h = None  # set when a projection already folded its output into the residual stream (fused epilogue)
         for li, lw in enumerate(w.layers):
             if h is None:
                 h, residual = self._add_rmsnorm(x, residual, lw.attn_norm, pending_reduce, **pf(lw.wqkv, "qkv"))

@@ -112,6 +112,10 @@ def _sine_turns(width: int, device: torch.device) -> torch.Tensor:
     return torch.stack((hi, (f - hi.double()).float()), 1).contiguous().to(device)
 
 
+def select_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
+    return native().select_rows(x, None, idx)[0] if x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0 and x.stride(1) == 1 else torch.index_select(x, 0, idx)
+
+
 def embed_stream(table: torch.Tensor, tokens: torch.Tensor, feed: torch.Tensor, prev_ids: torch.Tensor, ld: int, scale: float = 1.0, positions: Optional[torch.Tensor] = None,
                  keep: bool = False) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     t = tokens.numel()

@@ -62,6 +62,10 @@ def cache_pads(m: Any, dtype: torch.dtype, block_size: int = 16) -> Tuple[int, .
 Join = Optional[Tuple[Optional[torch.Tensor], torch.Tensor]]  # what the stream takes between two layers: rows (or none) and a vector
 
 
+def select_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
+    return torch.index_select(x, 0, idx)
+
+
 def embed_stream(table: torch.Tensor, tokens: torch.Tensor, feed: torch.Tensor, prev_ids: torch.Tensor, ld: int, scale: float = 1.0, positions: Optional[torch.Tensor] = None,
                  keep: bool = False) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """(stream, the first product's input, a copy of the stream if ``keep``): embedding rows times ``scale``, with ``positions`` plus

@@ -1860,6 +1860,62 @@ def test_split_kv_decode_attention_matches_the_unsplit_kernel(rep, kv8):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv8,n_split,lengths", [
+    ((8, 2), False, 1, [1, 2, 17, 300, 0, 64]), ((2, 2), False, 32, [5, 3000, 16, 0, 257]), ((6, 2), True, 1, [1, 33, 100]), ((8, 2), True, 32, [2500, 15, 0, 900]), ((4, 2), False, 1, [129] * 20),
+])
+def test_fused_decode_attention_of_heads_of_64(heads, kv8, n_split, lengths):
+    """One launch against the two it stands for, which share its cache layout and roundings: the cache byte for byte, the output within two roundings
+    to bf16 (2^-7 of the largest value)."""
+    from kvmini.models.llama import LlamaConfig, rope_tables
+    from kvmini.ops import hip_ops
+
+    (nh, nkv), hd, bs, dev = heads, 64, 16, _dev()
+    torch.manual_seed(nh)
+    ctx = torch.tensor(lengths, device=dev, dtype=torch.int32)
+    rows, longest = len(lengths), max(lengths)
+    per = -(-longest // bs)
+    cos, sin = rope_tables(LlamaConfig(head_dim=hd), longest, dev)
+    pos = (ctx - 1).clamp(min=0)
+    bt = torch.randperm(rows * per, device=dev).view(rows, per).int()
+    slots = torch.where(ctx > 0, bt[torch.arange(rows, device=dev), (pos // bs).long()] * bs + pos % bs, -1).int()
+    part = hip_ops.Partial(torch.randn(3, rows, (nh + 2 * nkv) * hd, device=dev) * 0.4, torch.rand(rows, 1, device=dev) * 512 + 1.0, 1e-5, 512)
+    sc = torch.rand(2, nkv, device=dev) + 0.5 if kv8 else None
+    k, v = (_fp8_cache(rows * per, nkv, bs, hd, i) if kv8 else torch.randn(rows * per, nkv, bs, hd, device=dev).bfloat16() for i in (1, 2))
+    seq = torch.arange(rows, device=dev, dtype=torch.int32)
+    k2, v2 = k.clone(), v.clone()
+    assert hip_ops.supports_fused_decode_attention(part, nh, k) is (nh // nkv <= 4 and (not kv8 or rows <= 16))
+    got = hip_ops.rope_attention_fused(part, pos, cos, sin, k, v, slots, bt, seq, ctx, nh, hd**-0.5, kv_scale=sc, n_split=n_split)
+    q = hip_ops.rope_kv_write(part, pos, cos, sin, k2, v2, slots, nh, nkv, hd, sc)
+    want = hip_ops.paged_attention(q, k2, v2, bt, seq, ctx, hd**-0.5, per, sc)
+    live = ctx > 0
+    assert torch.equal(k, k2) and torch.equal(v, v2) and not got[~live].any()
+    assert (got[live].float() - want[live].float()).abs().max() <= 2.0**-7 * want[live].float().abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,rows", [(8, 1), (504, 3), (512, 64), (520, 5), (4096, 20)])
+def test_embedding_with_its_sums_and_chosen_rows_equal_the_launches_they_stand_for(C, width, rows):
+    from kvmini.ops import hip_ops
+
+    torch.manual_seed(width)
+    table = torch.randn(50, width, device="cuda").bfloat16()
+    tokens = torch.randint(0, 50, (rows,), device="cuda", dtype=torch.int32)
+    tokens[0] = -1  # (out of range: row 0)
+    feed = torch.zeros(rows, device="cuda", dtype=torch.int32)
+    feed[rows // 2] = 2
+    prev = torch.tensor([7, 9], device="cuda")
+    x = hip_ops.embed_tokens(table, tokens, feed, prev)
+    want, residual = hip_ops.add_rmsnorm(x, None, None, 1e-5)
+    got, out = hip_ops.embed_residual(table, tokens, feed, prev, 1e-5)
+    assert torch.equal(out, residual) and torch.equal(got.ss, want.ss) and torch.equal(got.x, out)
+    idx = torch.tensor([rows - 1, 0, rows // 2, rows - 1], device="cuda", dtype=torch.int32)
+    sel = hip_ops.select_rows(got, idx)
+    assert torch.equal(sel.x, out[idx.long()]) and torch.equal(sel.ss, got.ss[idx.long()])
+    wide = torch.cat((out, out), 1)[:, width:]
+    assert torch.equal(C.select_rows(wide, None, idx)[0], out[idx.long()])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,longest", [(1, 4000), (63, 300), (64, 1100), (65, 1100), (127, 1500)])
 def test_split_kv_shares_cover_every_row_once(rows, longest):
     """Ranges of the launch's fair share and of the least one, rows on both sides of a wave's width, padding rows in between: each row's blocks are
