@@ -549,35 +549,36 @@ __global__ __launch_bounds__(256, 3) void delta_tile_kernel(const T* __restrict_
   }
 }
 
-// grid (heads, dvp / 16, portions): 16 columns of S, the dkp = 64 RT key channels over four waves (RT row tiles of 16 each).
+// A workgroup has 16 CT columns of S and the dkp = 64 RT key channels over four waves (RT row tiles of 16 each).
 // mfma_f32_16x16x4: A lane (row l & 15, k l >> 4), B lane (column l & 15, k l >> 4), D lane rows 4 (l >> 4) + r.  The k order of the
 // products with S is chosen so that an accumulator register is a B operand as it is: step s takes the channels 4 q + s.
-template <typename T, int RT>
-__global__ __launch_bounds__(256) void delta_chain_kernel(const float* __restrict__ ws, float* __restrict__ o, const T* __restrict__ proj, T* __restrict__ ring, const int* __restrict__ seg_row,
-                                                          const int* __restrict__ seg_n, const int* __restrict__ seg_pos, const int* __restrict__ seg_slot,
-                                                          const int* __restrict__ seg_tile, int min_n, int dkp, int dvp, DeltaArgs a) {
-  __shared__ __attribute__((aligned(16))) f4 part[2][4][2][64];
+template <typename T, int RT, int CT>
+__device__ __attribute__((always_inline)) inline void delta_chain(f4* lds, int y, int n, const float* __restrict__ ws, float* __restrict__ o, const T* __restrict__ proj, T* __restrict__ ring, const int* __restrict__ seg_row,
+                                                                  const int* __restrict__ seg_pos, const int* __restrict__ seg_slot, const int* __restrict__ seg_tile, int dkp, int dvp, const DeltaArgs& a) {
+  f4(*part)[4][2 * CT][64] = reinterpret_cast<f4(*)[4][2 * CT][64]>(lds);
   const int h = blockIdx.x, sg = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n = seg_n[sg];
-  if (n == 0 || n < min_n) return;
   const int lr = lane & 15, lq = lane >> 4;
-  const int col = blockIdx.y * 16 + lr, base = wave * RT * 16;
-  const bool col_on = col < a.vdim;
+  const int col = y * (16 * CT) + lr, base = wave * RT * 16;  // (and the columns 16 further)
+  bool col_on[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) col_on[c] = col + 16 * c < a.vdim;
   const int pos0 = seg_pos[sg], slot = seg_slot[sg], nt = (n + 15) >> 4;
   const long long row0 = seg_row[sg];
   const long long tf = tile_floats(dkp, dvp), step = tf * a.heads;
   const float* w = ws + ((long long)seg_tile[sg] * a.heads + h) * tf;
   float* sp = a.state + ((long long)slot * a.heads + h) * a.dim * a.vdim + col;
-  f4 s[RT];
+  f4 s[CT][RT];
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
+  for (int c = 0; c < CT; ++c)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = base + 16 * t + 4 * lq + r;
-      s[t][r] = (pos0 > 0 && col_on && d < a.dim) ? sp[(long long)d * a.vdim] : 0.f;
-    }
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = base + 16 * t + 4 * lq + r;
+        s[c][t][r] = (pos0 > 0 && col_on[c] && d < a.dim) ? sp[(long long)d * a.vdim + 16 * c] : 0.f;
+      }
   // two tiles in flight: a tile's coefficients come from beyond this XCD's L2 the first time, and one tile takes less time than that
-  struct Tile { f4 tk[RT], qe[RT], ke[RT], gc[RT], tv; float ov; };
+  struct Tile { f4 tk[RT], qe[RT], ke[RT], gc[RT], tv[CT]; float ov[CT]; };
   Tile ta, tb;
   auto fetch = [&](Tile& x, int i) __attribute__((always_inline)) {
     const float* p = w + step * (i < nt ? i : nt - 1);
@@ -590,39 +591,55 @@ __global__ __launch_bounds__(256) void delta_chain_kernel(const float* __restric
       x.gc[t] = *reinterpret_cast<const f4*>(p + 48 * dkp + d + 4 * lq);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) x.tv[r] = p[49 * dkp + (4 * lq + r) * dvp + col];
-    x.ov = p[49 * dkp + (16 + 4 * lq + wave) * dvp + col];
+    for (int c = 0; c < CT; ++c) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x.tv[c][r] = p[49 * dkp + (4 * lq + r) * dvp + col + 16 * c];
+      x.ov[c] = p[49 * dkp + (16 + 4 * lq + wave) * dvp + col + 16 * c];
+    }
     __builtin_amdgcn_sched_barrier(0);  // the loads are issued here and not where they are used
   };
   auto run = [&](Tile& x, int i) __attribute__((always_inline)) {
-    f4 xk = {0.f, 0.f, 0.f, 0.f}, xq = xk;
+    f4 xk[CT], xq[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) xk[c] = xq[c] = (f4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        xk = __builtin_amdgcn_mfma_f32_16x16x4f32(x.tk[t][e], s[t][e], xk, 0, 0, 0);
-        xq = __builtin_amdgcn_mfma_f32_16x16x4f32(x.qe[t][e], s[t][e], xq, 0, 0, 0);
-      }
-    f4(*pb)[2][64] = part[i & 1];
-    pb[wave][0][lane] = xk;
-    pb[wave][1][lane] = xq;
-    __syncthreads();  // (the other buffer may still be read by slower waves, this one not: they are past the last barrier)
-    f4 sum = pb[0][0][lane];
-    float os = reinterpret_cast<const float*>(&pb[0][1][lane])[wave];
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-    for (int v = 1; v < 4; ++v) {
-      sum += pb[v][0][lane];
-      os += reinterpret_cast<const float*>(&pb[v][1][lane])[wave];
+        for (int c = 0; c < CT; ++c) {
+          xk[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.tk[t][e], s[c][t][e], xk[c], 0, 0, 0);
+          xq[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.qe[t][e], s[c][t][e], xq[c], 0, 0, 0);
+        }
+    f4(*pb)[2 * CT][64] = part[i & 1];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      pb[wave][2 * c][lane] = xk[c];
+      pb[wave][2 * c + 1][lane] = xq[c];
     }
-    const f4 u = x.tv - sum;
+    __syncthreads();  // (the other buffer may still be read by slower waves, this one not: they are past the last barrier)
     const int tok = 16 * i + 4 * lq + wave;
-    if (tok < n && col_on) o[((row0 + tok) * a.heads + h) * a.vdim + col] = x.ov + os;
+    f4 u[CT];
 #pragma unroll
-    for (int t = 0; t < RT; ++t) s[t] *= x.gc[t];
+    for (int c = 0; c < CT; ++c) {
+      f4 sum = pb[0][2 * c][lane];
+      float os = reinterpret_cast<const float*>(&pb[0][2 * c + 1][lane])[wave];
+#pragma unroll
+      for (int v = 1; v < 4; ++v) {
+        sum += pb[v][2 * c][lane];
+        os += reinterpret_cast<const float*>(&pb[v][2 * c + 1][lane])[wave];
+      }
+      u[c] = x.tv[c] - sum;
+      if (tok < n && col_on[c]) o[((row0 + tok) * a.heads + h) * a.vdim + col + 16 * c] = x.ov[c] + os;
+#pragma unroll
+      for (int t = 0; t < RT; ++t) s[c][t] *= x.gc[t];
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int t = 0; t < RT; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.ke[t][e], u[e], s[t], 0, 0, 0);
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) s[c][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.ke[t][e], u[c][e], s[c][t], 0, 0, 0);
   };
   fetch(ta, 0);
   fetch(tb, 1);
@@ -635,13 +652,15 @@ __global__ __launch_bounds__(256) void delta_chain_kernel(const float* __restric
   }
   if (i < nt) run(ta, i);
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
+  for (int c = 0; c < CT; ++c)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = base + 16 * t + 4 * lq + r;
-      if (col_on && d < a.dim) sp[(long long)d * a.vdim] = s[t][r];
-    }
-  if (blockIdx.y == 0) {  // the convolution inputs the next portion needs (their readers ran in the tile kernel)
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = base + 16 * t + 4 * lq + r;
+        if (col_on[c] && d < a.dim) sp[(long long)d * a.vdim + 16 * c] = s[c][t][r];
+      }
+  if (y == 0) {  // the convolution inputs the next portion needs (their readers ran in the tile kernel)
     const int rep = a.heads / a.kv_heads, g = h / rep, qk = a.kv_heads * a.dim;
     const int keep = n < a.taps ? n : a.taps;
     const int own = a.vdim + (h % rep == 0 ? 2 * a.dim : 0);
@@ -650,6 +669,29 @@ __global__ __launch_bounds__(256) void delta_chain_kernel(const float* __restric
       const T* p = proj + row0 * a.ldp + chan_col(a, c);
       for (int i = n - keep; i < n; ++i) ring[((long long)slot * a.taps + (pos0 + i) % a.taps) * a.channels + c] = p[i * a.ldp];
     }
+  }
+}
+
+// grid (heads, dvp / 16, portions).  What bounds a tile's step is what is read of it (25 KB for 128 key channels and 16 columns, from beyond the L2) and
+// the fp32 matrix instructions (0.35 us); its serial chain is about as long.  Two column tiles a workgroup read half as much and leave half the
+// workgroups: taken where one each would be more than two workgroups per CU (measured, 32 heads of 128 x 128: 4 x 512 tokens 109 -> 95 us, 16 x 100 95 -> 84;
+// below, one and two, 2 x 1000 105 and 108, 1 x 2048 133 and 202).  How many portions there are only the device knows.
+constexpr int CHAIN_WGS = 512;
+template <typename T, int RT>
+__global__ __launch_bounds__(256) void delta_chain_kernel(const float* __restrict__ ws, float* __restrict__ o, const T* __restrict__ proj, T* __restrict__ ring, const int* __restrict__ seg_row,
+                                                          const int* __restrict__ seg_n, const int* __restrict__ seg_pos, const int* __restrict__ seg_slot,
+                                                          const int* __restrict__ seg_tile, int min_n, int dkp, int dvp, DeltaArgs a) {
+  __shared__ __attribute__((aligned(16))) f4 part[2 * 4 * 4 * 64];
+  const int n = seg_n[blockIdx.z];
+  if (n == 0 || n < min_n) return;
+  int live = 0;
+  for (int i = threadIdx.x & 63; i - (int)(threadIdx.x & 63) < (int)gridDim.z; i += 64)
+    live += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < (int)gridDim.z && seg_n[i] > 0 && seg_n[i] >= min_n));
+  if (dvp % 32 == 0 && live * (int)(gridDim.x * gridDim.y) > CHAIN_WGS) {
+    if (blockIdx.y & 1) return;
+    delta_chain<T, RT, 2>(part, blockIdx.y >> 1, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
+  } else {
+    delta_chain<T, RT, 1>(part, blockIdx.y, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
   }
 }
 

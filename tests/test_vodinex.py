@@ -156,6 +156,40 @@ def test_chunked_attention_alone(backend, heads, kv, dim, vdim, chunk, rot):
     assert float(rows.max()) < (2e-5 if dtype == "fp32" else 0.08), int(rows.argmax())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,dim,vdim", [(8, 64, 256), (32, 128, 64), (16, 200, 128), (24, 128, 80)])
+def test_delta_portions_together_equal_each_alone(heads, dim, vdim):
+    """Enough portions that a workgroup takes two column tiles (a value size of 80 never does), against each portion in a step of its own: the sums of a
+    column are the same, so bit for bit, output and state."""
+    device, mx = torch.device("cuda:0"), mixers_of(torch.device("cuda:0"))
+    m = hybrid.DeltaSpec(heads, heads, dim, vdim, 4)
+    gen = torch.Generator().manual_seed(dim)
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    offs = [0, heads * dim, 2 * heads * dim, 2 * heads * dim + heads * vdim]
+    f = lambda x: x.float().contiguous().to(device)  # noqa: E731
+    w = hybrid.DeltaWeights(*offs, 0, 0, 0, heads * dim, 0, None, f(0.3 * rnd(4, m.channels)), f(rnd(heads) - 2), f(rnd(heads * dim) - 2), f(rnd(vdim)))
+    lens = [40, 17, 2, 33, 64, 16, 50]
+    proj, low = [rnd(n, offs[3] + heads).bfloat16() for n in lens], [rnd(n, heads * (dim + vdim)).bfloat16() for n in lens]
+
+    def run(which):
+        state, ring = torch.full((8, heads, dim, vdim), 7.0, device=device), torch.zeros(8, 4, m.channels, dtype=torch.bfloat16, device=device)
+        ds = mx.DeltaState(m, w, 1.0, 1e-5, state, ring)
+        st = make_step(mx, [(lens[i], 0, i + 1) for i in which], device, n_blocks=160)
+        x, lo = (torch.zeros(st.rows, v[0].shape[1], dtype=torch.bfloat16, device=device) for v in (proj, low))
+        n = sum(lens[i] for i in which)
+        x[:n], lo[:n] = torch.cat([proj[i] for i in which]).to(device), torch.cat([low[i] for i in which]).to(device)
+        mix = torch.zeros(st.rows, heads * vdim, dtype=torch.bfloat16, device=device)
+        ds.run(x, lo, mix, st)
+        return mix[:n], state
+
+    together, state = run(range(len(lens)))
+    at = 0
+    for i, n in enumerate(lens):
+        alone, one = run([i])
+        assert torch.equal(together[at : at + n], alone) and torch.equal(state[i + 1], one[i + 1]), i
+        at += n
+
+
 @pytest.mark.parametrize("backend", BACKENDS)
 @pytest.mark.parametrize("heads,kv,dim,vdim,taps,strong", [(4, 2, 24, 16, 3, 0.0), (2, 2, 128, 128, 4, 0.0), (3, 1, 40, 6, 1, 3.0), (4, 4, 28, 36, 2, 4.0), (2, 1, 200, 48, 6, 1.0), (8, 2, 64, 256, 4, 0.0), (2, 2, 256, 128, 3, 0.0), (1, 1, 260, 64, 4, 0.0)])
 def test_delta_rule_alone(backend, heads, kv, dim, vdim, taps, strong):
