@@ -76,21 +76,36 @@ __device__ __forceinline__ void attend_tile(const bf16raw* k_img, const bf16raw*
                                             bool edge, int last_key, int first_key, frag_acc st, int keep_key = 0, Finish finish = Finish()) {
   const int lane = threadIdx.x & 63, lr = lane & 31, hi = lane >> 5;
   const int vq = (lane >> 2) & 3, vp = lane & 3, vodd = (lane >> 4) & 1;
+  // the keys' fragments all at once (in pairs, each behind the products of the pair before, the LDS answered four times a step)
+  constexpr int KG = DK / 16 < 8 ? DK / 16 : 8;
 #pragma unroll
-  for (int ks = 0; ks < DK / 16; ++ks) {
-    const frag_ab kf = *reinterpret_cast<const frag_ab*>(&k_img[lr * DK + (((2 * ks + hi) ^ (ONE ? kv_swz<DK>(lr) : k_swz<DK>(lr))) << 3)]);
-    st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qa[ks], st, 0, 0, 0);
+  for (int k0 = 0; k0 < DK / 16; k0 += KG) {
+    frag_ab kf[KG];
+#pragma unroll
+    for (int i = 0; i < KG; ++i) kf[i] = *reinterpret_cast<const frag_ab*>(&k_img[lr * DK + (((2 * (k0 + i) + hi) ^ (ONE ? kv_swz<DK>(lr) : k_swz<DK>(lr))) << 3)]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < KG; ++i) st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qa[k0 + i], st, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
   }
-  // V^T fragments of key half h, dims 32 n + lr: two transposed reads (4 keys each); the first half's are read under the softmax
+  // V^T fragments of key half h, dims 32 n + lr: two transposed reads (4 keys each), read under the softmax
   auto v_read = [&](int h, int n, int j) __attribute__((always_inline)) {
     const int r = 16 * h + 8 * j + 4 * hi + vq, c = 4 * n + 2 * vodd + (vp >> 1);
     return lds_read_tr(v_img + r * DV + ((c ^ (ONE ? kv_swz<DV>(r) : v_swz<DV>(r))) << 3) + (vp & 1) * 4);
   };
+  constexpr bool BOTH = DV <= 128;  // (wider, the second half's registers are the first one's: read behind its products)
   tr_b64 v0[DV / 16], v1[DV / 16];
 #pragma unroll
   for (int n = 0; n < DV / 32; ++n) {
     v0[2 * n] = v_read(0, n, 0);
     v0[2 * n + 1] = v_read(0, n, 1);
+  }
+  if constexpr (BOTH) {
+#pragma unroll
+    for (int n = 0; n < DV / 32; ++n) {
+      v1[2 * n] = v_read(1, n, 0);
+      v1[2 * n + 1] = v_read(1, n, 1);
+    }
   }
   // accumulator register r: key 8 (r / 4) + 4 hi + r % 4
   float sc[16];
@@ -109,12 +124,12 @@ __device__ __forceinline__ void attend_tile(const bf16raw* k_img, const bf16raw*
   for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
   const float m_old = m_run, m_new = fmaxf(m_old, mx);
+  const float m_sub = m_new > -1e29f ? m_new : 1e30f;  // (a query none of whose keys have come up yet: nothing counts)
   float psum = 0.f;
   frag_ab pb[2];
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
-    // (a query none of whose keys have come up yet: nothing counts)
-    const float p = m_new > -1e29f ? __builtin_amdgcn_exp2f(sc[r] - m_new) : 0.f;
+    const float p = __builtin_amdgcn_exp2f(sc[r] - m_sub);
     psum += p;
     pb[r >> 3][r & 7] = (__bf16)p;
   }
@@ -128,10 +143,12 @@ __device__ __forceinline__ void attend_tile(const bf16raw* k_img, const bf16raw*
       for (int r = 0; r < 16; ++r) o[n][r] *= corr;
   }
   lds_landed(v0);
+  if constexpr (!BOTH) {
 #pragma unroll
-  for (int n = 0; n < DV / 32; ++n) {
-    v1[2 * n] = v_read(1, n, 0);
-    v1[2 * n + 1] = v_read(1, n, 1);
+    for (int n = 0; n < DV / 32; ++n) {
+      v1[2 * n] = v_read(1, n, 0);
+      v1[2 * n + 1] = v_read(1, n, 1);
+    }
   }
 #pragma unroll
   for (int n = 0; n < DV / 32; ++n) {
@@ -143,6 +160,29 @@ __device__ __forceinline__ void attend_tile(const bf16raw* k_img, const bf16raw*
   for (int n = 0; n < DV / 32; ++n) {
     const struct { tr_b64 lo, hi; } vf = {v1[2 * n], v1[2 * n + 1]};
     o[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(frag_ab, vf), pb[1], o[n], 0, 0, 0);
+  }
+}
+
+// A lane's part of a query's output, o times f and, behind a gate (gp, else null), sigmoid(gate): dims 32 n + 8 r + 4 hi .. + 3, in pieces of 8 bytes.
+// All gates are read before the first store: a load behind a store waits for it (16 of them: 16 us of a kernel's end).
+template <int DV>
+__device__ __forceinline__ void store_output(bf16raw* op, const bf16raw* gp, const frag_acc (&o)[DV / 32], float f, int vdim, int hi) {
+  float4 z[DV / 8];
+  if (gp) {
+#pragma unroll
+    for (int i = 0; i < DV / 8; ++i) {
+      const int d = 8 * i + 4 * hi;
+      z[i] = d < vdim ? ld4(gp + d) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < DV / 8; ++i) {
+    const int d = 8 * i + 4 * hi, r = 4 * (i & 3);
+    float4 v = make_float4(o[i >> 2][r] * f, o[i >> 2][r + 1] * f, o[i >> 2][r + 2] * f, o[i >> 2][r + 3] * f);
+    if (gp) {
+      v.x *= sigmoid(z[i].x); v.y *= sigmoid(z[i].y); v.z *= sigmoid(z[i].z); v.w *= sigmoid(z[i].w);
+    }
+    if (d < vdim) st4(op + d, v);
   }
 }
 

@@ -178,6 +178,10 @@ __global__ __launch_bounds__(64 * NW, DV <= 128 ? 2 : 1) void chunk_prefill_kern
   bf16raw* op = out + row * a.ldo + a.o_off + (long long)head * a.vdim;
   const bool vec = (a.vdim & 3) == 0 && (a.ldo & 3) == 0 && (a.o_off & 3) == 0 && (a.gated != 2 || ((a.ld_gate | a.gate_off) & 3) == 0);
   const bf16raw* gp = a.gated == 2 ? gate + row * a.ld_gate + a.gate_off + (long long)head * a.vdim : nullptr;
+  if (vec) {
+    store_output<DV>(op, gp, o, f, a.vdim, hi);
+    return;
+  }
 #pragma unroll
   for (int n = 0; n < DV / 32; ++n)
 #pragma unroll
@@ -186,24 +190,16 @@ __global__ __launch_bounds__(64 * NW, DV <= 128 ? 2 : 1) void chunk_prefill_kern
       float4 v = make_float4(o[n][4 * rr] * f, o[n][4 * rr + 1] * f, o[n][4 * rr + 2] * f, o[n][4 * rr + 3] * f);
       if (gp && d < a.vdim) {
         float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (vec) {
-          z = ld4(gp + d);
-        } else {
-          z.x = ld(gp + d);
-          if (d + 1 < a.vdim) z.y = ld(gp + d + 1);
-          if (d + 2 < a.vdim) z.z = ld(gp + d + 2);
-          if (d + 3 < a.vdim) z.w = ld(gp + d + 3);
-        }
+        z.x = ld(gp + d);
+        if (d + 1 < a.vdim) z.y = ld(gp + d + 1);
+        if (d + 2 < a.vdim) z.z = ld(gp + d + 2);
+        if (d + 3 < a.vdim) z.w = ld(gp + d + 3);
         v.x *= sigmoid(z.x); v.y *= sigmoid(z.y); v.z *= sigmoid(z.z); v.w *= sigmoid(z.w);
       }
-      if (vec) {
-        if (d < a.vdim) st4(op + d, v);
-      } else {
-        if (d < a.vdim) st(op + d, v.x);
-        if (d + 1 < a.vdim) st(op + d + 1, v.y);
-        if (d + 2 < a.vdim) st(op + d + 2, v.z);
-        if (d + 3 < a.vdim) st(op + d + 3, v.w);
-      }
+      if (d < a.vdim) st(op + d, v.x);
+      if (d + 1 < a.vdim) st(op + d + 1, v.y);
+      if (d + 2 < a.vdim) st(op + d + 2, v.z);
+      if (d + 3 < a.vdim) st(op + d + 3, v.w);
     }
 }
 
