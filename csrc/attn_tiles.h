@@ -164,7 +164,7 @@ __device__ __forceinline__ void attend_tile(const bf16raw* k_img, const bf16raw*
 }
 
 // A lane's part of a query's output, o times f and, behind a gate (gp, else null), sigmoid(gate): dims 32 n + 8 r + 4 hi .. + 3, in pieces of 8 bytes.
-// All gates are read before the first store: a load behind a store waits for it (16 of them: 16 us of a kernel's end).
+// All gates are read before the first store: a load behind a store waits for it (16 of them: 8 us of a kernel's end).
 template <int DV>
 __device__ __forceinline__ void store_output(bf16raw* op, const bf16raw* gp, const frag_acc (&o)[DV / 32], float f, int vdim, int hi) {
   float4 z[DV / 8];

@@ -14,7 +14,13 @@ using namespace attn;
 
 // ---- routing: logits (fp32 products, plus a bias), scores sigmoid(logit), softmax(logits), or softmax over the chosen logits alone (the
 // scores to choose by are then the logits), the `top` largest score + correction (the first of equals), their scores times `scale`.  With shared_of, row E of the router is the shared expert's gate: its sigmoid.
-// Workgroup: 16 tokens, 16 waves — which share K (bf16, matrix cores) or take a token each (fp32), then choose for a token each.
+// fp32, and bf16 of more than 1024 tokens: one launch.  bf16 of fewer: a launch for the products, one for the choice — the matrix of 64 experts
+// of 4096 is 512 KB, and where each workgroup of 16 tokens reads all of it the rate at which one compute unit reads is the time; here a
+// workgroup has a share of K.  With many tokens the sums of the shares are what costs (8 MB of them for 2048 tokens of 64).  Measured on
+// MI355X, cold, us (one launch, two): 64 experts and a shared one of 4096, 16 / 64 / 512 / 2048 tokens 24.4, 10.4 / 20.5, 11.1 / 20.4, 12.0 /
+// 21.5, 21.3; 64 of 2304 14.6, 9.3 / 13.8, 9.8 / 14.0, 10.8 / 14.9, 17.8; 8 of 1024 9.8, 9.3 / 9.8, 9.3 / 10.0, 9.0 / 10.4, 11.6.  The
+// shares are the ones the waves of the one launch have and are summed in the same order: the results are the same bits.
+constexpr int ROUTE_SHARES = 16;  // of K
 enum Scores { SIGMOID = 0, SOFTMAX = 1, CHOSEN = 2 };
 struct RouteArgs {
   int T, E, Ep, top, K; long long ldh;  // Ep: experts in the packed matrix (a multiple of 16)
@@ -24,6 +30,149 @@ struct RouteArgs {
   const float* bias;
 };
 
+// bf16 products: workgroup = 64 tokens x 64 experts (32 x 32 a wave) x a share of K; part: fp32 [ROUTE_SHARES][T][Ep]
+__global__ __launch_bounds__(256) void route_products_kernel(const bf16raw* __restrict__ h, const bf16raw* __restrict__ w, float* __restrict__ part, int T, int Ep, int K, long long ldh) {
+  constexpr int U = 8;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
+  const int tile = blockIdx.z * 4 + 2 * (wave & 1), t0 = blockIdx.x * 64 + 32 * (wave >> 1), nks = K / 32;
+  const int k0 = nks * (int)blockIdx.y / ROUTE_SHARES, k1 = nks * ((int)blockIdx.y + 1) / ROUTE_SHARES;
+  if (16 * tile >= Ep || t0 >= T) return;
+  const frag_ab* wp[2];
+  const bf16raw* hp[2];
+  frag_acc4 acc[2][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int t = t0 + 16 * j + lr;
+    hp[j] = h + (long long)(t < T ? t : T - 1) * ldh + lq * 8;
+    wp[j] = reinterpret_cast<const frag_ab*>(w) + (long long)(16 * (tile + j) < Ep ? tile + j : tile) * nks * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) acc[i][j] = (frag_acc4){0.f, 0.f, 0.f, 0.f};
+  }
+  for (int ks = k0; ks < k1; ks += U) {
+    frag_ab m[U][2], x[U][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = ks + u < k1 ? ks + u : k1 - 1;  // (steps past the end are not multiplied)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        m[u][j] = wp[j][(long long)k * 64];
+        x[u][j] = *reinterpret_cast<const frag_ab*>(hp[j] + k * 32);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (ks + u < k1) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m[u][i], x[u][j], acc[i][j], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int t = t0 + 16 * j + lr;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (t < T && 16 * (tile + i) < Ep) *reinterpret_cast<frag_acc4*>(part + ((long long)blockIdx.y * T + t) * Ep + 16 * (tile + i) + 4 * lq) = acc[i][j];
+  }
+}
+
+// One wave's choice for its token.  NC: experts per lane; z: the token's logits; corr: the corrections of the lane's experts
+template <int NC>
+__device__ inline void choose(const float* z, const float (&corr)[NC], bool pad, int t, int lane, const RouteArgs& a) {
+  if (a.shared_of && lane == 0) a.shared_of[t] = pad ? 0.f : 1.f / (1.f + expf(-z[a.E]));
+  float top_z = 0.f, unit = 1.f;  // a score: sigmoid(z), or exp(z - top_z) over the sum of them
+  if (a.scores != SIGMOID) {
+    top_z = -INFINITY;
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (lane + 64 * i < a.E) top_z = fmaxf(top_z, z[lane + 64 * i]);
+    top_z = wave_max(top_z);
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (lane + 64 * i < a.E) sum += expf(z[lane + 64 * i] - top_z);
+    unit = 1.f / wave_sum(sum);
+  }
+  auto score = [&](int e) { return a.scores != SIGMOID ? expf(z[e] - top_z) * unit : 1.f / (1.f + expf(-z[e])); };
+  float c[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int e = lane + 64 * i;
+    c[i] = e < a.E ? (a.scores == CHOSEN ? z[e] : score(e)) + corr[i] : -INFINITY;
+    if (!(c[i] == c[i])) c[i] = -INFINITY;  // (padding rows may hold anything: every choice below must be written all the same)
+  }
+  if constexpr (NC == 1) {  // an expert per lane: its rank is the number of better ones (of equals, the earlier)
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+      const float o = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c[0]), j));
+      rank += (o > c[0] || (o == c[0] && j < lane)) ? 1 : 0;
+    }
+    if (a.scores == CHOSEN) unit = 1.f / wave_sum(lane < a.E && rank < a.top ? expf(z[lane] - top_z) : 0.f);
+    if (lane < a.E && rank < a.top) {
+      a.expert_of[t * a.top + rank] = pad ? -1 : lane;
+      a.weight_of[t * a.top + rank] = pad ? 0.f : score(lane) * a.scale;
+    }
+    return;
+  }
+  int mine = -1;  // lane k: choice k
+  for (int k = 0; k < a.top; ++k) {
+    float best = -INFINITY;
+    int idx = 0x7fffffff;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (c[i] > best) { best = c[i]; idx = lane + 64 * i; }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const float v = __shfl_xor(best, o, 64);
+      const int j = __shfl_xor(idx, o, 64);
+      if (v > best || (v == best && j < idx)) { best = v; idx = j; }
+    }
+    if (lane == k) mine = idx;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (lane + 64 * i == idx) c[i] = -INFINITY;
+  }
+  const bool ok = !pad && lane < a.top && mine >= 0 && mine < a.E;
+  if (a.scores == CHOSEN) unit = 1.f / wave_sum(ok ? expf(z[mine] - top_z) : 0.f);
+  if (lane >= a.top) return;
+  a.expert_of[t * a.top + lane] = ok ? mine : -1;
+  a.weight_of[t * a.top + lane] = ok ? score(mine) * a.scale : 0.f;
+}
+
+template <int NC>
+__device__ inline void load_corrections(float (&corr)[NC], int lane, const RouteArgs& a) {
+#pragma unroll
+  for (int i = 0; i < NC; ++i) corr[i] = lane + 64 * i < a.E ? a.correction[lane + 64 * i] : 0.f;
+}
+
+// bf16: the shares' sums and the choice.  Workgroup: 4 tokens, a wave each; all that is read is asked for before the first use
+template <int NC>
+__global__ __launch_bounds__(256) void route_choose_kernel(const float* __restrict__ part, RouteArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float rt_lds[];  // logits [4][Ep + 1]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + wave;
+  if (t >= a.T) return;
+  float* z = rt_lds + wave * (a.Ep + 1);
+  const bool pad = a.slots[t] < 0;
+  float corr[NC];
+  load_corrections<NC>(corr, lane, a);
+  for (int e = lane; e < a.Ep; e += 64) {
+    const float b = a.bias && e < a.E ? a.bias[e] : 0.f;
+    float v[ROUTE_SHARES], s = 0.f;
+#pragma unroll
+    for (int k = 0; k < ROUTE_SHARES; ++k) v[k] = part[((long long)k * a.T + t) * a.Ep + e];
+#pragma unroll
+    for (int k = 0; k < ROUTE_SHARES; ++k) s += v[k];
+    z[e] = s + b;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // (a wave reads what its own lanes wrote)
+  __builtin_amdgcn_wave_barrier();
+  choose<NC>(z, corr, pad, t, lane, a);
+}
+
+// One launch.  Workgroup: 16 tokens, 16 waves — which share K (bf16, matrix cores) or take a token each (fp32), then choose for a token each.
 // NC: experts per lane of a token's wave; TL: tiles of 16 experts multiplied at a time (bf16)
 template <typename T, int NC, int TL>
 __global__ __launch_bounds__(1024) void route_kernel(const T* __restrict__ h, const T* __restrict__ w, RouteArgs a) {
@@ -85,67 +234,9 @@ __global__ __launch_bounds__(1024) void route_kernel(const T* __restrict__ h, co
   }
   const int t = t0 + wave;
   if (t >= a.T) return;
-  const bool pad = a.slots[t] < 0;
-  const float* z = rt_lds + wave * ls;
-  if (a.shared_of && lane == 0) a.shared_of[t] = pad ? 0.f : 1.f / (1.f + expf(-z[a.E]));
-  float top_z = 0.f, unit = 1.f;  // a score: sigmoid(z), or exp(z - top_z) over the sum of them
-  if (a.scores != SIGMOID) {
-    top_z = -INFINITY;
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < NC; ++i)
-      if (lane + 64 * i < a.E) top_z = fmaxf(top_z, z[lane + 64 * i]);
-    top_z = wave_max(top_z);
-#pragma unroll
-    for (int i = 0; i < NC; ++i)
-      if (lane + 64 * i < a.E) sum += expf(z[lane + 64 * i] - top_z);
-    unit = 1.f / wave_sum(sum);
-  }
-  auto score = [&](int e) { return a.scores != SIGMOID ? expf(z[e] - top_z) * unit : 1.f / (1.f + expf(-z[e])); };
-  float c[NC];
-#pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const int e = lane + 64 * i;
-    c[i] = e < a.E ? (a.scores == CHOSEN ? z[e] : score(e)) + a.correction[e] : -INFINITY;
-    if (!(c[i] == c[i])) c[i] = -INFINITY;  // (padding rows may hold anything: every choice below must be written all the same)
-  }
-  if constexpr (NC == 1) {  // an expert per lane: its rank is the number of better ones (of equals, the earlier)
-    int rank = 0;
-#pragma unroll
-    for (int j = 0; j < 64; ++j) {
-      const float o = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c[0]), j));
-      rank += (o > c[0] || (o == c[0] && j < lane)) ? 1 : 0;
-    }
-    if (a.scores == CHOSEN) unit = 1.f / wave_sum(lane < a.E && rank < a.top ? expf(z[lane] - top_z) : 0.f);
-    if (lane < a.E && rank < a.top) {
-      a.expert_of[t * a.top + rank] = pad ? -1 : lane;
-      a.weight_of[t * a.top + rank] = pad ? 0.f : score(lane) * a.scale;
-    }
-    return;
-  }
-  int mine = -1;  // lane k: choice k
-  for (int k = 0; k < a.top; ++k) {
-    float best = -INFINITY;
-    int idx = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < NC; ++i)
-      if (c[i] > best) { best = c[i]; idx = lane + 64 * i; }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float v = __shfl_xor(best, o, 64);
-      const int j = __shfl_xor(idx, o, 64);
-      if (v > best || (v == best && j < idx)) { best = v; idx = j; }
-    }
-    if (lane == k) mine = idx;
-#pragma unroll
-    for (int i = 0; i < NC; ++i)
-      if (lane + 64 * i == idx) c[i] = -INFINITY;
-  }
-  const bool ok = !pad && lane < a.top && mine >= 0 && mine < a.E;
-  if (a.scores == CHOSEN) unit = 1.f / wave_sum(ok ? expf(z[mine] - top_z) : 0.f);
-  if (lane >= a.top) return;
-  a.expert_of[t * a.top + lane] = ok ? mine : -1;
-  a.weight_of[t * a.top + lane] = ok ? score(mine) * a.scale : 0.f;
+  float corr[NC];
+  load_corrections<NC>(corr, lane, a);
+  choose<NC>(rt_lds + wave * ls, corr, a.slots[t] < 0, t, lane, a);
 }
 
 // ---- grouping for many rows: pairs in the order of their experts, an expert's in equal tiles of at most `bm` pairs (whole 32s: what the products
@@ -346,10 +437,23 @@ __global__ __launch_bounds__(256) void expert_pairs_kernel(const float* __restri
 
 extern "C" {
 
+// floats of workspace that a call takes (0: one launch, none)
+long long kve_route_workspace(int f32, int T, int Ep) { return f32 || T > 1024 ? 0 : (long long)ROUTE_SHARES * T * Ep; }
+
 int kve_route(const void* h, int f32, long long ldh, const void* w, const float* correction, const int* slots, int T, int E, int Ep, int top, int K, int* expert_of, float* weight_of, int scores, float scale, float* shared_of, const float* bias,
-              hipStream_t s) {
+              float* ws, hipStream_t s) {
   if (T <= 0 || E <= 0 || E > 1024 || Ep < E + (shared_of ? 1 : 0) || top <= 0 || top > E || top > 64 || K <= 0 || scores < SIGMOID || scores > CHOSEN || (!f32 && ((Ep & 15) || (K & 31) || (ldh & 7)))) return -1;
   const RouteArgs a{T, E, Ep, top, K, ldh, correction, slots, expert_of, weight_of, scores, scale, shared_of, bias};
+  if (kve_route_workspace(f32, T, Ep)) {
+    if (!ws) return -1;
+    hipLaunchKernelGGL(route_products_kernel, dim3((T + 63) / 64, ROUTE_SHARES, (Ep + 63) / 64), dim3(256), 0, s, (const bf16raw*)h, (const bf16raw*)w, ws, T, Ep, K, ldh);
+#define KV_RC(NC) hipLaunchKernelGGL((route_choose_kernel<NC>), dim3((T + 3) / 4), dim3(256), (size_t)4 * (Ep + 1) * 4, s, (const float*)ws, a)
+    if (E <= 64) KV_RC(1);
+    else if (E <= 256) KV_RC(4);
+    else KV_RC(16);
+#undef KV_RC
+    return (int)hipGetLastError();
+  }
   const int tl = Ep > 64 && Ep <= 80 ? 5 : 4;  // (64 experts and a shared one: all at a time)
   const size_t lds = ((size_t)16 * (Ep + 1) + 4 + (f32 ? 0 : 16 * 16 * tl * 16)) * 4;
   const dim3 grid((T + 15) / 16);

@@ -77,7 +77,8 @@ int kvl_decode(const void* q_lat, const void* cache, void* lat, float* part, con
 int kvl_up(const void* lat, const void* w, const void* proj, long long ldp, int gate_off, int gate_each, void* out, long long ldo, int o_off, const int* rows, int n_rows, const int* slots, int nh,
            int rk, int vdim, int dvp, float out_scale, int parts, hipStream_t s);
 int kve_route(const void* h, int f32, long long ldh, const void* w, const float* correction, const int* slots, int T, int E, int Ep, int top, int K, int* expert_of, float* weight_of, int scores, float scale, float* shared_of, const float* bias,
-              hipStream_t s);
+              float* ws, hipStream_t s);
+long long kve_route_workspace(int f32, int T, int Ep);
 int kve_group(const int* expert_of, int n_pairs, int E, int bm, int* order, int* tiles, int max_tiles, int* n_tiles, hipStream_t s);
 int kve_rows(const void* w, const void* x, void* y, int f32, int mode, const int* expert_of, int n_pairs, int top, int E, int N, int K, long long ldx, long long ldy, float limit, float slope, float shift, hipStream_t s);
 int kv_expert_panels(const void* Wp, const void* x, void* y, int N, int K, long long ldx, long long ldy, long long x_rows, int mode, float limit, float slope, float shift, int* order, int* tiles, int max_tiles, int* n_tiles,
@@ -498,8 +499,9 @@ std::vector<Tensor> route(Tensor h, Tensor router, Tensor correction, Tensor slo
   rows2d(h, h.scalar_type(), T, K, "route: rows");
   TORCH_CHECK(router.size(0) >= E + shared && (!f || router.size(0) == E + shared), "route: router rows");
   Tensor idx = at::empty({T, top}, h.options().dtype(at::kInt)), wt = at::empty({T, top}, h.options().dtype(at::kFloat)), sg = at::empty({shared ? T : 0}, wt.options());
+  Tensor ws = at::empty({kve_route_workspace(f, (int)T, (int)router.size(0))}, wt.options());
   check(kve_route(h.data_ptr(), f, h.stride(0), router.data_ptr(), f32p(correction, E, "correction"), i32p(slots, T, "slots"), (int)T, (int)E, (int)router.size(0), (int)top, (int)K, (int*)idx.data_ptr(),
-                  (float*)wt.data_ptr(), (int)scores, (float)scale, shared ? (float*)sg.data_ptr() : nullptr, f32p(bias, E, "router bias"), stream()), "route");
+                  (float*)wt.data_ptr(), (int)scores, (float)scale, shared ? (float*)sg.data_ptr() : nullptr, f32p(bias, E, "router bias"), ws.numel() ? (float*)ws.data_ptr() : nullptr, stream()), "route");
   return {idx, wt, sg};
 }
 

@@ -2743,3 +2743,40 @@ def test_expert_panels_at_every_number_of_rows(C, ff, width, gated):
         want = h.bfloat16().float() @ down[e].float().T
         # bf16 rounding of the hidden row (2^-9 relative each, ff independent terms) and of the result
         assert ((y[at] - want).norm(dim=1) / want.norm(dim=1)).max().item() < 1e-2, (e, counts[e])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("experts,top,width,shared", [(8, 2, 64, False), (16, 16, 576, True), (64, 6, 4160, True), (64, 8, 2304, False), (200, 4, 1024, True), (1000, 64, 9216, False)])
+def test_routes_of_every_number_of_rows_and_shares_of_the_width(C, experts, top, width, shared):
+    """Rows that fill no tile of 64, widths of fewer steps than shares, of many and of uneven shares, both forms (two launches up to 1024 rows,
+    one beyond): a row's route is the same in a step of any size."""
+    from kvmini.ops.hip_mixers import layout
+
+    torch.manual_seed(width + experts)
+    n = experts + shared
+    w = (torch.randn(n, width, device=_dev()) / width ** 0.5).bfloat16()
+    packed = layout(torch.bfloat16).router(w)
+    corr, bias = torch.randn(experts, device=_dev()) * 0.1, torch.randn(experts, device=_dev()) * 0.1
+    x = torch.randn(1025, width + 64, device=_dev()).bfloat16()[:, :width]  # (rows further apart than they are long)
+    slots = torch.arange(1025, dtype=torch.int32, device=_dev())
+    slots[5] = -1
+    logits = x.double() @ w.double().T
+    # fp32 sums of exact products, in any order: (width + 1) 2^-24 of the sum of their sizes
+    err = ((width + 1) * 2.0**-24 * (x.double().abs() @ w.double().abs().T)).max().item()
+    score = torch.sigmoid(logits[:, :experts] + bias.double())
+    cut = (score + corr.double()).topk(top, dim=1).values[:, -1:]
+    whole = C.route(x, packed, corr, slots, top, 0, 2.5, shared, bias)
+    for rows in (1, 4, 15, 16, 17, 32, 33, 63, 64, 65, 131, 1024):
+        idx, wt, gate = C.route(x[:rows], packed, corr, slots[:rows].contiguous(), top, 0, 2.5, shared, bias)
+        assert torch.equal(idx, whole[0][:rows]) and torch.equal(wt, whole[1][:rows]) and torch.equal(gate, whole[2][:rows])
+    idx, wt, gate = whole
+    assert (idx[5] == -1).all() and not wt[5].any() and (not shared or gate[5] == 0)
+    live = slots >= 0
+    at = idx[live].long()
+    assert all(len(set(r)) == top for r in at.tolist())
+    got = score[live].gather(1, at)
+    tol = 0.25 * err + 2.0**-20  # a sigmoid's slope is a quarter at most; the rest for its own fp32 rounding and the sum with the correction
+    assert (got + corr.double()[at] >= cut[live] - 2 * tol).all()
+    assert (wt[live].double() - 2.5 * got).abs().max() <= 2.5 * tol
+    if shared:
+        assert (gate[live].double() - torch.sigmoid(logits[live, experts])).abs().max() <= tol
