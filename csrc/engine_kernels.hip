@@ -606,6 +606,75 @@ __global__ __launch_bounds__(64) void rope_kv_write_kernel(unsigned short* __res
   }
 }
 
+// The bf16 form for prompts: a wave does one task of four tokens, whose rows, positions and slots are all in flight together.  With a token a
+// wave the 2048 tokens of a prompt (32 + 8 heads of 128) are 14336 waves of three dependent reads each, and their number is the time.
+// Measured on MI355X, us (a token a wave, four): 512 tokens 6.3, 6.7; 1024 10.9, 9.5; 2048 19.9, 12.8; 4096 32.0, 20.7 (50 and 101 MB of
+// reads and writes for the last two; e4m3 caches the same): from 1024 tokens on (ROPE_ROWS_MIN).
+template <bool KV8>
+__global__ __launch_bounds__(64) void rope_kv_write_rows_kernel(unsigned short* __restrict__ qkv, const int* __restrict__ positions, const float* __restrict__ cos_t,
+                                                                const float* __restrict__ sin_t, void* __restrict__ k_cache, void* __restrict__ v_cache,
+                                                                const int* __restrict__ slot_mapping, int T, int nh, int nkv, int hd, int block_size,
+                                                                const float* __restrict__ kv_scale) {
+  constexpr int R = 4;
+  const int t0 = blockIdx.x * R, tid = blockIdx.y * 64 + threadIdx.x;
+  const int half = hd >> 1, tasks_per_head = half >> 3, width = (nh + 2 * nkv) * hd;
+  const int rot_tasks = (nh + nkv) * tasks_per_head, v_tasks = nkv * (hd >> 3);
+  if (tid >= rot_tasks + v_tasks) return;
+  const bool rot = tid < rot_tasks;
+  const int per = rot ? tasks_per_head : hd >> 3, task = rot ? tid : tid - rot_tasks;
+  const int head = task / per, d0 = (task % per) << 3;  // head: of q and k together, or of v
+  const int col = (rot ? head : nh + nkv + head) * hd + d0;
+  int pos[R], slot[R];
+  bf16x8 a[R], b[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int t = t0 + r < T ? t0 + r : T - 1;
+    pos[r] = positions[t];
+    slot[r] = t0 + r < T ? slot_mapping[t] : -1;
+    a[r] = *reinterpret_cast<const bf16x8*>(qkv + (long long)t * width + col);
+    if (rot) b[r] = *reinterpret_cast<const bf16x8*>(qkv + (long long)t * width + col + half);
+  }
+  const bool keys = rot && head >= nh;
+  const int g = rot ? head - nh : head;
+  const float inv = KV8 && (keys || !rot) ? 1.f / kv_scale[rot ? g : nkv + g] : 1.f;
+  if (rot) {
+    float c[R][8], s[R][8];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        c[r][j] = cos_t[(long long)pos[r] * half + d0 + j];
+        s[r][j] = sin_t[(long long)pos[r] * half + d0 + j];
+      }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      bf16x8 oa, ob;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float x1 = bf2f(a[r][j]), x2 = bf2f(b[r][j]);
+        oa[j] = f2bf(x1 * c[r][j] - x2 * s[r][j]);
+        ob[j] = f2bf(x2 * c[r][j] + x1 * s[r][j]);
+      }
+      a[r] = oa;
+      b[r] = ob;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (rot && !keys) {
+      if (t0 + r < T) {
+        unsigned short* hp = qkv + (long long)(t0 + r) * width + col;
+        *reinterpret_cast<bf16x8*>(hp) = a[r];
+        *reinterpret_cast<bf16x8*>(hp + half) = b[r];
+      }
+    } else if (slot[r] >= 0) {
+      const long long at = (((long long)(slot[r] / block_size) * nkv + g) * block_size + slot[r] % block_size) * hd + d0;
+      kv_store8<KV8>(rot ? k_cache : v_cache, at, a[r], inv);
+      if (rot) kv_store8<KV8>(k_cache, at + half, b[r], inv);
+    }
+  }
+}
+
 // All-reduce over the 4 lanes {l, l^16, l^32, l^48} in the VALU: v_permlane16_swap exchanges the
 // odd 16-lane rows of one register with the even rows of another, v_permlane32_swap the upper
 // half of one with the lower half of the other; fed the same value twice they leave a pair
@@ -3052,6 +3121,7 @@ int kv_add_rmsnorm_slabs(const float* slabs, int n_slabs, long long slab_stride,
   return (int)hipGetLastError();
 }
 
+constexpr int ROPE_ROWS_MIN = 1024;  // tokens: see rope_kv_write_rows_kernel
 static inline int rope_grid_y(int nh, int nkv, int hd) {
   const int tasks = (nh + nkv) * (hd >> 4) + nkv * (hd >> 3);
   return (tasks + 63) / 64;
@@ -3100,6 +3170,15 @@ int kv_rope_kv_write(void* qkv, const int* positions, const float* cos_t, const 
                      int nh, int nkv, int hd, int block_size, const float* kv_scale, hipStream_t stream) {
   if (T <= 0) return 0;
   if (hd % 16) return -1;
+  if (T >= ROPE_ROWS_MIN) {
+    const dim3 grid((T + 3) / 4, rope_grid_y(nh, nkv, hd));
+#define KV_ROPE_ROWS(K8)                                                                                                                                        \
+  hipLaunchKernelGGL((rope_kv_write_rows_kernel<K8>), grid, dim3(64), 0, stream, (unsigned short*)qkv, positions, cos_t, sin_t, k_cache, v_cache, slot_mapping, \
+                     T, nh, nkv, hd, block_size, kv_scale)
+    if (kv_scale) KV_ROPE_ROWS(true); else KV_ROPE_ROWS(false);
+#undef KV_ROPE_ROWS
+    return (int)hipGetLastError();
+  }
 #define KV_ROPE(K8)                                                                                                                                               \
   hipLaunchKernelGGL((rope_kv_write_kernel<false, K8>), dim3(T, rope_grid_y(nh, nkv, hd)), dim3(64), 0, stream, (unsigned short*)qkv, (const float*)nullptr, 0, 0LL, \
                      (unsigned short*)nullptr, positions, cos_t, sin_t, k_cache, v_cache, slot_mapping, nh, nkv, hd, block_size, (const float*)nullptr, 0, 0.f,      \

@@ -2780,3 +2780,29 @@ def test_routes_of_every_number_of_rows_and_shares_of_the_width(C, experts, top,
     assert (wt[live].double() - 2.5 * got).abs().max() <= 2.5 * tol
     if shared:
         assert (gate[live].double() - torch.sigmoid(logits[live, experts])).abs().max() <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,nh,nkv,hd,kv8", [(1024, 32, 8, 128, False), (1025, 4, 2, 64, False), (1026, 7, 1, 16, False), (1027, 32, 8, 128, True), (2047, 8, 8, 64, True)])
+def test_rope_of_many_rows_equals_that_of_few(C, rows, nh, nkv, hd, kv8):
+    """A wave's four tokens, cut off at the end: rows and cache are the bits of calls of 100 rows each."""
+    torch.manual_seed(rows)
+    dev, bs = _dev(), 16
+    qkv = torch.randn(rows, (nh + 2 * nkv) * hd, device=dev).bfloat16()
+    pos = torch.randint(0, 3000, (rows,), dtype=torch.int32, device=dev)
+    cos, sin = torch.randn(3000, hd // 2, device=dev), torch.randn(3000, hd // 2, device=dev)
+    blocks = rows // bs + 2
+    slots = torch.randperm(blocks * bs, device=dev)[:rows].int()
+    slots[::7] = -1
+    slots[-1] = 3 if not (slots == 3).any() else slots[-1]
+    scale = torch.rand(2, nkv, device=dev) + 0.5 if kv8 else None
+    out = []
+    for step in (rows, 100):
+        x = qkv.clone()
+        k, v = (torch.zeros(blocks, nkv, bs, hd, dtype=torch.uint8 if kv8 else torch.bfloat16, device=dev) for _ in range(2))
+        if kv8:
+            k, v = k.view(torch.float8_e4m3fn), v.view(torch.float8_e4m3fn)
+        for i in range(0, rows, step):
+            C.rope_kv_write(x[i : i + step], pos[i : i + step], cos, sin, k, v, slots[i : i + step], nh, nkv, hd, scale)
+        out.append([x] + [c.view(torch.uint8) if kv8 else c for c in (k, v)])
+    assert all(torch.equal(a, b) for a, b in zip(*out))
