@@ -674,8 +674,11 @@ __device__ __attribute__((always_inline)) inline void delta_chain(f4* lds, int y
 
 // grid (heads, dvp / 16, portions).  What bounds a tile's step is what is read of it (25 KB for 128 key channels and 16 columns, from beyond the L2) and
 // the fp32 matrix instructions (0.35 us); its serial chain is about as long.  Two column tiles a workgroup read half as much and leave half the
-// workgroups: taken where one each would be more than two workgroups per CU (measured, 32 heads of 128 x 128: 4 x 512 tokens 109 -> 95 us, 16 x 100 95 -> 84;
-// below, one and two, 2 x 1000 105 and 108, 1 x 2048 133 and 202).  How many portions there are only the device knows.
+// workgroups: taken where one each would be more than two workgroups per CU (measured, us, one and two: 32 heads of 128 x 128, 4 x 512 tokens 109, 95;
+// 16 x 128 121, 104; 16 x 40 57, 55; below 512 workgroups 2 x 1000 105, 108, 1 x 2048 133, 202; 16 heads, 8 x 256 60, 52; 18 x 40 37, 37).  Portions
+// of one tile pay for it (16 x 13 27, 32): the registers of two tiles leave fewer workgroups on a CU, also where one is taken.  The half of the
+// grid that has nothing to do is the upper half of the columns: with every other column idle, 16 heads put all live workgroups on half of an XCD's
+// engines (18 x 40: 54 us).  How many portions there are only the device knows.
 constexpr int CHAIN_WGS = 512;
 template <typename T, int RT>
 __global__ __launch_bounds__(256) void delta_chain_kernel(const float* __restrict__ ws, float* __restrict__ o, const T* __restrict__ proj, T* __restrict__ ring, const int* __restrict__ seg_row,
@@ -688,8 +691,8 @@ __global__ __launch_bounds__(256) void delta_chain_kernel(const float* __restric
   for (int i = threadIdx.x & 63; i - (int)(threadIdx.x & 63) < (int)gridDim.z; i += 64)
     live += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < (int)gridDim.z && seg_n[i] > 0 && seg_n[i] >= min_n));
   if (dvp % 32 == 0 && live * (int)(gridDim.x * gridDim.y) > CHAIN_WGS) {
-    if (blockIdx.y & 1) return;
-    delta_chain<T, RT, 2>(part, blockIdx.y >> 1, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
+    if (blockIdx.y >= gridDim.y / 2) return;
+    delta_chain<T, RT, 2>(part, blockIdx.y, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
   } else {
     delta_chain<T, RT, 1>(part, blockIdx.y, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
   }
