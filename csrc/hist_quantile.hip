@@ -403,11 +403,12 @@ __global__ __launch_bounds__(SEL_THREADS) void select_pass_kernel(const T* __res
     if (c) atomicAdd(&gh[i], c);
   }
   if constexpr (PICK) {
+    // The adds above are asynchronous, and neither the barrier nor a workgroup-scope release waits for them on this target: every wave waits until
+    // its own have been performed, then the barrier, and only then is the arrival counted — whoever sees the full count sees all adds.  No fence:
+    // what the last workgroup reads was written by device-scope atomics alone (a fence would write an XCD's L2 back, from every wave 80 us a pass).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // also a compiler barrier: no add may sink below it
     __syncthreads();
-    if (tid == 0) {  // (one fence a workgroup: each one writes an XCD's L2 back, from every wave they took 80 us a pass)
-      __threadfence();
-      last = atomicAdd(&done[m], 1u) == gridDim.x - 1;
-    }
+    if (tid == 0) last = __hip_atomic_fetch_add(&done[m], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     __syncthreads();
     if (!last) return;
     unsigned int c[PER];
