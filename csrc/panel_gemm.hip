@@ -13,11 +13,11 @@
 // while it issues memory operations.
 //
 // Experts (the (token, choice) pairs that chose one, up to 256 a tile, y[pair] = W[expert] x[row of the pair]) are bound by the matrices: every one is
-// read once (1.2 GB for 64 of 2304 x 4096) for some 100 to 300 rows, so bytes and matrix work take about as long.  They are read past the
-// caches' reuse (nobody else wants them) and every workgroup starts at another column and goes round: panels lie a power of two apart, and in step
-// they would all ask the same memory channels.  (293 -> 262 us; either alone 278 and 292.)
-// Measured, 64 experts of 2304 x 4096 with 187 rows each: 282 us; a tile of 256 x 256 through LDS (all 256 rows multiplied) 338 us.  64 rows: 246
-// against 311 us.
+// read once (1.2 GB for 64 of 2304 x 4096) for some 100 to 300 rows, so bytes and matrix work take about as long.  Every sum goes through the columns
+// from the first to the last, so that a row's outputs do not depend on the tile and panel it falls into, and are those of the tiled kernel.  (Workgroups
+// that start at columns of their own, past the caches' reuse, ask other memory channels at a time and take 3 to 5 % less, but round otherwise.)
+// Measured, gate / up and down of 64 experts of 2304 x 4096 chosen by 187 rows each: 874 us; by tiles of 256 x 256 through LDS, all 256 rows multiplied,
+// 1055; 300 rows 1306 and 2004, 64 rows 685 and 749.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -58,9 +58,7 @@ __device__ inline unsigned int f2bf(float f) {
 __device__ inline uint2 pack4(frag_cd v) { return make_uint2(f2bf(v[0]) | f2bf(v[1]) << 16, f2bf(v[2]) | f2bf(v[3]) << 16); }
 
 __device__ inline rsrc_t buffer_of(const void* p, unsigned int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00027000); }
-enum Caching { REUSED = 0, ONCE = 2 };  // of a load: ONCE is past the caches' reuse
-template <int CACHING>
-__device__ inline raw16 load16(rsrc_t r, int lane_off, int off) { return __builtin_bit_cast(raw16, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, CACHING)); }
+__device__ inline raw16 load16(rsrc_t r, int lane_off, int off) { return __builtin_bit_cast(raw16, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0)); }
 // one LDS-DMA piece: lane l's 16 bytes land at lds + 16 l
 __device__ inline void dma16(rsrc_t r, int lane_off, int off, void* lds) { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, lane_off, off, 0, 0); }
 
@@ -75,8 +73,8 @@ template <class F, int... U>
 __device__ __attribute__((always_inline)) inline void each(const F& f, std::integer_sequence<int, U...>) { (f(std::integral_constant<int, U>{}), ...); }
 
 // acc[i][j] += the wave's feature tile i x rows 16 j .. of NF row tiles (a multiple of two), over n stages of 64 columns
-template <int NF, int CACHING>
-__device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int start, int wave, int lane) {
+template <int NF>
+__device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
   constexpr int AHEAD = ahead(NF), RING = AHEAD + 1, STAGE = NF * 2048;
   static_assert(RING * STAGE <= RING_BYTES, "ring");
   constexpr int PX = (2 * NF + 7) / 8, OPS = 4 + PX;  // pieces of x and memory operations per wave and stage
@@ -96,10 +94,7 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
       b[set][e] = *reinterpret_cast<const frag_ab*>(img + xo[f / NF] + f % NF * 2048);
     }
   };
-  auto column = [&](int s) __attribute__((always_inline)) {  // of stage s (behind the end the last one is fetched again)
-    const int c = (s < n ? s : n - 1) + start;
-    return c < n ? c : c - n;
-  };
+  auto column = [&](int s) __attribute__((always_inline)) { return s < n ? s : n - 1; };  // of stage s (behind the end the last one is fetched again)
   // memory operations behind batch t: pieces of x spread over the stage, weights where those they replace have been multiplied
   auto fetch = [&](int t, int u, int st, unsigned char* dst) __attribute__((always_inline)) {
 #pragma unroll
@@ -108,8 +103,8 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
 #pragma unroll
     for (int k = 0; k < 2; ++k)
       if (t == (k == 0 ? (NF - 1) / 4 : NB - 1)) {
-        w[u][k][0] = load16<CACHING>(wr, w0, st * 2048 + k * 1024);
-        w[u][k][1] = load16<CACHING>(wr, w1, st * 2048 + k * 1024);
+        w[u][k][0] = load16(wr, w0, st * 2048 + k * 1024);
+        w[u][k][1] = load16(wr, w1, st * 2048 + k * 1024);
       }
   };
 #pragma unroll
@@ -170,17 +165,16 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
 }
 
-template <int CACHING>
-__device__ __attribute__((always_inline)) inline void multiply(int nf, frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int start, int wave, int lane) {
+__device__ __attribute__((always_inline)) inline void multiply(int nf, frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
   switch (nf) {
-    case 16: multiply_rows<16, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 14: multiply_rows<14, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 12: multiply_rows<12, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 10: multiply_rows<10, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 8: multiply_rows<8, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 6: multiply_rows<6, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    case 4: multiply_rows<4, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
-    default: multiply_rows<2, CACHING>(acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane); break;
+    case 16: multiply_rows<16>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
+    case 14: multiply_rows<14>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
+    case 12: multiply_rows<12>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
+    case 10: multiply_rows<10>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
+    case 8: multiply_rows<8>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
+    case 6: multiply_rows<6>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
+    case 4: multiply_rows<4>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
+    default: multiply_rows<2>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
   }
 }
 
@@ -267,9 +261,7 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  // (the column a workgroup starts at is its expert's and panel's: which of the expert's tiles a row falls into changes from run to run, its sums must not)
-  const int n = p.K / 64, start = (p.groups.tile_expert[tile] * p.n_panels + panel) * 5 % n;
-  multiply<ONCE>(nf, acc, wr, w0, w1, xr, xsrc, ring, n, start, wave, lane);
+  multiply(nf, acc, wr, w0, w1, xr, xsrc, ring, p.K / 64, wave, lane);
   const int f0 = panel * FEATURES + wave * 32;
   if (f0 >= p.N) return;
   store_rows<MODE>(acc, rows, f0, lane, [](int) { return 1.f; }, [&](float g, float u) { return expert_gate(g, u, p.gate); },
@@ -323,7 +315,7 @@ __global__ __launch_bounds__(512) void dense_panel_kernel(const DenseArgs p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  multiply<REUSED>(nf, acc, wr, w0, w1, xr, xsrc, ring, p.K / 64, 0, wave, lane);
+  multiply(nf, acc, wr, w0, w1, xr, xsrc, ring, p.K / 64, wave, lane);
   if (p.row_ss != nullptr) __syncthreads();
   const int f0 = panel * FEATURES + wave * 32;
   if (f0 >= p.N) return;

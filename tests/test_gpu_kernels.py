@@ -2746,6 +2746,30 @@ def test_expert_panels_at_every_number_of_rows(C, ff, width, gated):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ff,width", [(128, 256), (384, 1024), (1408, 512)])
+def test_expert_panels_add_up_in_the_order_of_the_columns(C, ff, width):
+    """Whatever panel and expert a row falls into, its sums go through the columns from the first to the last: bit for bit what the tiled kernel makes of
+    the expert's rows and matrices alone."""
+    from kvmini.ops.hip_mixers import layout
+
+    counts = [5, 130, 257, 40]
+    torch.manual_seed(ff)
+    expert = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
+    expert = expert[torch.randperm(expert.numel())].to(_dev())
+    lay = layout(torch.bfloat16)
+    up = (torch.randn(len(counts), ff, width, device=_dev()) / width ** 0.5).bfloat16()
+    down = (torch.randn(len(counts), width, ff, device=_dev()) / ff ** 0.5).bfloat16()
+    x = torch.randn(expert.numel(), width, device=_dev()).bfloat16()
+    y = C.expert_outputs(x, expert.int().view(-1, 1), lay.experts(up), lay.experts(down), False, math.inf, 1.0, 0.0, True)
+    for e, n in enumerate(counts):
+        at = (expert == e).nonzero().view(-1)
+        act, want = (torch.empty(n, m, device=_dev(), dtype=torch.bfloat16) for m in (ff, width))
+        C.wide_gemm(C.pack_weight(up[e]), ff, width, x[at].contiguous(), act, 5, 128, 128, 0, 1, width // 64)
+        C.wide_gemm(C.pack_weight(down[e]), width, ff, act, want, 0, 128, 128, 0, 1, ff // 64)
+        assert torch.equal(y[at], want), e
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("experts,top,width,shared", [(8, 2, 64, False), (16, 16, 576, True), (64, 6, 4160, True), (64, 8, 2304, False), (200, 4, 1024, True), (1000, 64, 9216, False)])
 def test_routes_of_every_number_of_rows_and_shares_of_the_width(C, experts, top, width, shared):
     """Rows that fill no tile of 64, widths of fewer steps than shares, of many and of uneven shares, both forms (two launches up to 1024 rows,
