@@ -301,11 +301,12 @@ def _plan_slabs(n_pad: int, k: int, m: int = 32, group_cols: int = 256) -> Tuple
 
 
 # Tiled (wide) GEMM: (token tile, feature tile, pipeline variant) -> measured microseconds per
-# 64-wide K step of one workgroup with every CU busy (Llama-3-8B shapes, 1 x MI355X).  The smaller
-# tiles trade efficiency for more workgroups; 256 x 224 and 256 x 192 (FP8 weights) exist for feature
-# counts whose 256-wide tiles leave a ragged last round over the 256 CUs.  bf16 weights come here
-# only with few outputs (_plan_panels).
-_WIDE_TILES_BF16 = (((256, 128, 0), 0.84), ((128, 256, 0), 0.87), ((128, 128, 0), 0.62), ((256, 64, 0), 0.65))
+# 64-wide K step of one workgroup with every CU busy (Llama-3-8B shapes, 1 x MI355X).  Per FLOP
+# 256 x 256 and 256 x 128 are alike (~1.28 PFLOP/s with every CU busy); the smaller tiles trade
+# efficiency for more workgroups; 256 x 224 and 256 x 192 exist for feature counts whose
+# 256-wide tiles leave a ragged last round over the 256 CUs, whole or with K split (6144 = 32 x 192).
+# bf16 weights come here with few outputs or where K is split (_plan_panels).
+_WIDE_TILES_BF16 = (((256, 256, 1), 1.68), ((256, 224, 1), 1.615), ((256, 192, 0), 1.36), ((256, 128, 0), 0.84), ((128, 256, 0), 0.87), ((128, 128, 0), 0.62), ((256, 64, 0), 0.65))
 _WIDE_TILES_FP8 = (((256, 256, 0), 1.9), ((256, 224, 0), 1.85), ((256, 192, 0), 1.55), ((256, 128, 0), 0.84), ((128, 256, 0), 0.87), ((128, 128, 0), 0.62))
 # The 128-wide tiles move 1.5 x the operand bytes per MAC of the 256-wide ones from L2 into LDS; on
 # grids of many rounds that traffic shows: + this many microseconds per step and round
@@ -372,9 +373,12 @@ PANEL_HEIGHTS = (256, 224, 192, 160, 128, 96)  # rows of a tile (64 and 32: the 
 
 
 @functools.lru_cache(maxsize=None)
-def _plan_panels(m: int, n: int, k: int) -> Optional[Tuple[int, int, int]]:
+def _plan_panels(m: int, n: int, k: int, may_split: bool = False) -> Optional[Tuple[int, int, int]]:
     """How bf16 weights of many outputs are multiplied by panels of 256 features (``csrc/panel_gemm.hip``): (rows of a tile,
     panels cut like that, rows of the tiles of the panels behind them), or None for the tiled GEMM above.
+
+    None where the tiled GEMM would split K (``may_split``: the caller takes slabs): its partial sums reach the consumer in fp32, panels write bf16
+    (2304 outputs of 9216 at 1800 rows, 3072 of 24576 at 1536: single matrices among the wide and flat ones).
 
     None up to one round of 128 x 128 tiles: there what counts is that all CUs have work, and a panel's tile is at least twice as wide
     (measured on MI355X, us, this tiled GEMM and panels: 2048 rows x 2048 x 8192 77 and 89, 512 x 6144 x 4096 41 and 45, 256 x 4096 x 4096
@@ -386,7 +390,7 @@ def _plan_panels(m: int, n: int, k: int) -> Optional[Tuple[int, int, int]]:
     to 1.12 times as fast as the best single one, 1.035 in the mean over 16 sizes (2048 x 28672 x 4096: 372 -> 358 us); with 96 rows behind
     whole rounds it was 0.97 over six others, so that is left out."""
     cus = _num_cus()
-    if -(-m // 128) * -(-n // 128) <= cus:
+    if -(-m // 128) * -(-n // 128) <= cus or (may_split and _plan_wide(m, n, k, 0, True)[3] > 1):
         return None
     panels = -(-n // 256)
 
@@ -427,7 +431,7 @@ def _wide(w: Union[PackedLinear, "_ExpandedView"], h: Union[torch.Tensor, "Norme
         C.wide_gemm_fp8a(w.wp, w.n_pad, w.k, x8, a_scale, out, epi, bm, bn, variant, 1, sps, ss, eps, w.wscale, True)
         n_true = w.n // 2 if epi in GATED else w.n
         return out if n_true == n_out else out[:, :n_true]
-    cut = _plan_panels(m, w.n_pad, w.k) if w.wscale is None and x.data_ptr() % 16 == 0 and w.k <= x.stride(0) < 1 << 22 else None
+    cut = _plan_panels(m, w.n_pad, w.k, may_split) if w.wscale is None and x.data_ptr() % 16 == 0 and w.k <= x.stride(0) < 1 << 22 else None
     if cut is not None:
         out = torch.empty((m, w.n_pad // 2 if epi in GATED else w.n_pad), dtype=torch.bfloat16, device=x.device)
         C.dense_panels(w.wp, w.n_pad, w.k, x, out, epi, *cut, ss, eps)

@@ -555,6 +555,24 @@ def test_gemm_workgroup_planner_fills_the_cus_evenly():
     assert _decode_attention_waves(10, 32) == 4 and _decode_attention_waves(64, 8) == 4
 
 
+@pytest.mark.parametrize("m,n,k", [(1281, 3072, 24576), (2048, 3072, 24576), (1800, 2304, 9216), (900, 4608, 36864), (129, 24576, 9216)])
+def test_products_whose_sums_were_split_stay_in_fp32(monkeypatch, m, n, k):
+    """A consumer that takes slabs gets the fp32 partial sums of a product whose K the tiled GEMM splits, also where it has enough outputs for
+    panels, which round to bf16; a consumer that takes none gets panels."""
+    from kvmini.ops import hip_ops
+
+    monkeypatch.setattr(hip_ops, "_num_cus", lambda: 256)
+    for plan in (hip_ops._plan_wide, hip_ops._plan_panels):
+        plan.cache_clear()
+    assert hip_ops._plan_wide(m, n, k, 0, True)[3] > 1
+    assert hip_ops._plan_panels(m, n, k, True) is None
+    assert hip_ops._plan_panels(m, n, k, False) is not None
+    for n2, k2 in ((28672, 4096), (9216, 4096), (16384, 2048)):  # (whole sums either way)
+        assert hip_ops._plan_wide(2048, n2, k2, 0, True)[3] == 1 and hip_ops._plan_panels(2048, n2, k2, True) == hip_ops._plan_panels(2048, n2, k2)
+    for plan in (hip_ops._plan_wide, hip_ops._plan_panels):
+        plan.cache_clear()
+
+
 def test_unseeded_sampling_rides_the_pipeline():
     """temperature > 0 without a seed is sampled by device ops behind the forward pass, so the
     step after it can still be launched ahead.  top_k = 1 makes sampling deterministic: the

@@ -1860,6 +1860,23 @@ def test_split_kv_decode_attention_matches_the_unsplit_kernel(rep, kv8):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1281, 3072, 24576), (1536, 3072, 24576), (1800, 2304, 9216), (900, 4608, 9216)])
+def test_split_products_reach_their_consumer_in_fp32(m, n, k):
+    """Where the tiled GEMM splits K its slabs are fp32, however many outputs there are: their sum is within fp32 rounding, 2^-20 of the sum of magnitudes
+    (each slab adds products of 32 in up to 384 steps), where a result rounded to bf16 would be within 2^-9 of the value at best."""
+    from kvmini.ops import hip_ops as ops
+
+    torch.manual_seed(n)
+    x = torch.randn(m, k, device="cuda").bfloat16()
+    w = (torch.randn(n, k, device="cuda") * 0.05).bfloat16()
+    got = ops.linear(x, ops.PackedLinear(w), allow_slabs=True)
+    assert isinstance(got, ops.Partial) and got.slabs.dtype == torch.float32 and got.slabs.shape[0] > 1
+    rows = torch.randperm(m)[:64].cuda()
+    xd, wd = x[rows].double(), w.double()
+    assert ((got.slabs.double().sum(0)[rows] - xd @ wd.T).abs() <= 2.0**-20 * (xd.abs() @ wd.abs().T)).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv8,n_split,lengths", [
     ((8, 2), False, 1, [1, 2, 17, 300, 0, 64]), ((2, 2), False, 32, [5, 3000, 16, 0, 257]), ((6, 2), True, 1, [1, 33, 100]), ((8, 2), True, 32, [2500, 15, 0, 900]), ((4, 2), False, 1, [129] * 20),
 ])
