@@ -552,7 +552,9 @@ __global__ __launch_bounds__(256, 3) void delta_tile_kernel(const T* __restrict_
 // A workgroup has 16 CT columns of S and the dkp = 64 RT key channels over four waves (RT row tiles of 16 each).
 // mfma_f32_16x16x4: A lane (row l & 15, k l >> 4), B lane (column l & 15, k l >> 4), D lane rows 4 (l >> 4) + r.  The k order of the
 // products with S is chosen so that an accumulator register is a B operand as it is: step s takes the channels 4 q + s.
-template <typename T, int RT, int CT>
+// LEAN: addresses are scalars and four 32-bit offsets of a lane; as pointers of a lane they take some thirty registers, and a long chain is 2 % faster
+// (1 x 2048 tokens: 251 us, 257).
+template <typename T, int RT, int CT, bool LEAN>
 __device__ __attribute__((always_inline)) inline void delta_chain(f4* lds, int y, int n, const float* __restrict__ ws, float* __restrict__ o, const T* __restrict__ proj, T* __restrict__ ring, const int* __restrict__ seg_row,
                                                                   const int* __restrict__ seg_pos, const int* __restrict__ seg_slot, const int* __restrict__ seg_tile, int dkp, int dvp, const DeltaArgs& a) {
   f4(*part)[4][2 * CT][64] = reinterpret_cast<f4(*)[4][2 * CT][64]>(lds);
@@ -580,21 +582,39 @@ __device__ __attribute__((always_inline)) inline void delta_chain(f4* lds, int y
   // two tiles in flight: a tile's coefficients come from beyond this XCD's L2 the first time, and one tile takes less time than that
   struct Tile { f4 tk[RT], qe[RT], ke[RT], gc[RT], tv[CT]; float ov[CT]; };
   Tile ta, tb;
+  const unsigned int at_row = (lr * dkp + base + 4 * lq) * 4, at_ke = ((base + lr) * 16 + 4 * lq) * 4, at_gc = (base + 4 * lq) * 4, at_col = (4 * lq * dvp + col) * 4;
   auto fetch = [&](Tile& x, int i) __attribute__((always_inline)) {
     const float* p = w + step * (i < nt ? i : nt - 1);
+    if constexpr (LEAN) {
+      auto at = [](const float* from, unsigned int off) __attribute__((always_inline)) { return reinterpret_cast<const char*>(from) + off; };
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      const int d = base + 16 * t;
-      x.tk[t] = *reinterpret_cast<const f4*>(p + lr * dkp + d + 4 * lq);
-      x.qe[t] = *reinterpret_cast<const f4*>(p + (16 + lr) * dkp + d + 4 * lq);
-      x.ke[t] = *reinterpret_cast<const f4*>(p + 32 * dkp + (d + lr) * 16 + 4 * lq);
-      x.gc[t] = *reinterpret_cast<const f4*>(p + 48 * dkp + d + 4 * lq);
-    }
+      for (int t = 0; t < RT; ++t) {
+        x.tk[t] = *reinterpret_cast<const f4*>(at(p, at_row) + 64 * t);
+        x.qe[t] = *reinterpret_cast<const f4*>(at(p + 16 * dkp, at_row) + 64 * t);
+        x.ke[t] = *reinterpret_cast<const f4*>(at(p + 32 * dkp, at_ke) + 1024 * t);
+        x.gc[t] = *reinterpret_cast<const f4*>(at(p + 48 * dkp, at_gc) + 64 * t);
+      }
 #pragma unroll
-    for (int c = 0; c < CT; ++c) {
+      for (int c = 0; c < CT; ++c) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) x.tv[c][r] = p[49 * dkp + (4 * lq + r) * dvp + col + 16 * c];
-      x.ov[c] = p[49 * dkp + (16 + 4 * lq + wave) * dvp + col + 16 * c];
+        for (int r = 0; r < 4; ++r) x.tv[c][r] = *reinterpret_cast<const float*>(at(p + 49 * dkp + r * dvp, at_col) + 64 * c);
+        x.ov[c] = *reinterpret_cast<const float*>(at(p + 49 * dkp + (16 + wave) * dvp, at_col) + 64 * c);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const int d = base + 16 * t;
+        x.tk[t] = *reinterpret_cast<const f4*>(p + lr * dkp + d + 4 * lq);
+        x.qe[t] = *reinterpret_cast<const f4*>(p + (16 + lr) * dkp + d + 4 * lq);
+        x.ke[t] = *reinterpret_cast<const f4*>(p + 32 * dkp + (d + lr) * 16 + 4 * lq);
+        x.gc[t] = *reinterpret_cast<const f4*>(p + 48 * dkp + d + 4 * lq);
+      }
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x.tv[c][r] = p[49 * dkp + (4 * lq + r) * dvp + col + 16 * c];
+        x.ov[c] = p[49 * dkp + (16 + 4 * lq + wave) * dvp + col + 16 * c];
+      }
     }
     __builtin_amdgcn_sched_barrier(0);  // the loads are issued here and not where they are used
   };
@@ -674,28 +694,33 @@ __device__ __attribute__((always_inline)) inline void delta_chain(f4* lds, int y
 
 // grid (heads, dvp / 16, portions).  What bounds a tile's step is what is read of it (25 KB for 128 key channels and 16 columns, from beyond the L2) and
 // the fp32 matrix instructions (0.35 us); its serial chain is about as long.  Two column tiles a workgroup read half as much and leave half the
-// workgroups: taken where one each would be more than two workgroups per CU (measured, us, one and two: 32 heads of 128 x 128, 4 x 512 tokens 109, 95;
-// 16 x 128 121, 104; 16 x 40 57, 55; below 512 workgroups 2 x 1000 105, 108, 1 x 2048 133, 202; 16 heads, 8 x 256 60, 52; 18 x 40 37, 37).  Portions
-// of one tile pay for it (16 x 13 27, 32): the registers of two tiles leave fewer workgroups on a CU, also where one is taken.  The half of the
-// grid that has nothing to do is the upper half of the columns: with every other column idle, 16 heads put all live workgroups on half of an XCD's
-// engines (18 x 40: 54 us).  How many portions there are only the device knows.
-constexpr int CHAIN_WGS = 512;
-template <typename T, int RT>
-__global__ __launch_bounds__(256) void delta_chain_kernel(const float* __restrict__ ws, float* __restrict__ o, const T* __restrict__ proj, T* __restrict__ ring, const int* __restrict__ seg_row,
-                                                          const int* __restrict__ seg_n, const int* __restrict__ seg_pos, const int* __restrict__ seg_slot,
-                                                          const int* __restrict__ seg_tile, int min_n, int dkp, int dvp, DeltaArgs a) {
-  __shared__ __attribute__((aligned(16))) f4 part[2 * 4 * 4 * 64];
+// workgroups.  Measured for 128 x 128, us of a layer's launches for portions, one tile a workgroup and two: 32 heads, 4 x 512 tokens 225, 204; 16 x 128
+// 240, 220; 64 x 20 305, 281; 16 heads, 8 x 256 123, 111; with few workgroups (1 x 2048) the chain alone 133, 202.  For key sizes up to 64 two gain nothing (8 x 256
+// tokens of 32 heads of 64: 99, 104), above 128 their registers leave one workgroup on a CU (16 heads of 256 x 128, 4 x 300: 144, 159).
+// How many portions there are only the device knows, how long they are in the mean the host: with up to a tile for each there might be, they may be
+// many of one tile, which wait for memory and want workgroups beside them (64 x 13: 147, and 165 where the registers are left to the compiler, 142
+// here).  So WGS is the workgroups a CU holds: 0, one column tile each, as the registers allow; 3, two where they are more than two workgroups per CU
+// (as many as that are dealt out unevenly when three find room: 4 x 256 tokens 128 against 122 by one); 2, two where they are more than one (at 513
+// to 768 of one tile that costs 3 %: 3 x 683 226, 234).  The half of the grid that has nothing to do is the upper half of the columns: with every
+// other column idle, 16 heads put all live workgroups on half of an XCD's engines.
+template <typename T, int RT, int WGS>
+__global__ __launch_bounds__(256, WGS == 3 ? 3 : 1) void delta_chain_kernel(const float* __restrict__ ws, float* __restrict__ o, const T* __restrict__ proj, T* __restrict__ ring,
+                                                                            const int* __restrict__ seg_row, const int* __restrict__ seg_n, const int* __restrict__ seg_pos,
+                                                                            const int* __restrict__ seg_slot, const int* __restrict__ seg_tile, int min_n, int dkp, int dvp, DeltaArgs a) {
+  __shared__ __attribute__((aligned(16))) f4 part[2 * 4 * (WGS ? 4 : 2) * 64];
   const int n = seg_n[blockIdx.z];
   if (n == 0 || n < min_n) return;
-  int live = 0;
-  for (int i = threadIdx.x & 63; i - (int)(threadIdx.x & 63) < (int)gridDim.z; i += 64)
-    live += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < (int)gridDim.z && seg_n[i] > 0 && seg_n[i] >= min_n));
-  if (dvp % 32 == 0 && live * (int)(gridDim.x * gridDim.y) > CHAIN_WGS) {
-    if (blockIdx.y >= gridDim.y / 2) return;
-    delta_chain<T, RT, 2>(part, blockIdx.y, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
-  } else {
-    delta_chain<T, RT, 1>(part, blockIdx.y, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
+  if constexpr (WGS > 0) {
+    int live = 0;
+    for (int i = threadIdx.x & 63; i - (int)(threadIdx.x & 63) < (int)gridDim.z; i += 64)
+      live += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < (int)gridDim.z && seg_n[i] > 0 && seg_n[i] >= min_n));
+    if (live * (int)(gridDim.x * gridDim.y) > (WGS == 3 ? 1024 : 512)) {
+      if (blockIdx.y >= gridDim.y / 2) return;
+      delta_chain<T, RT, 2, WGS == 3>(part, blockIdx.y, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
+      return;
+    }
   }
+  delta_chain<T, RT, 1, WGS == 3>(part, blockIdx.y, n, ws, o, proj, ring, seg_row, seg_pos, seg_slot, seg_tile, dkp, dvp, a);
 }
 
 }  // namespace
@@ -786,8 +811,8 @@ int kvd_tile_dkp(int dim) { return dim <= 64 ? 64 : dim <= 128 ? 128 : dim <= 25
 long long kvd_tile_floats(int dkp, int dvp) { return tile_floats(dkp, dvp); }
 
 // tiles: int32 [4, tile_stride]: first row, tokens (0 = unused), first position, slot of up to 16 tokens, the first n_tiles in use;
-// segs: int32 [5, n_segs]: ... and the portion's first tile.  ws: n_tiles * heads * kvd_tile_floats floats.
-int kvd_tiles(const KvdArgs* k, const void* proj, const void* low, void* ring, int f32, const int* tiles, int tile_stride, int n_tiles, const int* segs, int n_segs, int min_n, float* ws,
+// segs: int32 [5, n_segs]: ... and the portion's first tile; T: rows of the step.  ws: n_tiles * heads * kvd_tile_floats floats.
+int kvd_tiles(const KvdArgs* k, const void* proj, const void* low, void* ring, int f32, const int* tiles, int tile_stride, int n_tiles, const int* segs, int n_segs, int min_n, int T, float* ws,
               float* o, hipStream_t s) {
   const int dkp = bad(*k) ? 0 : kvd_tile_dkp(k->dim);
   if (dkp == 0 || n_tiles <= 0 || n_tiles > tile_stride || n_segs <= 0) return -1;
@@ -812,11 +837,13 @@ int kvd_tiles(const KvdArgs* k, const void* proj, const void* low, void* ring, i
   int rc = (int)hipGetLastError();
   if (rc) return rc;
   const dim3 grid(a.heads, dvp / 16, n_segs);
-#define KV_CH(Tt, RT) hipLaunchKernelGGL((delta_chain_kernel<Tt, RT>), grid, dim3(256), 0, s, ws, o, (const Tt*)proj, (Tt*)ring, row, n, pos, slot, first, min_n, dkp, dvp, a)
-#define KV_CH2(RT) do { if (f32) KV_CH(float, RT); else KV_CH(bf16raw, RT); } while (0)
-  if (dkp == 64) KV_CH2(1);
-  else if (dkp == 128) KV_CH2(2);
-  else KV_CH2(4);
+#define KV_CH(Tt, RT, WGS) hipLaunchKernelGGL((delta_chain_kernel<Tt, RT, WGS>), grid, dim3(256), 0, s, ws, o, (const Tt*)proj, (Tt*)ring, row, n, pos, slot, first, min_n, dkp, dvp, a)
+#define KV_CH2(RT, WGS) do { if (f32) KV_CH(float, RT, WGS); else KV_CH(bf16raw, RT, WGS); } while (0)
+  if (dkp == 64) KV_CH2(1, 0);
+  else if (dkp == 256) KV_CH2(4, 0);
+  else if (dvp % 32) KV_CH2(2, 0);
+  else if (T <= 16 * (long long)n_segs) KV_CH2(2, 3);
+  else KV_CH2(2, 2);
 #undef KV_CH2
 #undef KV_CH
   return (int)hipGetLastError();

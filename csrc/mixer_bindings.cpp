@@ -107,7 +107,7 @@ int kvc_decode(const void* q, const void* proj, long long ldp, int q_off, int k_
 int kvd_step(const KvdArgs* k, const void* proj, const void* low, void* ring, void* out, int f32, const int* row_list, int n_rows, hipStream_t s);
 int kvd_tile_dkp(int dim);
 long long kvd_tile_floats(int dkp, int dvp);
-int kvd_tiles(const KvdArgs* k, const void* proj, const void* low, void* ring, int f32, const int* tiles, int tile_stride, int n_tiles, const int* segs, int n_segs, int min_n, float* ws,
+int kvd_tiles(const KvdArgs* k, const void* proj, const void* low, void* ring, int f32, const int* tiles, int tile_stride, int n_tiles, const int* segs, int n_segs, int min_n, int T, float* ws,
               float* o, hipStream_t s);
 int kvd_prep(const KvdArgs* k, const void* proj, const void* low, const void* ring, int f32, float* qn, float* kn, float* vv, float* dec, float* beta, int dimp, int min_kind, int T,
              hipStream_t s);
@@ -606,7 +606,7 @@ struct DeltaLayer {
       const int64_t dvp = (k.vdim + 15) / 16 * 16;
       Tensor ws = at::empty({n_tiles * k.heads * (int64_t)kvd_tile_floats(kvd_tile_dkp(k.dim), (int)dvp)}, fo), oc = at::empty({T, k.heads, k.vdim}, fo);
       check(kvd_tiles(&a, proj.data_ptr(), low.data_ptr(), ring.data_ptr(), f, i32p(tiles, 4 * n_tiles, "tiles"), (int)tiles.size(1), (int)n_tiles, i32p(segs, 5 * n_segs, "segs"), (int)n_segs,
-                      (int)min_n, (float*)ws.data_ptr(), (float*)oc.data_ptr(), stream()), "delta tiles");
+                      (int)min_n, (int)T, (float*)ws.data_ptr(), (float*)oc.data_ptr(), stream()), "delta tiles");
       check(kvd_out(&a, (const float*)oc.data_ptr(), low.data_ptr(), out.data_ptr(), f, (int)min_n, (int)T, stream()), "delta out");
       return;
     }

@@ -190,6 +190,44 @@ def test_delta_portions_together_equal_each_alone(heads, dim, vdim):
         at += n
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,dim,vdim,lens", [(32, 128, 128, [16, 2, 13, 33, 9]), (32, 100, 96, [5] * 12), (8, 128, 256, [40, 16, 3, 64, 17, 31, 2, 15, 16]), (24, 128, 80, [16] * 9), (16, 256, 128, [20] * 9)])
+def test_delta_portions_among_many_that_could_be(heads, dim, vdim, lens):
+    """The portion table of an engine, most of it idle and idle entries in between: a step of fewer rows than a tile for each entry takes the kernel for
+    many short portions.  Outputs and states are those of each portion in a table of its own, bit for bit."""
+    device, mx = torch.device("cuda:0"), mixers_of(torch.device("cuda:0"))
+    m = hybrid.DeltaSpec(heads, heads, dim, vdim, 4)
+    gen = torch.Generator().manual_seed(dim + len(lens))
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    offs = [0, heads * dim, 2 * heads * dim, 2 * heads * dim + heads * vdim]
+    f = lambda x: x.float().contiguous().to(device)  # noqa: E731
+    w = hybrid.DeltaWeights(*offs, 0, 0, 0, heads * dim, 0, None, f(0.3 * rnd(4, m.channels)), f(rnd(heads) - 2), f(rnd(heads * dim) - 2), f(rnd(vdim)))
+    proj, low = [rnd(n, offs[3] + heads).bfloat16() for n in lens], [rnd(n, heads * (dim + vdim)).bfloat16() for n in lens]
+
+    def run(which, table):
+        state, ring = torch.full((len(lens) + 1, heads, dim, vdim), 7.0, device=device), torch.zeros(len(lens) + 1, 4, m.channels, dtype=torch.bfloat16, device=device)
+        ds = mx.DeltaState(m, w, 1.0, 1e-5, state, ring)
+        st = make_step(mx, [(lens[i], 0, i + 1) for i in which], device, n_blocks=240)
+        if table:
+            wide = torch.zeros(5, table, dtype=torch.int32, device=device)
+            wide[:, (torch.arange(len(which), device=device) * 7 + 3) % table] = st.portions
+            st.portions = wide
+        n = sum(lens[i] for i in which)
+        x, lo = (torch.zeros(st.rows, v[0].shape[1], dtype=torch.bfloat16, device=device) for v in (proj, low))
+        x[:n], lo[:n] = torch.cat([proj[i] for i in which]).to(device), torch.cat([low[i] for i in which]).to(device)
+        mix = torch.zeros(st.rows, heads * vdim, dtype=torch.bfloat16, device=device)
+        ds.run(x, lo, mix, st)
+        return mix[:n], state
+
+    for table in (64, 100):
+        together, state = run(range(len(lens)), table)
+        at = 0
+        for i, n in enumerate(lens):
+            alone, one = run([i], 0)
+            assert torch.equal(together[at : at + n], alone) and torch.equal(state[i + 1], one[i + 1]), (table, i)
+            at += n
+
+
 @pytest.mark.parametrize("backend", BACKENDS)
 @pytest.mark.parametrize("heads,kv,dim,vdim,taps,strong", [(4, 2, 24, 16, 3, 0.0), (2, 2, 128, 128, 4, 0.0), (3, 1, 40, 6, 1, 3.0), (4, 4, 28, 36, 2, 4.0), (2, 1, 200, 48, 6, 1.0), (8, 2, 64, 256, 4, 0.0), (2, 2, 256, 128, 3, 0.0), (1, 1, 260, 64, 4, 0.0)])
 def test_delta_rule_alone(backend, heads, kv, dim, vdim, taps, strong):
