@@ -2636,16 +2636,20 @@ __global__ __launch_bounds__(256) void embed_fed_kernel(const unsigned short* __
   }
 }
 
-// rows idx[i] of x (bf16, H columns) and of its sums of squares (fp32, `parts`; none: null), in one launch.  One workgroup per row.
+// rows idx[i] of x (bf16, H columns) and of its sums of squares (fp32, `parts`; none: null), in one launch.  One workgroup per row.  An index outside x
+// gives a row of NaN: nothing is read there, and what comes of it cannot pass for a result.
 __global__ __launch_bounds__(256) void select_rows_kernel(const unsigned short* __restrict__ x, long long ldx, const float* __restrict__ ss, int parts, const int* __restrict__ idx, int T,
                                                           unsigned short* __restrict__ out, float* __restrict__ out_ss, int H) {
   const int i = blockIdx.x, r = idx[i];
-  if (r < 0 || r >= T) return;
-  const bf16x8* src = reinterpret_cast<const bf16x8*>(x + r * ldx);
+  const bool inside = r >= 0 && r < T;
+  const bf16x8* src = reinterpret_cast<const bf16x8*>(x + (inside ? r : 0) * ldx);
   bf16x8* dst = reinterpret_cast<bf16x8*>(out + (long long)i * H);
   if (ss != nullptr)
-    for (int p = threadIdx.x; p < parts; p += 256) out_ss[(long long)i * parts + p] = ss[(long long)r * parts + p];
-  for (int c = threadIdx.x; c < (H >> 3); c += 256) dst[c] = src[c];
+    for (int p = threadIdx.x; p < parts; p += 256) out_ss[(long long)i * parts + p] = inside ? ss[(long long)r * parts + p] : __builtin_nanf("");
+  bf16x8 nan;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) nan[j] = 0x7fc0;
+  for (int c = threadIdx.x; c < (H >> 3); c += 256) dst[c] = inside ? src[c] : nan;
 }
 
 // y[t] = bf16(x[t] / rms(x[t])) from the per-row partial sums of squares of the residual
@@ -3563,7 +3567,7 @@ int kv_embed_fed(const void* table, const int* tokens, const int* feed, const lo
   return (int)hipGetLastError();
 }
 
-// out[i] = x[idx[i]] of [T, H] (bf16, rows of whole 16-byte pieces) for n rows, and out_ss[i] = ss[idx[i]] of [T, parts] (ss null: none); rows outside x are left
+// out[i] = x[idx[i]] of [T, H] (bf16, rows of whole 16-byte pieces) for n rows, and out_ss[i] = ss[idx[i]] of [T, parts] (ss null: none); NaN for indices outside x
 int kv_select_rows(const void* x, long long ldx, const float* ss, int parts, const int* idx, int n, int T, void* out, float* out_ss, int H, hipStream_t stream) {
   if (n <= 0) return 0;
   if (T <= 0 || H <= 0 || (H & 7) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)out & 15) || (ss != nullptr && (parts < 1 || out_ss == nullptr))) return -1;

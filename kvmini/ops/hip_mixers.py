@@ -113,7 +113,9 @@ def _sine_turns(width: int, device: torch.device) -> torch.Tensor:
 
 
 def select_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
-    return native().select_rows(x, None, idx)[0] if x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0 and x.stride(1) == 1 else torch.index_select(x, 0, idx)
+    from .hip_ops import rows_in_pieces
+
+    return native().select_rows(x, None, idx)[0] if rows_in_pieces(x, idx) else torch.index_select(x, 0, idx)
 
 
 def embed_stream(table: torch.Tensor, tokens: torch.Tensor, feed: torch.Tensor, prev_ids: torch.Tensor, ld: int, scale: float = 1.0, positions: Optional[torch.Tensor] = None,

@@ -847,7 +847,16 @@ def embed_residual(table: torch.Tensor, tokens: torch.Tensor, feed: torch.Tensor
     return Normed(out, ss, eps), out
 
 
+def rows_in_pieces(x: torch.Tensor, idx: torch.Tensor) -> bool:
+    """What the row selection kernel takes: bf16 rows of whole 16-byte pieces that start at such, int32 indices."""
+    return (x.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and idx.dtype == torch.int32 and idx.dim() == 1 and idx.is_contiguous())
+
+
 def select_rows(h: Normed, idx: torch.Tensor) -> Normed:
+    """Rows ``idx``; those outside ``h`` are NaN (indices of other types: ``index_select``, which refuses them)."""
+    if not rows_in_pieces(h.x, idx) or not h.ss.is_contiguous():
+        return Normed(torch.index_select(h.x, 0, idx), torch.index_select(h.ss, 0, idx), h.eps)
     x, ss = native().select_rows(h.x, h.ss, idx)
     return Normed(x, ss, h.eps)
 

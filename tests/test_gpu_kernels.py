@@ -1933,6 +1933,24 @@ def test_embedding_with_its_sums_and_chosen_rows_equal_the_launches_they_stand_f
 
 
 @pytest.mark.gpu
+def test_chosen_rows_outside_and_of_other_forms(C):
+    """An index outside the rows gives NaN, never what the memory held; rows that are no whole 16-byte pieces and 64-bit indices are taken as before."""
+    from kvmini.ops import hip_mixers, hip_ops
+
+    torch.manual_seed(0)
+    x, ss = torch.randn(6, 64, device="cuda").bfloat16(), torch.rand(6, 1, device="cuda")
+    idx = torch.tensor([5, -1, 0, 6, 2**31 - 1], device="cuda", dtype=torch.int32)
+    for sel, part in (C.select_rows(x, ss, idx), (hip_mixers.select_rows(x, idx), None)):
+        assert torch.equal(sel[[0, 2]], x[[5, 0]]) and sel[[1, 3, 4]].isnan().all()
+        assert part is None or (torch.equal(part[[0, 2]], ss[[5, 0]]) and part[[1, 3, 4]].isnan().all())
+    good = torch.tensor([5, 0, 5], device="cuda")
+    for rows in (x, x[:, 4:60], torch.randn(6, 20, device="cuda").bfloat16(), torch.randn(6, 8, device="cuda").bfloat16().t().contiguous().t()):
+        for i in (good, good.int()):
+            got = hip_ops.select_rows(hip_ops.Normed(rows, ss, 1e-5), i)
+            assert torch.equal(got.x, rows[good]) and torch.equal(got.ss, ss[good]) and torch.equal(hip_mixers.select_rows(rows, i), rows[good])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,longest", [(1, 4000), (63, 300), (64, 1100), (65, 1100), (127, 1500)])
 def test_split_kv_shares_cover_every_row_once(rows, longest):
     """Ranges of the launch's fair share and of the least one, rows on both sides of a wave's width, padding rows in between: each row's blocks are
