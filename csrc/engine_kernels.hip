@@ -2111,9 +2111,10 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   int t = bx, listed = bx, z = 0, eff = 1, ctx;
   if constexpr (SPLIT) {
     // Which (row, share of its blocks) is workgroup bx of this kv head's?  Every wave reads all lengths, the shares follow from them.
-    auto length = [&](int i) __attribute__((always_inline)) {  // (-1: not in use)
+    constexpr int UNUSED = (int)0x80000000;
+    auto length = [&](int i) __attribute__((always_inline)) {
       const int r = i >= n_rows ? -1 : ATTN ? row_list[i] : i;
-      return r < 0 ? -1 : ctx_lens[r];
+      return r < 0 ? UNUSED : ctx_lens[r];
     };
     auto blocks = [&](int c) __attribute__((always_inline)) { return c > !ATTN ? (c - !ATTN + BS - 1) / BS : 0; };
     const int c0 = length(lane);
@@ -2125,7 +2126,7 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
     int left = bx, base = 0;
     for (;; base += 64) {
       if (base >= n_rows) return;
-      const int c = base ? length(base + lane) : c0, e = c < 0 ? 0 : max(1, min(n_z, (blocks(c) + up) / share));
+      const int c = base ? length(base + lane) : c0, e = c == UNUSED ? 0 : max(1, min(n_z, (blocks(c) + up) / share));
       const int sum = wave_running_sum(e);
       const unsigned long long past = __builtin_amdgcn_ballot_w64(sum > left);
       if (past != 0) {

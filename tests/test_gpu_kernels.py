@@ -1951,6 +1951,29 @@ def test_chosen_rows_outside_and_of_other_forms(C):
 
 
 @pytest.mark.gpu
+def test_split_kv_rows_without_context_are_zero():
+    """A length of zero or less is a padding row's: zeros, in shares as by one workgroup per pair, whatever the output held."""
+    from kvmini.models.llama import LlamaConfig, rope_tables
+    from kvmini.ops import hip_ops
+
+    torch.manual_seed(3)
+    dev, nkv, rep, hd, bs = _dev(), 2, 4, 128, 16
+    ctx = torch.tensor([700, -1, 0, -16, 40], device=dev, dtype=torch.int32)
+    cos, sin = rope_tables(LlamaConfig(head_dim=hd), 700, dev)
+    bt = torch.arange(5 * 44, device=dev).view(5, 44).int()
+    pos = (ctx - 1).clamp(min=0)
+    slots = torch.where(ctx > 0, bt[torch.arange(5, device=dev), (pos // bs).long()] * bs + pos % bs, -1).int()
+    part = hip_ops.Partial(torch.randn(2, 5, (rep * nkv + 2 * nkv) * hd, device=dev) * 0.4, torch.rand(5, 1, device=dev) * 512 + 1.0, 1e-5, 512)
+    k, v = (torch.randn(5 * 44, nkv, bs, hd, device=dev).bfloat16() for _ in range(2))
+    seq = torch.arange(5, device=dev, dtype=torch.int32)
+    for n_split in (1, 32):
+        junk = torch.full((5, rep * nkv * hd), 9.0, device=dev, dtype=torch.bfloat16)  # (what the allocator gives again)
+        del junk
+        out = hip_ops.rope_attention_fused(part, pos, cos, sin, k.clone(), v.clone(), slots, bt, seq, ctx, rep * nkv, hd**-0.5, n_split=n_split)
+        assert not out[ctx <= 0].any() and out[ctx > 0].any(1).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,longest", [(1, 4000), (63, 300), (64, 1100), (65, 1100), (127, 1500)])
 def test_split_kv_shares_cover_every_row_once(rows, longest):
     """Ranges of the launch's fair share and of the least one, rows on both sides of a wave's width, padding rows in between: each row's blocks are
