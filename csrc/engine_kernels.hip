@@ -3439,21 +3439,18 @@ int kv_decode_attention_fused(const float* slabs, int n_slabs, long long slab_st
   } else {                                                                                     \
     if (kv_scale) { KV_LAUNCH_64(R, W, true, false); } else { KV_LAUNCH_64(R, W, false, false); } \
   }
-#define KV_LAUNCH_64W(R)                      \
-  if (waves == 8) {                           \
-    KV_LAUNCH_64K(R, ((R) <= 4 ? 8 : 4));     \
-  } else {                                    \
-    KV_LAUNCH_64K(R, 4);                      \
+#define KV_LAUNCH_64W(R)  \
+  if (waves == 8) {       \
+    KV_LAUNCH_64K(R, 8);  \
+  } else {                \
+    KV_LAUNCH_64K(R, 4);  \
   }
-  if (hd == 64) {
+  if (hd == 64) {  // (wider groups are as fast in two launches: supports_fused_decode_attention)
     switch (rep) {
       case 1: KV_LAUNCH_64W(1); break;
       case 2: KV_LAUNCH_64W(2); break;
       case 3: KV_LAUNCH_64W(3); break;
       case 4: KV_LAUNCH_64W(4); break;
-      case 6: KV_LAUNCH_64W(6); break;
-      case 7: KV_LAUNCH_64W(7); break;
-      case 8: KV_LAUNCH_64W(8); break;
       default: return -1;
     }
     return (int)hipGetLastError();

@@ -505,9 +505,9 @@ std::vector<Tensor> route(Tensor h, Tensor router, Tensor correction, Tensor slo
   return {idx, wt, sg};
 }
 
-// The chosen experts' outputs, one row per pair: [T * top, K of gate_up].  gate_up [E, 2 ffp, K] (gated) or [E, ffp, K] (squared relu), down [E, K, ffp].  tile: rows per tile of the
-// grouped products (64, 128 or 256), 0: the few-row kernels (bf16: at most 128 tokens).
-// grouped: the pairs are sorted by expert and multiplied in tiles (many rows, bf16); else workgroups look their expert's rows up themselves
+// The chosen experts' outputs, one row per pair: [T * top, K of gate_up].  gate_up [E, 2 ffp, K] (gated) or [E, ffp, K] (squared relu), down [E, K, ffp].
+// grouped: the pairs are sorted by expert and multiplied in tiles (many rows, bf16); else workgroups look their expert's rows up themselves (bf16: at most
+// 128 tokens)
 Tensor expert_outputs(Tensor h, Tensor idx, Tensor gate_up, Tensor down, bool gated, double limit, double slope, double shift, bool grouped) {
   const bool f = is_f32(h);
   const int64_t T = h.size(0), top = idx.size(1), P = T * top, E = gate_up.size(0), N = gate_up.size(1), K = gate_up.size(2), ffp = gated ? N / 2 : N;

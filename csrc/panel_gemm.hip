@@ -153,13 +153,9 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
     slot = next;
   };
   int s = 0;
-  for (; s + AHEAD <= n; s += AHEAD) {
+  static_assert(AHEAD * NB % 2 == 0, "a round of stages leaves the fragments' two sets as they were");
+  for (; s + AHEAD <= n; s += AHEAD)
     each([&](auto uc) __attribute__((always_inline)) { stage(uc, std::true_type{}, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD>{});
-    if constexpr ((AHEAD * NB) & 1) {  // (an odd number of batches: the sets have swapped)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) { const frag_ab v = b[0][e]; b[0][e] = b[1][e]; b[1][e] = v; }
-    }
-  }
   // (the last stages fetch nothing: the compiler would drop loads of weights that no stage multiplies, and the counts be wrong)
   each([&](auto uc) __attribute__((always_inline)) { if (s + decltype(uc)::value < n) stage(uc, std::false_type{}, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD - 1>{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
