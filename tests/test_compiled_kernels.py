@@ -1,15 +1,68 @@
-"""What the compiled kernels must have and no run shows reliably — waits, registers, spills — read from the assembly, which needs no GPU."""
+"""What the compiled kernels must have and no run shows reliably — waits, counts of operations in flight, registers — read from the
+built library's gfx950 code, which needs no GPU."""
 
 import os
 import re
 import shutil
+import struct
 import subprocess
 
 import pytest
 
 import build_native
 
-pytestmark = pytest.mark.skipif(shutil.which(build_native.HIPCC) is None, reason="no hipcc")
+TOOLS = os.path.join(build_native.ROCM, "llvm", "bin")
+pytestmark = pytest.mark.skipif(shutil.which(os.path.join(TOOLS, "llvm-objdump")) is None or not build_native.ext_path().exists(), reason="no library or no tools to read it")
+
+
+@pytest.fixture(scope="module")
+def code_objects(tmp_path_factory):
+    """Files of the device code, one for each source."""
+    data, files, folder = build_native.ext_path().read_bytes(), [], tmp_path_factory.mktemp("code")
+    for bundle in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data):
+        at, entry = bundle.start(), bundle.start() + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            offset, size, name = struct.unpack_from("<QQQ", data, entry)
+            entry += 24 + name
+            if size:
+                files.append(folder / f"{len(files)}.o")
+                files[-1].write_bytes(data[at + offset : at + offset + size])
+    return files
+
+
+def read(tool, *args):
+    return subprocess.run([os.path.join(TOOLS, tool), *map(os.fspath, args)], check=True, capture_output=True, text=True).stdout
+
+
+@pytest.fixture(scope="module")
+def functions(code_objects):
+    """``functions(part)``: {mangled name: instructions} of the kernels whose names hold ``part``."""
+
+    def of(part):
+        found = {}
+        for file in code_objects:
+            names = [line.split()[-1] for line in read("llvm-objdump", "-t", file).splitlines() if " F .text" in line and part in line]
+            body = None
+            for line in read("llvm-objdump", "-d", "--no-show-raw-insn", f"--disassemble-symbols={','.join(names)}", file).splitlines() if names else ():
+                label = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+                if label:
+                    body = found.setdefault(label.group(1), [])
+                elif line.startswith("\t"):
+                    body.append(line.split("//")[0].strip())
+        return found
+
+    return of
+
+
+@pytest.fixture(scope="module")
+def resources(code_objects):
+    """{mangled name: (registers, spilled registers, bytes of scratch, bytes of LDS)} of all kernels."""
+    found = {}
+    for file in code_objects:
+        for entry in re.split(r"\n\s+- (?=\.agpr_count)", read("llvm-readelf", "--notes", file))[1:]:
+            field = lambda name: re.search(rf"\.{name}:\s+(\S+)", entry).group(1)  # noqa: B023, E731
+            found[field("name")] = tuple(int(field(n)) for n in ("vgpr_count", "vgpr_spill_count", "private_segment_fixed_size", "group_segment_fixed_size"))
+    return found
 
 
 def unwaited_arrivals(body):
@@ -26,7 +79,7 @@ def unwaited_arrivals(body):
     return bad
 
 
-def test_the_check_itself():
+def test_unwaited_arrivals_are_found():
     add, barrier, arrive = "global_atomic_add v[2:3], v1, off", "s_barrier", "global_atomic_add v1, v1, v2, s[10:11] sc0"
     assert unwaited_arrivals([add, "s_waitcnt lgkmcnt(0)", barrier, arrive]) == [3]
     assert unwaited_arrivals([add, "s_waitcnt lgkmcnt(0)", barrier, "s_waitcnt vmcnt(0)", arrive]) == [4]  # (one wave's wait: too late)
@@ -34,46 +87,77 @@ def test_the_check_itself():
     assert unwaited_arrivals([add, "s_waitcnt vmcnt(0) lgkmcnt(0)", barrier, arrive]) == []
 
 
-def assembly(tmp_path, source):
-    asm = tmp_path / "kernels.s"
-    subprocess.run([build_native.HIPCC, f"--offload-arch={build_native.ARCH}", *build_native.DEVICE_FLAGS, "-O3", "-std=c++17", *build_native.SOURCE_FLAGS.get(source, []), "-S", "--cuda-device-only",
-                    str(build_native.CSRC / source), "-o", os.fspath(asm)], check=True, capture_output=True)
-    return asm.read_text()
+def test_every_wave_waits_before_an_arrival_is_counted(functions):
+    """Workgroups that count themselves as finished — with a pass of the exact quantiles, with their share of a decode step's keys, with their part of
+    a split product: every wave waits for what it wrote or added before the barrier behind which the arrival is counted."""
+    for part, least in (("select_pass_kernel", 2), ("decode_attention_fused_kernel", 8), ("stream_gemm", 1)):
+        arriving = {n: b for n, b in functions(part).items() if any(re.match(r"global_atomic_add\b.*\bsc0\b", line) for line in b)}
+        assert len(arriving) >= least, part
+        assert {n: unwaited_arrivals(b) for n, b in arriving.items()} == {n: [] for n in arriving}
 
 
-def resources(text):
-    """{mangled name: (registers, spilled registers, LDS bytes)} of an assembly's kernels."""
-    found = {}
-    for entry in re.split(r"\n  - (?=\.agpr_count)", text[text.index("amdhsa.kernels:") :])[1:]:
-        field = lambda name: re.search(rf"\.{name}:\s+(\S+)", entry).group(1)  # noqa: B023, E731
-        found[field("name")] = (int(field("vgpr_count")), int(field("vgpr_spill_count")), int(field("group_segment_fixed_size")))
+def test_the_delta_chain_keeps_its_workgroups_on_a_compute_unit(resources):
+    """Kernels of one column tile have the registers of one (a SIMD has 512, a workgroup of four waves one on each): 4, 3 and 2 workgroups for keys of up
+    to 64, 128 and 256 channels; the one that may take two tiles of many short portions has room for 3.  None spills."""
+    kernels = {n: r for n, r in resources.items() if "delta_chain_kernel" in n}
+    want = {"Li1ELi0E": 4, "Li2ELi0E": 3, "Li4ELi0E": 2, "Li2ELi3E": 3, "Li2ELi2E": 2}
+    assert len(kernels) == 2 * len(want)  # of bf16 and fp32 rows
+    for name, (registers, spilled, _scratch, lds) in kernels.items():
+        workgroups = next(w for form, w in want.items() if form in name)
+        assert min(512 // (-(-registers // 8) * 8), 160 * 1024 // lds) >= workgroups and spilled == 0, (name, registers, spilled, lds)
+
+
+def test_panels_have_in_flight_what_they_wait_for(functions):
+    """The products by panels wait for a stage by the number of operations issued behind it.  In the loop of each height that is a count of its own, and
+    from one barrier to the next exactly a stage's loads are issued: four of weights, and the pieces of rows."""
+    loads = {14: 8, 22: 8, 26: 7, 33: 7, 28: 6, 23: 5, 20: 5}  # {operations that may be in flight: a stage's}, 256 rows to 32
+    kernels = functions("panel_kernel")
+    assert len(kernels) == 6
+    for name, body in kernels.items():
+        before, issued, seen = -1, 0, set()
+        for i, line in enumerate(body):
+            issued += line.startswith("buffer_load")
+            if line.startswith(("s_branch", "s_cbranch")):
+                before = -1  # (what follows in the text need not follow in the run)
+            if line != "s_barrier":
+                continue
+            wait = re.match(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)", body[i - 1])
+            allowed = int(wait.group(1)) if wait else -1
+            if allowed == before and allowed in loads:
+                assert issued == loads[allowed], (name, allowed, issued)
+                seen.add(allowed)
+            before, issued = allowed, 0
+        assert seen == set(loads), (name, seen)
+
+
+def registers_of(text):
+    found = set()
+    for many in re.finditer(r"\bv\[(\d+):(\d+)\]|\bv(\d+)\b", text):
+        found |= {int(many.group(3))} if many.group(3) else set(range(int(many.group(1)), int(many.group(2)) + 1))
     return found
 
 
-def test_every_wave_waits_before_the_arrival_is_counted(tmp_path):
-    """Workgroups that count themselves as finished with a pass of the exact quantiles: every wave waits for its adds to the shared histogram before
-    the barrier behind which the arrival is counted."""
-    bodies, name = {}, None
-    for line in assembly(tmp_path, "hist_quantile.hip").splitlines():
-        label = re.match(r"(_Z\w+):", line)
-        if label:
-            name = label.group(1)
-            bodies[name] = []
-        elif line.startswith(".Lfunc_end"):
-            name = None
-        elif name and line.startswith("\t") and line.strip()[:1] not in (".", ";"):
-            bodies[name].append(line.split(";")[0].strip())
-    picking = {n: b for n, b in bodies.items() if "select_pass_kernel" in n and any(re.match(r"global_atomic_add\b.*\bsc0\b", l) for l in b)}
-    assert len(picking) == 2  # of floats, of doubles
-    assert {n: unwaited_arrivals(b) for n, b in picking.items()} == {n: [] for n in picking}
-
-
-def test_the_delta_chain_keeps_its_workgroups_on_a_compute_unit(tmp_path):
-    """Kernels of one column tile have the registers of one (a SIMD has 512, a workgroup of four waves one on each): 4, 3 and 2 workgroups for keys of up
-    to 64, 128 and 256 channels; the one that may take two tiles of many short portions has room for 3.  None spills."""
-    kernels = {n: r for n, r in resources(assembly(tmp_path, "delta_rule.hip")).items() if "delta_chain_kernel" in n}
-    want = {"Li1ELi0E": 4, "Li2ELi0E": 3, "Li4ELi0E": 2, "Li2ELi3E": 3, "Li2ELi2E": 2}
-    assert len(kernels) == 2 * len(want)  # of bf16 and fp32 rows
-    for name, (registers, spilled, lds) in kernels.items():
-        workgroups = next(w for form, w in want.items() if form in name)
-        assert min(512 // (-(-registers // 8) * 8), 160 * 1024 // lds) >= workgroups and spilled == 0, (name, registers, spilled, lds)
+def test_nothing_touches_a_transposed_read_in_flight(functions):
+    """The prompt attention kernels issue LDS reads that the compiler takes as done at once: until a wait has answered them (the LDS answers in
+    order) no instruction reads, moves or overwrites their registers."""
+    for part in ("chunk_prefill_kernel", "latent_prefill_kernel"):
+        reads = 0
+        for name, body in functions(part).items():
+            flying = []
+            for line in body:
+                if line.startswith("s_waitcnt"):
+                    left = re.search(r"lgkmcnt\((\d+)\)", line)
+                    if left:
+                        flying = flying[max(0, len(flying) - int(left.group(1))) :]
+                    continue
+                if line.startswith(("s_endpgm", "s_branch")):
+                    flying = []
+                    continue
+                used = registers_of(line)
+                assert not any(used & target for target in flying), (name, line)
+                if line.startswith("ds_read_b64_tr"):
+                    flying.append(registers_of(line.split(None, 1)[1].split(",", 1)[0]))
+                    reads += 1
+                elif line.startswith(("ds_", "s_load", "s_buffer_load")):
+                    flying.append(set())
+        assert reads > 100, part
