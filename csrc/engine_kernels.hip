@@ -2019,11 +2019,17 @@ __global__ __launch_bounds__(256) void prefill_split_combine_kernel(const float*
 // (a few KB of slabs); only split 0 writes the cache and folds in the token's own key / value.
 // A range is at least the launch's blocks divided by the workgroups that are resident at once, and at least SPLIT_MIN_BLOCKS: a workgroup
 // costs some 10 us besides its blocks, so a second round of them, or short ranges, cost more than they spread.  The grid
-// holds the workgroups that can have work, not all (token, share) pairs: an idle one holds a CU's registers for a microsecond.
-// Measured, 16 rows of 8 kv heads and 4 heads each, ranges of 16 blocks from a grid of 32 shares per pair -> these: 16 x 4096 tokens 174 -> 59 us (e4m3 163 -> 38),
-// 16 x 1024 46 -> 23, 4 x 16384 82 -> 60, 2 x 32768 (14 rows of padding) 68 -> 59, 1 x 2000 15.6 -> 14.1, 1 x 100 10.8 -> 11.3.
+// holds the workgroups that can have work, not all (token, share) pairs: an idle one holds a CU's registers for a microsecond; kv heads are fastest,
+// so that those with work come first (idle ones between them left two on one CU beside an empty one: one row of 32000 tokens, groups of 8, e4m3 80 us, so 63).
+// How many ranges a row has follows from the lengths of all rows, and the order in which its partials are merged with it: a row's output is the same
+// for the same step, but beside other rows may round differently.  (Ranges that follow from the row's own length, several to a workgroup, cost a merge
+// each: 2 x 32768 tokens 62 -> 80 us, 16 x 4096 62 -> 84.)
+// Measured, 16 rows of 8 kv heads and 4 heads each, ranges of 16 blocks from a grid of 32 shares per pair -> these: 16 x 4096 tokens 172 -> 62 us (e4m3 159 -> 38),
+// 16 x 1024 44 -> 22, 4 x 16384 81 -> 63, 2 x 32768 (14 rows of padding) 68 -> 62, 1 x 2000 15.3 -> 14.1; groups of 8, 5000 + 9000 + 300 tokens 45 -> 41
+// (63 when the resident waves were taken for 2048), 4 kv heads with groups of 7, 5 x 9000 63 -> 44 (71).
 constexpr int SPLIT_MIN_BLOCKS = 16;
-constexpr int SPLIT_WAVES = 2048;  // 256 CUs of 8 waves with up to 256 registers
+// waves that are resident at once: 256 CUs of 8 waves with up to 256 registers, of 4 where wide groups take more (not with scores from the matrix cores)
+constexpr int split_waves(int rep, bool matrix_scores) { return rep <= 4 || matrix_scores ? 2048 : 1024; }
 // running sum over the lanes
 __device__ inline int wave_running_sum(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // from 1, 2, 4, 8 lanes in front in the row
@@ -2035,8 +2041,8 @@ __device__ inline int wave_running_sum(int v) {
 }
 // workgroups per kv head: each row has one, and what the ranges allow in addition fits the resident waves
 inline dim3 split_grid(int n_z, int n_rows, int nkv, int waves) {
-  const long long a = (long long)n_z * n_rows, b = SPLIT_WAVES / ((long long)waves * nkv) + n_rows;
-  return dim3((unsigned)(a < b ? a : b), nkv);
+  const long long a = (long long)n_z * n_rows, b = split_waves(1, false) / ((long long)waves * nkv) + n_rows;
+  return dim3(nkv, (unsigned)(a < b ? a : b));
 }
 
 // all-reduce over the four lane quarters (lanes l, l ^ 16, l ^ 32, l ^ 48) with the two gfx950 row / half swaps
@@ -2121,7 +2127,8 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
     int total = blocks(c0);
     for (int i = lane + 64; i < n_rows; i += 64) total += blocks(length(i));
     total = __builtin_amdgcn_readlane(wave_running_sum(total), 63);
-    const int fair = (int)(((long long)total * nkv * NWAVE + SPLIT_WAVES - 1) / SPLIT_WAVES), share = max(fair, SPLIT_MIN_BLOCKS);
+    constexpr int RESIDENT = split_waves(REP, MF);
+    const int fair = (int)(((long long)total * nkv * NWAVE + RESIDENT - 1) / RESIDENT), share = max(fair, SPLIT_MIN_BLOCKS);
     const int up = fair < SPLIT_MIN_BLOCKS ? SPLIT_MIN_BLOCKS - 1 : 0;  // (rounded up where all of them are resident all the same)
     int left = bx, base = 0;
     for (;; base += 64) {
@@ -2562,7 +2569,7 @@ __global__ __launch_bounds__(64 * NWAVE) void decode_attention_fused_kernel(cons
       return;
     }
   }
-  decode_attention_body<REP, NWAVE, KV8, SPLIT, ATTN, MF, HD>((int)blockIdx.x, (int)blockIdx.y, n_z, n_rows, slabs, n_slabs, slab_stride, positions, cos_t, sin_t,
+  decode_attention_body<REP, NWAVE, KV8, SPLIT, ATTN, MF, HD>(SPLIT ? (int)blockIdx.y : (int)blockIdx.x, SPLIT ? (int)blockIdx.x : (int)blockIdx.y, n_z, n_rows, slabs, n_slabs, slab_stride, positions, cos_t, sin_t,
                                                       k_cache, v_cache, slot_mapping, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, out, nh, nkv, row_ss,
                                                       ss_parts, inv_h, eps, scale_log2e, kv_scale, part_o, part_ml, counters, q_in, q_row_stride, row_list);
 }

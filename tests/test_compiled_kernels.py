@@ -107,6 +107,18 @@ def test_the_delta_chain_keeps_its_workgroups_on_a_compute_unit(resources):
         assert min(512 // (-(-registers // 8) * 8), 160 * 1024 // lds) >= workgroups and spilled == 0, (name, registers, spilled, lds)
 
 
+def test_split_decode_attention_has_the_waves_its_shares_are_made_for(resources):
+    """Ranges are cut for 2048 resident waves, two on a SIMD, and for 1024 where groups of more than four heads take their scores from the vector unit."""
+    seen = set()
+    for name, (registers, *_rest) in resources.items():
+        form = re.search(r"decode_attention_fused_kernelILi(\d+)ELi[48]ELb[01]ELb1ELb[01]ELb([01])E", name)
+        if form:
+            wide = int(form.group(1)) > 4 and form.group(2) == "0"
+            assert registers <= (512 if wide else 256), name
+            seen.add(wide)
+    assert seen == {True, False}
+
+
 def test_panels_have_in_flight_what_they_wait_for(functions):
     """The products by panels wait for a stage by the number of operations issued behind it.  In the loop of each height that is a count of its own, and
     from one barrier to the next exactly a stage's loads are issued: four of weights, and the pieces of rows."""

@@ -1951,6 +1951,34 @@ def test_chosen_rows_outside_and_of_other_forms(C):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nkv,rep,kv8,lengths", [(2, 7, False, [5200] * 8 + [0, 37]), (3, 8, True, [3000, 9000, 300, 0, 16, 9001]), (8, 6, False, [5000, 1, 0, 9000, 300]), (8, 8, False, [17, 2600] * 6)])
+def test_split_kv_shares_of_wide_groups(nkv, rep, kv8, lengths):
+    """Groups of more than four heads, several kv heads: ranges of the launch's fair share of half as many resident waves (of as many, with an e4m3
+    cache) and of the least one; the same output as one workgroup per pair, within two roundings to bf16 (2^-7 of the largest value), the same cache."""
+    from kvmini.models.llama import LlamaConfig, rope_tables
+    from kvmini.ops import hip_ops
+
+    torch.manual_seed(rep)
+    dev, hd, bs, rows, longest = _dev(), 128, 16, len(lengths), max(lengths)
+    ctx = torch.tensor(lengths, device=dev, dtype=torch.int32)
+    per = -(-longest // bs)
+    cos, sin = rope_tables(LlamaConfig(head_dim=hd), longest, dev)
+    bt = torch.randperm(rows * per, device=dev).view(rows, per).int()
+    pos = (ctx - 1).clamp(min=0)
+    slots = torch.where(ctx > 0, bt[torch.arange(rows, device=dev), (pos // bs).long()] * bs + pos % bs, -1).int()
+    part = hip_ops.Partial(torch.randn(2, rows, (rep + 2) * nkv * hd, device=dev) * 0.4, torch.rand(rows, 1, device=dev) * 512 + 1.0, 1e-5, 512)
+    sc = torch.rand(2, nkv, device=dev) + 0.5 if kv8 else None
+    k, v = (_fp8_cache(rows * per, nkv, bs, hd, i) if kv8 else torch.randn(rows * per, nkv, bs, hd, device=dev).bfloat16() for i in (1, 2))
+    seq, got = torch.arange(rows, device=dev, dtype=torch.int32), []
+    for n_split in (1, 3, 16):
+        kc, vc = k.clone(), v.clone()
+        got.append((hip_ops.rope_attention_fused(part, pos, cos, sin, kc, vc, slots, bt, seq, ctx, rep * nkv, hd**-0.5, kv_scale=sc, n_split=n_split), kc, vc))
+    for out, kc, vc in got[1:]:
+        assert torch.equal(kc.view(torch.uint8), got[0][1].view(torch.uint8)) and torch.equal(vc.view(torch.uint8), got[0][2].view(torch.uint8))
+        assert (out.float() - got[0][0].float()).abs().max() <= 2.0**-7 * got[0][0].float().abs().max() and not out[ctx == 0].any()
+
+
+@pytest.mark.gpu
 def test_split_kv_rows_without_context_are_zero():
     """A length of zero or less is a padding row's: zeros, in shares as by one workgroup per pair, whatever the output held."""
     from kvmini.models.llama import LlamaConfig, rope_tables
