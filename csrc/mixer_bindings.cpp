@@ -82,7 +82,7 @@ long long kve_route_workspace(int f32, int T, int Ep);
 int kve_group(const int* expert_of, int n_pairs, int E, int bm, int* order, int* tiles, int max_tiles, int* n_tiles, hipStream_t s);
 int kve_rows(const void* w, const void* x, void* y, int f32, int mode, const int* expert_of, int n_pairs, int top, int E, int N, int K, long long ldx, long long ldy, float limit, float slope, float shift, hipStream_t s);
 int kv_expert_panels(const void* Wp, const void* x, void* y, int N, int K, long long ldx, long long ldy, long long x_rows, int mode, float limit, float slope, float shift, int* order, int* tiles, int max_tiles, int* n_tiles,
-                     int row_div, hipStream_t stream);
+                     int row_div, int features, hipStream_t stream);
 int kvm_norm_rope_write(const void* proj, int f32, void* q, void* k_cache, void* v_cache, long long ldp, int q_off, int k_off, int v_off, const float* bias, const float* q_norm,
                         const float* k_norm, const int* positions, const int* slots, const float* cos_t, const float* sin_t, int rot_dims, int T, int nh, int nkv, int dim, int vdim,
                         int dkp, int dvp, int block_size, float eps, hipStream_t s);
@@ -525,18 +525,30 @@ Tensor expert_outputs(Tensor h, Tensor idx, Tensor gate_up, Tensor down, bool ga
   }
   TORCH_CHECK(!f, "experts: grouped rows are bf16");
   // (as many tokens at a time as 32-bit offsets reach)
+  int device = 0, cus = 256;
+  if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) cus = 256;
   const int64_t most = std::max<int64_t>(1, ((1ll << 31) - 1) / (2 * std::max(h.stride(0), top * ffp)) - 1);
   for (int64_t t0 = 0; t0 < T; t0 += most) {
-    const int64_t n = std::min(most, T - t0), pairs = n * top, max_tiles = pairs / 256 + std::min(E, pairs);
+    const int64_t n = std::min(most, T - t0), pairs = n * top;
+    // Few experts: as few rows a tile (whole 64s), then half as many features a panel, as leave no compute unit without work — some experts have more
+    // rows than the mean, hence the eighth.  Measured, gate / up and down in us by tiles of 256 x 256 and so: 8 experts of 1024 x 1024, 256 rows each 67, 49
+    // (150 rows 56, 34), of 2048 x 2048, 40 rows 70, 59, 256 rows 113, 93; 4 of 4096 x 4096, 40 rows 120, 99, 200 rows 176, 161.  Where the units have
+    // work, higher and wider tiles read weights and rows less often (32 of 1024 x 2048, 200 rows: 137 by 256 rows, 160 by 192; 40 rows: 88 by 256
+    // features, 97 by 128).
+    auto tiles_of = [&](int64_t rows, int64_t bm) { return E * ((rows + E * bm - 1) / (E * bm)); };
+    int64_t bm = 256;
+    while (bm > 64 && tiles_of(pairs, bm) * ((N + 255) / 256) < cus) bm -= 64;
+    auto features = [&](int64_t outputs) { return 2 * tiles_of(pairs + pairs / 8, bm) * ((outputs + 255) / 256) <= cus ? 128 : 256; };
+    const int64_t max_tiles = pairs / bm + std::min(E, pairs);
     Tensor ws = at::empty({pairs + 3 * max_tiles + 1}, idx.options());
     int* order = (int*)ws.data_ptr();
     int* tiles = order + pairs;
     int* n_tiles = tiles + 3 * max_tiles;
     auto rows = [&](const Tensor& x, int64_t row) { return (char*)x.data_ptr() + row * x.stride(0) * 2; };
-    check(kve_group(ip + t0 * top, (int)pairs, (int)E, 256, order, tiles, (int)max_tiles, n_tiles, stream()), "expert grouping");
-    check(kv_expert_panels(gate_up.data_ptr(), rows(h, t0), rows(act, t0 * top), (int)N, (int)K, h.stride(0), ffp, n, mode, (float)limit, (float)slope, (float)shift, order, tiles, (int)max_tiles, n_tiles, (int)top, stream()),
+    check(kve_group(ip + t0 * top, (int)pairs, (int)E, (int)bm, order, tiles, (int)max_tiles, n_tiles, stream()), "expert grouping");
+    check(kv_expert_panels(gate_up.data_ptr(), rows(h, t0), rows(act, t0 * top), (int)N, (int)K, h.stride(0), ffp, n, mode, (float)limit, (float)slope, (float)shift, order, tiles, (int)max_tiles, n_tiles, (int)top, features(N), stream()),
           "grouped gate / up");
-    check(kv_expert_panels(down.data_ptr(), rows(act, t0 * top), rows(y, t0 * top), (int)K, (int)ffp, ffp, K, pairs, 0, (float)limit, (float)slope, (float)shift, order, tiles, (int)max_tiles, n_tiles, 1, stream()), "grouped down");
+    check(kv_expert_panels(down.data_ptr(), rows(act, t0 * top), rows(y, t0 * top), (int)K, (int)ffp, ffp, K, pairs, 0, (float)limit, (float)slope, (float)shift, order, tiles, (int)max_tiles, n_tiles, 1, features(K), stream()), "grouped down");
   }
   return y;
 }

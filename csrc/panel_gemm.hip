@@ -44,7 +44,7 @@ constexpr int ahead(int nf) { return nf > 14 ? 3 : nf > 12 ? 4 : nf > 10 ? 5 : 6
 struct PanelArgs {
   const unsigned char* w; const __bf16* x; unsigned short* y;
   int N, K; long long ldx, ldy;
-  int n_panels;
+  int n_panels, features;  // of a panel: all eight waves', or four's
   unsigned int x_bytes;
   ExpertGate gate;
   GroupedRows groups;
@@ -240,9 +240,9 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
   const int* row_of = p.groups.order + p.groups.tile_first[tile];
   const int rows = p.groups.tile_rows[tile];
   const int nf = (rows + 31) / 32 * 2, nks = p.K / 32;
-  // the expert's panel; past the last feature reads give zeros
-  const int tiles = p.N / 16 - panel * (FEATURES / 16) < FEATURES / 16 ? p.N / 16 - panel * (FEATURES / 16) : FEATURES / 16;
-  const rsrc_t wr = buffer_of(p.w + ((long long)p.groups.tile_expert[tile] * (p.N / 16) + panel * (FEATURES / 16)) * nks * 1024, (unsigned int)tiles * nks * 1024);
+  // the expert's panel; past its last feature reads give zeros (and ask no memory)
+  const int ft = p.features / 16, tiles = p.N / 16 - panel * ft < ft ? p.N / 16 - panel * ft : ft;
+  const rsrc_t wr = buffer_of(p.w + ((long long)p.groups.tile_expert[tile] * (p.N / 16) + panel * ft) * nks * 1024, (unsigned int)tiles * nks * 1024);
   const int w0 = 2 * wave * nks * 1024 + lane * 16, w1 = w0 + nks * 1024;
   const rsrc_t xr = buffer_of(p.x, p.x_bytes);
   int xsrc[4];
@@ -258,8 +258,8 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
   multiply(nf, acc, wr, w0, w1, xr, xsrc, ring, p.K / 64, wave, lane);
-  const int f0 = panel * FEATURES + wave * 32;
-  if (f0 >= p.N) return;
+  const int f0 = panel * p.features + wave * 32;
+  if (wave * 32 >= p.features || f0 >= p.N) return;
   store_rows<MODE>(acc, rows, f0, lane, [](int) { return 1.f; }, [&](float g, float u) { return expert_gate(g, u, p.gate); },
                    [&](int row) { return p.y + (long long)row_of[row] * p.ldy; });
 }
@@ -338,16 +338,18 @@ extern "C" {
 
 // Wp holds the packed matrices [N, K] of all experts, one behind the other; row i of the tiled rows (kve_group, at most 256 a tile) is pair order[i],
 // x's row is pair / row_div, y's row the pair.  mode 1: bf16 y[pairs, N / 2] with the experts' gate; 2: bf16 max(y, 0)^2 [pairs, N]; 0: bf16 y[pairs, N].
-// N % 32 == 0, K % 64 == 0, rows of x and y of whole 16-byte pieces; x_rows rows of x must lie within 2 GiB (offsets are 32-bit).
+// features: of a panel, 256 or 128 (then four waves of a workgroup copy rows only).  N % 32 == 0, K % 64 == 0, rows of x and y of whole 16-byte pieces;
+// x_rows rows of x must lie within 2 GiB (offsets are 32-bit).
 int kv_expert_panels(const void* Wp, const void* x, void* y, int N, int K, long long ldx, long long ldy, long long x_rows, int mode, float limit, float slope, float shift, int* order, int* tiles, int max_tiles, int* n_tiles,
-                     int row_div, hipStream_t stream) {
-  if (N <= 0 || K <= 0 || (N & 31) || (K & 63) || K > (1 << 21) || (ldx & 7) || (ldy & 7) || max_tiles <= 0 || row_div <= 0 || x_rows <= 0 || mode < PLAIN || mode > SQUARED) return -1;
+                     int row_div, int features, hipStream_t stream) {
+  if ((features != FEATURES && features != FEATURES / 2) || N <= 0 || K <= 0 || (N & 31) || (K & 63) || K > (1 << 21) || (ldx & 7) || (ldy & 7) || max_tiles <= 0 || row_div <= 0 || x_rows <= 0 || mode < PLAIN || mode > SQUARED) return -1;
   const long long bytes = ((x_rows - 1) * ldx + K) * 2;
   if (bytes >= (1ll << 31) || ldx < K) return -1;
   PanelArgs a;
   a.w = (const unsigned char*)Wp; a.x = (const __bf16*)x; a.y = (unsigned short*)y;
   a.N = N; a.K = K; a.ldx = ldx; a.ldy = ldy;
-  a.n_panels = (N + FEATURES - 1) / FEATURES;
+  a.n_panels = (N + features - 1) / features;
+  a.features = features;
   a.x_bytes = (unsigned int)bytes;
   a.gate = ExpertGate{limit, slope, shift};
   a.groups = GroupedRows{order, tiles, tiles + max_tiles, tiles + 2 * max_tiles, n_tiles, max_tiles, row_div};

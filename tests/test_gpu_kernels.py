@@ -2832,6 +2832,13 @@ def test_expert_panels_at_every_number_of_rows(C, ff, width, gated):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ff,width,gated", [(3072, 192, False), (1536, 128, True), (2048, 128, False), (1280, 64, True)])
+def test_expert_panels_of_every_height(C, ff, width, gated):
+    """Enough panels that tiles are of 256, 192 or 128 rows (fewer panels: of 64): every number of row tiles of each."""
+    test_expert_panels_at_every_number_of_rows(C, ff, width, gated)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("ff,width", [(128, 256), (384, 1024), (1408, 512)])
 def test_expert_panels_add_up_in_the_order_of_the_columns(C, ff, width):
     """Whatever panel and expert a row falls into, its sums go through the columns from the first to the last: bit for bit what the tiled kernel makes of
