@@ -609,7 +609,10 @@ __global__ __launch_bounds__(64) void rope_kv_write_kernel(unsigned short* __res
 // The bf16 form for prompts: a wave does one task of four tokens, whose rows, positions and slots are all in flight together.  With a token a
 // wave the 2048 tokens of a prompt (32 + 8 heads of 128) are 14336 waves of three dependent reads each, and their number is the time.
 // Measured on MI355X, us (a token a wave, four): 512 tokens 6.3, 6.7; 1024 10.9, 9.5; 2048 19.9, 12.8; 4096 32.0, 20.7 (50 and 101 MB of
-// reads and writes for the last two; e4m3 caches the same): from 1024 tokens on (ROPE_ROWS_MIN).
+// reads and writes for the last two; e4m3 caches the same).  Fewer or narrower heads make fewer waves, which are resident together for longer:
+// 32 + 8 heads of 64, 1024 tokens 5.8, 6.7, 4096 13.3, 11.1; 9 + 3 of 64, 4096 tokens 6.8, 7.4; 8 + 8 of 128, 1100 tokens 6.1, 6.7, 2048 8.8, 7.7;
+// but 16 + 2 of 256, 1024 tokens 12.9, 8.0.  The line that has all of these on the right side: tokens x tasks x head dim of 1024 tokens of 32 + 8 heads of
+// 128 (ROPE_ROWS_MIN).
 template <bool KV8>
 __global__ __launch_bounds__(64) void rope_kv_write_rows_kernel(unsigned short* __restrict__ qkv, const int* __restrict__ positions, const float* __restrict__ cos_t,
                                                                 const float* __restrict__ sin_t, void* __restrict__ k_cache, void* __restrict__ v_cache,
@@ -3133,11 +3136,9 @@ int kv_add_rmsnorm_slabs(const float* slabs, int n_slabs, long long slab_stride,
   return (int)hipGetLastError();
 }
 
-constexpr int ROPE_ROWS_MIN = 1024;  // tokens: see rope_kv_write_rows_kernel
-static inline int rope_grid_y(int nh, int nkv, int hd) {
-  const int tasks = (nh + nkv) * (hd >> 4) + nkv * (hd >> 3);
-  return (tasks + 63) / 64;
-}
+constexpr long long ROPE_ROWS_MIN = 1024ll * 448 * 128;  // tokens x tasks x head dim: see rope_kv_write_rows_kernel
+static inline int rope_tasks(int nh, int nkv, int hd) { return (nh + nkv) * (hd >> 4) + nkv * (hd >> 3); }
+static inline int rope_grid_y(int nh, int nkv, int hd) { return (rope_tasks(nh, nkv, hd) + 63) / 64; }
 
 // row_ss (nullable): [T][ss_parts] partial sums of squares of the GEMM's input rows; when
 // given, the summed projection is scaled by rsqrt(sum/H_in + eps) (folded RMSNorm).
@@ -3182,7 +3183,7 @@ int kv_rope_kv_write(void* qkv, const int* positions, const float* cos_t, const 
                      int nh, int nkv, int hd, int block_size, const float* kv_scale, hipStream_t stream) {
   if (T <= 0) return 0;
   if (hd % 16) return -1;
-  if (T >= ROPE_ROWS_MIN) {
+  if ((long long)T * rope_tasks(nh, nkv, hd) * hd >= ROPE_ROWS_MIN) {
     const dim3 grid((T + 3) / 4, rope_grid_y(nh, nkv, hd));
 #define KV_ROPE_ROWS(K8)                                                                                                                                        \
   hipLaunchKernelGGL((rope_kv_write_rows_kernel<K8>), grid, dim3(64), 0, stream, (unsigned short*)qkv, positions, cos_t, sin_t, k_cache, v_cache, slot_mapping, \

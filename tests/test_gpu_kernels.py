@@ -2923,3 +2923,29 @@ def test_rope_of_many_rows_equals_that_of_few(C, rows, nh, nkv, hd, kv8):
             C.rope_kv_write(x[i : i + step], pos[i : i + step], cos, sin, k, v, slots[i : i + step], nh, nkv, hd, scale)
         out.append([x] + [c.view(torch.uint8) if kv8 else c for c in (k, v)])
     assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv,hd,kv8", [(32, 8, 128, False), (32, 8, 128, True), (16, 2, 256, False), (32, 8, 64, True), (8, 8, 64, False), (4, 2, 64, True), (7, 1, 64, False)])
+@pytest.mark.parametrize("more", [-1, 0, 1, 2, 3])
+def test_rope_at_the_line_between_its_kernels(C, nh, nkv, hd, kv8, more):
+    """The calls on both sides of the rule (tokens x tasks x head dim), the last wave's tokens cut off in every way, against calls of few rows."""
+    tasks = (nh + nkv) * (hd // 16) + nkv * (hd // 8)
+    rows = -(-1024 * 448 * 128 // (tasks * hd)) + more
+    torch.manual_seed(rows)
+    dev, bs = _dev(), 16
+    qkv = torch.randn(rows, (nh + 2 * nkv) * hd, device=dev).bfloat16()
+    pos = torch.randint(0, 3000, (rows,), dtype=torch.int32, device=dev)
+    cos, sin = torch.randn(3000, hd // 2, device=dev), torch.randn(3000, hd // 2, device=dev)
+    blocks = rows // bs + 2
+    slots = torch.randperm(blocks * bs, device=dev)[:rows].int()
+    slots[::7] = -1
+    scale = torch.rand(2, nkv, device=dev) + 0.5 if kv8 else None
+    out = []
+    for step in (rows, rows // 9):
+        x = qkv.clone()
+        k, v = (torch.zeros(blocks, nkv, bs, hd, dtype=torch.float8_e4m3fn if kv8 else torch.bfloat16, device=dev) for _ in range(2))
+        for i in range(0, rows, step):
+            C.rope_kv_write(x[i : i + step], pos[i : i + step], cos, sin, k, v, slots[i : i + step], nh, nkv, hd, scale)
+        out.append([x.view(torch.uint8), k.view(torch.uint8), v.view(torch.uint8)])
+    assert all(torch.equal(a, b) for a, b in zip(*out))
