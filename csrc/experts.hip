@@ -104,7 +104,7 @@ __device__ inline void choose(const float* z, const float (&corr)[NC], bool pad,
   }
   if constexpr (NC == 1) {  // an expert per lane: its rank is the number of better ones (of equals, the earlier)
     int rank = 0;
-#pragma unroll 8
+#pragma unroll  // (whole: by 8 the 1025 tokens of 8 experts x 1024 columns are 10.6 us for 9.8, the few of one token 6.9 for 6.6)
     for (int j = 0; j < 64; ++j) {
       const float o = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c[0]), j));
       rank += (o > c[0] || (o == c[0] && j < lane)) ? 1 : 0;
