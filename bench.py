@@ -402,10 +402,10 @@ def main() -> int:
             itl_hist_q = [snap.get(p, float("nan")) for p in (0.5, 0.95, 0.99)]  # the live view's 2048-bin estimate, merged over the ranks
         if itl_exact is not None:
             qi = [itl_exact]
-            itl_engine = ("hip:radix_hist/scan" if cdev.type == "cuda" else "numpy radix select") + " + all-reduce of the digit histograms per pass (exact)"
+            itl_engine = ("hip:select_pass/scan" if cdev.type == "cuda" else "numpy radix select") + " + all-reduce of the digit histograms per pass (exact)"
         elif on_gpu and itl.size:
             qi, _ = hq.batched_quantiles(torch.from_numpy(itl).to(device).reshape(1, -1), (0.5, 0.95, 0.99), return_stats=True)
-            itl_engine = "hip:kv_radix_select"
+            itl_engine = "hip:kv_select_quantiles"
         else:
             qi = [np.nanquantile(itl, (0.5, 0.95, 0.99)).tolist()] if itl.size else [[float("nan")] * 3]
             itl_engine = "numpy"
@@ -491,7 +491,7 @@ def main() -> int:
                 "cost_per_1k_tokens": round(cost_1k / BASELINE["cost_per_1k_tokens"], 4) if cost_1k else None,
                 "wh_per_1k_tokens": round(wh_1k / BASELINE["wh_per_1k_tokens"], 5) if wh_1k else None,
             },
-            "quantile_engine": "hip:kv_radix_select" if on_gpu else "numpy (cpu rehearsal)",
+            "quantile_engine": "hip:kv_select_quantiles" if on_gpu else "numpy (cpu rehearsal)",
             "itl_quantile_engine": itl_engine,
             "itl_histogram_p50_p95_p99_ms": itl_hist_q,
             "collective_backend": (dist.get_backend() if world > 1 else None),

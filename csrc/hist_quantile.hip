@@ -217,7 +217,7 @@ __device__ inline unsigned long long rank_of(const Levels& lv, int r, unsigned l
 // of a wave's 64 samples share it), so what bounds a pass is LDS atomics that meet on one address: a workgroup of 16 waves keeps the histogram
 // 16 times (fewer times when there are more prefixes), bin by bin next to each other, and a lane uses copy lane % 16 — at most 4 lanes
 // of an instruction meet, in different banks.  One global atomic per non-empty bin and workgroup adds it up, so there are few workgroups,
-// one a CU.  3 x 4 M floats: 27 us a pass, picking included, where one histogram a wave with ballot aggregation took 48 and picking 14 more.
+// one a CU.  3 x 4 M floats: 25 us a pass, picking included, where one histogram a wave with ballot aggregation took 48 and picking 14 more.
 constexpr int SEL_THREADS = 1024;
 constexpr int SEL_WORDS = 16 * KV_BINS;  // LDS words of the copies: 128 KiB
 constexpr int PER = KV_MAX_RANKS * KV_BINS / SEL_THREADS;  // bins per thread, of all prefixes

@@ -268,8 +268,8 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
 // y[M, N] = x[M, K] W[N, K]^T, the matrix multiplied by panels of 256 features x `height` rows: workgroups of one matrix share what they read through
 // the L2, panels in order, a panel's tiles next to one another.  The height is free in steps of 32, so that panels x tiles fill the CUs in whole rounds;
 // the panels of a last round may have another.  Bound by the matrix cores and the power they draw (2048 x 28672 x 4096 of zeros takes 308 us, of random
-// numbers 373) and by some 8 us per round outside the K loop.  Against tiles of up to 256 x 256 with both operands through LDS, 2048 rows:
-// 28672 x 4096 416 -> 358 us (1.34 PFLOP/s), 9216 x 4096 161 -> 129, 16384 x 2048 130 -> 111, 4096 x 14336 196 -> 190, 5632 x 2048 53 -> 44.
+// numbers 369) and by some 8 us per round outside the K loop.  Against tiles of up to 256 x 256 with both operands through LDS, 2048 rows:
+// 28672 x 4096 411 -> 369 us (1.30 PFLOP/s), 9216 x 4096 147 -> 128, 16384 x 2048 123 -> 112, 4096 x 14336 206 -> 190, 5632 x 2048 51 -> 45.
 struct DenseArgs {
   const unsigned char* w; const __bf16* x; unsigned short* y;
   int M, N, K; long long ldx, ldy;

@@ -382,12 +382,12 @@ def _plan_panels(m: int, n: int, k: int, may_split: bool = False) -> Optional[Tu
 
     None up to one round of 128 x 128 tiles: there what counts is that all CUs have work, and a panel's tile is at least twice as wide
     (measured on MI355X, us, this tiled GEMM and panels: 2048 rows x 2048 x 8192 77 and 89, 512 x 6144 x 4096 41 and 45, 256 x 4096 x 4096
-    40 and 45; beyond, 144 x 28672 x 4096 74 and 59, 1024 x 9216 x 4096 81 and 65, 2048 x 4096 x 14336 196 and 190, 2048 x 28672 x 4096 416 and 373).
+    40 and 45; beyond, 129 x 28672 x 4096 77 and 63, 1024 x 9216 x 4096 68 and 66, 2048 x 4096 x 14336 206 and 190, 2048 x 28672 x 4096 411 and 369).
 
     The heights are those of the least modelled time: rounds over the CUs, each 8 us outside the K loop and 0.1 + 0.005 us per row in each
     64 columns, less what CUs that stay empty in a last round leave to the others in power and bandwidth (0.7 of their share).  Fitted on ten
     matrices at 144 to 4096 rows (5 % standard deviation); what it picks is within 1 % of the best height on all but one.  Two heights were 0.99
-    to 1.12 times as fast as the best single one, 1.035 in the mean over 16 sizes (2048 x 28672 x 4096: 372 -> 358 us); with 96 rows behind
+    to 1.12 times as fast as the best single one, 1.035 in the mean over 16 sizes; with 96 rows behind
     whole rounds it was 0.97 over six others, so that is left out."""
     cus = _num_cus()
     if -(-m // 128) * -(-n // 128) <= cus or (may_split and _plan_wide(m, n, k, 0, True)[3] > 1):
