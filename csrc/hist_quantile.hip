@@ -20,7 +20,9 @@
 //                        into the next prefix (kv_radix_pass_*: a launch of its own, for samples
 //                        spread over ranks).  Up to 8 ranks are tracked at once (floor and
 //                        ceil rank of p50/p95/p99), so three quantiles of 10^8 doubles cost 6
-//                        streaming passes and no sort.  The result is bit-exact: the CPU
+//                        streaming passes and no sort.  Rows of 16 k (doubles: 512) to 32 M samples take two
+//                        passes instead, between values that a sample of them gives (kv_split_quantiles).
+//                        The result is bit-exact: the CPU
 //                        interpolates between the two selected samples exactly like
 //                        analyze.py does.
 //   kv_equal_hist       the 20-bin equal-width histogram over [min, max] (last bin closed),
@@ -35,6 +37,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #define KV_BINS 2048
 #define KV_WAVES 4
@@ -229,51 +233,36 @@ __device__ inline int log2_copies(int prefixes, long long n) {
   return room < wanted ? room : wanted;
 }
 
-// counts the digits of the samples first, first + stride, ... (in 16-byte pieces) of a row into h[prefix][bin][copy]; MOST: at least U prefixes
-// (0: the first pass, which has none)
-template <typename T, int MOST>
-__device__ void count_digits(const T* __restrict__ row, long long n, long long first, long long stride, unsigned int* h, const unsigned long long* uniq, int U, int shift, int digit_bits) {
-  using KT = typename KeyOf<T>::type;
+// visit(v) for the samples first, first + stride, ... (in 16-byte pieces) of a row, `first` consecutive in a wave.  All lanes of a wave visit together:
+// those that are past the end, a NaN.  after_piece(): after 16 bytes of each lane, or less.
+struct Nothing { __device__ void operator()() const {} };
+template <typename T, typename F, typename G = Nothing>
+__device__ __forceinline__ void for_samples(const T* __restrict__ row, long long n, long long first, long long stride, F&& visit, G&& after_piece = G{}) {
   constexpr int VEC = 16 / sizeof(T);
-  const int cl = log2_copies(U, n), copy = threadIdx.x & ((1 << cl) - 1);
-  const KT dmask = (KT)((1u << digit_bits) - 1u);
-  const int hi_shift = shift + digit_bits;  // bits above the current digit
-  KT pre[MOST > 0 ? MOST : 1] = {};
-#pragma unroll
-  for (int u = 0; u < MOST; ++u) pre[u] = (KT)((KT)(uniq[u < U ? u : 0] >> (64 - KeyOf<T>::bits)) >> hi_shift);  // (unused ones repeat the first)
-  auto visit = [&](T v) {
-    if (!(v == v)) return;
-    const KT key = KeyOf<T>::key(v);
-    int bin = (int)((key >> shift) & dmask);
-    if constexpr (MOST > 0) {
-      const KT hi = (KT)(key >> hi_shift);
-      int at = -1;
-#pragma unroll
-      for (int u = MOST - 1; u >= 0; --u) at = hi == pre[u] ? u : at;
-      if (at < 0) return;
-      bin += at * KV_BINS;
-    }
-    atomicAdd(&h[(bin << cl) + copy], 1u);
-  };
   struct alignas(16) Pack { T v[VEC]; };
+  const T none = (T)__builtin_nanf("");
+  const long long lane = threadIdx.x & 63;
   // (rows need not start at a multiple of 16 bytes: the samples in front of the first whole piece and behind the last go one by one)
   long long head = (VEC - (long long)((uintptr_t)row / sizeof(T)) % VEC) % VEC;
   head = head < n ? head : n;
-  const Pack* pv = reinterpret_cast<const Pack*>(row + head);
+  const Pack* pv = reinterpret_cast<const Pack*>(row + head) + lane;
   const long long nvec = (n - head) / VEC, tail = head + nvec * VEC;
   auto visit_pack = [&](const Pack& p) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) visit(p.v[j]);
+    after_piece();
   };
   constexpr int AHEAD = 4;  // loads in flight per lane while the ones before are counted
   Pack p[AHEAD];
-  long long i = first;
-  if (i + (AHEAD - 1) * stride < nvec) {
+  // (of the wave's first lane: the loops are the same for all)
+  const long long start = (long long)((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(first >> 32)) << 32 | (unsigned int)__builtin_amdgcn_readfirstlane((int)first));
+  long long i = start;
+  if (i + (AHEAD - 1) * stride + 63 < nvec) {
 #pragma unroll
     for (int k = 0; k < AHEAD; ++k) p[k] = pv[i + k * stride];
     for (;;) {
       i += AHEAD * stride;
-      const bool more = i + (AHEAD - 1) * stride < nvec;
+      const bool more = i + (AHEAD - 1) * stride + 63 < nvec;
       Pack q[AHEAD];
       if (more) {
 #pragma unroll
@@ -286,9 +275,43 @@ __device__ void count_digits(const T* __restrict__ row, long long n, long long f
       for (int k = 0; k < AHEAD; ++k) p[k] = q[k];
     }
   }
-  for (; i < nvec; i += stride) visit_pack(pv[i]);
-  if (first < head) visit(row[first]);
-  if (tail + first < n) visit(row[tail + first]);
+  for (; i < nvec; i += stride) {
+    Pack q;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) q.v[j] = none;
+    if (i + lane < nvec) q = pv[i];
+    visit_pack(q);
+  }
+  if (start < head) visit(first < head ? row[first] : none);
+  if (tail + start < n) visit(tail + first < n ? row[tail + first] : none);
+  after_piece();
+}
+
+// counts the digits of the samples first, first + stride, ... (in 16-byte pieces) of a row into h[prefix][bin][copy]; MOST: at least U prefixes
+// (0: the first pass, which has none)
+template <typename T, int MOST>
+__device__ void count_digits(const T* __restrict__ row, long long n, long long first, long long stride, unsigned int* h, const unsigned long long* uniq, int U, int shift, int digit_bits) {
+  using KT = typename KeyOf<T>::type;
+  const int cl = log2_copies(U, n), copy = threadIdx.x & ((1 << cl) - 1);
+  const KT dmask = (KT)((1u << digit_bits) - 1u);
+  const int hi_shift = shift + digit_bits;  // bits above the current digit
+  KT pre[MOST > 0 ? MOST : 1] = {};
+#pragma unroll
+  for (int u = 0; u < MOST; ++u) pre[u] = (KT)((KT)(uniq[u < U ? u : 0] >> (64 - KeyOf<T>::bits)) >> hi_shift);  // (unused ones repeat the first)
+  for_samples(row, n, first, stride, [&](T v) {
+    if (!(v == v)) return;
+    const KT key = KeyOf<T>::key(v);
+    int bin = (int)((key >> shift) & dmask);
+    if constexpr (MOST > 0) {
+      const KT hi = (KT)(key >> hi_shift);
+      int at = -1;
+#pragma unroll
+      for (int u = MOST - 1; u >= 0; --u) at = hi == pre[u] ? u : at;
+      if (at < 0) return;
+      bin += at * KV_BINS;
+    }
+    atomicAdd(&h[(bin << cl) + copy], 1u);
+  });
 }
 
 // the copies of bin i (counted over all prefixes)
@@ -430,33 +453,62 @@ __global__ __launch_bounds__(SEL_THREADS) void select_pass_kernel(const T* __res
   }
 }
 
-// Up to 1024 samples (a run's requests): a thread per sample counts how many come in front of it.  A workgroup per metric.
+// a sample's key; a NaN's is the largest, which no sample has (that one is a NaN's too)
 template <typename T>
-__global__ __launch_bounds__(SEL_THREADS) void select_by_rank_kernel(const T* __restrict__ x, int n, long long row_stride, Levels levels, unsigned long long* out) {
-  __shared__ __attribute__((aligned(16))) unsigned long long keys[SEL_THREADS + 1];
-  const int tid = threadIdx.x, m = blockIdx.x;
-  const T v = tid < n ? x[(long long)m * row_stride + tid] : (T)0;
-  const bool on = tid < n && v == v;
-  const unsigned long long key = (unsigned long long)KeyOf<T>::key(v) << (64 - KeyOf<T>::bits);
-  const int count = __syncthreads_count(on);
-  keys[tid] = on ? key : ~0ull;  // (no sample's key: that one is a NaN's)
-  if (tid == 0) keys[SEL_THREADS] = ~0ull;
-  __syncthreads();
-  int before = 0;
-  const int pairs = (tid & ~63) < n ? n : 0;  // (waves without a sample need not count)
-#pragma unroll 4
-  for (int j = 0; j < pairs; j += 2) {
-    const ulonglong2 k = *reinterpret_cast<const ulonglong2*>(&keys[j]);
-    before += (k.x < key || (k.x == key && j < tid) ? 1 : 0) + (k.y < key || (k.y == key && j + 1 < tid) ? 1 : 0);
-  }
-  unsigned long long* o = out + (long long)m * SEL_OUT;
-  if (tid == 0) o[KV_MAX_RANKS] = (unsigned long long)count;
-  if (on)
-    for (int r = 0; r < 2 * levels.n; ++r)
-      if (rank_of(levels, r, (unsigned long long)count) == (unsigned long long)before) o[r] = key;
+__device__ inline typename KeyOf<T>::type key_or_last(T v) {
+  using KT = typename KeyOf<T>::type;
+  return v == v ? KeyOf<T>::key(v) : ~(KT)0;
 }
 
-// Few samples: all passes in one launch, a workgroup per metric.
+// How many of keys[from ... from + stretch) (whole 16 bytes) come in front of the key at `at`; of equal ones the one in front is the smaller.  A wave's
+// lanes have the same stretch.
+template <typename KT>
+__device__ inline unsigned int count_in_front(const KT* keys, int from, int stretch, int at, KT key) {
+  constexpr int VEC = 16 / sizeof(KT);
+  struct alignas(16) Some { KT k[VEC]; };
+  unsigned int less = 0;
+  auto count = [&](auto&& in_front) {
+#pragma unroll 4
+    for (int j = from; j < from + stretch; j += VEC) {
+      const Some k = *reinterpret_cast<const Some*>(&keys[j]);
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) less += in_front(k.k[i], j + i);
+    }
+  };
+  // a stretch in front of this key counts those up to it, one behind it those below: one comparison each (NaNs count nowhere)
+  const KT upto = from + stretch <= at && key != ~(KT)0 ? key + 1 : key;
+  if (__any(from <= at && at < from + stretch)) count([&](KT k, int j) { return k < key || (k == key && j < at); });
+  else count([&](KT k, int) { return k < upto; });
+  return less;
+}
+
+// Up to 512 samples (a run's requests): each is ranked among all, by as many threads as there are per sample.  A workgroup per metric.
+constexpr int SEL_RANKED = 512;
+template <typename T>
+__global__ __launch_bounds__(SEL_THREADS) void select_by_rank_kernel(const T* __restrict__ x, int n, long long row_stride, Levels levels, unsigned long long* out) {
+  using KT = typename KeyOf<T>::type;
+  __shared__ __attribute__((aligned(16))) KT keys[SEL_RANKED];
+  __shared__ unsigned int before[SEL_RANKED];
+  const int tid = threadIdx.x, m = blockIdx.x;
+  if (tid < SEL_RANKED) {
+    keys[tid] = tid < n ? key_or_last(x[(long long)m * row_stride + tid]) : ~(KT)0;
+    before[tid] = 0;
+  }
+  const int count = __syncthreads_count(tid < n && keys[tid < n ? tid : 0] != ~(KT)0);
+  int together = 64;
+  while (together < n) together *= 2;
+  const int stretch = together * together / SEL_THREADS, at = tid % together;
+  const KT key = keys[at];
+  atomicAdd(&before[at], count_in_front(keys, tid / together * stretch, stretch, at, key));
+  __syncthreads();
+  unsigned long long* o = out + (long long)m * SEL_OUT;
+  if (tid == 0) o[KV_MAX_RANKS] = (unsigned long long)count;
+  if (tid < n && key != ~(KT)0)
+    for (int r = 0; r < 2 * levels.n; ++r)
+      if (rank_of(levels, r, (unsigned long long)count) == (unsigned long long)before[tid]) o[r] = (unsigned long long)key << (64 - KeyOf<T>::bits);
+}
+
+// Some thousand samples: all passes in one launch, a workgroup per metric.
 template <typename T>
 __global__ __launch_bounds__(SEL_THREADS) void select_few_kernel(const T* __restrict__ x, long long n, long long row_stride, Levels levels, unsigned long long* out) {
   extern __shared__ __attribute__((aligned(16))) unsigned int h[];
@@ -485,6 +537,520 @@ __global__ __launch_bounds__(SEL_THREADS) void select_few_kernel(const T* __rest
     pick_digits(&s, h, top + 64 - KeyOf<T>::bits, first, first ? &levels : nullptr);
   }
   if (tid < SEL_OUT) out[(long long)m * SEL_OUT + tid] = tid < KV_MAX_RANKS ? s.prefix[tid] : s.count;
+}
+
+// ---------------------------------------------------------------------------------
+// Many samples, in two passes over them instead of one per digit (3 for floats, 6 for doubles).  What bounds a digit's pass is not memory but one
+// LDS atomic per sample.  Here 2048 samples (of long rows 4096), one from each stretch of the row, say between which two values a level's order statistics lie: an
+// interval that holds a few per cent of the samples.  The first pass counts the samples below each interval in registers, and only those inside
+// go to a histogram, a thousand linear bins of the interval's keys; the second collects the few hundred of the bins that hold the ranks, and the
+// last workgroup to finish ranks them.  Exact whatever the samples are: where an interval misses a rank (4 standard deviations aside: about one
+// call in 5000) or a bin of several values holds more than fit, the count of samples says so and the digits' passes answer (two distant
+// clusters with a rank between them: 157 us for 95).
+// Whole calls by digits and so, 3 rows: 33 k floats 54 and 48 us, 1 M 69 and 52, 4 M 88 and 69;
+// 4 M doubles 198 and 79.  Of the 56 us of kernels for 3 x 4 M floats the passes are 14 and 10, the sample 6, the last workgroup's ranking 9: chains of
+// dependent steps, about one us each.
+constexpr int SAMPLE_PARTS = 64;                     // workgroups that rank a row's sample, at most
+constexpr int SPANS = KV_MAX_RANKS / 2;              // intervals: one per level, fewer where they overlap
+constexpr int SPAN_BINS = 1024, SPAN_COPIES = 2;     // LDS: 4 x 1024 x 2 counts, 32 KiB (a lane uses copy lane % 2: values that many samples share)
+constexpr int FOUND = 16384;                         // samples of a bin that are ranked
+constexpr unsigned long long UNDECIDED = ~0ull;      // as a count: the digits' passes have to answer
+constexpr long long SPLIT_MOST = 1ll << 25;          // of a row: beyond, what a sample says is too wide for FOUND (60 M floats: 182 us, by digits 179)
+
+// What the sample says about a row, and what the passes count.  Keys are the samples' own, in the low bits.
+struct SplitState {
+  unsigned long long ends[KV_MAX_RANKS];             // level -> sampled keys at the ends of its interval
+  unsigned long long below[SPANS];                   // samples in front of each interval, as Spans orders them
+  unsigned long long count;                          // samples
+  unsigned long long least[KV_MAX_RANKS], most[KV_MAX_RANKS];  // of the samples in a chosen bin
+  unsigned int found[KV_MAX_RANKS];                  // how many those are
+  unsigned int done;
+  unsigned int open;                                 // ends beyond which the interval goes on (a bit each): no sampled key is as far out as it has to be
+};
+constexpr int SPLIT_WORDS = sizeof(SplitState) / 4;
+constexpr long long SPLIT_BYTES = sizeof(SplitState) + SPANS * SPAN_BINS * 4 + (long long)KV_MAX_RANKS * FOUND * 8;
+static_assert(sizeof(SplitState) % 16 == 0, "16-byte reads of the bins behind it");
+
+struct SplitRow {
+  SplitState* state;
+  unsigned int* bins;           // [SPANS][SPAN_BINS]
+  unsigned long long* found;    // [KV_MAX_RANKS][FOUND]
+  __device__ SplitRow(void* work, int metric) {
+    char* p = (char*)work + metric * SPLIT_BYTES;
+    state = (SplitState*)p;
+    bins = (unsigned int*)(p + sizeof(SplitState));
+    found = (unsigned long long*)(bins + SPANS * SPAN_BINS);
+  }
+};
+
+// Linear bins of `wide` + 1 keys: key - first >> bin_shift
+template <int BINS>
+__device__ inline int bin_shift(unsigned long long wide) {
+  static_assert((BINS & (BINS - 1)) == 0, "a power of two");
+  return wide < BINS ? 0 : 64 - __clzll((long long)wide) - (31 - __builtin_clz(BINS));
+}
+
+// The levels' intervals in order, those that overlap as one.  By one thread, in registers.
+struct Spans {
+  unsigned long long lo[SPANS], hi[SPANS];  // ends
+  unsigned long long from[SPANS];           // the bins are those of from ... upto: the first takes in what is below, the last what is above
+  int shift[SPANS];
+  int of[SPANS];                            // level -> interval
+  int n;
+};
+template <typename T>
+__device__ inline void find_spans(const SplitState& s, int levels, Spans* to) {
+  unsigned long long lo[SPANS], hi[SPANS], from[SPANS], upto[SPANS];
+  int level[SPANS];
+  const unsigned int open = s.open;
+#pragma unroll
+  for (int i = 0; i < SPANS; ++i) {
+    from[i] = i < levels ? s.ends[2 * i] : ~0ull;
+    upto[i] = i < levels ? s.ends[2 * i + 1] : ~0ull;
+    // (as values: both zeros, which compare as one, are in or out together)
+    lo[i] = open >> 2 * i & 1 ? KeyOf<T>::key(-(T)INFINITY) : from[i] == KeyOf<T>::key((T)0) ? KeyOf<T>::key(-(T)0) : from[i];
+    hi[i] = open >> (2 * i + 1) & 1 ? KeyOf<T>::key((T)INFINITY) : upto[i] == KeyOf<T>::key(-(T)0) ? KeyOf<T>::key((T)0) : upto[i];
+    if (i >= levels) lo[i] = ~0ull;  // (no key: behind all others)
+    level[i] = i;
+  }
+#pragma unroll
+  for (int i = 1; i < SPANS; ++i)
+#pragma unroll
+    for (int j = i; j > 0; --j)
+      if (lo[j - 1] > lo[j]) {
+        const unsigned long long a = lo[j], b = hi[j], c = from[j], d = upto[j];
+        const int l = level[j];
+        lo[j] = lo[j - 1]; hi[j] = hi[j - 1]; from[j] = from[j - 1]; upto[j] = upto[j - 1]; level[j] = level[j - 1];
+        lo[j - 1] = a; hi[j - 1] = b; from[j - 1] = c; upto[j - 1] = d; level[j - 1] = l;
+      }
+  int n = 0;
+  unsigned long long first = 0, last = 0, in = 0, out = 0;
+#pragma unroll
+  for (int i = 0; i < SPANS; ++i) {
+    if (i >= levels) break;
+    const bool apart = n == 0 || lo[i] > last;
+    n += apart;
+    first = apart ? lo[i] : first;
+    last = apart || hi[i] > last ? hi[i] : last;
+    in = apart || from[i] < in ? from[i] : in;
+    out = apart || upto[i] > out ? upto[i] : out;
+    to->lo[n - 1] = first;
+    to->hi[n - 1] = last;
+    to->from[n - 1] = in;
+    to->shift[n - 1] = bin_shift<SPAN_BINS>(out - in);
+    to->of[level[i]] = n - 1;
+  }
+  to->n = n;
+}
+
+// The levels' intervals, from EACH samples per thread.  Grid (workgroups, metrics): each takes in all sampled keys, ranks its share of them against all, and writes those whose
+// rank is that of an end.  (One workgroup that selects by digits took 45 us: a chain of loads, LDS sums and scans on one compute unit.)
+template <typename T, int EACH>
+__global__ __launch_bounds__(SEL_THREADS) void select_sample_kernel(const T* __restrict__ x, long long n, long long row_stride, Levels levels, void* work) {
+  using KT = typename KeyOf<T>::type;
+  constexpr int SAMPLED = EACH * SEL_THREADS;
+  __shared__ __attribute__((aligned(16))) KT keys[SAMPLED];
+  __shared__ unsigned int before[SEL_THREADS];
+  __shared__ unsigned int rank[KV_MAX_RANKS];
+  const int tid = threadIdx.x, m = blockIdx.y;
+  const SplitRow row(work, m);
+  const T* xr = x + (long long)m * row_stride;
+  T v[EACH];
+#pragma unroll
+  for (int j = 0; j < EACH; ++j) {
+    // somewhere in the stretch: samples at even distances would all be, say, a request's first
+    const unsigned long long at = tid + j * SEL_THREADS, from = at * (unsigned long long)n / SAMPLED, len = (at + 1) * (unsigned long long)n / SAMPLED - from;
+    unsigned int r = (unsigned int)at * 2654435761u + (unsigned int)m * 40503u;
+    r ^= r >> 15; r *= 2246822519u; r ^= r >> 13; r *= 3266489917u; r ^= r >> 16;
+    v[j] = xr[from + (((unsigned long long)r * len) >> 32)];
+  }
+  int got = 0;
+#pragma unroll
+  for (int j = 0; j < EACH; ++j) {
+    keys[tid + j * SEL_THREADS] = key_or_last(v[j]);
+    got += __syncthreads_count(v[j] == v[j]);
+  }
+  const int R = 2 * levels.n;
+  if (tid < KV_MAX_RANKS) {
+    double p = levels.p[tid >> 1];
+    p = p < 0.0 ? 0.0 : (p > 1.0 ? 1.0 : p);
+    const double at = p * (double)(got - 1), apart = 4.0 * sqrt((double)got * p * (1.0 - p)) + 2.0;
+    const double end = (tid & 1) ? ceil(at + apart) : floor(at - apart);
+    const bool open = end < 0.0 || end > (double)(got - 1);
+    rank[tid] = end < 0.0 ? 0 : end > (double)(got - 1) ? (unsigned int)(got - 1) : (unsigned int)end;
+    const unsigned int opens = (unsigned int)__ballot(open);
+    if (blockIdx.x == 0) {
+      if (got == 0) row.state->ends[tid] = KeyOf<T>::key((tid & 1) ? (T)INFINITY : -(T)INFINITY);
+      row.state->least[tid] = ~0ull;
+      row.state->most[tid] = 0;
+      row.state->found[tid] = 0;
+      if (tid < SPANS) row.state->below[tid] = 0;
+      if (tid == 0) { row.state->count = 0; row.state->done = 0; row.state->open = opens; }
+    }
+  }
+  for (int i = blockIdx.x * SEL_THREADS + tid; i < SPANS * SPAN_BINS; i += gridDim.x * SEL_THREADS) row.bins[i] = 0;
+  // as many threads per key as there are, each for a stretch of the others
+  const int ours = SAMPLED / (int)gridDim.x, together = ours < SEL_THREADS ? ours : SEL_THREADS, stretch = SAMPLED / (SEL_THREADS / together);
+  const int mine = tid % together, from = tid / together * stretch;
+  for (int base = 0; base < ours; base += together) {
+    const int at = (int)blockIdx.x * ours + base + mine;
+    before[tid] = 0;
+    __syncthreads();
+    const KT key = keys[at];
+    atomicAdd(&before[mine], count_in_front(keys, from, stretch, at, key));
+    __syncthreads();
+    if (tid < together && key != ~(KT)0)
+      for (int r = 0; r < R; ++r)
+        if (rank[r] == before[tid]) row.state->ends[r] = key;
+    __syncthreads();
+  }
+}
+
+constexpr int QUEUE_BYTES = 2048;  // of a wave: room for fewer than 64 samples that wait and 16 bytes of each lane
+
+template <typename K> __device__ inline auto value_of(K key) {
+  if constexpr (sizeof(K) == 4) return __uint_as_float(key & 0x80000000u ? key & 0x7fffffffu : ~key);
+  else return __longlong_as_double((long long)(key & 0x8000000000000000ull ? key & 0x7fffffffffffffffull : ~key));
+}
+
+// The same in all lanes: kept in scalar registers, not read from LDS again for each sample that needs one of several.
+__device__ inline uint32_t in_sgpr(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ inline uint64_t in_sgpr(uint64_t v) { return (uint64_t)in_sgpr((uint32_t)(v >> 32)) << 32 | in_sgpr((uint32_t)v); }
+
+// The first pass of a workgroup: V intervals.
+//
+// What bounds it is instructions per sample, not memory: the samples are compared as they are (two instructions per interval, the masks they leave
+// counted by the scalar unit), and those inside queue up per wave, so that the two dozen instructions that bin one run on full waves and not on the five lanes
+// of 64 that have one.  (The pass over 3 x 4 M floats: 16.5 us with each instruction's few lanes on their own, 14.4 so.)
+template <typename T, int V>
+__device__ void split_pass(const T* row, long long n, int part, int parts, const Spans& s, T* queue, unsigned int* h, unsigned int* below, unsigned int* valid) {
+  using KT = typename KeyOf<T>::type;
+  constexpr int QUEUE = QUEUE_BYTES / sizeof(T);
+  T lo[V], hi[V];
+  KT from[V];
+  int shift[V];
+  unsigned int under[V] = {}, on = 0;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    lo[i] = value_of(in_sgpr((KT)s.lo[i]));
+    hi[i] = value_of(in_sgpr((KT)s.hi[i]));
+    from[i] = in_sgpr((KT)s.from[i]);
+    shift[i] = (int)in_sgpr((uint32_t)s.shift[i]);
+  }
+  const int copy = threadIdx.x & (SPAN_COPIES - 1), lane = threadIdx.x & 63;
+  unsigned int queued = 0, binned = 0;  // of this wave; the queue is a ring
+  auto bin_one = [&](T v) {
+    const KT key = KeyOf<T>::key(v);
+    KT first = from[0];
+    int sh = shift[0], base = 0;
+    asm("" : "+s"(first), "+s"(sh));
+#pragma unroll
+    for (int i = 1; i < V; ++i) {
+      KT f = from[i];
+      int t = shift[i];
+      asm("" : "+s"(f), "+s"(t));  // values: the compiler would choose between their addresses and read memory
+      const bool up = v >= lo[i];  // (the intervals ascend)
+      first = up ? f : first;
+      sh = up ? t : sh;
+      base = up ? i * SPAN_BINS : base;
+    }
+    const KT bin = (key > first ? key - first : 0) >> sh;
+    atomicAdd(&h[(base + (int)(bin < SPAN_BINS ? bin : SPAN_BINS - 1)) * SPAN_COPIES + copy], 1u);
+  };
+  for_samples(row, n, (long long)part * SEL_THREADS + threadIdx.x, (long long)parts * SEL_THREADS, [&](T v) {
+    on += __popcll(__ballot(v == v));
+    asm("" : "+s"(on));  // now: put off, the masks of a dozen samples take more scalar registers than there are
+    unsigned long long who = 0;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const unsigned long long low = __ballot(v < lo[i]);
+      under[i] += __popcll(low);
+      asm("" : "+s"(under[i]));
+      who |= __ballot(v <= hi[i]) & ~low;
+    }
+    if (__builtin_amdgcn_inverse_ballot_w64(who)) queue[(queued + __builtin_amdgcn_mbcnt_hi((unsigned int)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)who, 0u))) & (QUEUE - 1)] = v;
+    queued += __popcll(who);
+  }, [&] {
+    for (; queued - binned >= 64; binned += 64) bin_one(queue[(binned + lane) & (QUEUE - 1)]);
+  });
+  if (lane < (int)(queued - binned)) bin_one(queue[(binned + lane) & (QUEUE - 1)]);
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) atomicAdd(&below[i], under[i]);
+    atomicAdd(valid, on);
+  }
+}
+
+constexpr int SPLIT_LDS = SPANS * SPAN_BINS * SPAN_COPIES * 4 + SEL_THREADS / 64 * QUEUE_BYTES;
+
+// Grid (workgroups, metrics).
+template <typename T>
+__global__ __launch_bounds__(SEL_THREADS) void select_split_kernel(const T* __restrict__ x, long long n, long long row_stride, int levels, void* work) {
+  extern __shared__ __attribute__((aligned(16))) unsigned int h[];  // [SPANS][SPAN_BINS][SPAN_COPIES], then the waves' queues
+  __shared__ Spans s;
+  __shared__ unsigned int below[SPANS + 1];
+  const int tid = threadIdx.x, m = blockIdx.y;
+  const SplitRow row(work, m);
+  if (tid == 0) find_spans<T>(*row.state, levels, &s);
+  for (int i = tid; i < SPANS * SPAN_BINS * SPAN_COPIES; i += SEL_THREADS) h[i] = 0;
+  if (tid <= SPANS) below[tid] = 0;
+  T* queue = reinterpret_cast<T*>(reinterpret_cast<char*>(h + SPANS * SPAN_BINS * SPAN_COPIES) + (tid >> 6) * QUEUE_BYTES);
+  __syncthreads();
+  const T* xr = x + (long long)m * row_stride;
+  const int V = s.n;
+  if (V <= 1) split_pass<T, 1>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
+  else if (V == 2) split_pass<T, 2>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
+  else if (V == 3) split_pass<T, 3>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
+  else split_pass<T, SPANS>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
+  __syncthreads();
+  for (int i = tid; i < V * SPAN_BINS; i += SEL_THREADS) {
+    const unsigned int c = sum_copies(h, i, 1);
+    if (c) atomicAdd(&row.bins[i], c);
+  }
+  if (tid < V) atomicAdd(&row.state->below[tid], (unsigned long long)below[tid]);
+  if (tid == SPANS) atomicAdd(&row.state->count, (unsigned long long)below[SPANS]);
+}
+
+// A wave: the bin that holds the k-th sample, and its place in there; -1: there are not as many.
+template <int BINS>
+__device__ inline int pick_bin(const unsigned int* bins, unsigned long long k, unsigned long long* place) {
+  constexpr int EACH = BINS / 64;
+  const int lane = threadIdx.x & 63;
+  const uint4* p = reinterpret_cast<const uint4*>(bins) + lane * (EACH / 4);
+  unsigned int t[EACH];
+#pragma unroll
+  for (int j = 0; j < EACH / 4; ++j) { const uint4 v = p[j]; t[4 * j] = v.x; t[4 * j + 1] = v.y; t[4 * j + 2] = v.z; t[4 * j + 3] = v.w; }
+  unsigned long long local = 0;
+#pragma unroll
+  for (int j = 0; j < EACH; ++j) local += t[j];
+  unsigned long long upto = local;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned long long v = __shfl_up(upto, o, 64);
+    if (lane >= o) upto += v;
+  }
+  unsigned long long run = upto - local;
+  const unsigned long long here = __ballot(k >= run && k < upto);
+  if (here == 0) return -1;
+  int bin = 0;
+  unsigned long long below = 0;
+#pragma unroll
+  for (int j = 0; j < EACH; ++j) {
+    if (k >= run && k < run + t[j]) { bin = lane * EACH + j; below = run; }
+    run += t[j];
+  }
+  const int at = __ffsll((long long)here) - 1;
+  *place = k - __shfl(below, at, 64);
+  return __shfl(bin, at, 64);
+}
+
+// The bins that hold ranks, as every workgroup of the second pass finds them again.
+struct Chosen {
+  unsigned long long lo[KV_MAX_RANKS], wide[KV_MAX_RANKS];  // keys of a bin
+  unsigned long long place[KV_MAX_RANKS];                   // of a rank in its bin
+  int id[KV_MAX_RANKS];                                     // of a rank's bin, -1: its interval misses it
+  int bin_of[KV_MAX_RANKS];                                 // rank -> bin
+};
+
+// The last workgroup: ranks what was found in the U chosen bins.  Each rank has its own, narrower bins of them, again and again until what is left
+// is one value or fits a wave's lanes: at once for most samples, at most log(keys) / log(RANK_BINS) times.
+constexpr int RANK_BINS = 1024;
+template <typename T>
+__device__ void rank_found(const SplitRow& row, const Chosen& c, int R, int U, unsigned int* h, unsigned long long count, unsigned long long* out) {
+  __shared__ unsigned long long few[KV_MAX_RANKS][64], from[KV_MAX_RANKS], upto[KV_MAX_RANKS], least[KV_MAX_RANKS], most[KV_MAX_RANKS];  // of a rank
+  __shared__ int bin_of[KV_MAX_RANKS], picked[KV_MAX_RANKS], held[KV_MAX_RANKS], cnt[KV_MAX_RANKS];
+  __shared__ bool undecided;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, rest = 64 - KeyOf<T>::bits;
+  if (tid == 0) undecided = false;
+  if (tid < KV_MAX_RANKS) {
+    const unsigned int f = tid < U ? __hip_atomic_load(&row.state->found[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    cnt[tid] = f <= FOUND ? (int)f : 0;
+  }
+  __syncthreads();
+  if (tid < KV_MAX_RANKS) {
+    int u = tid < R ? c.bin_of[tid] : -1;
+    if (tid < R && u < 0) undecided = true;
+    if (u >= 0) {
+      from[tid] = __hip_atomic_load(&row.state->least[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      upto[tid] = __hip_atomic_load(&row.state->most[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (from[tid] == upto[tid]) {  // one value
+        out[tid] = from[tid] << rest;
+        u = -1;
+      } else if (cnt[u] == 0) {
+        undecided = true;
+        u = -1;
+      }
+    }
+    bin_of[tid] = u;  // -1: nothing left to do
+  }
+  __syncthreads();
+  constexpr int HELD = 4;  // samples per thread that stay in registers
+  int total = 0;
+  for (int u = 0; u < U; ++u) total += cnt[u];
+  unsigned long long key[HELD];
+  int bin[HELD];
+  auto read = [&](int first) {
+#pragma unroll
+    for (int j = 0; j < HELD; ++j) {
+      int i = first + j * SEL_THREADS + tid;
+      bin[j] = -1;
+      key[j] = 0;
+      for (int u = 0; u < U && i >= 0; i -= cnt[u++])
+        if (i < cnt[u]) { bin[j] = u; key[j] = __hip_atomic_load(&row.found[(long long)u * FOUND + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    }
+  };
+  auto each = [&](auto visit) {  // visit(rank, key, its bin) for what may be the rank's
+    int of[KV_MAX_RANKS], shift[KV_MAX_RANKS];
+    unsigned long long lo[KV_MAX_RANKS], wide[KV_MAX_RANKS];
+#pragma unroll
+    for (int r = 0; r < KV_MAX_RANKS; ++r) {  // (all on their way at once)
+      of[r] = r < R ? bin_of[r] : -1;
+      lo[r] = from[r];
+      wide[r] = upto[r] - lo[r];
+    }
+#pragma unroll
+    for (int r = 0; r < KV_MAX_RANKS; ++r) shift[r] = bin_shift<RANK_BINS>(wide[r]);
+    for (int first = 0; first < total; first += HELD * SEL_THREADS) {
+      if (total > HELD * SEL_THREADS) read(first);
+#pragma unroll
+      for (int j = 0; j < HELD; ++j) {
+        if (bin[j] < 0) continue;
+#pragma unroll
+        for (int r = 0; r < KV_MAX_RANKS; ++r)
+          if (of[r] == bin[j] && key[j] - lo[r] <= wide[r]) visit(r, key[j], (int)((key[j] - lo[r]) >> shift[r]));
+      }
+    }
+  };
+  if (total <= HELD * SEL_THREADS) read(0);
+  unsigned long long place = wave < R ? c.place[wave] : 0;
+  bool more = true;
+  while (more) {
+    for (int i = tid; i < R * RANK_BINS; i += SEL_THREADS) h[i] = 0;
+    if (tid < KV_MAX_RANKS) { least[tid] = ~0ull; most[tid] = 0; held[tid] = 0; }
+    __syncthreads();
+    each([&](int r, unsigned long long, int bin) { atomicAdd(&h[r * RANK_BINS + bin], 1u); });
+    __syncthreads();
+    if (wave < R && bin_of[wave] >= 0) {
+      const int bin = pick_bin<RANK_BINS>(h + wave * RANK_BINS, place, &place);
+      if (lane == 0) picked[wave] = bin;
+    }
+    __syncthreads();
+    each([&](int r, unsigned long long key, int bin) {
+      if (bin != picked[r]) return;
+      const int i = atomicAdd(&held[r], 1);
+      if (i < 64) few[r][i] = key;
+      atomicMin(&least[r], key);
+      atomicMax(&most[r], key);
+    });
+    __syncthreads();
+    bool left = false;
+    if (wave < R && bin_of[wave] >= 0) {
+      const int have = held[wave];
+      left = have > 64 && least[wave] != most[wave];
+      if (least[wave] == most[wave]) {
+        if (lane == 0) out[wave] = least[wave] << rest;
+      } else if (!left) {
+        const unsigned long long key = lane < have ? few[wave][lane] : ~0ull;
+        unsigned int before = 0;
+        for (int j = 0; j < have; ++j) before += few[wave][j] < key || (few[wave][j] == key && j < lane);
+        if (lane < have && before == place) out[wave] = key << rest;
+      }
+      if (lane == 0) {
+        from[wave] = least[wave];
+        upto[wave] = most[wave];
+        if (!left) bin_of[wave] = -1;
+      }
+    }
+    more = __syncthreads_or(left);
+  }
+  if (tid == 0) out[KV_MAX_RANKS] = undecided ? UNDECIDED : count;
+}
+
+// The second pass.  Grid (workgroups, metrics).
+template <typename T>
+__global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __restrict__ x, long long n, long long row_stride, Levels levels, void* work, unsigned long long* out) {
+  using KT = typename KeyOf<T>::type;
+  constexpr int ROOM = 6144;
+  static_assert(ROOM * 2 >= KV_MAX_RANKS * RANK_BINS, "rank_found's bins");
+  __shared__ __attribute__((aligned(16))) unsigned long long keys[ROOM];  // what this workgroup finds, [bin][ours]
+  __shared__ Spans s;
+  __shared__ Chosen c;
+  __shared__ unsigned int found[KV_MAX_RANKS], from[KV_MAX_RANKS];
+  __shared__ unsigned long long least[KV_MAX_RANKS], most[KV_MAX_RANKS];
+  __shared__ bool last;
+  const int tid = threadIdx.x, m = blockIdx.y, wave = tid >> 6, lane = tid & 63;
+  const SplitRow row(work, m);
+  const unsigned long long count = row.state->count;
+  const int R = count ? 2 * levels.n : 0;
+  if (tid == 0) find_spans<T>(*row.state, levels.n, &s);
+  if (tid < KV_MAX_RANKS) { found[tid] = 0; least[tid] = ~0ull; most[tid] = 0; c.id[tid] = -1; }
+  __syncthreads();
+  if (wave < R) {  // a wave per rank
+    const int span = s.of[wave >> 1];
+    const unsigned long long rank = rank_of(levels, wave, count), below = row.state->below[span];
+    unsigned long long place = 0;
+    const int bin = rank >= below ? pick_bin<SPAN_BINS>(row.bins + span * SPAN_BINS, rank - below, &place) : -1;
+    if (lane == 0 && bin >= 0) { c.id[wave] = span * SPAN_BINS + bin; c.place[wave] = place; }
+  }
+  __syncthreads();
+  int first = lane;  // a lane per rank: the first rank with the same bin, and how many such firsts there are in front of it
+  const int id = c.id[lane < KV_MAX_RANKS ? lane : 0];
+#pragma unroll
+  for (int r = KV_MAX_RANKS - 1; r >= 0; --r) first = __shfl(id, r, 64) == id ? r : first;
+  const unsigned long long firsts = __ballot(lane < R && id >= 0 && first == lane);
+  const int U = __popcll(firsts);
+  if (tid < KV_MAX_RANKS) {
+    const int u = tid < R && id >= 0 ? __popcll(firsts & ((1ull << first) - 1)) : -1;
+    c.bin_of[tid] = u;
+    if (u >= 0 && first == tid) {
+      const int span = id / SPAN_BINS, bin = id % SPAN_BINS;
+      const unsigned long long first = bin == 0 ? s.lo[span] : s.from[span] + ((unsigned long long)bin << s.shift[span]);
+      const unsigned long long behind = s.from[span] + ((unsigned long long)(bin + 1) << s.shift[span]) - 1;
+      c.lo[u] = first;
+      c.wide[u] = (bin == SPAN_BINS - 1 || behind > s.hi[span] ? s.hi[span] : behind) - first;
+    }
+  }
+  __syncthreads();
+  const unsigned int ours = U ? (ROOM / U < FOUND ? ROOM / U : FOUND) : 0;
+  auto pass = [&](auto most_bins) {
+    constexpr int MOST = decltype(most_bins)::value;
+    KT lo[MOST], wide[MOST];
+#pragma unroll
+    for (int u = 0; u < MOST; ++u) { lo[u] = in_sgpr((KT)c.lo[u < U ? u : 0]); wide[u] = in_sgpr((KT)c.wide[u < U ? u : 0]); }  // (unused ones repeat the first)
+    for_samples(x + (long long)m * row_stride, n, (long long)blockIdx.x * SEL_THREADS + tid, (long long)gridDim.x * SEL_THREADS, [&](T v) {
+      const KT key = key_or_last(v);
+      int at = -1;
+#pragma unroll
+      for (int u = MOST - 1; u >= 0; --u) at = (KT)(key - lo[u]) <= wide[u] ? u : at;
+      if (at < 0) return;
+      if (found[at] <= ours) {
+        const unsigned int i = atomicAdd(&found[at], 1u);
+        if (i < ours) keys[at * ours + i] = key;
+      }
+      if ((unsigned long long)key < least[at]) atomicMin(&least[at], (unsigned long long)key);
+      if ((unsigned long long)key > most[at]) atomicMax(&most[at], (unsigned long long)key);
+    });
+  };
+  if (U == 1) pass(std::integral_constant<int, 1>{});
+  else if (U > 1 && U <= 3) pass(std::integral_constant<int, 3>{});
+  else if (U > 3) pass(std::integral_constant<int, KV_MAX_RANKS>{});
+  __syncthreads();
+  if (tid < U && found[tid]) {
+    from[tid] = atomicAdd(&row.state->found[tid], found[tid] <= ours ? found[tid] : FOUND + 1u);  // (too many here: too many in all)
+    atomicMin(&row.state->least[tid], least[tid]);
+    atomicMax(&row.state->most[tid], most[tid]);
+  }
+  __syncthreads();
+  for (int u = 0; u < U; ++u) {
+    if (found[u] > ours) continue;
+    for (unsigned int j = tid; j < found[u] && from[u] + j < FOUND; j += SEL_THREADS)
+      __hip_atomic_store(&row.found[u * FOUND + from[u] + j], keys[u * ours + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (as in select_pass_kernel: every wave's own have been performed before its workgroup is counted)
+  __syncthreads();
+  if (tid == 0) last = __hip_atomic_fetch_add(&row.state->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  __syncthreads();
+  if (last) rank_found<T>(row, c, R, U, reinterpret_cast<unsigned int*>(keys), count, out + (long long)m * SEL_OUT);
 }
 
 // clears a selection's state, histograms and counters (a kernel, not a memset: callers may capture it)
@@ -643,9 +1209,11 @@ __global__ __launch_bounds__(256) void gap_commit_kernel(const long long* __rest
   atomicMax(&last_t[req], t);
 }
 
-// Up to SEL_FEW samples a row one workgroup per row makes all passes, beyond a launch per pass (and one that clears) spreads them.  The line lies where
-// whole calls take as long: 3 x 32768 floats 59 us in the one form, one sample more a row 63 in the other; 5000 take 43, 100000 65.
-constexpr long long SEL_FEW = 32768;
+// Which form a row's length takes, by whole calls of 3 rows (us).  Up to 512 samples each is ranked (512: 26, with one thread for each 33; by digits
+// 34 for floats, 56 for doubles).  Longer rows of floats go by digits in one workgroup per row up to SEL_FEW: 1025 take 34, 4096 36, 16384 44, by the
+// sample's intervals 41 to 44 whatever the length; 32768 take 50 and 45.  Doubles have twice the digits and go by intervals from there: 1025 take 41
+// for 57.
+constexpr long long SEL_FEW = 16384;
 
 long long select_work_bytes(int n_metrics) { return (long long)n_metrics * (sizeof(RadixState) + KV_MAX_RANKS * KV_BINS * 4 + 8); }
 
@@ -669,10 +1237,25 @@ int select_parts(long long n, int n_metrics, int dtype) {
 }
 
 template <typename T>
+int select_split(const T* x, long long n, long long row_stride, int n_metrics, int dtype, const Levels& lv, void* work, unsigned long long* out, hipStream_t stream) {
+  int parts = SAMPLE_PARTS;
+  while (parts > 1 && parts * n_metrics > 256) parts /= 2;
+  // (a larger sample of longer rows: it takes 6 us more, and what lies beyond its largest has to fit FOUND)
+  auto sample = n <= 1 << 22 ? select_sample_kernel<T, 2> : select_sample_kernel<T, 4>;
+  hipLaunchKernelGGL(sample, dim3(parts, n_metrics), dim3(SEL_THREADS), 0, stream, x, n, row_stride, lv, work);
+  const dim3 grid(select_parts(n, n_metrics, dtype), n_metrics);
+  static const bool ok = big_lds(select_split_kernel<T>);
+  if (!ok) return -2;
+  hipLaunchKernelGGL(select_split_kernel<T>, grid, dim3(SEL_THREADS), SPLIT_LDS, stream, x, n, row_stride, lv.n, work);
+  hipLaunchKernelGGL(select_collect_kernel<T>, grid, dim3(SEL_THREADS), 0, stream, x, n, row_stride, lv, work, out);
+  return (int)hipGetLastError();
+}
+
+template <typename T>
 int select(const T* x, long long n, long long row_stride, int n_metrics, int dtype, const Levels& lv, void* work, unsigned long long* out, hipStream_t stream) {
   static const bool ok = big_lds(select_few_kernel<T>) && big_lds(select_pass_kernel<T, true>);
   if (!ok) return -2;
-  if (n <= SEL_THREADS) {
+  if (n <= SEL_RANKED) {
     hipLaunchKernelGGL(select_by_rank_kernel<T>, dim3(n_metrics), dim3(SEL_THREADS), 0, stream, x, (int)n, row_stride, lv, out);
     return (int)hipGetLastError();
   }
@@ -746,6 +1329,21 @@ int kv_select_quantiles(const void* x, long long n, long long row_stride, int n_
   lv.n = n_ps;
   for (int i = 0; i < n_ps; ++i) lv.p[i] = ps[i];
   return dtype == 0 ? select((const float*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream) : select((const double*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream);
+}
+
+// The same by a sample's intervals, for the rows that kv_split_takes (scratch memory: kv_split_work_bytes): a count of kv_undecided() says that
+// kv_select_quantiles has to answer.
+int kv_split_takes(long long n, int n_metrics, int dtype) { return n > (dtype == 0 ? SEL_FEW : SEL_RANKED) && n <= SPLIT_MOST && n_metrics <= 64; }
+long long kv_split_work_bytes(int n_metrics) { return n_metrics * SPLIT_BYTES; }
+unsigned long long kv_undecided() { return UNDECIDED; }
+
+int kv_split_quantiles(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const double* ps, int n_ps, void* work, unsigned long long* out, hipStream_t stream) {
+  if (n_metrics <= 0 || !kv_split_takes(n, n_metrics, dtype) || n_ps < 1 || n_ps > KV_MAX_RANKS / 2) return -1;
+  Levels lv{};
+  lv.n = n_ps;
+  for (int i = 0; i < n_ps; ++i) lv.p[i] = ps[i];
+  return dtype == 0 ? select_split((const float*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream)
+                    : select_split((const double*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream);
 }
 
 // The same selection one pass at a time, for samples spread over several ranks: every rank runs

@@ -93,19 +93,7 @@ def batched_quantiles(samples: Any, ps: Sequence[float] = (0.5, 0.95, 0.99), ret
         x = x.unsqueeze(0)
     m = x.shape[0]
     is_double = x.dtype == torch.float64
-    found = C.select_quantiles(x, [float(p) for p in ps]).numpy().view(np.uint64).tolist()
-    out = np.full((m, len(ps)), np.nan, dtype=np.float64)
-    for i in range(m):
-        *keys, cnt = found[i]
-        if cnt == 0:
-            continue
-        for j, p in enumerate(ps):
-            p = max(0.0, min(float(p), 1.0))
-            pos = p * (cnt - 1)
-            lo = math.floor(pos)
-            v_lo = _key_to_value(keys[2 * j], is_double)
-            v_hi = _key_to_value(keys[2 * j + 1], is_double)
-            out[i, j] = v_lo if cnt == 1 or lo == math.ceil(pos) else v_lo + (pos - lo) * (v_hi - v_lo)
+    out = C.select_quantiles(x, [float(p) for p in ps]).numpy()
     if not return_stats:
         return out
     state, hist = _new_stream_state(m, x.device)

@@ -180,6 +180,31 @@ def test_quantiles_at_every_form_of_the_selection(m, n, dtype):
     assert np.array_equal(hq.distributed_quantiles(x[0], (0.5, 0.95, 0.99), OneRank, device=_dev()), hq.batched_quantiles(d[:1], (0.5, 0.95, 0.99))[0])
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [511, 513, 16385, 300_007, 5_000_001])
+def test_quantiles_whatever_the_samples_are(n, dtype):
+    """Selection by a sample's intervals on rows that a sample says little about: in order, few values, one value, two clusters with the
+    median between them (a bin with more samples than are ranked), a narrow range far from zero, mostly missing, none, infinities."""
+    from kvmini.ops import hist_quantile as hq
+
+    rng = np.random.default_rng(n)
+    g = (12 * np.exp(0.35 * rng.normal(size=n))).astype(dtype)
+    near = (rng.random(n) < 0.5) * 1e6 + 1.0 + 1e-4 * rng.random(n)
+    rows = [g, np.sort(g), np.sort(g)[::-1], np.round(g), np.full(n, 7.5), np.where(rng.random(n) < 0.5, 10.0, 20.0), near, 1e9 + rng.random(n), -g,
+            np.where(rng.random(n) < 0.01, g, np.nan), np.full(n, np.nan), np.where(rng.random(n) < 0.03, np.inf, np.where(rng.random(n) < 0.5, -np.inf, g)),
+            np.where(rng.random(n) < 0.5, -0.0, 0.0), np.where(np.arange(n) < 5, g, np.nan)]
+    x = np.stack(rows[: 14 if n < 1_000_000 else 7]).astype(dtype)
+    d = torch.from_numpy(x).to(_dev())
+    for ps in ((0.5, 0.95, 0.99), (0.0, 0.499, 0.5, 1.0), (0.9999,)):
+        got = hq.batched_quantiles(d, ps)
+        for i, row in enumerate(x):
+            v = np.sort(row[~np.isnan(row)]).astype(np.float64)
+            with np.errstate(invalid="ignore"):
+                at = [p * (len(v) - 1) for p in ps]
+                want = [v[int(a)] if a == int(a) else v[int(a)] + (a - int(a)) * (v[int(a) + 1] - v[int(a)]) for a in at] if len(v) else [np.nan] * len(ps)
+            assert np.array_equal(got[i], want, equal_nan=True), (ps, i, got[i], want)
+
+
 def test_equal_width_histogram_matches_cpu():
     from kvmini.analysis.histograms import compute_histogram
     from kvmini.ops import hist_quantile as hq
