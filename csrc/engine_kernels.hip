@@ -712,12 +712,12 @@ __device__ inline float lane_value(float v, int lane) { return __uint_as_float((
 //   PV: lane = 16*tg + dv; it owns 1/16 of the output dims and tokens {tg, tg+4, tg+8,
 //       tg+12} of the block; the 4 token groups are summed once at the end.
 template <int REP, int HD, int NWAVE, bool KV8>
-__global__ __launch_bounds__(64 * NWAVE) void paged_attention_kernel(const unsigned short* __restrict__ q, long long q_row_stride,
-                                                              const void* __restrict__ k_cache, const void* __restrict__ v_cache,
-                                                              const int* __restrict__ block_tables, int max_blocks_per_seq,
-                                                              const int* __restrict__ tok_seq, const int* __restrict__ ctx_lens,
-                                                              unsigned short* __restrict__ out, int nh, int nkv, float scale_log2e,
-                                                              const float* __restrict__ kv_scale) {
+__device__ __forceinline__ void paged_attention_row(const unsigned short* __restrict__ q, long long q_row_stride,
+                                                    const void* __restrict__ k_cache, const void* __restrict__ v_cache,
+                                                    const int* __restrict__ block_tables, int max_blocks_per_seq,
+                                                    const int* __restrict__ tok_seq, const int* __restrict__ ctx_lens,
+                                                    unsigned short* __restrict__ out, int nh, int nkv, float scale_log2e,
+                                                    const float* __restrict__ kv_scale, int t, int g) {
   constexpr int BS = 16, NT = 64 * NWAVE;
   constexpr int DQ = HD / 4;   // dims of the QK dot owned by a lane
   constexpr int NV = DQ / 8;   // 16-byte K loads per lane
@@ -727,7 +727,6 @@ __global__ __launch_bounds__(64 * NWAVE) void paged_attention_kernel(const unsig
   __shared__ float p_lds[NWAVE][REP][BS];    // per-wave probabilities of the current block
   __shared__ float m_lds[NWAVE][REP], l_lds[NWAVE][REP];
   __shared__ float o_lds[NWAVE][REP][HD];
-  const int t = blockIdx.x, g = blockIdx.y;
   // wave index in a scalar register: the block-table reads below become scalar loads, which do
   // not queue behind (and so do not drain) the K/V loads in flight
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -973,6 +972,16 @@ __global__ __launch_bounds__(64 * NWAVE) void paged_attention_kernel(const unsig
     }
     orow[i] = f2bf(den > 0.f ? num / den * v_scale : 0.f);
   }
+}
+
+template <int REP, int HD, int NWAVE, bool KV8>
+__global__ __launch_bounds__(64 * NWAVE) void paged_attention_kernel(const unsigned short* __restrict__ q, long long q_row_stride,
+                                                              const void* __restrict__ k_cache, const void* __restrict__ v_cache,
+                                                              const int* __restrict__ block_tables, int max_blocks_per_seq,
+                                                              const int* __restrict__ tok_seq, const int* __restrict__ ctx_lens,
+                                                              unsigned short* __restrict__ out, int nh, int nkv, float scale_log2e,
+                                                              const float* __restrict__ kv_scale) {
+  paged_attention_row<REP, HD, NWAVE, KV8>(q, q_row_stride, k_cache, v_cache, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, out, nh, nkv, scale_log2e, kv_scale, blockIdx.x, blockIdx.y);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1890,6 +1899,214 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const unsigne
         prefill_attention_tiles16<REP, KV8>(q, q_row_stride, k_cache, v_cache, block_tables + (long long)tile_seq[t0] * max_blocks_per_seq, tile_row0[t0], tile_pos0[t0],
                                              n0, out, nh, nkv, scale_log2e, v_scale, v_lds, k_lds);
     }
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// The same for heads of 64: 32 columns of v_mfma_f32_32x32x16_bf16 per wave, two neighbouring 16-query tiles of one head (a tile alone leaves half
+// of them idle), the pipeline of prefill_attention_tiles16 and the operand layouts of prefill_attention_tiles32.  Four heads of a group per
+// workgroup; wider groups take several.  A key row is 128 bytes: each of the 256 threads stages one 16-byte piece of K and of V per step of 32 keys.
+// The weights stay what they were in the kernel this takes over from, fp32: P = hi + lo in two bf16 operands (16 bits of mantissa; the products'
+// errors are below an output's rounding, and the errors against 64 bits are alike), for which the P V products run twice.
+// Bound by the vector unit (the exponentials and the split of the weights: some 16 instructions per score against 12 matrix instructions per 512).
+// 32 heads over 8 of keys, one prompt of 2048 tokens: 471 us with a workgroup per token (paged_attention_kernel), 62 so.
+constexpr int PA64_K_RS = 72, PA64_V_RS = 96;  // row strides (elements): 144 and 192 bytes, by the bank analysis of the 32-column path
+template <bool KV8>
+__device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* __restrict__ q, long long q_row_stride, const void* __restrict__ k_cache,
+                                                          const void* __restrict__ v_cache, const int* __restrict__ bt, int row0, int pos0, int n_q,
+                                                          unsigned short* __restrict__ out, int nh, int nkv, int g, int head, bool head_on, float scale_log2e, float v_scale,
+                                                          unsigned short* v_lds, unsigned short* k_lds) {
+  constexpr int HD = 64, BS = 16, KSTEP = 32;
+  constexpr int K_RS = PA64_K_RS, V_RS = PA64_V_RS, K_TILE = KSTEP * K_RS, V_TILE = KSTEP * V_RS;
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, hi = lane >> 5;
+  const int last_key = pos0 + n_q - 1;
+  mfma_ab qa[4];  // lane = Q[query lr][dims 16*ks + 8*hi .. +8]
+  if (head_on) {
+    const unsigned short* qp = q + (long long)(row0 + (lr < n_q ? lr : n_q - 1)) * q_row_stride + (long long)head * HD + hi * 8;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qa[ks] = *reinterpret_cast<const mfma_ab*>(qp + ks * 16);
+  }
+  mfma_cd16 o[2];
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[nt][r] = 0.f;
+  float m_run = -1e30f, l_run = 0.f;
+  // staging: thread = (key tid >> 3 of the step, piece tid & 7 of its row).  A wave's keys are rows of one cache block: its table entry and base address
+  // are scalar.  Loads run three steps ahead of the products, table entries four; past the last key they repeat it (masked in the softmax).
+  constexpr int ESZ = KV8 ? 1 : 2;
+  const int sub = __builtin_amdgcn_readfirstlane(tid >> 7), row = (tid >> 3) & 15, piece = tid & 7;
+  const int k_st = (tid >> 3) * K_RS + piece * 8, v_st = (tid >> 3) * V_RS + piece * 8;
+  const int last_blk = last_key >> 4, last_row = last_key & 15;
+  const unsigned off_row = (unsigned)((row * HD + piece * 8) * ESZ), off_end = (unsigned)(((row < last_row ? row : last_row) * HD + piece * 8) * ESZ);
+  const long long blk_bytes = (long long)nkv * BS * HD * ESZ, head_bytes = (long long)g * BS * HD * ESZ;
+  bf16x8 kr, vr;
+  auto entry = [&](int kb) __attribute__((always_inline)) {
+    const int bi = (kb >> 4) + sub;
+    return bt[bi < last_blk ? bi : last_blk];
+  };
+  auto load = [&](int kb, int blk) __attribute__((always_inline)) {
+    const long long base = (long long)blk * blk_bytes + head_bytes;
+    const unsigned off = (kb >> 4) + sub < last_blk ? off_row : off_end;
+    kr = kv_load8_at<KV8>(reinterpret_cast<const char*>(k_cache) + base, off);
+    vr = kv_load8_at<KV8>(reinterpret_cast<const char*>(v_cache) + base, off);
+  };
+  auto stage = [&](int slot) __attribute__((always_inline)) {
+    *reinterpret_cast<bf16x8*>(k_lds + slot * K_TILE + k_st) = kr;
+    *reinterpret_cast<bf16x8*>(v_lds + slot * V_TILE + v_st) = vr;
+  };
+  const int kf_base = lr * K_RS + hi * 8;
+  const int vf_base = (4 * hi + ((lane >> 2) & 3)) * V_RS + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+  // S^T of a step: register r = score(key (r & 3) + 8*(r >> 2) + 4*hi, query lr)
+  auto scores = [&](int slot) __attribute__((always_inline)) {
+    mfma_cd16 st;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st[r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const mfma_ab*>(k_lds + slot * K_TILE + kf_base + 16 * ks), qa[ks], st, 0, 0, 0);
+    return st;
+  };
+  int blk = entry(0);
+  load(0, blk);
+  blk = entry(KSTEP);
+  stage(0);
+  load(KSTEP, blk);
+  blk = entry(2 * KSTEP);
+  stage(1);
+  load(2 * KSTEP, blk);
+  blk = entry(3 * KSTEP);
+  __syncthreads();
+  mfma_cd16 cur;
+  if (head_on) cur = scores(0);
+  // One step: the rows of step i + 2 go to LDS, those of i + 3 are asked for; V of step i and K of i + 1 are read; the scores of i + 1 run beside the
+  // softmax of i, whose products end it.  MASKED: a step that reaches the diagonal of some query.
+  auto step = [&](auto masked_c, int kb, int s_v, int s_k, int s_w) __attribute__((always_inline)) {
+    constexpr bool MASKED = decltype(masked_c)::value;
+    stage(s_w);
+    load(kb + 3 * KSTEP, blk);
+    blk = entry(kb + 4 * KSTEP);
+    if (head_on) {
+      const unsigned short* vt = v_lds + s_v * V_TILE + vf_base;
+      mfma_ab va[2][2];  // V^T[dim 32*nt + lr][keys 16*s2 ..]
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+          struct { tr_b64 lo, hi; } vf;
+          vf.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_b64*)(vt + (16 * s2) * V_RS + 32 * nt));
+          vf.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_b64*)(vt + (16 * s2 + 8) * V_RS + 32 * nt));
+          va[nt][s2] = __builtin_bit_cast(mfma_ab, vf);
+        }
+      const mfma_cd16 nxt = scores(s_k);
+      float sc[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sc[r] = cur[r] * scale_log2e;
+      if constexpr (MASKED) {
+        const int lim = pos0 + lr - kb - 4 * hi;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[r] = (r & 3) + 8 * (r >> 2) <= lim ? sc[r] : -1e30f;
+      }
+      float mx = sc[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
+      const float m_old = m_run, m_new = fmaxf(m_old, half_rows_max(mx));
+      m_run = m_new;
+      mfma_ab hp[2], lp[2];
+      float psum = 0.f;
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float p = __builtin_amdgcn_exp2f(sc[8 * s2 + j] - m_new);
+          psum += p;
+          hp[s2][j] = (__bf16)p;
+          lp[s2][j] = (__bf16)(p - (float)hp[s2][j]);
+        }
+      const float corr = __builtin_amdgcn_exp2f(m_old - m_new);
+      l_run = l_run * corr + psum;  // this lane's keys only; folded after the loop
+      if (__builtin_amdgcn_ballot_w64(m_new != m_old) != 0) {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[nt][r] *= corr;
+      }
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          o[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[nt][s2], hp[s2], o[nt], 0, 0, 0);
+          o[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[nt][s2], lp[s2], o[nt], 0, 0, 0);
+        }
+      cur = nxt;
+    }
+    __syncthreads();  // step i + 2 is staged, and every wave is done with slot i % 3
+  };
+  int kb = 0, s_v = 0, s_k = 1, s_w = 2;
+  auto rotate = [&]() __attribute__((always_inline)) {
+    const int t = s_v;
+    s_v = s_k;
+    s_k = s_w;
+    s_w = t;
+  };
+  for (; kb + KSTEP - 1 <= pos0; kb += KSTEP) {
+    step(std::false_type{}, kb, s_v, s_k, s_w);
+    rotate();
+  }
+  for (; kb <= last_key; kb += KSTEP) {
+    step(std::true_type{}, kb, s_v, s_k, s_w);
+    rotate();
+  }
+  const float l = half_rows_sum(l_run);
+  if (!head_on || lr >= n_q) return;
+  const float inv = l > 0.f ? v_scale / l : 0.f;
+  unsigned short* op = out + (long long)(row0 + lr) * nh * HD + (long long)head * HD + 4 * hi;
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq) {
+      typedef __attribute__((ext_vector_type(4))) unsigned short us4;
+      us4 w;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[r] = f2bf(o[nt][4 * rq + r] * inv);
+      *reinterpret_cast<us4*>(op + 32 * nt + 8 * rq) = w;
+    }
+}
+
+// A step's attention in one launch: workgroups of a pair of tiles and four heads, then (rows > 0) one per row and kv head as in
+// paged_attention_kernel, which leave rows of prompts (context length negative) alone.  Apart, the launch that finds nothing to do costs 3 to 6 us a layer.
+template <int REP, bool KV8>
+__global__ __launch_bounds__(256, 2) void prompt_attention_64_kernel(const unsigned short* __restrict__ q, long long q_row_stride, const void* __restrict__ k_cache, const void* __restrict__ v_cache,
+                                                                     const int* __restrict__ block_tables, int max_blocks_per_seq, const int* __restrict__ tile_row0, const int* __restrict__ tile_n,
+                                                                     const int* __restrict__ tile_pos0, const int* __restrict__ tile_seq, int n_tiles, const int* __restrict__ tok_seq,
+                                                                     const int* __restrict__ ctx_lens, int rows, unsigned short* __restrict__ out, int nh, int nkv, float scale_log2e,
+                                                                     const float* __restrict__ kv_scale) {
+  __shared__ __attribute__((aligned(256))) unsigned short v_lds[3 * 32 * PA64_V_RS];
+  __shared__ __attribute__((aligned(256))) unsigned short k_lds[3 * 32 * PA64_K_RS];
+  constexpr int FOURS = (REP + 3) / 4;
+  const int pairs = (n_tiles + 1) / 2, across = nkv * FOURS, id = blockIdx.x;
+  if (id >= pairs * across) {
+    const int i = id - pairs * across;
+    paged_attention_row<REP, 64, 4, KV8>(q, q_row_stride, k_cache, v_cache, block_tables, max_blocks_per_seq, tok_seq, ctx_lens, out, nh, nkv, scale_log2e, kv_scale, i % rows, i / rows);
+    return;
+  }
+  const int g = id % across / FOURS, first = id % FOURS * 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool head_on = first + wave < REP;
+  const int head = g * REP + (head_on ? first + wave : first);
+  float v_scale = 1.f;
+  if constexpr (KV8) {
+    scale_log2e *= kv_scale[g];
+    v_scale = kv_scale[nkv + g];
+  }
+  const int t0 = (pairs - 1 - id / across) * 2, t1 = t0 + 1;  // (later tiles of a prompt see more keys: they start first)
+  const int n0 = tile_n[t0], n1 = t1 < n_tiles ? tile_n[t1] : 0;
+  const bool pair = n0 == 16 && n1 > 0 && tile_seq[t1] == tile_seq[t0] && tile_pos0[t1] == tile_pos0[t0] + 16 && tile_row0[t1] == tile_row0[t0] + 16;
+  for (int i = 0; i < 2; ++i) {
+    const int t = t0 + i, n = i ? (pair ? 0 : n1) : (pair ? 16 + n1 : n0);
+    if (n <= 0) continue;
+    __syncthreads();  // (a pass before it is done with the images)
+    prefill_attention_tiles64<KV8>(q, q_row_stride, k_cache, v_cache, block_tables + (long long)tile_seq[t] * max_blocks_per_seq, tile_row0[t], tile_pos0[t], n, out, nh, nkv, g, head, head_on, scale_log2e,
+                                   v_scale, v_lds, k_lds);
   }
 }
 
@@ -3246,15 +3463,51 @@ int kv_paged_attention(const void* q, long long q_row_stride, const void* k_cach
   return (int)hipGetLastError();
 }
 
+// Heads of 64: tiles of prompt chunks and, with rows > 0, the rows 0 .. rows - 1 by themselves (context lengths as in kv_paged_attention, negative: a
+// row of a tile), in one launch.
+int kv_prompt_attention_64(const void* q, long long q_row_stride, const void* k_cache, const void* v_cache, const int* block_tables, int max_blocks_per_seq, const int* tile_row0, const int* tile_n, const int* tile_pos0,
+                           const int* tile_seq, int n_tiles, const int* tok_seq, const int* ctx_lens, int rows, void* out, int nh, int nkv, int block_size, float scale, const float* kv_scale, hipStream_t stream) {
+  if (block_size != 16 || nkv <= 0 || nh % nkv || n_tiles < 0 || rows < 0) return -1;
+  const int rep = nh / nkv;
+  const long long grid = ((long long)(n_tiles + 1) / 2 * ((rep + 3) / 4) + rows) * nkv;
+  if (grid == 0) return 0;
+  if (grid > 0x7fffffffll) return -1;
+#define KV_LAUNCH_K(R, K8)                                                                                                                                                                       \
+  hipLaunchKernelGGL((prompt_attention_64_kernel<R, K8>), dim3((unsigned int)grid), dim3(256), 0, stream, (const unsigned short*)q, q_row_stride, k_cache, v_cache, block_tables, max_blocks_per_seq, \
+                     tile_row0, tile_n, tile_pos0, tile_seq, n_tiles, tok_seq, ctx_lens, rows, (unsigned short*)out, nh, nkv, scale * 1.4426950408889634f, kv_scale)
+#define KV_LAUNCH(R)        \
+  if (kv_scale) {           \
+    KV_LAUNCH_K(R, true);   \
+  } else {                  \
+    KV_LAUNCH_K(R, false);  \
+  }
+  switch (rep) {
+    case 1: KV_LAUNCH(1); break;
+    case 2: KV_LAUNCH(2); break;
+    case 3: KV_LAUNCH(3); break;
+    case 4: KV_LAUNCH(4); break;
+    case 6: KV_LAUNCH(6); break;
+    case 7: KV_LAUNCH(7); break;
+    case 8: KV_LAUNCH(8); break;
+    default: return -1;
+  }
+#undef KV_LAUNCH
+#undef KV_LAUNCH_K
+  return (int)hipGetLastError();
+}
+
 // Tiled causal attention for prompt chunks (see prefill_attention_kernel).  Tile arrays have
 // n_tiles entries; rows of `out` not covered by a tile are left untouched.
 int kv_prefill_attention(const void* q, long long q_row_stride, const void* k_cache, const void* v_cache, const int* block_tables, int max_blocks_per_seq,
                          const int* tile_row0, const int* tile_n, const int* tile_pos0, const int* tile_seq, void* out, int n_tiles, int nh, int nkv, int hd,
                          int block_size, float scale, const float* kv_scale, int quads, hipStream_t stream) {
   if (n_tiles <= 0) return 0;
-  if (hd != 128 || block_size != 16 || nh % nkv) return -1;
+  if ((hd != 128 && hd != 64) || block_size != 16 || nh % nkv) return -1;
   const int rep = nh / nkv;
   const float sl = scale * 1.4426950408889634f;
+  if (hd == 64)
+    return quads ? -1 : kv_prompt_attention_64(q, q_row_stride, k_cache, v_cache, block_tables, max_blocks_per_seq, tile_row0, tile_n, tile_pos0, tile_seq, n_tiles, nullptr, nullptr, 0, out, nh, nkv, block_size, scale,
+                                               kv_scale, stream);
   if (quads) {
     // every aligned group of four tiles is consecutive tiles of ONE chunk (the caller pads each
     // chunk's tiles to a multiple of four with unused ones): the 8-wave kernel, head groups of at most 4

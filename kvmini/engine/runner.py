@@ -183,6 +183,7 @@ class ModelRunner:
         # attention kernel, which spreads each context over many workgroups — the per-token kernel
         # walks a context with one workgroup per kv head (a 128k-token context: 1.9 ms per layer)
         self.dec_split_ok = bool(hasattr(self.ops, "split_decode_attention") and self.device.type == "cuda" and self.hd == 128 and self.block_size == 16)
+        self.rows_64 = getattr(self.ops, "PROMPT_ROWS_64", (0, 0)) if self.hd == 64 else (0, 0)  # short chunks of heads of 64 that are no tiles
         # a few prompt tiles deep inside a long context: every tile's key range is shared out over several workgroups
         self.pf_split_ok = bool(hasattr(self.ops, "prefill_attention_split") and self.device.type == "cuda" and self.hd == 128 and self.block_size == 16
                                 and os.environ.get("KVMINI_PREFILL_SPLIT", "1") != "0")
@@ -443,7 +444,10 @@ class ModelRunner:
                         ops.prefetch_weight(lw.wo, self._side_wgs)
                 a = ops.rope_attention_fused(qkv, positions, self.cos, self.sin, kc, vc, slots, bt, tok_seq, ctx, self.nh, self.scale, n_split=None if decode_only == 2 else 1, **kw,
                                              **(pf(lw.wo, "o") if decode_only == 1 else {}))
-            elif not decode_only and self._tiled_ok(kc):
+            elif not decode_only and self.hd == 64 and t_pad >= getattr(ops, "PROMPT_TILES_64_FROM", t_pad + 1) and self._tiled_ok(kc):
+                q = ops.rope_kv_write(qkv, positions, self.cos, self.sin, kc, vc, slots, self.nh, self.nkv, self.hd, **kw)
+                a = ops.prompt_attention_64(q, kc, vc, bt, tok_seq, self._dev("ctx_decode", t_pad), self._dev("tiles").view(4, self.max_tiles), self.scale, **kw)
+            elif not decode_only and self.hd != 64 and self._tiled_ok(kc):
                 # decode tokens: one workgroup per token; prompt chunks: 16-query MFMA tiles
                 q = ops.rope_kv_write(qkv, positions, self.cos, self.sin, kc, vc, slots, self.nh, self.nkv, self.hd, **kw)
                 if dec_split:  # few decode tokens, long contexts: split-KV over the listed rows (padding rows stay zero)
@@ -822,11 +826,14 @@ class ModelRunner:
                 # tile whose workgroup walks the whole context per kv head; as listed rows (each with its own
                 # causal length) the split-KV kernel spreads every row's walk over the chip instead.
                 as_rows = self.dec_split_ok and n <= self.DEC_SPLIT_ROWS and p0 >= self.DEC_SPLIT_MIN_CTX and n_dec + n <= self.DEC_SPLIT_ROWS
+                alone = n <= self.rows_64[0] and p0 >= self.rows_64[1]
                 if as_rows:
                     st[o_cd + i : o_cd + i + n] = pos + 1
                     st[o_dr + n_dec : o_dr + n_dec + n] = np.arange(i, i + n, dtype=np.int32)
                     n_dec += n
                     dec_max_ctx = max(dec_max_ctx, p0 + n)
+                elif alone:
+                    st[o_cd + i : o_cd + i + n] = pos + 1
                 else:
                     st[o_cd + i : o_cd + i + n] = -1  # rows of a prompt chunk: left to the tiled kernel (0 = padding row, zeroed)
                 if self.tile_quads and not as_rows:
@@ -838,7 +845,7 @@ class ModelRunner:
                         quad_min_pos = min(quad_min_pos, p0)
                 if not as_rows:
                     tile_max_ctx = max(tile_max_ctx, p0 + n)
-                for off in range(0, 0 if as_rows else n, 16):
+                for off in range(0, 0 if as_rows or alone else n, 16):
                     st[o_tl + n_tiles], st[o_tl + mt + n_tiles], st[o_tl + 2 * mt + n_tiles], st[o_tl + 3 * mt + n_tiles] = i + off, min(16, n - off), p0 + off, seq.slot
                     n_tiles += 1
                 if ch.logit_rows is not None:

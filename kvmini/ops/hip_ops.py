@@ -1181,7 +1181,7 @@ class DecodeLayers:
 
 def supports_prefill_attention(n_heads: int, k_cache: torch.Tensor) -> bool:
     nkv, bs, hd = k_cache.shape[1], k_cache.shape[2], k_cache.shape[3]
-    return hd == 128 and bs == 16 and n_heads % nkv == 0 and n_heads // nkv in GQA_RATIOS
+    return hd in (64, 128) and bs == 16 and n_heads % nkv == 0 and n_heads // nkv in GQA_RATIOS
 
 
 def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor, tiles: torch.Tensor, out: torch.Tensor, scale: float,
@@ -1194,6 +1194,24 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     so every aligned group of four is consecutive tiles of one chunk: the 8-wave kernel then
     serves a group (up to 64 queries) per workgroup (head groups of at most 4)."""
     native().prefill_attention(q, k_cache, v_cache, block_tables, tiles, out, scale, kv_scale, quads)
+    return out
+
+
+# Heads of 64: rows of a step from which its prompts go by tiles (smaller steps: each row by itself).  Measured on MI355X, steps of four layers of a 1B
+# decoder, us, by rows and by tiles: 16 rows 276 and 281, 64 345 and 361, 128 458 and 457, 192 448 and 448 (FP8 weights), 256 511 and 483 (one prompt),
+# 476 and 466 (eight), 512 723 and 611, 2048 2985 and 1359 (one), 1551 and 1158 (four).
+PROMPT_TILES_64_FROM = 192
+# ... except the rows of a short chunk behind a context (drafts to verify, the end of a prompt): a tile is walked by one workgroup per kv head, a row by one
+# whose four waves share the keys.  Chunks of 16 / 64 / 128 rows behind 64 tokens, us, by rows and by tiles: 7, 6 / 7, 7 / 11, 8; behind 512: 10, 15 /
+# 15, 16 / 27, 17; behind 8192: 103, 163 / 153, 164 / 266, 166.
+PROMPT_ROWS_64 = (64, 256)  # up to so many rows, from this position on
+
+
+def prompt_attention_64(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor, tok_seq: torch.Tensor, ctx_lens: torch.Tensor, tiles: torch.Tensor, scale: float,
+                        kv_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`paged_attention` of the rows whose context length is not negative and :func:`prefill_attention` of the tiles, heads of 64, in one launch."""
+    out = torch.empty((q.shape[0], q.shape[1] * 64), dtype=q.dtype, device=q.device)
+    native().prompt_attention_64(q, k_cache, v_cache, block_tables, tok_seq, ctx_lens, tiles, out, scale, kv_scale)
     return out
 
 

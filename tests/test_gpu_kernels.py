@@ -851,6 +851,53 @@ def test_prefill_attention_tiles_match_reference(rep, nkv, chunks):
     assert (out[~owned] == 7.0).all()
 
 
+@pytest.mark.parametrize("rep,kv8", [(1, False), (3, False), (4, False), (4, True), (6, True), (8, False)])
+def test_prefill_attention_of_heads_of_64(C, rep, kv8):
+    """Prompts of heads of 64 against attention in 64 bits: one tile, a partial one, pairs that are and are not neighbours, chunks that start inside a
+    block and behind whole steps, groups of heads that do and do not fill a workgroup's waves.  The weights are two bf16 parts: the error is that
+    of the kernel that keeps them in fp32, a rounding of the output to bf16 (2^-9 of it, in the mean about 0.6 of that)."""
+    from kvmini.ops import hip_ops
+
+    torch.manual_seed(rep)
+    nkv, hd, bs = 2, 64, 16
+    nh, max_blocks = nkv * rep, 40
+    chunks = [(0, 0, 1), (1, 0, 16), (2, 0, 33), (3, 31, 32), (4, 5, 64), (5, 200, 17), (6, 0, 300), (7, 64, 15), (8, 527, 40)]
+    nb = len(chunks) * max_blocks
+    bt = torch.randperm(nb, device=_dev()).view(len(chunks), max_blocks).int()
+    sc = (torch.rand(2, nkv, device=_dev()) + 0.5).contiguous() if kv8 else None
+    kc, vc = (_fp8_cache(nb, nkv, bs, hd, 1), _fp8_cache(nb, nkv, bs, hd, 2)) if kv8 else (_rand_cache(nb, nkv, bs, hd), _rand_cache(nb, nkv, bs, hd))
+    rows, tok_seq, ctx, tiles = 0, [], [], []
+    for seq, p0, n in chunks:
+        tiles += [(rows + off, min(16, n - off), p0 + off, seq) for off in range(0, n, 16)]
+        tok_seq += [seq] * n
+        ctx += [p0 + j + 1 for j in range(n)]
+        rows += n
+    tok_seq_t, ctx_t = (torch.tensor(v, device=_dev(), dtype=torch.int32) for v in (tok_seq, ctx))
+    q = (2 * torch.randn(rows + 1, nh, hd, device=_dev())).bfloat16()[:rows]
+    scale, kw = 1 / math.sqrt(hd), {"kv_scale": sc} if kv8 else {}
+    assert hip_ops.supports_prefill_attention(nh, kc)
+    out = torch.full((rows, nh * hd), 7.0, device=_dev(), dtype=torch.bfloat16)
+    hip_ops.prefill_attention(q, kc, vc, bt, torch.tensor(tiles + [(0, 0, 0, 0)] * 2, device=_dev(), dtype=torch.int32).T.contiguous(), out, scale, **kw)
+    per_token = hip_ops.paged_attention(q, kc, vc, bt, tok_seq_t, ctx_t, scale, max_blocks, **kw)
+    want = torch.empty(rows, nh, hd, dtype=torch.float64, device=_dev())
+    for i in range(rows):
+        k, v = (c[bt[tok_seq[i]].long()].float().double().transpose(1, 2).reshape(-1, nkv, hd)[: ctx[i]] for c in (kc, vc))
+        if kv8:
+            k, v = k * sc[0, :, None].double(), v * sc[1, :, None].double()
+        s = (q[i].double().view(nkv, rep, 1, hd) * k.transpose(0, 1)[:, None]).sum(-1) * scale
+        want[i] = (s.softmax(-1)[..., None] * v.transpose(0, 1)[:, None]).sum(2).view(nh, hd)
+    error = lambda got: ((got.double().view_as(want) - want).norm() / want.norm()).item()  # noqa: E731
+    assert error(out) <= 2.0 ** -9 and error(out) <= 1.01 * error(per_token), (error(out), error(per_token))
+    assert (out.double().view_as(want) - want).abs().max() <= 2.0 ** -7 * want.abs().max()
+    # a step of both: some chunks by rows, a padding row, and the others by tiles
+    rows_of = torch.tensor([seq in (0, 3, 7) for seq in tok_seq], device=_dev())
+    step = torch.cat((torch.where(rows_of, ctx_t, -1), torch.zeros(1, device=_dev(), dtype=torch.int32)))
+    q1 = torch.cat((q, q[:1]))
+    tiles_t = torch.tensor([t for t in tiles if t[3] not in (0, 3, 7)], device=_dev(), dtype=torch.int32).T.contiguous()
+    both = hip_ops.prompt_attention_64(q1, kc, vc, bt, torch.cat((tok_seq_t, tok_seq_t[:1])), step, tiles_t, scale, **kw)
+    assert torch.equal(both[:rows][~rows_of], out[~rows_of]) and torch.equal(both[:rows][rows_of], per_token[rows_of]) and (both[rows] == 0).all()
+
+
 @pytest.mark.parametrize("seed,rep,kv8,quads", [(1, 4, False, False), (2, 4, True, False), (3, 1, False, False), (4, 2, False, False), (5, 8, False, False), (6, 6, True, False),
                                                (7, 3, True, False), (8, 4, False, True), (9, 4, True, True), (10, 1, False, True), (11, 3, True, True), (12, 2, False, True)])
 def test_prefill_attention_random_chunk_layouts(seed, rep, kv8, quads):
