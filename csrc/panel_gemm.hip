@@ -323,12 +323,162 @@ __global__ __launch_bounds__(512) void dense_panel_kernel(const DenseArgs p) {
                    [&](int row) { return p.y + (m0 + row) * p.ldy; });
 }
 
+// ---- few tiles: panels of 128 features x up to 128 rows, K shared out where that fills the CUs -----------------------------
+// The same with one feature tile a wave (products of steps of some hundred rows: what counts is how fast one CU goes through its columns).  Eight stages
+// ahead, weights 16 KB a stage straight to registers and rows up to 16 KB through the ring.  A CU takes in 59 GB/s of what has to come from HBM and
+// 150 GB/s of what its L2 holds (measured; however much is in flight), so a stage of 64 columns is 0.27 us at best.
+// By tiles of 128 x 128 of the kernel with both operands through LDS (four waves, one a SIMD) a stage was 0.52 to 0.62 us, by tiles
+// of 32, 64 and 96 rows here 0.35, 0.39 and 0.44, of 128 0.53 (us: 256 x 3072 x 2048 22.5 -> 15.5, 1024 x 2048 x 2048 22.4 -> 16.8, 640 x 4096 x 4096 39.6 -> 34.2).
+// Eight waves of 16 features: with two feature tiles a wave, as above, only four would share a tile of 128 and each would hold twice as many weights in flight.
+struct NarrowArgs {
+  const unsigned char* w; const __bf16* x; void* y;
+  int M, N, K; long long ldx, ldy;
+  int height, tiles, stages; long long slab;  // of a tile; tiles; of a share of K; elements of a share's sums
+  const float* row_ss; int ss_parts; float inv_k, eps; int gelu;
+};
+enum NarrowMode { SUMS = 3 };  // beside Mode: fp32 sums of a share of K
+constexpr int NARROW_FEATURES = 128, NARROW_AHEAD = 8;
+__host__ __device__ constexpr int narrow_ring(int height) { return (NARROW_AHEAD + 1) * height * 128; }  // bytes: what lower tiles leave of the LDS is room for other kernels' workgroups
+constexpr int NOWHERE = 0x7ffffff0;  // a lane's offset past any buffer (no scalar offset added to it comes round to its beginning)
+
+template <int NF>
+__device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&acc)[8], rsrc_t wr, int wlane, int w0, rsrc_t xr, const int (&xsrc)[2], unsigned char* ring, int c0, int n, int wave, int lane) {
+  constexpr int AHEAD = NARROW_AHEAD, RING = AHEAD + 1, STAGE = NF * 2048;
+  static_assert(RING * STAGE <= RING_BYTES, "ring");
+  constexpr int PX = (2 * NF + 7) / 8, OPS = 2 + PX, BEFORE = PX + 1;  // memory operations of a stage, and those in front of its barrier
+  const int r = lane & 15, q = lane >> 4;
+  int xdst[PX];
+#pragma unroll
+  for (int i = 0; i < PX; ++i) xdst[i] = piece_of(wave, i, 2 * NF) * 1024;
+  const int xo[2] = {r * 128 + ((q ^ (r >> 1)) << 4), r * 128 + (((4 + q) ^ (r >> 1)) << 4)};
+  raw16 w[AHEAD][2];
+  frag_ab b[2][NF];
+  auto read = [&](int k, const unsigned char* img) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NF; ++j) b[k][j] = *reinterpret_cast<const frag_ab*>(img + xo[k] + j * 2048);
+  };
+  // stages behind the end: offsets past the buffers, where reads give zeros and ask no memory (the same number is in flight throughout)
+  auto fetch = [&](int k, int u, int st, unsigned char* dst) __attribute__((always_inline)) {
+    const bool there = st < n;
+    if (k == 0) {
+#pragma unroll
+      for (int i = 0; i < PX; ++i) dma16(xr, there ? xsrc[i] : NOWHERE, (c0 + st) * 128, dst + xdst[i]);
+    }
+    w[u][k] = load16(wr, there ? wlane : NOWHERE, w0 + (c0 + st) * 2048 + k * 1024);
+  };
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) {
+    fetch(0, s, s, ring + s * STAGE);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(1, s, s, ring + s * STAGE);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * OPS) : "memory");
+  __builtin_amdgcn_s_barrier();
+  read(0, ring);
+  int slot = 0;
+  auto stage = [&](auto uc, int s) __attribute__((always_inline)) {
+    constexpr int u = decltype(uc)::value;
+    const int next = slot + 1 == RING ? 0 : slot + 1;
+    unsigned char* dst = ring + (slot == 0 ? RING - 1 : slot - 1) * STAGE;
+    read(1, ring + slot * STAGE);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][0]), b[0][j], acc[j], 0, 0, 0);
+    fetch(0, u, s + AHEAD, dst);
+    __builtin_amdgcn_sched_barrier(0);
+    // everybody's pieces of the next stage, read from here on, have landed, and everybody's reads of this one, whose place the next fetch takes, are answered
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 2) * OPS + BEFORE) : "memory");
+    __builtin_amdgcn_s_barrier();
+    read(0, ring + next * STAGE);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][1]), b[1][j], acc[j], 0, 0, 0);
+    fetch(1, u, s + AHEAD, dst);
+    __builtin_amdgcn_sched_barrier(0);
+    slot = next;
+  };
+  int s = 0;
+  for (; s + AHEAD <= n; s += AHEAD)
+    each([&](auto uc) __attribute__((always_inline)) { stage(uc, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD>{});
+  each([&](auto uc) __attribute__((always_inline)) { if (s + decltype(uc)::value < n) stage(uc, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD - 1>{});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
+}
+
+template <int MODE>
+__global__ __launch_bounds__(512) void narrow_tiles_kernel(const NarrowArgs p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+  float* const row_scale = reinterpret_cast<float*>(ring + narrow_ring(p.height));
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // blockIdx -> (share of K, panel, tile): each XCD has a contiguous range, a panel's tiles next to one another (they share its weights through that L2)
+  const int id = xcd_range(blockIdx.x, gridDim.x), panels = p.N / NARROW_FEATURES;
+  const int m0 = id % p.tiles * p.height, panel = id / p.tiles % panels, share = id / p.tiles / panels;
+  const int rows = p.M - m0 < p.height ? p.M - m0 : p.height, nf = (rows + 31) / 32 * 2, nks = p.K / 32;
+  const int c0 = share * p.stages, n = p.K / 64 - c0 < p.stages ? p.K / 64 - c0 : p.stages;
+  if (MODE != SUMS && p.row_ss != nullptr && threadIdx.x < rows) {
+    float ss = 0.f;
+    for (int k = 0; k < p.ss_parts; ++k) ss += p.row_ss[(long long)(m0 + (int)threadIdx.x) * p.ss_parts + k];
+    row_scale[threadIdx.x] = rsqrtf(ss * p.inv_k + p.eps);
+  }
+  const rsrc_t wr = buffer_of(p.w + (long long)panel * (NARROW_FEATURES / 16) * nks * 1024, (unsigned int)(NARROW_FEATURES / 16) * nks * 1024);
+  const rsrc_t xr = buffer_of(p.x + m0 * p.ldx, (unsigned int)(((rows - 1) * p.ldx + p.K) * 2));
+  int xsrc[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 8 * piece_of(wave, i, 2 * nf) + (lane >> 3);
+    xsrc[i] = (row < rows ? row : rows - 1) * (int)(p.ldx * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+  }
+  frag_cd acc[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
+  const int w0 = wave * nks * 1024;
+  switch (nf) {
+    case 8: multiply_narrow<8>(acc, wr, lane * 16, w0, xr, xsrc, ring, c0, n, wave, lane); break;
+    case 6: multiply_narrow<6>(acc, wr, lane * 16, w0, xr, xsrc, ring, c0, n, wave, lane); break;
+    case 4: multiply_narrow<4>(acc, wr, lane * 16, w0, xr, xsrc, ring, c0, n, wave, lane); break;
+    default: multiply_narrow<2>(acc, wr, lane * 16, w0, xr, xsrc, ring, c0, n, wave, lane); break;
+  }
+  if (MODE != SUMS && p.row_ss != nullptr) __syncthreads();
+  // acc[j][e]: feature 4 q + e of the wave's 16, row 16 j + r
+  const int r = lane & 15, q = lane >> 4, f0 = panel * NARROW_FEATURES + wave * 16;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int row = 16 * j + r;
+    if (16 * j >= rows) break;
+    const long long m = m0 + row;
+    frag_cd v = acc[j];
+    if constexpr (MODE == SUMS) {
+      if (row < rows) *reinterpret_cast<frag_cd*>(reinterpret_cast<float*>(p.y) + share * p.slab + m * p.ldy + f0 + 4 * q) = v;
+    } else {
+      const float by = p.row_ss != nullptr ? row_scale[row] : 1.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] *= by;
+      unsigned short* const y = reinterpret_cast<unsigned short*>(p.y) + m * p.ldy;
+      if constexpr (MODE == GATED) {  // a tile is 8 gate rows and their 8 up rows: lanes q < 2 have gates, q + 2 the ups of the same features
+        frag_cd o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float up = __shfl_xor(v[e], 32, 64), z = p.gelu ? 1.5957691216057308f * (v[e] + 0.044715f * v[e] * v[e] * v[e]) : v[e];
+          o[e] = v[e] / (1.f + __expf(-z)) * up;
+        }
+        if (q < 2 && row < rows) *reinterpret_cast<uint2*>(y + f0 / 2 + 4 * q) = pack4(o);
+      } else {
+        if constexpr (MODE == SQUARED) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { v[e] = fmaxf(v[e], 0.f); v[e] *= v[e]; }
+        }
+        if (row < rows) *reinterpret_cast<uint2*>(y + f0 + 4 * q) = pack4(v);
+      }
+    }
+  }
+}
+
 template <auto KERNEL, class Args>
-int launch(const Args& a, int grid, hipStream_t s) {
+int launch(const Args& a, int grid, hipStream_t s, int lds = RING_BYTES + ROWS * 4) {
   constexpr int LDS = RING_BYTES + ROWS * 4;
   static const hipError_t lds_ok = hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (lds_ok != hipSuccess) return -2;
-  hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(512), LDS, s, a);
+  hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(512), lds, s, a);
   return (int)hipGetLastError();
 }
 
@@ -381,6 +531,29 @@ int kv_dense_panels(const void* Wp, const void* x, void* y, int M, int N, int K,
     case 0: return launch<dense_panel_kernel<PLAIN>>(a, (int)grid, stream);
     case 2: case 4: return launch<dense_panel_kernel<GATED>>(a, (int)grid, stream);
     case 5: return launch<dense_panel_kernel<SQUARED>>(a, (int)grid, stream);
+  }
+  return -1;
+}
+
+// Wp: one packed matrix [N, K].  Tiles of `height` rows (a multiple of 32 up to 128) x 128 features; epi 0, 2, 4, 5 as above, 1: fp32 sums
+// [splits][M][N] of shares of `stages` x 64 columns (`slab` elements apart; other epilogues: one share).  N % 128 == 0, the rest as above.
+int kv_narrow_tiles(const void* Wp, const void* x, void* y, int M, int N, int K, long long ldx, long long ldy, int epi, int height, int splits, int stages, long long slab, const float* row_ss, int ss_parts, float eps,
+                    hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || N % NARROW_FEATURES || (K & 63) || K > (1 << 21) || (ldx & 7) || ldx < K || ldx >= (1 << 22) || ((uintptr_t)x & 15) || ((uintptr_t)y & 15) || (ldy & 3)) return -1;
+  if (height <= 0 || height > 128 || (height & 31) || splits <= 0 || stages <= 0 || (long long)(splits - 1) * stages >= K / 64 || (long long)splits * stages < K / 64 || (epi != 1 && splits != 1)) return -1;
+  NarrowArgs a;
+  a.w = (const unsigned char*)Wp; a.x = (const __bf16*)x; a.y = y;
+  a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldy = ldy;
+  a.height = height; a.tiles = (M + height - 1) / height; a.stages = stages; a.slab = slab;
+  a.row_ss = row_ss; a.ss_parts = ss_parts; a.inv_k = 1.f / (float)K; a.eps = eps; a.gelu = epi == 4;
+  const long long grid = (long long)splits * (N / NARROW_FEATURES) * a.tiles;
+  if (grid > 0x7fffffffll) return -1;
+  const int lds = narrow_ring(height) + height * 4;
+  switch (epi) {
+    case 0: return launch<narrow_tiles_kernel<PLAIN>>(a, (int)grid, stream, lds);
+    case 1: return launch<narrow_tiles_kernel<SUMS>>(a, (int)grid, stream, lds);
+    case 2: case 4: return launch<narrow_tiles_kernel<GATED>>(a, (int)grid, stream, lds);
+    case 5: return launch<narrow_tiles_kernel<SQUARED>>(a, (int)grid, stream, lds);
   }
   return -1;
 }

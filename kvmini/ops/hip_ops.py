@@ -369,6 +369,36 @@ def _plan_wide(m: int, n_pad: int, k: int, fp8: int, may_split: bool) -> Tuple[i
     return best[1]
 
 
+NARROW_HEIGHTS = (32, 64, 96)  # rows of a tile
+
+
+@functools.lru_cache(maxsize=None)
+def _plan_narrow(m: int, n: int, k: int, may_split: bool = False) -> Optional[Tuple[int, int, int]]:
+    """How bf16 weights are multiplied by one round of tiles of 128 features x up to 96 rows (``csrc/panel_gemm.hip``): (rows of a tile, K splits,
+    stages of 64 columns per split), or None for the kernels below.
+
+    Only where the tiles fit the CUs in one round: there the time is how fast one CU goes through its columns, and these tiles do 64 of them in 0.35 to
+    0.44 us where the tiled GEMM's 128 x 128 take 0.52 to 0.62.  Over more rounds both are bound by what the chip reads, and wider tiles read less
+    (512 tiles of 64 rows, 1024 x 4096 x 4096: 60 us, tiled GEMM 41).  With 128 rows a stage is 0.53 us and both are alike (1024 x 4096 x 4096 42 and
+    41), so that height is not offered.  The lowest height that fits: the lower, the faster a stage.
+
+    K in as many splits as the tiled GEMM takes: partial sums stay in fp32, and as many slabs are read behind it.  Fewer gave back in the loop what
+    they saved in slabs (256 x 4096 x 4096 in 2 and 4 splits 22.1 and 22.2 us, 380 x 4096 x 14336 70.7 and 65.6).  In splits only for up to 2048
+    outputs: CUs have work in either kernel then, and what is left to gain in the loop can be lost around it (steps of four layers, us: 150 rows with
+    products of 2048 x 8192 506 and 485, 136 rows with 4096 x 4096 904 and 916).
+
+    Measured on MI355X with cold weights, us, tiled GEMM and this: 136 x 2048 x 2048 9.2 and 4.4, 500 x 2048 x 2048 14.2 and 11.1, 1000 x 2048 x 2048 23.7
+    and 17.7, 256 x 3072 x 2048 21.9 and 15.4, 380 x 8192 x 2048 25.4 and 22.8, 176 x 16384 x 2048 28.4 and 29.3 (the only one of 45 sizes that is
+    slower), 500 x 1024 x 4096 37.8 and 26.0, 760 x 4096 x 4096 42.4 and 39.4, 256 x 9216 x 4096 45.4 and 39.7."""
+    splits, nst = _plan_wide(m, n, k, 0, may_split)[3], k // 64
+    if n % 128 or (splits > 1 and n > 2048):
+        return None
+    for height in NARROW_HEIGHTS:
+        if -(-m // height) * (n // 128) * splits <= _num_cus():
+            return height, splits, -(-nst // splits)
+    return None
+
+
 PANEL_HEIGHTS = (256, 224, 192, 160, 128, 96)  # rows of a tile (64 and 32: the panels' weights are then read more often than they are multiplied)
 
 
@@ -431,7 +461,19 @@ def _wide(w: Union[PackedLinear, "_ExpandedView"], h: Union[torch.Tensor, "Norme
         C.wide_gemm_fp8a(w.wp, w.n_pad, w.k, x8, a_scale, out, epi, bm, bn, variant, 1, sps, ss, eps, w.wscale, True)
         n_true = w.n // 2 if epi in GATED else w.n
         return out if n_true == n_out else out[:, :n_true]
-    cut = _plan_panels(m, w.n_pad, w.k, may_split) if w.wscale is None and x.data_ptr() % 16 == 0 and w.k <= x.stride(0) < 1 << 22 else None
+    panels = w.wscale is None and x.data_ptr() % 16 == 0 and w.k <= 1 << 21 and w.k <= x.stride(0) < 1 << 22
+    narrow = _plan_narrow(m, w.n_pad, w.k, may_split) if panels else None
+    if narrow is not None:
+        height, splits, sps = narrow
+        if splits > 1:
+            out = torch.empty((splits, m, w.n_pad), dtype=torch.float32, device=x.device)
+            C.narrow_tiles(w.wp, w.n_pad, w.k, x, out, 1, height, splits, sps, None, 0.0)
+            return Partial(out, ss, eps, w.k)
+        out = torch.empty((m, w.n_pad // 2 if epi in GATED else w.n_pad), dtype=torch.bfloat16, device=x.device)
+        C.narrow_tiles(w.wp, w.n_pad, w.k, x, out, epi, height, 1, sps, ss, eps)
+        n_true = w.n // 2 if epi in GATED else w.n
+        return out if n_true == out.shape[1] else out[:, :n_true]
+    cut = _plan_panels(m, w.n_pad, w.k, may_split) if panels else None
     if cut is not None:
         out = torch.empty((m, w.n_pad // 2 if epi in GATED else w.n_pad), dtype=torch.bfloat16, device=x.device)
         C.dense_panels(w.wp, w.n_pad, w.k, x, out, epi, *cut, ss, eps)

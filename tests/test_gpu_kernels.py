@@ -1389,6 +1389,52 @@ def test_dense_panels_of_every_height(C, M, N, K, cut):
             assert (out[M] == 7).all()
 
 
+@pytest.mark.parametrize("M,N,K,splits", [(1, 128, 64, 1), (31, 128, 576, 3), (65, 384, 640, 2), (95, 256, 1152, 5), (128, 256, 512, 8), (129, 640, 960, 4), (200, 128, 4096, 7), (300, 384, 1088, 2)])
+def test_narrow_tiles_of_every_height(C, M, N, K, splits):
+    """Tiles of 128 features by 32 to 128 rows: ragged last tiles and last shares of K, shares shorter and longer than the stages in flight, rows at a
+    stride, each epilogue.  One matrix instruction per 32 columns in order, as the tiled kernel's: the same bits, for sums of shares of K too."""
+    torch.manual_seed(M)
+    x = torch.randn(M, K + 16, device="cuda").bfloat16()[:, 8 : 8 + K]
+    wp = C.pack_weight((torch.randn(N, K, device="cuda") * 0.1).bfloat16())
+    ss, stages = torch.rand(M, 3, device="cuda") * K, -(-(K // 64) // splits)
+    for height in (32, 64, 96, 128):
+        for epi in (0, 2, 4, 5):
+            for rows in (None, ss):
+                want = torch.empty((M, N // 2 if epi in (2, 4) else N), device="cuda", dtype=torch.bfloat16)
+                got = torch.full((M + 1, want.shape[1]), 7.0, device="cuda", dtype=torch.bfloat16)
+                C.wide_gemm(wp, N, K, x, want, epi, 128, 128, 0, 1, K // 64, rows, 1e-5, None, True)
+                C.narrow_tiles(wp, N, K, x, got[:M], epi, height, 1, K // 64, rows, 1e-5)
+                assert torch.equal(got[:M], want) and (got[M] == 7).all(), (height, epi)
+        want, got = (torch.full((splits, M, N), float("nan"), device="cuda") for _ in range(2))
+        C.wide_gemm(wp, N, K, x, want, 1, 128, 128, 0, splits, stages, None, 0.0, None, True)
+        C.narrow_tiles(wp, N, K, x, got, 1, height, splits, stages, None, 0.0)
+        assert torch.equal(got, want), height
+
+
+def test_one_round_of_narrow_tiles():
+    """The op layer's rule: narrow tiles where they are one round over the CUs, split where the tiled GEMM splits, the same result at a stride and with
+    outputs that are no multiple of 128 (which stay where they were)."""
+    from kvmini.ops import hip_ops as ops
+
+    cus, taken = ops._num_cus(), 0
+    for m in range(129, 2049, 61):
+        for n, k, may_split in ((2048, 2048, True), (3072, 2048, False), (4096, 14336, True), (1024, 4096, False), (9216, 4096, False), (16384, 2048, False)):
+            plan = ops._plan_narrow(m, n, k, may_split)
+            if plan is not None:
+                height, splits, stages = plan
+                taken += 1
+                assert -(-m // height) * (n // 128) * splits <= cus and (splits - 1) * stages < k // 64 <= splits * stages
+                assert splits > 1 or ops._plan_wide(m, n, k, 0, may_split)[3] == 1
+    assert taken > 20 and ops._plan_narrow(200, 2112, 2048) is None
+    torch.manual_seed(2)
+    for m, n, k in ((150, 1024, 2048), (150, 1056, 2048), (400, 2048, 2048)):
+        x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") * 0.1).bfloat16()
+        pw, ref = ops.PackedLinear(w), x.double() @ w.double().T
+        for rows in (x, torch.cat((x, x), 1)[:, :k]):
+            got = ops.linear(rows, pw)
+            assert ((got.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2.0**-20 * (x.double().abs() @ w.double().abs().T)).all()
+
+
 def test_matrices_of_many_outputs_go_by_panels():
     """The op layer's rule: up to one round of 128 x 128 tiles the tiled kernel, beyond it panels whose cut covers all of them; the same rows either way."""
     from kvmini.ops import hip_ops as ops
