@@ -41,6 +41,11 @@ constexpr int RING_BYTES = 144 * 1024;
 // stages of 64 columns in flight, and one more in the ring: as many as registers (16 of weights a stage) and LDS (2 KiB of rows per row tile) hold
 constexpr int ahead(int nf) { return nf > 14 ? 3 : nf > 12 ? 4 : nf > 10 ? 5 : 6; }
 
+// What is multiplied: bf16 by bf16, or e4m3 rows by e4m3 weights or by MXFP4 ones (e2m1 in blocks of 32, an E8M0 scale each).  Of rows of bytes K, ldx
+// and a stage's columns count pairs: then a stage is 128 columns and as many bytes of rows and of e4m3 weights as one of 64 columns of bf16.
+enum Numbers { BF16 = 0, FP8 = 1, MXFP4 = 2 };
+struct Scales { const float* w; const float* x; const int* blocks; };  // of the outputs (e4m3 weights) and of the rows; of the blocks, [N/16][stages][16], a byte each
+
 struct PanelArgs {
   const unsigned char* w; const __bf16* x; unsigned short* y;
   int N, K; long long ldx, ldy;
@@ -58,9 +63,26 @@ __device__ inline unsigned int f2bf(float f) {
 __device__ inline uint2 pack4(frag_cd v) { return make_uint2(f2bf(v[0]) | f2bf(v[1]) << 16, f2bf(v[2]) | f2bf(v[3]) << 16); }
 
 __device__ inline rsrc_t buffer_of(const void* p, unsigned int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00027000); }
+__device__ inline int load4(rsrc_t r, int lane_off, int off) { return __builtin_bit_cast(int, __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, off, 0)); }
 __device__ inline raw16 load16(rsrc_t r, int lane_off, int off) { return __builtin_bit_cast(raw16, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0)); }
 // one LDS-DMA piece: lane l's 16 bytes land at lds + 16 l
 __device__ inline void dma16(rsrc_t r, int lane_off, int off, void* lds) { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, lane_off, off, 0, 0); }
+
+typedef __attribute__((ext_vector_type(8))) int raw32;
+// an operand of 128 bytes' columns from its two pieces of 64
+template <class T>
+__device__ inline raw32 both(T a, T b) { return __builtin_shufflevector(__builtin_bit_cast(__attribute__((ext_vector_type(4))) int, a), __builtin_bit_cast(__attribute__((ext_vector_type(4))) int, b), 0, 1, 2, 3, 4, 5, 6, 7); }
+// packed e2m1 weights (a lane has 4 x 8 columns, 32 apart) to the operand, where it has 32 in a row: a transposition over the quarters of the lanes
+__device__ inline raw32 fp4_operand(raw16 w) {
+  const auto a = __builtin_amdgcn_permlane16_swap(w[0], w[1], false, false), b = __builtin_amdgcn_permlane16_swap(w[2], w[3], false, false);
+  const auto c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false), d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  return (raw32){(int)c[0], (int)d[0], (int)c[1], (int)d[1], 0, 0, 0, 0};
+}
+constexpr int UNIT = 0x7f7f7f7f;  // block scales of one
+template <int Q>
+__device__ inline frag_cd product(raw32 w, raw32 x, frag_cd c, int blocks) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, x, c, Q == MXFP4 ? 4 : 0, 0, 0, Q == MXFP4 ? blocks : UNIT, 0, UNIT);
+}
 
 // The 8-row piece of a stage that slot i of a wave copies; where there are fewer pieces than slots a piece is copied twice (the same bytes), so
 // that every wave has the same number in flight.
@@ -72,9 +94,10 @@ __device__ inline int piece_of(int wave, int i, int pieces) {
 template <class F, int... U>
 __device__ __attribute__((always_inline)) inline void each(const F& f, std::integer_sequence<int, U...>) { (f(std::integral_constant<int, U>{}), ...); }
 
-// acc[i][j] += the wave's feature tile i x rows 16 j .. of NF row tiles (a multiple of two), over n stages of 64 columns
-template <int NF>
-__device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
+// acc[i][j] += the wave's feature tile i x rows 16 j .. of NF row tiles (a multiple of two), over n stages of 64 columns.  MXFP4: sr, s0 and s1 of the
+// block scales as wr, w0 and w1 of the weights.
+template <int NF, int Q>
+__device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t sr, int s0, int s1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
   constexpr int AHEAD = ahead(NF), RING = AHEAD + 1, STAGE = NF * 2048;
   static_assert(RING * STAGE <= RING_BYTES, "ring");
   constexpr int PX = (2 * NF + 7) / 8, OPS = 4 + PX;  // pieces of x and memory operations per wave and stage
@@ -86,12 +109,13 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
   // rows of 128 bytes whose 16-byte chunks are swizzled by (row >> 1) & 7: a fragment read touches 16 distinct chunks per 16 lanes
   const int xo[2] = {r * 128 + ((q ^ (r >> 1)) << 4), r * 128 + (((4 + q) ^ (r >> 1)) << 4)};
   raw16 w[AHEAD][2][2];
-  frag_ab b[2][4];
+  int scale[AHEAD][2];
+  frag_ab b[2][4];  // of a batch: four row tiles' k-step, or two row tiles' both halves of a stage
   auto read = [&](int set, const unsigned char* img, int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int f = 4 * t + e;
-      b[set][e] = *reinterpret_cast<const frag_ab*>(img + xo[f / NF] + f % NF * 2048);
+      b[set][e] = *reinterpret_cast<const frag_ab*>(img + (Q == BF16 ? xo[f / NF] + f % NF * 2048 : xo[f & 1] + f / 2 * 2048));
     }
   };
   auto column = [&](int s) __attribute__((always_inline)) { return s < n ? s : n - 1; };  // of stage s (behind the end the last one is fetched again)
@@ -102,9 +126,14 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
       if (t == i * NB / PX) dma16(xr, xsrc[i], st * 128, dst + xdst[i]);
 #pragma unroll
     for (int k = 0; k < 2; ++k)
-      if (t == (k == 0 ? (NF - 1) / 4 : NB - 1)) {
-        w[u][k][0] = load16(wr, w0, st * 2048 + k * 1024);
-        w[u][k][1] = load16(wr, w1, st * 2048 + k * 1024);
+      if (t == (k == 0 && Q == BF16 ? (NF - 1) / 4 : NB - 1)) {
+        if (Q == MXFP4 && k == 1) {
+          scale[u][0] = load4(sr, s0, st * 64);
+          scale[u][1] = load4(sr, s1, st * 64);
+        } else {
+          w[u][k][0] = load16(wr, w0, st * (Q == MXFP4 ? 1024 : 2048) + k * 1024);
+          w[u][k][1] = load16(wr, w1, st * (Q == MXFP4 ? 1024 : 2048) + k * 1024);
+        }
       }
   };
 #pragma unroll
@@ -121,7 +150,7 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
   // The barrier before the last batch of stage s: everybody's pieces of stage s + 1, read from there on, have landed, and everybody's reads of stage s,
   // whose place stage s + RING takes, are answered.
   constexpr int BEFORE = [] {  // memory operations of a stage in front of its last batch
-    int c = (NF - 1) / 4 < NB - 1 ? 2 : 0;
+    int c = Q == BF16 && (NF - 1) / 4 < NB - 1 ? 2 : 0;
     for (int i = 0; i < PX; ++i) c += i * NB / PX < NB - 1;
     return c;
   }();
@@ -132,6 +161,8 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
     const unsigned char* nxt = ring + next * STAGE;
     unsigned char* dst = ring + (slot == 0 ? RING - 1 : slot - 1) * STAGE;
     const int sa = column(s + AHEAD);
+    raw32 a[2];
+    int by[2];
 #pragma unroll
     for (int t = 0; t < NB; ++t) {
       const int set = (u * NB + t) & 1;
@@ -141,11 +172,25 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
       }
       read(set ^ 1, t + 1 < NB ? cur : nxt, t + 1 < NB ? t + 1 : 0);
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (Q == BF16) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int f = 4 * t + e, k = f / NF, j = f % NF;
+        for (int e = 0; e < 4; ++e) {
+          const int f = 4 * t + e, k = f / NF, j = f % NF;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][k][i]), b[set][e], acc[i][j], 0, 0, 0);
+          for (int i = 0; i < 2; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][k][i]), b[set][e], acc[i][j], 0, 0, 0);
+        }
+      } else {
+        if (t == 0) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            a[i] = Q == MXFP4 ? fp4_operand(w[u][0][i]) : both(w[u][0][i], w[u][1][i]);
+            by[i] = Q == MXFP4 ? scale[u][i] >> (8 * q) : 0;
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e += 2)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) acc[i][2 * t + e / 2] = product<Q>(a[i], both(b[set][e], b[set][e + 1]), acc[i][2 * t + e / 2], by[i]);
       }
       if constexpr (more) fetch(t, u, sa, dst);
       __builtin_amdgcn_sched_barrier(0);
@@ -161,23 +206,24 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
 }
 
-__device__ __attribute__((always_inline)) inline void multiply(int nf, frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
+template <int Q>
+__device__ __attribute__((always_inline)) inline void multiply(int nf, frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t sr, int s0, int s1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
   switch (nf) {
-    case 16: multiply_rows<16>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
-    case 14: multiply_rows<14>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
-    case 12: multiply_rows<12>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
-    case 10: multiply_rows<10>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
-    case 8: multiply_rows<8>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
-    case 6: multiply_rows<6>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
-    case 4: multiply_rows<4>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
-    default: multiply_rows<2>(acc, wr, w0, w1, xr, xsrc, ring, n, wave, lane); break;
+    case 16: if constexpr (Q != MXFP4) multiply_rows<16, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;  // (of MXFP4 224 rows: what transposes its weights takes the registers)
+    case 14: multiply_rows<14, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 12: multiply_rows<12, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 10: multiply_rows<10, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 8: multiply_rows<8, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 6: multiply_rows<6, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 4: multiply_rows<4, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    default: multiply_rows<2, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
   }
 }
 
-// What a wave stores of its 32 features from f0 on.  acc[i][j][e]: feature 16 i + 4 q + e, row 16 j + r, to be multiplied by scale(j); gate(g, u) of a
+// What a wave stores of its 32 features from f0 on.  acc[i][j][e]: feature 16 i + 4 q + e, row 16 j + r, to be multiplied by scale(i, j); gate(g, u) of a
 // gated product; out(row): the row's outputs.
 template <int MODE, class Scale, class Gate, class Out>
-__device__ __attribute__((always_inline)) inline void store_rows(frag_cd (&acc)[2][16], int rows, int f0, int lane, Scale scale, Gate gate, Out out) {
+__device__ __attribute__((always_inline)) inline void store_rows(const frag_cd (&acc)[2][16], int rows, int f0, int lane, Scale scale, Gate gate, Out out) {
   const int r = lane & 15, q = lane >> 4;
 #pragma unroll
   for (int j = 0; j < 16; j += 2) {
@@ -186,9 +232,9 @@ __device__ __attribute__((always_inline)) inline void store_rows(frag_cd (&acc)[
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       frag_cd a = acc[0][j + t], b = acc[1][j + t];
-      const float by = scale(j + t);
+      const frag_cd by_a = scale(0, j + t), by_b = scale(1, j + t);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { a[e] *= by; b[e] *= by; }
+      for (int e = 0; e < 4; ++e) { a[e] *= by_a[e]; b[e] *= by_b[e]; }
       if constexpr (MODE == GATED) {  // a tile is 8 gate rows and their 8 up rows: the upper half of the lanes takes the other tile's
         frag_cd o;
 #pragma unroll
@@ -257,10 +303,10 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  multiply(nf, acc, wr, w0, w1, xr, xsrc, ring, p.K / 64, wave, lane);
+  multiply<BF16>(nf, acc, wr, w0, w1, wr, 0, 0, xr, xsrc, ring, p.K / 64, wave, lane);
   const int f0 = panel * p.features + wave * 32;
   if (wave * 32 >= p.features || f0 >= p.N) return;
-  store_rows<MODE>(acc, rows, f0, lane, [](int) { return 1.f; }, [&](float g, float u) { return expert_gate(g, u, p.gate); },
+  store_rows<MODE>(acc, rows, f0, lane, [](int, int) { return (frag_cd){1.f, 1.f, 1.f, 1.f}; }, [&](float g, float u) { return expert_gate(g, u, p.gate); },
                    [&](int row) { return p.y + (long long)row_of[row] * p.ldy; });
 }
 
@@ -276,11 +322,23 @@ struct DenseArgs {
   int height[2], tiles[2];  // of a tile, and tiles per panel: of the first `panels`, and of those behind them
   int panels;
   const float* row_ss; int ss_parts; float inv_k, eps; int gelu;
+  Scales scales;
 };
 
-template <int MODE>
-__global__ __launch_bounds__(512) void dense_panel_kernel(const DenseArgs p) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+// of row i of a tile from row m0: the root of its mean square, and the scale of its bytes
+template <int Q, class Args>
+__device__ inline float scale_of_row(const Args& p, long long m) {
+  float by = 1.f;
+  if (p.row_ss != nullptr) {
+    float ss = 0.f;
+    for (int k = 0; k < p.ss_parts; ++k) ss += p.row_ss[m * p.ss_parts + k];
+    by = rsqrtf(ss * p.inv_k + p.eps);
+  }
+  return Q == BF16 ? by : by * p.scales.x[m];
+}
+
+template <int MODE, int Q>
+__device__ __attribute__((always_inline)) inline void dense_panel(const DenseArgs& p, unsigned char* ring) {
   float* const row_scale = reinterpret_cast<float*>(ring + RING_BYTES);  // [ROWS]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int first = p.panels * p.tiles[0];
@@ -290,15 +348,14 @@ __global__ __launch_bounds__(512) void dense_panel_kernel(const DenseArgs p) {
   const int panel = (behind ? p.panels : 0) + id / tiles, m0 = id % tiles * height;
   const int rows = p.M - m0 < height ? p.M - m0 : height;
   const int nf = (rows + 31) / 32 * 2, nks = p.K / 32;
-  if (p.row_ss != nullptr) {
-    const int i = threadIdx.x < rows ? threadIdx.x : rows - 1;
-    float ss = 0.f;
-    for (int k = 0; k < p.ss_parts; ++k) ss += p.row_ss[(long long)(m0 + i) * p.ss_parts + k];
-    if (threadIdx.x < ROWS) row_scale[threadIdx.x] = rsqrtf(ss * p.inv_k + p.eps);
-  }
+  const bool scaled = Q != BF16 || p.row_ss != nullptr;
+  if (scaled && threadIdx.x < rows) row_scale[threadIdx.x] = scale_of_row<Q>(p, m0 + (int)threadIdx.x);
   const int have = p.N / 16 - panel * (FEATURES / 16) < FEATURES / 16 ? p.N / 16 - panel * (FEATURES / 16) : FEATURES / 16;  // feature tiles; past them reads give zeros
-  const rsrc_t wr = buffer_of(p.w + (long long)panel * (FEATURES / 16) * nks * 1024, (unsigned int)have * nks * 1024);
-  const int w0 = 2 * wave * nks * 1024 + lane * 16, w1 = w0 + nks * 1024;
+  const int tile_bytes = nks * (Q == MXFP4 ? 512 : 1024);
+  const rsrc_t wr = buffer_of(p.w + (long long)panel * (FEATURES / 16) * tile_bytes, (unsigned int)have * tile_bytes);
+  const int w0 = 2 * wave * tile_bytes + lane * 16, w1 = w0 + tile_bytes;
+  const rsrc_t sr = Q == MXFP4 ? buffer_of(p.scales.blocks + (long long)panel * (FEATURES / 16) * nks * 8, (unsigned int)have * nks * 32) : wr;
+  const int s0 = 2 * wave * nks * 32 + (lane & 15) * 4, s1 = s0 + nks * 32;
   const rsrc_t xr = buffer_of(p.x + m0 * p.ldx, (unsigned int)(((rows - 1) * p.ldx + p.K) * 2));
   int xsrc[4];
 #pragma unroll
@@ -311,16 +368,38 @@ __global__ __launch_bounds__(512) void dense_panel_kernel(const DenseArgs p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  multiply(nf, acc, wr, w0, w1, xr, xsrc, ring, p.K / 64, wave, lane);
-  if (p.row_ss != nullptr) __syncthreads();
+  multiply<Q>(nf, acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, p.K / 64, wave, lane);
+  if (scaled) __syncthreads();
   const int f0 = panel * FEATURES + wave * 32;
   if (f0 >= p.N) return;
-  store_rows<MODE>(acc, rows, f0, lane, [&](int j) { return p.row_ss != nullptr ? row_scale[16 * j + (lane & 15)] : 1.f; },
+  frag_cd of_features[2] = {{1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}};
+  if constexpr (Q == FP8) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) of_features[i] = *reinterpret_cast<const frag_cd*>(p.scales.w + f0 + 16 * i + 4 * (lane >> 4));
+  }
+  store_rows<MODE>(acc, rows, f0, lane, [&](int i, int j) { return of_features[i] * (scaled ? row_scale[16 * j + (lane & 15)] : 1.f); },
                    [&](float g, float u) {  // silu(z) = z sigmoid(z); gelu_tanh(z) = z sigmoid(2 sqrt(2 / pi) (z + 0.044715 z^3))
                      const float z = p.gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
                      return g / (1.f + __expf(-z)) * u;
                    },
                    [&](int row) { return p.y + (m0 + row) * p.ldy; });
+}
+
+template <int MODE>
+__global__ __launch_bounds__(512) void dense_panel_kernel(const DenseArgs p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+  dense_panel<MODE, BF16>(p, ring);
+}
+
+// Quantised weights and rows: the bytes of a stage and its time are those of bf16, its columns twice as many (the scaled matrix
+// instruction takes 128 columns in the time of two of 32 of bf16).  A stage's fragments come in batches of two row tiles and both halves, and its weights
+// stay until its last batch.  MXFP4 weights are half the bytes, a block's scales their own load; they are transposed once a stage.  Against tiles of 128 and 256 rows
+// through LDS (us): e4m3 2048 x 28672 x 4096 269 -> 212 (2.27 PFLOP/s), 400 x 28672 x 4096 71 -> 49, 2048 x 6144 x 4096 67 -> 47, MXFP4 192 x 28672 x 4096
+// 37 -> 27; narrow tiles e4m3 640 x 4096 x 14336 69 -> 52, MXFP4 400 x 4096 x 4096 26 -> 14.
+template <int MODE, int Q>
+__global__ __launch_bounds__(512) void quantised_rows_kernel(const DenseArgs p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+  dense_panel<MODE, Q>(p, ring);
 }
 
 // ---- few tiles: panels of 128 features x up to 128 rows, K shared out where that fills the CUs -----------------------------
@@ -335,27 +414,45 @@ struct NarrowArgs {
   int M, N, K; long long ldx, ldy;
   int height, tiles, stages; long long slab;  // of a tile; tiles; of a share of K; elements of a share's sums
   const float* row_ss; int ss_parts; float inv_k, eps; int gelu;
+  Scales scales;
 };
 enum NarrowMode { SUMS = 3 };  // beside Mode: fp32 sums of a share of K
 constexpr int NARROW_FEATURES = 128, NARROW_AHEAD = 8;
 __host__ __device__ constexpr int narrow_ring(int height) { return (NARROW_AHEAD + 1) * height * 128; }  // bytes: what lower tiles leave of the LDS is room for other kernels' workgroups
 constexpr int NOWHERE = 0x7ffffff0;  // a lane's offset past any buffer (no scalar offset added to it comes round to its beginning)
 
-template <int NF>
-__device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&acc)[8], rsrc_t wr, int wlane, int w0, rsrc_t xr, const int (&xsrc)[2], unsigned char* ring, int c0, int n, int wave, int lane) {
+template <int NF, int Q>
+__device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&acc)[8], rsrc_t wr, int wlane, int w0, rsrc_t sr, int slane, int s0, rsrc_t xr, const int (&xsrc)[2], unsigned char* ring, int c0, int n, int wave, int lane) {
   constexpr int AHEAD = NARROW_AHEAD, RING = AHEAD + 1, STAGE = NF * 2048;
   static_assert(RING * STAGE <= RING_BYTES, "ring");
-  constexpr int PX = (2 * NF + 7) / 8, OPS = 2 + PX, BEFORE = PX + 1;  // memory operations of a stage, and those in front of its barrier
+  constexpr int PX = (2 * NF + 7) / 8, OPS = 2 + PX, BEFORE = Q == BF16 ? PX + 1 : PX;  // memory operations of a stage, and those in front of its barrier
   const int r = lane & 15, q = lane >> 4;
   int xdst[PX];
 #pragma unroll
   for (int i = 0; i < PX; ++i) xdst[i] = piece_of(wave, i, 2 * NF) * 1024;
   const int xo[2] = {r * 128 + ((q ^ (r >> 1)) << 4), r * 128 + (((4 + q) ^ (r >> 1)) << 4)};
   raw16 w[AHEAD][2];
-  frag_ab b[2][NF];
-  auto read = [&](int k, const unsigned char* img) __attribute__((always_inline)) {
+  int scale[AHEAD];
+  frag_ab b[2][NF];  // of a batch: all row tiles' k-step, or half of the row tiles' both halves of a stage
+  auto read = [&](int t, const unsigned char* img) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < NF; ++j) b[k][j] = *reinterpret_cast<const frag_ab*>(img + xo[k] + j * 2048);
+    for (int j = 0; j < NF; ++j) b[t][j] = *reinterpret_cast<const frag_ab*>(img + (Q == BF16 ? xo[t] + j * 2048 : xo[j & 1] + (t * NF + j) / 2 * 2048));
+  };
+  auto weights = [&](int k, int u, int st) __attribute__((always_inline)) {
+    const bool there = st < n;
+    if (Q == MXFP4 && k == 1) scale[u] = load4(sr, there ? slane : NOWHERE, s0 + (c0 + st) * 64);
+    else w[u][k] = load16(wr, there ? wlane : NOWHERE, w0 + (c0 + st) * (Q == MXFP4 ? 1024 : 2048) + k * 1024);
+  };
+  auto multiply = [&](int t, int u) __attribute__((always_inline)) {
+    if constexpr (Q == BF16) {
+#pragma unroll
+      for (int j = 0; j < NF; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][t]), b[t][j], acc[j], 0, 0, 0);
+    } else {
+      const raw32 a = Q == MXFP4 ? fp4_operand(w[u][0]) : both(w[u][0], w[u][1]);
+      const int by = Q == MXFP4 ? scale[u] >> (8 * q) : 0;
+#pragma unroll
+      for (int j = 0; j < NF; j += 2) acc[(t * NF + j) / 2] = product<Q>(a, both(b[t][j], b[t][j + 1]), acc[(t * NF + j) / 2], by);
+    }
   };
   // stages behind the end: offsets past the buffers, where reads give zeros and ask no memory (the same number is in flight throughout)
   auto fetch = [&](int k, int u, int st, unsigned char* dst) __attribute__((always_inline)) {
@@ -364,7 +461,8 @@ __device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&
 #pragma unroll
       for (int i = 0; i < PX; ++i) dma16(xr, there ? xsrc[i] : NOWHERE, (c0 + st) * 128, dst + xdst[i]);
     }
-    w[u][k] = load16(wr, there ? wlane : NOWHERE, w0 + (c0 + st) * 2048 + k * 1024);
+    if (Q == BF16) weights(k, u, st);  // (else both are multiplied to the stage's end)
+    else if (k == 1) { weights(0, u, st); weights(1, u, st); }
   };
 #pragma unroll
   for (int s = 0; s < AHEAD; ++s) {
@@ -383,8 +481,7 @@ __device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&
     unsigned char* dst = ring + (slot == 0 ? RING - 1 : slot - 1) * STAGE;
     read(1, ring + slot * STAGE);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < NF; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][0]), b[0][j], acc[j], 0, 0, 0);
+    multiply(0, u);
     fetch(0, u, s + AHEAD, dst);
     __builtin_amdgcn_sched_barrier(0);
     // everybody's pieces of the next stage, read from here on, have landed, and everybody's reads of this one, whose place the next fetch takes, are answered
@@ -392,8 +489,7 @@ __device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&
     __builtin_amdgcn_s_barrier();
     read(0, ring + next * STAGE);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < NF; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_ab, w[u][1]), b[1][j], acc[j], 0, 0, 0);
+    multiply(1, u);
     fetch(1, u, s + AHEAD, dst);
     __builtin_amdgcn_sched_barrier(0);
     slot = next;
@@ -405,7 +501,7 @@ __device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
 }
 
-template <int MODE>
+template <int MODE, int Q>
 __global__ __launch_bounds__(512) void narrow_tiles_kernel(const NarrowArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
   float* const row_scale = reinterpret_cast<float*>(ring + narrow_ring(p.height));
@@ -415,12 +511,11 @@ __global__ __launch_bounds__(512) void narrow_tiles_kernel(const NarrowArgs p) {
   const int m0 = id % p.tiles * p.height, panel = id / p.tiles % panels, share = id / p.tiles / panels;
   const int rows = p.M - m0 < p.height ? p.M - m0 : p.height, nf = (rows + 31) / 32 * 2, nks = p.K / 32;
   const int c0 = share * p.stages, n = p.K / 64 - c0 < p.stages ? p.K / 64 - c0 : p.stages;
-  if (MODE != SUMS && p.row_ss != nullptr && threadIdx.x < rows) {
-    float ss = 0.f;
-    for (int k = 0; k < p.ss_parts; ++k) ss += p.row_ss[(long long)(m0 + (int)threadIdx.x) * p.ss_parts + k];
-    row_scale[threadIdx.x] = rsqrtf(ss * p.inv_k + p.eps);
-  }
-  const rsrc_t wr = buffer_of(p.w + (long long)panel * (NARROW_FEATURES / 16) * nks * 1024, (unsigned int)(NARROW_FEATURES / 16) * nks * 1024);
+  const bool scaled = Q != BF16 || (MODE != SUMS && p.row_ss != nullptr);  // (sums: by the scale of the bytes alone)
+  if (scaled && threadIdx.x < rows) row_scale[threadIdx.x] = MODE == SUMS ? p.scales.x[m0 + (int)threadIdx.x] : scale_of_row<Q>(p, m0 + (int)threadIdx.x);
+  const int tile_bytes = nks * (Q == MXFP4 ? 512 : 1024);
+  const rsrc_t wr = buffer_of(p.w + (long long)panel * (NARROW_FEATURES / 16) * tile_bytes, (unsigned int)(NARROW_FEATURES / 16) * tile_bytes);
+  const rsrc_t sr = Q == MXFP4 ? buffer_of(p.scales.blocks + (long long)panel * (NARROW_FEATURES / 16) * nks * 8, (unsigned int)(NARROW_FEATURES / 16) * nks * 32) : wr;
   const rsrc_t xr = buffer_of(p.x + m0 * p.ldx, (unsigned int)(((rows - 1) * p.ldx + p.K) * 2));
   int xsrc[2];
 #pragma unroll
@@ -431,28 +526,32 @@ __global__ __launch_bounds__(512) void narrow_tiles_kernel(const NarrowArgs p) {
   frag_cd acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  const int w0 = wave * nks * 1024;
+  const int w0 = wave * tile_bytes, s0 = wave * nks * 32;
   switch (nf) {
-    case 8: multiply_narrow<8>(acc, wr, lane * 16, w0, xr, xsrc, ring, c0, n, wave, lane); break;
-    case 6: multiply_narrow<6>(acc, wr, lane * 16, w0, xr, xsrc, ring, c0, n, wave, lane); break;
-    case 4: multiply_narrow<4>(acc, wr, lane * 16, w0, xr, xsrc, ring, c0, n, wave, lane); break;
-    default: multiply_narrow<2>(acc, wr, lane * 16, w0, xr, xsrc, ring, c0, n, wave, lane); break;
+    case 8: multiply_narrow<8, Q>(acc, wr, lane * 16, w0, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
+    case 6: multiply_narrow<6, Q>(acc, wr, lane * 16, w0, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
+    case 4: multiply_narrow<4, Q>(acc, wr, lane * 16, w0, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
+    default: multiply_narrow<2, Q>(acc, wr, lane * 16, w0, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
   }
-  if (MODE != SUMS && p.row_ss != nullptr) __syncthreads();
+  if (scaled) __syncthreads();
   // acc[j][e]: feature 4 q + e of the wave's 16, row 16 j + r
   const int r = lane & 15, q = lane >> 4, f0 = panel * NARROW_FEATURES + wave * 16;
+  frag_cd of_features = {1.f, 1.f, 1.f, 1.f};
+  if constexpr (Q == FP8) of_features = *reinterpret_cast<const frag_cd*>(p.scales.w + f0 + 4 * q);
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const int row = 16 * j + r;
     if (16 * j >= rows) break;
     const long long m = m0 + row;
     frag_cd v = acc[j];
+    if (scaled) {
+      const frag_cd by = of_features * row_scale[row];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] *= by[e];
+    }
     if constexpr (MODE == SUMS) {
       if (row < rows) *reinterpret_cast<frag_cd*>(reinterpret_cast<float*>(p.y) + share * p.slab + m * p.ldy + f0 + 4 * q) = v;
     } else {
-      const float by = p.row_ss != nullptr ? row_scale[row] : 1.f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] *= by;
       unsigned short* const y = reinterpret_cast<unsigned short*>(p.y) + m * p.ldy;
       if constexpr (MODE == GATED) {  // a tile is 8 gate rows and their 8 up rows: lanes q < 2 have gates, q + 2 the ups of the same features
         frag_cd o;
@@ -482,6 +581,26 @@ int launch(const Args& a, int grid, hipStream_t s, int lds = RING_BYTES + ROWS *
   return (int)hipGetLastError();
 }
 
+template <int Q>
+int launch_narrow(const NarrowArgs& a, int epi, int grid, hipStream_t s) {
+  const int lds = narrow_ring(a.height) + a.height * 4;
+  switch (epi) {
+    case 0: return launch<narrow_tiles_kernel<PLAIN, Q>>(a, grid, s, lds);
+    case 1: return launch<narrow_tiles_kernel<SUMS, Q>>(a, grid, s, lds);
+    case 2: case 4: return launch<narrow_tiles_kernel<GATED, Q>>(a, grid, s, lds);
+    case 5: if constexpr (Q == BF16) return launch<narrow_tiles_kernel<SQUARED, BF16>>(a, grid, s, lds);
+  }
+  return -1;
+}
+
+// Whether there are the scales that numbers need; of bytes, K and ldx in pairs.
+bool in_pairs(int numbers, int& K, long long& ldx, const float* w_scale, const float* x_scale, const int* blocks) {
+  if (numbers == BF16) return true;
+  if ((numbers != FP8 && numbers != MXFP4) || (K & 127) || (ldx & 15) || !x_scale || (numbers == FP8 ? !w_scale || ((uintptr_t)w_scale & 15) : !blocks)) return false;
+  K /= 2; ldx /= 2;
+  return true;
+}
+
 }  // namespace
 
 extern "C" {
@@ -508,15 +627,19 @@ int kv_expert_panels(const void* Wp, const void* x, void* y, int N, int K, long 
 }
 
 // Wp: one packed matrix [N, K]; epi 0: bf16 y[M, N], 2: the gated y[M, N / 2] with silu, 4: with gelu (tanh form), 5: max(y, 0)^2 [M, N].  The first
-// `panels` of the ceil(N / 256) panels are cut into tiles of `height` rows, those behind them of `height_behind` (multiples of 32 up to 256).  row_ss
+// `panels` of the ceil(N / 256) panels are cut into tiles of `height` rows, those behind them of `height_behind` (multiples of 32 up to 256, of MXFP4 224).  row_ss
 // (or null): fp32 [M][ss_parts] whose sums over K are the rows' mean squares; products are divided by the root of that.
 // N % 32 == 0, K % 64 == 0, rows of x and y of whole 16-byte pieces that start at such; 256 rows of x must lie within 2 GiB.
+// numbers (Numbers): of bytes, K and ldx count them (K % 128 == 0, no epi 5), x_scale[M] are the rows' scales, w_scale[N] those of e4m3 weights (in the order
+// of whose fragments x then is), blocks those of MXFP4 ones (x in order).
 int kv_dense_panels(const void* Wp, const void* x, void* y, int M, int N, int K, long long ldx, long long ldy, int epi, int height, int panels, int height_behind, const float* row_ss, int ss_parts, float eps,
-                    hipStream_t stream) {
+                    int numbers, const float* w_scale, const float* x_scale, const int* blocks, hipStream_t stream) {
+  const float inv_k = 1.f / (float)K;
+  if (!in_pairs(numbers, K, ldx, w_scale, x_scale, blocks)) return -1;
   if (M <= 0 || N <= 0 || K <= 0 || (N & 31) || (K & 63) || K > (1 << 21) || (ldx & 7) || (ldy & 7) || ldx < K || ldx >= (1 << 22) || ((uintptr_t)x & 15) || ((uintptr_t)y & 15)) return -1;
   const int all = (N + FEATURES - 1) / FEATURES;
   for (int h : {height, height_behind})
-    if (h <= 0 || h > ROWS || (h & 31)) return -1;
+    if (h <= 0 || h > (numbers == MXFP4 ? ROWS - 32 : ROWS) || (h & 31)) return -1;
   if (panels < 0 || panels > all) return -1;
   DenseArgs a;
   a.w = (const unsigned char*)Wp; a.x = (const __bf16*)x; a.y = (unsigned short*)y;
@@ -524,38 +647,40 @@ int kv_dense_panels(const void* Wp, const void* x, void* y, int M, int N, int K,
   a.height[0] = height; a.height[1] = height_behind;
   a.tiles[0] = (M + height - 1) / height; a.tiles[1] = (M + height_behind - 1) / height_behind;
   a.panels = panels;
-  a.row_ss = row_ss; a.ss_parts = ss_parts; a.inv_k = 1.f / (float)K; a.eps = eps; a.gelu = epi == 4;
+  a.row_ss = row_ss; a.ss_parts = ss_parts; a.inv_k = inv_k; a.eps = eps; a.gelu = epi == 4;
+  a.scales = Scales{w_scale, x_scale, blocks};
   const long long grid = (long long)panels * a.tiles[0] + (long long)(all - panels) * a.tiles[1];
   if (grid > 0x7fffffffll) return -1;
-  switch (epi) {
-    case 0: return launch<dense_panel_kernel<PLAIN>>(a, (int)grid, stream);
-    case 2: case 4: return launch<dense_panel_kernel<GATED>>(a, (int)grid, stream);
-    case 5: return launch<dense_panel_kernel<SQUARED>>(a, (int)grid, stream);
+  const bool gated = epi == 2 || epi == 4;
+  if (!gated && epi != 0 && (epi != 5 || numbers != BF16)) return -1;
+  switch (numbers) {
+    case FP8: return gated ? launch<quantised_rows_kernel<GATED, FP8>>(a, (int)grid, stream) : launch<quantised_rows_kernel<PLAIN, FP8>>(a, (int)grid, stream);
+    case MXFP4: return gated ? launch<quantised_rows_kernel<GATED, MXFP4>>(a, (int)grid, stream) : launch<quantised_rows_kernel<PLAIN, MXFP4>>(a, (int)grid, stream);
   }
-  return -1;
+  return gated ? launch<dense_panel_kernel<GATED>>(a, (int)grid, stream) : epi == 5 ? launch<dense_panel_kernel<SQUARED>>(a, (int)grid, stream) : launch<dense_panel_kernel<PLAIN>>(a, (int)grid, stream);
 }
 
 // Wp: one packed matrix [N, K].  Tiles of `height` rows (a multiple of 32 up to 128) x 128 features; epi 0, 2, 4, 5 as above, 1: fp32 sums
-// [splits][M][N] of shares of `stages` x 64 columns (`slab` elements apart; other epilogues: one share).  N % 128 == 0, the rest as above.
+// [splits][M][N] of shares of `stages` x 64 columns (128 of bytes; `slab` elements apart; other epilogues: one share).  N % 128 == 0, the rest as above.
 int kv_narrow_tiles(const void* Wp, const void* x, void* y, int M, int N, int K, long long ldx, long long ldy, int epi, int height, int splits, int stages, long long slab, const float* row_ss, int ss_parts, float eps,
-                    hipStream_t stream) {
+                    int numbers, const float* w_scale, const float* x_scale, const int* blocks, hipStream_t stream) {
+  const float inv_k = 1.f / (float)K;
+  if (!in_pairs(numbers, K, ldx, w_scale, x_scale, blocks)) return -1;
   if (M <= 0 || N <= 0 || K <= 0 || N % NARROW_FEATURES || (K & 63) || K > (1 << 21) || (ldx & 7) || ldx < K || ldx >= (1 << 22) || ((uintptr_t)x & 15) || ((uintptr_t)y & 15) || (ldy & 3)) return -1;
   if (height <= 0 || height > 128 || (height & 31) || splits <= 0 || stages <= 0 || (long long)(splits - 1) * stages >= K / 64 || (long long)splits * stages < K / 64 || (epi != 1 && splits != 1)) return -1;
   NarrowArgs a;
   a.w = (const unsigned char*)Wp; a.x = (const __bf16*)x; a.y = y;
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldy = ldy;
   a.height = height; a.tiles = (M + height - 1) / height; a.stages = stages; a.slab = slab;
-  a.row_ss = row_ss; a.ss_parts = ss_parts; a.inv_k = 1.f / (float)K; a.eps = eps; a.gelu = epi == 4;
+  a.row_ss = row_ss; a.ss_parts = ss_parts; a.inv_k = inv_k; a.eps = eps; a.gelu = epi == 4;
+  a.scales = Scales{w_scale, x_scale, blocks};
   const long long grid = (long long)splits * (N / NARROW_FEATURES) * a.tiles;
   if (grid > 0x7fffffffll) return -1;
-  const int lds = narrow_ring(height) + height * 4;
-  switch (epi) {
-    case 0: return launch<narrow_tiles_kernel<PLAIN>>(a, (int)grid, stream, lds);
-    case 1: return launch<narrow_tiles_kernel<SUMS>>(a, (int)grid, stream, lds);
-    case 2: case 4: return launch<narrow_tiles_kernel<GATED>>(a, (int)grid, stream, lds);
-    case 5: return launch<narrow_tiles_kernel<SQUARED>>(a, (int)grid, stream, lds);
+  switch (numbers) {
+    case FP8: return launch_narrow<FP8>(a, epi, (int)grid, stream);
+    case MXFP4: return launch_narrow<MXFP4>(a, epi, (int)grid, stream);
   }
-  return -1;
+  return launch_narrow<BF16>(a, epi, (int)grid, stream);
 }
 
 }  // extern "C"

@@ -318,6 +318,7 @@ _WIDE_TILES_FP8 = (((256, 256, 0), 1.9), ((256, 224, 0), 1.85), ((256, 192, 0), 
 # plus 32-byte operands do not fit the register file (630 us on the down projection).
 # Third number: microseconds per round outside the K loop (ring prologue, epilogue), fitted on pairs of shapes with
 # K = 4096 and K = 14336 (e.g. 128 x 128 at 256 rows: o projection 24.4 us over 32 stages, down 67.5 us over 112).
+# Most such products go by narrow tiles and panels (_plan_narrow, _plan_panels): here the splits are chosen.
 _WIDE_TILES_FP8A = (((256, 128, 0), 0.92, 7.4), ((128, 256, 0), 0.92, 8.8), ((128, 128, 0), 0.54, 7.2))
 # Wide steps with FP8 weights quantise the activations per token to e4m3 as well and multiply on the
 # block-scaled matrix instruction (twice the bf16 MFMA rate); "0" keeps bf16 activations (the weights
@@ -369,11 +370,11 @@ def _plan_wide(m: int, n_pad: int, k: int, fp8: int, may_split: bool) -> Tuple[i
     return best[1]
 
 
-NARROW_HEIGHTS = (32, 64, 96)  # rows of a tile
+NARROW_HEIGHTS = (32, 64, 96, 128)  # rows of a tile
 
 
 @functools.lru_cache(maxsize=None)
-def _plan_narrow(m: int, n: int, k: int, may_split: bool = False) -> Optional[Tuple[int, int, int]]:
+def _plan_narrow(m: int, n: int, k: int, may_split: bool = False, numbers: int = 0) -> Optional[Tuple[int, int, int]]:
     """How bf16 weights are multiplied by one round of tiles of 128 features x up to 96 rows (``csrc/panel_gemm.hip``): (rows of a tile, K splits,
     stages of 64 columns per split), or None for the kernels below.
 
@@ -389,11 +390,16 @@ def _plan_narrow(m: int, n: int, k: int, may_split: bool = False) -> Optional[Tu
 
     Measured on MI355X with cold weights, us, tiled GEMM and this: 136 x 2048 x 2048 9.2 and 4.4, 500 x 2048 x 2048 14.2 and 11.1, 1000 x 2048 x 2048 23.7
     and 17.7, 256 x 3072 x 2048 21.9 and 15.4, 380 x 8192 x 2048 25.4 and 22.8, 176 x 16384 x 2048 28.4 and 29.3 (the only one of 45 sizes that is
-    slower), 500 x 1024 x 4096 37.8 and 26.0, 760 x 4096 x 4096 42.4 and 39.4, 256 x 9216 x 4096 45.4 and 39.7."""
-    splits, nst = _plan_wide(m, n, k, 0, may_split)[3], k // 64
-    if n % 128 or (splits > 1 and n > 2048):
+    slower), 500 x 1024 x 4096 37.8 and 26.0, 760 x 4096 x 4096 42.4 and 39.4, 256 x 9216 x 4096 45.4 and 39.7.
+
+    ``numbers`` 2 and 3 (FP8 rows with FP8 and MXFP4 weights; k counts pairs): the tiled GEMM's stage is 0.54 us too, but its round has 7 us more, so
+    that 128 rows and splits for any number of outputs are as fast or faster (us, tiled GEMM and this; FP8: 192 x 6144 x 4096 16.4 and 15.3, 136 x
+    4096 x 4096 11.8 and 11.8, 640 x 4096 x 14336 68.9 and 52.3, 1024 x 2048 x 2048 15.1 and 9.8, 1024 x 4096 x 4096 26.6 and 24.3; MXFP4: 72 x 28672 x 4096
+    32.5 and 20.5, 192 x 4096 x 14336 24.4 and 18.3, 640 x 4096 x 4096 26.0 and 17.7).  A step of four layers, 192 rows with FP8 weights: 750 and 674."""
+    splits, nst = _plan_wide(m, n, k, numbers, may_split)[3], k // 64
+    if n % 128 or (splits > 1 and n > 2048 and numbers == 0):
         return None
-    for height in NARROW_HEIGHTS:
+    for height in NARROW_HEIGHTS if numbers else NARROW_HEIGHTS[:3]:
         if -(-m // height) * (n // 128) * splits <= _num_cus():
             return height, splits, -(-nst // splits)
     return None
@@ -403,7 +409,7 @@ PANEL_HEIGHTS = (256, 224, 192, 160, 128, 96)  # rows of a tile (64 and 32: the 
 
 
 @functools.lru_cache(maxsize=None)
-def _plan_panels(m: int, n: int, k: int, may_split: bool = False) -> Optional[Tuple[int, int, int]]:
+def _plan_panels(m: int, n: int, k: int, may_split: bool = False, numbers: int = 0) -> Optional[Tuple[int, int, int]]:
     """How bf16 weights of many outputs are multiplied by panels of 256 features (``csrc/panel_gemm.hip``): (rows of a tile,
     panels cut like that, rows of the tiles of the panels behind them), or None for the tiled GEMM above.
 
@@ -418,9 +424,15 @@ def _plan_panels(m: int, n: int, k: int, may_split: bool = False) -> Optional[Tu
     64 columns, less what CUs that stay empty in a last round leave to the others in power and bandwidth (0.7 of their share).  Fitted on ten
     matrices at 144 to 4096 rows (5 % standard deviation); what it picks is within 1 % of the best height on all but one.  Two heights were 0.99
     to 1.12 times as fast as the best single one, 1.035 in the mean over 16 sizes; with 96 rows behind
-    whole rounds it was 0.97 over six others, so that is left out."""
+    whole rounds it was 0.97 over six others, so that is left out.
+
+    ``numbers`` 2 and 3 (FP8 rows with FP8 and MXFP4 weights; k counts pairs, as many bytes of rows a stage): the same model; up to one round of
+    128 x 128 tiles too (what narrow tiles leave).  Tiled GEMM and panels, us, FP8: 192 x 28672 x 4096 39.2 and 37.1, 400 x 28672 x 4096 71.5 and 49.2, 2048 x
+    28672 x 4096 269 and 212, 2048 x 6144 x 4096 67 and 47, 1024 x 16384 x 2048 49 and 36; MXFP4: 192 x 28672 x 4096 37.1 and 26.7, 640 x 16384 x 2048 45 and
+    24, 2048 x 4096 x 14336 105 and 89.  All of some 90 sizes were faster than the tiled GEMM unsplit; it keeps the splits that are more than one round
+    of narrow tiles (8192 outputs of 28672 at 129 to 324 rows)."""
     cus = _num_cus()
-    if -(-m // 128) * -(-n // 128) <= cus or (may_split and _plan_wide(m, n, k, 0, True)[3] > 1):
+    if (numbers == 0 and -(-m // 128) * -(-n // 128) <= cus) or (may_split and _plan_wide(m, n, k, numbers, True)[3] > 1):
         return None
     panels = -(-n // 256)
 
@@ -430,13 +442,36 @@ def _plan_panels(m: int, n: int, k: int, may_split: bool = False) -> Optional[Tu
         empty = 1.0 - last / cus if last else 0.0
         return rounds * (8.0 + k / 64 * (0.1 + 0.005 * height)) - k / 64 * 0.7 * empty * height / 256
 
-    best = min((time(panels, h), (h, panels, h)) for h in PANEL_HEIGHTS)
-    for h in PANEL_HEIGHTS:  # whole rounds of one height, the panels left over of another
+    heights = PANEL_HEIGHTS[1:] if numbers == 3 else PANEL_HEIGHTS
+    best = min((time(panels, h), (h, panels, h)) for h in heights)
+    for h in heights:  # whole rounds of one height, the panels left over of another
         per = -(-m // h)
         whole = panels * per // cus * cus // per
         if 0 < whole < panels:
-            best = min(best, min((time(whole, h) + time(panels - whole, rest), (h, whole, rest)) for rest in PANEL_HEIGHTS[:-1] if rest != h))
+            best = min(best, min((time(whole, h) + time(panels - whole, rest), (h, whole, rest)) for rest in heights[:-1] if rest != h))
     return best[1]
+
+
+def _by_panels(w: Union[PackedLinear, "_ExpandedView"], x: torch.Tensor, epi: int, ss: Optional[torch.Tensor], eps: float, may_split: bool, numbers: int = 0, **scales: torch.Tensor) -> Union[torch.Tensor, "Partial", None]:
+    """The product by narrow tiles or panels (``csrc/panel_gemm.hip``), or None where it is the tiled GEMM's."""
+    m, k = x.shape[0], w.k // 2 if numbers else w.k
+    if x.data_ptr() % 16 or k > 1 << 21 or not w.k <= x.stride(0) < (1 << 23 if numbers else 1 << 22):
+        return None
+    narrow = _plan_narrow(m, w.n_pad, k, may_split, numbers)
+    cut = _plan_panels(m, w.n_pad, k, may_split, numbers) if narrow is None else None
+    if narrow is not None and narrow[1] > 1:
+        out = torch.empty((narrow[1], m, w.n_pad), dtype=torch.float32, device=x.device)
+        native().narrow_tiles(w.wp, w.n_pad, w.k, x, out, 1, *narrow, None, 0.0, **scales)
+        return Partial(out, ss, eps, w.k)
+    if narrow is None and cut is None:
+        return None
+    out = torch.empty((m, w.n_pad // 2 if epi in GATED else w.n_pad), dtype=torch.bfloat16, device=x.device)
+    if narrow is not None:
+        native().narrow_tiles(w.wp, w.n_pad, w.k, x, out, epi, *narrow, ss, eps, **scales)
+    else:
+        native().dense_panels(w.wp, w.n_pad, w.k, x, out, epi, *cut, ss, eps, **scales)
+    n_true = w.n // 2 if epi in GATED else w.n
+    return out if n_true == out.shape[1] else out[:, :n_true]
 
 
 def _wide(w: Union[PackedLinear, "_ExpandedView"], h: Union[torch.Tensor, "Normed"], epi: int, allow_slabs: bool) -> Union[torch.Tensor, "Partial"]:
@@ -451,6 +486,9 @@ def _wide(w: Union[PackedLinear, "_ExpandedView"], h: Union[torch.Tensor, "Norme
     if FP8_ACTIVATIONS and isinstance(w, PackedLinear) and w.bits == 8 and w.k % 128 == 0:
         # FP8 x FP8: the activations get one dynamic scale per token (1/rms of a folded norm stays in the epilogue)
         x8, a_scale = C.quantize_rows_fp8(x)
+        out = _by_panels(w, x8, epi, ss, eps, may_split, 2, w_scale=w.wscale, x_scale=a_scale) if epi != 5 else None
+        if out is not None:
+            return out
         bm, bn, variant, splits, sps = _plan_wide(m, w.n_pad, w.k // 2, 2, may_split)
         if splits > 1:
             out = torch.empty((splits, m, w.n_pad), dtype=torch.float32, device=x.device)
@@ -461,24 +499,9 @@ def _wide(w: Union[PackedLinear, "_ExpandedView"], h: Union[torch.Tensor, "Norme
         C.wide_gemm_fp8a(w.wp, w.n_pad, w.k, x8, a_scale, out, epi, bm, bn, variant, 1, sps, ss, eps, w.wscale, True)
         n_true = w.n // 2 if epi in GATED else w.n
         return out if n_true == n_out else out[:, :n_true]
-    panels = w.wscale is None and x.data_ptr() % 16 == 0 and w.k <= 1 << 21 and w.k <= x.stride(0) < 1 << 22
-    narrow = _plan_narrow(m, w.n_pad, w.k, may_split) if panels else None
-    if narrow is not None:
-        height, splits, sps = narrow
-        if splits > 1:
-            out = torch.empty((splits, m, w.n_pad), dtype=torch.float32, device=x.device)
-            C.narrow_tiles(w.wp, w.n_pad, w.k, x, out, 1, height, splits, sps, None, 0.0)
-            return Partial(out, ss, eps, w.k)
-        out = torch.empty((m, w.n_pad // 2 if epi in GATED else w.n_pad), dtype=torch.bfloat16, device=x.device)
-        C.narrow_tiles(w.wp, w.n_pad, w.k, x, out, epi, height, 1, sps, ss, eps)
-        n_true = w.n // 2 if epi in GATED else w.n
-        return out if n_true == out.shape[1] else out[:, :n_true]
-    cut = _plan_panels(m, w.n_pad, w.k, may_split) if panels else None
-    if cut is not None:
-        out = torch.empty((m, w.n_pad // 2 if epi in GATED else w.n_pad), dtype=torch.bfloat16, device=x.device)
-        C.dense_panels(w.wp, w.n_pad, w.k, x, out, epi, *cut, ss, eps)
-        n_true = w.n // 2 if epi in GATED else w.n
-        return out if n_true == out.shape[1] else out[:, :n_true]
+    out = _by_panels(w, x, epi, ss, eps, may_split) if w.wscale is None else None
+    if out is not None:
+        return out
     bm, bn, variant, splits, sps = _plan_wide(m, w.n_pad, w.k, int(w.wscale is not None), may_split)
     if splits > 1:
         out = torch.empty((splits, m, w.n_pad), dtype=torch.float32, device=x.device)
@@ -640,6 +663,9 @@ def _stream_fp4(w: PackedLinear, h: Union[torch.Tensor, Normed], epi: int, allow
         # MFMA against per-token FP8 activations (no expansion pass, no scratch buffer, any matrix size)
         x8, a_scale = C.quantize_rows_fp8(x, False)
         may_split = allow_slabs and epi == 0 and w.n == w.n_pad
+        out = _by_panels(w, x8, epi, ss, eps, may_split, 3, blocks=w.wscale, x_scale=a_scale) if epi != 5 else None
+        if out is not None:
+            return out
         bm, bn, variant, splits, sps = _plan_wide(m, w.n_pad, w.k // 2, 3, may_split)
         if splits > 1:
             out = torch.empty((splits, m, w.n_pad), dtype=torch.float32, device=x.device)

@@ -1411,6 +1411,60 @@ def test_narrow_tiles_of_every_height(C, M, N, K, splits):
         assert torch.equal(got, want), height
 
 
+@pytest.mark.parametrize("mxfp4", [False, True])
+@pytest.mark.parametrize("M,N,K,splits", [(1, 128, 256, 2), (33, 256, 1024, 3), (95, 384, 1280, 5), (129, 640, 1536, 4), (300, 128, 4096, 7), (513, 320, 1792, 1)])
+def test_quantised_panels_and_narrow_tiles(C, M, N, K, splits, mxfp4):
+    """FP8 rows with FP8 and MXFP4 weights by panels and narrow tiles of each height: ragged last tiles, panels and shares, shares shorter and longer than the
+    stages in flight, rows at a stride, each epilogue with and without the norm's scale.  One scaled matrix instruction per 128 columns in order, as the
+    tiled kernels': the same bits."""
+    from kvmini.ops import hip_ops as ops
+
+    torch.manual_seed(M)
+    x = (torch.randn(M, K, device="cuda") * torch.rand(M, 1, device="cuda")).bfloat16()
+    pw = ops.PackedLinear((torch.randn(N, K, device="cuda") * 0.1).bfloat16(), fp8=not mxfp4, mxfp4=mxfp4)
+    x8, scale = C.quantize_rows_fp8(x, not mxfp4)
+    x8 = torch.cat((x8, x8), 1)[:, :K]
+    scales = {"blocks": pw.wscale} if mxfp4 else {"w_scale": pw.wscale}
+    ss, stages = torch.rand(M, 3, device="cuda") * K, -(-(K // 128) // splits)
+
+    def tiled(out, epi, splits, stages, rows):
+        if mxfp4:
+            C.wide_gemm_w4a8(pw.wp, pw.wscale, N, K, x8, scale, out, epi, 128, 128, 0, splits, stages, rows, 1e-5, True)
+        else:
+            C.wide_gemm_fp8a(pw.wp, N, K, x8, scale, out, epi, 128, 128, 0, splits, stages, rows, 1e-5, pw.wscale, True)
+        return out
+
+    wide = N % 128 == 0  # (else panels only, the last one cut short, against the matrix with 64 more outputs)
+    for epi in (0, 2, 4):
+        for rows in (None, ss):
+            outs = N // 2 if epi else N
+            if wide:
+                want = tiled(torch.empty((M, outs), device="cuda", dtype=torch.bfloat16), epi, 1, K // 128, rows)
+            else:
+                padded = ops.PackedLinear(torch.zeros(128, K, device="cuda").bfloat16(), fp8=not mxfp4, mxfp4=mxfp4)
+                wp, ws = torch.cat((pw.wp.flatten(), padded.wp.flatten()))[: pw.wp.numel() // N * (N + 64)], torch.cat((pw.wscale.flatten(), padded.wscale.flatten()))[: pw.wscale.numel() // N * (N + 64)]
+                want = torch.empty((M, (N + 64) // 2 if epi else N + 64), device="cuda", dtype=torch.bfloat16)
+                if mxfp4:
+                    C.wide_gemm_w4a8(wp, ws, N + 64, K, x8, scale, want, epi, 128, 128, 0, 1, K // 128, rows, 1e-5, True)
+                else:
+                    C.wide_gemm_fp8a(wp, N + 64, K, x8, scale, want, epi, 128, 128, 0, 1, K // 128, rows, 1e-5, ws, True)
+                want = want[:, :outs]
+            for height in range(32, 225 if mxfp4 else 257, 32):
+                got = torch.full((M + 1, outs), 7.0, device="cuda", dtype=torch.bfloat16)
+                C.dense_panels(pw.wp, N, K, x8, got[:M], epi, height, 1, 64, rows, 1e-5, x_scale=scale, **scales)
+                assert torch.equal(got[:M], want) and (got[M] == 7).all(), (height, epi)
+                if wide and height <= 128:
+                    got.fill_(7)
+                    C.narrow_tiles(pw.wp, N, K, x8, got[:M], epi, height, 1, K // 128, rows, 1e-5, x_scale=scale, **scales)
+                    assert torch.equal(got[:M], want) and (got[M] == 7).all(), (height, epi)
+    if wide:
+        want = tiled(torch.empty((splits, M, N), device="cuda"), 1, splits, stages, None)
+        for height in (32, 64, 96, 128):
+            got = torch.full((splits, M, N), float("nan"), device="cuda")
+            C.narrow_tiles(pw.wp, N, K, x8, got, 1, height, splits, stages, None, 0.0, x_scale=scale, **scales)
+            assert torch.equal(got, want), height
+
+
 def test_one_round_of_narrow_tiles():
     """The op layer's rule: narrow tiles where they are one round over the CUs, split where the tiled GEMM splits, the same result at a stride and with
     outputs that are no multiple of 128 (which stay where they were)."""
