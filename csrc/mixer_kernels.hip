@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void embed_stream_kernel(const T* __restrict__
 
 // ---- one sublayer's end: x += mult * g * unit((y + bias) * sigmoid(gate + gate_bias)), unit(r) = r / sqrt(mean r^2 + eps).
 // y and gate: fp32 split-K slabs (n_slabs > 0, summed here) or rows of T; y also as weighted rows (w: row t is the sum of
-// w[t n + k] times row t n + k over k < n = n_slabs; rows of weight zero are not read) or nothing (p = null: x stays).
+// w[t n + k] times row t n + k over k < n = n_slabs; rows of weight zero count for nothing, whatever they hold) or nothing (p = null: x stays).
 // Then the stream takes a row of join_rows and join_vec, where given, and xb receives the new stream in T — or, with
 // next_g, next_g * unit(x), the next product's input.  Gains g and next_g: one number, or one per column (g_step 1).
 struct RowSource { const void* p; long long ld, slab_stride; int n_slabs; const float* w; };
@@ -77,12 +77,21 @@ struct ResidualArgs {
 template <typename T>
 __device__ inline float4 row4(const RowSource& s, long long t, int c) {
   if (s.w) {
+    // (six rows are asked for before the first is added: one by one their latencies were the launch's time)
+    constexpr int B = 6;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int k = 0; k < s.n_slabs; ++k) {
-      const float w = s.w[t * s.n_slabs + k];
-      if (w == 0.f) continue;
-      const float4 b = ld4(reinterpret_cast<const T*>(s.p) + (t * s.n_slabs + k) * s.ld + c);
-      a.x += w * b.x; a.y += w * b.y; a.z += w * b.z; a.w += w * b.w;
+    for (int k0 = 0; k0 < s.n_slabs; k0 += B) {
+      float w[B];
+      float4 b[B];
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        const int k = k0 + i < s.n_slabs ? k0 + i : s.n_slabs - 1;
+        w[i] = k0 + i < s.n_slabs ? s.w[t * s.n_slabs + k] : 0.f;
+        b[i] = ld4(reinterpret_cast<const T*>(s.p) + (t * s.n_slabs + k) * s.ld + c);
+      }
+#pragma unroll
+      for (int i = 0; i < B; ++i)
+        if (w[i] != 0.f) { a.x += w[i] * b[i].x; a.y += w[i] * b[i].y; a.z += w[i] * b[i].z; a.w += w[i] * b[i].w; }
     }
     return a;
   }
@@ -114,7 +123,39 @@ __device__ inline float4 gain4(const float* g, int step, int c) {
   return make_float4(g[0], g[0], g[0], g[0]);
 }
 
-template <typename T, int NT>
+// The row of a workgroup of NT threads: each thread has the columns 4 threadIdx.x + 4 NT i.  IT > 0: at most IT of them, held in registers, so that all of a
+// row can be asked for at once, the stream's beside the result's, in front of the first sum; 0: any number, held in LDS and read again.  Bound by the chain of
+// loads, two sums over the workgroup and stores of the few rows that a CU has at a time.  512 threads: 256 and 1024 are slower (26.6, 31.0, 27.6 us gated).
+// With LDS and expert rows one by one, and now, us in steps of 2000 rows: 4096 columns gated 28.7 and 25.9, parallel 45.1 and 35.9 (beside other kernels), two streams of
+// 2048 21.1 and 19.0.
+template <int NT, int IT, typename F>
+__device__ __attribute__((always_inline)) inline void each_column(int ld, F f) {
+  if constexpr (IT > 0) {
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      const int c = (threadIdx.x + i * NT) * 4;
+      if (c < ld) f(i, c);
+    }
+  } else {
+    for (int c = threadIdx.x * 4; c < ld; c += NT * 4) f(0, c);
+  }
+}
+template <int IT>
+struct HeldRow {
+  float4 v[IT];
+  __device__ __attribute__((always_inline)) inline HeldRow(float*) {}
+  __device__ __attribute__((always_inline)) inline void put(int i, int, float4 x) { v[i] = x; }
+  __device__ __attribute__((always_inline)) inline float4 get(int i, int) const { return v[i]; }
+};
+template <>
+struct HeldRow<0> {
+  float* row;
+  __device__ inline HeldRow(float* lds) : row(lds) {}
+  __device__ inline void put(int, int c, float4 x) { st4(row + c, x); }
+  __device__ inline float4 get(int, int c) const { return ld4(row + c); }
+};
+
+template <typename T, int NT, int IT>
 __global__ __launch_bounds__(NT) void gated_residual_kernel(float* __restrict__ x, T* __restrict__ xb, RowSource y, RowSource gate, ResidualArgs a) {
   extern __shared__ __attribute__((aligned(16))) float row[];  // ld floats
   __shared__ float red[NT / 64];
@@ -122,10 +163,13 @@ __global__ __launch_bounds__(NT) void gated_residual_kernel(float* __restrict__ 
   const int ld = a.ld;
   const float inv_h = 1.f / (float)a.H;
   float k = 0.f;
+  float* xr = x + t * ld;
+  HeldRow<IT> held(row), before(nullptr);
+  if constexpr (IT > 0) each_column<NT, IT>(ld, [&](int i, int c) __attribute__((always_inline)) { before.put(i, c, ld4(xr + c)); });
   // (columns H .. ld: weights, biases and stream are zero there, so every term is)
   if (y.p) {
     float ss = 0.f;
-    for (int c = threadIdx.x * 4; c < ld; c += NT * 4) {
+    each_column<NT, IT>(ld, [&](int i, int c) __attribute__((always_inline)) {
       float4 v = row4<T>(y, t, c);
       if (a.bias) { const float4 b = ld4(a.bias + c); v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
       if (gate.p) {
@@ -134,16 +178,17 @@ __global__ __launch_bounds__(NT) void gated_residual_kernel(float* __restrict__ 
         v.x *= sigmoid(z.x + b.x); v.y *= sigmoid(z.y + b.y); v.z *= sigmoid(z.z + b.z); v.w *= sigmoid(z.w + b.w);
       }
       ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-      st4(row + c, v);
-    }
+      held.put(i, c, v);
+    });
     k = a.mult / sqrtf(block_sum<NT>(ss, red) * inv_h + a.eps);
   }
-  float* xr = x + t * ld;
   float xs = 0.f;
-  for (int c = threadIdx.x * 4; c < ld; c += NT * 4) {
-    float4 v = ld4(xr + c);
+  each_column<NT, IT>(ld, [&](int i, int c) __attribute__((always_inline)) {
+    float4 v;
+    if constexpr (IT > 0) v = before.get(i, c);
+    else v = ld4(xr + c);
     if (y.p) {
-      const float4 r = ld4(row + c), g = gain4(a.g, a.g_step, c);
+      const float4 r = held.get(i, c), g = gain4(a.g, a.g_step, c);
       v.x += k * g.x * r.x; v.y += k * g.y * r.y; v.z += k * g.z * r.z; v.w += k * g.w * r.w;
     }
     if (a.join_vec) {
@@ -154,26 +199,26 @@ __global__ __launch_bounds__(NT) void gated_residual_kernel(float* __restrict__ 
     st4(xr + c, v);
     if (a.next_g) {
       xs += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-      st4(row + c, v);
+      held.put(i, c, v);
     } else {
       st4(xb + t * ld + c, v);
     }
-  }
+  });
   if (!a.next_g) return;
   const float f = 1.f / sqrtf(block_sum<NT>(xs, red) * inv_h + a.eps);
-  for (int c = threadIdx.x * 4; c < ld; c += NT * 4) {
-    float4 v = ld4(row + c);
+  each_column<NT, IT>(ld, [&](int i, int c) __attribute__((always_inline)) {
+    float4 v = held.get(i, c);
     const float4 g = gain4(a.next_g, a.next_step, c);
     v.x *= f * g.x; v.y *= f * g.y; v.z *= f * g.z; v.w *= f * g.w;
     st4(xb + t * ld + c, v);
-  }
+  });
 }
 
 // ---- the end of a layer whose mixer and feed-forward read the same stream: x += y + bias + y2 + y3 (rows as above, whichever are given);
 // xb and xb2 receive g * unit(x) and g2 * unit(x), the next layer's inputs (no g2: xb alone).
 struct ParallelArgs { const float* bias; const float* g; const float* g2; float eps; int H, ld; };
 
-template <typename T, int NT>
+template <typename T, int NT, int IT>
 __global__ __launch_bounds__(NT) void parallel_residual_kernel(float* __restrict__ x, T* __restrict__ xb, T* __restrict__ xb2, RowSource y, RowSource y2, RowSource y3, ParallelArgs a) {
   extern __shared__ __attribute__((aligned(16))) float row[];  // ld floats
   __shared__ float red[NT / 64];
@@ -183,7 +228,8 @@ __global__ __launch_bounds__(NT) void parallel_residual_kernel(float* __restrict
   const bool more = y.p || y2.p || y3.p || a.bias;
   float ss = 0.f;
   auto add = [](float4& v, float4 b) __attribute__((always_inline)) { v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; };
-  for (int c = threadIdx.x * 4; c < ld; c += NT * 4) {
+  HeldRow<IT> held(row);
+  each_column<NT, IT>(ld, [&](int i, int c) __attribute__((always_inline)) {
     float4 v = ld4(xr + c);
     if (more) {
       float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -195,11 +241,11 @@ __global__ __launch_bounds__(NT) void parallel_residual_kernel(float* __restrict
       st4(xr + c, v);
     }
     ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;  // (columns H .. ld are zero)
-    st4(row + c, v);
-  }
+    held.put(i, c, v);
+  });
   const float f = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)a.H + a.eps);
-  for (int c = threadIdx.x * 4; c < ld; c += NT * 4) {
-    float4 v = ld4(row + c);
+  each_column<NT, IT>(ld, [&](int i, int c) __attribute__((always_inline)) {
+    float4 v = held.get(i, c);
     v.x *= f; v.y *= f; v.z *= f; v.w *= f;
     const float4 g = ld4(a.g + c);
     st4(xb + t * ld + c, make_float4(v.x * g.x, v.y * g.y, v.z * g.z, v.w * g.w));
@@ -207,7 +253,7 @@ __global__ __launch_bounds__(NT) void parallel_residual_kernel(float* __restrict
       const float4 k = ld4(a.g2 + c);
       st4(xb2 + t * ld + c, make_float4(v.x * k.x, v.y * k.y, v.z * k.z, v.w * k.w));
     }
-  }
+  });
 }
 
 // ---- the end of a sublayer between several streams: every stream becomes sum_s mix[s][t] x_s + out[t] y (y: rows as above, plus gate2[row]
@@ -221,7 +267,7 @@ struct HyperArgs {
   int H, ld;
 };
 
-template <typename T, int NT, int NS, bool EXACT>
+template <typename T, int NT, int NS, bool EXACT, int IT>
 __global__ __launch_bounds__(NT) void hyper_residual_kernel(float* __restrict__ x, T* __restrict__ xb, RowSource y, RowSource y2, HyperArgs a) {
   extern __shared__ __attribute__((aligned(16))) float row[];  // ld floats
   __shared__ float red[NT / 64];
@@ -230,7 +276,8 @@ __global__ __launch_bounds__(NT) void hyper_residual_kernel(float* __restrict__ 
   float* xr = x + t * n * ld;
   const float f2 = y2.p ? a.gate2[t] : 0.f;
   float ss = 0.f;
-  for (int c = threadIdx.x * 4; c < ld; c += NT * 4) {
+  HeldRow<IT> held(row);
+  each_column<NT, IT>(ld, [&](int k, int c) __attribute__((always_inline)) {
     float4 s[NS];
 #pragma unroll
     for (int i = 0; i < NS; ++i)
@@ -260,14 +307,14 @@ __global__ __launch_bounds__(NT) void hyper_residual_kernel(float* __restrict__ 
       u.x += r * z.x; u.y += r * z.y; u.z += r * z.z; u.w += r * z.w;
     }
     ss += u.x * u.x + u.y * u.y + u.z * u.z + u.w * u.w;  // (columns H .. ld are zero)
-    st4(row + c, u);
-  }
+    held.put(k, c, u);
+  });
   const float f = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)a.H + a.eps);
-  for (int c = threadIdx.x * 4; c < ld; c += NT * 4) {
-    float4 u = ld4(row + c);
+  each_column<NT, IT>(ld, [&](int k, int c) __attribute__((always_inline)) {
+    const float4 u = held.get(k, c);
     const float4 g = ld4(a.next_g + c);
     st4(xb + t * ld + c, make_float4(u.x * f * g.x, u.y * f * g.y, u.z * f * g.z, u.w * f * g.w));
-  }
+  });
 }
 
 // ---- cap * tanh(logit / cap), in place
@@ -758,6 +805,24 @@ int kvm_embed_stream(const void* table, int f32, const int* tokens, const int* f
   return (int)hipGetLastError();
 }
 
+// KERNEL(type, threads, IT) of a residual kernel: bf16 rows of up to 8192 columns are held in registers (IT columns of four a thread); few rows: with 1024 threads
+#define KV_ROW_FORMS(KERNEL, FEW)                                        \
+  do {                                                                   \
+    if (f32) {                                                           \
+      if (ld <= 1024) KERNEL(float, 256, 0);                             \
+      else if (FEW) KERNEL(float, 1024, 0);                              \
+      else KERNEL(float, 512, 0);                                        \
+    } else if (ld <= 1024) KERNEL(bf16raw, 256, 1);                      \
+    else if (FEW) {                                                      \
+      if (ld <= 4096) KERNEL(bf16raw, 1024, 1);                          \
+      else if (ld <= 8192) KERNEL(bf16raw, 1024, 2);                     \
+      else KERNEL(bf16raw, 1024, 0);                                     \
+    } else if (ld <= 2048) KERNEL(bf16raw, 512, 1);                      \
+    else if (ld <= 4096) KERNEL(bf16raw, 512, 2);                        \
+    else if (ld <= 8192) KERNEL(bf16raw, 512, 4);                        \
+    else KERNEL(bf16raw, 512, 0);                                        \
+  } while (0)
+
 int kvm_gated_residual(float* x, void* xb, int f32, const void* y, long long y_ld, long long y_stride, int y_slabs, const float* y_weights, const float* bias, const void* gate,
                        long long gate_ld, long long gate_stride, int gate_slabs, const float* gate_bias, const float* g, int g_step, const float* next_g, int next_step,
                        const float* join_rows, const float* join_vec, float mult, float eps, int T, int H, int ld, hipStream_t s) {
@@ -765,14 +830,12 @@ int kvm_gated_residual(float* x, void* xb, int f32, const void* y, long long y_l
   const RowSource ys{y, y_ld, y_stride, y_slabs, y_weights}, gs{gate, gate_ld, gate_stride, gate_slabs, nullptr};
   const ResidualArgs a{bias, gate_bias, g, g_step, next_g, next_step, join_rows, join_vec, mult, eps, H, ld};
   const size_t lds = (size_t)ld * 4;
-#define KV_GR(Tt, NT)                                                                                                                                             \
-  do {                                                                                                                                                            \
-    if (lds > 65536 && hipFuncSetAttribute((const void*)gated_residual_kernel<Tt, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1; \
-    hipLaunchKernelGGL((gated_residual_kernel<Tt, NT>), dim3(T), dim3(NT), lds, s, x, (Tt*)xb, ys, gs, a);                                                          \
+#define KV_GR(Tt, NT, IT)                                                                                                                                                               \
+  do {                                                                                                                                                                                  \
+    if (!IT && lds > 65536 && hipFuncSetAttribute((const void*)gated_residual_kernel<Tt, NT, IT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1;          \
+    hipLaunchKernelGGL((gated_residual_kernel<Tt, NT, IT>), dim3(T), dim3(NT), IT ? 0 : lds, s, x, (Tt*)xb, ys, gs, a);                                                                  \
   } while (0)
-  if (ld <= 1024) { if (f32) KV_GR(float, 256); else KV_GR(bf16raw, 256); }
-  else if (T <= 128) { if (f32) KV_GR(float, 1024); else KV_GR(bf16raw, 1024); }  // few rows: the whole row at once
-  else { if (f32) KV_GR(float, 512); else KV_GR(bf16raw, 512); }
+  KV_ROW_FORMS(KV_GR, T <= 128);
 #undef KV_GR
   return (int)hipGetLastError();
 }
@@ -851,22 +914,20 @@ int kvm_hyper_residual(float* x, int streams, void* xb, int f32, const void* y, 
   const RowSource ys{y, y_ld, y_stride, y_slabs, y_weights}, y2s{y2, y2_ld, y2_stride, y2_slabs, nullptr};
   const HyperArgs a{streams, mix, out, read, next_g, start, gate2, eps, H, ld};
   const size_t lds = (size_t)ld * 4;
-#define KV_HR(Tt, NT, NS, EX)                                                                                                                                                \
-  do {                                                                                                                                                                       \
-    if (lds > 65536 && hipFuncSetAttribute((const void*)hyper_residual_kernel<Tt, NT, NS, EX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1; \
-    hipLaunchKernelGGL((hyper_residual_kernel<Tt, NT, NS, EX>), dim3(T), dim3(NT), lds, s, x, (Tt*)xb, ys, y2s, a);                                                            \
+#define KV_HR(Tt, NT, NS, EX, IT)                                                                                                                                                            \
+  do {                                                                                                                                                                                       \
+    if (!IT && lds > 65536 && hipFuncSetAttribute((const void*)hyper_residual_kernel<Tt, NT, NS, EX, IT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1;      \
+    hipLaunchKernelGGL((hyper_residual_kernel<Tt, NT, NS, EX, IT>), dim3(T), dim3(NT), IT ? 0 : lds, s, x, (Tt*)xb, ys, y2s, a);                                                              \
   } while (0)
-#define KV_HRS(Tt, NT)                          \
-  do {                                          \
-    if (streams == 1) KV_HR(Tt, NT, 1, true);   \
-    else if (streams == 2) KV_HR(Tt, NT, 2, true); \
-    else if (streams == 3) KV_HR(Tt, NT, 3, true); \
-    else if (streams == 4) KV_HR(Tt, NT, 4, true); \
-    else KV_HR(Tt, NT, 16, false);              \
+#define KV_HRS(Tt, NT, IT)                          \
+  do {                                              \
+    if (streams == 1) KV_HR(Tt, NT, 1, true, IT);   \
+    else if (streams == 2) KV_HR(Tt, NT, 2, true, IT); \
+    else if (streams == 3) KV_HR(Tt, NT, 3, true, 0); \
+    else if (streams == 4) KV_HR(Tt, NT, 4, true, 0); \
+    else KV_HR(Tt, NT, 16, false, 0);               \
   } while (0)
-  if (ld <= 1024) { if (f32) KV_HRS(float, 256); else KV_HRS(bf16raw, 256); }
-  else if (T <= 128 && streams <= 4) { if (f32) KV_HRS(float, 1024); else KV_HRS(bf16raw, 1024); }
-  else { if (f32) KV_HRS(float, 512); else KV_HRS(bf16raw, 512); }
+  KV_ROW_FORMS(KV_HRS, T <= 128 && streams <= 4);
 #undef KV_HRS
 #undef KV_HR
   return (int)hipGetLastError();
@@ -879,14 +940,12 @@ int kvm_parallel_residual(float* x, void* xb, void* xb2, int f32, const void* y,
   const RowSource ys{y, y_ld, y_stride, y_slabs, nullptr}, y2s{y2, y2_ld, 0, top, y2_weights}, y3s{y3, y3_ld, y3_stride, y3_slabs, nullptr};
   const ParallelArgs a{bias, g, g2, eps, H, ld};
   const size_t lds = (size_t)ld * 4;
-#define KV_PR(Tt, NT)                                                                                                                                                \
-  do {                                                                                                                                                               \
-    if (lds > 65536 && hipFuncSetAttribute((const void*)parallel_residual_kernel<Tt, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1; \
-    hipLaunchKernelGGL((parallel_residual_kernel<Tt, NT>), dim3(T), dim3(NT), lds, s, x, (Tt*)xb, (Tt*)xb2, ys, y2s, y3s, a);                                          \
+#define KV_PR(Tt, NT, IT)                                                                                                                                                                 \
+  do {                                                                                                                                                                                    \
+    if (!IT && lds > 65536 && hipFuncSetAttribute((const void*)parallel_residual_kernel<Tt, NT, IT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1;         \
+    hipLaunchKernelGGL((parallel_residual_kernel<Tt, NT, IT>), dim3(T), dim3(NT), IT ? 0 : lds, s, x, (Tt*)xb, (Tt*)xb2, ys, y2s, y3s, a);                                                  \
   } while (0)
-  if (ld <= 1024) { if (f32) KV_PR(float, 256); else KV_PR(bf16raw, 256); }
-  else if (T <= 128) { if (f32) KV_PR(float, 1024); else KV_PR(bf16raw, 1024); }  // few rows: the whole row at once
-  else { if (f32) KV_PR(float, 512); else KV_PR(bf16raw, 512); }
+  KV_ROW_FORMS(KV_PR, T <= 128);
 #undef KV_PR
   return (int)hipGetLastError();
 }

@@ -3121,3 +3121,38 @@ def test_rope_at_the_line_between_its_kernels(C, nh, nkv, hd, kv8, more):
             C.rope_kv_write(x[i : i + step], pos[i : i + step], cos, sin, k, v, slots[i : i + step], nh, nkv, hd, scale)
         out.append([x.view(torch.uint8), k.view(torch.uint8), v.view(torch.uint8)])
     assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+@pytest.mark.parametrize("top", [1, 6, 7])
+@pytest.mark.parametrize("t", [3, 130])
+@pytest.mark.parametrize("ld", [64, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196])
+def test_residuals_of_experts_rows_at_the_edges_of_their_forms(ld, t, top):
+    """The three residual kernels on weighted rows (more and fewer than are asked for at once; rows of weight zero hold NaN) with rows held in registers and in LDS, few and many rows.
+    The stream is fp32: at most top + 3 roundings of 2^-24 of terms that add up without cancelling in the norm; what it feeds is bf16, half a unit of 2^-8."""
+    from kvmini.models.hybrid import HyperWeights
+    from kvmini.ops import hip_mixers as mx
+
+    gen = torch.Generator().manual_seed(ld + t + top)
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    dev = lambda v: v.float().cuda().contiguous()  # noqa: E731
+    unit = lambda v: v / (v.square().mean(-1, keepdim=True) + 1e-5).sqrt()  # noqa: E731
+    rel = lambda a, b: float((a.double().cpu() - b).norm() / b.norm())  # noqa: E731
+    rows, w = rnd(t * top, ld).bfloat16(), torch.rand(t, top, generator=gen)
+    w[0, 0] = 0
+    w[2] = 0
+    y = (w.double()[:, :, None] * rows.double().view(t, top, ld)).sum(1)
+    rows[(w == 0).view(-1)] = float("nan")
+    e = lambda shared=None, gate=None: mx.ExpertRows(rows.cuda(), w.cuda(), shared, gate)  # noqa: E731
+    x0, g, ng, sh, sg = rnd(t, ld), 1 + 0.2 * rnd(ld), 1 + 0.2 * rnd(ld), rnd(t, ld).bfloat16(), torch.rand(t, generator=gen)
+
+    x, want = dev(x0), x0.double() + unit(y) * g.double()
+    out = mx.gated_residual(x, e(), None, None, None, dev(g), 1.0, 1e-5, ld, torch.bfloat16, dev(ng))
+    assert rel(x, want) < 2e-6 and rel(out, unit(want) * ng.double()) < 4e-3
+    x, want = dev(x0), x0.double() + y + sh.double()
+    a, b = mx.parallel_residual(x, sh.cuda(), None, e(), dev(g), dev(ng), 1e-5, ld, torch.bfloat16)
+    assert rel(x, want) < 2e-6 and rel(a, unit(want) * g.double()) < 4e-3 and rel(b, unit(want) * ng.double()) < 4e-3
+    for n in (1, 2):
+        s0, mix, o, read = rnd(t, n, ld), rnd(n, n), rnd(n), rnd(n)
+        x, want = dev(s0), torch.einsum("st,bsc->btc", mix.double(), s0.double()) + o.double()[:, None] * (y + sg.double()[:, None] * sh.double())[:, None]
+        out = mx.hyper_residual(x, e(sh.cuda(), dev(sg)), HyperWeights(dev(read), dev(o), dev(mix)), dev(read), dev(g), 1e-5, ld, torch.bfloat16)
+        assert rel(x, want) < 2e-6 and rel(out, unit((want * read.double()[:, None]).sum(1)) * g.double()) < 4e-3
