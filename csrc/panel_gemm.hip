@@ -220,10 +220,10 @@ __device__ __attribute__((always_inline)) inline void multiply(int nf, frag_cd (
   }
 }
 
-// What a wave stores of its 32 features from f0 on.  acc[i][j][e]: feature 16 i + 4 q + e, row 16 j + r, to be multiplied by scale(i, j); gate(g, u) of a
+// What a wave stores of its 32 features from f0 on.  acc[i][j][e]: feature 16 i + 4 q + e, row 16 j + r, to be multiplied by scale(j), and by of_features[i][e] if PER_FEATURE; gate(g, u) of a
 // gated product; out(row): the row's outputs.
-template <int MODE, class Scale, class Gate, class Out>
-__device__ __attribute__((always_inline)) inline void store_rows(const frag_cd (&acc)[2][16], int rows, int f0, int lane, Scale scale, Gate gate, Out out) {
+template <int MODE, bool PER_FEATURE, class Scale, class Gate, class Out>
+__device__ __attribute__((always_inline)) inline void store_rows(const frag_cd (&acc)[2][16], const frag_cd (&of_features)[2], int rows, int f0, int lane, Scale scale, Gate gate, Out out) {
   const int r = lane & 15, q = lane >> 4;
 #pragma unroll
   for (int j = 0; j < 16; j += 2) {
@@ -232,9 +232,9 @@ __device__ __attribute__((always_inline)) inline void store_rows(const frag_cd (
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       frag_cd a = acc[0][j + t], b = acc[1][j + t];
-      const frag_cd by_a = scale(0, j + t), by_b = scale(1, j + t);
+      const float by = scale(j + t);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { a[e] *= by_a[e]; b[e] *= by_b[e]; }
+      for (int e = 0; e < 4; ++e) { a[e] *= PER_FEATURE ? of_features[0][e] * by : by; b[e] *= PER_FEATURE ? of_features[1][e] * by : by; }
       if constexpr (MODE == GATED) {  // a tile is 8 gate rows and their 8 up rows: the upper half of the lanes takes the other tile's
         frag_cd o;
 #pragma unroll
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
   multiply<BF16>(nf, acc, wr, w0, w1, wr, 0, 0, xr, xsrc, ring, p.K / 64, wave, lane);
   const int f0 = panel * p.features + wave * 32;
   if (wave * 32 >= p.features || f0 >= p.N) return;
-  store_rows<MODE>(acc, rows, f0, lane, [](int, int) { return (frag_cd){1.f, 1.f, 1.f, 1.f}; }, [&](float g, float u) { return expert_gate(g, u, p.gate); },
+  store_rows<MODE, false>(acc, {}, rows, f0, lane, [](int) { return 1.f; }, [&](float g, float u) { return expert_gate(g, u, p.gate); },
                    [&](int row) { return p.y + (long long)row_of[row] * p.ldy; });
 }
 
@@ -377,7 +377,7 @@ __device__ __attribute__((always_inline)) inline void dense_panel(const DenseArg
 #pragma unroll
     for (int i = 0; i < 2; ++i) of_features[i] = *reinterpret_cast<const frag_cd*>(p.scales.w + f0 + 16 * i + 4 * (lane >> 4));
   }
-  store_rows<MODE>(acc, rows, f0, lane, [&](int i, int j) { return of_features[i] * (scaled ? row_scale[16 * j + (lane & 15)] : 1.f); },
+  store_rows<MODE, Q == FP8>(acc, of_features, rows, f0, lane, [&](int j) { return scaled ? row_scale[16 * j + (lane & 15)] : 1.f; },
                    [&](float g, float u) {  // silu(z) = z sigmoid(z); gelu_tanh(z) = z sigmoid(2 sqrt(2 / pi) (z + 0.044715 z^3))
                      const float z = p.gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
                      return g / (1.f + __expf(-z)) * u;
