@@ -1265,8 +1265,8 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     return out
 
 
-# Heads of 64: rows of a step from which its prompts go by tiles (smaller steps: each row by itself).  Measured on MI355X, steps of four layers of a 1B
-# decoder, us, by rows and by tiles: 16 rows 276 and 281, 64 345 and 361, 128 458 and 457, 192 448 and 448 (FP8 weights), 256 511 and 483 (one prompt),
+# Heads of 64, bf16 weights: rows of a step from which its prompts go by tiles (smaller steps: each row by itself).  Measured on MI355X, steps of four layers of a 1B
+# decoder, us, by rows and by tiles: 16 rows 276 and 281, 64 345 and 361, 128 458 and 457, 256 511 and 483 (one prompt),
 # 476 and 466 (eight), 512 723 and 611, 2048 2985 and 1359 (one), 1551 and 1158 (four).
 PROMPT_TILES_64_FROM = 192
 # ... except the rows of a short chunk behind a context (drafts to verify, the end of a prompt): a tile is walked by one workgroup per kv head, a row by one

@@ -3156,3 +3156,20 @@ def test_residuals_of_experts_rows_at_the_edges_of_their_forms(ld, t, top):
         x, want = dev(s0), torch.einsum("st,bsc->btc", mix.double(), s0.double()) + o.double()[:, None] * (y + sg.double()[:, None] * sh.double())[:, None]
         out = mx.hyper_residual(x, e(sh.cuda(), dev(sg)), HyperWeights(dev(read), dev(o), dev(mix)), dev(read), dev(g), 1e-5, ld, torch.bfloat16)
         assert rel(x, want) < 2e-6 and rel(out, unit((want * read.double()[:, None]).sum(1)) * g.double()) < 4e-3
+
+
+@pytest.mark.parametrize("quantization", [None, "fp8", "mxfp4"])
+def test_prompts_of_heads_of_64_go_by_tiles_with_bf16_weights_only(monkeypatch, quantization):
+    """Rows that are rounded to e4m3 behind attention keep the kernel by rows, whose sums are in the order they were."""
+    from kvmini.engine.engine import EngineConfig, LLMEngine
+    from kvmini.engine.scheduler import SamplingParams
+    from kvmini.models.llama import LlamaConfig, random_weights
+    from kvmini.ops import hip_ops as ops
+
+    by_tiles, real = [], ops.prompt_attention_64
+    monkeypatch.setattr(ops, "prompt_attention_64", lambda *a, **k: by_tiles.append(1) or real(*a, **k))
+    cfg = LlamaConfig("small-hd64", 1024, 512, 1024, 2, 8, 2, 64, 500000.0, 1e-5, 2048, 1, 2)
+    eng = LLMEngine(EngineConfig(model="small-hd64", device="cuda:0", max_num_seqs=4, max_batched_tokens=256, max_model_len=512, num_blocks=128, kernels="hip", quantization=quantization),
+                    weights=random_weights(cfg, "cuda:0", torch.bfloat16, seed=0))
+    out = eng.generate([[1 + i % 900 for i in range(250)]], SamplingParams(max_tokens=2, ignore_eos=True))
+    assert len(out[0]) == 2 and bool(by_tiles) == (quantization is None)
