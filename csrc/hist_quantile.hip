@@ -1005,9 +1005,10 @@ __global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __
     if (u >= 0 && first == tid) {
       const int span = id / SPAN_BINS, bin = id % SPAN_BINS;
       const unsigned long long first = bin == 0 ? s.lo[span] : s.from[span] + ((unsigned long long)bin << s.shift[span]);
-      const unsigned long long behind = s.from[span] + ((unsigned long long)(bin + 1) << s.shift[span]) - 1;
+      // by what is left up to the interval's end: the bin's own end, as a key, can lie past the last one and come round to zero
+      const unsigned long long left = s.hi[span] - first, below = bin == 0 ? s.from[span] - first : 0, whole = (1ull << s.shift[span]) - 1;
       c.lo[u] = first;
-      c.wide[u] = (bin == SPAN_BINS - 1 || behind > s.hi[span] ? s.hi[span] : behind) - first;
+      c.wide[u] = bin == SPAN_BINS - 1 || left - below < whole ? left : below + whole;
     }
   }
   __syncthreads();

@@ -205,6 +205,22 @@ def test_quantiles_whatever_the_samples_are(n, dtype):
             assert np.array_equal(got[i], want, equal_nan=True), (ps, i, got[i], want)
 
 
+@pytest.mark.parametrize("largest", [math.inf, 1.6e308])
+@pytest.mark.parametrize("middle", [-0.9, -0.3])
+@pytest.mark.parametrize("n", [4097, 16385])
+def test_quantiles_of_an_interval_up_to_the_largest_values(n, middle, largest):
+    """Doubles whose level lies between a negative value and the largest ones there are: the interval's last keys are less than a bin from the end of
+    64 bits, and the row holds the smallest keys too."""
+    from kvmini.ops import hist_quantile as hq
+
+    x = np.full(n, largest)
+    x[: int(0.3 * n)] = -largest
+    x[int(0.3 * n) : int(0.55 * n)] = middle
+    p = round(0.56 * (n - 1)) / (n - 1)  # (a rank itself: n - 1 is a power of two)
+    got = hq.batched_quantiles(torch.from_numpy(np.random.default_rng(n).permutation(x)).to(_dev()), (p, 0.4))
+    assert np.array_equal(got[0], [largest, middle]), got
+
+
 def test_equal_width_histogram_matches_cpu():
     from kvmini.analysis.histograms import compute_histogram
     from kvmini.ops import hist_quantile as hq
