@@ -454,7 +454,7 @@ __device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&
       for (int j = 0; j < NF; j += 2) acc[(t * NF + j) / 2] = product<Q>(a, both(b[t][j], b[t][j + 1]), acc[(t * NF + j) / 2], by);
     }
   };
-  // stages behind the end: offsets past the buffers, where reads give zeros and ask no memory (the same number is in flight throughout)
+  // stages behind the end: offsets past the buffers, where reads give zeros and ask no memory (the same number is in flight as long as stages are fetched)
   auto fetch = [&](int k, int u, int st, unsigned char* dst) __attribute__((always_inline)) {
     const bool there = st < n;
     if (k == 0) {
@@ -475,29 +475,30 @@ __device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&
   __builtin_amdgcn_s_barrier();
   read(0, ring);
   int slot = 0;
-  auto stage = [&](auto uc, int s) __attribute__((always_inline)) {
+  auto stage = [&](auto uc, auto more, int s) __attribute__((always_inline)) {
     constexpr int u = decltype(uc)::value;
     const int next = slot + 1 == RING ? 0 : slot + 1;
     unsigned char* dst = ring + (slot == 0 ? RING - 1 : slot - 1) * STAGE;
     read(1, ring + slot * STAGE);
     __builtin_amdgcn_sched_barrier(0);
     multiply(0, u);
-    fetch(0, u, s + AHEAD, dst);
+    if constexpr (more) fetch(0, u, s + AHEAD, dst);
     __builtin_amdgcn_sched_barrier(0);
     // everybody's pieces of the next stage, read from here on, have landed, and everybody's reads of this one, whose place the next fetch takes, are answered
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 2) * OPS + BEFORE) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(more ? (AHEAD - 2) * OPS + BEFORE : (AHEAD - 2 - u) * OPS) : "memory");
     __builtin_amdgcn_s_barrier();
     read(0, ring + next * STAGE);
     __builtin_amdgcn_sched_barrier(0);
     multiply(1, u);
-    fetch(1, u, s + AHEAD, dst);
+    if constexpr (more) fetch(1, u, s + AHEAD, dst);
     __builtin_amdgcn_sched_barrier(0);
     slot = next;
   };
   int s = 0;
   for (; s + AHEAD <= n; s += AHEAD)
-    each([&](auto uc) __attribute__((always_inline)) { stage(uc, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD>{});
-  each([&](auto uc) __attribute__((always_inline)) { if (s + decltype(uc)::value < n) stage(uc, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD - 1>{});
+    each([&](auto uc) __attribute__((always_inline)) { stage(uc, std::true_type{}, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD>{});
+  // (the last stages fetch nothing, as above)
+  each([&](auto uc) __attribute__((always_inline)) { if (s + decltype(uc)::value < n) stage(uc, std::false_type{}, s + decltype(uc)::value); }, std::make_integer_sequence<int, AHEAD - 1>{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
 }
 

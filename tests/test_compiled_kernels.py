@@ -142,6 +142,36 @@ def test_panels_have_in_flight_what_they_wait_for(functions):
         assert seen == set(loads), (name, seen)
 
 
+def test_narrow_tiles_have_in_flight_what_they_wait_for(functions):
+    """Narrow tiles wait for a stage's rows by the number of operations issued behind them too.  Rows are fetched nowhere without their weights (the compiler
+    drops loads that nothing multiplies: stages behind the loop must fetch neither); in the loop, from one barrier to the next, exactly a stage's."""
+    kernels = functions("narrow_tiles_kernel")
+    assert len(kernels) == 10
+    for name, body in kernels.items():
+        behind = 1 if "ELi0EEEv" in name else 0  # of a stage's two loads of weights, in front of its barrier: one of bf16, else none
+        loops, seen = {6 * (2 + px) + px + behind: 2 + px for px in (1, 2)}, set()
+        stretch, stretches = [], []
+        for line in body:
+            stretch.append(line)
+            if line.startswith(("s_branch", "s_cbranch", "s_endpgm")):
+                stretches.append(stretch)
+                stretch = []
+        for lines in stretches:
+            at = [i for i, line in enumerate(lines) if line == "s_barrier"]
+            fetched = [i for i, line in enumerate(lines) if line.startswith("buffer_load")]
+            rows = sum(lines[i].endswith("lds") for i in fetched)
+            assert len(fetched) in (2 * rows, 3 * rows), (name, rows, len(fetched))  # (two or one pieces of rows a stage)
+            before, last = -1, 0
+            for i in at:
+                wait = re.match(r"s_waitcnt vmcnt\((\d+)\)", lines[i - 1])
+                allowed = int(wait.group(1)) if wait else -1
+                if allowed in loops and allowed == before:
+                    assert sum(last < f < i for f in fetched) == loops[allowed], (name, allowed)
+                    seen.add(allowed)
+                before, last = allowed, i
+        assert seen == set(loops), (name, seen)
+
+
 def registers_of(text):
     found = set()
     for many in re.finditer(r"\bv\[(\d+):(\d+)\]|\bv(\d+)\b", text):
