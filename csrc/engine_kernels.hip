@@ -1644,11 +1644,26 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const unsigne
 // The same for heads of 64: 32 columns of v_mfma_f32_32x32x16_bf16 per wave, two neighbouring 16-query tiles of one head (a tile alone leaves half
 // of them idle), the pipeline of prefill_attention_tiles16 and the operand layouts of prefill_attention_tiles32.  Four heads of a group per
 // workgroup; wider groups take several.  A key row is 128 bytes: each of the 256 threads stages one 16-byte piece of K and of V per step of 32 keys.
-// The weights stay what they were in the kernel this takes over from, fp32: P = hi + lo in two bf16 operands (16 bits of mantissa; the products'
-// errors are below an output's rounding, and the errors against 64 bits are alike), for which the P V products run twice.
-// Bound by the vector unit (the exponentials and the split of the weights: some 16 instructions per score against 12 matrix instructions per 512).
-// 32 heads over 8 of keys, one prompt of 2048 tokens: 471 us with a workgroup per token (paged_attention_kernel), 62 so.
+// The weights stay what they were in the kernel this takes over from, fp32: P in three bf16 operands whose sum is exactly P's 24 bits (weight_parts),
+// for which the P V products run three times.
+// Bound by the vector unit (the exponentials and the split of the weights: some 21 instructions per score against 16 matrix instructions per 512).
+// 32 heads over 8 of keys, one prompt of 2048 tokens: 470 us with a workgroup per token (paged_attention_kernel), 73 so;
+// 64 with two bf16 parts, whose 16 bits show where values cancel (errors near zero 19 times those of fp32 weights, 1.0 times so).
 constexpr int PA64_K_RS = 72, PA64_V_RS = 96;  // row strides (elements): 144 and 192 bytes, by the bank analysis of the 32-column path
+// Two weights p >= 0 as the halves of three words of bf16 parts: p = a + b + c, each part the eight leading bits of what is left below the one in front (strictly
+// below: where p > 0 all parts are positive, so that a weight times an infinite value is infinite and no part of it 0 x infinity).
+__device__ __forceinline__ void weight_parts(float p0, float p1, int& a, int& b, int& c) {
+  const auto upper = [](float v) { return __builtin_elementwise_sub_sat(__float_as_uint(v), 1u); };
+  const auto rest = [](float v, unsigned int u) { return v - __uint_as_float(u & 0xffff0000u); };
+  const auto halves = [](unsigned int lo, unsigned int hi) { return (int)__builtin_amdgcn_perm(hi, lo, 0x07060302u); };
+  const unsigned int a0 = upper(p0), a1 = upper(p1);
+  const float r0 = rest(p0, a0), r1 = rest(p1, a1);
+  const unsigned int b0 = upper(r0), b1 = upper(r1);
+  a = halves(a0, a1);
+  b = halves(b0, b1);
+  c = halves(__float_as_uint(rest(r0, b0)), __float_as_uint(rest(r1, b1)));
+}
+
 template <bool KV8>
 __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* __restrict__ q, long long q_row_stride, const void* __restrict__ k_cache,
                                                           const void* __restrict__ v_cache, const int* __restrict__ bt, int row0, int pos0, int n_q,
@@ -1749,16 +1764,21 @@ __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* 
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
       const float m_old = m_run, m_new = fmaxf(m_old, half_rows_max(mx));
       m_run = m_new;
-      mfma_ab hp[2], lp[2];
+      typedef __attribute__((ext_vector_type(4))) int words;
+      words parts[3][2];  // of the weights: the leading bits, the middle, the last
       float psum = 0.f;
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float p = __builtin_amdgcn_exp2f(sc[8 * s2 + j] - m_new);
-          psum += p;
-          hp[s2][j] = (__bf16)p;
-          lp[s2][j] = (__bf16)(p - (float)hp[s2][j]);
+        for (int j = 0; j < 8; j += 2) {
+          const float p0 = __builtin_amdgcn_exp2f(sc[8 * s2 + j] - m_new), p1 = __builtin_amdgcn_exp2f(sc[8 * s2 + j + 1] - m_new);
+          psum += p0;
+          psum += p1;
+          int a, b, c;
+          weight_parts(p0, p1, a, b, c);
+          parts[0][s2][j / 2] = a;
+          parts[1][s2][j / 2] = b;
+          parts[2][s2][j / 2] = c;
         }
       const float corr = __builtin_amdgcn_exp2f(m_old - m_new);
       l_run = l_run * corr + psum;  // this lane's keys only; folded after the loop
@@ -1772,8 +1792,8 @@ __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* 
       for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
-          o[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[nt][s2], hp[s2], o[nt], 0, 0, 0);
-          o[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[nt][s2], lp[s2], o[nt], 0, 0, 0);
+#pragma unroll
+          for (int i = 2; i >= 0; --i) o[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[nt][s2], __builtin_bit_cast(mfma_ab, parts[i][s2]), o[nt], 0, 0, 0);
         }
       cur = nxt;
     }

@@ -914,6 +914,30 @@ def test_prefill_attention_of_heads_of_64(C, rep, kv8):
     assert torch.equal(both[:rows][~rows_of], out[~rows_of]) and torch.equal(both[:rows][rows_of], per_token[rows_of]) and (both[rows] == 0).all()
 
 
+def test_prefill_attention_of_heads_of_64_keeps_its_weights_in_32_bits():
+    """Values of 1 and -1, so that the results near zero, which bf16 holds to 2^-9 of themselves, show the weights' errors: no larger than those of the kernel by
+    rows, whose weights are fp32 (half as much again for sums in another order; weights of 16 bits show some ten times as much)."""
+    from kvmini.ops import hip_ops
+
+    torch.manual_seed(5)
+    seqs, n, nkv, rep, hd, bs = 64, 32, 2, 4, 64, 16
+    nh, rows = nkv * rep, seqs * n
+    bt = torch.randperm(seqs * 2, device=_dev()).view(seqs, 2).int()
+    kc, vc = _rand_cache(seqs * 2, nkv, bs, hd), _rand_cache(seqs * 2, nkv, bs, hd).sign()
+    q = (0.25 * torch.randn(rows, nh, hd, device=_dev())).bfloat16()
+    tok_seq, ctx = (torch.arange(rows, device=_dev()) // n).int(), (torch.arange(rows, device=_dev()) % n + 1).int()
+    tiles = torch.tensor([(s * n + off, 16, off, s) for s in range(seqs) for off in (0, 16)], device=_dev(), dtype=torch.int32).T.contiguous()
+    tiled = hip_ops.prefill_attention(q, kc, vc, bt, tiles, torch.empty((rows, nh * hd), device=_dev(), dtype=torch.bfloat16), 0.125)
+    by_rows = hip_ops.paged_attention(q, kc, vc, bt, tok_seq, ctx, 0.125, 2)
+    k, v = (c[bt.long()].double().transpose(2, 3).reshape(seqs, n, nkv, 1, hd) for c in (kc, vc))
+    s = (q.double().view(seqs, n, 1, nkv, rep, hd) * k[:, None]).sum(-1) * 0.125  # [sequence, query, key, head of keys, head]
+    s = s.masked_fill(torch.ones(n, n, device=_dev()).triu(1).bool()[None, :, :, None, None], -math.inf).softmax(2)
+    want = (s[..., None] * v[:, None]).sum(2).reshape(rows, nh * hd)
+    near = (want.abs() < 2.0 ** -15) & (ctx > 4)[:, None]
+    error = lambda got: (got.double() - want)[near].square().mean().sqrt().item()  # noqa: E731
+    assert near.sum() > 40 and error(tiled) <= 1.5 * error(by_rows), (int(near.sum()), error(tiled), error(by_rows))
+
+
 @pytest.mark.parametrize("seed,rep,kv8,quads", [(1, 4, False, False), (2, 4, True, False), (3, 1, False, False), (4, 2, False, False), (5, 8, False, False), (6, 6, True, False),
                                                (7, 3, True, False), (8, 4, False, True), (9, 4, True, True), (10, 1, False, True), (11, 3, True, True), (12, 2, False, True)])
 def test_prefill_attention_random_chunk_layouts(seed, rep, kv8, quads):
