@@ -1686,25 +1686,26 @@ __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* 
     for (int r = 0; r < 16; ++r) o[nt][r] = 0.f;
   float m_run = -1e30f, l_run = 0.f;
   // staging: thread = (key tid >> 3 of the step, piece tid & 7 of its row).  A wave's keys are rows of one cache block: its table entry and base address
-  // are scalar.  Loads run three steps ahead of the products, table entries four; past the last key they repeat it (masked in the softmax).
+  // are scalar.  Loads run three steps ahead of the products, table entries four; past the last block they repeat it.  Keys past the last one are masked in the
+  // softmax, their values are zeros (what the cache holds there, or the last key's again, need be no number).
   constexpr int ESZ = KV8 ? 1 : 2;
   const int sub = __builtin_amdgcn_readfirstlane(tid >> 7), row = (tid >> 3) & 15, piece = tid & 7;
   const int k_st = (tid >> 3) * K_RS + piece * 8, v_st = (tid >> 3) * V_RS + piece * 8;
-  const int last_blk = last_key >> 4, last_row = last_key & 15;
-  const unsigned off_row = (unsigned)((row * HD + piece * 8) * ESZ), off_end = (unsigned)(((row < last_row ? row : last_row) * HD + piece * 8) * ESZ);
+  const int last_blk = last_key >> 4;
+  const unsigned off_row = (unsigned)((row * HD + piece * 8) * ESZ);
   const long long blk_bytes = (long long)nkv * BS * HD * ESZ, head_bytes = (long long)g * BS * HD * ESZ;
   bf16x8 kr, vr;
   auto entry = [&](int kb) __attribute__((always_inline)) {
     const int bi = (kb >> 4) + sub;
     return bt[bi < last_blk ? bi : last_blk];
   };
-  auto load = [&](int kb, int blk) __attribute__((always_inline)) {
+  auto load = [&](int blk) __attribute__((always_inline)) {
     const long long base = (long long)blk * blk_bytes + head_bytes;
-    const unsigned off = (kb >> 4) + sub < last_blk ? off_row : off_end;
-    kr = kv_load8_at<KV8>(reinterpret_cast<const char*>(k_cache) + base, off);
-    vr = kv_load8_at<KV8>(reinterpret_cast<const char*>(v_cache) + base, off);
+    kr = kv_load8_at<KV8>(reinterpret_cast<const char*>(k_cache) + base, off_row);
+    vr = kv_load8_at<KV8>(reinterpret_cast<const char*>(v_cache) + base, off_row);
   };
-  auto stage = [&](int slot) __attribute__((always_inline)) {
+  auto stage = [&](int slot, int kb) __attribute__((always_inline)) {
+    if (kb + KSTEP - 1 > last_key && kb + (tid >> 3) > last_key) vr = (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
     *reinterpret_cast<bf16x8*>(k_lds + slot * K_TILE + k_st) = kr;
     *reinterpret_cast<bf16x8*>(v_lds + slot * V_TILE + v_st) = vr;
   };
@@ -1720,13 +1721,13 @@ __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* 
     return st;
   };
   int blk = entry(0);
-  load(0, blk);
+  load(blk);
   blk = entry(KSTEP);
-  stage(0);
-  load(KSTEP, blk);
+  stage(0, 0);
+  load(blk);
   blk = entry(2 * KSTEP);
-  stage(1);
-  load(2 * KSTEP, blk);
+  stage(1, KSTEP);
+  load(blk);
   blk = entry(3 * KSTEP);
   __syncthreads();
   mfma_cd16 cur;
@@ -1735,8 +1736,8 @@ __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* 
   // softmax of i, whose products end it.  MASKED: a step that reaches the diagonal of some query.
   auto step = [&](auto masked_c, int kb, int s_v, int s_k, int s_w) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_c)::value;
-    stage(s_w);
-    load(kb + 3 * KSTEP, blk);
+    stage(s_w, kb + 2 * KSTEP);
+    load(blk);
     blk = entry(kb + 4 * KSTEP);
     if (head_on) {
       const unsigned short* vt = v_lds + s_v * V_TILE + vf_base;
@@ -1792,8 +1793,13 @@ __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* 
       for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
+          mfma_cd16 sum = o[nt];
 #pragma unroll
-          for (int i = 2; i >= 0; --i) o[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[nt][s2], __builtin_bit_cast(mfma_ab, parts[i][s2]), o[nt], 0, 0, 0);
+          for (int i = 2; i >= 0; --i) sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[nt][s2], __builtin_bit_cast(mfma_ab, parts[i][s2]), sum, 0, 0, 0);
+          // (a block behind a query's own counts for nothing, whatever it holds: a weight of zero times a value that is no number is none)
+          const bool meets = !MASKED || kb + 16 * s2 <= pos0 + lr;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[nt][r] = meets ? sum[r] : o[nt][r];
         }
       cur = nxt;
     }
@@ -1816,7 +1822,7 @@ __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* 
   }
   const float l = half_rows_sum(l_run);
   if (!head_on || lr >= n_q) return;
-  const float inv = l > 0.f ? v_scale / l : 0.f;
+  const float inv = v_scale / l;
   unsigned short* op = out + (long long)(row0 + lr) * nh * HD + (long long)head * HD + 4 * hi;
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt)
@@ -1825,7 +1831,7 @@ __device__ __forceinline__ void prefill_attention_tiles64(const unsigned short* 
       typedef __attribute__((ext_vector_type(4))) unsigned short us4;
       us4 w;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) w[r] = f2bf(o[nt][4 * rq + r] * inv);
+      for (int r = 0; r < 4; ++r) w[r] = f2bf(l > 0.f ? o[nt][4 * rq + r] * inv : 0.f);  // (0 where a weight is no number, as by rows)
       *reinterpret_cast<us4*>(op + 32 * nt + 8 * rq) = w;
     }
 }

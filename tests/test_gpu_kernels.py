@@ -914,6 +914,45 @@ def test_prefill_attention_of_heads_of_64(C, rep, kv8):
     assert torch.equal(both[:rows][~rows_of], out[~rows_of]) and torch.equal(both[:rows][rows_of], per_token[rows_of]) and (both[rows] == 0).all()
 
 
+@pytest.mark.parametrize("where", ["k", "v"])
+@pytest.mark.parametrize("value", [math.nan, math.inf, -math.inf])
+def test_prefill_attention_of_heads_of_64_beside_values_that_are_no_numbers(value, where):
+    """Keys and values that are no numbers, at the ends and in the middle of blocks and behind the prompt: a query they are in front of has the NaN, infinity or zeros
+    (where a weight is no number) of the kernel by rows; one of an earlier block meets none, however its tile's steps lie.  (A value in a query's own block
+    but behind it counts by a weight of zero, which by rows it does too; keys behind all of a tile count for nothing.)"""
+    from kvmini.ops import hip_ops
+
+    torch.manual_seed(3)
+    nkv, rep, hd, bs, max_blocks = 2, 4, 64, 16, 12
+    nh = nkv * rep
+    chunks = [(0, 0, 100), (1, 16, 70), (2, 5, 90), (3, 56, 33), (4, 0, 17)]
+    bad = {0: (40, 63, 99, 101), 1: (33, 47), 2: (15, 16, 70), 3: (60, 80, 89), 4: (16, 25)}
+    nb = len(chunks) * max_blocks
+    bt = torch.randperm(nb, device=_dev()).view(len(chunks), max_blocks).int()
+    kc, vc = _rand_cache(nb, nkv, bs, hd), _rand_cache(nb, nkv, bs, hd)
+    rows, tok_seq, ctx, tiles, met = 0, [], [], [], []
+    for seq, p0, n in chunks:
+        for i, pos in enumerate(bad[seq]):
+            (kc if where == "k" else vc)[bt[seq, pos // bs].long(), i % nkv, pos % bs, 7 * i + 3] = value
+        tiles += [(rows + off, min(16, n - off), p0 + off, seq) for off in range(0, n, 16)]
+        tok_seq += [seq] * n
+        ctx += [p0 + j + 1 for j in range(n)]
+        met.append(torch.zeros(n, nkv, rep, hd, dtype=torch.bool))
+        for i, pos in enumerate(bad[seq]):  # (a value concerns one column)
+            met[-1][max(0, pos - p0) :, i % nkv, :, slice(None) if where == "k" else 7 * i + 3] = True
+        rows += n
+    q = torch.randn(rows, nh, hd, device=_dev()).bfloat16()
+    out = torch.full((rows, nh * hd), 7.0, device=_dev(), dtype=torch.bfloat16)
+    hip_ops.prefill_attention(q, kc, vc, bt, torch.tensor(tiles, device=_dev(), dtype=torch.int32).T.contiguous(), out, 0.125)
+    want = hip_ops.paged_attention(q, kc, vc, bt, *(torch.tensor(v, device=_dev(), dtype=torch.int32) for v in (tok_seq, ctx)), 0.125, max_blocks)
+    met = torch.cat(met).view(rows, nh * hd).to(_dev())
+    special = lambda v: (v.isnan(), v.isposinf(), v.isneginf(), (v == 0) & (where == "k"))  # noqa: E731
+    for got, by_rows in zip(special(out), special(want)):
+        assert torch.equal(got & met, by_rows & met) and not (got & ~by_rows).any()
+    on = want.isfinite() & (want != 0)
+    assert 0 < (~on).sum() < on.numel() and ((out - want)[on].float().norm() / want[on].float().norm()).item() < 2.0 ** -8  # (both are rounded once, 2^-9 at most)
+
+
 def test_prefill_attention_of_heads_of_64_keeps_its_weights_in_32_bits():
     """Values of 1 and -1, so that the results near zero, which bf16 holds to 2^-9 of themselves, show the weights' errors: no larger than those of the kernel by
     rows, whose weights are fp32 (half as much again for sums in another order; weights of 16 bits show some ten times as much)."""
