@@ -185,8 +185,7 @@ class ModelRunner:
         self.dec_split_ok = bool(hasattr(self.ops, "split_decode_attention") and self.device.type == "cuda" and self.hd == 128 and self.block_size == 16)
         # heads of 64 by tiles: not with quantised weights, whose rows are rounded to e4m3 behind attention: sums in another order move
         # their codes, and results by 4 % of their norm where bf16 weights move 0.6 % (the errors against 64 bits stay: 0.052 and 0.052)
-        self.tiles_64 = self.hd == 64 and hasattr(self.ops, "PROMPT_TILES_64_FROM") and getattr(self.w, "quantization", None) is None
-        self.rows_64 = getattr(self.ops, "PROMPT_ROWS_64", (0, 0)) if self.hd == 64 else (0, 0)  # short chunks of heads of 64 that are no tiles
+        self.tiles_64 = bool(self.hd == 64 and hasattr(self.ops, "PROMPT_TILES_64_FROM") and getattr(self.w, "quantization", None) is None and self._tiled_ok(self.kv_cache[0, 0]))
         # a few prompt tiles deep inside a long context: every tile's key range is shared out over several workgroups
         self.pf_split_ok = bool(hasattr(self.ops, "prefill_attention_split") and self.device.type == "cuda" and self.hd == 128 and self.block_size == 16
                                 and os.environ.get("KVMINI_PREFILL_SPLIT", "1") != "0")
@@ -219,7 +218,8 @@ class ModelRunner:
         self.s_cap = tmax
         self.set_spec_width(1)
         # (token bucket, step kind) -> (graph, logits); kind 0 = mixed step, 1 = decode-only (fused
-        # RoPE + attention kernel), 2 = decode-only with the context split over several workgroups
+        # RoPE + attention kernel), 2 = decode-only with the context split over several workgroups, 3 = mixed without prompt tiles
+        # (tiles_64: the attention kernel by rows alone; kind 0 serves such a step too)
         self.graphs: Dict[Tuple[int, ...], Any] = {}
         self._graph_pool = None
         # Weight read-ahead on a second stream beside the decode attention kernel (a parallel branch of the
@@ -397,6 +397,9 @@ class ModelRunner:
         the 8-wave attention kernel (see ``tile_quads``).  ``pf_split``: ``shares | tiles << 8`` — the step's first ``tiles`` prompt tiles
         go to the split form of the tile kernel with ``shares`` key ranges each (see ``PF_SPLIT_MAX_TILES``)."""
         ops, cfg, w = self.ops, self.cfg, self.w
+        by_rows = decode_only == 3
+        if by_rows:
+            decode_only = 0
         tokens = self._dev("tokens", t_pad)
         positions = self._dev("positions", t_pad)
         slots = self._dev("slots", t_pad)
@@ -447,7 +450,7 @@ class ModelRunner:
                         ops.prefetch_weight(lw.wo, self._side_wgs)
                 a = ops.rope_attention_fused(qkv, positions, self.cos, self.sin, kc, vc, slots, bt, tok_seq, ctx, self.nh, self.scale, n_split=None if decode_only == 2 else 1, **kw,
                                              **(pf(lw.wo, "o") if decode_only == 1 else {}))
-            elif not decode_only and self.tiles_64 and t_pad >= ops.PROMPT_TILES_64_FROM and self._tiled_ok(kc):
+            elif not decode_only and self.tiles_64 and not by_rows:
                 q = ops.rope_kv_write(qkv, positions, self.cos, self.sin, kc, vc, slots, self.nh, self.nkv, self.hd, **kw)
                 a = ops.prompt_attention_64(q, kc, vc, bt, tok_seq, self._dev("ctx_decode", t_pad), self._dev("tiles").view(4, self.max_tiles), self.scale, **kw)
             elif not decode_only and self.hd != 64 and self._tiled_ok(kc):
@@ -579,6 +582,7 @@ class ModelRunner:
         # kernel without the launch of the prompt-tile kernel that the general graph carries — 5.3 us per layer)
         variants += [(b, 1) for b, _ in variants if b <= dec_max and b <= max(self.DECODE_FUSED_MAX_ROWS, 256) and hasattr(self.ops, "rope_attention_fused")]
         variants += [(b, 2) for b, k in variants if k == 1 and self.step_kind(b, True, self.rcfg.max_model_len) == 2]
+        variants += [(b, 3) for b, k in variants if k == 0 and self.tiles_64]
         for b, dec in variants:
             key = (b, dec)
             if key in self.graphs:
@@ -787,7 +791,9 @@ class ModelRunner:
             # (a draft runner launching proposal j + 1 on top of proposal j: the chunk's one token is the
             # previous proposal, still a placeholder in draft_ids and fed on the device like any other)
             drafting = bool(seq.draft_ids) and seq.draft_feed and p0 >= seq.num_tokens
-            if n == 1 and (not seq.draft_ids or drafting):
+            # heads of 64: tiles or rows by the length of the run alone, so that a prompt's results are the same beside whatever other rows a step has
+            tiled = not self.tiles_64 or ch.run_tokens >= self.ops.PROMPT_TILES_64_FROM
+            if n == 1 and (not seq.draft_ids or drafting) and not (self.tiles_64 and tiled):
                 npmt = len(seq.prompt_ids)
                 tok = seq.draft_ids[p0 - seq.num_tokens] if drafting else (seq.prompt_ids[p0] if p0 < npmt else seq.output_ids[p0 - npmt])
                 if tok == PLACEHOLDER:
@@ -829,13 +835,12 @@ class ModelRunner:
                 # tile whose workgroup walks the whole context per kv head; as listed rows (each with its own
                 # causal length) the split-KV kernel spreads every row's walk over the chip instead.
                 as_rows = self.dec_split_ok and n <= self.DEC_SPLIT_ROWS and p0 >= self.DEC_SPLIT_MIN_CTX and n_dec + n <= self.DEC_SPLIT_ROWS
-                alone = n <= self.rows_64[0] and p0 >= self.rows_64[1]
                 if as_rows:
                     st[o_cd + i : o_cd + i + n] = pos + 1
                     st[o_dr + n_dec : o_dr + n_dec + n] = np.arange(i, i + n, dtype=np.int32)
                     n_dec += n
                     dec_max_ctx = max(dec_max_ctx, p0 + n)
-                elif alone:
+                elif not tiled:
                     st[o_cd + i : o_cd + i + n] = pos + 1
                 else:
                     st[o_cd + i : o_cd + i + n] = -1  # rows of a prompt chunk: left to the tiled kernel (0 = padding row, zeroed)
@@ -848,7 +853,7 @@ class ModelRunner:
                         quad_min_pos = min(quad_min_pos, p0)
                 if not as_rows:
                     tile_max_ctx = max(tile_max_ctx, p0 + n)
-                for off in range(0, 0 if as_rows or alone else n, 16):
+                for off in range(0, 0 if as_rows or not tiled else n, 16):
                     st[o_tl + n_tiles], st[o_tl + mt + n_tiles], st[o_tl + 2 * mt + n_tiles], st[o_tl + 3 * mt + n_tiles] = i + off, min(16, n - off), p0 + off, seq.slot
                     n_tiles += 1
                 if ch.logit_rows is not None:
@@ -878,7 +883,9 @@ class ModelRunner:
         self._stage_portions(st, portions, t, t_pad)
 
         # plain decoding step: every chunk is one token (no prompt chunk, no drafts to verify)
-        decode_only = self.step_kind(t_pad, all(ch.n_tokens == 1 for ch in batch.chunks), max_ctx)
+        decode_only = self.step_kind(t_pad, all(ch.n_tokens == 1 for ch in batch.chunks) and not (self.tiles_64 and n_tiles), max_ctx)
+        if self.tiles_64 and not decode_only and not n_tiles:
+            decode_only = 3
         o_h = self._off["header"][0]
         quads = int(self.tile_quads and not decode_only and quad_groups * self.nkv >= self.quads_min_groups and quad_min_pos >= self.quads_min_pos)
         # a few tiles, deep inside a long context: key ranges shared out (the tile count rounded up to a power of two: fewer graph shapes)

@@ -80,6 +80,7 @@ class Sequence:
     published_blocks: int = 0
     slot: int = -1  # row in the block-table tensor
     cached_prefix_tokens: int = 0
+    run: Tuple[int, int] = (0, 0)  # first and last + 1 of the positions its admission set out to compute, in however many steps
     first_token_time: Optional[float] = None
     finish_reason: Optional[str] = None
     user: Any = None  # opaque handle for the front-end (stream queue, ...)
@@ -118,6 +119,13 @@ class ScheduledChunk:
     n_sample: int = -1
     logit_rows: Optional[List[int]] = None  # explicit positions (counted inside the chunk) whose logits are wanted, instead of the above
     out_index: int = -1  # pipelined stepping: index in ``output_ids`` of the placeholder this chunk fills
+
+    @property
+    def run_tokens(self) -> int:
+        """Tokens of the run that the chunk is a part of: those its sequence was admitted with, however steps' budgets cut them, or the chunk's own (drafts,
+        portions that the caller chose)."""
+        first, end = self.seq.run
+        return end - first if self.start < end else self.n_tokens
 
 
 @dataclass
@@ -345,6 +353,7 @@ class Scheduler:
                 seq.blocks_epoch += 1
                 seq.num_computed = cached_tokens
                 seq.cached_prefix_tokens = cached_tokens
+                seq.run = (cached_tokens, seq.num_tokens)
                 seq.published_blocks = len(cached_blocks)
             n_new = seq.num_tokens - seq.num_computed
             n = min(n_new, budget)

@@ -1265,14 +1265,12 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     return out
 
 
-# Heads of 64, bf16 weights: rows of a step from which its prompts go by tiles (smaller steps: each row by itself).  Measured on MI355X, steps of four layers of a 1B
-# decoder, us, by rows and by tiles: 16 rows 276 and 281, 64 345 and 361, 128 458 and 457, 256 511 and 483 (one prompt),
-# 476 and 466 (eight), 512 723 and 611, 2048 2985 and 1359 (one), 1551 and 1158 (four).
-PROMPT_TILES_64_FROM = 192
-# ... except the rows of a short chunk behind a context (drafts to verify, the end of a prompt): a tile is walked by one workgroup per kv head, a row by one
-# whose four waves share the keys.  Chunks of 16 / 64 / 128 rows behind 64 tokens, us, by rows and by tiles: 7, 6 / 7, 7 / 11, 8; behind 512: 10, 15 /
-# 15, 16 / 27, 17; behind 8192: 103, 163 / 153, 164 / 266, 166.
-PROMPT_ROWS_64 = (64, 256)  # up to so many rows, from this position on
+# Heads of 64, bf16 weights: tokens of a prompt (without its cached prefix) from which it goes by tiles, a shorter one by rows: by its own length and not
+# by the step's rows or the chunk's, which depend on what else is served.  Measured on MI355X, steps of four layers of a 1B decoder, us, by rows and by tiles: one
+# prompt of 16 tokens 276 and 284, 32 298 and 307, 64 350 and 358, 100 457 and 460, 128 460 and 459, 200 508 and 490, 2048 3280 and 1457; 8 of 16 447 and
+# 465, 18 of 15 485 and 494, 4 of 32 449 and 452, 8 of 32 488 and 475, 16 of 64 860 and 798, 20 of 100 1322 and 1172, 4 of 180 750 and 654.  A few rows
+# behind a long context are better by rows, where four waves share a row's keys (16 behind 8192: 73 and 191 us a layer; 128: 254 and 197).
+PROMPT_TILES_64_FROM = 65
 
 
 def prompt_attention_64(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor, tok_seq: torch.Tensor, ctx_lens: torch.Tensor, tiles: torch.Tensor, scale: float,

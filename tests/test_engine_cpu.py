@@ -1005,3 +1005,48 @@ def test_logit_bias_and_min_tokens(async_scheduling):
                       (dict(min_tokens=99), "min_tokens"), (dict(min_tokens=2, stop_token_ids=[cfg.vocab_size + 5]), "min_tokens")):
         seq = eng.make_sequence(prompt, SamplingParams(max_tokens=12, **bad))
         assert word in (eng.scheduler.validate(seq) or ""), bad
+
+
+def test_prompts_of_heads_of_64_go_by_tiles_or_rows_by_their_own_length(monkeypatch):
+    """Which kernel attends for a prompt's tokens does not depend on what else a step holds nor on where its budget cuts the prompt, down to a last token; every row
+    is served once, and the results are those of the engine without tiles."""
+    from kvmini.models.llama import LlamaConfig
+    from kvmini.ops import torch_ops as ops
+
+    cfg = LlamaConfig("small-hd64", 512, 128, 128, 2, 2, 1, 64, 10000.0, 1e-5, 512, 1, 2)
+    weights = random_weights(cfg, "cpu", torch.float32, seed=1)
+    prompts = {n: [1 + (7 * i + n) % 500 for i in range(n)] for n in (20, 64, 65, 100, 129, 150)}
+
+    def engine(budget):
+        return LLMEngine(EngineConfig(model=cfg.name, device="cpu", dtype="fp32", max_num_seqs=4, max_batched_tokens=budget, max_model_len=256, num_blocks=80, block_size=16), weights=weights)
+
+    def by_tiles(q, kc, vc, bt, tok_seq, ctx, tiles, scale):
+        ctx = ctx.clone()
+        for row, n, pos, seq in tiles.T.tolist():
+            assert (ctx[row : row + n] == -1).all() and (tok_seq[row : row + n] == seq).all()
+            ctx[row : row + n] = torch.arange(pos + 1, pos + n + 1)
+        assert (ctx >= 0).all()
+        return ops.paged_attention(q, kc, vc, bt, tok_seq, ctx, scale, bt.shape[1])
+
+    monkeypatch.setattr(ops, "PROMPT_TILES_64_FROM", 65, raising=False)
+    monkeypatch.setattr(ops, "prompt_attention_64", by_tiles, raising=False)
+    ways = {}  # (tokens of the prompt, position) -> how it was served
+    for together in ((20,), (64,), (65,), (100,), (129,), (20, 150), (100, 150), (64, 129), (100, 64, 129), (150, 65, 20, 64)):
+        for budget in (256, 64, 48):
+            eng = engine(budget)
+            runner, real = eng.runner, eng.runner._run_staged
+            runner.tiles_64 = True
+
+            def staged(t_pad, max_ctx, decode_only=0, *rest):
+                rows = [runner._dev(k, t_pad).tolist() for k in ("tok_seq", "positions", "ctx", "ctx_decode")]
+                prompt_of = {s.slot: len(s.prompt_ids) for s in eng.scheduler.running}
+                for slot, pos, ctx, alone in zip(*rows):
+                    if ctx and pos < prompt_of[slot]:
+                        ways.setdefault((prompt_of[slot], pos), set()).add("tiles" if decode_only == 0 and alone == -1 else "rows")
+                return real(t_pad, max_ctx, decode_only, *rest)
+
+            monkeypatch.setattr(runner, "_run_staged", staged)
+            params = SamplingParams(max_tokens=3, ignore_eos=True)
+            assert eng.generate([prompts[n] for n in together], params) == engine(budget).generate([prompts[n] for n in together], params)
+    assert {n for n, _pos in ways} == set(prompts)
+    assert {key: way for key, way in ways.items() if way != {"tiles" if key[0] >= 65 else "rows"}} == {}

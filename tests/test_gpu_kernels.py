@@ -3252,3 +3252,39 @@ def test_prompts_of_heads_of_64_go_by_tiles_with_bf16_weights_only(monkeypatch, 
                     weights=random_weights(cfg, "cuda:0", torch.bfloat16, seed=0))
     out = eng.generate([[1 + i % 900 for i in range(250)]], SamplingParams(max_tokens=2, ignore_eos=True))
     assert len(out[0]) == 2 and bool(by_tiles) == (quantization is None)
+
+
+def test_a_step_of_heads_of_64_with_tiles_and_rows(monkeypatch):
+    """A decode row, the short end of a prompt (by rows), a longer one and a fresh prompt (by tiles) in one step, captured and not, against the same step with
+    all rows by themselves: bf16 results of sums in another order, 0.6 % of the norm apart behind four layers; twice that is allowed."""
+    from kvmini.engine.engine import EngineConfig, LLMEngine
+    from kvmini.models.llama import LlamaConfig, random_weights
+    from kvmini.ops import hip_ops as ops
+
+    cfg = LlamaConfig("small-hd64", 1024, 512, 1024, 4, 8, 2, 64, 500000.0, 1e-5, 2048, 1, 2)
+    weights = random_weights(cfg, "cuda:0", torch.bfloat16, seed=0)
+    held, new, by_tiles, real = (299, 300, 0, 260), (1, 30, 200, 70), [], ops.prompt_attention_64
+
+    def step(graphs):
+        eng = LLMEngine(EngineConfig(model=cfg.name, device="cuda:0", max_num_seqs=4, max_batched_tokens=1024, max_model_len=512, num_blocks=128, kernels="hip", use_graphs=False), weights=weights)
+        seqs = [eng.make_sequence([1 + (i * (j + 3)) % 1000 for i in range(h + n)]) for j, (h, n) in enumerate(zip(held, new))]
+        batch = eng.scheduler.schedule_given([(s, h, []) for s, h in zip(seqs, held) if h])
+        eng.runner.execute(batch)
+        eng.scheduler.note_computed(batch)
+        if graphs:
+            eng.runner.rcfg.use_graphs = True
+            eng.runner.capture_graphs([eng.runner.bucket_for(sum(new))])
+        return eng.runner.execute(eng.scheduler.schedule_given([(s, n, list(range(max(0, n - 4), n))) for s, n in zip(seqs, new)]))[1].float(), eng.runner.kv_cache.float()
+
+    monkeypatch.setattr(ops, "prompt_attention_64", lambda *a, **k: by_tiles.append(a[6].clone()) or real(*a, **k))
+    got = step(False)
+    last = by_tiles[-1][1].tolist()
+    assert sum(last) == 270 and sum(n > 0 for n in last) == 13 + 5  # 200 rows and 70
+    replayed = step(True)
+    monkeypatch.setattr(ops, "PROMPT_TILES_64_FROM", 1 << 30)
+    before = len(by_tiles)
+    want = step(False)
+    assert len(by_tiles) == before
+    for a, b, c in zip(got, replayed, want):
+        assert torch.equal(a, b) and ((a - c).norm() / c.norm()).item() < 1.2e-2
+    assert not torch.equal(got[0], want[0])
