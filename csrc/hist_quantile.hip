@@ -545,8 +545,10 @@ __global__ __launch_bounds__(SEL_THREADS) void select_few_kernel(const T* __rest
 // interval that holds a few per cent of the samples.  The first pass counts the samples below each interval in registers, and only those inside
 // go to a histogram, a thousand linear bins of the interval's keys; the second collects the few hundred of the bins that hold the ranks, and the
 // last workgroup to finish ranks them.  Exact whatever the samples are: where an interval misses a rank (4 standard deviations aside: about one
-// call in 5000) or a bin of several values holds more than fit, the count of samples says so and the digits' passes answer (two distant
-// clusters with a rank between them: 157 us for 95).
+// call in 5000) the row's count of samples says so and the digits' passes answer for it.  Where a bin of several values holds more than fit (narrow
+// clusters far apart with a rank between them) the count says that the two passes are to be made again, between the least and the most of that bin (4 M doubles 112 us,
+// by digits 142, 3 x 1 M floats 90 and 73).
+// (Pieces between 32 sampled values with bins of their own, or intervals cut at their widest gap, leave no such bin and cost every call 4 to 7 us.)
 // Whole calls by digits and so, 3 rows: 33 k floats 54 and 48 us, 1 M 69 and 52, 4 M 88 and 69;
 // 4 M doubles 198 and 79.  Of the 56 us of kernels for 3 x 4 M floats the passes are 14 and 10, the sample 6, the last workgroup's ranking 9: chains of
 // dependent steps, about one us each.
@@ -555,6 +557,7 @@ constexpr int SPANS = KV_MAX_RANKS / 2;              // intervals: one per level
 constexpr int SPAN_BINS = 1024, SPAN_COPIES = 2;     // LDS: 4 x 1024 x 2 counts, 32 KiB (a lane uses copy lane % 2: values that many samples share)
 constexpr int FOUND = 16384;                         // samples of a bin that are ranked
 constexpr unsigned long long UNDECIDED = ~0ull;      // as a count: the digits' passes have to answer
+constexpr unsigned long long CROWDED = ~0ull - 1;    // as a count: the intervals are narrower now, the passes have to be made again
 constexpr long long SPLIT_MOST = 1ll << 25;          // of a row: beyond, what a sample says is too wide for FOUND (60 M floats: 182 us, by digits 179)
 
 // What the sample says about a row, and what the passes count.  Keys are the samples' own, in the low bits.
@@ -658,7 +661,7 @@ __global__ __launch_bounds__(SEL_THREADS) void select_sample_kernel(const T* __r
   T v[EACH];
 #pragma unroll
   for (int j = 0; j < EACH; ++j) {
-    // somewhere in the stretch: samples at even distances would all be, say, a request's first
+    // somewhere in the stretch: samples at even distances would all be, say, a request's first (mixed as 32-bit xxHash ends, by Yann Collet)
     const unsigned long long at = tid + j * SEL_THREADS, from = at * (unsigned long long)n / SAMPLED, len = (at + 1) * (unsigned long long)n / SAMPLED - from;
     unsigned int r = (unsigned int)at * 2654435761u + (unsigned int)m * 40503u;
     r ^= r >> 15; r *= 2246822519u; r ^= r >> 13; r *= 3266489917u; r ^= r >> 16;
@@ -854,15 +857,18 @@ struct Chosen {
 
 // The last workgroup: ranks what was found in the U chosen bins.  Each rank has its own, narrower bins of them, again and again until what is left
 // is one value or fits a wave's lanes: at once for most samples, at most log(keys) / log(RANK_BINS) times.
+// (Inlined: as a call the compiler's choice, it cost the passes 4 us.)
 constexpr int RANK_BINS = 1024;
 template <typename T>
-__device__ void rank_found(const SplitRow& row, const Chosen& c, int R, int U, unsigned int* h, unsigned long long count, unsigned long long* out) {
+__device__ __forceinline__ void rank_found(const SplitRow& row, const Chosen& c, int R, int U, unsigned int* h, unsigned long long count, unsigned long long* out) {
   __shared__ unsigned long long few[KV_MAX_RANKS][64], from[KV_MAX_RANKS], upto[KV_MAX_RANKS], least[KV_MAX_RANKS], most[KV_MAX_RANKS];  // of a rank
+  __shared__ unsigned long long answer[KV_MAX_RANKS];
   __shared__ int bin_of[KV_MAX_RANKS], picked[KV_MAX_RANKS], held[KV_MAX_RANKS], cnt[KV_MAX_RANKS];
-  __shared__ bool undecided;
+  __shared__ bool undecided, crowded[KV_MAX_RANKS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, rest = 64 - KeyOf<T>::bits;
   if (tid == 0) undecided = false;
   if (tid < KV_MAX_RANKS) {
+    crowded[tid] = false;
     const unsigned int f = tid < U ? __hip_atomic_load(&row.state->found[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
     cnt[tid] = f <= FOUND ? (int)f : 0;
   }
@@ -871,13 +877,15 @@ __device__ void rank_found(const SplitRow& row, const Chosen& c, int R, int U, u
     int u = tid < R ? c.bin_of[tid] : -1;
     if (tid < R && u < 0) undecided = true;
     if (u >= 0) {
+      const unsigned int in_bin = row.bins[c.id[tid]];
       from[tid] = __hip_atomic_load(&row.state->least[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       upto[tid] = __hip_atomic_load(&row.state->most[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (from[tid] == upto[tid]) {  // one value
-        out[tid] = from[tid] << rest;
+      const bool first = c.place[tid] == 0;
+      if (first || c.place[tid] + 1 == in_bin || from[tid] == upto[tid]) {  // the least, the most, one value
+        answer[tid] = first ? from[tid] : upto[tid];
         u = -1;
       } else if (cnt[u] == 0) {
-        undecided = true;
+        crowded[tid] = true;
         u = -1;
       }
     }
@@ -948,12 +956,12 @@ __device__ void rank_found(const SplitRow& row, const Chosen& c, int R, int U, u
       const int have = held[wave];
       left = have > 64 && least[wave] != most[wave];
       if (least[wave] == most[wave]) {
-        if (lane == 0) out[wave] = least[wave] << rest;
+        if (lane == 0) answer[wave] = least[wave];
       } else if (!left) {
         const unsigned long long key = lane < have ? few[wave][lane] : ~0ull;
         unsigned int before = 0;
         for (int j = 0; j < have; ++j) before += few[wave][j] < key || (few[wave][j] == key && j < lane);
-        if (lane < have && before == place) out[wave] = key << rest;
+        if (lane < have && before == place) answer[wave] = key;
       }
       if (lane == 0) {
         from[wave] = least[wave];
@@ -963,7 +971,17 @@ __device__ void rank_found(const SplitRow& row, const Chosen& c, int R, int U, u
     }
     more = __syncthreads_or(left);
   }
-  if (tid == 0) out[KV_MAX_RANKS] = undecided ? UNDECIDED : count;
+  if (wave > 0) return;  // (behind the loop's last barrier)
+  const bool again = __ballot(lane < R && crowded[lane < R ? lane : 0]) != 0;
+  if (lane < R) out[lane] = answer[lane] << rest;
+  if (lane == 0) out[KV_MAX_RANKS] = undecided ? UNDECIDED : again ? CROWDED : count;
+  if (again && lane < R / 2) {
+    // a level's ranks follow one another: beside one in a crowded bin the other is in there too, or it would be the bin's first or last and not be crowded
+    const int l = 2 * lane, r = crowded[l] ? l : l + 1;
+    row.state->ends[l] = crowded[r] ? from[r] : answer[l];
+    row.state->ends[l + 1] = crowded[r] ? upto[r] : answer[l + 1];
+    if (lane == 0) row.state->open = 0;
+  }
 }
 
 // The second pass.  Grid (workgroups, metrics).
@@ -1052,6 +1070,20 @@ __global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __
   if (tid == 0) last = __hip_atomic_fetch_add(&row.state->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
   __syncthreads();
   if (last) rank_found<T>(row, c, R, U, reinterpret_cast<unsigned int*>(keys), count, out + (long long)m * SEL_OUT);
+}
+
+// Before the passes are made again between the ends that the last ones left.  Grid (workgroups, metrics).
+__global__ __launch_bounds__(SEL_THREADS) void select_again_kernel(void* work) {
+  const SplitRow row(work, blockIdx.y);
+  const int i = blockIdx.x * SEL_THREADS + threadIdx.x;
+  if (i < SPANS * SPAN_BINS) row.bins[i] = 0;
+  if (i < SPANS) row.state->below[i] = 0;
+  if (i < KV_MAX_RANKS) {
+    row.state->least[i] = ~0ull;
+    row.state->most[i] = 0;
+    row.state->found[i] = 0;
+  }
+  if (i == 0) { row.state->count = 0; row.state->done = 0; }
 }
 
 // clears a selection's state, histograms and counters (a kernel, not a memset: callers may capture it)
@@ -1238,12 +1270,16 @@ int select_parts(long long n, int n_metrics, int dtype) {
 }
 
 template <typename T>
-int select_split(const T* x, long long n, long long row_stride, int n_metrics, int dtype, const Levels& lv, void* work, unsigned long long* out, hipStream_t stream) {
-  int parts = SAMPLE_PARTS;
-  while (parts > 1 && parts * n_metrics > 256) parts /= 2;
-  // (a larger sample of longer rows: it takes 6 us more, and what lies beyond its largest has to fit FOUND)
-  auto sample = n <= 1 << 22 ? select_sample_kernel<T, 2> : select_sample_kernel<T, 4>;
-  hipLaunchKernelGGL(sample, dim3(parts, n_metrics), dim3(SEL_THREADS), 0, stream, x, n, row_stride, lv, work);
+int select_split(const T* x, long long n, long long row_stride, int n_metrics, int dtype, const Levels& lv, void* work, unsigned long long* out, bool again, hipStream_t stream) {
+  if (again) {
+    hipLaunchKernelGGL(select_again_kernel, dim3(SPANS * SPAN_BINS / SEL_THREADS, n_metrics), dim3(SEL_THREADS), 0, stream, work);
+  } else {
+    int parts = SAMPLE_PARTS;
+    while (parts > 1 && parts * n_metrics > 256) parts /= 2;
+    // (a larger sample of longer rows: it takes 6 us more, and what lies beyond its largest has to fit FOUND)
+    auto sample = n <= 1 << 22 ? select_sample_kernel<T, 2> : select_sample_kernel<T, 4>;
+    hipLaunchKernelGGL(sample, dim3(parts, n_metrics), dim3(SEL_THREADS), 0, stream, x, n, row_stride, lv, work);
+  }
   const dim3 grid(select_parts(n, n_metrics, dtype), n_metrics);
   static const bool ok = big_lds(select_split_kernel<T>);
   if (!ok) return -2;
@@ -1333,18 +1369,19 @@ int kv_select_quantiles(const void* x, long long n, long long row_stride, int n_
 }
 
 // The same by a sample's intervals, for the rows that kv_split_takes (scratch memory: kv_split_work_bytes): a count of kv_undecided() says that
-// kv_select_quantiles has to answer.
+// kv_select_quantiles has to answer, one of kv_crowded() that this has to be called again with what it left in the scratch memory.
 int kv_split_takes(long long n, int n_metrics, int dtype) { return n > (dtype == 0 ? SEL_FEW : SEL_RANKED) && n <= SPLIT_MOST && n_metrics <= 64; }
 long long kv_split_work_bytes(int n_metrics) { return n_metrics * SPLIT_BYTES; }
 unsigned long long kv_undecided() { return UNDECIDED; }
+unsigned long long kv_crowded() { return CROWDED; }
 
-int kv_split_quantiles(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const double* ps, int n_ps, void* work, unsigned long long* out, hipStream_t stream) {
+int kv_split_quantiles(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const double* ps, int n_ps, void* work, unsigned long long* out, int again, hipStream_t stream) {
   if (n_metrics <= 0 || !kv_split_takes(n, n_metrics, dtype) || n_ps < 1 || n_ps > KV_MAX_RANKS / 2) return -1;
   Levels lv{};
   lv.n = n_ps;
   for (int i = 0; i < n_ps; ++i) lv.p[i] = ps[i];
-  return dtype == 0 ? select_split((const float*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream)
-                    : select_split((const double*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream);
+  return dtype == 0 ? select_split((const float*)x, n, row_stride, n_metrics, dtype, lv, work, out, again != 0, stream)
+                    : select_split((const double*)x, n, row_stride, n_metrics, dtype, lv, work, out, again != 0, stream);
 }
 
 // The same selection one pass at a time, for samples spread over several ranks: every rank runs

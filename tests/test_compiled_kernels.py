@@ -90,7 +90,7 @@ def test_unwaited_arrivals_are_found():
 def test_every_wave_waits_before_an_arrival_is_counted(functions):
     """Workgroups that count themselves as finished — with a pass of the exact quantiles, with their share of a decode step's keys, with their part of
     a split product: every wave waits for what it wrote or added before the barrier behind which the arrival is counted."""
-    for part, least in (("select_pass_kernel", 2), ("decode_attention_fused_kernel", 8), ("stream_gemm", 1)):
+    for part, least in (("select_pass_kernel", 2), ("select_collect_kernel", 2), ("decode_attention_fused_kernel", 8), ("stream_gemm", 1)):
         arriving = {n: b for n, b in functions(part).items() if any(re.match(r"global_atomic_add\b.*\bsc0\b", line) for line in b)}
         assert len(arriving) >= least, part
         assert {n: unwaited_arrivals(b) for n, b in arriving.items()} == {n: [] for n in arriving}

@@ -221,6 +221,47 @@ def test_quantiles_of_an_interval_up_to_the_largest_values(n, middle, largest):
     assert np.array_equal(got[0], [largest, middle]), got
 
 
+def _sampled_places(n):
+    """Where the selection by a sample's intervals looks at the first row of a call."""
+    sampled = 2048 if n <= 1 << 22 else 4096
+    at = np.arange(sampled, dtype=np.uint64)
+    first = at * np.uint64(n) // np.uint64(sampled)
+    r = (at * np.uint64(2654435761)).astype(np.uint32)
+    for shift, times in ((15, 2246822519), (13, 3266489917)):
+        r = (r ^ (r >> np.uint32(shift))) * np.uint32(times)
+    r ^= r >> np.uint32(16)
+    return first + (r.astype(np.uint64) * ((at + np.uint64(1)) * np.uint64(n) // np.uint64(sampled) - first) >> np.uint64(32))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [16385, 300_007, 5_000_001])
+def test_quantiles_by_intervals_row_by_row(C, n, dtype):
+    """Which form answers for a row, and that it does so exactly, alone and beside the others: the intervals of a sample; the same again where a bin is crowded (narrow
+    clusters far apart, three of them too, the rank inside one and at its edge); the digits where the sample says nothing true about the row."""
+    from kvmini.ops import hist_quantile as hq
+
+    rng = np.random.default_rng(n)
+    g = 12 * np.exp(0.35 * rng.normal(size=n))
+    narrow = 1e-4 if dtype is np.float64 else 0.02
+    cluster = lambda shares: np.select([rng.permutation(n) < int(n * s) for s in shares], [1e3 ** i for i in range(len(shares))]) * (1 + narrow * rng.random(n))  # noqa: E731
+    misled = 100 + rng.random(n)
+    misled[_sampled_places(n).astype(np.int64)] = rng.random(_sampled_places(n).size)
+    rows = {"misled": misled, "normal": g, "sorted": np.sort(g), "few": np.round(g), "halves": np.where(rng.random(n) < 0.5, 10.0, 20.0), "gap": cluster((0.5, 1.0)), "inside": cluster((0.51, 1.0)),
+            "three": cluster((0.499, 0.003, 1.0))}
+    x, ps, forms = np.stack(list(rows.values())).astype(dtype), (0.5, 0.95, 0.99), {}
+    d = torch.from_numpy(x).to(_dev())
+    together = hq.batched_quantiles(d, ps)
+    for i, name in enumerate(rows):
+        v = np.sort(x[i]).astype(np.float64)
+        at = [p * (n - 1) for p in ps]
+        want = [v[int(a)] if a == int(a) else v[int(a)] + (a - int(a)) * (v[int(a) + 1] - v[int(a)]) for a in at]
+        assert np.array_equal(together[i], want) and np.array_equal(hq.batched_quantiles(d[i : i + 1], ps)[0], want), (name, together[i], want)
+        forms[name] = int(C.quantiles_by_intervals(d[i : i + 1].contiguous(), list(ps))[0])
+    assert forms["misled"] == -1 and all(forms[name] == 1 for name in ("normal", "sorted", "few", "halves")), forms
+    if n > 1_000_000:
+        assert forms["inside"] == 0, forms
+
+
 def test_equal_width_histogram_matches_cpu():
     from kvmini.analysis.histograms import compute_histogram
     from kvmini.ops import hist_quantile as hq
