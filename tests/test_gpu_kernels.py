@@ -3243,7 +3243,7 @@ def test_rope_at_the_line_between_its_kernels(C, nh, nkv, hd, kv8, more):
     assert all(torch.equal(a, b) for a, b in zip(*out))
 
 
-@pytest.mark.parametrize("top", [1, 6, 7])
+@pytest.mark.parametrize("top", [1, 6, 7, 13])
 @pytest.mark.parametrize("t", [3, 130])
 @pytest.mark.parametrize("ld", [64, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196])
 def test_residuals_of_experts_rows_at_the_edges_of_their_forms(ld, t, top):
