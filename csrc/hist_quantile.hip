@@ -546,12 +546,12 @@ __global__ __launch_bounds__(SEL_THREADS) void select_few_kernel(const T* __rest
 // go to a histogram, a thousand linear bins of the interval's keys; the second collects the few hundred of the bins that hold the ranks, and the
 // last workgroup to finish ranks them.  Exact whatever the samples are: where an interval misses a rank (4 standard deviations aside: about one
 // call in 5000) the row's count of samples says so and the digits' passes answer for it.  Where a bin of several values holds more than fit (narrow
-// clusters far apart with a rank between them) the count says that the two passes are to be made again, between the least and the most of that bin (4 M doubles 112 us,
-// by digits 142, 3 x 1 M floats 90 and 73).
+// clusters far apart with a rank between them) the count says that the two passes are to be made again, between the least and the most of that bin (a row of 4 M
+// doubles 112 us, by digits 142; 3 of 1 M floats 90 and 73).
 // (Pieces between 32 sampled values with bins of their own, or intervals cut at their widest gap, leave no such bin and cost every call 4 to 7 us.)
 // Whole calls by digits and so, 3 rows: 33 k floats 54 and 48 us, 1 M 69 and 52, 4 M 88 and 69;
-// 4 M doubles 198 and 79.  Of the 56 us of kernels for 3 x 4 M floats the passes are 14 and 10, the sample 6, the last workgroup's ranking 9: chains of
-// dependent steps, about one us each.
+// 4 M doubles 198 and 79.  Of the 55 us of kernels for 3 x 4 M floats the sample takes 9, the first pass 20 and the second 26, the last workgroup's ranking
+// among them: beside reading (10 us a pass at 5 TB/s) chains of dependent steps, about one us each.
 constexpr int SAMPLE_PARTS = 64;                     // workgroups that rank a row's sample, at most
 constexpr int SPANS = KV_MAX_RANKS / 2;              // intervals: one per level, fewer where they overlap
 constexpr int SPAN_BINS = 1024, SPAN_COPIES = 2;     // LDS: 4 x 1024 x 2 counts, 32 KiB (a lane uses copy lane % 2: values that many samples share)
@@ -724,7 +724,7 @@ __device__ inline uint64_t in_sgpr(uint64_t v) { return (uint64_t)in_sgpr((uint3
 //
 // What bounds it is instructions per sample, not memory: the samples are compared as they are (two instructions per interval, the masks they leave
 // counted by the scalar unit), and those inside queue up per wave, so that the two dozen instructions that bin one run on full waves and not on the five lanes
-// of 64 that have one.  (The pass over 3 x 4 M floats: 16.5 us with each instruction's few lanes on their own, 14.4 so.)
+// of 64 that have one.  (With each instruction's few lanes on their own the pass over 3 x 4 M floats took 2 us more of its 20.)
 template <typename T, int V>
 __device__ void split_pass(const T* row, long long n, int part, int parts, const Spans& s, T* queue, unsigned int* h, unsigned int* below, unsigned int* valid) {
   using KT = typename KeyOf<T>::type;

@@ -77,7 +77,10 @@ struct ResidualArgs {
 template <typename T>
 __device__ inline float4 row4(const RowSource& s, long long t, int c) {
   if (s.w) {
-    // (six rows are asked for before the first is added: one by one their latencies were the launch's time)
+    // Six rows are asked for before the first is added: one by one their latencies were the launch's time.  Behind the last row it is asked for again, and rows of
+    // weight zero with the others: from the cache, or bytes that cost less than the wait for the weights would.  2000 rows of 4096 columns, gated, one by one
+    // and so, us: 1 of experts 20.9 and 21.1, 2 27.0 and 25.0, 4 33.6 and 28.1, 6 41.5 and 33.7, 8 49.6 and 40.1, 12 63.6 and 49.5; a quarter of the rows with no
+    // weight: 2 24.3 and 25.1, 6 33.8 and 32.6; 16 rows of 2048: 1 3.9 and 3.6, 8 5.1 and 4.2.
     constexpr int B = 6;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int k0 = 0; k0 < s.n_slabs; k0 += B) {

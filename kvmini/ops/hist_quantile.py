@@ -1,10 +1,13 @@
 """Python side of ``csrc/hist_quantile.hip``: exact batched quantiles, 20-bin
 histograms and a persistent streaming histogram on the GPU.
 
-Exactness: the kernel selects the order statistics ``floor(p*(n-1))`` and
-``ceil(p*(n-1))`` exactly (radix select on order-preserving keys); the linear
-interpolation between them happens here in float64 with the reference's formula
-(``analyze.py:75-81``), so results equal the CPU oracle bit for bit on float64
+Exactness: the kernels select the order statistics ``floor(p*(n-1))`` and
+``ceil(p*(n-1))`` exactly on order-preserving keys — short rows by rank, rows of
+middle sizes between values that a sample of them gives, the others and those that
+a sample does not decide digit by digit.  The linear interpolation between them, in float64
+with the reference's formula (``analyze.py:75-81``), is the extension's for
+:func:`batched_quantiles` (``select_quantiles`` in ``csrc/bindings.cpp``) and this module's for
+:func:`distributed_quantiles`, whose ranks go by digits; either way results equal the CPU oracle bit for bit on float64
 input.
 """
 
