@@ -545,16 +545,15 @@ __global__ __launch_bounds__(SEL_THREADS) void select_few_kernel(const T* __rest
 // interval that holds a few per cent of the samples.  The first pass counts the samples below each interval in registers, and only those inside
 // go to a histogram, a thousand linear bins of the interval's keys; the second collects the few hundred of the bins that hold the ranks, and the
 // last workgroup to finish ranks them.  Exact whatever the samples are: where an interval misses a rank (4 standard deviations aside: about one
-// call in 5000) the row's count of samples says so and the digits' passes answer for it.  Where a bin of several values holds more than fit (narrow
-// clusters far apart with a rank between them) the count says that the two passes are to be made again, between the least and the most of that bin (a row of 4 M
-// doubles 112 us, by digits 142; 3 of 1 M floats 90 and 73).
-// (Pieces between 32 sampled values with bins of their own, or intervals cut at their widest gap, leave no such bin and cost every call 4 to 7 us.)
+// call in 5000) the row's count of samples says so and the digits' passes answer for it.  Where a bin of several values holds more than fit all the same
+// (Spans says what is done against that) the count says that the two passes are to be made again, between the least and the most of that bin.
 // Whole calls by digits and so, 3 rows: 33 k floats 54 and 48 us, 1 M 69 and 52, 4 M 88 and 69;
 // 4 M doubles 198 and 79.  Of the 55 us of kernels for 3 x 4 M floats the sample takes 9, the first pass 20 and the second 26, the last workgroup's ranking
 // among them: beside reading (10 us a pass at 5 TB/s) chains of dependent steps, about one us each.
 constexpr int SAMPLE_PARTS = 64;                     // workgroups that rank a row's sample, at most
 constexpr int SPANS = KV_MAX_RANKS / 2;              // intervals: one per level, fewer where they overlap
 constexpr int SPAN_BINS = 1024, SPAN_COPIES = 2;     // LDS: 4 x 1024 x 2 counts, 32 KiB (a lane uses copy lane % 2: values that many samples share)
+constexpr int PIECES = 32, PIECE_BINS = SPAN_BINS / PIECES;  // of an interval with a gap
 constexpr int FOUND = 16384;                         // samples of a bin that are ranked
 constexpr unsigned long long UNDECIDED = ~0ull;      // as a count: the digits' passes have to answer
 constexpr unsigned long long CROWDED = ~0ull - 1;    // as a count: the intervals are narrower now, the passes have to be made again
@@ -562,13 +561,14 @@ constexpr long long SPLIT_MOST = 1ll << 25;          // of a row: beyond, what a
 
 // What the sample says about a row, and what the passes count.  Keys are the samples' own, in the low bits.
 struct SplitState {
-  unsigned long long ends[KV_MAX_RANKS];             // level -> sampled keys at the ends of its interval
+  unsigned long long cuts[SPANS][PIECES + 1];        // level -> sampled keys at the ends of its interval and, evenly many apart, between them
   unsigned long long below[SPANS];                   // samples in front of each interval, as Spans orders them
   unsigned long long count;                          // samples
   unsigned long long least[KV_MAX_RANKS], most[KV_MAX_RANKS];  // of the samples in a chosen bin
   unsigned int found[KV_MAX_RANKS];                  // how many those are
   unsigned int done;
-  unsigned int open;                                 // ends beyond which the interval goes on (a bit each): no sampled key is as far out as it has to be
+  unsigned int open;                                 // ends (two per level) beyond which the interval goes on: no sampled key is as far out as it has to be
+  int together[SPANS];                               // level -> a bin with this many pieces between cuts, or more, is too full for FOUND
 };
 constexpr int SPLIT_WORDS = sizeof(SplitState) / 4;
 constexpr long long SPLIT_BYTES = sizeof(SplitState) + SPANS * SPAN_BINS * 4 + (long long)KV_MAX_RANKS * FOUND * 8;
@@ -593,23 +593,32 @@ __device__ inline int bin_shift(unsigned long long wide) {
   return wide < BINS ? 0 : 64 - __clzll((long long)wide) - (31 - __builtin_clz(BINS));
 }
 
-// The levels' intervals in order, those that overlap as one.  By one thread, in registers.
+// The levels' intervals in order, those that overlap as one, with linear bins.  Where so many cuts fall into one bin that it is too full for FOUND (a gap takes nearly all bins: hits
+// and misses of a cache, with a rank between them) and no intervals overlap, each has 32 pieces between its cuts instead, of 32 linear bins: 3 x 4 M floats in two clusters 75 us
+// a call, by passes made again 137, by digits 98.  Not for all rows: linear bins need no search for the piece (1 to 2 us), and the piece around a small gap
+// holds more than any of them (clusters of 5 % 82 and 69 us).
+template <typename KT>
 struct Spans {
   unsigned long long lo[SPANS], hi[SPANS];  // ends
   unsigned long long from[SPANS];           // the bins are those of from ... upto: the first takes in what is below, the last what is above
   int shift[SPANS];
   int of[SPANS];                            // level -> interval
   int n;
+  bool crowded;                             // a bin is too full: there are pieces, of use if no intervals overlap
+  KT search[SPANS * PIECES];                // keys from here on ...
+  KT base[SPANS * PIECES];                  // ... in linear bins from here on, the first takes in what is below, the last what is above
+  int piece_shift[SPANS * PIECES];
 };
+// By one thread, in registers: the intervals.
 template <typename T>
-__device__ inline void find_spans(const SplitState& s, int levels, Spans* to) {
+__device__ inline void find_linear(const SplitState& s, int levels, Spans<typename KeyOf<T>::type>* to) {
   unsigned long long lo[SPANS], hi[SPANS], from[SPANS], upto[SPANS];
   int level[SPANS];
   const unsigned int open = s.open;
 #pragma unroll
   for (int i = 0; i < SPANS; ++i) {
-    from[i] = i < levels ? s.ends[2 * i] : ~0ull;
-    upto[i] = i < levels ? s.ends[2 * i + 1] : ~0ull;
+    from[i] = i < levels ? s.cuts[i][0] : ~0ull;
+    upto[i] = i < levels ? s.cuts[i][PIECES] : ~0ull;
     // (as values: both zeros, which compare as one, are in or out together)
     lo[i] = open >> 2 * i & 1 ? KeyOf<T>::key(-(T)INFINITY) : from[i] == KeyOf<T>::key((T)0) ? KeyOf<T>::key(-(T)0) : from[i];
     hi[i] = open >> (2 * i + 1) & 1 ? KeyOf<T>::key((T)INFINITY) : upto[i] == KeyOf<T>::key(-(T)0) ? KeyOf<T>::key((T)0) : upto[i];
@@ -642,9 +651,52 @@ __device__ inline void find_spans(const SplitState& s, int levels, Spans* to) {
     to->from[n - 1] = in;
     to->shift[n - 1] = bin_shift<SPAN_BINS>(out - in);
     to->of[level[i]] = n - 1;
+    to->search[(n - 1) * PIECES] = (typename KeyOf<T>::type)first;
   }
+  for (int i = n; i < SPANS; ++i) to->search[i * PIECES] = ~(typename KeyOf<T>::type)0;
   to->n = n;
 }
+// By a wave, meanwhile: the pieces, two a lane.
+template <typename T>
+__device__ inline void find_pieces(const SplitState& s, int levels, Spans<typename KeyOf<T>::type>* to) {
+  using KT = typename KeyOf<T>::type;
+  static_assert(SPANS * PIECES == 2 * 64, "of all levels");
+  constexpr int LANES = PIECES / 2;  // of a level
+  const int lane = threadIdx.x & 63, l = lane / LANES, j = lane % LANES * 2, q = s.together[l];
+  const unsigned long long before = s.cuts[l][j > 0 ? j - 1 : 0], cut[3] = {s.cuts[l][j], s.cuts[l][j + 1], s.cuts[l][j + 2]};
+  const unsigned long long from = __shfl(cut[0], l * LANES, 64), upto = __shfl(cut[2], l * LANES + LANES - 1, 64);
+  const int shift = bin_shift<SPAN_BINS>(upto - from), bin[2] = {(int)((cut[0] - from) >> shift), (int)((cut[1] - from) >> shift)};
+  bool full = false;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int k = j + e + q, at = (l * LANES + k / 2) & 63, even = __shfl(bin[0], at, 64), odd = __shfl(bin[1], at, 64);
+    full = full || (k < PIECES && (k & 1 ? odd : even) == bin[e]);
+  }
+  int place = 0;  // of the level's interval among all
+#pragma unroll
+  for (int i = 0; i < SPANS; ++i) place += i < levels && __shfl(from, i * LANES, 64) < from;
+  const bool crowded = __ballot(full && l < levels && shift > 0) != 0;
+  if (lane == 0) to->crowded = crowded;
+  if (!crowded) return;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    // (a key that is several cuts, a timeout, say, has a piece of its own: the last of them begins behind it)
+    const bool again = e == 0 ? j > 0 && cut[0] == before : cut[1] == cut[0];
+    const unsigned long long base = cut[e] + (again && cut[e + 1] != cut[e] ? 1 : 0);
+    const int p = (l < levels ? place : l) * PIECES + j + e;
+    to->base[p] = l < levels ? (KT)base : ~(KT)0;
+    if (j + e > 0) to->search[p] = l < levels ? (KT)base : ~(KT)0;
+    to->piece_shift[p] = cut[e + 1] > base ? bin_shift<PIECE_BINS>(cut[e + 1] - base) : 0;
+  }
+}
+template <typename T>
+__device__ inline void find_spans(const SplitState& s, int levels, Spans<typename KeyOf<T>::type>* to) {
+  if (threadIdx.x == 0) find_linear<T>(s, levels, to);
+  if (threadIdx.x / 64 == 1) find_pieces<T>(s, levels, to);
+  __syncthreads();
+}
+template <typename KT>
+__device__ inline bool pieced(const Spans<KT>& s, int levels) { return s.crowded && s.n == levels; }
 
 // The levels' intervals, from EACH samples per thread.  Grid (workgroups, metrics): each takes in all sampled keys, ranks its share of them against all, and writes those whose
 // rank is that of an end.  (One workgroup that selects by digits took 45 us: a chain of loads, LDS sums and scans on one compute unit.)
@@ -654,7 +706,7 @@ __global__ __launch_bounds__(SEL_THREADS) void select_sample_kernel(const T* __r
   constexpr int SAMPLED = EACH * SEL_THREADS;
   __shared__ __attribute__((aligned(16))) KT keys[SAMPLED];
   __shared__ unsigned int before[SEL_THREADS];
-  __shared__ unsigned int rank[KV_MAX_RANKS];
+  __shared__ unsigned int rank[KV_MAX_RANKS];  // of the levels' ends
   const int tid = threadIdx.x, m = blockIdx.y;
   const SplitRow row(work, m);
   const T* xr = x + (long long)m * row_stride;
@@ -673,7 +725,6 @@ __global__ __launch_bounds__(SEL_THREADS) void select_sample_kernel(const T* __r
     keys[tid + j * SEL_THREADS] = key_or_last(v[j]);
     got += __syncthreads_count(v[j] == v[j]);
   }
-  const int R = 2 * levels.n;
   if (tid < KV_MAX_RANKS) {
     double p = levels.p[tid >> 1];
     p = p < 0.0 ? 0.0 : (p > 1.0 ? 1.0 : p);
@@ -683,7 +734,9 @@ __global__ __launch_bounds__(SEL_THREADS) void select_sample_kernel(const T* __r
     rank[tid] = end < 0.0 ? 0 : end > (double)(got - 1) ? (unsigned int)(got - 1) : (unsigned int)end;
     const unsigned int opens = (unsigned int)__ballot(open);
     if (blockIdx.x == 0) {
-      if (got == 0) row.state->ends[tid] = KeyOf<T>::key((tid & 1) ? (T)INFINITY : -(T)INFINITY);
+      // samples of a piece: those of the row over those of the sample, times the ranks between two cuts
+      const float ranks = (float)(rank[tid | 1] - rank[tid & ~1] + 1), each = (float)n * ranks * __builtin_amdgcn_rcpf((float)got * PIECES);
+      if (tid & 1) row.state->together[tid >> 1] = 1 + (int)fminf(0.75f * FOUND * __builtin_amdgcn_rcpf(each), (float)PIECES);
       row.state->least[tid] = ~0ull;
       row.state->most[tid] = 0;
       row.state->found[tid] = 0;
@@ -691,6 +744,7 @@ __global__ __launch_bounds__(SEL_THREADS) void select_sample_kernel(const T* __r
       if (tid == 0) { row.state->count = 0; row.state->done = 0; row.state->open = opens; }
     }
   }
+  if (got == 0 && blockIdx.x == 0 && tid < SPANS * (PIECES + 1)) row.state->cuts[tid / (PIECES + 1)][tid % (PIECES + 1)] = KeyOf<T>::key(tid % (PIECES + 1) == PIECES ? (T)INFINITY : -(T)INFINITY);
   for (int i = blockIdx.x * SEL_THREADS + tid; i < SPANS * SPAN_BINS; i += gridDim.x * SEL_THREADS) row.bins[i] = 0;
   // as many threads per key as there are, each for a stretch of the others
   const int ours = SAMPLED / (int)gridDim.x, together = ours < SEL_THREADS ? ours : SEL_THREADS, stretch = SAMPLED / (SEL_THREADS / together);
@@ -703,8 +757,14 @@ __global__ __launch_bounds__(SEL_THREADS) void select_sample_kernel(const T* __r
     atomicAdd(&before[mine], count_in_front(keys, from, stretch, at, key));
     __syncthreads();
     if (tid < together && key != ~(KT)0)
-      for (int r = 0; r < R; ++r)
-        if (rank[r] == before[tid]) row.state->ends[r] = key;
+      for (int l = 0; l < levels.n; ++l) {
+        const unsigned int at = before[tid] - rank[2 * l], wide = rank[2 * l + 1] - rank[2 * l];
+        if (at > wide) continue;
+        // the cuts j with wide j / PIECES = at, whole numbers: few, from one that the quotient names (it is rounded) or a neighbour on
+        const int j = (int)((float)(at * PIECES) * __builtin_amdgcn_rcpf((float)wide));
+        for (unsigned int k = wide && j > 0 ? j - 1 : 0; k <= PIECES && wide * k / PIECES <= at; ++k)
+          if (wide * k / PIECES == at) row.state->cuts[l][k] = key;
+      }
     __syncthreads();
   }
 }
@@ -725,8 +785,8 @@ __device__ inline uint64_t in_sgpr(uint64_t v) { return (uint64_t)in_sgpr((uint3
 // What bounds it is instructions per sample, not memory: the samples are compared as they are (two instructions per interval, the masks they leave
 // counted by the scalar unit), and those inside queue up per wave, so that the two dozen instructions that bin one run on full waves and not on the five lanes
 // of 64 that have one.  (With each instruction's few lanes on their own the pass over 3 x 4 M floats took 2 us more of its 20.)
-template <typename T, int V>
-__device__ void split_pass(const T* row, long long n, int part, int parts, const Spans& s, T* queue, unsigned int* h, unsigned int* below, unsigned int* valid) {
+template <typename T, int V, bool PIECED>
+__device__ void split_pass(const T* row, long long n, int part, int parts, const Spans<typename KeyOf<T>::type>& s, T* queue, unsigned int* h, unsigned int* below, unsigned int* valid) {
   using KT = typename KeyOf<T>::type;
   constexpr int QUEUE = QUEUE_BYTES / sizeof(T);
   T lo[V], hi[V];
@@ -744,6 +804,14 @@ __device__ void split_pass(const T* row, long long n, int part, int parts, const
   unsigned int queued = 0, binned = 0;  // of this wave; the queue is a ring
   auto bin_one = [&](T v) {
     const KT key = KeyOf<T>::key(v);
+    if constexpr (PIECED) {
+      int at = 0;
+#pragma unroll
+      for (int step = SPANS * PIECES / 2; step > 0; step /= 2) at += s.search[at + step] <= key ? step : 0;
+      const KT begin = s.base[at], in_piece = (key > begin ? key - begin : 0) >> s.piece_shift[at];
+      atomicAdd(&h[(at * PIECE_BINS + (int)(in_piece < PIECE_BINS ? in_piece : PIECE_BINS - 1)) * SPAN_COPIES + copy], 1u);
+      return;
+    }
     KT first = from[0];
     int sh = shift[0], base = 0;
     asm("" : "+s"(first), "+s"(sh));
@@ -790,21 +858,24 @@ constexpr int SPLIT_LDS = SPANS * SPAN_BINS * SPAN_COPIES * 4 + SEL_THREADS / 64
 template <typename T>
 __global__ __launch_bounds__(SEL_THREADS) void select_split_kernel(const T* __restrict__ x, long long n, long long row_stride, int levels, void* work) {
   extern __shared__ __attribute__((aligned(16))) unsigned int h[];  // [SPANS][SPAN_BINS][SPAN_COPIES], then the waves' queues
-  __shared__ Spans s;
+  __shared__ Spans<typename KeyOf<T>::type> s;
   __shared__ unsigned int below[SPANS + 1];
   const int tid = threadIdx.x, m = blockIdx.y;
   const SplitRow row(work, m);
-  if (tid == 0) find_spans<T>(*row.state, levels, &s);
   for (int i = tid; i < SPANS * SPAN_BINS * SPAN_COPIES; i += SEL_THREADS) h[i] = 0;
   if (tid <= SPANS) below[tid] = 0;
   T* queue = reinterpret_cast<T*>(reinterpret_cast<char*>(h + SPANS * SPAN_BINS * SPAN_COPIES) + (tid >> 6) * QUEUE_BYTES);
-  __syncthreads();
+  find_spans<T>(*row.state, levels, &s);
   const T* xr = x + (long long)m * row_stride;
   const int V = s.n;
-  if (V <= 1) split_pass<T, 1>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
-  else if (V == 2) split_pass<T, 2>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
-  else if (V == 3) split_pass<T, 3>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
-  else split_pass<T, SPANS>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
+  auto pass = [&](auto v) {
+    if (pieced(s, levels)) split_pass<T, decltype(v)::value, true>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
+    else split_pass<T, decltype(v)::value, false>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
+  };
+  if (V <= 1) pass(std::integral_constant<int, 1>{});
+  else if (V == 2) pass(std::integral_constant<int, 2>{});
+  else if (V == 3) pass(std::integral_constant<int, 3>{});
+  else pass(std::integral_constant<int, SPANS>{});
   __syncthreads();
   for (int i = tid; i < V * SPAN_BINS; i += SEL_THREADS) {
     const unsigned int c = sum_copies(h, i, 1);
@@ -978,8 +1049,9 @@ __device__ __forceinline__ void rank_found(const SplitRow& row, const Chosen& c,
   if (again && lane < R / 2) {
     // a level's ranks follow one another: beside one in a crowded bin the other is in there too, or it would be the bin's first or last and not be crowded
     const int l = 2 * lane, r = crowded[l] ? l : l + 1;
-    row.state->ends[l] = crowded[r] ? from[r] : answer[l];
-    row.state->ends[l + 1] = crowded[r] ? upto[r] : answer[l + 1];
+    row.state->cuts[lane][0] = crowded[r] ? from[r] : answer[l];
+    row.state->cuts[lane][PIECES] = crowded[r] ? upto[r] : answer[l + 1];
+    row.state->together[lane] = PIECES;  // (linear bins)
     if (lane == 0) row.state->open = 0;
   }
 }
@@ -991,7 +1063,7 @@ __global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __
   constexpr int ROOM = 6144;
   static_assert(ROOM * 2 >= KV_MAX_RANKS * RANK_BINS, "rank_found's bins");
   __shared__ __attribute__((aligned(16))) unsigned long long keys[ROOM];  // what this workgroup finds, [bin][ours]
-  __shared__ Spans s;
+  __shared__ Spans<typename KeyOf<T>::type> s;
   __shared__ Chosen c;
   __shared__ unsigned int found[KV_MAX_RANKS], from[KV_MAX_RANKS];
   __shared__ unsigned long long least[KV_MAX_RANKS], most[KV_MAX_RANKS];
@@ -1000,9 +1072,8 @@ __global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __
   const SplitRow row(work, m);
   const unsigned long long count = row.state->count;
   const int R = count ? 2 * levels.n : 0;
-  if (tid == 0) find_spans<T>(*row.state, levels.n, &s);
   if (tid < KV_MAX_RANKS) { found[tid] = 0; least[tid] = ~0ull; most[tid] = 0; c.id[tid] = -1; }
-  __syncthreads();
+  find_spans<T>(*row.state, levels.n, &s);
   if (wave < R) {  // a wave per rank
     const int span = s.of[wave >> 1];
     const unsigned long long rank = rank_of(levels, wave, count), below = row.state->below[span];
@@ -1021,12 +1092,15 @@ __global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __
     const int u = tid < R && id >= 0 ? __popcll(firsts & ((1ull << first) - 1)) : -1;
     c.bin_of[tid] = u;
     if (u >= 0 && first == tid) {
-      const int span = id / SPAN_BINS, bin = id % SPAN_BINS;
-      const unsigned long long first = bin == 0 ? s.lo[span] : s.from[span] + ((unsigned long long)bin << s.shift[span]);
-      // by what is left up to the interval's end: the bin's own end, as a key, can lie past the last one and come round to zero
-      const unsigned long long left = s.hi[span] - first, below = bin == 0 ? s.from[span] - first : 0, whole = (1ull << s.shift[span]) - 1;
+      const int span = id / SPAN_BINS;
+      const bool in_pieces = pieced(s, levels.n);
+      const int p = id / PIECE_BINS, bins = in_pieces ? PIECE_BINS : SPAN_BINS, bin = id % bins, shift = in_pieces ? s.piece_shift[p] : s.shift[span];
+      const unsigned long long from = in_pieces ? s.base[p] : s.from[span], begin = from + ((unsigned long long)bin << shift);
+      const unsigned long long first = bin > 0 ? begin : in_pieces ? s.search[p] : s.lo[span], end = in_pieces && (p + 1) % PIECES ? s.search[p + 1] - 1 : s.hi[span];
+      // by what is left up to the end of the interval or piece: the bin's own end, as a key, can lie past the last one and come round to zero
+      const unsigned long long whole = (1ull << shift) - 1;
       c.lo[u] = first;
-      c.wide[u] = bin == SPAN_BINS - 1 || left - below < whole ? left : below + whole;
+      c.wide[u] = bin == bins - 1 || end < begin || end - begin <= whole ? end - first : begin - first + whole;
     }
   }
   __syncthreads();

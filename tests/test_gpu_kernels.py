@@ -236,8 +236,9 @@ def _sampled_places(n):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n", [16385, 300_007, 5_000_001])
 def test_quantiles_by_intervals_row_by_row(C, n, dtype):
-    """Which form answers for a row, and that it does so exactly, alone and beside the others: the intervals of a sample; the same again where a bin is crowded (narrow
-    clusters far apart, three of them too, the rank inside one and at its edge); the digits where the sample says nothing true about the row."""
+    """Which form answers for a row, and that it does so exactly, alone and beside the others: the intervals of a sample, by pieces too (narrow clusters far apart,
+    three of them, the rank inside one and at its edge, many samples of the largest value); the passes made again where a bin is crowded all the same; the digits where
+    the sample says nothing true about the row."""
     from kvmini.ops import hist_quantile as hq
 
     rng = np.random.default_rng(n)
@@ -247,7 +248,7 @@ def test_quantiles_by_intervals_row_by_row(C, n, dtype):
     misled = 100 + rng.random(n)
     misled[_sampled_places(n).astype(np.int64)] = rng.random(_sampled_places(n).size)
     rows = {"misled": misled, "normal": g, "sorted": np.sort(g), "few": np.round(g), "halves": np.where(rng.random(n) < 0.5, 10.0, 20.0), "gap": cluster((0.5, 1.0)), "inside": cluster((0.51, 1.0)),
-            "three": cluster((0.499, 0.003, 1.0))}
+            "three": cluster((0.499, 0.003, 1.0)), "capped": np.minimum(g, 24.0), "both": np.clip(g, 11.9, 24.0)}
     x, ps, forms = np.stack(list(rows.values())).astype(dtype), (0.5, 0.95, 0.99), {}
     d = torch.from_numpy(x).to(_dev())
     together = hq.batched_quantiles(d, ps)
@@ -257,9 +258,17 @@ def test_quantiles_by_intervals_row_by_row(C, n, dtype):
         want = [v[int(a)] if a == int(a) else v[int(a)] + (a - int(a)) * (v[int(a) + 1] - v[int(a)]) for a in at]
         assert np.array_equal(together[i], want) and np.array_equal(hq.batched_quantiles(d[i : i + 1], ps)[0], want), (name, together[i], want)
         forms[name] = int(C.quantiles_by_intervals(d[i : i + 1].contiguous(), list(ps))[0])
-    assert forms["misled"] == -1 and all(forms[name] == 1 for name in ("normal", "sorted", "few", "halves")), forms
-    if n > 1_000_000:
-        assert forms["inside"] == 0, forms
+    assert forms.pop("misled") == -1 and forms.pop("three") >= 0 and set(forms.values()) == {1}, forms
+    # the samples that are looked at spread evenly, the others in a bin between them: crowded (the short rows nearly fit)
+    x = 500 + 1e-2 * rng.random(n)
+    x[_sampled_places(n).astype(np.int64)] = 1000 * rng.random(_sampled_places(n).size)
+    d = torch.from_numpy(np.stack((rng.random(n), x)).astype(dtype)[1:]).to(_dev())
+    assert int(C.quantiles_by_intervals(d, [0.5])[0]) == 0 or n < 20_000
+    v, at = np.sort(d[0].cpu().numpy()).astype(np.float64), 0.5 * (n - 1)
+    assert hq.batched_quantiles(d, (0.5,))[0, 0] == v[int(at)] + (at - int(at)) * (v[math.ceil(at)] - v[int(at)])
+    # ... a level in there beside one that needs no more, in a row between others
+    d = torch.from_numpy(np.stack((g, x, np.round(g)))).to(_dev(), torch.float32 if dtype is np.float32 else torch.float64)
+    assert np.array_equal(hq.batched_quantiles(d, (0.0, 0.5, 0.5, 0.51))[1], np.concatenate([hq.batched_quantiles(d[1:2], (p,))[0] for p in (0.0, 0.5, 0.5, 0.51)]))
 
 
 def test_equal_width_histogram_matches_cpu():
