@@ -583,6 +583,7 @@ class ModelRunner:
         variants += [(b, 1) for b, _ in variants if b <= dec_max and b <= max(self.DECODE_FUSED_MAX_ROWS, 256) and hasattr(self.ops, "rope_attention_fused")]
         variants += [(b, 2) for b, k in variants if k == 1 and self.step_kind(b, True, self.rcfg.max_model_len) == 2]
         variants += [(b, 3) for b, k in variants if k == 0 and self.tiles_64]
+        s = None
         for b, dec in variants:
             key = (b, dec)
             if key in self.graphs:
@@ -590,7 +591,9 @@ class ModelRunner:
             if self.tp_active and self.tp_size > 1 and not self.rcfg.tp_rccl_graphs and not (self.xgmi is not None and self.xgmi.fits(b * self.cfg.hidden_size * 2)):
                 continue  # this bucket's all-reduce would be RCCL's: left eager unless asked for (every rank must capture in step)
             # warm-up on a side stream (allocator + lazy init), then capture
-            s = torch.cuda.Stream(self.device)
+            # (kind 3 on the last one's: streams come from a pool in turn, and with how many were taken turns the hardware queue that another engine's
+            # second stream gets; steps on two streams take up to 6 % longer on some than on others)
+            s = torch.cuda.Stream(self.device) if dec != 3 or s is None else s
             s.wait_stream(torch.cuda.current_stream(self.device))
             with torch.cuda.stream(s):
                 for _ in range(2):
