@@ -15,12 +15,7 @@ namespace {
 typedef __attribute__((ext_vector_type(8))) unsigned short bf16x8;  // 16 bytes
 
 __device__ inline float bf2f(unsigned short b) { return __uint_as_float(((unsigned int)b) << 16); }
-__device__ inline unsigned short f2bf(float f) {  // round-to-nearest-even, NaN kept quiet
-  unsigned int u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
-}
+__device__ inline unsigned short f2bf(float f) { return __builtin_bit_cast(unsigned short, (__bf16)f); }  // round to nearest even, NaN kept quiet (hardware conversion)
 // value of lane dpp_ctrl(lane) within the lane's row of 16 (data-parallel primitive: one VALU op)
 template <int CTRL>
 __device__ inline float dpp_f32(float v) {

@@ -55,12 +55,12 @@ struct PanelArgs {
   GroupedRows groups;
 };
 
-__device__ inline unsigned int f2bf(float f) {
-  unsigned int u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40;
-  return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+// round to nearest even, NaN kept quiet (hardware conversion, two at a time)
+__device__ inline unsigned int pack2(float a, float b) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  return __builtin_bit_cast(unsigned int, (bf16x2){(__bf16)a, (__bf16)b});
 }
-__device__ inline uint2 pack4(frag_cd v) { return make_uint2(f2bf(v[0]) | f2bf(v[1]) << 16, f2bf(v[2]) | f2bf(v[3]) << 16); }
+__device__ inline uint2 pack4(frag_cd v) { return make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3])); }
 
 __device__ inline rsrc_t buffer_of(const void* p, unsigned int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00027000); }
 __device__ inline int load4(rsrc_t r, int lane_off, int off) { return __builtin_bit_cast(int, __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, off, 0)); }

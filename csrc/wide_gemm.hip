@@ -79,12 +79,7 @@ constexpr int EPI_GEGLU = 4;  // at the interface: the gated epilogue (EPI_SWIGL
 constexpr int EPI_RELU2 = 5;   // at the interface: bf16 (EPI_BF16), max(y, 0)^2
 constexpr int ACT_RELU2 = 2;   // Params::act of EPI_BF16: max(y, 0)^2
 
-__device__ inline unsigned short f2bf(float f) {
-  unsigned int u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
-}
+__device__ inline unsigned short f2bf(float f) { return __builtin_bit_cast(unsigned short, (__bf16)f); }  // round to nearest even, NaN kept quiet (hardware conversion)
 
 // 8 e4m3 bytes (two dwords) -> 8 bf16, exact
 __device__ inline frag_ab fp8x8_to_bf16(unsigned int lo, unsigned int hi) {

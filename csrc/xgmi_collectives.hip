@@ -51,12 +51,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(8))) unsigned short bf16x8;
 
 __device__ inline float bf2f(unsigned short v) { return __uint_as_float((unsigned int)v << 16); }
-__device__ inline unsigned short f2bf(float f) {
-  unsigned int u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
-}
+__device__ inline unsigned short f2bf(float f) { return __builtin_bit_cast(unsigned short, (__bf16)f); }  // round to nearest even, NaN kept quiet (hardware conversion)
 
 __device__ inline unsigned int* flag_ptr(const Comm& c, int on_rank, int parity, int phase, int from_rank, int wg) {
   return reinterpret_cast<unsigned int*>(c.peer[on_rank] + c.flags_off) + ((long long)((parity * 2 + phase) * MAX_WORLD + from_rank) * c.max_wg + wg);

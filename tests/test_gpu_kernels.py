@@ -1641,6 +1641,26 @@ def test_matrices_of_many_outputs_go_by_panels():
         assert ((got.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2.0**-20 * (x.double().abs() @ w.double().abs().T)).all()
 
 
+@pytest.mark.parametrize("m", [3, 40, 150, 600])  # rows of the streaming kernel (narrow and wide), of narrow tiles, of panels
+def test_outputs_are_rounded_to_the_nearest_even(m):
+    """One product a sum: 16 bits of mantissa, of which bf16 keeps eight (ties in one of 256), and infinities and NaN as they are.  A product is exact in fp32, so
+    every output is the reference's bits."""
+    from kvmini.ops import hip_ops as ops
+
+    torch.manual_seed(m)
+    n, k = 256 * ops._num_cus() if m == 600 else 1024, 256
+    x, w = torch.zeros(m, k), torch.zeros(n, k)
+    x[:, 0] = torch.randn(m).bfloat16() * 2.0 ** torch.randint(-20, 20, (m,))
+    w[:, 0] = torch.randn(n).bfloat16() * 2.0 ** torch.randint(-20, 20, (n,))
+    x[:3, 0] = torch.tensor([float("inf"), float("nan"), -0.0])
+    w[:2, 0] = torch.tensor([3.3e38, -3.3e38]).bfloat16()
+    want = (x[:, :1] * w[:, 0]).bfloat16()
+    rest = torch.isfinite(x[:, 0])  # (elsewhere zero times infinity is no number)
+    got = ops.linear(x.bfloat16().to(_dev()), ops.PackedLinear(w.bfloat16().to(_dev()))).cpu()
+    assert got.shape == want.shape and torch.equal(got[rest], want[rest])
+    assert torch.equal(got[0].isnan(), want[0].isnan()) and torch.equal(got[0, :2], want[0, :2]) and got[1].isnan().all()
+
+
 @pytest.mark.parametrize("bn,variant", [(224, 0), (224, 1), (224, 3), (192, 0), (192, 1), (192, 3)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_tiled_gemm_224_and_192_feature_tiles(C, bn, variant, fp8):
