@@ -17,12 +17,13 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "quantise.h"
+
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) int v8i;
 typedef __attribute__((ext_vector_type(4))) float v4f;
 typedef __attribute__((ext_vector_type(4))) unsigned int raw16;
-typedef __attribute__((ext_vector_type(2))) unsigned int raw8;
 
 template <int FA, int FB>
 __global__ __launch_bounds__(64) void mfma_scale_probe_kernel(const int* __restrict__ a, const int* __restrict__ b, const int* __restrict__ sa, const int* __restrict__ sb,
@@ -39,11 +40,7 @@ __global__ __launch_bounds__(64) void mfma_scale_probe_kernel(const int* __restr
 
 __device__ inline float bf2f(unsigned short b) { return __uint_as_float(((unsigned int)b) << 16); }
 
-// One workgroup (256 threads) per token row.  x: bf16 [M][ldx]; x8: e4m3 [M][K]; scale[t] = absmax / 448
-// (1 for an all-zero row), so x ~= x8 * scale[t].  Inside every group of 64 K-elements the bytes
-// are stored in the order of the packed FP8 weight fragments (kv_pack_weight_fp8): byte 16 q + j
-// holds k = 8 q + j for j < 8 and k = 32 + 8 q + (j - 8) for j >= 8, so that a 16-byte chunk of
-// the row is exactly what lane quarter q of a weight fragment multiplies.
+// One workgroup (256 threads) per token row.  x: bf16 [M][ldx]; x8: e4m3 [M][K]; scale[t] = absmax / 448 (1 for an all-zero row), so x ~= x8 * scale[t].
 template <bool PERMUTE>
 __global__ __launch_bounds__(256) void quantize_rows_fp8_kernel(const unsigned short* __restrict__ x, long long ldx, int K, unsigned char* __restrict__ x8,
                                                                 float* __restrict__ scale) {
@@ -64,31 +61,19 @@ __global__ __launch_bounds__(256) void quantize_rows_fp8_kernel(const unsigned s
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  const float sc = amax > 0.f ? amax * (1.f / 448.f) : 1.f;
+  const float sc = quantise::scale_of(amax);
   const float inv = 1.f / sc;
   if (tid == 0) scale[t] = sc;
-  unsigned char* orow = x8 + (long long)t * K;
   // thread handles 8 consecutive k (one 16-byte load) -> 8 bytes at the permuted position
   for (int i = tid * 8; i < K; i += 256 * 8) {
     const raw16 v = *reinterpret_cast<const raw16*>(row + i);
     float f[8];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      f[2 * j] = bf2f((unsigned short)(v[j] & 0xffffu)) * inv;
-      f[2 * j + 1] = bf2f((unsigned short)(v[j] >> 16)) * inv;
+      f[2 * j] = bf2f((unsigned short)(v[j] & 0xffffu));
+      f[2 * j + 1] = bf2f((unsigned short)(v[j] >> 16));
     }
-    unsigned int lo = 0, hi = 0;
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], lo, false);
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
-    if constexpr (PERMUTE) {
-      const int g = i >> 6, w = i & 63;           // 64-element group, offset inside it (a multiple of 8)
-      const int half = w >> 5, qq = (w & 31) >> 3;  // k = 32 half + 8 qq + j
-      *reinterpret_cast<raw8*>(orow + g * 64 + 16 * qq + 8 * half) = (raw8){lo, hi};
-    } else {
-      *reinterpret_cast<raw8*>(orow + i) = (raw8){lo, hi};  // natural k order (MXFP4 weights: the FP4 operand is in k order)
-    }
+    quantise::store8<PERMUTE>(x8 + (long long)t * K, i, f, inv);
   }
 }
 

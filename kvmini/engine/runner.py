@@ -415,12 +415,14 @@ class ModelRunner:
             plan = None
 
         def pf(wt: Any, site: str) -> Dict[str, Any]:
-            p = plan(wt, t_pad, site) if plan is not None else None
-            return {"prefetch": p} if p is not None else {}
+            if plan is None:
+                return {}
+            p = plan(wt, t_pad, site)
+            return {"prefetch": p} if p is not None else {} if site == "o" else {"ahead": wt}
 
         ahead = pf(w.layers[0].wqkv, "qkv")
         first = getattr(ops, "embed_residual", None)  # the embedding is the first residual stream: its sums of squares come with it
-        start = first(w.embed, tokens, self._dev("feed", t_pad), self.out_ids, cfg.rms_eps) if first is not None and not ahead else None
+        start = first(w.embed, tokens, self._dev("feed", t_pad), self.out_ids, cfg.rms_eps) if first is not None and "prefetch" not in ahead else None
         x = ops.embed_tokens(w.embed, tokens, self._dev("feed", t_pad), self.out_ids) if start is None else None
         if decode_only == 1 and self.decode_layers is not None and t_pad <= 64:
             # plain decoding step: every layer in one persistent launch (phases separated by device-wide

@@ -160,12 +160,21 @@ Weight = Union[torch.Tensor, PackedLinear]
 
 class Normed:
     """Residual stream ``x`` (bf16 ``[T, H]``, NOT normalised) plus the per-row partial
-    sums of squares ``ss`` (``[T, ceil(H/512)]``) from which consumers derive 1/rms."""
+    sums of squares ``ss`` (``[T, ceil(H/512)]``) from which consumers derive 1/rms.
+    ``rows8``: where the update wrote them, ``x`` as e4m3 bytes, the rows' scales, and whether
+    the bytes are in the order of FP8 weight fragments."""
 
-    __slots__ = ("x", "ss", "eps")
+    __slots__ = ("x", "ss", "eps", "rows8")
 
-    def __init__(self, x: torch.Tensor, ss: torch.Tensor, eps: float):
-        self.x, self.ss, self.eps = x, ss, eps
+    def __init__(self, x: torch.Tensor, ss: torch.Tensor, eps: float, rows8: Optional[Tuple[torch.Tensor, torch.Tensor, bool]] = None):
+        self.x, self.ss, self.eps, self.rows8 = x, ss, eps, rows8
+
+
+def _byte_rows(h: Union[torch.Tensor, Normed], x: torch.Tensor, permute: bool) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``x`` (the rows of ``h``) as e4m3 bytes and scales."""
+    if isinstance(h, Normed) and h.rows8 is not None and h.rows8[2] == permute:
+        return h.rows8[:2]
+    return native().quantize_rows_fp8(x, permute)
 
 
 class Partial:
@@ -483,9 +492,9 @@ def _wide(w: Union[PackedLinear, "_ExpandedView"], h: Union[torch.Tensor, "Norme
         x = x.contiguous()
     m = x.shape[0]
     may_split = allow_slabs and epi == 0 and w.n == w.n_pad
-    if FP8_ACTIVATIONS and isinstance(w, PackedLinear) and w.bits == 8 and w.k % 128 == 0:
+    if isinstance(w, PackedLinear) and _multiplies_bytes(w, m):
         # FP8 x FP8: the activations get one dynamic scale per token (1/rms of a folded norm stays in the epilogue)
-        x8, a_scale = C.quantize_rows_fp8(x)
+        x8, a_scale = _byte_rows(h, x, True)
         out = _by_panels(w, x8, epi, ss, eps, may_split, 2, w_scale=w.wscale, x_scale=a_scale) if epi != 5 else None
         if out is not None:
             return out
@@ -525,6 +534,13 @@ def _warn_once(msg: str) -> None:
         warnings.warn(msg, RuntimeWarning, stacklevel=3)
 
 
+def _multiplies_bytes(w: PackedLinear, rows: int) -> bool:
+    """Whether ``rows`` rows meet these weights as e4m3 bytes on the scaled matrix instruction."""
+    if not FP8_ACTIVATIONS or w.bits not in (4, 8) or w.k % 128:
+        return False
+    return rows >= min(STREAM_MAX_M + 1, QUANT_WIDE_FROM) if w.bits == 8 else rows >= min(129, QUANT_WIDE_FROM_FP4) and w.n_pad % 128 == 0
+
+
 def _pad_rows(x: torch.Tensor) -> Tuple[torch.Tensor, int]:
     m = x.shape[0]
     mp = (m + 15) // 16 * 16
@@ -541,7 +557,7 @@ def _stream(w: PackedLinear, h: Union[torch.Tensor, Normed], epi: int, allow_sla
         return _stream_fp4(w, h, epi, allow_slabs)
     if rows > STREAM_MAX_M and w.k % 64 == 0:
         return _wide(w, h, epi, allow_slabs)
-    if rows >= QUANT_WIDE_FROM and w.bits == 8 and FP8_ACTIVATIONS and w.k % 128 == 0:
+    if w.bits == 8 and _multiplies_bytes(w, rows):
         return _wide(w, h, epi, allow_slabs)  # FP8 weights: the scaled-MFMA tiled kernel from this many rows on (see QUANT_WIDE_FROM)
     if 96 < rows <= STREAM_MAX_M and epi in GATED and w.bits == 16 and w.k % 64 == 0 and w.n_pad % 128 == 0 and TILED_GATE_UP_128:
         # the gate/up projection at 97-128 rows on the tiled kernel's 128 x 128 tile (both operands by LDS-DMA).  OFF by
@@ -658,10 +674,10 @@ def _stream_fp4(w: PackedLinear, h: Union[torch.Tensor, Normed], epi: int, allow
     m = x.shape[0]
     n_out = w.n_pad // 2 if epi in GATED else w.n_pad
     n_true = w.n // 2 if epi in GATED else w.n
-    if m >= min(129, QUANT_WIDE_FROM_FP4) and FP8_ACTIVATIONS and w.k % 128 == 0 and w.n_pad % 128 == 0:
+    if _multiplies_bytes(w, m):
         # the tiled kernel reads the MXFP4 weights themselves: FP4 operand + hardware block scales on the scaled
         # MFMA against per-token FP8 activations (no expansion pass, no scratch buffer, any matrix size)
-        x8, a_scale = C.quantize_rows_fp8(x, False)
+        x8, a_scale = _byte_rows(h, x, False)
         may_split = allow_slabs and epi == 0 and w.n == w.n_pad
         out = _by_panels(w, x8, epi, ss, eps, may_split, 3, blocks=w.wscale, x_scale=a_scale) if epi != 5 else None
         if out is not None:
@@ -871,12 +887,13 @@ def linear_residual(x: torch.Tensor, w: Weight, residual: torch.Tensor, eps: flo
 
 
 def add_rmsnorm(x: Union[torch.Tensor, Partial], residual: Optional[torch.Tensor], w: torch.Tensor, eps: float,
-                prefetch: Optional[Tuple[torch.Tensor, list, torch.Tensor]] = None) -> Tuple[Normed, torch.Tensor]:
+                prefetch: Optional[Tuple[torch.Tensor, list, torch.Tensor]] = None, ahead: Optional[Weight] = None) -> Tuple[Normed, torch.Tensor]:
     """Residual update of the folded-norm pipeline.  ``x``: bf16 ``[T, H]`` or a
     :class:`Partial` (split-K slabs of the previous projection); ``residual``: bf16
     ``[T, H]`` updated in place, or None for the first layer.  ``w`` (the gain) must
     already be folded into the consuming projection (:func:`prepare_weights`).
-    ``prefetch``: a :func:`prefetch_plan` for the projection that runs next."""
+    ``prefetch``: a :func:`prefetch_plan` for the projection that runs next; ``ahead``: its
+    weights — where they multiply bytes the rows are quantised in the same launch."""
     C = native()
     if isinstance(x, Partial):
         assert x.ss is None, "slabs that still need a row scale cannot feed a residual add"
@@ -888,6 +905,10 @@ def add_rmsnorm(x: Union[torch.Tensor, Partial], residual: Optional[torch.Tensor
     has_res = residual is not None
     if residual is None:
         residual = torch.empty((t, hdim), dtype=torch.bfloat16, device=src.device)
+    if prefetch is None and isinstance(ahead, PackedLinear) and ahead.k == hdim <= 16384 and _multiplies_bytes(ahead, t):
+        permute = ahead.bits == 8
+        ss, x8, scale = C.residual_quantise(src, residual, has_res, permute)
+        return Normed(residual, ss, eps, (x8, scale, permute)), residual
     ss = C.residual_reduce(src, residual, has_res, *(prefetch or ()))
     return Normed(residual, ss, eps), residual
 

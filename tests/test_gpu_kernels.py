@@ -1641,6 +1641,25 @@ def test_matrices_of_many_outputs_go_by_panels():
         assert ((got.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2.0**-20 * (x.double().abs() @ w.double().abs().T)).all()
 
 
+@pytest.mark.parametrize("T,H,slabs", [(1, 64, 0), (3, 512, 1), (250, 4096, 2), (7, 576, 17), (65, 2048, 0), (5, 4160, 3), (2, 8192, 16), (3, 12288, 0), (2, 16384, 4)])
+def test_residual_and_quantisation_in_one_launch(C, T, H, slabs):
+    """The bits of the two launches: residual, sums of squares, bytes in both orders, scales (rows of zeros and of infinities among them)."""
+    torch.manual_seed(T + H)
+    x = (torch.randn((slabs, T, H) if slabs else (T, H), device="cuda") * 3).to(torch.float32 if slabs else torch.bfloat16)
+    r = (torch.randn(T, H, device="cuda") * 2.0 ** torch.randint(-6, 6, (T, 1), device="cuda")).bfloat16()
+    if T > 2:
+        x[..., 0, :], r[0] = 0, 0
+        r[1, H // 2] = float("inf")
+    for has in (True, False):
+        for permute in (True, False):
+            want, got = r.clone(), r.clone()
+            ss = C.residual_reduce(x, want, has)
+            x8, scale = C.quantize_rows_fp8(want, permute)
+            ss2, y8, scale2 = C.residual_quantise(x, got, has, permute)
+            for a, b in ((got, want), (ss2, ss), (y8, x8), (scale2, scale)):
+                assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
 @pytest.mark.parametrize("m", [3, 40, 150, 600])  # rows of the streaming kernel (narrow and wide), of narrow tiles, of panels
 def test_outputs_are_rounded_to_the_nearest_even(m):
     """One product a sum: 16 bits of mantissa, of which bf16 keeps eight (ties in one of 256), and infinities and NaN as they are.  A product is exact in fp32, so
