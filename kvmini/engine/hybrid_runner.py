@@ -295,7 +295,7 @@ class HybridRunner(ModelRunner):
         logits = ops.linear(hs, w.lm_head)
         if cfg.logit_softcap:
             mx.softcap(logits, cfg.logit_softcap)
-        self.out_ids[: logits.shape[0]].copy_(ops.greedy_sample(logits))
+        ops.greedy_sample(logits, self.out_ids)
         return logits
 
     def _feed_forward(self, la: LayerSpec, lw: HybridLayer, xb: torch.Tensor, st: Any) -> Any:

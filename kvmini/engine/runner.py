@@ -431,7 +431,7 @@ class ModelRunner:
             self.decode_layers.run(residual, h.ss, positions, self.cos, self.sin, slots, bt, tok_seq, ctx, cfg.rms_eps, self.scale)
             hs = ops.select_rows(h, sample_idx[: self.sample_rows(t_pad)])
             logits = ops.linear(hs, w.lm_head)
-            self.out_ids[: logits.shape[0]].copy_(ops.greedy_sample(logits))
+            ops.greedy_sample(logits, self.out_ids)
             return logits
         side = self._side_stream if (decode_only == 1 and plan is not None and hasattr(ops, "prefetch_weight")) else None
         # the first residual add is a copy; h: set when the residual stream and its sums are there already (embedding, fused epilogue)
@@ -485,7 +485,7 @@ class ModelRunner:
             torch.cuda.current_stream().wait_stream(side)
         hs = ops.select_rows(h, sample_idx[: self.sample_rows(t_pad)])
         logits = ops.linear(hs, w.lm_head)
-        self.out_ids[: logits.shape[0]].copy_(ops.greedy_sample(logits))
+        ops.greedy_sample(logits, self.out_ids)
         return logits
 
     def _fused_residual(self, x: torch.Tensor, w: Any, residual: Optional[torch.Tensor]) -> Optional[Tuple[Any, torch.Tensor]]:
@@ -709,7 +709,7 @@ class ModelRunner:
             t_pad, n_samples, max_ctx, cmd, dec, tile_form, dec_split, ids_sync = (int(v) for v in sb.np[o_h : o_h + 8])
             if cmd == 1:
                 return n
-            self.stage_dev.copy_(sb.cpu, non_blocking=True)
+            self._stage_in(sb)
             self._run_staged(t_pad, max_ctx, dec, bool(tile_form & 1), dec_split, tile_form >> 1)
             if ids_sync:
                 self.sync_sampled_ids(n_samples)  # the scheduling rank sampled: take its ids instead of the local argmax
@@ -718,6 +718,14 @@ class ModelRunner:
                     sb.event = torch.cuda.Event()
                 sb.event.record(torch.cuda.current_stream(self.device))
             n += 1
+
+    def _stage_in(self, sb: _Stage) -> None:
+        """The staged image to the device, in stream order."""
+        stage_in = getattr(self.ops, "stage_in", None)
+        if stage_in is not None and self.device.type == "cuda":
+            stage_in(sb.cpu, self.stage_dev)
+        else:
+            self.stage_dev.copy_(sb.cpu, non_blocking=True)
 
     def stop_followers(self) -> None:
         """Scheduling rank: release the followers from :meth:`follow`."""
@@ -912,7 +920,7 @@ class ModelRunner:
             # every rank runs the same step: hand the staged image to the followers first (host
             # shared memory, see follow()), so that they enqueue it while this rank does
             self.channel.publish(st)
-        self.stage_dev.copy_(sb.cpu, non_blocking=True)
+        self._stage_in(sb)
         logits = self._run_staged(t_pad, max_ctx, decode_only, bool(quads), dec_split, pf_split)
         if sampler is not None:
             sampler(logits, self.out_ids)

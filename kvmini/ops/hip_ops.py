@@ -913,6 +913,14 @@ def add_rmsnorm(x: Union[torch.Tensor, Partial], residual: Optional[torch.Tensor
     return Normed(residual, ss, eps), residual
 
 
+def stage_in(src: torch.Tensor, dst: torch.Tensor) -> None:
+    """A step's staged image (int32, pinned) to the device, in stream order: read by a kernel, 15 us a step less than a copy of 73 KB (see there)."""
+    if src.numel() % 2:
+        dst.copy_(src, non_blocking=True)
+    else:
+        native().stage_in(src, dst)
+
+
 def embed_tokens(table: torch.Tensor, tokens: torch.Tensor, feed: torch.Tensor, prev_ids: torch.Tensor) -> torch.Tensor:
     """Embedding lookup with device-side token feed (see ``torch_ops.embed_tokens``): one
     kernel, so a step can be launched before the host has read the previous step's ids."""
@@ -1374,7 +1382,9 @@ def guided_advance(out_ids: torch.Tensor, rows: torch.Tensor, slots: torch.Tenso
     native().guided_advance(out_ids, rows, slots, state, cls, script, cursor)
 
 
-def greedy_sample(logits: torch.Tensor) -> torch.Tensor:
-    out = torch.empty(logits.shape[0], dtype=torch.int64, device=logits.device)
+def greedy_sample(logits: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The first largest logit of every row; ``out`` (int64, at least as many): where they go (as a copy behind it, a launch of 3 to 4 us in a replayed step)."""
+    if out is None:
+        out = torch.empty(logits.shape[0], dtype=torch.int64, device=logits.device)
     (native().argmax_f32 if logits.dtype == torch.float32 else native().argmax)(logits, out)
-    return out
+    return out[: logits.shape[0]]

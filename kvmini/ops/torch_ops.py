@@ -171,8 +171,10 @@ def linear_relu2(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.relu(F.linear(x, w).float()).square().to(x.dtype)
 
 
-def greedy_sample(logits: torch.Tensor) -> torch.Tensor:
-    return logits.argmax(dim=-1)
+def greedy_sample(logits: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The first largest logit of every row; ``out``: where they go."""
+    ids = logits.argmax(dim=-1)
+    return ids if out is None else out[: logits.shape[0]].copy_(ids)
 
 
 def guided_mask(logits: torch.Tensor, rows: torch.Tensor, slots: torch.Tensor, init: torch.Tensor, state: torch.Tensor, cls: torch.Tensor, vc: int,

@@ -1641,6 +1641,20 @@ def test_matrices_of_many_outputs_go_by_panels():
         assert ((got.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2.0**-20 * (x.double().abs() @ w.double().abs().T)).all()
 
 
+@pytest.mark.parametrize("n", [2, 510, 512, 514, 18200, (1 << 19) + 6])
+def test_staged_images_arrive_as_they_are_when_launched(C, n):
+    """One place in host memory, written again for every image: each arrives whole, none of an earlier one is left in a cache."""
+    image, there = torch.zeros(n, dtype=torch.int32).pin_memory(), torch.empty(n + 2, dtype=torch.int32, device="cuda")
+    for i in range(20):
+        image.random_()
+        there.fill_(7)
+        C.stage_in(image, there[:n])
+        got = there.cpu()
+        assert torch.equal(got[:n], image) and (got[n:] == 7).all()
+    with pytest.raises(RuntimeError):
+        C.stage_in(torch.zeros(n, dtype=torch.int32), there[:n])
+
+
 @pytest.mark.parametrize("T,H,slabs", [(1, 64, 0), (3, 512, 1), (250, 4096, 2), (7, 576, 17), (65, 2048, 0), (5, 4160, 3), (2, 8192, 16), (3, 12288, 0), (2, 16384, 4)])
 def test_residual_and_quantisation_in_one_launch(C, T, H, slabs):
     """The bits of the two launches: residual, sums of squares, bytes in both orders, scales (rows of zeros and of infinities among them)."""
