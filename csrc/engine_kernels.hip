@@ -506,7 +506,7 @@ __global__ __launch_bounds__(64) void residual_reduce_kernel(const float* __rest
 // ---------------------------------------------------------------------------------
 // The same update where the next projection multiplies e4m3 rows: a workgroup has a whole row (a wave each segment of 512 columns, P of them in turn),
 // so that the row's largest magnitude is known while the row is still in registers, and its bytes and scale leave with it.  As two launches the
-// second one reads back what the first has just written, and is a dependent launch more: 5.7 + 5.2 us at 245 rows of 4096 with two slabs, together 6.2.
+// second one reads back what the first has just written, and is a dependent launch more: 5.7 + 5.2 us at 245 rows of 4096 with two slabs, together 5.6.
 template <bool SLAB, bool PERMUTE, int P>
 __global__ __launch_bounds__(512) void residual_quantise_kernel(const float* __restrict__ slabs, int n_slabs, long long slab_stride, const unsigned short* __restrict__ x,
                                                                 unsigned short* __restrict__ residual, int has_residual, float* __restrict__ ss_part, int H,

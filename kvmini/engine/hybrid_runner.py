@@ -19,6 +19,7 @@ other reads is held until the join, and the second stream starts every layer beh
 
 from __future__ import annotations
 
+import dataclasses
 from typing import Any, Callable, Dict, List, Optional, Tuple
 
 import numpy as np
@@ -98,6 +99,7 @@ class HybridRunner(ModelRunner):
     def _alloc_cache(self) -> None:
         self.kv_scale = None
         self.decode_layers = None
+        self._row_slots = torch.zeros(self.rcfg.max_batched_tokens, dtype=torch.int32, device=self.device)  # of rows that are all in use
         self.memory = MixerMemory(self.cfg, self.num_blocks, self.block_size, self.rcfg.max_num_seqs, self.dtype, self.device, self._pads)
         # what a branch does, with its weights and memory: one callable (projections, outputs, staged step) per branch of every run
         self.branches: List[List[Callable[..., None]]] = []
@@ -246,26 +248,36 @@ class HybridRunner(ModelRunner):
         elif not gated:
             xb = mx.stream_norm(x, join(runs[0]), w.layers[runs[0].layer].pre, eps, width, dt)
         observed = self._after_layer is not None
+        some = None if observed else self.last_rows(t_pad)
         for ri, run in enumerate(runs):
             la, lw = cfg.layers[run.layer], w.layers[run.layer]
             # behind the run: the norm its successor's input takes (gated: only the head's does) and what the stream takes first
             ahead = runs[ri + 1] if ri + 1 < len(runs) else None
             fin = w.final_norm if ahead is None else None if gated else w.layers[ahead.layer].pre
             jn = None if ahead is None else join(ahead)
+            few = some is not None and ahead is None  # what feeds the last layer's feed-forward, and what comes behind its mixer
+            if few:
+                x, st_ff = mx.select_rows(x, some), dataclasses.replace(st, slots=self._row_slots[: some.numel()])
+                if parallel:
+                    xb2 = mx.select_rows(xb2, some)
+            else:
+                st_ff = st
             if parallel and la.feeds_forward and self.aside is not None:
                 main = torch.cuda.current_stream(self.device)
                 self.aside.wait_stream(main)
                 with torch.cuda.stream(self.aside):
-                    chosen = mx.experts(la.moe, lw.moe, xb2, st, shared=False)
+                    chosen = mx.experts(la.moe, lw.moe, xb2, st_ff, shared=False)
             proj = ops.linear(xb, lw.proj)
             mix = (torch.zeros if lw.out_gaps else torch.empty)((t_pad, lw.out_k), dtype=dt, device=self.device)
             for branch in self.branches[ri]:
                 branch(proj, mix, st)
+            if few:
+                mix = mx.select_rows(mix, some)
             last = not la.feeds_forward
             if parallel:
                 y, y2 = ops.linear(mix, lw.out, allow_slabs=True), None
                 if not last and self.aside is None:
-                    y2 = self._feed_forward(la, lw, xb2, st)
+                    y2 = self._feed_forward(la, lw, xb2, st_ff)
                 elif not last:
                     y2 = mx.with_shared(chosen, la.moe, lw.moe, xb2)
                     main.wait_stream(self.aside)
@@ -277,21 +289,23 @@ class HybridRunner(ModelRunner):
                 done = (mx.all_streams(cfg.streams, self.device), fin) if ahead is None else (w.layers[ahead.layer].hyper.read, fin)
                 xb = mx.hyper_residual(x, ops.linear(mix, lw.out, allow_slabs=True), lw.hyper, *(done if last else (lw.hyper2.read, lw.pre2)), eps, width, dt)
                 if not last:
-                    xb = mx.hyper_residual(x, self._feed_forward(la, lw, xb, st), lw.hyper2, *done, eps, width, dt)
+                    xb = mx.hyper_residual(x, self._feed_forward(la, lw, xb, st_ff), lw.hyper2, *done, eps, width, dt)
                 if observed:
                     self._after_layer(ri, x.sum(1))
                 continue
             gate = proj[:, lw.gate_off : lw.gate_off + cfg.ld] if gated else None
+            if few and gated:
+                gate = mx.select_rows(gate, some)
             xb = mx.gated_residual(x, ops.linear(mix, lw.out, allow_slabs=True), lw.out_bias, gate, lw.gate_bias, lw.norm, cfg.residual_mult, eps, width, dt,
                                    lw.pre2 if not last else None if observed else fin, jn if last and not observed else None)
             if not last:
                 if gated:
                     gate = ops.linear(xb, lw.gate2, allow_slabs=True)
-                xb = mx.gated_residual(x, self._feed_forward(la, lw, xb, st), None, gate, lw.gate2_bias, lw.norm2, cfg.residual_mult, eps, width, dt, None if observed else fin, None if observed else jn)
+                xb = mx.gated_residual(x, self._feed_forward(la, lw, xb, st_ff), None, gate, lw.gate2_bias, lw.norm2, cfg.residual_mult, eps, width, dt, None if observed else fin, None if observed else jn)
             if observed:
                 self._after_layer(ri, x)
                 xb = mx.stream_norm(x, jn, fin, eps, width, dt)
-        hs = mx.select_rows(xb, self._dev("sample_idx", t_pad)[: self.sample_rows(t_pad)])
+        hs = xb if some is not None else mx.select_rows(xb, self._dev("sample_idx", t_pad)[: self.sample_rows(t_pad)])
         logits = ops.linear(hs, w.lm_head)
         if cfg.logit_softcap:
             mx.softcap(logits, cfg.logit_softcap)

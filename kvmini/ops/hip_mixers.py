@@ -14,6 +14,7 @@ from kvmini.models.hybrid import (AttentionSpec, AttentionWeights, DeltaSpec, De
 
 from . import native
 from .hip_ops import PackedLinear, Partial, _num_cus
+from .hip_ops import take_rows as select_rows  # noqa: F401 (part of this module's call surface)
 from .torch_mixers import Join, Step
 
 __all__ = ["Step", "head_pads", "cache_pads", "layout", "embed_stream", "stream_norm", "gated_residual", "all_streams", "split_streams", "hyper_residual", "parallel_residual", "softcap", "attention", "latent_attention", "experts", "shared_expert", "with_shared", "decode_plan", "DeltaState", "Retention", "StateSpace"]
@@ -110,12 +111,6 @@ def _sine_turns(width: int, device: torch.device) -> torch.Tensor:
     f = 10000.0 ** (-2.0 * torch.arange((width + 1) // 2, dtype=torch.float64) / width) / (2 * math.pi)
     hi = f.float()
     return torch.stack((hi, (f - hi.double()).float()), 1).contiguous().to(device)
-
-
-def select_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
-    from .hip_ops import rows_in_pieces
-
-    return native().select_rows(x, None, idx)[0] if rows_in_pieces(x, idx) else torch.index_select(x, 0, idx)
 
 
 def embed_stream(table: torch.Tensor, tokens: torch.Tensor, feed: torch.Tensor, prev_ids: torch.Tensor, ld: int, scale: float = 1.0, positions: Optional[torch.Tensor] = None,

@@ -950,6 +950,15 @@ def rows_in_pieces(x: torch.Tensor, idx: torch.Tensor) -> bool:
             and idx.dtype == torch.int32 and idx.dim() == 1 and idx.is_contiguous())
 
 
+def take_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
+    """Rows ``idx`` of a tensor (fp32 ones as pairs of 16 bits each, which the selection moves as they are)."""
+    if x.dtype == torch.float32 and x.is_contiguous():
+        flat = x.view(x.shape[0], -1)
+        if rows_in_pieces(flat.view(torch.bfloat16), idx):
+            return native().select_rows(flat.view(torch.bfloat16), None, idx)[0].view(torch.float32).view(-1, *x.shape[1:])
+    return native().select_rows(x, None, idx)[0] if rows_in_pieces(x, idx) else torch.index_select(x, 0, idx)
+
+
 def select_rows(h: Normed, idx: torch.Tensor) -> Normed:
     """Rows ``idx``; those outside ``h`` are NaN (indices of other types: ``index_select``, which refuses them)."""
     if not rows_in_pieces(h.x, idx) or not h.ss.is_contiguous():

@@ -50,6 +50,9 @@ def select_rows(h: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
     return torch.index_select(h, 0, idx.long() if h.device.type == "cpu" else idx)
 
 
+take_rows = select_rows  # (norms are applied here: the rows of any tensor)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, allow_slabs: bool = False) -> torch.Tensor:
     """``allow_slabs`` is a hint for the HIP path (split-K partial sums); ignored here."""
     return F.linear(x, w)

@@ -1,0 +1,47 @@
+"""Behind the last layer's attention only the rows go on whose logits are asked for: the same logits and the same memory as with all rows."""
+
+import pytest
+import torch
+
+from kvmini.engine.engine import EngineConfig, LLMEngine
+from kvmini.models import registry
+from kvmini.models.llama import LlamaConfig
+
+LLAMA = LlamaConfig("few-rows", 512, 256, 512, 3, 4, 2, 64, 500000.0, 1e-5, 512, 1, 2)
+BACKENDS = [pytest.param("cpu", torch.float32, False, id="cpu"), pytest.param("cuda:0", torch.float32, False, id="hip-fp32", marks=pytest.mark.gpu),
+            pytest.param("cuda:0", torch.bfloat16, False, id="hip-bf16", marks=pytest.mark.gpu), pytest.param("cuda:0", torch.bfloat16, True, id="hip-bf16-graphs", marks=pytest.mark.gpu)]
+
+
+@pytest.mark.parametrize("design", ["llama", "vodinex-tiny", "pipilix-tiny", "zipelix-tiny", "gebasun-tiny"])
+@pytest.mark.parametrize("device,dtype,graphs", BACKENDS)
+def test_rows_that_nobody_asks_for_end_at_the_last_layer(design, device, dtype, graphs):
+    """A decode row, the end of a prompt and a fresh one, with several rows, one and none asked for.  The selected rows' products are those of fewer rows:
+    fp32 sums in another order, within 2e-5 of the logits' spread; in bf16 a last layer rounded otherwise, within 2 % of it."""
+    if design == "llama" and device != "cpu" and dtype == torch.float32:
+        pytest.skip("this family's kernels are bf16")
+    cfg = LLAMA if design == "llama" else registry.resolve_model(design)[0]
+    weights = registry.random_weights(cfg, device, dtype, seed=1)
+    held, new, want = (40, 30, 0, 3), (1, 25, 70, 20), ([0], [3, 24], [69], [])
+
+    def step(few):
+        eng = LLMEngine(EngineConfig(model=cfg.name, device=device, max_num_seqs=4, max_batched_tokens=256, max_model_len=256, num_blocks=80, use_graphs=False), weights=weights)
+        eng.runner.few_at_last = few
+        seqs = [eng.make_sequence([1 + (i * (j + 3)) % 500 for i in range(h + n)]) for j, (h, n) in enumerate(zip(held, new))]
+        batch = eng.scheduler.schedule_given([(s, h, []) for s, h in zip(seqs, held) if h])
+        eng.runner.execute(batch)
+        eng.scheduler.note_computed(batch)
+        if graphs:
+            eng.runner.rcfg.use_graphs = True
+            eng.runner.capture_graphs([eng.runner.bucket_for(sum(new))])
+            assert eng.runner.graphs
+        assert (eng.runner.last_rows(eng.runner.bucket_for(sum(new))) is not None) == few
+        for _ in range(3 if graphs else 1):
+            logits = eng.runner.execute(eng.scheduler.schedule_given([(s, n, w) for s, n, w in zip(seqs, new, want)]))[1].clone()
+        memory = [eng.runner.kv_cache] if design == "llama" else [t for run in eng.runner.memory.runs for branch in run for t in branch]
+        return logits.double(), memory
+
+    (got, mine), (ref, theirs) = step(True), step(False)
+    assert got.shape == ref.shape == (4, cfg.vocab_size)
+    assert ((got - ref).pow(2).mean(-1).sqrt() / ref.std(-1)).max().item() < (2e-5 if dtype == torch.float32 else 0.02)
+    for a, b in zip(mine, theirs):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
