@@ -718,12 +718,13 @@ struct StateSpaceLayer {
     rows2d(proj, proj.scalar_type(), T, std::max({k.z_off + inner, (int64_t)k.x_off + k.channels, (int64_t)k.dt_off + k.heads}), "projections");
     rows2d(out, proj.scalar_type(), T, k.o_off + inner, "output");
     TORCH_CHECK(ring.scalar_type() == proj.scalar_type(), "state space: the convolution's last inputs have the activations' type");
-    TORCH_CHECK(rows.numel() >= 1 && rows.numel() <= T, "state space: at most one listed row per row");
+    TORCH_CHECK(rows.numel() <= T && rows.numel() + n_chunks >= 1, "state space: at most one listed row per row; rows or chunks");
     a.ldp = proj.stride(0); a.ldo = out.stride(0);
     a.tok_seq = i32p(tok_seq, T, "tok_seq"); a.positions = i32p(positions, T, "positions"); a.tok_kind = i32p(tok_kind, T, "tok_kind"); a.tok_off = i32p(tok_off, T, "tok_off");
     auto fo = proj.options().dtype(at::kFloat);
     Tensor y = at::empty({T, inner}, fo);
-    check(kvs_step(&a, proj.data_ptr(), ring.data_ptr(), (float*)y.data_ptr(), f, i32p(rows, 1, "rows"), (int)rows.numel(), stream()), "state-space step");
+    if (rows.numel() > 0)
+      check(kvs_step(&a, proj.data_ptr(), ring.data_ptr(), (float*)y.data_ptr(), f, i32p(rows, 1, "rows"), (int)rows.numel(), stream()), "state-space step");
     if (n_chunks > 0) {
       TORCH_CHECK(chunks.has_value() && first_chunk.has_value() && segs.dim() == 2 && segs.size(0) == 5 && chunks->dim() == 2 && chunks->size(0) == 4 && n_chunks <= chunks->size(1),
                   "state space: segs [5, n], chunks [4, m]");

@@ -70,6 +70,7 @@ class HybridRunner(ModelRunner):
         self.expands = any(getattr(b, "expand", None) is not None for la in weights.layers for b in la.branches)
         self.retains = any(isinstance(m, (RetentionSpec, StateSpaceSpec)) for m in mixers_)
         self.aside = torch.cuda.Stream(self.device) if self.cfg.wiring == "parallel" and self.device.type == "cuda" and hasattr(mixers, "shared_expert") else None
+        self.rows_apart = self.device.type == "cuda"
         self.span_rows = 0  # rows of the expansion workspace the staged step needs
         self._rot: Dict[Tuple[float, int], Tuple[torch.Tensor, torch.Tensor]] = {}
 
@@ -219,12 +220,13 @@ class HybridRunner(ModelRunner):
     def forward(self, t_pad: int, max_blocks: Optional[int] = None, decode_only: int = 0, quads: bool = False, dec_split: int = 0, pf_split: int = 0) -> torch.Tensor:
         ops, mx, cfg, w = self.ops, self.mixers, self.cfg, self.w
         smax = self.rcfg.max_num_seqs
+        prompts_only, decode_only = decode_only == 4, decode_only if decode_only < 4 else 0
         few = min(smax, t_pad)
         n_blocks = min(self.max_query_blocks, t_pad // self.QUERY_BLOCK + few)
         n_tiles = min(self.max_tiles, t_pad // 16 + min(smax, t_pad // 2))
         st = mx.Step(*(self._dev(k, t_pad) for k in ("tokens", "positions", "slots", "tok_seq", "tok_kind", "tok_off")), self._dev("block_tables").view(smax, self.max_blocks_per_seq),
                      self._dev("singles", few), self._dev("portions").view(5, smax), self._dev("query_blocks").view(4, self.max_query_blocks), n_blocks,
-                     self._dev("tiles").view(4, self.max_tiles), n_tiles, bool(decode_only), decode_only == 2)
+                     self._dev("tiles").view(4, self.max_tiles), n_tiles, bool(decode_only), decode_only == 2, prompts_only=prompts_only)
         if self.expands and not decode_only:
             st.spans, st.latent_blocks = self._dev("spans").view(3, smax), self._dev("latent_blocks").view(4, self.max_latent_blocks)
             st.n_latent_blocks = min(self.max_latent_blocks, t_pad // self.LATENT_BLOCK + min(smax, t_pad // 2))

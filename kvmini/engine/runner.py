@@ -102,6 +102,8 @@ class StepHandle:
 
 
 class ModelRunner:
+    rows_apart: Optional[bool] = None
+
     def __init__(self, weights: LlamaWeights, rcfg: RunnerConfig, tp_group: Any = None):
         self.w = weights
         self.cfg: LlamaConfig = weights.cfg
@@ -186,6 +188,9 @@ class ModelRunner:
         # heads of 64 by tiles: not with quantised weights, whose rows are rounded to e4m3 behind attention: sums in another order move
         # their codes, and results by 4 % of their norm where bf16 weights move 0.6 % (the errors against 64 bits stay: 0.052 and 0.052)
         self.tiles_64 = bool(self.hd == 64 and hasattr(self.ops, "PROMPT_TILES_64_FROM") and getattr(self.w, "quantization", None) is None and self._tiled_ok(self.kv_cache[0, 0]))
+        # prompts by tiles, and a launch beside them for rows that are the only ones of their sequence
+        if self.rows_apart is None:
+            self.rows_apart = self.device.type == "cuda" and self.hd != 64 and self._tiled_ok(self.kv_cache[0, 0])
         # a few prompt tiles deep inside a long context: every tile's key range is shared out over several workgroups
         self.pf_split_ok = bool(hasattr(self.ops, "prefill_attention_split") and self.device.type == "cuda" and self.hd == 128 and self.block_size == 16
                                 and os.environ.get("KVMINI_PREFILL_SPLIT", "1") != "0")
@@ -222,7 +227,8 @@ class ModelRunner:
         self.few_at_last = not self.tp_active and getattr(self.w, "quantization", None) is None
         # (token bucket, step kind) -> (graph, logits); kind 0 = mixed step, 1 = decode-only (fused
         # RoPE + attention kernel), 2 = decode-only with the context split over several workgroups, 3 = mixed without prompt tiles
-        # (tiles_64: the attention kernel by rows alone; kind 0 serves such a step too)
+        # (tiles_64: the attention kernel by rows alone), 4 = prompts alone, without the launches for rows that are the only ones of their sequence
+        # (rows_apart: where those are launches of their own; 4.5 to 15 us a layer).  Kind 0 serves the last two as well.
         self.graphs: Dict[Tuple[int, ...], Any] = {}
         self._graph_pool = None
         # Weight read-ahead on a second stream beside the decode attention kernel (a parallel branch of the
@@ -409,8 +415,8 @@ class ModelRunner:
         the 8-wave attention kernel (see ``tile_quads``).  ``pf_split``: ``shares | tiles << 8`` — the step's first ``tiles`` prompt tiles
         go to the split form of the tile kernel with ``shares`` key ranges each (see ``PF_SPLIT_MAX_TILES``)."""
         ops, cfg, w = self.ops, self.cfg, self.w
-        by_rows = decode_only == 3
-        if by_rows:
+        by_rows, prompts_only = decode_only == 3, decode_only == 4
+        if decode_only >= 3:
             decode_only = 0
         tokens = self._dev("tokens", t_pad)
         positions = self._dev("positions", t_pad)
@@ -474,6 +480,8 @@ class ModelRunner:
                 if dec_split:  # few decode tokens, long contexts: split-KV over the listed rows (padding rows stay zero)
                     a = ops.split_decode_attention(q, kc, vc, bt, tok_seq, self._dev("ctx_decode", t_pad), self._dev("dec_rows", dec_split),
                                                    torch.zeros((t_pad, self.nh * self.hd), dtype=q.dtype, device=q.device), self.scale, **kw)
+                elif prompts_only:  # (padding rows hold anything: nothing is kept of them or asked for)
+                    a = torch.empty((t_pad, self.nh * self.hd), dtype=q.dtype, device=q.device)
                 else:
                     a = ops.paged_attention(q, kc, vc, bt, tok_seq, self._dev("ctx_decode", t_pad), self.scale, max_blocks, **kw)
                 if pf_split:
@@ -599,7 +607,7 @@ class ModelRunner:
         # kernel without the launch of the prompt-tile kernel that the general graph carries — 5.3 us per layer)
         variants += [(b, 1) for b, _ in variants if b <= dec_max and b <= max(self.DECODE_FUSED_MAX_ROWS, 256) and hasattr(self.ops, "rope_attention_fused")]
         variants += [(b, 2) for b, k in variants if k == 1 and self.step_kind(b, True, self.rcfg.max_model_len) == 2]
-        variants += [(b, 3) for b, k in variants if k == 0 and self.tiles_64]
+        variants += [(b, 3 if self.tiles_64 else 4) for b, k in variants if k == 0 and (self.tiles_64 or self.rows_apart)]
         s = None
         for b, dec in variants:
             key = (b, dec)
@@ -610,13 +618,15 @@ class ModelRunner:
             # warm-up on a side stream (allocator + lazy init), then capture
             # (kind 3 on the last one's: streams come from a pool in turn, and with how many were taken turns the hardware queue that another engine's
             # second stream gets; steps on two streams take up to 6 % longer on some than on others)
-            s = torch.cuda.Stream(self.device) if dec != 3 or s is None else s
-            s.wait_stream(torch.cuda.current_stream(self.device))
-            with torch.cuda.stream(s):
-                for _ in range(2):
-                    self.forward(b, decode_only=dec)
-            torch.cuda.current_stream(self.device).wait_stream(s)
-            torch.cuda.synchronize(self.device)
+            # (kind 4: nothing runs there that kind 0 has not run)
+            if dec != 4 or (b, 0) not in self.graphs:
+                s = torch.cuda.Stream(self.device) if dec != 3 or s is None else s
+                s.wait_stream(torch.cuda.current_stream(self.device))
+                with torch.cuda.stream(s):
+                    for _ in range(2):
+                        self.forward(b, decode_only=dec)
+                torch.cuda.current_stream(self.device).wait_stream(s)
+                torch.cuda.synchronize(self.device)
             g = torch.cuda.CUDAGraph()
             # thread_local: other threads of the process (HTTP front-end, RCCL watchdog) may
             # touch the HIP runtime while this thread captures
@@ -660,7 +670,9 @@ class ModelRunner:
         self.graphs[key] = (g, logits)
         return g, logits
 
-    def _run_staged(self, t_pad: int, max_ctx: int, decode_only: int = 0, quads: bool = False, dec_split: int = 0, pf_split: int = 0) -> torch.Tensor:
+    def _run_staged(self, t_pad: int, max_ctx: int, decode_only: int = 0, quads: bool = False, dec_split: int = 0, pf_split: int = 0, prompts_only: bool = False) -> torch.Tensor:
+        if prompts_only:
+            decode_only = 4
         if quads or dec_split or pf_split:
             entry = self._variant_graph(t_pad, quads, dec_split, pf_split)
             self.variant_graph_steps += entry is not None
@@ -725,7 +737,7 @@ class ModelRunner:
             if cmd == 1:
                 return n
             self._stage_in(sb)
-            self._run_staged(t_pad, max_ctx, dec, bool(tile_form & 1), dec_split, tile_form >> 1)
+            self._run_staged(t_pad, max_ctx, dec & 15, bool(tile_form & 1), dec_split, tile_form >> 1, bool(dec >> 4))
             if ids_sync:
                 self.sync_sampled_ids(n_samples)  # the scheduling rank sampled: take its ids instead of the local argmax
             if self.device.type == "cuda":
@@ -924,19 +936,20 @@ class ModelRunner:
             if shares >= 2:
                 pf_split = shares | (pf_tiles << 8)
         pf_split = pf_split or self._step_variant(t_pad, decode_only)
+        prompts_only = bool(self.rows_apart and not decode_only and not quads and not pf_split and not (st[o_cd : o_cd + t] > 0).any())
         # (the header carries the listed rows rounded up to a power of two: fewer rows, more workgroups per context)
         dec_split = 0
         if self.dec_split_ok and not decode_only and 0 < n_dec <= self.DEC_SPLIT_ROWS and dec_max_ctx >= self.DEC_SPLIT_MIN_CTX:
             dec_split = 1 << (n_dec - 1).bit_length()
         st[o_dr + min(n_dec, self.DEC_SPLIT_ROWS) : o_dr + self.DEC_SPLIT_ROWS] = -1
         ids_sync = int(sampler is not None and self.tp_size > 1)  # the followers must take this rank's sampled ids
-        st[o_h : o_h + 8] = (t_pad, n_samples, max_ctx, 0, decode_only, quads | (pf_split << 1), dec_split, ids_sync)
+        st[o_h : o_h + 8] = (t_pad, n_samples, max_ctx, 0, decode_only | prompts_only << 4, quads | (pf_split << 1), dec_split, ids_sync)
         if self.channel is not None:
             # every rank runs the same step: hand the staged image to the followers first (host
             # shared memory, see follow()), so that they enqueue it while this rank does
             self.channel.publish(st)
         self._stage_in(sb)
-        logits = self._run_staged(t_pad, max_ctx, decode_only, bool(quads), dec_split, pf_split)
+        logits = self._run_staged(t_pad, max_ctx, decode_only, bool(quads), dec_split, pf_split, prompts_only)
         if sampler is not None:
             sampler(logits, self.out_ids)
             if ids_sync:
@@ -947,4 +960,4 @@ class ModelRunner:
             if sb.event is None:
                 sb.event = torch.cuda.Event()
             sb.event.record(torch.cuda.current_stream(self.device))
-        return StepHandle(n_samples, logits, sb, (t_pad, decode_only))
+        return StepHandle(n_samples, logits, sb, (t_pad, 4 if prompts_only else decode_only))

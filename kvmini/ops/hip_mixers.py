@@ -211,6 +211,8 @@ def attention(m: AttentionSpec, w: AttentionWeights, scale: float, eps: float, p
         return
     if not st.decode_only:
         C.chunk_prefill(q, kc, vc, st.block_tables, st.blocks, st.n_blocks, proj, w.g_off, gates, mix, w.o_off, m.vdim, *see, m.scale, scale)
+    if st.prompts_only:
+        return
     waves, shares = decode_plan(st.singles.numel(), m.kv_heads * -(-(m.heads // m.kv_heads) // 16), st.long)
     C.chunk_decode(q, proj, w.q_off, w.k_off, w.v_off, w.bias, w.q_norm, w.k_norm, rot[0], rot[1], m.rot_dims, eps, kc, vc, st.block_tables, st.singles, st.tok_seq, st.positions, st.slots,
                    w.g_off, gates, mix, w.o_off, m.heads, m.dim, m.vdim, *see, m.scale, scale, waves, shares)
@@ -252,6 +254,8 @@ def latent_attention(m: LatentSpec, w: LatentWeights, scale: float, eps: float, 
             C.latent_gather(cache, st.spans, st.block_tables, ws)
         C.latent_prefill(proj, w.q_off, w.r_off, w.g_off, each, linear(ws[:, : w.rkp], w.expand), ws[:, w.rkp :] if w.rtp else None, st.latent_blocks, st.n_latent_blocks, mix, w.o_off, m.heads,
                          w.dkp, m.vdim, w.dvp, m.window, m.scale, scale)
+    if st.prompts_only:
+        return
     shares, parts = latent_plan(st.singles.numel(), m.heads, w.dvp, m.window, st.long)
     C.latent_rows(proj, w.q_off, w.r_off, w.c_off, w.kr_off, w.g_off, each, w.absorb, w.up, norm, m.kv_rank, eps, cos, sin, cache, own and st.decode_only, st.decode_only, st.block_tables,
                   st.singles, st.tok_seq, st.positions, st.slots, mix, w.o_off, m.vdim, m.window, m.scale, scale, shares, parts)
@@ -297,7 +301,7 @@ class DeltaState:
 
     def run(self, proj: torch.Tensor, low: torch.Tensor, mix: torch.Tensor, st: Step) -> None:
         per_token = (st.tok_seq, st.positions, st.tok_kind, st.tok_off)
-        if self.has_step:  # the rows that are alone
+        if self.has_step and not st.prompts_only:  # the rows that are alone
             self.impl.step(proj, low, mix, *per_token, st.singles)
             if st.decode_only:
                 return
@@ -313,7 +317,8 @@ class Retention:
 
     def run(self, proj: torch.Tensor, mix: torch.Tensor, st: Step) -> None:
         per_token = (st.tok_seq, st.positions, st.tok_kind)
-        self.impl.step(proj, mix, *per_token, st.singles)  # the rows that are alone
+        if not st.prompts_only:
+            self.impl.step(proj, mix, *per_token, st.singles)  # the rows that are alone
         if not st.decode_only:
             self.impl.portions(proj, mix, *per_token, st.portions, st.chunks, st.n_chunks if self.chunked else 0, st.first_chunk)
 
@@ -324,4 +329,4 @@ class StateSpace:
                                              state, ring)
 
     def run(self, proj: torch.Tensor, mix: torch.Tensor, st: Step) -> None:
-        self.impl.run(proj, mix, st.tok_seq, st.positions, st.tok_kind, st.tok_off, st.singles, st.portions, st.chunks, 0 if st.decode_only else st.n_chunks, st.first_chunk)
+        self.impl.run(proj, mix, st.tok_seq, st.positions, st.tok_kind, st.tok_off, st.singles[:0] if st.prompts_only else st.singles, st.portions, st.chunks, 0 if st.decode_only else st.n_chunks, st.first_chunk)

@@ -43,6 +43,7 @@ class Step:
     chunks: Optional[torch.Tensor] = None  # [4, m]: pieces of at most 64 tokens of portions of several tokens: first row, tokens (0 = unused), first position, sequence slot
     n_chunks: int = 0  # at most that many of them are in use
     first_chunk: Optional[torch.Tensor] = None  # [n]: a portion's first piece
+    prompts_only: bool = False  # no row is the only token of its sequence
 
     @property
     def rows(self) -> int:

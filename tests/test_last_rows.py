@@ -45,3 +45,33 @@ def test_rows_that_nobody_asks_for_end_at_the_last_layer(design, device, dtype, 
     assert ((got - ref).pow(2).mean(-1).sqrt() / ref.std(-1)).max().item() < (2e-5 if dtype == torch.float32 else 0.02)
     for a, b in zip(mine, theirs):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("design", ["llama-128", "llama", "vodinex-tiny", "pipilix-tiny", "zipelix-tiny", "gebasun-tiny"])
+def test_prompts_alone_leave_out_the_launches_for_single_rows(design, graphs):
+    """A step without a row that is the only one of its sequence, and one with such a row: as with those launches, bit for bit."""
+    cfg = LlamaConfig("alone", 512, 512, 512, 2, 4, 2, 128, 500000.0, 1e-5, 512, 1, 2) if design == "llama-128" else LLAMA if design == "llama" else registry.resolve_model(design)[0]
+    weights = registry.random_weights(cfg, "cuda:0", torch.bfloat16, seed=1)
+
+    def steps(apart):
+        eng = LLMEngine(EngineConfig(model=cfg.name, device="cuda:0", max_num_seqs=4, max_batched_tokens=256, max_model_len=256, num_blocks=80, use_graphs=graphs), weights=weights)
+        eng.runner.rows_apart = eng.runner.rows_apart and apart
+        eng.warmup()
+        kinds = []
+        launch = eng.runner.launch
+        eng.runner.launch = lambda *a, **k: (lambda h: (kinds.append(h.key[1]), h)[1])(launch(*a, **k))
+        seqs = [eng.make_sequence([1 + (i * (j + 3)) % 500 for i in range(150)]) for j in range(3)]
+        out = []
+        for part in ((70, 33, 0), (80, 17, 100), (0, 1, 50), (0, 99, 0)):
+            batch = eng.scheduler.schedule_given([(s, n, [0, n - 1]) for s, n in zip(seqs, part) if n > 1] + [(s, n, [0]) for s, n in zip(seqs, part) if n == 1])
+            out.append(eng.runner.execute(batch)[1].clone())
+            eng.scheduler.note_computed(batch)
+        memory = [eng.runner.kv_cache] if "llama" in design else [t for run in eng.runner.memory.runs for branch in run for t in branch]
+        return out + memory, kinds
+
+    (got, kinds), (want, old) = steps(True), steps(False)
+    assert 4 not in old and (kinds == old if design == "llama" else kinds[0] == 4 and kinds[2] == 0)  # (heads of 64 have one launch for both)
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
