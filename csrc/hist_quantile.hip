@@ -547,9 +547,9 @@ __global__ __launch_bounds__(SEL_THREADS) void select_few_kernel(const T* __rest
 // last workgroup to finish ranks them.  Exact whatever the samples are: where an interval misses a rank (4 standard deviations aside: about one
 // call in 5000) the row's count of samples says so and the digits' passes answer for it.  Where a bin of several values holds more than fit all the same
 // (Spans says what is done against that) the count says that the two passes are to be made again, between the least and the most of that bin.
-// Whole calls by digits and so, 3 rows: 33 k floats 54 and 48 us, 1 M 69 and 52, 4 M 88 and 69;
-// 4 M doubles 198 and 79.  Of the 56 us of kernels for 3 x 4 M floats the sample takes 10, the first pass 20 and the second 27, the last workgroup's ranking
-// among them: beside reading (10 us a pass at 5 TB/s) chains of dependent steps, about one us each.
+// Whole calls by digits and so, 3 rows: 33 k floats 54 and 48 us, 1 M 69 and 52, 4 M 88 and 64;
+// 4 M doubles 198 and 79.  Of the 50 us of kernels for 3 x 4 M floats the sample takes 10, the first pass 21 and the second 20, the last workgroup's ranking
+// among them: beside reading (10 us a pass at 5 TB/s) chains of dependent steps, about one us each.  Fewer bins (512, 256) are not faster: their sums are not what counts.
 constexpr int SAMPLE_PARTS = 64;                     // workgroups that rank a row's sample, at most
 constexpr int SPANS = KV_MAX_RANKS / 2;              // intervals: one per level, fewer where they overlap
 constexpr int SPAN_BINS = 1024, SPAN_COPIES = 2;     // LDS: 4 x 1024 x 2 counts, 32 KiB (a lane uses copy lane % 2: values that many samples share)
@@ -585,6 +585,28 @@ struct SplitRow {
     found = (unsigned long long*)(bins + SPANS * SPAN_BINS);
   }
 };
+
+// What the first pass keeps for the second: each wave the samples inside the intervals, up to `room`, and how many there were.  15 % of a row at the usual three
+// levels, so that the second pass reads those and not the row again; a wave that had more goes through its samples again.  Where a workgroup has more than 32 k
+// samples (room -1: nothing is kept): calls of 3 x 4 M floats (47 k) 69.8 -> 64.5 us, the second pass 27 -> 19.6, of 30 M (117 k) 113 -> 99; of 1 x 4 M doubles (16 k) and
+// 3 x 1 M floats (12 k) the same, of a thousand samples 1.4 more (and kernels that know both ways half of that).  Rows of which half is one value: 69 -> 71.
+constexpr int WAVES = SEL_THREADS / 64, MOST_PARTS = 256, SPARE = 32;  // of a workgroup; workgroups per row, at most; of a wave, beside 3 / 16 of its samples
+template <typename T>
+struct Kept {
+  unsigned int* counts;  // [parts][WAVES]
+  T* samples;            // [parts][WAVES][room]
+  int room;
+  __device__ Kept(void* kept, long long row_bytes, int metric, int r) {
+    char* p = (char*)kept + metric * row_bytes;
+    counts = (unsigned int*)p;
+    samples = (T*)(p + MOST_PARTS * WAVES * 4);
+    room = r;
+  }
+  __device__ unsigned int& count(int part, int wave) const { return counts[part * WAVES + wave]; }
+  __device__ T* of(int part, int wave) const { return samples + ((long long)part * WAVES + wave) * room; }
+};
+inline int kept_room(long long n, int parts) { return n / parts > 32768 ? (int)(n * 3 / 16 / (parts * WAVES)) + SPARE : -1; }
+inline long long kept_bytes(long long n, int dtype) { return MOST_PARTS * WAVES * 4 + (n * 3 / 16 + MOST_PARTS * WAVES * SPARE) / 2 * 2 * (dtype == 0 ? 4 : 8); }
 
 // Linear bins of `wide` + 1 keys: key - first >> bin_shift
 template <int BINS>
@@ -785,8 +807,8 @@ __device__ inline uint64_t in_sgpr(uint64_t v) { return (uint64_t)in_sgpr((uint3
 // What bounds it is instructions per sample, not memory: the samples are compared as they are (two instructions per interval, the masks they leave
 // counted by the scalar unit), and those inside queue up per wave, so that the two dozen instructions that bin one run on full waves and not on the five lanes
 // of 64 that have one.  (With each instruction's few lanes on their own the pass over 3 x 4 M floats took 2 us more of its 20.)
-template <typename T, int V, bool PIECED>
-__device__ void split_pass(const T* row, long long n, int part, int parts, const Spans<typename KeyOf<T>::type>& s, T* queue, unsigned int* h, unsigned int* below, unsigned int* valid) {
+template <typename T, int V, bool PIECED, bool KEEP>
+__device__ void split_pass(const T* row, long long n, int part, int parts, const Spans<typename KeyOf<T>::type>& s, T* queue, unsigned int* h, unsigned int* below, unsigned int* valid, const Kept<T>& kept) {
   using KT = typename KeyOf<T>::type;
   constexpr int QUEUE = QUEUE_BYTES / sizeof(T);
   T lo[V], hi[V];
@@ -800,7 +822,9 @@ __device__ void split_pass(const T* row, long long n, int part, int parts, const
     from[i] = in_sgpr((KT)s.from[i]);
     shift[i] = (int)in_sgpr((uint32_t)s.shift[i]);
   }
-  const int copy = threadIdx.x & (SPAN_COPIES - 1), lane = threadIdx.x & 63;
+  const int copy = threadIdx.x & (SPAN_COPIES - 1), lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  T* const mine = kept.of(part, wave);
+  const int room = kept.room;
   unsigned int queued = 0, binned = 0;  // of this wave; the queue is a ring
   auto bin_one = [&](T v) {
     const KT key = KeyOf<T>::key(v);
@@ -842,10 +866,19 @@ __device__ void split_pass(const T* row, long long n, int part, int parts, const
     if (__builtin_amdgcn_inverse_ballot_w64(who)) queue[(queued + __builtin_amdgcn_mbcnt_hi((unsigned int)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)who, 0u))) & (QUEUE - 1)] = v;
     queued += __popcll(who);
   }, [&] {
-    for (; queued - binned >= 64; binned += 64) bin_one(queue[(binned + lane) & (QUEUE - 1)]);
+    for (; queued - binned >= 64; binned += 64) {
+      const T v = queue[(binned + lane) & (QUEUE - 1)];
+      if (KEEP && (int)binned + 64 <= room) mine[binned + lane] = v;
+      bin_one(v);
+    }
   });
-  if (lane < (int)(queued - binned)) bin_one(queue[(binned + lane) & (QUEUE - 1)]);
+  if (lane < (int)(queued - binned)) {
+    const T v = queue[(binned + lane) & (QUEUE - 1)];
+    if (KEEP && (int)binned + lane < room) mine[binned + lane] = v;
+    bin_one(v);
+  }
   if (lane == 0) {
+    if (KEEP) kept.count(part, wave) = queued;
 #pragma unroll
     for (int i = 0; i < V; ++i) atomicAdd(&below[i], under[i]);
     atomicAdd(valid, on);
@@ -855,8 +888,8 @@ __device__ void split_pass(const T* row, long long n, int part, int parts, const
 constexpr int SPLIT_LDS = SPANS * SPAN_BINS * SPAN_COPIES * 4 + SEL_THREADS / 64 * QUEUE_BYTES;
 
 // Grid (workgroups, metrics).
-template <typename T>
-__global__ __launch_bounds__(SEL_THREADS) void select_split_kernel(const T* __restrict__ x, long long n, long long row_stride, int levels, void* work) {
+template <typename T, bool KEEP>
+__global__ __launch_bounds__(SEL_THREADS) void select_split_kernel(const T* __restrict__ x, long long n, long long row_stride, int levels, void* work, void* kept_, long long kept_row, int room) {
   extern __shared__ __attribute__((aligned(16))) unsigned int h[];  // [SPANS][SPAN_BINS][SPAN_COPIES], then the waves' queues
   __shared__ Spans<typename KeyOf<T>::type> s;
   __shared__ unsigned int below[SPANS + 1];
@@ -864,13 +897,14 @@ __global__ __launch_bounds__(SEL_THREADS) void select_split_kernel(const T* __re
   const SplitRow row(work, m);
   for (int i = tid; i < SPANS * SPAN_BINS * SPAN_COPIES; i += SEL_THREADS) h[i] = 0;
   if (tid <= SPANS) below[tid] = 0;
+  const Kept<T> kept(kept_, kept_row, m, room);
   T* queue = reinterpret_cast<T*>(reinterpret_cast<char*>(h + SPANS * SPAN_BINS * SPAN_COPIES) + (tid >> 6) * QUEUE_BYTES);
   find_spans<T>(*row.state, levels, &s);
   const T* xr = x + (long long)m * row_stride;
   const int V = s.n;
   auto pass = [&](auto v) {
-    if (pieced(s, levels)) split_pass<T, decltype(v)::value, true>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
-    else split_pass<T, decltype(v)::value, false>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS);
+    if (pieced(s, levels)) split_pass<T, decltype(v)::value, true, KEEP>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS, kept);
+    else split_pass<T, decltype(v)::value, false, KEEP>(xr, n, blockIdx.x, gridDim.x, s, queue, h, below, below + SPANS, kept);
   };
   if (V <= 1) pass(std::integral_constant<int, 1>{});
   else if (V == 2) pass(std::integral_constant<int, 2>{});
@@ -1057,8 +1091,8 @@ __device__ __forceinline__ void rank_found(const SplitRow& row, const Chosen& c,
 }
 
 // The second pass.  Grid (workgroups, metrics).
-template <typename T>
-__global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __restrict__ x, long long n, long long row_stride, Levels levels, void* work, unsigned long long* out) {
+template <typename T, bool KEEP>
+__global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __restrict__ x, long long n, long long row_stride, Levels levels, void* work, unsigned long long* out, void* kept_, long long kept_row, int room) {
   using KT = typename KeyOf<T>::type;
   constexpr int ROOM = 6144;
   static_assert(ROOM * 2 >= KV_MAX_RANKS * RANK_BINS, "rank_found's bins");
@@ -1104,13 +1138,17 @@ __global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __
     }
   }
   __syncthreads();
+  const Kept<T> kept(kept_, kept_row, m, room);
+  const int our_wave = __builtin_amdgcn_readfirstlane(wave);
+  const unsigned int have = KEEP ? in_sgpr((uint32_t)kept.count(blockIdx.x, our_wave)) : 0;
+  const T* const mine = kept.of(blockIdx.x, our_wave);
   const unsigned int ours = U ? (ROOM / U < FOUND ? ROOM / U : FOUND) : 0;
   auto pass = [&](auto most_bins) {
     constexpr int MOST = decltype(most_bins)::value;
     KT lo[MOST], wide[MOST];
 #pragma unroll
     for (int u = 0; u < MOST; ++u) { lo[u] = in_sgpr((KT)c.lo[u < U ? u : 0]); wide[u] = in_sgpr((KT)c.wide[u < U ? u : 0]); }  // (unused ones repeat the first)
-    for_samples(x + (long long)m * row_stride, n, (long long)blockIdx.x * SEL_THREADS + tid, (long long)gridDim.x * SEL_THREADS, [&](T v) {
+    auto visit = [&](T v) __attribute__((always_inline)) {
       const KT key = key_or_last(v);
       int at = -1;
 #pragma unroll
@@ -1122,7 +1160,19 @@ __global__ __launch_bounds__(SEL_THREADS) void select_collect_kernel(const T* __
       }
       if ((unsigned long long)key < least[at]) atomicMin(&least[at], (unsigned long long)key);
       if ((unsigned long long)key > most[at]) atomicMax(&most[at], (unsigned long long)key);
-    });
+    };
+    if (!KEEP || have > (unsigned int)room) {
+      for_samples(x + (long long)m * row_stride, n, (long long)blockIdx.x * SEL_THREADS + tid, (long long)gridDim.x * SEL_THREADS, visit);
+      return;
+    }
+    constexpr int AT_ONCE = 8;
+    for (unsigned int i = lane; i < have + lane; i += AT_ONCE * 64) {  // (the same for all lanes)
+      T v[AT_ONCE];
+#pragma unroll
+      for (int j = 0; j < AT_ONCE; ++j) v[j] = i + j * 64 < have ? mine[i + j * 64] : (T)__builtin_nanf("");
+#pragma unroll
+      for (int j = 0; j < AT_ONCE; ++j) visit(v[j]);
+    }
   };
   if (U == 1) pass(std::integral_constant<int, 1>{});
   else if (U > 1 && U <= 3) pass(std::integral_constant<int, 3>{});
@@ -1344,7 +1394,7 @@ int select_parts(long long n, int n_metrics, int dtype) {
 }
 
 template <typename T>
-int select_split(const T* x, long long n, long long row_stride, int n_metrics, int dtype, const Levels& lv, void* work, unsigned long long* out, bool again, hipStream_t stream) {
+int select_split(const T* x, long long n, long long row_stride, int n_metrics, int dtype, const Levels& lv, void* work, void* kept, unsigned long long* out, bool again, hipStream_t stream) {
   if (again) {
     hipLaunchKernelGGL(select_again_kernel, dim3(SPANS * SPAN_BINS / SEL_THREADS, n_metrics), dim3(SEL_THREADS), 0, stream, work);
   } else {
@@ -1355,10 +1405,16 @@ int select_split(const T* x, long long n, long long row_stride, int n_metrics, i
     hipLaunchKernelGGL(sample, dim3(parts, n_metrics), dim3(SEL_THREADS), 0, stream, x, n, row_stride, lv, work);
   }
   const dim3 grid(select_parts(n, n_metrics, dtype), n_metrics);
-  static const bool ok = big_lds(select_split_kernel<T>);
+  static const bool ok = big_lds(select_split_kernel<T, true>) && big_lds(select_split_kernel<T, false>);
   if (!ok) return -2;
-  hipLaunchKernelGGL(select_split_kernel<T>, grid, dim3(SEL_THREADS), SPLIT_LDS, stream, x, n, row_stride, lv.n, work);
-  hipLaunchKernelGGL(select_collect_kernel<T>, grid, dim3(SEL_THREADS), 0, stream, x, n, row_stride, lv, work, out);
+  const int room = kept_room(n, grid.x);
+  const long long row = kept_bytes(n, dtype);
+  auto passes = [&](auto keep) {
+    hipLaunchKernelGGL((select_split_kernel<T, decltype(keep)::value>), grid, dim3(SEL_THREADS), SPLIT_LDS, stream, x, n, row_stride, lv.n, work, kept, row, room);
+    hipLaunchKernelGGL((select_collect_kernel<T, decltype(keep)::value>), grid, dim3(SEL_THREADS), 0, stream, x, n, row_stride, lv, work, out, kept, row, room);
+  };
+  if (room >= 0) passes(std::true_type{});
+  else passes(std::false_type{});
   return (int)hipGetLastError();
 }
 
@@ -1442,20 +1498,22 @@ int kv_select_quantiles(const void* x, long long n, long long row_stride, int n_
   return dtype == 0 ? select((const float*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream) : select((const double*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream);
 }
 
-// The same by a sample's intervals, for the rows that kv_split_takes (scratch memory: kv_split_work_bytes): a count of kv_undecided() says that
+// The same by a sample's intervals, for the rows that kv_split_takes (scratch memory: kv_split_work_bytes, and what the passes keep of rows of n samples,
+// kv_split_kept_bytes — enough for calls of fewer rows as well): a count of kv_undecided() says that
 // kv_select_quantiles has to answer, one of kv_crowded() that this has to be called again with what it left in the scratch memory.
 int kv_split_takes(long long n, int n_metrics, int dtype) { return n > (dtype == 0 ? SEL_FEW : SEL_RANKED) && n <= SPLIT_MOST && n_metrics <= 64; }
 long long kv_split_work_bytes(int n_metrics) { return n_metrics * SPLIT_BYTES; }
+long long kv_split_kept_bytes(long long n, int n_metrics, int dtype) { return kept_room(n, select_parts(n, n_metrics, dtype)) < 0 ? 0 : n_metrics * kept_bytes(n, dtype); }
 unsigned long long kv_undecided() { return UNDECIDED; }
 unsigned long long kv_crowded() { return CROWDED; }
 
-int kv_split_quantiles(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const double* ps, int n_ps, void* work, unsigned long long* out, int again, hipStream_t stream) {
+int kv_split_quantiles(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const double* ps, int n_ps, void* work, void* kept, unsigned long long* out, int again, hipStream_t stream) {
   if (n_metrics <= 0 || !kv_split_takes(n, n_metrics, dtype) || n_ps < 1 || n_ps > KV_MAX_RANKS / 2) return -1;
   Levels lv{};
   lv.n = n_ps;
   for (int i = 0; i < n_ps; ++i) lv.p[i] = ps[i];
-  return dtype == 0 ? select_split((const float*)x, n, row_stride, n_metrics, dtype, lv, work, out, again != 0, stream)
-                    : select_split((const double*)x, n, row_stride, n_metrics, dtype, lv, work, out, again != 0, stream);
+  return dtype == 0 ? select_split((const float*)x, n, row_stride, n_metrics, dtype, lv, work, kept, out, again != 0, stream)
+                    : select_split((const double*)x, n, row_stride, n_metrics, dtype, lv, work, kept, out, again != 0, stream);
 }
 
 // The same selection one pass at a time, for samples spread over several ranks: every rank runs

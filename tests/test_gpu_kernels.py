@@ -234,6 +234,29 @@ def _sampled_places(n):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [131_071, 131_073, 140_007])
+def test_quantiles_of_rows_whose_first_pass_keeps_what_is_inside(n, dtype):
+    """64 rows, four workgroups each: below 32 k samples a workgroup nothing is kept, above the waves keep up to 3 / 16 of theirs, and those with more (rows of few values,
+    of one, with the samples inside side by side) go through them again."""
+    from kvmini.ops import hist_quantile as hq
+
+    rng = np.random.default_rng(n)
+    g = 12 * np.exp(0.35 * rng.normal(size=(64, n)))
+    g[1::8] = np.round(g[1::8])
+    g[2::8] = 7.0
+    g[3::8] = np.sort(g[3::8], 1)
+    g[4::8, ::3] = np.nan
+    g[5::8] = np.repeat(g[5::8, : n // 64 + 1], 64, 1)[:, :n]
+    g[6::8] = np.where(rng.random((8, n)) < 0.3, 3.0, g[6::8])
+    x, ps = g.astype(dtype), (0.5, 0.95, 0.99, 0.3)
+    got = hq.batched_quantiles(torch.from_numpy(x).to(_dev()), ps)
+    for row, q in zip(x, got):
+        v = np.sort(row[~np.isnan(row)]).astype(np.float64)
+        at = [p * (v.size - 1) for p in ps]
+        assert np.array_equal(q, [v[int(a)] + (a - int(a)) * (v[math.ceil(a)] - v[int(a)]) for a in at])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n", [16385, 300_007, 5_000_001])
 def test_quantiles_by_intervals_row_by_row(C, n, dtype):
     """Which form answers for a row, and that it does so exactly, alone and beside the others: the intervals of a sample, by pieces too (narrow clusters far apart,
