@@ -17,6 +17,8 @@
 // a portion that starts at position 0 takes S as zero, and inputs before position 0 are zero by their index.
 // Channels are ordered q [kv_heads dim], k [kv_heads dim], v [heads vdim].
 
+#include <type_traits>
+
 #include "elem.h"
 
 namespace {
@@ -346,22 +348,37 @@ __host__ __device__ inline long long tile_floats(int dkp, int dvp) { return 49LL
 
 typedef __attribute__((ext_vector_type(4))) float f4;
 
-// Half of delta_tile_kernel's time is the vector unit's, the rest waits for the loads of its first part and for barriers: what counts is how many workgroups a
-// CU holds.  Partial sums of the pairs with j <= i alone (the 36 blocks of 2 x 2) make that four, of 40 KB, with 128 channels and columns: 2100 tokens
-// of 32 heads 112 us a layer in the profile of a step with three, 100.
+// What counts in delta_tile_kernel is how many workgroups a CU holds, and that none of them waits for long.  Partial sums of the pairs with j < i alone (the
+// 36 blocks of 2 x 2) make that four, of 40 KB, with 128 channels and columns.  All rows that a workgroup reads are on their way before the first is used, a
+// row of 16 tokens is summed by sixteen lanes, and all lanes have pairs with j < i to work out (on the diagonal B is the product of the unit vectors, which
+// their sums give).  4 x 560 tokens of 32 heads, us a layer in the profile of a step: 72 (one column's rows at a time, sums over a wave, 28 lanes of 64
+// idle over the pairs 100); the bytes it writes alone would take 37.
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ inline rsrc_t rows_of(const void* p) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, -1, 0x00027000); }
+template <typename T> __device__ inline T load(rsrc_t from, unsigned lane_off, unsigned off);
+template <> __device__ inline float load<float>(rsrc_t from, unsigned lane_off, unsigned off) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, lane_off, off, 0)); }
+template <> __device__ inline bf16raw load<bf16raw>(rsrc_t from, unsigned lane_off, unsigned off) { return __builtin_amdgcn_raw_buffer_load_b16(from, lane_off, off, 0); }
+// the sum over the sixteen lanes of a row, in each of them
+__device__ inline float row16_sum(float v) {
+  auto turned = [&](auto by) __attribute__((always_inline)) { return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x120 + decltype(by)::value, 0xf, 0xf, true)); };
+  v += turned(std::integral_constant<int, 8>{});
+  v += turned(std::integral_constant<int, 4>{});
+  v += turned(std::integral_constant<int, 2>{});
+  return v + turned(std::integral_constant<int, 1>{});
+}
 // where the pair (i, j) of a tile's rows is kept
 constexpr int PAIRS = 144;
 __device__ inline int pair_of(int i, int j) { return ((i >> 1) * ((i >> 1) + 1) / 2 + (j >> 1)) * 4 + (i & 1) * 2 + (j & 1); }
 
-template <typename T, int TAPS>
+template <typename T, int TAPS, int DKP>
 __global__ __launch_bounds__(256, 4) void delta_tile_kernel(const T* __restrict__ proj, const T* __restrict__ low, const T* __restrict__ ring, float* __restrict__ ws,
                                                          const int* __restrict__ tile_row, const int* __restrict__ tile_n, const int* __restrict__ tile_pos,
-                                                         const int* __restrict__ tile_slot, int dkp, int dvp, DeltaArgs a) {
+                                                         const int* __restrict__ tile_slot, int dvp, DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
+  constexpr int dkp = DKP, rs = DKP + 4;
   const int b = blockIdx.y, h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = tile_n[b];
   if (n == 0) return;
-  const int rs = dkp + 4;
   float* qs = sm;              // [16][rs]
   float* ks = qs + 16 * rs;    // [16][rs]
   float* gs = ks + 16 * rs;    // [16][rs] running log2 decays
@@ -369,141 +386,183 @@ __global__ __launch_bounds__(256, 4) void delta_tile_kernel(const T* __restrict_
   float* pp = vs + 16 * dvp;   // [4 waves][2][PAIRS] partial A, B
   float* am = pp + 8 * PAIRS;  // [16][20] beta_i A_ij
   float* bm = am + 320;        // [16][20]
-  __shared__ float beta[16];
+  __shared__ float beta[16], own[16];  // own: B_ii, a product without a decay
   const long long row0 = tile_row[b];
   const int pos0 = tile_pos[b], slot = tile_slot[b], back0 = a.tok_off[row0];
   const int rep = a.heads / a.kv_heads, g = h / rep, qk = a.kv_heads * a.dim;
-  const int taps = TAPS ? TAPS : a.taps;
-
-  for (int task = tid; task < 3 * dkp + dvp; task += 256) {
-    const int kind = task < 3 * dkp ? task / dkp : 3;  // q, k, decay, v
-    const int d = task - kind * dkp;
-    const int stride = kind == 3 ? dvp : rs;
-    float* dst = (kind == 0 ? qs : kind == 1 ? ks : kind == 2 ? gs : vs) + d;
-    if (d >= (kind == 3 ? a.vdim : a.dim)) {
-      for (int i = 0; i < 16; ++i) dst[i * stride] = 0.f;
-      continue;
+  const float beta_in = ld(proj + (row0 + (tid < n ? tid : 0)) * a.ldp + a.b_off + h);
+  // A task is a column of q, k, the decay inputs or v.  The rows of two are on their way at once, each by as many loads, whatever it is: behind a branch the
+  // first one's would be waited for together with the second's.  A row's place is a scalar, the column a lane's.
+  struct Task { T x[TAPS + 15]; float w[TAPS ? TAPS : 1], bias; int kind, d; bool live; };
+  auto fetch = [&](Task& t, int first) __attribute__((always_inline)) {  // first: of the wave's (sizes are multiples of 64 but for the last kind's)
+    t.kind = first < 3 * dkp ? first / dkp : 3;
+    t.d = first - t.kind * dkp + lane;
+    const bool gate = t.kind == 2;
+    const int most = t.kind == 3 ? a.vdim : a.dim, at = t.d < most ? t.d : most - 1;
+    t.live = t.d < most;
+    const int c = gate ? 0 : t.kind == 0 ? g * a.dim + at : t.kind == 1 ? qk + g * a.dim + at : 2 * qk + h * a.vdim + at;
+    const unsigned col = gate ? a.z_off + h * a.dim + at : chan_col(a, c), ld_bytes = (unsigned)(gate ? a.ldl : a.ldp) * sizeof(T);
+#pragma unroll
+    for (int i = 1 - TAPS; i < 0; ++i) {  // inputs in front of the tile: of the same portion, else from the ring
+      const bool same = -i <= back0 && !gate;
+      const T* from = same ? proj + (row0 + i) * a.ldp : ring + ((long long)slot * TAPS + (pos0 + i >= 0 ? pos0 + i : 0) % TAPS) * a.channels;
+      t.x[i + TAPS - 1] = from[same ? col : (unsigned)c];
     }
-    if (kind == 2) {
-      // (rows past the tile's last one: the last one again; base address per row in scalar registers)
-      const T* zr = low + row0 * a.ldl;
-      const unsigned zc = a.z_off + h * a.dim + d;
-      float z[16], sum = 0.f;
+    const rsrc_t from = rows_of(gate ? low + row0 * a.ldl : proj + row0 * a.ldp);
+    unsigned row = 0;  // (rows past the tile's last one: the last one again)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      t.x[TAPS - 1 + i] = load<T>(from, col * sizeof(T), row);
+      row += i + 1 < n ? ld_bytes : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) t.w[j] = a.conv_w[j * a.channels + c];
+    t.bias = a.dt_bias[h * a.dim + (gate ? at : 0)];
+  };
+  auto finish = [&](const Task& t) __attribute__((always_inline)) {
+    if (t.kind == 3 && t.d >= dvp) return;
+    const int stride = t.kind == 3 ? dvp : rs;
+    float* dst = (t.kind == 0 ? qs : t.kind == 1 ? ks : t.kind == 2 ? gs : vs) + t.d;
+    if (t.kind == 2) {
+      const float rate = -1.4426950408889634f * fast_exp(a.a_log[h]);
+      float sum = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        z[i] = ld(zr + zc);
-        zr += i + 1 < n ? a.ldl : 0;
-      }
-      const float rate = -1.4426950408889634f * fast_exp(a.a_log[h]), bias = a.dt_bias[h * a.dim + d];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float step = rate * softplus(z[i] + bias);
+        const float step = rate * softplus(ld(&t.x[TAPS - 1 + i]) + t.bias);
         sum += i < n ? step : 0.f;
-        dst[i * stride] = sum;
+        dst[i * stride] = t.live ? sum : 0.f;
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
       }
-      continue;
+      return;
     }
-    const int c = kind == 0 ? g * a.dim + d : kind == 1 ? qk + g * a.dim + d : 2 * qk + h * a.vdim + d;
-    if constexpr (TAPS > 0) {
-      const unsigned col = chan_col(a, c);
-      float x[TAPS + 15], w[TAPS];
+    float x[TAPS + 15];
 #pragma unroll
-      for (int j = 0; j < TAPS; ++j) w[j] = a.conv_w[j * a.channels + c];
+    for (int i = 0; i < TAPS + 15; ++i) x[i] = i >= TAPS - 1 || pos0 + i - (TAPS - 1) >= 0 ? ld(&t.x[i]) : 0.f;
 #pragma unroll
-      for (int i = 1 - TAPS; i < 0; ++i) {  // inputs in front of the tile: of the same portion, else from the ring
-        float v;
-        if (-i <= back0) v = ld(proj + (row0 + i) * a.ldp + col);
-        else v = ld(ring + ((long long)slot * TAPS + (pos0 + i >= 0 ? pos0 + i : 0) % TAPS) * a.channels + c);
-        x[i + TAPS - 1] = pos0 + i >= 0 ? v : 0.f;
-      }
-      const T* pr = proj + row0 * a.ldp;
+    for (int i = 0; i < 16; ++i) {
+      float y = 0.f;
 #pragma unroll
+      for (int j = TAPS - 1; j >= 0; --j) y += t.w[j] * x[i + j];
+      y = silu(y);
+      dst[i * stride] = t.live && i < n ? y : 0.f;
+      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  const int tasks = 3 * dkp + dvp;
+  if constexpr (TAPS > 0) {
+    for (int t0 = 64 * __builtin_amdgcn_readfirstlane(wave); t0 < tasks; t0 += 512) {
+      Task one, two;
+      const bool more = t0 + 256 < tasks;
+      fetch(one, t0);
+      fetch(two, more ? t0 + 256 : t0);
+      __builtin_amdgcn_sched_barrier(0);
+      finish(one);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) finish(two);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    for (int task = tid; task < tasks; task += 256) {
+      const int kind = task < 3 * dkp ? task / dkp : 3, d = task - kind * dkp, stride = kind == 3 ? dvp : rs;
+      float* dst = (kind == 0 ? qs : kind == 1 ? ks : kind == 2 ? gs : vs) + d;
+      const bool live = d < (kind == 3 ? a.vdim : a.dim);
+      const int c = kind == 0 ? g * a.dim + d : kind == 1 ? qk + g * a.dim + d : 2 * qk + h * a.vdim + d;
+      float sum = 0.f;
       for (int i = 0; i < 16; ++i) {
-        x[i + TAPS - 1] = ld(pr + col);
-        pr += i + 1 < n ? a.ldp : 0;
+        if (kind == 2 && live && i < n) sum += 1.4426950408889634f * decay_log(a, ld(low + (row0 + i) * a.ldl + a.z_off + h * a.dim + d), h, d);
+        dst[i * stride] = kind == 2 ? sum : live && i < n ? conv_silu<T, 0>(a, proj, ring, row0 + i, pos0 + i, back0 + i, slot, c) : 0.f;
       }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        float y = 0.f;
-#pragma unroll
-        for (int j = TAPS - 1; j >= 0; --j) y += w[j] * x[i + j];
-        y = silu(y);
-        dst[i * stride] = i < n ? y : 0.f;
-      }
-    } else {
-      for (int i = 0; i < 16; ++i) dst[i * stride] = i < n ? conv_silu<T, 0>(a, proj, ring, row0 + i, pos0 + i, back0 + i, slot, c) : 0.f;
     }
   }
-  if (tid < 16) beta[tid] = tid < n ? sigmoid(ld(proj + (row0 + tid) * a.ldp + a.b_off + h)) : 0.f;
-  (void)taps;
+  if (tid < 16) beta[tid] = tid < n ? sigmoid(beta_in) : 0.f;
   __syncthreads();
+  {  // sixteen lanes a row
+    const int i = tid >> 4, d0 = 4 * (tid & 15);
+    float sq = 0.f, sk = 0.f, sb = 0.f;
+    for (int d = d0; d < dkp; d += 64) {
+      const f4 q = *reinterpret_cast<const f4*>(qs + i * rs + d), k = *reinterpret_cast<const f4*>(ks + i * rs + d);
 #pragma unroll
-  for (int i = 4 * wave; i < 4 * wave + 4; ++i) {
-    float sq = 0.f, sk = 0.f;
-    for (int d = lane; d < dkp; d += 64) {
-      sq += qs[i * rs + d] * qs[i * rs + d];
-      sk += ks[i * rs + d] * ks[i * rs + d];
+      for (int e = 0; e < 4; ++e) {
+        sq += q[e] * q[e];
+        sk += k[e] * k[e];
+        sb += q[e] * k[e];
+      }
     }
-    const float nq = 1.f / (sqrtf(wave_sum(sq) + 1e-6f) * sqrtf((float)a.dim)), nk = 1.f / sqrtf(wave_sum(sk) + 1e-6f);
-    for (int d = lane; d < dkp; d += 64) {
-      qs[i * rs + d] *= nq;
-      ks[i * rs + d] *= nk;
+    sq = row16_sum(sq);
+    sk = row16_sum(sk);
+    sb = row16_sum(sb);
+    const float nq = 1.f / (sqrtf(sq + 1e-6f) * sqrtf((float)a.dim)), nk = 1.f / sqrtf(sk + 1e-6f);
+    if (d0 == 0) own[i] = sb * nq * nk;
+    for (int d = d0; d < dkp; d += 64) {
+      *reinterpret_cast<f4*>(qs + i * rs + d) *= nq;
+      *reinterpret_cast<f4*>(ks + i * rs + d) *= nk;
     }
   }
   __syncthreads();
-  {  // partial A, B: a lane has the pairs (2 bi + x, 2 bj + y), a wave a quarter of the channels
-    const int bi = lane >> 3, bj = lane & 7;
-    if (bi >= bj) {
-      float pa[2][2] = {{0.f, 0.f}, {0.f, 0.f}}, pb[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-      const int d1 = (wave + 1) * (dkp >> 2);
-      for (int d = wave * (dkp >> 2); d < d1; d += 4) {
-        f4 ki[2], qi[2], gi[2], kj[2], gj[2];
+  {  // partial A, B: a wave has a quarter of the channels, two lanes every other four of them for the pairs (2 bi + x, 2 bj + y), bi > bj; a lane on
+     // the diagonal, where only (2 bi + 1, 2 bi) is left, has that pair twice, and (x, x) of its products count
+    const int bi = lane >> 3, bj = lane & 7, hi = bi > bj ? bi : bj, lo = bi > bj ? bj : bi, quarter = dkp >> 2;
+    int oi[2], oj[2];
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-          const int oi = (2 * bi + x) * rs + d, oj = (2 * bj + x) * rs + d;
-          ki[x] = *reinterpret_cast<const f4*>(ks + oi);
-          qi[x] = *reinterpret_cast<const f4*>(qs + oi);
-          gi[x] = *reinterpret_cast<const f4*>(gs + oi);
-          kj[x] = *reinterpret_cast<const f4*>(ks + oj);
-          gj[x] = *reinterpret_cast<const f4*>(gs + oj);
-        }
+    for (int x = 0; x < 2; ++x) {
+      oi[x] = (2 * hi + (hi == lo ? 1 : x)) * rs + wave * quarter + (hi == lo ? 4 * x : bi < bj ? 4 : 0);
+      oj[x] = (2 * lo + (hi == lo ? 0 : x)) * rs + wave * quarter + (hi == lo ? 4 * x : bi < bj ? 4 : 0);
+    }
+    float pa[2][2] = {{0.f, 0.f}, {0.f, 0.f}}, pb[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+#pragma unroll 1
+    for (int d = 0; d < quarter; d += 8) {
+      f4 ki[2], qi[2], gi[2], kj[2], gj[2];
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-          for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float w = kj[y][e] * __builtin_amdgcn_exp2f(gi[x][e] - gj[y][e]);  // (i < j, on the diagonal blocks: may overflow, not used)
-              pa[x][y] += ki[x][e] * w;
-              pb[x][y] += qi[x][e] * w;
-            }
+      for (int x = 0; x < 2; ++x) {
+        ki[x] = *reinterpret_cast<const f4*>(ks + oi[x] + d);
+        qi[x] = *reinterpret_cast<const f4*>(qs + oi[x] + d);
+        gi[x] = *reinterpret_cast<const f4*>(gs + oi[x] + d);
+        kj[x] = *reinterpret_cast<const f4*>(ks + oj[x] + d);
+        gj[x] = *reinterpret_cast<const f4*>(gs + oj[x] + d);
       }
 #pragma unroll
       for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) {
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float w = kj[y][e] * __builtin_amdgcn_exp2f(gi[x][e] - gj[y][e]);  // (on the diagonal, x != y: may overflow, not used)
+            pa[x][y] += ki[x][e] * w;
+            pb[x][y] += qi[x][e] * w;
+          }
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        const float oa = __shfl(pa[x][y], 8 * bj + bi), ob = __shfl(pb[x][y], 8 * bj + bi);
+        if (bi > bj) {
           const int i = pair_of(2 * bi + x, 2 * bj + y);
-          pp[wave * 2 * PAIRS + i] = pa[x][y];
-          pp[(wave * 2 + 1) * PAIRS + i] = pb[x][y];
+          pp[wave * 2 * PAIRS + i] = pa[x][y] + oa;
+          pp[(wave * 2 + 1) * PAIRS + i] = pb[x][y] + ob;
         }
+      }
+    if (bi == bj) {
+      const int i = pair_of(2 * bi + 1, 2 * bi);
+      pp[wave * 2 * PAIRS + i] = pa[0][0] + pa[1][1];
+      pp[(wave * 2 + 1) * PAIRS + i] = pb[0][0] + pb[1][1];
     }
   }
   __syncthreads();
   {
     const int i = tid >> 4, j = tid & 15;
-    const float* p = pp + (j <= i ? pair_of(i, j) : 0);
+    const float* p = pp + (j < i ? pair_of(i, j) : 2);  // (2: the pair (1, 0))
     am[i * 20 + j] = j < i ? beta[i] * (p[0] + p[2 * PAIRS] + p[4 * PAIRS] + p[6 * PAIRS]) : 0.f;
-    bm[i * 20 + j] = j <= i ? p[PAIRS] + p[3 * PAIRS] + p[5 * PAIRS] + p[7 * PAIRS] : 0.f;
+    bm[i * 20 + j] = j < i ? p[PAIRS] + p[3 * PAIRS] + p[5 * PAIRS] + p[7 * PAIRS] : j == i ? own[i] : 0.f;
   }
   __syncthreads();
   float* w = ws + ((long long)b * a.heads + h) * tile_floats(dkp, dvp);
-  float* tk = w;
-  float* qe = tk + 16 * dkp;
-  float* ke = qe + 16 * dkp;
+  float* ke = w + 32 * dkp;
   float* gc = ke + 16 * dkp;
-  float* tv = gc + dkp;
-  float* ov = tv + 16 * dvp;
-  for (int c = tid; c < dkp + dvp; c += 256) {
+  const rsrc_t wr = rows_of(w);
+  for (int c0 = tid; c0 < dkp + dvp; c0 += 256) {
+    int c = c0;
+    asm volatile("" : "+v"(c));  // (the rows' places are worked out where they are needed and not in front of the loop, where they would fill the registers)
     const bool is_k = c < dkp;
     float x[16], y[16];
     if (is_k) {
@@ -515,6 +574,7 @@ __global__ __launch_bounds__(256, 4) void delta_tile_kernel(const T* __restrict_
         x[i] = kk * eg;
         y[i] = qs[i * rs + c] * eg;
         kv[i >> 2][i & 3] = kk * __builtin_amdgcn_exp2f(gl - gg);
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) *reinterpret_cast<f4*>(ke + c * 16 + 4 * i) = kv[i];
@@ -546,13 +606,11 @@ __global__ __launch_bounds__(256, 4) void delta_tile_kernel(const T* __restrict_
       y[i] += sgn * r;
       asm volatile("" ::: "memory");  // (a row's coefficients are read when they are needed: all of them at once would fill the registers)
     }
-    float* d0 = is_k ? tk + c : tv + c - dkp;
-    float* d1 = is_k ? qe + c : ov + c - dkp;
-    const int st = is_k ? dkp : dvp;
+    const unsigned row = (__builtin_amdgcn_readfirstlane(c) < dkp ? dkp : dvp) * 4, at = (is_k ? c : 48 * dkp + c) * 4;  // (a wave has keys or values)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      d0[i * st] = x[i];
-      d1[i * st] = y[i];
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[i]), wr, at, i * row, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[i]), wr, at, (16 + i) * row, 0);
     }
   }
 }
@@ -830,19 +888,25 @@ int kvd_tiles(const KvdArgs* k, const void* proj, const void* low, void* ring, i
   if (lds > 160 * 1024 - 256) return -1;
   const int *tr = tiles, *tn = tiles + tile_stride, *tp = tiles + 2 * tile_stride, *ts = tiles + 3 * tile_stride;
   const int *row = segs, *n = segs + n_segs, *pos = segs + 2 * n_segs, *slot = segs + 3 * n_segs, *first = segs + 4 * n_segs;
-#define KV_TI(Tt, TP)                                                                                                                                             \
-  do {                                                                                                                                                            \
-    if (lds > 65536 && hipFuncSetAttribute((const void*)delta_tile_kernel<Tt, TP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1; \
-    hipLaunchKernelGGL((delta_tile_kernel<Tt, TP>), dim3(a.heads, n_tiles), dim3(256), lds, s, (const Tt*)proj, (const Tt*)low, (const Tt*)ring, ws, tr, tn, tp, ts, dkp, dvp, a); \
-  } while (0)
-#define KV_TI2(TP) do { if (f32) KV_TI(float, TP); else KV_TI(bf16raw, TP); } while (0)
-  if (a.taps == 4) KV_TI2(4);
-  else if (a.taps == 3) KV_TI2(3);
-  else if (a.taps == 2) KV_TI2(2);
-  else KV_TI2(0);
-#undef KV_TI2
-#undef KV_TI
-  int rc = (int)hipGetLastError();
+  auto tiles_of = [&](auto of, auto taps, auto keys) {
+    using Row = decltype(of);
+    constexpr auto kernel = delta_tile_kernel<Row, decltype(taps)::value, decltype(keys)::value>;
+    if (lds > 65536 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1;
+    hipLaunchKernelGGL(kernel, dim3(a.heads, n_tiles), dim3(256), lds, s, (const Row*)proj, (const Row*)low, (const Row*)ring, ws, tr, tn, tp, ts, dvp, a);
+    return (int)hipGetLastError();
+  };
+  auto of_keys = [&](auto of, auto taps) {
+    return dkp == 64 ? tiles_of(of, taps, std::integral_constant<int, 64>{}) : dkp == 128 ? tiles_of(of, taps, std::integral_constant<int, 128>{}) : tiles_of(of, taps, std::integral_constant<int, 256>{});
+  };
+  auto of_taps = [&](auto of) {
+    switch (a.taps) {
+      case 4: return of_keys(of, std::integral_constant<int, 4>{});
+      case 3: return of_keys(of, std::integral_constant<int, 3>{});
+      case 2: return of_keys(of, std::integral_constant<int, 2>{});
+      default: return of_keys(of, std::integral_constant<int, 0>{});
+    }
+  };
+  const int rc = f32 ? of_taps(float{}) : of_taps(bf16raw{});
   if (rc) return rc;
   const dim3 grid(a.heads, dvp / 16, n_segs);
 #define KV_CH(Tt, RT, WGS) hipLaunchKernelGGL((delta_chain_kernel<Tt, RT, WGS>), grid, dim3(256), 0, s, ws, o, (const Tt*)proj, (Tt*)ring, row, n, pos, slot, first, min_n, dkp, dvp, a)
