@@ -343,7 +343,8 @@ __global__ __launch_bounds__(256) void conv_tail_kernel(const T* __restrict__ pr
 // delta_tile_kernel solves the triangular part of a tile for all columns at once (forward substitution on [kb | v]), in parallel
 // over tiles and heads:  u = tv - tk S,  o = ov + qe S,  with ke_j = k_j e^{G_15 - G_j}.  delta_chain_kernel then walks the tiles
 // of a portion with S in matrix-core accumulators (fp32 in and out): two products and one update per tile.
-// Workspace of a (tile, head): tk [16][dkp], qe [16][dkp], ke [dkp][16], gc [dkp], tv [16][dvp], ov [16][dvp].
+// Workspace of a (tile, head), in the order in which the lanes of the chain read it, 16 bytes each: tk and qe [dkp / 4][16 tokens][4 channels],
+// ke [dkp / 16][4][16 channels][4 tokens], gc [dkp], tv and ov [4][dvp][4 tokens].
 __host__ __device__ inline long long tile_floats(int dkp, int dvp) { return 49LL * dkp + 32LL * dvp; }
 
 typedef __attribute__((ext_vector_type(4))) float f4;
@@ -557,36 +558,7 @@ __global__ __launch_bounds__(256, 4) void delta_tile_kernel(const T* __restrict_
   }
   __syncthreads();
   float* w = ws + ((long long)b * a.heads + h) * tile_floats(dkp, dvp);
-  float* ke = w + 32 * dkp;
-  float* gc = ke + 16 * dkp;
-  const rsrc_t wr = rows_of(w);
-  for (int c0 = tid; c0 < dkp + dvp; c0 += 256) {
-    int c = c0;
-    asm volatile("" : "+v"(c));  // (the rows' places are worked out where they are needed and not in front of the loop, where they would fill the registers)
-    const bool is_k = c < dkp;
-    float x[16], y[16];
-    if (is_k) {
-      const float gl = gs[15 * rs + c];
-      f4 kv[4];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float gg = gs[i * rs + c], kk = ks[i * rs + c], eg = __builtin_amdgcn_exp2f(gg);
-        x[i] = kk * eg;
-        y[i] = qs[i * rs + c] * eg;
-        kv[i >> 2][i & 3] = kk * __builtin_amdgcn_exp2f(gl - gg);
-        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<f4*>(ke + c * 16 + 4 * i) = kv[i];
-      gc[c] = __builtin_amdgcn_exp2f(gl);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        x[i] = vs[i * dvp + c - dkp];
-        y[i] = 0.f;
-      }
-    }
-    const float sgn = is_k ? -1.f : 1.f;
+  auto solve = [&](float (&x)[16], float (&y)[16], float sgn) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       f4 ar[4], br[4];
@@ -606,12 +578,56 @@ __global__ __launch_bounds__(256, 4) void delta_tile_kernel(const T* __restrict_
       y[i] += sgn * r;
       asm volatile("" ::: "memory");  // (a row's coefficients are read when they are needed: all of them at once would fill the registers)
     }
-    const unsigned row = (__builtin_amdgcn_readfirstlane(c) < dkp ? dkp : dvp) * 4, at = (is_k ? c : 48 * dkp + c) * 4;  // (a wave has keys or values)
+  };
+  {  // keys: their columns go back to where the rows of q and k were, and from there to memory
+    float x[16], y[16];
+    if (tid < dkp) {
+      const int c = tid;
+      const float gl = gs[15 * rs + c];
+      f4 kv[4];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float gg = gs[i * rs + c], kk = ks[i * rs + c], eg = __builtin_amdgcn_exp2f(gg);
+        x[i] = kk * eg;
+        y[i] = qs[i * rs + c] * eg;
+        kv[i >> 2][i & 3] = kk * __builtin_amdgcn_exp2f(gl - gg);
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<f4*>(w + 32 * dkp + (c >> 4) * 256 + i * 64 + (c & 15) * 4) = kv[i];
+      w[48 * dkp + c] = __builtin_amdgcn_exp2f(gl);
+    }
+    __syncthreads();
+    if (tid < dkp) {
+      solve(x, y, -1.f);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        qs[i * rs + tid] = x[i];
+        ks[i * rs + tid] = y[i];
+      }
+    }
+  }
+  for (int c0 = tid + (tid < dkp ? 256 : 0) - dkp; c0 < dvp; c0 += 256) {
+    int c = c0;
+    asm volatile("" : "+v"(c));  // (the rows' places are worked out where they are needed and not in front of the loop, where they would fill the registers)
+    float x[16], y[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[i]), wr, at, i * row, 0);
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[i]), wr, at, (16 + i) * row, 0);
+      x[i] = vs[i * dvp + c];
+      y[i] = 0.f;
     }
+    solve(x, y, 1.f);
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+      *reinterpret_cast<f4*>(w + 49 * dkp + (i * dvp + 4 * c)) = (f4){x[i], x[i + 1], x[i + 2], x[i + 3]};
+      *reinterpret_cast<f4*>(w + 49 * dkp + ((16 + i) * dvp + 4 * c)) = (f4){y[i], y[i + 1], y[i + 2], y[i + 3]};
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = tid; j < 8 * dkp; j += 256) {
+    const int piece = j % (4 * dkp);
+    *reinterpret_cast<f4*>(w + 4 * j) = *reinterpret_cast<const f4*>((j < 4 * dkp ? qs : ks) + (piece & 15) * rs + (piece >> 4) * 4);
   }
 }
 
@@ -648,38 +664,35 @@ __device__ __attribute__((always_inline)) inline void delta_chain(f4* lds, int y
   // two tiles in flight: a tile's coefficients come from beyond this XCD's L2 the first time, and one tile takes less time than that
   struct Tile { f4 tk[RT], qe[RT], ke[RT], gc[RT], tv[CT]; float ov[CT]; };
   Tile ta, tb;
-  const unsigned int at_row = (lr * dkp + base + 4 * lq) * 4, at_ke = ((base + lr) * 16 + 4 * lq) * 4, at_gc = (base + 4 * lq) * 4, at_col = (4 * lq * dvp + col) * 4;
+  const unsigned int at_row = base * 64 + lane * 16, at_gc = (base + 4 * lq) * 4, at_col = (lq * dvp + col) * 16;
   auto fetch = [&](Tile& x, int i) __attribute__((always_inline)) {
     const float* p = w + step * (i < nt ? i : nt - 1);
     if constexpr (LEAN) {
       auto at = [](const float* from, unsigned int off) __attribute__((always_inline)) { return reinterpret_cast<const char*>(from) + off; };
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
-        x.tk[t] = *reinterpret_cast<const f4*>(at(p, at_row) + 64 * t);
-        x.qe[t] = *reinterpret_cast<const f4*>(at(p + 16 * dkp, at_row) + 64 * t);
-        x.ke[t] = *reinterpret_cast<const f4*>(at(p + 32 * dkp, at_ke) + 1024 * t);
+        x.tk[t] = *reinterpret_cast<const f4*>(at(p, at_row) + 1024 * t);
+        x.qe[t] = *reinterpret_cast<const f4*>(at(p + 16 * dkp, at_row) + 1024 * t);
+        x.ke[t] = *reinterpret_cast<const f4*>(at(p + 32 * dkp, at_row) + 1024 * t);
         x.gc[t] = *reinterpret_cast<const f4*>(at(p + 48 * dkp, at_gc) + 64 * t);
       }
 #pragma unroll
       for (int c = 0; c < CT; ++c) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x.tv[c][r] = *reinterpret_cast<const float*>(at(p + 49 * dkp + r * dvp, at_col) + 64 * c);
-        x.ov[c] = *reinterpret_cast<const float*>(at(p + 49 * dkp + (16 + wave) * dvp, at_col) + 64 * c);
+        x.tv[c] = *reinterpret_cast<const f4*>(at(p + 49 * dkp, at_col) + 256 * c);
+        x.ov[c] = *reinterpret_cast<const float*>(at(p + 49 * dkp + 16 * dvp + wave, at_col) + 256 * c);
       }
     } else {
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
-        const int d = base + 16 * t;
-        x.tk[t] = *reinterpret_cast<const f4*>(p + lr * dkp + d + 4 * lq);
-        x.qe[t] = *reinterpret_cast<const f4*>(p + (16 + lr) * dkp + d + 4 * lq);
-        x.ke[t] = *reinterpret_cast<const f4*>(p + 32 * dkp + (d + lr) * 16 + 4 * lq);
-        x.gc[t] = *reinterpret_cast<const f4*>(p + 48 * dkp + d + 4 * lq);
+        x.tk[t] = *reinterpret_cast<const f4*>(p + (base + 16 * t) * 16 + 4 * lane);
+        x.qe[t] = *reinterpret_cast<const f4*>(p + (dkp + base + 16 * t) * 16 + 4 * lane);
+        x.ke[t] = *reinterpret_cast<const f4*>(p + (2 * dkp + base + 16 * t) * 16 + 4 * lane);
+        x.gc[t] = *reinterpret_cast<const f4*>(p + 48 * dkp + base + 16 * t + 4 * lq);
       }
 #pragma unroll
       for (int c = 0; c < CT; ++c) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x.tv[c][r] = p[49 * dkp + (4 * lq + r) * dvp + col + 16 * c];
-        x.ov[c] = p[49 * dkp + (16 + 4 * lq + wave) * dvp + col + 16 * c];
+        x.tv[c] = *reinterpret_cast<const f4*>(p + 49 * dkp + (lq * dvp + col + 16 * c) * 4);
+        x.ov[c] = p[49 * dkp + ((4 + lq) * dvp + col + 16 * c) * 4 + wave];
       }
     }
     __builtin_amdgcn_sched_barrier(0);  // the loads are issued here and not where they are used
@@ -758,6 +771,9 @@ __device__ __attribute__((always_inline)) inline void delta_chain(f4* lds, int y
   }
 }
 
+// Sixteen lanes of a load read 256 bytes in a row: as rows of tokens the coefficients were sixteen places, and the loads took a quarter of the time (us a layer,
+// rows and now: 4 x 560 tokens of 32 heads 97 and 87, all of the delta rule for 1 x 2048 218 and 201, 64 x 20 246 and 226, 16 heads of 256 channels 4 x 300 131
+// and 115; without any loads the first takes 81).  The figures below are from before.
 // grid (heads, dvp / 16, portions).  What bounds a tile's step is what is read of it (25 KB for 128 key channels and 16 columns, from beyond the L2) and
 // the fp32 matrix instructions (0.35 us); its serial chain is about as long.  Two column tiles a workgroup read half as much and leave half the
 // workgroups.  Measured for 128 x 128, us of a layer's launches for portions, one tile a workgroup and two: 32 heads, 4 x 512 tokens 225, 204; 16 x 128
