@@ -651,8 +651,10 @@ int dispatch_tile(int bm, int bn, int variant, int epi, const Params& p, hipStre
     // 128 x 256, 8 waves (wave: 64 x 64)
     case 1282560: return dispatch_epi<128, 256, 2, 4, 2, 3, WQ>(epi, p, s);
     case 1282562: return dispatch_epi<128, 256, 2, 4, 2, 2, WQ>(epi, p, s);
-    // 128 x 128, 4 waves (wave: 64 x 64); two workgroups per CU with two stages
-    case 1281280: return dispatch_epi<128, 128, 2, 2, 2, 4, WQ>(epi, p, s);
+    // 128 x 128: with bf16 weights 8 waves (wave: 32 tokens x 64 features), two on a SIMD, of which one multiplies while the other waits at a stage's barrier;
+    // they read half as much LDS again.  2048 x 2048 at K = 2048, 2816 and 8192: 25.5, 33.1 and 80.7 us by 4 waves (64 x 64), 23.5, 31.0 and 74.2 (64 x 32 a wave: 23.9,
+    // 30.8, 76.4).  Others 4; two workgroups per CU with two stages
+    case 1281280: return dispatch_epi<128, 128, WQ == 0 ? 4 : 2, 2, 2, 4, WQ>(epi, p, s);
     case 1281282: return dispatch_epi<128, 128, 2, 2, 2, 2, WQ>(epi, p, s);
   }
   if constexpr (WQ != 3) switch (key * 10 + variant) {
