@@ -170,6 +170,9 @@ class HybridRunner(ModelRunner):
         st[o_k + t : o_k + t_pad] = 0
         st[o_o + t : o_o + t_pad] = 0
 
+    def _rows_alone(self, st: np.ndarray, portions: List[Tuple[int, int, int, int]], t: int) -> bool:
+        return any(n == 1 for _row, n, _pos, _slot in portions)  # what `singles` lists, a chunk of drafts that was cut to one token among them
+
     def _stage_spans(self, st: np.ndarray, portions: List[Tuple[int, int, int, int]]) -> None:
         """Where the keys of the step's prompt portions lie in the expansion workspace, and its query blocks."""
         smax, mb = self.rcfg.max_num_seqs, self.max_latent_blocks

@@ -746,6 +746,11 @@ class ModelRunner:
                 sb.event.record(torch.cuda.current_stream(self.device))
             n += 1
 
+    def _rows_alone(self, st: np.ndarray, portions: List[Tuple[int, int, int, int]], t: int) -> bool:
+        """Whether the launch for single rows has any in the staged step: here the rows that no tile has."""
+        o_cd = self._off["ctx_decode"][0]
+        return bool((st[o_cd : o_cd + t] > 0).any())
+
     def _stage_in(self, sb: _Stage) -> None:
         """The staged image to the device, in stream order."""
         stage_in = getattr(self.ops, "stage_in", None)
@@ -936,7 +941,7 @@ class ModelRunner:
             if shares >= 2:
                 pf_split = shares | (pf_tiles << 8)
         pf_split = pf_split or self._step_variant(t_pad, decode_only)
-        prompts_only = bool(self.rows_apart and not decode_only and not quads and not pf_split and not (st[o_cd : o_cd + t] > 0).any())
+        prompts_only = bool(self.rows_apart and not decode_only and not quads and not pf_split and not self._rows_alone(st, portions, t))
         # (the header carries the listed rows rounded up to a power of two: fewer rows, more workgroups per context)
         dec_split = 0
         if self.dec_split_ok and not decode_only and 0 < n_dec <= self.DEC_SPLIT_ROWS and dec_max_ctx >= self.DEC_SPLIT_MIN_CTX:

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from kvmini.engine.engine import EngineConfig, LLMEngine
+from kvmini.engine.scheduler import Batch, ScheduledChunk
 from kvmini.models import registry
 from kvmini.models.llama import LlamaConfig
 
@@ -73,5 +74,35 @@ def test_prompts_alone_leave_out_the_launches_for_single_rows(design, graphs):
 
     (got, kinds), (want, old) = steps(True), steps(False)
     assert 4 not in old and (kinds == old if design == "llama" else kinds[0] == 4 and kinds[2] == 0)  # (heads of 64 have one launch for both)
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.parametrize("device,graphs", [pytest.param("cpu", False, id="cpu"), pytest.param("cuda:0", False, id="hip", marks=pytest.mark.gpu), pytest.param("cuda:0", True, id="hip-graphs", marks=pytest.mark.gpu)])
+def test_drafts_cut_to_one_token_are_a_single_row(device, graphs):
+    """A chunk of drafts of which the step's budget leaves one token, beside longer chunks: a hybrid's kernels take it as a single row, so the step has the launches for
+    those, and what the row leaves in memory is that of a step that always has them."""
+    cfg = registry.resolve_model("pipilix-tiny")[0]
+    weights = registry.random_weights(cfg, device, torch.float32 if device == "cpu" else torch.bfloat16, seed=1)
+
+    def step(apart):
+        eng = LLMEngine(EngineConfig(model=cfg.name, device=device, max_num_seqs=4, max_batched_tokens=64, max_model_len=128, num_blocks=40, use_graphs=graphs), weights=weights)
+        eng.runner.rows_apart = apart
+        eng.warmup()
+        seqs = [eng.make_sequence([1 + (i * (j + 3)) % 500 for i in range(30)]) for j in range(2)]
+        first = eng.scheduler.schedule_given([(s, 20, [19]) for s in seqs])
+        eng.runner.execute(first)
+        eng.scheduler.note_computed(first)
+        seqs[0].prompt_ids, seqs[0].draft_ids = seqs[0].prompt_ids[:21], [7, 9]  # decoding, two drafts behind its last token
+        whole = eng.scheduler.schedule_given([(seqs[1], 10, [9])])
+        cut = ScheduledChunk(seqs[0], 20, 1, False)
+        missing = eng.scheduler._blocks_needed(seqs[0], 21)
+        seqs[0].blocks += eng.scheduler.bm.allocate(missing) if missing else []
+        handle = eng.runner.launch(Batch([cut] + whole.chunks, 11))
+        eng.runner.collect(handle)
+        return handle.key[1], [t.clone() for run in eng.runner.memory.runs for branch in run for t in branch]
+
+    (kind, got), (_, want) = step(True), step(False)
+    assert kind == 0  # (4: prompts alone)
     for a, b in zip(got, want):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
