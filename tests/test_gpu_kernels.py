@@ -1678,6 +1678,22 @@ def test_staged_images_arrive_as_they_are_when_launched(C, n):
         C.stage_in(torch.zeros(n, dtype=torch.int32), there[:n])
 
 
+def test_a_staged_image_dropped_behind_the_launch_arrives_all_the_same(C):
+    """The launch waits behind other work while its image is let go and host memory of that size asked for again: not the same memory before the image is read."""
+    image, there = torch.arange(40_000, dtype=torch.int32).pin_memory(), torch.empty(40_000, dtype=torch.int32, device="cuda")
+    done = torch.cuda.Event()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(200_000_000)  # about a tenth of a second
+    C.stage_in(image, there)
+    done.record()
+    at = image.data_ptr()
+    del image
+    others = [torch.full((40_000,), -1, dtype=torch.int32, pin_memory=True) for _ in range(4)]
+    assert not done.query()  # (else this shows nothing)
+    assert at not in [o.data_ptr() for o in others]
+    assert torch.equal(there.cpu(), torch.arange(40_000, dtype=torch.int32))
+
+
 @pytest.mark.parametrize("T,H,slabs", [(1, 64, 0), (3, 512, 1), (250, 4096, 2), (7, 576, 17), (65, 2048, 0), (5, 4160, 3), (2, 8192, 16), (3, 12288, 0), (2, 16384, 4)])
 def test_residual_and_quantisation_in_one_launch(C, T, H, slabs):
     """The bits of the two launches: residual, sums of squares, bytes in both orders, scales (rows of zeros and of infinities among them)."""
