@@ -1407,7 +1407,7 @@ int select_split(const T* x, long long n, long long row_stride, int n_metrics, i
   const dim3 grid(select_parts(n, n_metrics, dtype), n_metrics);
   static const bool ok = big_lds(select_split_kernel<T, true>) && big_lds(select_split_kernel<T, false>);
   if (!ok) return -2;
-  const int room = kept_room(n, grid.x);
+  const int room = kept ? kept_room(n, grid.x) : -1;
   const long long row = kept_bytes(n, dtype);
   auto passes = [&](auto keep) {
     hipLaunchKernelGGL((select_split_kernel<T, decltype(keep)::value>), grid, dim3(SEL_THREADS), SPLIT_LDS, stream, x, n, row_stride, lv.n, work, kept, row, room);
@@ -1499,7 +1499,7 @@ int kv_select_quantiles(const void* x, long long n, long long row_stride, int n_
 }
 
 // The same by a sample's intervals, for the rows that kv_split_takes (scratch memory: kv_split_work_bytes, and what the passes keep of rows of n samples,
-// kv_split_kept_bytes — enough for calls of fewer rows as well): a count of kv_undecided() says that
+// kv_split_kept_bytes — enough for calls of fewer rows as well; null: nothing is kept): a count of kv_undecided() says that
 // kv_select_quantiles has to answer, one of kv_crowded() that this has to be called again with what it left in the scratch memory.
 int kv_split_takes(long long n, int n_metrics, int dtype) { return n > (dtype == 0 ? SEL_FEW : SEL_RANKED) && n <= SPLIT_MOST && n_metrics <= 64; }
 long long kv_split_work_bytes(int n_metrics) { return n_metrics * SPLIT_BYTES; }

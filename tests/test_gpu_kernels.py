@@ -256,6 +256,23 @@ def test_quantiles_of_rows_whose_first_pass_keeps_what_is_inside(n, dtype):
         assert np.array_equal(q, [v[int(a)] + (a - int(a)) * (v[math.ceil(a)] - v[int(a)]) for a in at])
 
 
+def test_quantiles_without_room_for_what_the_first_pass_keeps():
+    """64 rows of a million floats: 69 MB of scratch memory, and 83 that the first pass would keep.  With room for 110 beside the samples the call does without."""
+    from kvmini.ops import hist_quantile as hq
+
+    x, ps = 12 * torch.exp(0.35 * torch.randn(64, 1_000_003, device=_dev())), (0.5, 0.95, 0.99)
+    want = hq.batched_quantiles(x, ps)
+    torch.cuda.empty_cache()
+    refused = torch.cuda.memory_stats()["num_ooms"]
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (110 << 20)) / torch.cuda.get_device_properties(0).total_memory)
+        got = hq.batched_quantiles(x, ps)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.cuda.memory_stats()["num_ooms"] > refused
+    assert np.array_equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n", [16385, 300_007, 5_000_001])
 def test_quantiles_by_intervals_row_by_row(C, n, dtype):
