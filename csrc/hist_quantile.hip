@@ -35,6 +35,7 @@
 //
 // Wavefront width is 64 on CDNA; workgroups are 256 threads = 4 waves, one per SIMD.
 
+#include <algorithm>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -574,6 +575,9 @@ constexpr int SPLIT_WORDS = sizeof(SplitState) / 4;
 constexpr long long SPLIT_BYTES = sizeof(SplitState) + SPANS * SPAN_BINS * 4 + (long long)KV_MAX_RANKS * FOUND * 8;
 static_assert(sizeof(SplitState) % 16 == 0, "16-byte reads of the bins behind it");
 
+// Sampled ranks between a level and the ends of its interval, of `got`
+__host__ __device__ inline double margin(int got, double p) { return 4.0 * sqrt((double)got * p * (1.0 - p)) + 2.0; }
+
 struct SplitRow {
   SplitState* state;
   unsigned int* bins;           // [SPANS][SPAN_BINS]
@@ -588,8 +592,11 @@ struct SplitRow {
 
 // What the first pass keeps for the second: each wave the samples inside the intervals, up to `room`, and how many there were.  15 % of a row at the usual three
 // levels, so that the second pass reads those and not the row again; a wave that had more goes through its samples again.  Where a workgroup has more than 32 k
-// samples (room -1: nothing is kept): calls of 3 x 4 M floats (47 k) 69.8 -> 64.5 us, the second pass 27 -> 19.6, of 30 M (117 k) 113 -> 99; of 1 x 4 M doubles (16 k) and
-// 3 x 1 M floats (12 k) the same, of a thousand samples 1.4 more (and kernels that know both ways half of that).  Rows of which half is one value: 69 -> 71.
+// samples (room -1: nothing is kept): calls of 3 x 4 M floats (47 k) 68.5 -> 62.7 us, the second pass 27 -> 19.6, of 30 M (117 k) 111 -> 97.5, of 64 x 1 M 205 -> 158; of
+// 1 x 4 M doubles (16 k) and 3 x 1 M floats (12 k) the same, of a thousand samples 1.4 more (and kernels that know both ways half of that).  And where the levels' intervals
+// fit what is kept: quartiles of 2048 samples have 24 % inside, and what would be kept in vain is up to 2 % of a call (3 x 4 M floats 69.4, 70.7, doubles 78.9, 81.1, 64 x 1 M
+// 210, 214); of 4096 17 % (30 M floats 113 -> 104).  A row of which half is one value is kept in vain all the same (78.4, 79.7; doubles 85.5, 88.2; 64 x 1 M 251, 256): the sample
+// could say so, by the values a little outside, and 2 to 4 us of a call of 64 rows would be back, but every other call takes 0.3 to 1 longer for it.
 constexpr int WAVES = SEL_THREADS / 64, MOST_PARTS = 256, SPARE = 32;  // of a workgroup; workgroups per row, at most; of a wave, beside 3 / 16 of its samples
 template <typename T>
 struct Kept {
@@ -606,6 +613,19 @@ struct Kept {
   __device__ T* of(int part, int wave) const { return samples + ((long long)part * WAVES + wave) * room; }
 };
 inline int kept_room(long long n, int parts) { return n / parts > 32768 ? (int)(n * 3 / 16 / (parts * WAVES)) + SPARE : -1; }
+// samples of a row that are ranked (a larger sample of longer rows: it takes 6 us more, and what lies beyond its largest has to fit FOUND)
+inline int sampled(long long n) { return (n <= 1 << 22 ? 2 : 4) * SEL_THREADS; }
+// the share of a row that lies inside the levels' intervals
+inline double inside(Levels lv, long long n) {
+  std::sort(lv.p, lv.p + lv.n);
+  double all = 0.0, upto = 0.0;
+  for (int i = 0; i < lv.n; ++i) {
+    const double p = std::clamp(lv.p[i], 0.0, 1.0), apart = margin(sampled(n), p) / sampled(n), end = std::min(p + apart, 1.0);
+    all += std::max(0.0, end - std::max(p - apart, upto));
+    upto = std::max(upto, end);
+  }
+  return all;
+}
 inline long long kept_bytes(long long n, int dtype) { return MOST_PARTS * WAVES * 4 + (n * 3 / 16 + MOST_PARTS * WAVES * SPARE) / 2 * 2 * (dtype == 0 ? 4 : 8); }
 
 // Linear bins of `wide` + 1 keys: key - first >> bin_shift
@@ -750,7 +770,7 @@ __global__ __launch_bounds__(SEL_THREADS) void select_sample_kernel(const T* __r
   if (tid < KV_MAX_RANKS) {
     double p = levels.p[tid >> 1];
     p = p < 0.0 ? 0.0 : (p > 1.0 ? 1.0 : p);
-    const double at = p * (double)(got - 1), apart = 4.0 * sqrt((double)got * p * (1.0 - p)) + 2.0;
+    const double at = p * (double)(got - 1), apart = margin(got, p);
     const double end = (tid & 1) ? ceil(at + apart) : floor(at - apart);
     const bool open = end < 0.0 || end > (double)(got - 1);
     rank[tid] = end < 0.0 ? 0 : end > (double)(got - 1) ? (unsigned int)(got - 1) : (unsigned int)end;
@@ -1393,6 +1413,13 @@ int select_parts(long long n, int n_metrics, int dtype) {
   return (int)(want < 1 ? 1 : want < most ? want : most);
 }
 
+Levels levels_of(const double* ps, int n_ps) {
+  Levels lv{};
+  lv.n = n_ps;
+  for (int i = 0; i < n_ps; ++i) lv.p[i] = ps[i];
+  return lv;
+}
+
 template <typename T>
 int select_split(const T* x, long long n, long long row_stride, int n_metrics, int dtype, const Levels& lv, void* work, void* kept, unsigned long long* out, bool again, hipStream_t stream) {
   if (again) {
@@ -1400,8 +1427,7 @@ int select_split(const T* x, long long n, long long row_stride, int n_metrics, i
   } else {
     int parts = SAMPLE_PARTS;
     while (parts > 1 && parts * n_metrics > 256) parts /= 2;
-    // (a larger sample of longer rows: it takes 6 us more, and what lies beyond its largest has to fit FOUND)
-    auto sample = n <= 1 << 22 ? select_sample_kernel<T, 2> : select_sample_kernel<T, 4>;
+    auto sample = sampled(n) == 2 * SEL_THREADS ? select_sample_kernel<T, 2> : select_sample_kernel<T, 4>;
     hipLaunchKernelGGL(sample, dim3(parts, n_metrics), dim3(SEL_THREADS), 0, stream, x, n, row_stride, lv, work);
   }
   const dim3 grid(select_parts(n, n_metrics, dtype), n_metrics);
@@ -1492,9 +1518,7 @@ int kv_radix_num_passes(int dtype) { return dtype == 0 ? 3 : 6; }
 
 int kv_select_quantiles(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const double* ps, int n_ps, void* work, unsigned long long* out, hipStream_t stream) {
   if (n <= 0 || n_metrics <= 0 || n_metrics > 65535 || n_ps < 1 || n_ps > KV_MAX_RANKS / 2) return -1;
-  Levels lv{};
-  lv.n = n_ps;
-  for (int i = 0; i < n_ps; ++i) lv.p[i] = ps[i];
+  const Levels lv = levels_of(ps, n_ps);
   return dtype == 0 ? select((const float*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream) : select((const double*)x, n, row_stride, n_metrics, dtype, lv, work, out, stream);
 }
 
@@ -1503,15 +1527,15 @@ int kv_select_quantiles(const void* x, long long n, long long row_stride, int n_
 // kv_select_quantiles has to answer, one of kv_crowded() that this has to be called again with what it left in the scratch memory.
 int kv_split_takes(long long n, int n_metrics, int dtype) { return n > (dtype == 0 ? SEL_FEW : SEL_RANKED) && n <= SPLIT_MOST && n_metrics <= 64; }
 long long kv_split_work_bytes(int n_metrics) { return n_metrics * SPLIT_BYTES; }
-long long kv_split_kept_bytes(long long n, int n_metrics, int dtype) { return kept_room(n, select_parts(n, n_metrics, dtype)) < 0 ? 0 : n_metrics * kept_bytes(n, dtype); }
+long long kv_split_kept_bytes(long long n, int n_metrics, int dtype, const double* ps, int n_ps) {
+  return kept_room(n, select_parts(n, n_metrics, dtype)) < 0 || inside(levels_of(ps, n_ps), n) > 3. / 16 ? 0 : n_metrics * kept_bytes(n, dtype);
+}
 unsigned long long kv_undecided() { return UNDECIDED; }
 unsigned long long kv_crowded() { return CROWDED; }
 
 int kv_split_quantiles(const void* x, long long n, long long row_stride, int n_metrics, int dtype, const double* ps, int n_ps, void* work, void* kept, unsigned long long* out, int again, hipStream_t stream) {
   if (n_metrics <= 0 || !kv_split_takes(n, n_metrics, dtype) || n_ps < 1 || n_ps > KV_MAX_RANKS / 2) return -1;
-  Levels lv{};
-  lv.n = n_ps;
-  for (int i = 0; i < n_ps; ++i) lv.p[i] = ps[i];
+  const Levels lv = levels_of(ps, n_ps);
   return dtype == 0 ? select_split((const float*)x, n, row_stride, n_metrics, dtype, lv, work, kept, out, again != 0, stream)
                     : select_split((const double*)x, n, row_stride, n_metrics, dtype, lv, work, kept, out, again != 0, stream);
 }

@@ -235,7 +235,8 @@ def _sampled_places(n):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n", [131_071, 131_073, 140_007])
-def test_quantiles_of_rows_whose_first_pass_keeps_what_is_inside(n, dtype):
+@pytest.mark.parametrize("ps", [(0.5, 0.95, 0.99), (0.5, 0.95, 0.99, 0.3)])  # (15 % and 23 % of a row inside: what is more than 3 / 16 is not kept)
+def test_quantiles_of_rows_whose_first_pass_keeps_what_is_inside(n, dtype, ps):
     """64 rows, four workgroups each: below 32 k samples a workgroup nothing is kept, above the waves keep up to 3 / 16 of theirs, and those with more (rows of few values,
     of one, with the samples inside side by side) go through them again."""
     from kvmini.ops import hist_quantile as hq
@@ -248,12 +249,24 @@ def test_quantiles_of_rows_whose_first_pass_keeps_what_is_inside(n, dtype):
     g[4::8, ::3] = np.nan
     g[5::8] = np.repeat(g[5::8, : n // 64 + 1], 64, 1)[:, :n]
     g[6::8] = np.where(rng.random((8, n)) < 0.3, 3.0, g[6::8])
-    x, ps = g.astype(dtype), (0.5, 0.95, 0.99, 0.3)
+    x = g.astype(dtype)
     got = hq.batched_quantiles(torch.from_numpy(x).to(_dev()), ps)
     for row, q in zip(x, got):
         v = np.sort(row[~np.isnan(row)]).astype(np.float64)
         at = [p * (v.size - 1) for p in ps]
         assert np.array_equal(q, [v[int(a)] + (a - int(a)) * (v[math.ceil(a)] - v[int(a)]) for a in at])
+
+
+@pytest.mark.parametrize("n,ps,kept", [(140_007, (0.5, 0.95, 0.99), True), (140_007, (0.25, 0.5, 0.75), False), (140_007, (0.5, 0.51, 0.52, 0.53), True), (130_000, (0.5,), False)])
+def test_quantiles_keep_what_fits(n, ps, kept):
+    """Scratch memory of 64 rows beside the passes' state, 1.1 MB each: where the levels' intervals (overlaps once) are at most 3 / 16 of a row of more than 4 x 32 k."""
+    from kvmini.ops import hist_quantile as hq
+
+    x = torch.rand(64, n, device=_dev())
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    hq.batched_quantiles(x, ps)
+    assert (torch.cuda.max_memory_allocated() - before > 64 * (1_150_000 + n * 3 // 16 * 4)) == kept
 
 
 def test_quantiles_without_room_for_what_the_first_pass_keeps():
