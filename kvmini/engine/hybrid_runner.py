@@ -71,6 +71,7 @@ class HybridRunner(ModelRunner):
         self.retains = any(isinstance(m, (RetentionSpec, StateSpaceSpec)) for m in mixers_)
         self.aside = torch.cuda.Stream(self.device) if self.cfg.wiring == "parallel" and self.device.type == "cuda" and hasattr(mixers, "shared_expert") else None
         self.rows_apart = self.device.type == "cuda"
+        self.routes_last = self.cfg.layers[self.cfg.runs[-1].layer].moe is not None  # the last layer has experts
         self.span_rows = 0  # rows of the expansion workspace the staged step needs
         self._rot: Dict[Tuple[float, int], Tuple[torch.Tensor, torch.Tensor]] = {}
 
@@ -100,7 +101,6 @@ class HybridRunner(ModelRunner):
     def _alloc_cache(self) -> None:
         self.kv_scale = None
         self.decode_layers = None
-        self._row_slots = torch.zeros(self.rcfg.max_batched_tokens, dtype=torch.int32, device=self.device)  # of rows that are all in use
         self.memory = MixerMemory(self.cfg, self.num_blocks, self.block_size, self.rcfg.max_num_seqs, self.dtype, self.device, self._pads)
         # what a branch does, with its weights and memory: one callable (projections, outputs, staged step) per branch of every run
         self.branches: List[List[Callable[..., None]]] = []
@@ -140,9 +140,11 @@ class HybridRunner(ModelRunner):
         if self.retains:
             self.max_chunks = self.tmax // self.CHUNK + smax
             spans += [("chunks", 4 * self.max_chunks), ("first_chunk", smax)]
+        if self.routes_last:
+            spans += [("sample_slots", self.tmax)]
         return spans + [("tok_kind", self.tmax), ("tok_off", self.tmax), ("singles", smax), ("portions", 5 * smax), ("query_blocks", 4 * self.max_query_blocks)]
 
-    def _stage_portions(self, st: np.ndarray, portions: List[Tuple[int, int, int, int]], t: int, t_pad: int) -> None:
+    def _stage_portions(self, st: np.ndarray, portions: List[Tuple[int, int, int, int]], t: int, t_pad: int, n_samples: int) -> None:
         o_k, o_o, o_s, o_p, o_b = (self._off[k][0] for k in ("tok_kind", "tok_off", "singles", "portions", "query_blocks"))
         smax, mb = self.rcfg.max_num_seqs, self.max_query_blocks
         pa = st[o_p : o_p + 5 * smax].reshape(5, smax)
@@ -162,6 +164,10 @@ class HybridRunner(ModelRunner):
                 for off in range(0, n, self.QUERY_BLOCK):
                     ba[:, nb] = (row + off, min(self.QUERY_BLOCK, n - off), pos + off, slot)
                     nb += 1
+        if self.routes_last:  # cache slots of the rows asked for; the others that are computed with them are padding
+            o_sl, o_sm, o_ss = (self._off[k][0] for k in ("slots", "sample_idx", "sample_slots"))
+            st[o_ss : o_ss + n_samples] = st[o_sl + st[o_sm : o_sm + n_samples]]
+            st[o_ss + n_samples : o_ss + t_pad] = -1
         if self.expands:
             self._stage_spans(st, portions)
         if self.retains:
@@ -262,7 +268,7 @@ class HybridRunner(ModelRunner):
             jn = None if ahead is None else join(ahead)
             few = some is not None and ahead is None  # what feeds the last layer's feed-forward, and what comes behind its mixer
             if few:
-                x, st_ff = mx.select_rows(x, some), dataclasses.replace(st, slots=self._row_slots[: some.numel()])
+                x, st_ff = mx.select_rows(x, some), dataclasses.replace(st, slots=self._dev("sample_slots", some.numel())) if self.routes_last else st
                 if parallel:
                     xb2 = mx.select_rows(xb2, some)
             else:

@@ -394,8 +394,9 @@ class ModelRunner:
         """Further int32 arrays of the staged image: (name, entries)."""
         return []
 
-    def _stage_portions(self, st: np.ndarray, portions: List[Tuple[int, int, int, int]], t: int, t_pad: int) -> None:
-        """Fill the arrays of :meth:`_extra_staging`; ``portions``: (first row, tokens, first position, slot) of the step's chunks."""
+    def _stage_portions(self, st: np.ndarray, portions: List[Tuple[int, int, int, int]], t: int, t_pad: int, n_samples: int) -> None:
+        """Fill the arrays of :meth:`_extra_staging`; ``portions``: (first row, tokens, first position, slot) of the step's chunks; ``n_samples``: rows
+        whose logits are asked for."""
 
     def _step_variant(self, t_pad: int, decode_only: int) -> int:
         """A number that names the staged step's graph besides its token bucket and kind (0: none), handed to :meth:`forward` as ``pf_split``."""
@@ -778,7 +779,7 @@ class ModelRunner:
             sb.np[:] = 0
             sb.bt_owner = [(None, 0)] * len(sb.bt_owner)
             sb.np[o : o + n] = -1
-            self._stage_portions(sb.np, [], 0, self.tmax)
+            self._stage_portions(sb.np, [], 0, self.tmax, 0)
         self.stage_dev.copy_(self.stages[0].cpu)
 
     # ------------------------------------------------------------------
@@ -925,7 +926,7 @@ class ModelRunner:
         st[o_smp + n_samples : o_smp + t_pad] = 0
         st[o_tl + mt + n_tiles : o_tl + 2 * mt] = 0  # unused tiles: zero valid queries
 
-        self._stage_portions(st, portions, t, t_pad)
+        self._stage_portions(st, portions, t, t_pad, n_samples)
 
         # plain decoding step: every chunk is one token (no prompt chunk, no drafts to verify)
         decode_only = self.step_kind(t_pad, all(ch.n_tokens == 1 for ch in batch.chunks) and not (self.tiles_64 and n_tiles), max_ctx)

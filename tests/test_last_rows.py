@@ -5,7 +5,7 @@ import torch
 
 from kvmini.engine.engine import EngineConfig, LLMEngine
 from kvmini.engine.scheduler import Batch, ScheduledChunk
-from kvmini.models import registry
+from kvmini.models import pipilix, registry
 from kvmini.models.llama import LlamaConfig
 
 LLAMA = LlamaConfig("few-rows", 512, 256, 512, 3, 4, 2, 64, 500000.0, 1e-5, 512, 1, 2)
@@ -106,3 +106,26 @@ def test_drafts_cut_to_one_token_are_a_single_row(device, graphs):
     assert kind == 0  # (4: prompts alone)
     for a, b in zip(got, want):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.parametrize("design", ["gebasun-tiny", "sandwich"])
+@pytest.mark.parametrize("device,dtype", [pytest.param("cpu", torch.float32, id="cpu"), pytest.param("cuda:0", torch.bfloat16, id="hip", marks=pytest.mark.gpu)])
+def test_the_last_layers_experts_have_no_rows_that_nobody_asks_for(design, device, dtype, monkeypatch):
+    """The rows behind the last layer's mixer are as many as a step may ask for: those beyond the ones it does ask for are padding, as the others are in warm-up."""
+    cfg = pipilix.stack("experts-last", 512, 96, "DM", 3, 24, 40, 48, 20, 112, 6, 2, 40) if design == "sandwich" else registry.resolve_model(design)[0]
+    assert cfg.layers[cfg.runs[-1].layer].moe is not None
+    eng = LLMEngine(EngineConfig(model=cfg.name, device=device, max_num_seqs=4, max_batched_tokens=256, max_model_len=256, num_blocks=80, use_graphs=False),
+                    weights=registry.random_weights(cfg, device, dtype, seed=1))
+    calls, experts = [], eng.runner.mixers.experts
+    monkeypatch.setattr(eng.runner.mixers, "experts", lambda m, w, h, st, **kw: (calls.append((h.shape[0], st.slots.tolist())), experts(m, w, h, st, **kw))[1])
+    seqs = [eng.make_sequence([1 + (i * (j + 3)) % 500 for i in range(60)]) for j in range(2)]
+    eng.runner.execute(eng.scheduler.schedule_given([(seqs[0], 60, [59]), (seqs[1], 40, [7, 39])]))
+    rows, slots = calls[-1]
+    assert rows == len(slots) == eng.runner.sample_rows(eng.runner.bucket_for(100)) > 3
+    at = lambda s, pos: s.blocks[pos // eng.runner.block_size] * eng.runner.block_size + pos % eng.runner.block_size
+    assert slots == [at(seqs[0], 59), at(seqs[1], 7), at(seqs[1], 39)] + [-1] * (rows - 3)
+    eng.runner._stage_dummy()
+    calls.clear()
+    with torch.no_grad():
+        eng.runner.forward(eng.runner.bucket_for(100))
+    assert all(s == -1 for _rows, slots in calls for s in slots)
