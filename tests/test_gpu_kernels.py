@@ -1743,6 +1743,33 @@ def test_residual_and_quantisation_in_one_launch(C, T, H, slabs):
                 assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
 
 
+@pytest.mark.parametrize("fmt", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("slabs", [0, 2])
+def test_rows_quantised_ahead_are_those_the_product_takes(C, fmt, gated, slabs, monkeypatch):
+    """The update that knows the weights behind it, around the row count from which those multiply bytes: the bits of the update and the product by themselves, bytes from that
+    count on, and then the rows are not quantised once more."""
+    from kvmini.ops import hip_ops as ops
+
+    torch.manual_seed(7)
+    n, k, first = 512, 1024, ops.STREAM_MAX_M + 1 if fmt == "fp8" else 65
+    w = ops.PackedLinear((torch.randn(n, k, device="cuda") * 0.02).bfloat16(), fp8=fmt == "fp8", mxfp4=fmt == "mxfp4")
+    product, calls, quantise = ops.linear_swiglu if gated else ops.linear, [], C.quantize_rows_fp8
+    monkeypatch.setattr(C, "quantize_rows_fp8", lambda *a: (calls.append(a), quantise(*a))[1])
+    for t in (1, first - 1, first, first + 1, 300):
+        src = torch.randn((slabs, t, k) if slabs else (t, k), device="cuda").to(torch.float32 if slabs else torch.bfloat16)
+        res = torch.randn(t, k, device="cuda").bfloat16()
+        out = []
+        for ahead in (None, w):
+            calls.clear()
+            h, left = ops.add_rmsnorm(ops.Partial(src, None, 0.0, k) if slabs else src, res.clone(), torch.ones(k, device="cuda").bfloat16(), 1e-5, ahead=ahead)
+            out.append((product(h, w), left))
+            assert (h.rows8 is not None) == (ahead is not None and t >= first)
+            assert len(calls) == (t >= first and ahead is None)
+        for a, b in zip(*out):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("m", [3, 40, 150, 600])  # rows of the streaming kernel (narrow and wide), of narrow tiles, of panels
 def test_outputs_are_rounded_to_the_nearest_even(m):
     """One product a sum: 16 bits of mantissa, of which bf16 keeps eight (ties in one of 256), and infinities and NaN as they are.  A product is exact in fp32, so
