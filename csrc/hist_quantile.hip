@@ -549,7 +549,7 @@ __global__ __launch_bounds__(SEL_THREADS) void select_few_kernel(const T* __rest
 // call in 5000) the row's count of samples says so and the digits' passes answer for it.  Where a bin of several values holds more than fit all the same
 // (Spans says what is done against that) the count says that the two passes are to be made again, between the least and the most of that bin.
 // Whole calls by digits and so, 3 rows: 33 k floats 54 and 48 us, 1 M 69 and 52, 4 M 88 and 64;
-// 4 M doubles 198 and 79.  Of the 50 us of kernels for 3 x 4 M floats the sample takes 10, the first pass 21 and the second 20, the last workgroup's ranking
+// 4 M doubles 198 and 79.  Of the 50 us of kernels for 3 x 4 M floats the sample takes 10, the first pass 21 and the second 19, the last workgroup's ranking
 // among them: beside reading (10 us a pass at 5 TB/s) chains of dependent steps, about one us each.  Fewer bins (512, 256) are not faster: their sums are not what counts.
 constexpr int SAMPLE_PARTS = 64;                     // workgroups that rank a row's sample, at most
 constexpr int SPANS = KV_MAX_RANKS / 2;              // intervals: one per level, fewer where they overlap

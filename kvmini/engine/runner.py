@@ -228,7 +228,7 @@ class ModelRunner:
         # (token bucket, step kind) -> (graph, logits); kind 0 = mixed step, 1 = decode-only (fused
         # RoPE + attention kernel), 2 = decode-only with the context split over several workgroups, 3 = mixed without prompt tiles
         # (tiles_64: the attention kernel by rows alone), 4 = prompts alone, without the launches for rows that are the only ones of their sequence
-        # (rows_apart: where those are launches of their own; 4.5 to 15 us a layer).  Kind 0 serves the last two as well.
+        # (rows_apart: where those are launches of their own; 4.5 to 15 us a layer, for 35 ms of capture a bucket at four layers).  Kind 0 serves the last two as well.
         self.graphs: Dict[Tuple[int, ...], Any] = {}
         self._graph_pool = None
         # Weight read-ahead on a second stream beside the decode attention kernel (a parallel branch of the

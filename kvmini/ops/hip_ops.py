@@ -315,7 +315,8 @@ def _plan_slabs(n_pad: int, k: int, m: int = 32, group_cols: int = 256) -> Tuple
 # efficiency for more workgroups; 256 x 224 and 256 x 192 exist for feature counts whose
 # 256-wide tiles leave a ragged last round over the 256 CUs, whole or with K split (6144 = 32 x 192).
 # bf16 weights come here with few outputs or where K is split (_plan_panels).
-# (128 x 128 has eight waves with bf16 weights since the fit, 0.57; the lines between the tiles stayed where they were.)
+# (128 x 128: four waves' 0.62.  With bf16 weights it has eight, which take 0.57; that number here would move K splits, and narrow tiles take theirs from this
+# plan: the lines between the tiles are four waves', and what eight would move has not been measured.)
 _WIDE_TILES_BF16 = (((256, 256, 1), 1.68), ((256, 224, 1), 1.615), ((256, 192, 0), 1.36), ((256, 128, 0), 0.84), ((128, 256, 0), 0.87), ((128, 128, 0), 0.62), ((256, 64, 0), 0.65))
 _WIDE_TILES_FP8 = (((256, 256, 0), 1.9), ((256, 224, 0), 1.85), ((256, 192, 0), 1.55), ((256, 128, 0), 0.84), ((128, 256, 0), 0.87), ((128, 128, 0), 0.62))
 # The 128-wide tiles move 1.5 x the operand bytes per MAC of the 256-wide ones from L2 into LDS; on
