@@ -351,8 +351,8 @@ typedef __attribute__((ext_vector_type(4))) float f4;
 
 // What counts in delta_tile_kernel is how many workgroups a CU holds, and that none of them waits for long.  Partial sums of the pairs with j < i alone (the
 // 36 blocks of 2 x 2) make that four, of 40 KB, with 128 channels and columns.  All rows that a workgroup reads are on their way before the first is used, a
-// row of 16 tokens is summed by sixteen lanes, and all lanes have pairs with j < i to work out (on the diagonal B is the product of the unit vectors, which
-// their sums give).  4 x 560 tokens of 32 heads, us a layer in the profile of a step: 72 (one column's rows at a time, sums over a wave, 28 lanes of 64
+// row of 16 tokens is summed by sixteen lanes, and all lanes have pairs with j < i to work out (on the diagonal B is the product of the unit vectors, summed as
+// they are made).  4 x 560 tokens of 32 heads, us a layer in the profile of a step: 72 (one column's rows at a time, sums over a wave, 28 lanes of 64
 // idle over the pairs 100); the bytes it writes alone would take 37.
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ inline rsrc_t rows_of(const void* p) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, -1, 0x00027000); }
@@ -486,18 +486,20 @@ __global__ __launch_bounds__(256, 4) void delta_tile_kernel(const T* __restrict_
       for (int e = 0; e < 4; ++e) {
         sq += q[e] * q[e];
         sk += k[e] * k[e];
-        sb += q[e] * k[e];
       }
     }
     sq = row16_sum(sq);
     sk = row16_sum(sk);
-    sb = row16_sum(sb);
     const float nq = 1.f / (sqrtf(sq + 1e-6f) * sqrtf((float)a.dim)), nk = 1.f / sqrtf(sk + 1e-6f);
-    if (d0 == 0) own[i] = sb * nq * nk;
     for (int d = d0; d < dkp; d += 64) {
-      *reinterpret_cast<f4*>(qs + i * rs + d) *= nq;
-      *reinterpret_cast<f4*>(ks + i * rs + d) *= nk;
+      const f4 q = *reinterpret_cast<const f4*>(qs + i * rs + d) * nq, k = *reinterpret_cast<const f4*>(ks + i * rs + d) * nk;
+      *reinterpret_cast<f4*>(qs + i * rs + d) = q;
+      *reinterpret_cast<f4*>(ks + i * rs + d) = k;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sb += q[e] * k[e];
     }
+    sb = row16_sum(sb);
+    if (d0 == 0) own[i] = sb;  // (of the normed rows: where a square overflows the norm makes zeros of them)
   }
   __syncthreads();
   {  // partial A, B: a wave has a quarter of the channels, two lanes every other four of them for the pairs (2 bi + x, 2 bj + y), bi > bj; a lane on

@@ -228,6 +228,45 @@ def test_delta_portions_among_many_that_could_be(heads, dim, vdim, lens):
             at += n
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim", [64, 128, 200])
+def test_delta_tiles_of_rows_whose_squares_overflow(dim, dtype):
+    """A query, a key and both so large that the sum of their squares is infinite: unit vectors of zeros, in a tile as token by token."""
+    device, mx = torch.device("cuda:0"), mixers_of(torch.device("cuda:0"))
+    heads, vdim, t = 4, 64, 20
+    m = hybrid.DeltaSpec(heads, heads, dim, vdim, 4)
+    gen = torch.Generator().manual_seed(dim)
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    nk = heads * dim
+    offs = [0, nk, 2 * nk, 2 * nk + heads * vdim]
+    f = lambda x: x.float().contiguous().to(device)  # noqa: E731
+    conv = torch.zeros(4, m.channels)
+    conv[3] = 1  # (a token's own input alone)
+    w = hybrid.DeltaWeights(*offs, 0, 0, 0, nk, 0, None, f(conv), f(rnd(heads) - 2), f(rnd(nk) - 2), f(1 + 0.2 * rnd(vdim)))
+    proj, low = rnd(t, offs[3] + heads), rnd(t, heads * (dim + vdim))
+    for at, first, last in ((3, 0, nk), (7, nk, 2 * nk), (12, 0, 2 * nk), (18, 0, dim)):
+        proj[at, first:last] = 4e19
+    proj, low = proj.to(dtype).to(device), low.to(dtype).to(device)
+
+    def run(lens):
+        state, ring = torch.full((3, heads, dim, vdim), 7.0, device=device), torch.zeros(3, 4, m.channels, dtype=dtype, device=device)
+        ds, out, at = mx.DeltaState(m, w, 1.0, 1e-5, state, ring), [], 0
+        for n in lens:
+            st = make_step(mx, [(n, at, 2)], device)
+            x, lo = torch.zeros(st.rows, proj.shape[1], dtype=dtype, device=device), torch.zeros(st.rows, low.shape[1], dtype=dtype, device=device)
+            x[:n], lo[:n] = proj[at : at + n], low[at : at + n]
+            mix = torch.zeros(st.rows, heads * vdim, dtype=dtype, device=device)
+            ds.run(x, lo, mix, st)
+            out.append(mix[:n].double().cpu())
+            at += n
+        return torch.cat(out), state[2].double().cpu()
+
+    (got, state), (want, left) = run([t]), run([1] * t)
+    assert got.isfinite().all() and (got[3] == 0).all()
+    assert rel(got, want) < (2e-6 if dtype == torch.float32 else 0.01) and rel(state, left) < 2e-6
+
+
 @pytest.mark.parametrize("backend", BACKENDS)
 @pytest.mark.parametrize("heads,kv,dim,vdim,taps,strong", [(4, 2, 24, 16, 3, 0.0), (2, 2, 128, 128, 4, 0.0), (3, 1, 40, 6, 1, 3.0), (4, 4, 28, 36, 2, 4.0), (2, 1, 200, 48, 6, 1.0), (8, 2, 64, 256, 4, 0.0), (2, 2, 256, 128, 3, 0.0), (1, 1, 260, 64, 4, 0.0)])
 def test_delta_rule_alone(backend, heads, kv, dim, vdim, taps, strong):
