@@ -10,6 +10,7 @@
 #include <stdint.h>
 #include <type_traits>
 
+#include "fragments.h"
 #include "quantise.h"
 
 namespace {
@@ -301,8 +302,8 @@ __device__ inline float row_ss_total(const float* __restrict__ p, int parts, int
 //
 // The plan mirrors the grid of stream_gemm3_kernel (csrc/stream_gemm.hip): workgroup (bx, by) of
 // a (gx, gy) grid streams, for each of its nw waves w, the bytes
-//     base + (bx * nw + w) * tile_bytes + by * split_bytes + [0, split_bytes)
-// of the packed weights; the first `kib` KiB of each such range are fetched here.
+//     units [by * split_bytes / 1024, + split_bytes / 1024) of tile bx * nw + w
+// of the packed weights (fragments.h); the first `kib` of each such range are fetched here.
 struct PrefetchPlan {
   const unsigned char* base;  // packed weights of the next GEMM (nullptr: no prefetch workgroups were launched)
   int gx, gy, nw, kib;
@@ -331,8 +332,10 @@ __device__ inline void prefetch_role(const PrefetchPlan& pf, int j0, int lin, in
     const int ii = rg / pf.nw, w = rg - ii * pf.nw;
     const int g = 8 * ii + x;
     const int by = g / pf.gx, bx = g - by * pf.gx;
-    const uint4* p = reinterpret_cast<const uint4*>(pf.base + ((long long)bx * pf.nw + w) * pf.tile_bytes + (long long)by * pf.split_bytes) + lane;
-    for (int k = 0; k < pf.kib; ++k) asm volatile("global_load_dwordx4 %0, %1, off" : "+v"(scratch) : "v"(p + k * 64) : "memory");
+    const int units = (int)(pf.tile_bytes >> 10), u0 = by * (int)(pf.split_bytes >> 10);
+    const bool grouped = frag_grouped((long long)pf.gx * pf.nw * 16, units);
+    const uint4* p = reinterpret_cast<const uint4*>(pf.base) + frag_first(bx * pf.nw + w, units, grouped) * 64 + lane;
+    for (int k = 0; k < pf.kib && u0 + k < units; ++k) asm volatile("global_load_dwordx4 %0, %1, off" : "+v"(scratch) : "v"(p + frag_behind(u0 + k, grouped) * 64) : "memory");
   }
   // `scratch` is an in/out operand of every load and of this wait, so it is live from the first
   // load to here and the compiler keeps other values out of the registers the loads land in.
@@ -2791,8 +2794,9 @@ int make_prefetch_plan(const void* base, const long long* v, unsigned int* sink,
   if (gx < 1 || gy < 1 || nw < 1 || kib < 1 || wgs < 8 || (wgs & 7) || wgs > 65536 || gx * gy > (1 << 20)) return -1;
   if (tile_bytes < 1024 || (tile_bytes & 1023) || split_bytes < 1024 || (split_bytes & 1023) || ((uintptr_t)base & 15)) return -1;
   if (kib * 1024 > split_bytes) return -1;
-  // the last range starts at ((gx * nw - 1) * tile_bytes + (gy - 1) * split_bytes) and is kib KiB long
-  if ((gx * nw - 1) * tile_bytes + (gy - 1) * split_bytes + kib * 1024 > bytes) return -1;
+  // the last range starts at ((gx * nw - 1) * tile_bytes + (gy - 1) * split_bytes) and is kib KiB long; tiles lie one behind another or in whole groups,
+  // and what a range has past its tile's end is not read
+  if ((gx * nw - 1) * tile_bytes + (gy - 1) * split_bytes + kib * 1024 > bytes || gx * nw > bytes / tile_bytes) return -1;
   *out = PrefetchPlan{(const unsigned char*)base, (int)gx, (int)gy, (int)nw, (int)kib, tile_bytes, split_bytes, (int)wgs, sink};
   return 0;
 }
@@ -2962,7 +2966,7 @@ __device__ __forceinline__ void dl_gemm(const void* __restrict__ Wp, const DlGem
 #define DL_ISSUE_W(slot, chunk)                                                                                                     \
   do {                                                                                                                              \
     if (active) {                                                                                                                   \
-      _Pragma("unroll") for (int u = 0; u < KS; ++u) a[slot][u] = __builtin_nontemporal_load(wp + ((long long)(chunk) * KS + u) * 64); \
+      _Pragma("unroll") for (int u = 0; u < KS; ++u) a[slot][u] = __builtin_nontemporal_load(wp + frag_behind((chunk) * KS + u, grouped) * 64); \
     }                                                                                                                               \
   } while (0)
 #define DL_ISSUE_X(slot, chunk)                                                                                                     \
@@ -2989,7 +2993,8 @@ __device__ __forceinline__ void dl_gemm(const void* __restrict__ Wp, const DlGem
   bool has = unit < n_units;
   int fg = has ? unit % groups : 0, sp = has ? unit / groups : 0;
   long long tile = (long long)fg * g.nw + wave;
-  const dl_raw16* wp = reinterpret_cast<const dl_raw16*>(Wp) + tile * (long long)ksteps * 64 + lane;
+  const bool grouped = frag_grouped(g.N, ksteps);
+  const dl_raw16* wp = reinterpret_cast<const dl_raw16*>(Wp) + frag_first((int)tile, ksteps, grouped) * 64 + lane;
   int c0 = sp * g.cps, c1 = c0 + g.cps < nchunks ? c0 + g.cps : nchunks;
   if (has) {
 #pragma unroll
@@ -3050,7 +3055,7 @@ __device__ __forceinline__ void dl_gemm(const void* __restrict__ Wp, const DlGem
     if (has) {  // further units of this workgroup (more units than workgroups): no barrier to hide behind
       fg = unit % groups; sp = unit / groups;
       tile = (long long)fg * g.nw + wave;
-      wp = reinterpret_cast<const dl_raw16*>(Wp) + tile * (long long)ksteps * 64 + lane;
+      wp = reinterpret_cast<const dl_raw16*>(Wp) + frag_first((int)tile, ksteps, grouped) * 64 + lane;
       c0 = sp * g.cps; c1 = c0 + g.cps < nchunks ? c0 + g.cps : nchunks;
 #pragma unroll
       for (int s = 0; s < PD; ++s)

@@ -1,5 +1,5 @@
 // Products by panels of 256 features on gfx950, for one matrix of many outputs and for a mixture of experts with many rows.
-//  * A workgroup is a panel x up to 256 rows; each of its 8 waves owns 32 features and all rows.  Weights (fragment order [N/16][K/32][64][8]) go
+//  * A workgroup is a panel x up to 256 rows; each of its 8 waves owns 32 features and all rows.  Weights (in fragments, fragments.h) go
 //    straight to registers, no byte twice, 3 to 6 stages of 64 columns ahead (96 KiB of them in flight per CU: through LDS there was room for
 //    48), the rows to LDS by LDS-DMA, as far ahead, in a ring; all waves read all rows from there.
 //  * The barrier of a stage stands before its last batch, where the first read of the next stage is issued, not at its top: what is fetched has a
@@ -25,6 +25,7 @@
 #include <utility>
 
 #include "experts.h"
+#include "fragments.h"
 
 namespace {
 
@@ -94,10 +95,14 @@ __device__ inline int piece_of(int wave, int i, int pieces) {
 template <class F, int... U>
 __device__ __attribute__((always_inline)) inline void each(const F& f, std::integer_sequence<int, U...>) { (f(std::integral_constant<int, U>{}), ...); }
 
+// Where a tile's bytes of stage st lie behind its first (bf16 and e4m3: a stage is a block of two units, MXFP4: a unit); block: bytes from one to the next
+template <int Q>
+__device__ inline int stage_bytes(int st, int block) { return Q == MXFP4 ? (st >> 1) * block + (st & 1) * 1024 : st * block; }
+
 // acc[i][j] += the wave's feature tile i x rows 16 j .. of NF row tiles (a multiple of two), over n stages of 64 columns.  MXFP4: sr, s0 and s1 of the
 // block scales as wr, w0 and w1 of the weights.
 template <int NF, int Q>
-__device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t sr, int s0, int s1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
+__device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, int block, rsrc_t sr, int s0, int s1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
   constexpr int AHEAD = ahead(NF), RING = AHEAD + 1, STAGE = NF * 2048;
   static_assert(RING * STAGE <= RING_BYTES, "ring");
   constexpr int PX = (2 * NF + 7) / 8, OPS = 4 + PX;  // pieces of x and memory operations per wave and stage
@@ -131,8 +136,8 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
           scale[u][0] = load4(sr, s0, st * 64);
           scale[u][1] = load4(sr, s1, st * 64);
         } else {
-          w[u][k][0] = load16(wr, w0, st * (Q == MXFP4 ? 1024 : 2048) + k * 1024);
-          w[u][k][1] = load16(wr, w1, st * (Q == MXFP4 ? 1024 : 2048) + k * 1024);
+          w[u][k][0] = load16(wr, w0, stage_bytes<Q>(st, block) + k * 1024);
+          w[u][k][1] = load16(wr, w1, stage_bytes<Q>(st, block) + k * 1024);
         }
       }
   };
@@ -207,16 +212,16 @@ __device__ __attribute__((always_inline)) inline void multiply_rows(frag_cd (&ac
 }
 
 template <int Q>
-__device__ __attribute__((always_inline)) inline void multiply(int nf, frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, rsrc_t sr, int s0, int s1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
+__device__ __attribute__((always_inline)) inline void multiply(int nf, frag_cd (&acc)[2][16], rsrc_t wr, int w0, int w1, int block, rsrc_t sr, int s0, int s1, rsrc_t xr, const int (&xsrc)[4], unsigned char* ring, int n, int wave, int lane) {
   switch (nf) {
-    case 16: if constexpr (Q != MXFP4) multiply_rows<16, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;  // (of MXFP4 224 rows: what transposes its weights takes the registers)
-    case 14: multiply_rows<14, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
-    case 12: multiply_rows<12, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
-    case 10: multiply_rows<10, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
-    case 8: multiply_rows<8, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
-    case 6: multiply_rows<6, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
-    case 4: multiply_rows<4, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
-    default: multiply_rows<2, Q>(acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 16: if constexpr (Q != MXFP4) multiply_rows<16, Q>(acc, wr, w0, w1, block, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;  // (of MXFP4 224 rows: what transposes its weights takes the registers)
+    case 14: multiply_rows<14, Q>(acc, wr, w0, w1, block, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 12: multiply_rows<12, Q>(acc, wr, w0, w1, block, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 10: multiply_rows<10, Q>(acc, wr, w0, w1, block, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 8: multiply_rows<8, Q>(acc, wr, w0, w1, block, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 6: multiply_rows<6, Q>(acc, wr, w0, w1, block, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    case 4: multiply_rows<4, Q>(acc, wr, w0, w1, block, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
+    default: multiply_rows<2, Q>(acc, wr, w0, w1, block, sr, s0, s1, xr, xsrc, ring, n, wave, lane); break;
   }
 }
 
@@ -303,7 +308,7 @@ __global__ __launch_bounds__(512) void expert_panel_kernel(const PanelArgs p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  multiply<BF16>(nf, acc, wr, w0, w1, wr, 0, 0, xr, xsrc, ring, p.K / 64, wave, lane);
+  multiply<BF16>(nf, acc, wr, w0, w1, FRAG_BLOCK * 1024, wr, 0, 0, xr, xsrc, ring, p.K / 64, wave, lane);
   const int f0 = panel * p.features + wave * 32;
   if (wave * 32 >= p.features || f0 >= p.N) return;
   store_rows<MODE, false>(acc, {}, rows, f0, lane, [](int) { return 1.f; }, [&](float g, float u) { return expert_gate(g, u, p.gate); },
@@ -353,7 +358,9 @@ __device__ __attribute__((always_inline)) inline void dense_panel(const DenseArg
   const int have = p.N / 16 - panel * (FEATURES / 16) < FEATURES / 16 ? p.N / 16 - panel * (FEATURES / 16) : FEATURES / 16;  // feature tiles; past them reads give zeros
   const int tile_bytes = nks * (Q == MXFP4 ? 512 : 1024);
   const rsrc_t wr = buffer_of(p.w + (long long)panel * (FEATURES / 16) * tile_bytes, (unsigned int)have * tile_bytes);
-  const int w0 = 2 * wave * tile_bytes + lane * 16, w1 = w0 + tile_bytes;
+  static_assert(FEATURES == 16 * FRAG_GROUP, "a panel is a group of tiles, where there are groups: the buffer ends with its last tile's bytes either way");
+  const bool grouped = frag_grouped(p.N, tile_bytes / 1024);
+  const int next = frag_next(tile_bytes / 1024, grouped) * 1024, w0 = 2 * wave * next + lane * 16, w1 = w0 + next;
   const rsrc_t sr = Q == MXFP4 ? buffer_of(p.scales.blocks + (long long)panel * (FEATURES / 16) * nks * 8, (unsigned int)have * nks * 32) : wr;
   const int s0 = 2 * wave * nks * 32 + (lane & 15) * 4, s1 = s0 + nks * 32;
   const rsrc_t xr = buffer_of(p.x + m0 * p.ldx, (unsigned int)(((rows - 1) * p.ldx + p.K) * 2));
@@ -368,7 +375,7 @@ __device__ __attribute__((always_inline)) inline void dense_panel(const DenseArg
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  multiply<Q>(nf, acc, wr, w0, w1, sr, s0, s1, xr, xsrc, ring, p.K / 64, wave, lane);
+  multiply<Q>(nf, acc, wr, w0, w1, frag_stride(grouped) * 1024, sr, s0, s1, xr, xsrc, ring, p.K / 64, wave, lane);
   if (scaled) __syncthreads();
   const int f0 = panel * FEATURES + wave * 32;
   if (f0 >= p.N) return;
@@ -422,7 +429,7 @@ __host__ __device__ constexpr int narrow_ring(int height) { return (NARROW_AHEAD
 constexpr int NOWHERE = 0x7ffffff0;  // a lane's offset past any buffer (no scalar offset added to it comes round to its beginning)
 
 template <int NF, int Q>
-__device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&acc)[8], rsrc_t wr, int wlane, int w0, rsrc_t sr, int slane, int s0, rsrc_t xr, const int (&xsrc)[2], unsigned char* ring, int c0, int n, int wave, int lane) {
+__device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&acc)[8], rsrc_t wr, int wlane, int w0, int block, rsrc_t sr, int slane, int s0, rsrc_t xr, const int (&xsrc)[2], unsigned char* ring, int c0, int n, int wave, int lane) {
   constexpr int AHEAD = NARROW_AHEAD, RING = AHEAD + 1, STAGE = NF * 2048;
   static_assert(RING * STAGE <= RING_BYTES, "ring");
   constexpr int PX = (2 * NF + 7) / 8, OPS = 2 + PX, BEFORE = Q == BF16 ? PX + 1 : PX;  // memory operations of a stage, and those in front of its barrier
@@ -441,7 +448,7 @@ __device__ __attribute__((always_inline)) inline void multiply_narrow(frag_cd (&
   auto weights = [&](int k, int u, int st) __attribute__((always_inline)) {
     const bool there = st < n;
     if (Q == MXFP4 && k == 1) scale[u] = load4(sr, there ? slane : NOWHERE, s0 + (c0 + st) * 64);
-    else w[u][k] = load16(wr, there ? wlane : NOWHERE, w0 + (c0 + st) * (Q == MXFP4 ? 1024 : 2048) + k * 1024);
+    else w[u][k] = load16(wr, there ? wlane : NOWHERE, w0 + stage_bytes<Q>(c0 + st, block) + k * 1024);
   };
   auto multiply = [&](int t, int u) __attribute__((always_inline)) {
     if constexpr (Q == BF16) {
@@ -515,7 +522,10 @@ __global__ __launch_bounds__(512) void narrow_tiles_kernel(const NarrowArgs p) {
   const bool scaled = Q != BF16 || (MODE != SUMS && p.row_ss != nullptr);  // (sums: by the scale of the bytes alone)
   if (scaled && threadIdx.x < rows) row_scale[threadIdx.x] = MODE == SUMS ? p.scales.x[m0 + (int)threadIdx.x] : scale_of_row<Q>(p, m0 + (int)threadIdx.x);
   const int tile_bytes = nks * (Q == MXFP4 ? 512 : 1024);
-  const rsrc_t wr = buffer_of(p.w + (long long)panel * (NARROW_FEATURES / 16) * tile_bytes, (unsigned int)(NARROW_FEATURES / 16) * tile_bytes);
+  // (a group of tiles is two panels)
+  const bool grouped = frag_grouped(p.N, tile_bytes / 1024);
+  const int from = grouped ? panel / (FRAG_GROUP * 16 / NARROW_FEATURES) * FRAG_GROUP : panel * (NARROW_FEATURES / 16), have = grouped ? FRAG_GROUP : NARROW_FEATURES / 16;
+  const rsrc_t wr = buffer_of(p.w + (long long)from * tile_bytes, (unsigned int)have * tile_bytes);
   const rsrc_t sr = Q == MXFP4 ? buffer_of(p.scales.blocks + (long long)panel * (NARROW_FEATURES / 16) * nks * 8, (unsigned int)(NARROW_FEATURES / 16) * nks * 32) : wr;
   const rsrc_t xr = buffer_of(p.x + m0 * p.ldx, (unsigned int)(((rows - 1) * p.ldx + p.K) * 2));
   int xsrc[2];
@@ -527,12 +537,12 @@ __global__ __launch_bounds__(512) void narrow_tiles_kernel(const NarrowArgs p) {
   frag_cd acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = (frag_cd){0.f, 0.f, 0.f, 0.f};
-  const int w0 = wave * tile_bytes, s0 = wave * nks * 32;
+  const int w0 = (panel * (NARROW_FEATURES / 16) - from + wave) * frag_next(tile_bytes / 1024, grouped) * 1024, s0 = wave * nks * 32;
   switch (nf) {
-    case 8: multiply_narrow<8, Q>(acc, wr, lane * 16, w0, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
-    case 6: multiply_narrow<6, Q>(acc, wr, lane * 16, w0, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
-    case 4: multiply_narrow<4, Q>(acc, wr, lane * 16, w0, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
-    default: multiply_narrow<2, Q>(acc, wr, lane * 16, w0, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
+    case 8: multiply_narrow<8, Q>(acc, wr, lane * 16, w0, frag_stride(grouped) * 1024, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
+    case 6: multiply_narrow<6, Q>(acc, wr, lane * 16, w0, frag_stride(grouped) * 1024, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
+    case 4: multiply_narrow<4, Q>(acc, wr, lane * 16, w0, frag_stride(grouped) * 1024, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
+    default: multiply_narrow<2, Q>(acc, wr, lane * 16, w0, frag_stride(grouped) * 1024, sr, (lane & 15) * 4, s0, xr, xsrc, ring, c0, n, wave, lane); break;
   }
   if (scaled) __syncthreads();
   // acc[j][e]: feature 4 q + e of the wave's 16, row 16 j + r

@@ -5,9 +5,9 @@
 // way.  Measured on the first kernel of this kind (no LDS staging of x), the time grew linearly with M
 // because every wave re-read its x fragments from L2 in 64-byte row pieces.  Here:
 //
-//  * W is stored pre-packed in MFMA fragment order [N/16][K/32][64 lanes][8 bf16], so a
-//    wave-level load of one A fragment tile is one contiguous 1 KiB, and a wave's k-steps
-//    are consecutive KiBs.  Weights go global -> VGPR directly (each byte is used once),
+//  * W is stored pre-packed in MFMA fragments [64 lanes][8 bf16], so a
+//    wave-level load of one A fragment tile is one contiguous 1 KiB, in an order in which
+//    neighbouring waves' lie side by side (fragments.h).  Weights go global -> VGPR directly (each byte is used once),
 //    register double-buffered one K-chunk ahead.
 //  * A workgroup = 4 waves = 64 output features (one 16-row tile per wave) x one K-slice.
 //    The x chunk [M x KC] is fetched ONCE per workgroup, written to LDS in B-fragment order
@@ -26,6 +26,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include "fragments.h"
 
 namespace {
 
@@ -99,16 +101,17 @@ __device__ inline frag_ab a_frag4(const raw16 raw, unsigned int sc, int u) {
 // One thread per (16-feature tile, 128-column group, lane): its 16 bytes are four k-steps of 8
 // values; each becomes the lane's 16-byte bf16 fragment of that k-step (1 KiB per wave and store).
 __global__ __launch_bounds__(256) void unpack_mxfp4_kernel(const raw16* __restrict__ wp4, const unsigned int* __restrict__ scales, raw16* __restrict__ wp,
-                                                           long long total) {
+                                                           long long total, int groups, int grouped4, int grouped) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
   const int lane = (int)(i & 63);
   const long long tg = i >> 6;  // tile * groups + group
-  const raw16 raw = wp4[i];
+  const int tile = (int)(tg / groups), g = (int)(tg % groups);
+  const raw16 raw = wp4[(frag_first(tile, groups, grouped4) + frag_behind(g, grouped4)) * 64 + lane];
   const unsigned int sc = scales[tg * 16 + (lane & 15)];
-  raw16* dst = wp + (tg * 4) * 64 + lane;  // k-step 4 * group + u of the same tile: 64 fragments further per u
+  raw16* dst = wp + frag_first(tile, 4 * groups, grouped) * 64 + lane;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) dst[u * 64] = __builtin_bit_cast(raw16, a_frag4(raw, sc, u));
+  for (int u = 0; u < 4; ++u) dst[frag_behind(4 * g + u, grouped) * 64] = __builtin_bit_cast(raw16, a_frag4(raw, sc, u));
 }
 
 // Shared epilogue.  Lane holds y[token j*16 + r][feature tile*16 + 4q + e], e = 0..3, in acc[j][e].
@@ -222,8 +225,9 @@ __global__ __launch_bounds__(256) void stream_gemm_kernel(const void* __restrict
   const int c0 = blockIdx.y * chunks_per_split;
   const int c1 = c0 + chunks_per_split < nchunks ? c0 + chunks_per_split : nchunks;
   const long long tile = (long long)blockIdx.x * 4 + wave;  // 16-row tile of W owned by this wave
-  // 16-byte units: bf16 [tile][kstep][lane], fp8 [tile][kstep pair][lane]
-  const raw16* wp = reinterpret_cast<const raw16*>(Wp) + tile * (W8 ? ksteps / 2 : ksteps) * 64 + lane;
+  const int units = W8 ? ksteps / 2 : ksteps;  // of a tile: a k-step, or two
+  const bool grouped = frag_grouped(N, units);
+  const raw16* wp = reinterpret_cast<const raw16*>(Wp) + frag_first((int)tile, units, grouped) * 64 + lane;
 
   // x fragment slot s = tid + 256*i  ->  tile f = s/64 (= wave + 4*i), ks = f / MT, j = f % MT
   const __bf16* xsrc[XL];
@@ -249,7 +253,7 @@ __global__ __launch_bounds__(256) void stream_gemm_kernel(const void* __restrict
     for (int i = 0; i < XL; ++i)
       if (xok[i]) xr[i] = *reinterpret_cast<const frag_ab*>(xsrc[i] + (long long)c0 * KS * 32);
 #pragma unroll
-    for (int u = 0; u < AL; ++u) a_cur[u] = wp[((long long)c0 * AL + u) * 64];
+    for (int u = 0; u < AL; ++u) a_cur[u] = wp[frag_behind(c0 * AL + u, grouped) * 64];
 #pragma unroll
     for (int i = 0; i < XL; ++i)
       if (xok[i]) xs[(0 * XF + wave + 4 * i) * 64 + lane] = xr[i];
@@ -263,7 +267,7 @@ __global__ __launch_bounds__(256) void stream_gemm_kernel(const void* __restrict
       for (int i = 0; i < XL; ++i)
         if (xok[i]) xr[i] = *reinterpret_cast<const frag_ab*>(xsrc[i] + (long long)(c + 1) * KS * 32);
 #pragma unroll
-      for (int u = 0; u < AL; ++u) a_nxt[u] = wp[((long long)(c + 1) * AL + u) * 64];
+      for (int u = 0; u < AL; ++u) a_nxt[u] = wp[frag_behind((c + 1) * AL + u, grouped) * 64];
     }
     __syncthreads();  // x chunk c is in LDS buffer `buf`; everyone is done reading buffer `buf^1`
 #pragma unroll
@@ -353,8 +357,10 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm3_kernel(const void* __res
   const long long tile_raw = ((long long)blockIdx.x * NW + wave) * FT;
   const bool tile_ok = tile_raw + FT <= ntiles;
   const long long tile = tile_ok ? tile_raw : ntiles - FT;  // the wave's first tile
-  const long long tile_units = (long long)(ksteps * AL / KS) * 64;    // 16-byte units of one tile's weights
-  const raw16* wp = reinterpret_cast<const raw16*>(Wp) + tile * tile_units + lane;
+  const int units = ksteps * AL / KS;                                 // of a tile, 1 KiB each
+  const bool grouped = frag_grouped(N, units);
+  const long long tile_step = (long long)frag_next(units, grouped) * 64, block_step = (long long)frag_stride(grouped) * 64;
+  const raw16* wp = reinterpret_cast<const raw16*>(Wp) + frag_first(__builtin_amdgcn_readfirstlane((int)tile), units, grouped) * 64 + lane;
   const long long sc_units = (long long)(ksteps / 4) * 16;            // scale words of one tile (W4)
   const unsigned int* scp = reinterpret_cast<const unsigned int*>(w_scale) + (W4 ? tile * sc_units + r : 0);  // W4: one word per chunk
   unsigned int sc[NB][FT][W4 ? AL : 1];
@@ -391,7 +397,7 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm3_kernel(const void* __res
     _Pragma("unroll") for (int i = 0; i < XL; ++i) if (wave + NW * i < XF)                                      \
         xr[slot][i] = *reinterpret_cast<const frag_ab*>(xsrc[i] + (long long)(chunk) * KS * 32);                \
     _Pragma("unroll") for (int f = 0; f < FT; ++f) {                                                            \
-      _Pragma("unroll") for (int u = 0; u < AL; ++u) a[slot][f][u] = ldw16<NT>(wp + f * tile_units + ((long long)(chunk) * AL + u) * 64); \
+      _Pragma("unroll") for (int u = 0; u < AL; ++u) a[slot][f][u] = ldw16<NT>(wp + f * tile_step + (((chunk) * AL + u) / FRAG_BLOCK) * block_step + ((chunk) * AL + u) % FRAG_BLOCK * 64); \
       if constexpr (W4) {                                                                                       \
         _Pragma("unroll") for (int u = 0; u < AL; ++u) sc[slot][f][u] = scp[f * sc_units + ((long long)(chunk) * AL + u) * 16]; \
       }                                                                                                         \
@@ -527,7 +533,9 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_rowsum_kernel(const void*
   const int r = lane & 15, q = lane >> 4;
   const int ksteps = K >> 5;
   const long long tile = blockIdx.x;
-  const raw16* wp = reinterpret_cast<const raw16*>(Wp) + tile * (long long)(ksteps * AL / KS) * 64 + (long long)wave * cpw * AL * 64 + lane;
+  const int units = ksteps * AL / KS;
+  const bool grouped = frag_grouped(N, units);
+  const raw16* wp = reinterpret_cast<const raw16*>(Wp) + (frag_first((int)tile, units, grouped) + frag_behind(wave * cpw * AL, grouped)) * 64 + lane;
   const __bf16* xp = x + (long long)r * ldx + (long long)wave * cpw * (KS * 32) + q * 8;
 
   frag_cd acc[MT];
@@ -542,7 +550,7 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_rowsum_kernel(const void*
       _Pragma("unroll") for (int j = 0; j < MT; ++j)                                                                       \
           xr[slot][u][j] = *reinterpret_cast<const frag_ab*>(xp + (long long)j * 16 * ldx + ((long long)(chunk) * KS + u) * 32); \
     }                                                                                                                      \
-    _Pragma("unroll") for (int u = 0; u < AL; ++u) a[slot][u] = ldw16<true>(wp + ((long long)(chunk) * AL + u) * 64);      \
+    _Pragma("unroll") for (int u = 0; u < AL; ++u) a[slot][u] = ldw16<true>(wp + frag_behind((chunk) * AL + u, grouped) * 64); \
   } while (0)
 
 #define KV_CONSUME(slot)                                                                                                   \
@@ -762,8 +770,8 @@ int dispatch3_wide_wb(int epi, int nw, int wb, const Args& a) {
   return wb == 4 ? dispatch3_wide<MT, 4>(epi, nw, a) : wb == 8 ? dispatch3_wide<MT, 8>(epi, nw, a) : dispatch3_wide<MT, 16>(epi, nw, a);
 }
 
-// W[N, K] fp8 bytes (row-major) -> [N/16][K/64][64 lanes][16 bytes]: lane l of a tile holds
-// W[row l&15][k = 32*(2p+h) + 8*(l>>4) .. +8) for h = 0, 1 in its two 8-byte halves.
+// W[N, K] fp8 bytes (row-major) -> units [64 lanes][16 bytes] of a tile's 64 columns, in the order of fragments.h: lane l of
+// unit p holds W[row l&15][k = 32*(2p+h) + 8*(l>>4) .. +8) for h = 0, 1 in its two 8-byte halves.
 __global__ __launch_bounds__(256) void pack_weight_fp8_kernel(const unsigned char* __restrict__ W, unsigned char* __restrict__ Wp, int N, int K) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;  // one 16-byte unit per thread
   const int kpairs = K >> 6;
@@ -777,14 +785,15 @@ __global__ __launch_bounds__(256) void pack_weight_fp8_kernel(const unsigned cha
   const unsigned char* row = W + (nt * 16 + r) * (long long)K + (long long)p * 64 + q * 8;
   const unsigned long long lo = *reinterpret_cast<const unsigned long long*>(row);
   const unsigned long long hi = *reinterpret_cast<const unsigned long long*>(row + 32);
-  unsigned long long* dst = reinterpret_cast<unsigned long long*>(Wp + idx * 16);
+  const bool grouped = frag_grouped(N, kpairs);
+  unsigned long long* dst = reinterpret_cast<unsigned long long*>(Wp + ((frag_first((int)nt, kpairs, grouped) + frag_behind(p, grouped)) * 64 + lane) * 16);
   dst[0] = lo;
   dst[1] = hi;
 }
 
-// Re-order W[N, K] (row-major bf16) into MFMA fragment order [N/16][K/32][64 lanes][8]: every
-// wave-level load of the streaming kernels then reads one contiguous 1 KiB.
-__global__ __launch_bounds__(256) void pack_weight_kernel(const unsigned short* __restrict__ W, unsigned short* __restrict__ Wp, int N, int K) {
+// Re-order W[N, K] (row-major bf16) into MFMA fragments [64 lanes][8] of a tile and k-step: every
+// wave-level load of the streaming kernels then reads one contiguous 1 KiB.  whole_tiles: [N/16][K/32] of them, else in the order of fragments.h.
+__global__ __launch_bounds__(256) void pack_weight_kernel(const unsigned short* __restrict__ W, unsigned short* __restrict__ Wp, int N, int K, int whole_tiles) {
   typedef __attribute__((ext_vector_type(4))) unsigned short pk_us4;
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;  // one 16-byte fragment per thread
   const int ksteps = K >> 5;
@@ -796,7 +805,8 @@ __global__ __launch_bounds__(256) void pack_weight_kernel(const unsigned short* 
   const long long nt = tile / ksteps;
   const int r = lane & 15, q = lane >> 4;
   const pk_us4* src = reinterpret_cast<const pk_us4*>(W + (nt * 16 + r) * K + (long long)ks * 32 + q * 8);
-  pk_us4* dst = reinterpret_cast<pk_us4*>(Wp + idx * 8);
+  const bool grouped = !whole_tiles && frag_grouped(N, ksteps);
+  pk_us4* dst = reinterpret_cast<pk_us4*>(Wp + (grouped ? (frag_first((int)nt, ksteps, true) + frag_behind(ks, true)) * 64 + lane : idx) * 8);
   dst[0] = src[0];
   dst[1] = src[1];
 }
@@ -805,10 +815,10 @@ __global__ __launch_bounds__(256) void pack_weight_kernel(const unsigned short* 
 
 extern "C" {
 
-int kv_pack_weight(const void* W, void* Wp, int N, int K, hipStream_t stream) {
+int kv_pack_weight(const void* W, void* Wp, int N, int K, int whole_tiles, hipStream_t stream) {
   if ((N & 15) || (K & 31)) return -1;
   const long long total = (long long)(N >> 4) * (K >> 5) * 64;
-  hipLaunchKernelGGL(pack_weight_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, (const unsigned short*)W, (unsigned short*)Wp, N, K);
+  hipLaunchKernelGGL(pack_weight_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, (const unsigned short*)W, (unsigned short*)Wp, N, K, whole_tiles);
   return (int)hipGetLastError();
 }
 
@@ -939,15 +949,16 @@ int kv_stream_gemm_rowsum(const void* Wp, const void* x, int M, int N, int K, lo
   return -1;
 }
 
-// MXFP4 packed weights (pack_mxfp4 order: [N/16][K/128][64 lanes][16 B] + E8M0 scale words
-// [N/16][K/128][16 rows]) -> the bf16 fragment order of kv_pack_weight ([N/16][K/32][64][8]),
+// MXFP4 packed weights (units [64 lanes][16 B] of a tile's 128 columns in the order of fragments.h + E8M0 scale words
+// [N/16][K/128][16 rows]) -> the bf16 fragments of kv_pack_weight, in that order too,
 // exact (e2m1 times a power of two fits in bf16).  Wide steps expand a matrix into a scratch
 // buffer with this and run the bf16 tiled GEMM on it: 0.5 bytes read and 2 written per weight,
 // once per use, instead of one 128-row pass of the streaming kernel per 128 token rows.
 int kv_unpack_mxfp4(const void* Wp4, const void* scales, void* Wp, int N, int K, hipStream_t stream) {
   if (N <= 0 || K <= 0 || (N & 15) || (K & 127)) return -1;
   const long long total = (long long)(N >> 4) * (K >> 7) * 64;
-  hipLaunchKernelGGL(unpack_mxfp4_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, (const raw16*)Wp4, (const unsigned int*)scales, (raw16*)Wp, total);
+  hipLaunchKernelGGL(unpack_mxfp4_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, (const raw16*)Wp4, (const unsigned int*)scales, (raw16*)Wp, total, K >> 7,
+                     frag_grouped(N, K >> 7) ? 1 : 0, frag_grouped(N, K >> 5) ? 1 : 0);
   return (int)hipGetLastError();
 }
 

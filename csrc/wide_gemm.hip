@@ -4,7 +4,7 @@
 // Above ~128 token rows the projection stops being a weight-streaming problem: every weight
 // byte feeds hundreds of MACs, so both operands have to be re-used from LDS by many waves.
 // This kernel reads the SAME packed weights as the streaming kernels (csrc/stream_gemm.hip:
-// MFMA fragment order [N/16][K/32][64 lanes][8 bf16], FP8 [N/16][K/64][64][16 B]), so a model
+// MFMA fragments in the order of fragments.h), so a model
 // keeps ONE copy of its weights for every batch width.
 //
 //  * Workgroup tile BM tokens x BN features, BK = 64 per step, WM x WN waves; a wave owns
@@ -34,6 +34,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include "fragments.h"
 
 namespace {
 
@@ -252,7 +254,12 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_kernel(const Params p)
   const int s1 = s0 + p.stages_per_split < nst ? s0 + p.stages_per_split : nst;
   const int n = s1 - s0;
 
-  // ---- per-lane LDS-DMA source pointers of stage s0 (a stage further = + A_TILE / + XROW bytes)
+  // ---- per-lane LDS-DMA source pointers: of the weights' first stage (the others: stage_bytes), and of stage s0 of x (a stage further = + XROW bytes)
+  constexpr int UNITS = A_TILE / 1024;  // of a tile per stage
+  const int units = nst * UNITS;        // of a tile
+  const bool grouped = frag_grouped(p.N, units);
+  const long long block = frag_stride(grouped) * 1024;
+  auto stage_bytes = [&](int st) __attribute__((always_inline)) { return UNITS == FRAG_BLOCK ? st * block : (st / FRAG_BLOCK) * block + st % FRAG_BLOCK * 1024; };
   const unsigned char* asrc[PA_W];
   const unsigned char* xsrc[PX_W];
   int apc[PA_W];  // W piece of slot i of this wave
@@ -260,12 +267,7 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_kernel(const Params p)
   for (int i = 0; i < PA_W; ++i) {
     const int pc = wave + NW * i < PA ? wave + NW * i : wave + NW * i - PA;
     apc[i] = pc;
-    if constexpr (W8) {
-      asrc[i] = p.Wp + ((((long long)(n0 >> 4) + pc) * nst + s0) * 64 + lane) * 16;
-    } else {
-      const int ti = pc / KS, sl = pc % KS;
-      asrc[i] = p.Wp + ((((long long)(n0 >> 4) + ti) * (nst * KS) + (long long)s0 * KS + sl) * 64 + lane) * 16;
-    }
+    asrc[i] = p.Wp + (frag_first((n0 >> 4) + pc / UNITS, units, grouped) * 64 + lane) * 16 + pc % UNITS * 1024;
   }
 #pragma unroll
   for (int i = 0; i < PX_W; ++i) {
@@ -314,7 +316,7 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_kernel(const Params p)
   // of the stage at `src` into register set SET
 #define WG_MEMOP(m, SET, dst, src, st)                                                                                                   \
   do {                                                                                                                                  \
-    if ((m) < PA_W) dma16(asrc[(m) < PA_W ? (m) : 0] + (long long)(st) * A_TILE, (dst) + apc[(m) < PA_W ? (m) : 0] * 1024);             \
+    if ((m) < PA_W) dma16(asrc[(m) < PA_W ? (m) : 0] + stage_bytes(s0 + (st)), (dst) + apc[(m) < PA_W ? (m) : 0] * 1024);             \
     else if ((m) < PA_W + PX_W) dma16(xsrc[(m) >= PA_W && (m) < PA_W + PX_W ? (m) - PA_W : 0] + (long long)(st) * XROW, (dst) + A_BYTES + (wave + NW * ((m) - PA_W)) * 1024); \
     else if ((m) < G) dma4(ssrc + (long long)(st) * 64, (dst) + A_BYTES + X_BYTES + spc * 256);                                         \
     else if ((m) - G < AR) ra[SET][(m) >= G && (m) - G < AR ? (m) - G : 0] = *reinterpret_cast<const raw16*>((src) + a_off + ((m) - G) * 1024); \
@@ -458,7 +460,10 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_rs_kernel(const Params
   const int s1 = s0 + p.stages_per_split < nst ? s0 + p.stages_per_split : nst;
   const int n = s1 - s0;
 
-  // ---- this wave's LDS-DMA pieces: source pointer at stage s0, byte offset inside a ring stage
+  // ---- this wave's LDS-DMA pieces: source pointer at its first stage (of x: s0), byte offset inside a ring stage
+  constexpr int UNITS = A_TILE / 1024;  // of a tile per stage
+  const bool grouped = frag_grouped(p.N, nst * UNITS);
+  const long long block = frag_stride(grouped) * 1024;
   const unsigned char* src[GMAX];
   int doff[GMAX];
 #pragma unroll
@@ -468,12 +473,7 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_rs_kernel(const Params
     if (w_role) {
       if (i < GA) {
         const int pc = lw + NL * i;
-        if constexpr (W8) {
-          src[i] = p.Wp + ((((long long)(n0 >> 4) + pc) * nst + s0) * 64 + lane) * 16;
-        } else {
-          const int ti = pc / KS, sl = pc % KS;
-          src[i] = p.Wp + ((((long long)(n0 >> 4) + ti) * (nst * KS) + (long long)s0 * KS + sl) * 64 + lane) * 16;
-        }
+        src[i] = p.Wp + (frag_first((n0 >> 4) + pc / UNITS, nst * UNITS, grouped) * 64 + lane) * 16 + pc % UNITS * 1024;
         doff[i] = pc * 1024;
       }
     } else if (i < GX) {
@@ -487,7 +487,11 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_rs_kernel(const Params
     }
   }
   const int n_mine = w_role ? GA : GX;           // pieces per stage of this wave
-  const int sstride = w_role ? A_TILE : XROW;    // source bytes from one stage to the next
+  auto stage_bytes = [&](int st) __attribute__((always_inline)) {  // of its operand, behind the first
+    if (!w_role) return (long long)st * XROW;
+    st += s0;
+    return UNITS == FRAG_BLOCK ? st * block : (st / FRAG_BLOCK) * block + st % FRAG_BLOCK * 1024;
+  };
   const int depth = w_role ? NSW : NSX;
   unsigned char* const ring = w_role ? a_ring : x_ring;
   const int ring_stage = w_role ? A_BYTES : X_BYTES;
@@ -511,7 +515,7 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_rs_kernel(const Params
 #define RS_MEMOP(m, SET, lb, sa, sx, st)                                                                                          \
   do {                                                                                                                           \
     if ((m) < GMAX) {                                                                                                            \
-      if ((m) < n_mine) dma16(src[(m) < GMAX ? (m) : 0] + (long long)(st) * sstride, ring + (lb) * ring_stage + doff[(m) < GMAX ? (m) : 0]); \
+      if ((m) < n_mine) dma16(src[(m) < GMAX ? (m) : 0] + stage_bytes(st), ring + (lb) * ring_stage + doff[(m) < GMAX ? (m) : 0]); \
     } else if ((m) - GMAX < AR) {                                                                                                \
       ra[SET][(m) >= GMAX && (m) - GMAX < AR ? (m) - GMAX : 0] = *reinterpret_cast<const raw16*>((sa) + a_off + ((m) - GMAX) * 1024); \
     } else {                                                                                                                     \
@@ -749,8 +753,8 @@ int kv_wide_gemm_fp8a(const void* Wp, const void* x8, void* out, int M, int N, i
   return dispatch_tile<2>(bm, bn, variant, epi, p, stream);
 }
 
-// MXFP4 weights x FP8 activations on the block-scaled MFMA: the weights as kv_pack_mxfp4 lays them out (the streaming
-// kernels' layout: [N/16][K/128][64 lanes][16 B]) with their E8M0 block scales w_blk (int32 [N/16][K/128][16]) applied by
+// MXFP4 weights x FP8 activations on the block-scaled MFMA: the weights in the streaming
+// kernels' units [64 lanes][16 B] of 128 columns, in the order of fragments.h, with their E8M0 block scales w_blk (int32 [N/16][K/128][16]) applied by
 // the instruction itself; x8: e4m3 [M][ldx8] in NATURAL k order (kv_quantize_rows_fp8 with permute = 0), a_scale[M].
 // Tiles (256,128), (128,256), (128,128), variants 0 and 2.  K % 128 == 0, N % 64 == 0.
 int kv_wide_gemm_w4a8(const void* Wp4, const int* w_blk, const void* x8, void* out, int M, int N, int K, long long ldx8, long long ldy, int epi, int bm, int bn, int variant,

@@ -76,7 +76,7 @@ class FragmentLayout(RowLayout):
 
     @staticmethod
     def _pack(w: torch.Tensor) -> torch.Tensor:
-        return native().pack_weight(w.reshape(-1, w.shape[-1]).contiguous()).view(w.shape)
+        return native().pack_weight(w.reshape(-1, w.shape[-1]).contiguous(), True).view(w.shape)
 
     def heads(self, w: torch.Tensor, m: LatentSpec) -> torch.Tensor:
         return self._pack(w) if self.expands(m) else w

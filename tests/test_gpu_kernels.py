@@ -1544,6 +1544,72 @@ def test_tiled_gemm_every_tile_and_pipeline_shape(C, tile, variant):
     assert (sl.sum(0) - ref).abs().max().item() <= 1e-4 * ref.abs().max().item()
 
 
+@pytest.mark.parametrize("N,K", [(256, 64), (512, 448), (768, 1024), (320, 128), (256, 96)])
+def test_order_of_packed_matrices(C, N, K):
+    """Units of 1 KiB (16 features x 32 columns of bf16, 64 of e4m3): groups of 256 features have their units in pairs, tile by tile; matrices of another number of
+    features or an odd number of units, and those packed as whole tiles, have one tile behind another."""
+    torch.manual_seed(N)
+    for byte in (False, True):
+        cols = 64 if byte else 32
+        if K % cols:
+            continue
+        w = torch.randint(0, 256, (N, K), device="cuda").byte() if byte else torch.randn(N, K, device="cuda").bfloat16()
+        # a unit's lane 16 q + r: row r, 8 columns from 8 q on of each 32
+        tiles = w.view(N // 16, 16, K // cols, cols // 32, 4, 8).permute(0, 2, 4, 1, 3, 5).reshape(N // 16, K // cols, -1)
+        even = N % 256 == 0 and K // cols % 2 == 0
+        want = tiles.view(N // 256, 16, K // cols // 2, -1).transpose(1, 2) if even else tiles
+        got = C.pack_weight_fp8(w) if byte else C.pack_weight(w)
+        assert torch.equal(got.flatten(), want.reshape(-1))
+        if not byte:
+            assert torch.equal(C.pack_weight(w, True).flatten(), tiles.reshape(-1))
+
+
+@pytest.mark.parametrize("K", [1024, 2048 + 1024])
+def test_products_of_either_order_are_the_same_bits(C, K):
+    """A matrix of 512 outputs (groups of tiles), and the same with 128 more (tile by tile): every kernel that multiplies packed weights."""
+    from kvmini.ops import hip_ops as ops
+
+    torch.manual_seed(K)
+    w = torch.cat(((torch.randn(512, K, device="cuda") * 0.1).bfloat16(), torch.zeros(128, K, device="cuda").bfloat16()))
+    pairs = [tuple(ops.PackedLinear(w[:n], fp8=bits == 8, mxfp4=bits == 4) for n in (512, 640)) for bits in (16, 8, 4)]
+
+    def same(run, m, pair, splits=0):
+        out = []
+        for p in pair:
+            y = torch.full((splits, m, p.n) if splits else (m, p.n), float("nan"), device="cuda", dtype=torch.float32 if splits else torch.bfloat16)
+            run(p, y)
+            out.append(y[..., :512])
+        assert torch.equal(*out) and not out[0].isnan().any()
+
+    for m in (16, 64, 128):
+        x = torch.randn(m, K, device="cuda").bfloat16()
+        for pair in pairs:
+            bits, nst = pair[0].bits, K // 256
+            for nw in (4, 8):
+                same(lambda p, y: C.stream_gemm3(p.wp, p.n, K, x, y, 0, 2, 1, nst, None, 0.0, p.wscale, nw, bits if bits == 4 else 0), m, pair)
+                same(lambda p, y: C.stream_gemm3(p.wp, p.n, K, x, y, 1, 2, 2, nst // 2, None, 0.0, p.wscale, nw, bits if bits == 4 else 0), m, pair, 2)
+            if bits > 4 and m <= 64:
+                same(lambda p, y: C.stream_gemm(p.wp, p.n, K, x, y, 0, 4, 1, K // 128, None, 0.0, p.wscale), m, pair)
+                same(lambda p, y: C.stream_gemm_rowsum(p.wp, p.n, K, x, y, False, p.wscale, 2), m, pair)
+    x = torch.randn(200, K, device="cuda").bfloat16()
+    bf16, fp8, mxfp4 = pairs
+    for variant in (0, 2, 4):
+        same(lambda p, y: C.wide_gemm(p.wp, p.n, K, x, y, 1, 128, 128, variant, 2, K // 128, None, 0.0, None, True), 200, bf16, 2)
+        same(lambda p, y: C.wide_gemm(p.wp, p.n, K, x, y, 0, 128, 128, variant, 1, K // 64, None, 0.0, p.wscale, True), 200, fp8)
+    same(lambda p, y: C.wide_gemm(p.wp, p.n, K, x, y, 0, 256, 128, 1, 1, K // 32, None, 0.0, None, True), 200, bf16)
+    same(lambda p, y: C.dense_panels(p.wp, p.n, K, x, y, 0, 96, 1, 64, None, 0.0), 200, bf16)
+    same(lambda p, y: C.narrow_tiles(p.wp, p.n, K, x, y, 1, 64, 2, K // 128, None, 0.0), 200, bf16, 2)
+    for pair, key in ((fp8, "w_scale"), (mxfp4, "blocks")):
+        x8, scale = C.quantize_rows_fp8(x, pair is fp8)
+        same(lambda p, y: C.dense_panels(p.wp, p.n, K, x8, y, 0, 96, 1, 64, None, 0.0, x_scale=scale, **{key: p.wscale}), 200, pair)
+        same(lambda p, y: C.narrow_tiles(p.wp, p.n, K, x8, y, 1, 64, 2, K // 256, None, 0.0, x_scale=scale, **{key: p.wscale}), 200, pair, 2)
+        args = (x8, scale)
+        if pair is fp8:
+            same(lambda p, y: C.wide_gemm_fp8a(p.wp, p.n, K, *args, y, 1, 128, 128, 0, 2, K // 256, None, 0.0, p.wscale, True), 200, pair, 2)
+        else:
+            same(lambda p, y: C.wide_gemm_w4a8(p.wp, p.wscale, p.n, K, *args, y, 1, 128, 128, 0, 2, K // 256, None, 0.0, True), 200, pair, 2)
+
+
 @pytest.mark.parametrize("M,N,K,cut", [
     (1, 32, 64, (32, 1, 32)), (129, 96, 64, (256, 0, 96)), (255, 256, 128, (256, 1, 256)), (300, 544, 192, (64, 2, 224)), (257, 448, 320, (160, 1, 32)),
     (1000, 288, 384, (192, 2, 256)), (513, 1024, 448, (128, 3, 96)), (448, 512, 832, (224, 1, 192)),
