@@ -122,7 +122,7 @@ __device__ __forceinline__ void attend_tile(const bf16raw* k_img, const bf16raw*
   float mx = sc[0];
 #pragma unroll
   for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = lanes::meet<32>(mx, lanes::Max{});
   const float m_old = m_run, m_new = fmaxf(m_old, mx);
   const float m_sub = m_new > -1e29f ? m_new : 1e30f;  // (a query none of whose keys have come up yet: nothing counts)
   float psum = 0.f;

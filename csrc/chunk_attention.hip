@@ -170,7 +170,7 @@ __global__ __launch_bounds__(64 * NW, DV <= 128 ? 2 : 1) void chunk_prefill_kern
     });
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
-  const float l = l_run + __shfl_xor(l_run, 32, 64);
+  const float l = lanes::meet<32>(l_run, lanes::Sum{});
   if (!head_on || lr >= nq) return;
   float f = a.out_scale / l;
   const long long row = row0 + lr;
@@ -424,8 +424,8 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
       sc[r] = ((k0 + r >= first || k0 + r < a.see.keep) && k0 + r <= pos) ? v : -1e30f;
     }
     float mx = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = lanes::meet<16>(mx, lanes::Max{});
+    mx = lanes::meet<32>(mx, lanes::Max{});
     const float m_new = fmaxf(m_run, mx);  // (a block holds at least one visible key)
     const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
     typedef __attribute__((ext_vector_type(4))) __bf16 bf4;
@@ -456,8 +456,8 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
       o[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, __builtin_bit_cast(frag_b64, vf), o[n], 0, 0, 0);
     }
   }
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = lanes::meet<16>(l_run, lanes::Sum{});
+  l_run = lanes::meet<32>(l_run, lanes::Sum{});
   if (lq == 0) { ml[wave][lr][0] = m_run; ml[wave][lr][1] = l_run; }
   float* os = reinterpret_cast<float*>(work) + wave * 16 * DV;  // (the wave's own LDS: its reads above are done)
 #pragma unroll

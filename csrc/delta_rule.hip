@@ -267,8 +267,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
       s[r] *= d[r];
       xk += s[r] * k[r];
     }
-#pragma unroll
-    for (int m = CPW; m < 64; m <<= 1) xk += __shfl_xor(xk, m, 64);
+    xk = lanes::meet_up<CPW, 64>(xk, lanes::Sum{});
     const float u = bi * (vi - xk);
     float xq = 0.f;
 #pragma unroll
@@ -276,8 +275,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
       s[r] += k[r] * u;
       xq += s[r] * q[r];
     }
-#pragma unroll
-    for (int m = CPW; m < 64; m <<= 1) xq += __shfl_xor(xq, m, 64);
+    xq = lanes::meet_up<CPW, 64>(xq, lanes::Sum{});
     if (rgi == 0 && on) o[(row * heads + h) * vdim + col] = xq;
   }
 #undef KV_FETCH
@@ -303,8 +301,7 @@ __global__ __launch_bounds__(256) void delta_out_kernel(const float* __restrict_
       const float4 v = ld4(src + d);
       ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
     }
-#pragma unroll
-    for (int m = 1; m < LPR; m <<= 1) ss += __shfl_xor(ss, m, 64);
+    ss = lanes::meet_up<1, LPR>(ss, lanes::Sum{});
     const float rs = a.out_scale / sqrtf(ss / (float)a.vdim + a.eps);
     for (int d = 4 * lane; d < a.vdim; d += 4 * LPR) {
       float4 v = ld4(src + d);
@@ -315,8 +312,7 @@ __global__ __launch_bounds__(256) void delta_out_kernel(const float* __restrict_
   } else {
     float ss = 0.f;
     for (int d = lane; d < a.vdim; d += LPR) ss += src[d] * src[d];
-#pragma unroll
-    for (int m = 1; m < LPR; m <<= 1) ss += __shfl_xor(ss, m, 64);
+    ss = lanes::meet_up<1, LPR>(ss, lanes::Sum{});
     const float rs = a.out_scale / sqrtf(ss / (float)a.vdim + a.eps);
     for (int d = lane; d < a.vdim; d += LPR) st(dst + d, src[d] * rs * a.o_norm[d] * sigmoid(ld(gl + d)));
   }

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lanes.h"
+
 namespace elem {
 
 typedef unsigned short bf16raw;
@@ -30,16 +32,8 @@ __device__ inline void st4(bf16raw* p, float4 v) {
   *reinterpret_cast<ushort4*>(p) = o;
 }
 
-__device__ inline float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-__device__ inline float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
+__device__ inline float wave_sum(float v) { return lanes::sum(v); }
+__device__ inline float wave_max(float v) { return lanes::max(v); }
 
 // On the hardware's exponential, logarithm and reciprocal (about one unit in the last place each).
 __device__ inline float fast_exp(float x) { return __builtin_amdgcn_exp2f(1.4426950408889634f * x); }

@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "fragments.h"
+#include "lanes.h"
 #include "quantise.h"
 
 namespace {
@@ -273,10 +274,7 @@ __device__ inline bf16x8 kv_store8(void* base, long long off, bf16x8 v, float in
   }
 }
 
-__device__ inline float wave_sum(float v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
+__device__ inline float wave_sum(float v) { return lanes::sum(v); }
 
 // Sum of the `parts` partial sums of squares of one token row, by a whole wave (lane-strided loads
 // + butterfly; every lane gets the total).  Rows carry 8 parts from the residual kernel and
@@ -570,8 +568,7 @@ __global__ __launch_bounds__(512) void residual_quantise_kernel(const float* __r
     ss = wave_sum(ss);
     if (lane == 0 && part < parts) ss_part[(long long)t * parts + part] = ss;
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+  amax = lanes::max(amax);
   if (lane == 0) red[wave] = amax;
   __syncthreads();
   for (int w = 0; w < waves; ++w) amax = fmaxf(amax, red[w]);
@@ -2580,11 +2577,9 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
         m = __hip_atomic_load(part_ml + ((pbase + s2) * REP + h) * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         den = __hip_atomic_load(part_ml + ((pbase + s2) * REP + h) * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-      float mx = m;
-      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      const float mx = lanes::max(m);
       const float c = s2 < eff ? __builtin_amdgcn_exp2f(m - mx) : 0.f;
-      float tot = den * c;
-      for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o, 64);
+      const float tot = lanes::sum(den * c);
       w_lds[h][s2] = tot > 0.f ? c / tot : 0.f;
     }
     __syncthreads();
@@ -2664,17 +2659,14 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const unsigned short* __re
     if (f > best) { best = f; besti = i; }
   }
   // first-index tie-break, like torch.argmax
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(best, o, 64);
-    int oi = __shfl_xor(besti, o, 64);
-    if (ov > best || (ov == best && oi < besti)) { best = ov; besti = oi; }
-  }
+  lanes::best(best, besti);
   if ((tid & 63) == 0) { bv[tid >> 6] = best; bi[tid >> 6] = besti; }
   __syncthreads();
-  if (tid == 0) {
-    for (int w = 1; w < 16; ++w)
-      if (bv[w] > best || (bv[w] == best && bi[w] < besti)) { best = bv[w]; besti = bi[w]; }
-    out[r] = besti;
+  if (tid < 64) {
+    best = bv[tid & 15];
+    besti = bi[tid & 15];
+    lanes::best_of<8>(best, besti); lanes::best_of<4>(best, besti); lanes::best_of<2>(best, besti); lanes::best_of<1>(best, besti);
+    if (tid == 0) out[r] = besti;
   }
 }
 
@@ -2760,8 +2752,7 @@ __global__ __launch_bounds__(256) void slab_add_bias_kernel(float* __restrict__ 
   if (row_ss != nullptr) {
     float ssum = 0.f;
     for (int i = tid; i < ss_parts; i += 256) ssum += row_ss[(long long)t * ss_parts + i];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ssum += __shfl_xor(ssum, o, 64);
+    ssum = lanes::sum(ssum);
     if ((tid & 63) == 0) red[tid >> 6] = ssum;
     __syncthreads();
     f = sqrtf((red[0] + red[1] + red[2] + red[3]) * inv_h + eps);

@@ -123,12 +123,7 @@ __device__ inline void choose(const float* z, const float (&corr)[NC], bool pad,
 #pragma unroll
     for (int i = 0; i < NC; ++i)
       if (c[i] > best) { best = c[i]; idx = lane + 64 * i; }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float v = __shfl_xor(best, o, 64);
-      const int j = __shfl_xor(idx, o, 64);
-      if (v > best || (v == best && j < idx)) { best = v; idx = j; }
-    }
+    lanes::best(best, idx);
     if (lane == k) mine = idx;
 #pragma unroll
     for (int i = 0; i < NC; ++i)

@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void latent_prefill_kernel(const bf16raw* __re
     attend_tile<DK, DV>(pf_lds + buf * KT, pf_lds + 3 * KT + buf * VT, qa, o, m_run, l_run, a.scale_log2e, edge, qpos - kb, q_first - kb, st);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece may be in flight when the workgroup gives its LDS back
-  const float l = l_run + __shfl_xor(l_run, 32, 64);
+  const float l = lanes::meet<32>(l_run, lanes::Sum{});
   if (!on || w0 + lr >= nq) return;
   const long long row = row0 + qi;
   const bf16raw* gate = proj + row * a.ld_gate + a.gate_off;
@@ -429,8 +429,8 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(const bf16raw* __res
 #pragma unroll
       for (int r = 0; r < 4; ++r) sc[r] = (k0 + r >= first && k0 + r <= pos) ? st[r] * a.scale_log2e : -1e30f;
       mx = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = lanes::meet<16>(mx, lanes::Max{});
+      mx = lanes::meet<32>(mx, lanes::Max{});
       if (b == me && !staged) m_run = mx;
       if (__builtin_amdgcn_ballot_w64(mx > m_run + 24.f) != 0) {
         lds_landed(va[0]);
@@ -476,8 +476,8 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(const bf16raw* __res
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[n][r] *= cr[r];
   }
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = lanes::meet<16>(l_run, lanes::Sum{});
+  l_run = lanes::meet<32>(l_run, lanes::Sum{});
   if (lq == 0) { ml[wave][lr][0] = m_run; ml[wave][lr][1] = l_run; }
   float* os = reinterpret_cast<float*>(mine);  // (the wave's own LDS: its reads above are done, nothing is in flight)
 #pragma unroll

@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lanes.h"
 #include "quantise.h"
 
 namespace {
@@ -56,8 +57,7 @@ __global__ __launch_bounds__(256) void quantize_rows_fp8_kernel(const unsigned s
       amax = fmaxf(amax, fabsf(bf2f((unsigned short)(v[j] >> 16))));
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+  amax = lanes::max(amax);
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));

@@ -427,8 +427,7 @@ __global__ __launch_bounds__(256) void norm_rope_write_vec_kernel(const bf16raw*
       float ss = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
-#pragma unroll
-      for (int m = 1; m < LPR; m <<= 1) ss += __shfl_xor(ss, m, 64);
+      ss = lanes::meet_up<1, LPR>(ss, lanes::Sum{});
       const float rs = 1.f / sqrtf(ss / (float)n + a.eps);
       if (on) {
         float nv[8];
@@ -499,8 +498,7 @@ __global__ __launch_bounds__(256) void key_value_write_vec_kernel(const bf16raw*
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
-#pragma unroll
-  for (int m = 1; m < LPR; m <<= 1) ss += __shfl_xor(ss, m, 64);
+  ss = lanes::meet_up<1, LPR>(ss, lanes::Sum{});
   const float rs = 1.f / sqrtf(ss / (float)a.dim + a.eps);
   float w[8];  // what turns: the normed query, or the key with its gains
 #pragma unroll
@@ -765,12 +763,7 @@ __global__ __launch_bounds__(1024) void argmax_f32_kernel(const float* __restric
     const float v = row[i];
     if (v > best || (v == best && i < idx)) { best = v; idx = i; }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float v = __shfl_xor(best, o, 64);
-    const int i = __shfl_xor(idx, o, 64);
-    if (v > best || (v == best && i < idx)) { best = v; idx = i; }
-  }
+  lanes::best(best, idx);
   if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = best; bi[threadIdx.x >> 6] = idx; }
   __syncthreads();
   if (threadIdx.x == 0) {

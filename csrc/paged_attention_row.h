@@ -228,8 +228,8 @@
 #pragma unroll
     for (int j = 0; j < DP; ++j) {
       float v = acc[h][j];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
+      v = lanes::meet<16>(v, lanes::Sum{});
+      v = lanes::meet<32>(v, lanes::Sum{});
       acc[h][j] = v;
     }
   if (pv_tg == 0) {

@@ -386,8 +386,7 @@ __global__ __launch_bounds__(256, NT <= 2 ? 3 : 2) void retention_out_kernel(con
     float ss = 0.f;
 #pragma unroll
     for (int y = 0; y < NT; ++y) ss += live[y] ? o[u >> 2][y][u & 3] * o[u >> 2][y][u & 3] : 0.f;
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) ss += __shfl_xor(ss, m, 64);
+    ss = lanes::meet_up<1, 16>(ss, lanes::Sum{});
     if (lr == 0) sums[wave][16 * (u >> 2) + 4 * lq + (u & 3)] = ss;
   }
   __syncthreads();

@@ -28,6 +28,7 @@
 #include <stdint.h>
 
 #include "fragments.h"
+#include "lanes.h"
 
 namespace {
 
@@ -118,15 +119,14 @@ __global__ __launch_bounds__(256) void unpack_mxfp4_kernel(const raw16* __restri
 // 1/rms of the token rows a workgroup's epilogue scales, left in LDS: row_ss holds `ss_parts` partial
 // sums of squares per row — 8 from the residual kernel (512-column segments), hidden/16 from the
 // row-parallel projections that update the residual themselves (one per feature tile) — so a row
-// is summed by a whole wave (lane-strided loads, butterfly), not by one lane in a serial loop.
+// is summed by a whole wave (lane-strided loads, then over the lanes), not by one lane in a serial loop.
 template <int ROWS, int NW>
 __device__ inline void row_scales_to_lds(float* rs_lds, const float* __restrict__ row_ss, int ss_parts, float inv_k, float eps, int wave, int lane) {
   for (int row = wave; row < ROWS; row += NW) {
     const float* p = row_ss + (long long)row * ss_parts;
     float ssum = 0.f;
     for (int i = lane; i < ss_parts; i += 64) ssum += p[i];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ssum += __shfl_xor(ssum, o, 64);
+    ssum = lanes::sum(ssum);
     if (lane == 0) rs_lds[row] = rsqrtf(ssum * inv_k + eps);
   }
 }
