@@ -19,6 +19,11 @@ template <typename T> __device__ inline void st(T* p, float v);
 template <> __device__ inline void st<float>(float* p, float v) { *p = v; }
 template <> __device__ inline void st<bf16raw>(bf16raw* p, float v) { *p = f2bf(v); }
 
+// an element's bits as they are loaded, and its value: what is loaded long before it is used is not waited for by its conversion
+__device__ inline unsigned int raw(const float* p) { return __float_as_uint(*p); }
+__device__ inline unsigned int raw(const bf16raw* p) { return *p; }
+template <typename T> __device__ inline float number(unsigned int v) { return __uint_as_float(sizeof(T) == 2 ? v << 16 : v); }
+
 // four consecutive elements (aligned to four)
 __device__ inline float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ inline float4 ld4(const bf16raw* p) {

@@ -1,6 +1,7 @@
 // Reductions over the lanes of a wave without LDS: lanes 1, 2, 4 and 8 apart by DPP moves, 16 and 32 apart by the swaps of rows and halves.  A shuffle through
 // LDS (ds_bpermute) is some 100 cycles until its answer is there, six of them in a row 0.3 us of a launch that has two or three such sums and takes 3 to 5 in all; these
-// take 60 cycles together.  The same pairs in the same order as a butterfly of shuffles: the same bits.
+// take 60 cycles together.  The same pairs in the same order as a butterfly of shuffles: the same bits, but for sums of one product a lane, of which shuffles
+// let the compiler fuse a lane's own with what it got: either half of the lanes had a rounding less in its own number and the other's.
 #pragma once
 #include <hip/hip_runtime.h>
 

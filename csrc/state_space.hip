@@ -63,14 +63,17 @@ __device__ inline float conv_silu(const KvsArgs& a, const T* __restrict__ proj, 
 __device__ inline float step_size(const KvsArgs& a, float raw, int h) { return softplus(raw + a.dt_bias[h]); }
 __device__ inline float log2_decay(const KvsArgs& a, float dt, int h) { return -1.4426950408889634f * fast_exp(a.a_log[h]) * dt; }
 
-// ---- single tokens: grid (listed rows, heads); thread = a group of state rows x 4 columns
-template <typename T>
+// ---- single tokens: grid (listed rows, heads); thread = a group of state rows x 4 columns.  Loads answer in the order they were asked for: the convolution's inputs are
+// asked for ahead of the state, and worked out while the state is on its way.  TAPS: those of the convolution (0: a.taps).  64 rows of 64 heads of 128 x 64
+// 76 -> 64 us (52 for the state's bytes).
+template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void space_step_kernel(const T* __restrict__ proj, T* __restrict__ ring, float* __restrict__ y, const int* __restrict__ rows, KvsArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const long long t = rows[blockIdx.x];
   const int h = blockIdx.y, tid = threadIdx.x;
-  if (t < 0 || a.tok_kind[t] != 1) return;  // unused entry, or a padding row
-  const int pos = a.positions[t], slot = a.tok_seq[t];
+  if (t < 0) return;  // unused entry
+  const int kind = a.tok_kind[t], pos = a.positions[t], slot = a.tok_seq[t];
+  if (kind != 1) return;  // a padding row
   const int rep = a.heads / a.groups, g = h / rep, inner = a.heads * a.vdim;
   const int nc = a.dvp >> 2, nrg = 256 / nc;
   const int rg = tid / nc, col = (tid - rg * nc) * 4;
@@ -79,39 +82,89 @@ __global__ __launch_bounds__(256) void space_step_kernel(const T* __restrict__ p
   float* cs = bs + a.dimp;     // [dimp]
   float* xs = cs + a.dimp;     // [dvp]
   float* red = xs + a.dvp;     // [nrg][dvp]
-  float* st = a.state + ((long long)slot * a.heads + h) * a.dimp * a.dvp + col;
+  const int b0 = inner + g * a.dim, c0 = b0 + a.groups * a.dim, items = 2 * a.dimp + a.dvp;
+  struct Item { int which, d, c; bool there; };
+  auto item = [&](int i) {  // of b, c, x, dealt over the threads; behind their sizes: zeros
+    Item it;
+    it.which = i < a.dimp ? 0 : i < 2 * a.dimp ? 1 : 2;
+    it.d = i - it.which * a.dimp;
+    it.there = it.d < (it.which == 2 ? a.vdim : a.dim);
+    it.c = (it.which == 0 ? b0 : it.which == 1 ? c0 : h * a.vdim) + (it.there ? it.d : 0);
+    return it;
+  };
+  const T* pr = proj + t * a.ldp + a.x_off;
+  // the first items of a thread, as loaded: no branches and no conversions, which would wait for them
+  constexpr int EARLY = TAPS > 0 ? 2 : 0, SIZE = TAPS > 0 ? TAPS : 1;
+  unsigned int in[2][SIZE];
+  float w[2][SIZE], bias[2];
+#pragma unroll
+  for (int e = 0; e < EARLY; ++e) {
+    const int c = item(tid + 256 * e < items ? tid + 256 * e : items - 1).c;
+    bias[e] = a.conv_b[c];
+    in[e][0] = raw(pr + c);
+    w[e][0] = a.conv_w[(TAPS - 1) * a.channels + c];
+#pragma unroll
+    for (int m = 1; m < TAPS; ++m) {
+      in[e][m] = raw(ring + ((long long)slot * TAPS + (m <= pos ? pos - m : 0) % TAPS) * a.channels + c);
+      w[e][m] = a.conv_w[(TAPS - 1 - m) * a.channels + c];
+    }
+  }
+  const unsigned int dt_of = raw(proj + t * a.ldp + a.dt_off + h);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // rows rg, rg + nrg, ... of the state, U at a time (behind the last one: the first again, which nothing uses)
+  float* st = a.state + ((long long)slot * a.heads + h) * a.dimp * a.dvp + (on && rg < a.dimp ? rg * a.dvp + col : 0);
+  const int stride = nrg * a.dvp, mine = on && rg < a.dimp ? (a.dimp - rg + nrg - 1) / nrg : 0, most = (a.dimp + nrg - 1) / nrg;
   constexpr int U = 8;
   float4 s[U];
-  auto fetch = [&](int r0) __attribute__((always_inline)) {
+  auto fetch = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int r = r0 + u * nrg;
-      s[u] = on && r < a.dimp && pos > 0 ? ld4(st + (long long)r * a.dvp) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+    for (int u = 0; u < U; ++u) s[u] = ld4(st + (i0 + u < mine ? (i0 + u) * stride : 0));
   };
-  fetch(rg);
-  const float dt = step_size(a, ld(proj + t * a.ldp + a.dt_off + h), h);
+  fetch(0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  const float dt = step_size(a, number<T>(dt_of), h);
   const float decay = __builtin_amdgcn_exp2f(log2_decay(a, dt, h));
-  const int b0 = inner + g * a.dim, c0 = b0 + a.groups * a.dim;
-  for (int i = tid; i < 2 * a.dimp + a.dvp; i += 256) {
-    const int which = i < a.dimp ? 0 : i < 2 * a.dimp ? 1 : 2, d = i - which * a.dimp;
-    float v = 0.f;
-    if (d < (which == 2 ? a.vdim : a.dim)) v = conv_silu<T>(a, proj, ring, t, pos, 0, slot, (which == 0 ? b0 : which == 1 ? c0 : h * a.vdim) + d);
-    sm[i] = which == 0 ? v * dt : v;
+  // the ring entry of this position was last used for position pos - taps, which nobody reads any more
+  T* rw = ring + ((long long)slot * a.taps + pos % a.taps) * a.channels;
+  auto keep = [&](int i, const Item& it, float v) {
+    v = it.there ? v : 0.f;
+    sm[i] = it.which == 0 ? v * dt : v;
+  };
+#pragma unroll
+  for (int e = 0; e < EARLY; ++e) {
+    const int i = tid + 256 * e;
+    if (i >= items) continue;
+    const Item it = item(i);
+    float v = bias[e] + w[e][0] * number<T>(in[e][0]);
+#pragma unroll
+    for (int m = 1; m < TAPS; ++m) v += w[e][m] * (m <= pos ? number<T>(in[e][m]) : 0.f);
+    keep(i, it, rounded<T>(silu(v)));
+    if (it.there && (it.which == 2 || h % rep == 0)) elem::st(rw + it.c, number<T>(in[e][0]));
+  }
+  for (int i = tid + 256 * EARLY; i < items; i += 256) {
+    const Item it = item(i);
+    keep(i, it, conv_silu<T>(a, proj, ring, t, pos, 0, slot, it.c));
+    if (it.there && (it.which == 2 || h % rep == 0)) rw[it.c] = pr[it.c];
   }
   __syncthreads();
   const float4 x = on ? ld4(xs + col) : make_float4(0.f, 0.f, 0.f, 0.f);
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int r0 = rg; r0 < a.dimp; r0 += U * nrg) {
-    if (r0 != rg) fetch(r0);
+  for (int i0 = 0; i0 < most; i0 += U) {
+    if (i0) fetch(i0);
+    if (pos == 0) {  // (here and not around the loads: where ways with and without them meet, all of them would be waited for)
+#pragma unroll
+      for (int u = 0; u < U; ++u) s[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int r = r0 + u * nrg;
-      if (on && r < a.dimp) {
+      if (i0 + u < mine) {
+        const int r = rg + (i0 + u) * nrg;
         const float b = bs[r], c = cs[r];
         s[u].x = s[u].x * decay + b * x.x; s[u].y = s[u].y * decay + b * x.y; s[u].z = s[u].z * decay + b * x.z; s[u].w = s[u].w * decay + b * x.w;
         o.x += c * s[u].x; o.y += c * s[u].y; o.z += c * s[u].z; o.w += c * s[u].w;
-        st4(st + (long long)r * a.dvp, s[u]);
+        st4(st + (i0 + u) * stride, s[u]);
       }
     }
   }
@@ -122,15 +175,6 @@ __global__ __launch_bounds__(256) void space_step_kernel(const T* __restrict__ p
     for (int r = 0; r < nrg; ++r) v += red[r * a.dvp + d];
     y[t * inner + h * a.vdim + d] = v;
   }
-  // the ring entry of this position was last used for position pos - taps, which nobody reads any more
-  T* rw = ring + ((long long)slot * a.taps + pos % a.taps) * a.channels;
-  const T* pr = proj + t * a.ldp + a.x_off;
-  for (int d = tid; d < a.vdim; d += 256) rw[h * a.vdim + d] = pr[h * a.vdim + d];
-  if (h % rep == 0)
-    for (int d = tid; d < a.dim; d += 256) {
-      rw[b0 + d] = pr[b0 + d];
-      rw[c0 + d] = pr[c0 + d];
-    }
 }
 
 // ---- portions: convolution of all channels (VEC per thread, RUN tokens one after the other); the last row of workgroups: steps and decays.
@@ -770,7 +814,8 @@ bool args_ok(const KvsArgs& a) {
 template <typename T>
 int step(const KvsArgs& a, const void* proj, void* ring, float* y, const int* rows, int n_rows, hipStream_t s) {
   const size_t lds = (size_t)(2 * a.dimp + a.dvp + 256 / (a.dvp / 4) * a.dvp) * 4;
-  hipLaunchKernelGGL((space_step_kernel<T>), dim3(n_rows, a.heads), dim3(256), lds, s, (const T*)proj, (T*)ring, y, rows, a);
+  if (a.taps == 4) hipLaunchKernelGGL((space_step_kernel<T, 4>), dim3(n_rows, a.heads), dim3(256), lds, s, (const T*)proj, (T*)ring, y, rows, a);
+  else hipLaunchKernelGGL((space_step_kernel<T, 0>), dim3(n_rows, a.heads), dim3(256), lds, s, (const T*)proj, (T*)ring, y, rows, a);
   return (int)hipGetLastError();
 }
 

@@ -303,6 +303,13 @@ def test_retention_alone(backend, heads, dim, vdim, rot, decay):
 
 
 @pytest.mark.parametrize("backend", BACKENDS)
+@pytest.mark.parametrize("heads,dim,vdim,rot,decay", [(2, 256, 64, 64, (0.97, 0.99)), (1, 260, 64, 8, (0.98,)), (1, 16, 1024, 16, (0.95,)), (1, 20, 1000, 8, (0.9,)), (2, 92, 100, 48, (0.9, 1.0))])
+def test_retention_of_heads_about_what_one_step_holds(backend, heads, dim, vdim, rot, decay):
+    """Single tokens go by a kernel that holds up to 16 state rows of each of its 256 threads' columns: just as many, a few more, and rows and columns that do not come out even."""
+    test_retention_alone(backend, heads, dim, vdim, rot, decay)
+
+
+@pytest.mark.parametrize("backend", BACKENDS)
 @pytest.mark.parametrize("experts,top,width,ff,shared,scale,t", [(5, 2, 75, 36, 50, 1.7, 20), (16, 1, 128, 64, 64, 1.0, 1), (70, 6, 300, 100, 0, 0.5, 77), (3, 3, 256, 40, 300, 2.0, 128), (64, 4, 140, 72, 130, 1.3, 200),
                                                                  (8, 4, 256, 96, 30, 1.0, 333), (300, 8, 64, 24, 40, 3.0, 150), (1, 1, 64, 200, 20, 0.7, 140), (79, 5, 64, 40, 24, 1.0, 33)])
 def test_experts_by_softmax_with_a_shared_one_alone(backend, experts, top, width, ff, shared, scale, t):
