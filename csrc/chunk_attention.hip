@@ -18,6 +18,8 @@
 // the others, so that query . row is the score but for the factor, which multiplies it afterwards; the same row, staged once, is the value.
 // Epilogue: 1 / sum, out_scale and the gate: sigmoid(gate[row][head]) (gated 1) or sigmoid(gate[row][head vdim + i]) (2).
 
+#include <type_traits>
+
 #include "attn_tiles.h"
 
 namespace {
@@ -225,7 +227,9 @@ int launch_prefill(const void* q, const void* kc, const void* vc, const void* ga
 // grid (listed rows, key heads x groups of 16 query heads, shares): the keys a row sees, in blocks of 16 dealt out to the waves of its
 // workgroups.  A wave multiplies a K block, straight from memory as the A operand, with the up to 16 query heads as columns
 // (S^T: a lane owns one head and 4 keys), and the weights, already in the A layout of mfma_f32_16x16x16_bf16, with the V block, which
-// passes through a piece of LDS of the wave's own for the transposed reads.  K / V of the next block are in flight meanwhile.
+// passes through a piece of LDS of the wave's own for the transposed reads.  K / V of the next block (separate keys and values: of two) are in flight meanwhile,
+// the first ones since before the queries were normed.  6 rows of 820 tokens, heads of 64: 11.4 -> 9.8 us; 3 rows of 2000, four layers of a hybrid 325 -> 313; with CUs full
+// of workgroups no difference (61 rows of 8 heads of 128 x 865 tokens 63 us, 3.4 TB/s).
 // FUSED: the kernel also does what norm_rope_write_kernel does for the row (query / key norm, rotation, K / V write).
 // RT >= 0 (one row is key and value): the keys' operands come out of the piece of LDS, too.
 // SPLIT: partial results (maximum, sum, unnormalised output per head) go to a workspace for chunk_decode_combine_kernel.
@@ -243,6 +247,8 @@ struct ChunkDecodeArgs {
   const float* bias; const float* q_norm; const float* k_norm; const float* cos_t; const float* sin_t;
   float* part;  // SPLIT: [row][head][share][2 + DV]
 };
+
+typedef const __attribute__((address_space(4))) int const_int;  // memory that nobody writes while the kernel runs
 
 template <int DK, int DV, int NW, bool FUSED, bool SPLIT, bool REL, int RT>
 __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __restrict__ q, const bf16raw* __restrict__ proj, bf16raw* k_cache, bf16raw* v_cache,
@@ -270,6 +276,43 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
   const int me = blockIdx.z * NW + wave;
   const int* __restrict__ bt = a.block_tables + (long long)a.tok_seq[t] * a.max_blocks;
   const int bs_mask = (1 << a.bs_shift) - 1;
+  // A block's page, by a scalar load and a block ahead of its use: among the vector loads, which are waited for in order, it would take all of them with it
+  auto page_of = [&](int b) { return reinterpret_cast<const_int*>((unsigned long long)bt)[block_key(b) >> a.bs_shift]; };
+
+  constexpr int KF = ONE ? (RW > 0 ? RW / 32 : 1) : DK / 32;  // key operands straight from memory: all, or the rotated parts'
+  constexpr int SETS = !ONE && DK <= 128 && DV <= 128 ? 2 : 1;  // blocks of a wave on their way (two: registers for 2 or 3 waves a SIMD; one row that is key and value has half the bytes)
+  raw16 kn[SETS][KF], vn[SETS][VIT];
+  float4 sn[SETS];
+  float rn[SETS][4];
+  const int head_lr = g * rep + h0 + (lr < nhd ? lr : nhd - 1);  // the lane's head
+  const float* rel = REL ? a.see.rel + (long long)head_lr * a.see.rel_n : nullptr;
+  const int v_row = lane / VCH, v_c = lane % VCH;  // piece `it` of a V block: row v_row + it * (64 / VCH)
+  auto fetch = [&](int b, int set, int page_index) __attribute__((always_inline)) {
+    const int key = block_key(b);
+    if constexpr (REL) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        int d = pos - key - 4 * lq - r;
+        d = d < 0 ? 0 : d;
+        rn[set][r] = rel[d < a.see.rel_n ? d : a.see.rel_n - 1];
+      }
+    }
+    const long long page = ((long long)page_index * a.nkv + g) * (bs_mask + 1) + (key & bs_mask);
+    if constexpr (!ONE || RW > 0) {
+      const bf16raw* kp = k_cache + (page + lr) * KST + (ONE ? DK : 0) + lq * 8;
+#pragma unroll
+      for (int ks = 0; ks < KF; ++ks) kn[set][ks] = *reinterpret_cast<const raw16*>(kp + ks * 32);
+    }
+    if constexpr (ONE) sn[set] = ld4(a.key_scale + page + 4 * lq);
+    const bf16raw* vp = ONE ? k_cache : v_cache;
+#pragma unroll
+    for (int it = 0; it < VIT; ++it) vn[set][it] = *reinterpret_cast<const raw16*>(vp + (page + v_row + it * (64 / VCH)) * VST + v_c * 8);
+  };
+  int first_page[SETS];
+  auto mine = [&](int b) { return b < nb ? b : nb - 1; };  // behind the last block: that one again, whose bytes the caches have
+
+#pragma unroll
+  for (int e = 0; e < SETS; ++e) first_page[e] = page_of(mine(me + e * stride));
 
   if constexpr (FUSED) {
     const bool owner = (nb - 1) % stride / NW == (int)blockIdx.z;  // this workgroup reads the block with the new key
@@ -279,30 +322,51 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
     const int slot = a.slots[t];
     const long long crow = ((long long)(slot >> a.bs_shift) * a.nkv + g) * (bs_mask + 1) + (slot & bs_mask);
     const int n_units = owner ? (ONE ? nhd + 1 : nhd + 2) : nhd;  // (more than 16 heads: every group's workgroup writes the same key)
-    for (int u = wave; u < n_units; u += NW) {
+    // What units need comes first, that of two units of a wave, then the first blocks of keys: loads answer in the order they were asked for
+    constexpr int E = (DK > DV ? DK : DV) / 64;
+    const float *cos_t = a.rot_dims ? a.cos_t + (long long)pos * half : a.q_norm, *sin_t = a.rot_dims ? a.sin_t + (long long)pos * half : a.q_norm;  // (no angles: nothing uses these)
+    struct Unit { unsigned int x[E]; float bias[E], nq[E], nk[E], c[E], s[E]; };
+    auto load = [&](int u) __attribute__((always_inline)) {
+      Unit n;
+      u = u < n_units ? u : 0;
+      const bool is_q = u < nhd, is_v = !ONE && u == nhd + 1;
+      const int hd = g * rep + h0 + u, len = is_v ? a.vdim : a.dim;
+      const bf16raw* src = pr + (is_v ? a.v_off + g * a.vdim : is_q ? a.q_off + hd * a.dim : a.k_off + g * a.dim);
+      const float* bias = a.bias + (is_v ? (a.nh + a.nkv) * a.dim + g * a.vdim : is_q ? hd * a.dim : (a.nh + g) * a.dim);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int i = lane + 64 * e < len ? lane + 64 * e : 0, d = i < a.dim ? i : 0, p = i < a.rot_dims ? (i < half ? i : i - half) : 0;
+        n.x[e] = raw(src + i);
+        n.bias[e] = bias[i];
+        n.nq[e] = a.q_norm[d];
+        n.nk[e] = a.k_norm[d];
+        n.c[e] = cos_t[p];
+        n.s[e] = sin_t[p];
+      }
+      return n;
+    };
+    auto make = [&](int u, const Unit& n) __attribute__((always_inline)) {
       if (!ONE && u == nhd + 1) {  // value
-        for (int i = lane; i < DV; i += 64)
-          v_cache[crow * DV + i] = i < a.vdim ? f2bf(bf2f(pr[a.v_off + g * a.vdim + i]) + a.bias[(a.nh + a.nkv) * a.dim + g * a.vdim + i]) : (bf16raw)0;
-        continue;
+#pragma unroll
+        for (int e = 0; e < DV / 64; ++e) {
+          const int i = lane + 64 * e;
+          v_cache[crow * DV + i] = i < a.vdim ? f2bf(number<bf16raw>(n.x[e]) + n.bias[e]) : (bf16raw)0;
+        }
+        return;
       }
       const bool is_q = u < nhd;
-      const int hd = is_q ? g * rep + h0 + u : g;
-      const bf16raw* src = pr + (is_q ? a.q_off : a.k_off) + hd * a.dim;
-      const float* bias = a.bias + (is_q ? hd : a.nh + hd) * a.dim;
-      const float* nw = is_q ? a.q_norm : a.k_norm;
       float x[DK / 64], ss = 0.f;
 #pragma unroll
       for (int e = 0; e < DK / 64; ++e) {
-        const int i = lane + 64 * e;
-        x[e] = i < a.dim ? bf2f(src[i]) + bias[i] : 0.f;
+        x[e] = lane + 64 * e < a.dim ? number<bf16raw>(n.x[e]) + n.bias[e] : 0.f;
         ss += x[e] * x[e];
       }
       const float rs = 1.f / sqrtf(wave_sum(ss) / (float)a.dim + a.eps);
 #pragma unroll
       for (int e = 0; e < DK / 64; ++e) {
         const int i = lane + 64 * e;
-        if constexpr (ONE) w[i] = i < a.dim ? (is_q ? x[e] * rs * nw[i] : x[e] * nw[i]) : 0.f;
-        else w[i] = i < a.dim ? x[e] * rs * nw[i] : 0.f;
+        if constexpr (ONE) w[i] = i < a.dim ? (is_q ? x[e] * rs * n.nq[e] : x[e] * n.nk[e]) : 0.f;
+        else w[i] = i < a.dim ? x[e] * rs * (is_q ? n.nq[e] : n.nk[e]) : 0.f;
       }
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -310,13 +374,9 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
       for (int e = 0; e < DK / 64; ++e) {
         const int i = lane + 64 * e;
         float v = w[i];
-        if (i < a.rot_dims) {
-          const int p = i < half ? i : i - half;
-          const float c = a.cos_t[(long long)pos * half + p], s = a.sin_t[(long long)pos * half + p];
-          v = i < half ? w[i] * c - w[i + half] * s : w[i] * c + w[i - half] * s;
-        }
+        if (i < a.rot_dims) v = i < half ? w[i] * n.c[e] - w[i + half] * n.s[e] : w[i] * n.c[e] + w[i - half] * n.s[e];
         if constexpr (ONE) {
-          if (is_q) q_s[u * QS + i] = i < a.dim && i >= a.rot_dims ? f2bf(v * a.k_norm[i]) : (bf16raw)0;
+          if (is_q) q_s[u * QS + i] = i < a.dim && i >= a.rot_dims ? f2bf(v * n.nk[e]) : (bf16raw)0;
           else k_cache[crow * KST + i] = f2bf(x[e]);
           if (i < RW) {
             const bf16raw z = i < a.rot_dims ? f2bf(v) : (bf16raw)0;
@@ -331,10 +391,20 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
-    }
+    };
+    const Unit first_unit = load(wave), second_unit = load(wave + NW);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < SETS; ++e) fetch(mine(me + e * stride), e, first_page[e]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (wave < n_units) make(wave, first_unit);
+    if (wave + NW < n_units) make(wave + NW, second_unit);
+    for (int u = wave + 2 * NW; u < n_units; u += NW) make(u, load(u));
     for (int i = tid; i < (16 - nhd) * KST; i += 64 * NW) q_s[(nhd + i / KST) * QS + i % KST] = 0;
     __threadfence_block();
   } else {
+#pragma unroll
+    for (int e = 0; e < SETS; ++e) fetch(mine(me + e * stride), e, first_page[e]);
     for (int i = tid; i < 16 * (KST / 8); i += 64 * NW) {
       const int h = i / (KST / 8), c = i % (KST / 8);
       raw16 v = {0, 0, 0, 0};
@@ -353,53 +423,42 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
 #pragma unroll
   for (int n = 0; n < DV / 16; ++n) o[n] = (frag_acc4){0.f, 0.f, 0.f, 0.f};
   float m_run = -1e30f, l_run = 0.f;
-  const int head_lr = g * rep + h0 + (lr < nhd ? lr : nhd - 1);  // the lane's head
   if (a.see.sink && me == 0) {  // (once per row)
     m_run = a.see.sink[head_lr] * LOG2E;
     l_run = lq == 0 ? 1.f : 0.f;
   }
-  const float* rel = REL ? a.see.rel + (long long)head_lr * a.see.rel_n : nullptr;
-  float rn[4] = {0.f, 0.f, 0.f, 0.f};
-  constexpr int KF = ONE ? (RW > 0 ? RW / 32 : 1) : DK / 32;  // key operands straight from memory: all, or the rotated parts'
-  raw16 kn[KF], vn[VIT];
-  float4 sn = make_float4(1.f, 1.f, 1.f, 1.f);
-  const int v_row = lane / VCH, v_c = lane % VCH;  // piece `it` of a V block: row v_row + it * (64 / VCH)
-  auto fetch = [&](int b) __attribute__((always_inline)) {
-    const int key = block_key(b);
-    if constexpr (REL) {
+  if constexpr (FUSED) {  // the block with the new key, where it was asked for before the key was there
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        int d = pos - key - 4 * lq - r;
-        d = d < 0 ? 0 : d;
-        rn[r] = rel[d < a.see.rel_n ? d : a.see.rel_n - 1];
+    for (int e = 0; e < SETS; ++e)
+      if (me + e * stride == nb - 1) {
+        fetch(nb - 1, e, first_page[e]);
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): (here, not in the loop, whose counts would have to do for this way in)
       }
-    }
-    const long long page = ((long long)bt[key >> a.bs_shift] * a.nkv + g) * (bs_mask + 1) + (key & bs_mask);
-    if constexpr (!ONE || RW > 0) {
-      const bf16raw* kp = k_cache + (page + lr) * KST + (ONE ? DK : 0) + lq * 8;
+  }
+  int page[SETS];  // of the blocks that are asked for next
 #pragma unroll
-      for (int ks = 0; ks < KF; ++ks) kn[ks] = *reinterpret_cast<const raw16*>(kp + ks * 32);
-    }
-    if constexpr (ONE) sn = ld4(a.key_scale + page + 4 * lq);
-    const bf16raw* vp = ONE ? k_cache : v_cache;
-#pragma unroll
-    for (int it = 0; it < VIT; ++it) vn[it] = *reinterpret_cast<const raw16*>(vp + (page + v_row + it * (64 / VCH)) * VST + v_c * 8);
-  };
-  if (me < nb) fetch(me);
-  for (int b = me; b < nb; b += stride) {
+  for (int e = 0; e < SETS; ++e) page[e] = page_of(mine(me + (SETS + e) * stride));
+  auto block = [&](int b, auto set_) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_)::value;
+    const float sk[4] = {sn[set].x, sn[set].y, sn[set].z, sn[set].w};
     raw16 kc[KF];
+    float rc[4];
 #pragma unroll
-    for (int ks = 0; ks < KF; ++ks) kc[ks] = kn[ks];
-    const float sk[4] = {sn.x, sn.y, sn.z, sn.w};
+    for (int ks = 0; ks < KF; ++ks) kc[ks] = kn[set][ks];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rc[r] = rn[set][r];
 #pragma unroll
     for (int it = 0; it < VIT; ++it) {
       const int r = v_row + it * (64 / VCH);
-      *reinterpret_cast<raw16*>(&vl[r * DV + ((v_c ^ (ONE ? kv_swz<DV>(r) : v_swz<DV>(r))) << 3)]) = vn[it];
+      *reinterpret_cast<raw16*>(&vl[r * DV + ((v_c ^ (ONE ? kv_swz<DV>(r) : v_swz<DV>(r))) << 3)]) = vn[set][it];
     }
-    float rc[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) rc[r] = rn[r];
-    if (b + stride < nb) fetch(b + stride);
+    // The next block's loads, always as many: what is waited for is counted exactly.  One block at a time: as early as there is room; two: where this one's were, when all
+    // of them are used (else they would move from one set of registers to the other, and be waited for there)
+    auto next = [&]() __attribute__((always_inline)) {
+      fetch(mine(b + SETS * stride), set, page[set]);
+      page[set] = page_of(mine(b + 2 * SETS * stride));
+    };
+    if constexpr (SETS == 1) next();
     frag_acc4 st = {0.f, 0.f, 0.f, 0.f};
     if constexpr (ONE) {
       if constexpr (RW > 0) {
@@ -422,6 +481,10 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
       if constexpr (ONE) v *= sk[r];
       if constexpr (REL) v += rc[r] * LOG2E;
       sc[r] = ((k0 + r >= first || k0 + r < a.see.keep) && k0 + r <= pos) ? v : -1e30f;
+    }
+    if constexpr (SETS > 1) {
+      __builtin_amdgcn_sched_barrier(0);
+      next();
     }
     float mx = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
     mx = lanes::meet<16>(mx, lanes::Max{});
@@ -454,6 +517,13 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
       const int r = 4 * lq + (lr >> 2), c = 2 * n + ((lr & 3) >> 1);
       const tr_b64 vf = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_b64*)(&vl[r * DV + ((c ^ (ONE ? kv_swz<DV>(r) : v_swz<DV>(r))) << 3) + (lr & 1) * 4]));
       o[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, __builtin_bit_cast(frag_b64, vf), o[n], 0, 0, 0);
+    }
+  };
+  for (int b = me; b < nb; b += SETS * stride) {
+    block(b, std::integral_constant<int, 0>{});
+    if constexpr (SETS > 1) {
+      if (b + stride >= nb) break;  // (and not around the block: one way round the loop, with all in flight)
+      block(b + stride, std::integral_constant<int, 1>{});
     }
   }
   l_run = lanes::meet<16>(l_run, lanes::Sum{});
