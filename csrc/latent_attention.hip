@@ -205,6 +205,7 @@ __global__ __launch_bounds__(256) void latent_prefill_kernel(const bf16raw* __re
 // ---- single tokens, first part: q' = W_uk[h]^T q for the listed rows, [rows][heads][RK].  Workgroup: 64 latent dimensions of one head x 16
 // rows.  WRITE: the workgroups behind the last head norm the rows' latents and write them into the cache.  With a rotated part, q' rows are
 // RK + RT long; `turn`: the projections' rotated parts have not been rotated yet.
+// Bound by the chains of loads: weights and queries are on their way before a rotated part's, a row's norm beside its latents.
 struct LatentRowsArgs {
   const int* rows; int n_rows; const int* slots;
   long long ldp; int q_off, c_off, gate_off, gate_each;
@@ -234,40 +235,51 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const bf16raw* __res
     for (int i = blockIdx.y * 4 + wave; i < 16; i += gridDim.y * 4) {
       if (rt + i >= a.n_rows) return;
       const int t = a.rows[rt + i];
-      const int slot = t < 0 ? -1 : a.slots[t];
-      if (slot < 0) continue;
+      if (t < 0) continue;
+      const int slot = a.slots[t];  // (negative: a padding row, whose latents are read and not written)
       const bf16raw* src = proj + (long long)t * a.ldp + a.c_off + lane * E;
-      float v[E], ss = 0.f;
+      float v[E], g[E], ss = 0.f;
+      float2 k = make_float2(0.f, 0.f);
 #pragma unroll
-      for (int e = 0; e < E; ++e) { v[e] = bf2f(src[e]); ss += v[e] * v[e]; }
+      for (int e = 0; e < E; ++e) { v[e] = bf2f(src[e]); g[e] = a.c_norm[lane * E + e]; }
+      if (RT > 0 && lane < RT / 2) k = turned(proj + (long long)t * a.ldp + a.kr_off, lane, a.positions[t], a, true);
+      if (slot < 0) continue;
+#pragma unroll
+      for (int e = 0; e < E; ++e) ss += v[e] * v[e];
       const float rs = 1.f / sqrtf(wave_sum(ss) / (float)a.rank + a.eps);
 #pragma unroll
-      for (int e = 0; e < E; ++e) cache[(long long)slot * KD + lane * E + e] = f2bf(v[e] * rs * a.c_norm[lane * E + e]);
+      for (int e = 0; e < E; ++e) cache[(long long)slot * KD + lane * E + e] = f2bf(v[e] * rs * g[e]);
       if (RT > 0 && lane < RT / 2) {
-        const float2 k = turned(proj + (long long)t * a.ldp + a.kr_off, lane, a.positions[t], a, true);
         cache[(long long)slot * KD + RK + 2 * lane] = f2bf(k.x);
         cache[(long long)slot * KD + RK + 2 * lane + 1] = f2bf(k.y);
       }
     }
     return;
   }
+  const int n0 = blockIdx.y * 64 + wave * 16;
+  const frag_ab* wp = reinterpret_cast<const frag_ab*>(w) + ((long long)(h * RK + n0) / 16 * (DK / 32)) * 64 + lane;
+  frag_ab wf[DK / 32];  // on their way before anything else
+#pragma unroll
+  for (int ks = 0; ks < DK / 32; ++ks) wf[ks] = wp[ks * 64];
+  const int r = rt + lr;
+  const int t = r < a.n_rows ? a.rows[r] : -1;
+  const bf16raw* qp = proj + (long long)(t < 0 ? 0 : t) * a.ldp + a.q_off + h * DK + lq * 8;
+  frag_ab q[DK / 32];
+#pragma unroll
+  for (int ks = 0; ks < DK / 32; ++ks) q[ks] = *reinterpret_cast<const frag_ab*>(qp + ks * 32);
+  __builtin_amdgcn_sched_barrier(0);
   if (RT > 0 && blockIdx.y == 0) {  // the queries' rotated parts, four elements a thread
     const int i = threadIdx.x >> 4, d = (threadIdx.x & 15) * 4;
     const int t = rt + i < a.n_rows ? a.rows[rt + i] : -1;
     if (t >= 0 && a.slots[t] >= 0) {
-      const bf16raw* q = proj + (long long)t * a.ldp + a.r_off + h * RT;
-      const float2 x = turned(q, d / 2, a.positions[t], a, a.turn), y = turned(q, d / 2 + 1, a.positions[t], a, a.turn);
+      const bf16raw* part = proj + (long long)t * a.ldp + a.r_off + h * RT;
+      const float2 x = turned(part, d / 2, a.positions[t], a, a.turn), y = turned(part, d / 2 + 1, a.positions[t], a, a.turn);
       st4(q_lat + ((long long)(rt + i) * a.nh + h) * KD + RK + d, make_float4(x.x, x.y, y.x, y.y));
     }
   }
-  const int n0 = blockIdx.y * 64 + wave * 16;
-  const frag_ab* wp = reinterpret_cast<const frag_ab*>(w) + ((long long)(h * RK + n0) / 16 * (DK / 32)) * 64 + lane;
-  const int r = rt + lr;
-  const int t = r < a.n_rows ? a.rows[r] : -1;
-  const bf16raw* qp = proj + (long long)(t < 0 ? 0 : t) * a.ldp + a.q_off + h * DK + lq * 8;
   frag_acc4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int ks = 0; ks < DK / 32; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[ks * 64], *reinterpret_cast<const frag_ab*>(qp + ks * 32), acc, 0, 0, 0);
+  for (int ks = 0; ks < DK / 32; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks], q[ks], acc, 0, 0, 0);
   if (t >= 0) st4(q_lat + ((long long)r * a.nh + h) * KD + n0 + 4 * lq, make_float4(acc[0], acc[1], acc[2], acc[3]));
 }
 
@@ -276,6 +288,8 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const bf16raw* __res
 // as A operand with the 16 heads' q' (S^T: a lane owns one head and 4 keys), and the weights, already in the A layout of
 // mfma_f32_16x16x16_bf16, with the same latents again, read transposed.  A rotated part (RT) lies behind the block's latents, rows of 128
 // bytes whose pieces are swizzled by pairs of rows, and only enters the scores.
+// Few rows are bound by the chain to a wave's first block and from block to block: the page of the next block but one is a scalar load that runs beside a
+// block (5 rows of 2306 tokens, 32 heads: 11.5 -> 10.6 us).
 struct LatentDecodeArgs {
   const int* block_tables; int max_blocks;
   const int* rows; const int* tok_seq; const int* positions; const int* slots;
@@ -334,9 +348,10 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(const bf16raw* __res
     const int r = p * RPP + lane / PC;
     piece[p] = (unsigned int)(r * KD + ((lane % PC) ^ lat_swz(r)) * 8) * 2;
   }
-  auto stage = [&](int b, int buf) __attribute__((always_inline)) {
+  auto page_of = [&](int b) { return bt[(b0 + (b < nb ? b : nb - 1)) << 4 >> a.bs_shift]; };
+  auto stage = [&](int b, int buf, int page) __attribute__((always_inline)) {
     const int key = (b0 + b) << 4;
-    const char* src = reinterpret_cast<const char*>(cache + (((long long)bt[key >> a.bs_shift] << a.bs_shift) + (key & bs_mask)) * KD);
+    const char* src = reinterpret_cast<const char*>(cache + (((long long)page << a.bs_shift) + (key & bs_mask)) * KD);
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
       unsigned int off = piece[p];
@@ -366,7 +381,9 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(const bf16raw* __res
 #pragma unroll
   for (int n = 0; n < RK / 16; ++n) o[n] = (frag_acc4){0.f, 0.f, 0.f, 0.f};
   float m_run = -1e30f, l_run = 0.f;
-  if (me < nb) stage(me, 0);
+  const int page0 = page_of(me);
+  int page = page_of(me + stride);  // of the block after the one that was asked for last: on its way during a block
+  if (me < nb) stage(me, 0, page0);
   int b = me;
   unsigned int flip = 0;  // byte offset of the block's buffer
   bool staged = false;    // the next block is on its way already
@@ -378,7 +395,10 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(const bf16raw* __res
     bool outgrown = false;
     for (; b < nb; b += stride, flip ^= BUF * 2, staged = false) {
       if (b + stride < nb) {
-        if (!staged) stage(b + stride, flip ? 0 : 1);
+        if (!staged) {
+          stage(b + stride, flip ? 0 : 1, page);
+          page = page_of(b + 2 * stride);
+        }
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES + NR) : "memory");
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -512,40 +532,51 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(const bf16raw* __res
   }
 }
 
-// ---- with shares: their partial sums [rows][heads][shares][RK + 4] -> bf16 [rows][heads][RK].  One wave per row and head.
+// ---- with shares: their partial sums [rows][heads][shares][RK + 4] -> bf16 [rows][heads][RK].  Workgroup: a row and head; lane: two elements.  Bound
+// by the loads' latency: the sums of all shares (at most 16 at a time) are asked for beside the maxima (one wave with eight elements a lane, four shares
+// at a time behind the maxima: 6.3 us for 5 rows of 32 heads, 16 shares of 512; now 4.9).
 template <int RK>
-__global__ __launch_bounds__(64) void latent_combine_kernel(const float* __restrict__ part, bf16raw* __restrict__ lat, const int* __restrict__ rows, const int* __restrict__ slots, int nh, int shares) {
-  constexpr int E = RK / 64;  // elements per lane
-  const int t = rows[blockIdx.x], lane = threadIdx.x;
-  if (t < 0 || slots[t] < 0) return;
+__global__ __launch_bounds__(RK / 2) void latent_combine_kernel(const float* __restrict__ part, bf16raw* __restrict__ lat, const int* __restrict__ rows, const int* __restrict__ slots, int nh, int shares) {
+  const int lane = threadIdx.x & 63;
   const long long row = (long long)blockIdx.x * nh + blockIdx.y;
   const float* p = part + row * shares * (RK + 4);
-  const bool on = lane < shares;  // (at most 64)
-  const float m = on ? p[(long long)lane * (RK + 4)] : -1e30f;
-  const float top = wave_max(m);
+  const int mine = lane < shares ? lane : shares - 1;  // (at most 64)
+  const float2 ml = *reinterpret_cast<const float2*>(p + (long long)mine * (RK + 4));
+  constexpr int AHEAD = 16;
+  float2 x[AHEAD];
+  const float* xp = p + 4 + 2 * threadIdx.x;
+  auto fetch = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      if (s0 + i < shares) x[i] = *reinterpret_cast<const float2*>(xp + (long long)(s0 + i) * (RK + 4));
+    }
+  };
+  fetch(0);
+  const int t = rows[blockIdx.x];
+  if (t < 0 || slots[t] < 0) return;
+  const bool on = lane < shares;
+  const float m = on ? ml.x : -1e30f;
+  const float top = lanes::max(m);
   const float f = on ? __builtin_amdgcn_exp2f(m - top) : 0.f;
-  const float l = wave_sum(on ? f * p[(long long)lane * (RK + 4) + 1] : 0.f);
+  const float l = lanes::sum(on ? f * ml.y : 0.f);
   const float w = f / l;
-  float v[E];
+  float2 v = make_float2(0.f, 0.f);
+  for (int s0 = 0; s0 < shares; s0 += AHEAD) {
+    if (s0 > 0) fetch(s0);
 #pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = 0.f;
-#pragma unroll 4
-  for (int s = 0; s < shares; ++s) {
-    const float ws = __shfl(w, s, 64);
-    const float* x = p + (long long)s * (RK + 4) + 4 + lane * E;
-#pragma unroll
-    for (int e = 0; e < E; e += 2) {
-      const float2 y = *reinterpret_cast<const float2*>(x + e);
-      v[e] += ws * y.x;
-      v[e + 1] += ws * y.y;
+    for (int i = 0; i < AHEAD; ++i) {
+      if (s0 + i >= shares) break;
+      const float ws = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), s0 + i));
+      v.x += ws * x[i].x;
+      v.y += ws * x[i].y;
     }
   }
-#pragma unroll
-  for (int e = 0; e < E; ++e) lat[row * RK + lane * E + e] = f2bf(v[e]);
+  *reinterpret_cast<unsigned int*>(lat + row * RK + 2 * threadIdx.x) = f2bf(v.x) | (unsigned int)f2bf(v.y) << 16;
 }
 
 // ---- third part: value = W_uv[h] (weighted latent), times out_scale and the head's gate.  Workgroup: one head x 16 listed rows x
 // DV / gridDim.z features.
+// The weights of a wave's first features are asked for ahead of the rows, their slots and latents, two trips that do not need them (5.4 -> 5.05 us).
 struct LatentUpArgs {
   LatentRowsArgs r;
   int vdim;
@@ -559,6 +590,16 @@ __global__ __launch_bounds__(256) void latent_up_kernel(const bf16raw* __restric
   __shared__ __attribute__((aligned(16))) bf16raw x_s[16 * LS];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
   const int h = blockIdx.x, rt = blockIdx.y * 16;
+  // the wave's first 16 features' weights, on their way before anything else
+  frag_ab wf[RK / 32];
+  auto weights = [&](int n) __attribute__((always_inline)) {
+    const frag_ab* wp = reinterpret_cast<const frag_ab*>(w) + ((long long)(h * DV + 16 * n) / 16 * (RK / 32)) * 64 + lane;
+#pragma unroll
+    for (int ks = 0; ks < RK / 32; ++ks) wf[ks] = wp[ks * 64];
+  };
+  const int n0 = blockIdx.z * 4 + wave;
+  if (n0 < DV / 16) weights(n0);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = threadIdx.x; i < 16 * (RK / 8); i += 256) {  // 16 rows x RK into LDS, 8 elements a time
     const int rr = i / (RK / 8), c = (i % (RK / 8)) * 8, r = rt + rr;
@@ -576,11 +617,11 @@ __global__ __launch_bounds__(256) void latent_up_kernel(const bf16raw* __restric
   if (live && !a.r.gate_each) f *= head_gate(gate, h, a.vdim, 0, 0);
   const bool vec = (a.vdim & 3) == 0 && (a.ldo & 3) == 0 && (a.o_off & 3) == 0;
   bf16raw* op = out + (long long)(t < 0 ? 0 : t) * a.ldo + a.o_off + (long long)h * a.vdim;
-  for (int n = blockIdx.z * 4 + wave; n < DV / 16; n += 4 * gridDim.z) {
-    const frag_ab* wp = reinterpret_cast<const frag_ab*>(w) + ((long long)(h * DV + 16 * n) / 16 * (RK / 32)) * 64 + lane;
+  for (int n = n0; n < DV / 16; n += 4 * gridDim.z) {
+    if (n != n0) weights(n);
     frag_acc4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < RK / 32; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[ks * 64], *reinterpret_cast<const frag_ab*>(&x_s[lr * LS + ks * 32 + lq * 8]), acc, 0, 0, 0);
+    for (int ks = 0; ks < RK / 32; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks], *reinterpret_cast<const frag_ab*>(&x_s[lr * LS + ks * 32 + lq * 8]), acc, 0, 0, 0);
     if (!live) continue;
     const int d = 16 * n + 4 * lq;
     if (d >= a.vdim) continue;
@@ -679,7 +720,7 @@ int kvl_decode(const void* q_lat, const void* cache, void* lat, float* part, con
   do {                                                                                                                                                         \
     if (shares == 1) { KV_LDR(RK, false); break; }                                                                                                             \
     KV_LDR(RK, true);                                                                                                                                          \
-    hipLaunchKernelGGL((latent_combine_kernel<RK>), dim3(n_rows, nh), dim3(64), 0, s, part, (bf16raw*)lat, rows, slots, nh, shares);                           \
+    hipLaunchKernelGGL((latent_combine_kernel<RK>), dim3(n_rows, nh), dim3(RK / 2), 0, s, part, (bf16raw*)lat, rows, slots, nh, shares);                           \
   } while (0)
   if (rk == 128) KV_LD2(128);
   else if (rk == 256) KV_LD2(256);
