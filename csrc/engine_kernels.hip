@@ -2210,14 +2210,49 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   } else {
     ctx = ctx_lens[t];
   }
+  // What phase A needs is asked for first, one 4-column piece of this head group's q / k / v rows a thread, of all slabs (independent loads, one memory
+  // round trip instead of n_slabs), the row's sums of squares and its RoPE angles.  The keys / values of earlier positions do not depend on phase A:
+  // each wave's first blocks come right behind, on every path, so that the sums wait for the slabs alone and the blocks' trip overlaps phase A.
+  // (With the blocks ahead and behind branches, every wait was one for all of them; us a step, before and now: 1B, one row of 900 tokens 244.2 and
+  // 240.4, 48 rows of 600 312.7 and 306.1; 8B, 20 rows of 700 472.7 and 469.5, 2 of 16000 513.9 and 511.2.)  Not where a thread has two pieces, the
+  // second of which would wait for the blocks (8 heads a group, 32 rows of 500: 30.5 us a launch, and 30.7), nor with single heads of an e4m3 cache,
+  // whose registers would be too many for four waves of a SIMD (32 heads, 64 rows of 300: 36.6 and 38.3).
+  constexpr int PIECES = (REP + 2) * (HD / 4);  // q heads, then k, then v
+  constexpr int MAX_S = 16, AHEAD = REP <= 2 ? 8 : MAX_S;  // (at most 8 slabs ahead where one or two heads fit four waves of a SIMD into its registers)
+  constexpr bool FIRST = PIECES <= NT && !(REP == 1 && KV8 && HD == 128);
+  constexpr int RP = HALF / 8, ROT = (REP + 1) * RP;  // (q heads + k) x pieces of 8 dims and their partners
+  const float* row0 = slabs + (long long)t * ((nh + 2 * nkv) * HD);
+  f32x4 slab_v[AHEAD], csr[2], snr[2];
+  float ss_first = 0.f;
+  int pos = 0, slot = -1;
+  auto slab_loads = [&](int pc, int s0) __attribute__((always_inline)) {
+    const int r = pc / (HD / 4), c4 = pc % (HD / 4) * 4;
+    const int col = (r < REP ? (g * REP + r) * HD : r == REP ? (nh + g) * HD : (nh + nkv + g) * HD) + c4;
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (s0 + i < n_slabs) slab_v[i] = *reinterpret_cast<const f32x4*>(row0 + (long long)(s0 + i) * slab_stride + col);
+  };
+  auto angles = [&]() __attribute__((always_inline)) {
+    const int d0 = tid % RP * 8;
+    const f32x4* cp = reinterpret_cast<const f32x4*>(cos_t + (long long)pos * HALF + d0);
+    const f32x4* sp = reinterpret_cast<const f32x4*>(sin_t + (long long)pos * HALF + d0);
+    csr[0] = cp[0]; csr[1] = cp[1]; snr[0] = sp[0]; snr[1] = sp[1];
+  };
+  auto sums = [&]() __attribute__((always_inline)) {
+    slab_loads(tid < PIECES ? tid : 0, 0);
+    if (row_ss != nullptr && lane < ss_parts) ss_first = row_ss[(long long)t * ss_parts + lane];
+  };
+  if constexpr (!ATTN) {
+    pos = positions[t];
+    slot = slot_mapping[t];
+    if constexpr (FIRST) sums();
+  }
   unsigned short* orow = out + (long long)t * nh * HD + (long long)g * REP * HD;
   if (ctx <= 0) {  // padding token: no KV write (slot -1), zero output
     if (z == 0)
       for (int i = tid; i < REP * HD; i += NT) orow[i] = 0;
     return;
   }
-  // The keys / values of earlier positions do not depend on phase A: each wave loads its
-  // first KV block now, so that round trip overlaps the slab loads and the RoPE phase.
   const int prev = ATTN ? ctx : ctx - 1;
   const int* bt = block_tables + (long long)tok_seq[t] * max_blocks_per_seq;
   const int all_blocks = (prev + BS - 1) / BS;
@@ -2232,46 +2267,44 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
   const int pv_tg = lane / DV, pv_dv = lane % DV;
   using Stage = typename KVStageOf<KV8, HD>::type;
   Stage st_cur, st_nxt;  // this wave's first block and the one after: two blocks (16 KB of bf16) per wave in flight at any time
-  if (b0 + wave < n_blocks) st_cur.load(k_cache, v_cache, ((long long)bt[b0 + wave] * nkv + g) * BS * HD, qk_tok, qk_c, pv_tg, pv_dv);
-  if (b0 + wave + NWAVE < n_blocks) st_nxt.load(k_cache, v_cache, ((long long)bt[b0 + wave + NWAVE] * nkv + g) * BS * HD, qk_tok, qk_c, pv_tg, pv_dv);
+  if constexpr (!ATTN && FIRST) angles();
+  if constexpr (FIRST) {
+    // (a wave without a block asks for one all the same, and no more of it)
+    const int some = max(n_blocks - 1, 0), first = min(b0 + wave, some), second = min(b0 + wave + NWAVE, some);
+    const long long at0 = ((long long)bt[first] * nkv + g) * BS * HD, at1 = ((long long)bt[second] * nkv + g) * BS * HD;
+    st_cur.load(k_cache, v_cache, at0, qk_tok, qk_c, pv_tg, pv_dv);
+    st_nxt.load(k_cache, v_cache, at1, qk_tok, qk_c, pv_tg, pv_dv);
+  } else {
+    if (b0 + wave < n_blocks) st_cur.load(k_cache, v_cache, ((long long)bt[b0 + wave] * nkv + g) * BS * HD, qk_tok, qk_c, pv_tg, pv_dv);
+    if (b0 + wave + NWAVE < n_blocks) st_nxt.load(k_cache, v_cache, ((long long)bt[b0 + wave + NWAVE] * nkv + g) * BS * HD, qk_tok, qk_c, pv_tg, pv_dv);
+  }
+  if constexpr (!ATTN && !FIRST) {
+    if (tid < ROT) angles();
+    sums();
+  }
   if constexpr (ATTN) {
     for (int pc = tid; pc < REP * (HD / 8); pc += NT) {
       const int h = pc / DV, d0 = pc % DV * 8;
       *reinterpret_cast<bf16x8*>(&xb_lds[h][d0]) = *reinterpret_cast<const bf16x8*>(q_in + (long long)t * q_row_stride + (long long)(g * REP + h) * HD + d0);
     }
   } else {
-  // likewise the RoPE table row of this token (needed in A.2)
-  constexpr int RP = HALF / 8, ROT = (REP + 1) * RP;  // (q heads + k) x pieces of 8 dims and their partners
-  const int pos = positions[t];
-  const int slot = slot_mapping[t];
-  f32x4 csr[2], snr[2];
-  if (tid < ROT) {
-    const int d0 = tid % RP * 8;
-    const f32x4* cp = reinterpret_cast<const f32x4*>(cos_t + (long long)pos * HALF + d0);
-    const f32x4* sp = reinterpret_cast<const f32x4*>(sin_t + (long long)pos * HALF + d0);
-    csr[0] = cp[0]; csr[1] = cp[1]; snr[0] = sp[0]; snr[1] = sp[1];
-  }
-  // ---- phase A.1: every thread sums ONE 4-column piece of this head group's q / k / v rows
-  // over all slabs.  The slab loads are independent and issued together (one memory round
-  // trip instead of n_slabs), and summed in slab order — the order of the two-kernel path.
+  // ---- phase A.1: the slabs' pieces are summed in slab order — the order of the two-kernel path
   {
     float rs = 1.f;
-    if (row_ss != nullptr) rs = rsqrtf(row_ss_total(row_ss + (long long)t * ss_parts, ss_parts, lane) * inv_h + eps);
-    const int width = (nh + 2 * nkv) * HD;
-    const float* row0 = slabs + (long long)t * width;
-    constexpr int PIECES = (REP + 2) * (HD / 4);  // q heads, then k, then v
-    constexpr int MAX_S = 16;
+    if (row_ss != nullptr) {
+      for (int i = lane + 64; i < ss_parts; i += 64) ss_first += row_ss[(long long)t * ss_parts + i];
+      rs = rsqrtf(wave_sum(ss_first) * inv_h + eps);
+    }
     for (int pc = tid; pc < PIECES; pc += NT) {
       const int r = pc / (HD / 4), c4 = pc % (HD / 4) * 4;
-      const int col = (r < REP ? (g * REP + r) * HD : r == REP ? (nh + g) * HD : (nh + nkv + g) * HD) + c4;
-      f32x4 v[MAX_S];
-#pragma unroll
-      for (int sidx = 0; sidx < MAX_S; ++sidx)
-        if (sidx < n_slabs) v[sidx] = *reinterpret_cast<const f32x4*>(row0 + (long long)sidx * slab_stride + col);
       f32x4 a = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int sidx = 0; sidx < MAX_S; ++sidx)
-        if (sidx < n_slabs) a += v[sidx];
+      for (int s0 = 0; s0 < MAX_S; s0 += AHEAD) {
+        if (pc != tid || s0 > 0) slab_loads(pc, s0);
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+          if (s0 + i < n_slabs) a += slab_v[i];
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) x_lds[r][c4 + j] = bf2f(f2bf(a[j] * rs));  // the GEMM output as bf16
     }

@@ -880,6 +880,34 @@ def test_fused_decode_attention_matches_two_kernel_path(rep):
     assert out[7].abs().max().item() == 0 and out[13].abs().max().item() == 0  # padding rows
 
 
+@pytest.mark.parametrize("rep,hd", [(1, 64), (1, 128), (2, 64), (2, 128), (4, 64), (6, 128), (7, 128)])
+@pytest.mark.parametrize("slabs", [1, 8, 9, 16])
+def test_fused_decode_attention_sums_any_number_of_slabs(rep, hd, slabs):
+    """Slabs beyond those that are read ahead, rows without an earlier key and without a place in the cache: the caches' new rows and (both paths round
+    weights and outputs to bf16: half an ulp each of values below 4) the outputs of rope_kv_write_slabs and paged_attention."""
+    from kvmini.models.llama import LlamaConfig, rope_tables
+    from kvmini.ops import hip_ops
+
+    torch.manual_seed(rep + slabs)
+    nkv, bs, mb, h_in = 2, 16, 20, 512
+    nh = nkv * rep
+    ctx = torch.tensor([1, 17, 0, 300, 16, 2, 129, 33], device=_dev(), dtype=torch.int32)
+    t = len(ctx)
+    cos, sin = rope_tables(LlamaConfig(head_dim=hd), 320, _dev())
+    positions, tok_seq = (ctx - 1).clamp(min=0), torch.arange(t, device=_dev(), dtype=torch.int32)
+    bt = torch.randperm(t * mb, device=_dev()).view(t, mb).int()
+    slots = torch.where(ctx > 0, bt[tok_seq.long(), (positions // bs).long()] * bs + positions % bs, torch.full_like(ctx, -1)).int()
+    part = hip_ops.Partial(torch.randn(slabs, t, (nh + 2 * nkv) * hd, device=_dev()) / slabs**0.5, torch.rand(t, 1, device=_dev()) * h_in + h_in, 1e-5, h_in)
+    kc, vc = (torch.randn(t * mb, nkv, bs, hd, device=_dev()).bfloat16() for _ in range(2))
+    kc2, vc2 = kc.clone(), vc.clone()
+    q = hip_ops.rope_kv_write(part, positions, cos, sin, kc, vc, slots, nh, nkv, hd)
+    ref = hip_ops.paged_attention(q, kc, vc, bt, tok_seq, ctx, 1 / math.sqrt(hd))
+    out = hip_ops.rope_attention_fused(part, positions, cos, sin, kc2, vc2, slots, bt, tok_seq, ctx, nh, 1 / math.sqrt(hd))
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    assert (out.float() - ref.float()).abs().max().item() <= 2 * 4 * 2**-9 and ref.abs().max().item() < 4
+    assert out[2].abs().max().item() == 0
+
+
 @pytest.mark.parametrize("graphs,custom", [(False, True), (True, True), (False, False), (True, False)])
 def test_engine_tp_collective_path_on_one_gpu(graphs, custom):
     """The tensor-parallel code path with a one-rank group must reproduce the plain engine's
