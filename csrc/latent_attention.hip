@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const bf16raw* __res
       float2 k = make_float2(0.f, 0.f);
 #pragma unroll
       for (int e = 0; e < E; ++e) { v[e] = bf2f(src[e]); g[e] = a.c_norm[lane * E + e]; }
-      if (RT > 0 && lane < RT / 2) k = turned(proj + (long long)t * a.ldp + a.kr_off, lane, a.positions[t], a, true);
+      if (RT > 0 && lane < RT / 2) k = turned(proj + (long long)t * a.ldp + a.kr_off, lane, slot < 0 ? 0 : a.positions[t], a, true);
       if (slot < 0) continue;
 #pragma unroll
       for (int e = 0; e < E; ++e) ss += v[e] * v[e];
