@@ -361,7 +361,8 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
         x[e] = lane + 64 * e < a.dim ? number<bf16raw>(n.x[e]) + n.bias[e] : 0.f;
         ss += x[e] * x[e];
       }
-      const float rs = 1.f / sqrtf(wave_sum(ss) / (float)a.dim + a.eps);
+      ss = DK == 64 ? lanes::sum_of_products(x[0], x[0]) : wave_sum(ss);
+      const float rs = 1.f / sqrtf(ss / (float)a.dim + a.eps);
 #pragma unroll
       for (int e = 0; e < DK / 64; ++e) {
         const int i = lane + 64 * e;

@@ -2612,7 +2612,7 @@ __device__ __forceinline__ void decode_attention_body(const int bx, const int by
       }
       const float mx = lanes::max(m);
       const float c = s2 < eff ? __builtin_amdgcn_exp2f(m - mx) : 0.f;
-      const float tot = lanes::sum(den * c);
+      const float tot = lanes::sum_of_products(den, c);
       w_lds[h][s2] = tot > 0.f ? c / tot : 0.f;
     }
     __syncthreads();

@@ -1,7 +1,7 @@
 // Reductions over the lanes of a wave without LDS: lanes 1, 2, 4 and 8 apart by DPP moves, 16 and 32 apart by the swaps of rows and halves.  A shuffle through
 // LDS (ds_bpermute) is some 100 cycles until its answer is there, six of them in a row 0.3 us of a launch that has two or three such sums and takes 3 to 5 in all; these
-// take 60 cycles together.  The same pairs in the same order as a butterfly of shuffles: the same bits, but for sums of one product a lane, of which shuffles
-// let the compiler fuse a lane's own with what it got: either half of the lanes had a rounding less in its own number and the other's.
+// take 60 cycles together.  The same pairs in the same order as a butterfly of shuffles: the same bits.  Where each lane brings one product, shuffles let the
+// compiler fuse a lane's own with the rounded one that it got; the swaps would not, so such sums have a form of their own.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -57,6 +57,13 @@ struct Max { __device__ float operator()(float a, float b) const { return fmaxf(
 // of all 64 lanes, in all of them
 __device__ inline float sum(float v) { return meet_down<32, 1>(v, Sum{}); }
 __device__ inline float max(float v) { return meet_down<32, 1>(v, Max{}); }
+
+// of all 64 lanes' a b: a lane's own product meets that of 32 lanes away unrounded (so the halves of the wave may differ in the last bit)
+__device__ inline float sum_of_products(float a, float b) {
+  const unsigned int u = __float_as_uint(a * b);
+  const auto halves = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return meet_down<16, 1>(__builtin_fmaf(a, b, __uint_as_float(halves[0] ^ halves[1] ^ u)), Sum{});
+}
 
 // the larger value and, of equal ones, the smaller index, in all lanes
 template <int M>

@@ -558,7 +558,7 @@ __global__ __launch_bounds__(RK / 2) void latent_combine_kernel(const float* __r
   const float m = on ? ml.x : -1e30f;
   const float top = lanes::max(m);
   const float f = on ? __builtin_amdgcn_exp2f(m - top) : 0.f;
-  const float l = lanes::sum(on ? f * ml.y : 0.f);
+  const float l = lanes::sum_of_products(f, on ? ml.y : 0.f);
   const float w = f / l;
   float2 v = make_float2(0.f, 0.f);
   for (int s0 = 0; s0 < shares; s0 += AHEAD) {

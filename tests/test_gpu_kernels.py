@@ -908,6 +908,33 @@ def test_fused_decode_attention_sums_any_number_of_slabs(rep, hd, slabs):
     assert out[2].abs().max().item() == 0
 
 
+@pytest.mark.parametrize("waves,shares", [(4, 1), (8, 3)])
+def test_norms_of_heads_of_64_round_a_lanes_own_square_once(C, waves, shares):
+    """A lane has one square of such a head: it meets that of the lane 32 away unrounded, the other sums are fp32.  Keys as decode attention caches them, of
+    tokens on which a square that is rounded first shows: the same bits."""
+    hd, eps = 64, 1e-5
+    gen = torch.Generator().manual_seed(9)
+    raw, bias, gain = torch.randn(1 << 17, hd, generator=gen).bfloat16(), torch.randn(hd, generator=gen), 1 + 0.1 * torch.randn(hd, generator=gen)
+    x, lane = (raw.float() + bias).numpy(), np.arange(hd)
+
+    def keys(ss):
+        for m in (16, 8, 4, 2, 1):
+            ss = ss + ss[:, lane ^ m]
+        rs = np.float32(1) / np.sqrt(ss / np.float32(hd) + np.float32(eps))
+        return torch.from_numpy(x * rs * gain.numpy()).bfloat16()
+
+    want = keys((x.astype(np.float64) ** 2 + (x * x)[:, lane ^ 32]).astype(np.float32))  # (the squares are exact)
+    telling = (want != keys(x * x + (x * x)[:, lane ^ 32])).any(1)
+    assert 4 <= telling.sum() < 64
+    proj, want = raw[telling].to(_dev()).repeat(1, 3), want[telling]
+    t, bias, gain, none = len(want), bias.to(_dev()).repeat(3), gain.to(_dev()), torch.zeros(0, device=_dev())
+    rows = torch.arange(t, device=_dev(), dtype=torch.int32)
+    kc, vc = (torch.zeros(t, 1, 16, hd, device=_dev(), dtype=torch.bfloat16) for _ in range(2))
+    C.chunk_decode(None, proj, 0, hd, 2 * hd, bias, gain, gain, none, none, 0, eps, kc, vc, rows.view(t, 1), rows, rows, torch.zeros_like(rows), rows * 16, 0, 0, torch.empty_like(proj[:, :hd]), 0, 1, hd, hd,
+                   0, 0, 0, None, None, 0.125, 1.0, waves, shares)
+    assert torch.equal(kc[:, 0, 0].cpu(), want)
+
+
 @pytest.mark.parametrize("graphs,custom", [(False, True), (True, True), (False, False), (True, False)])
 def test_engine_tp_collective_path_on_one_gpu(graphs, custom):
     """The tensor-parallel code path with a one-rank group must reproduce the plain engine's
