@@ -355,13 +355,18 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
         return;
       }
       const bool is_q = u < nhd;
-      float x[DK / 64], ss = 0.f;
+      float x[DK / 64], ss;
 #pragma unroll
-      for (int e = 0; e < DK / 64; ++e) {
-        x[e] = lane + 64 * e < a.dim ? number<bf16raw>(n.x[e]) + n.bias[e] : 0.f;
-        ss += x[e] * x[e];
+      for (int e = 0; e < DK / 64; ++e) x[e] = lane + 64 * e < a.dim ? number<bf16raw>(n.x[e]) + n.bias[e] : 0.f;
+      // (which product of a sum stays unrounded is said here and below, else it would be the compiler's choice for each copy of this code)
+      if constexpr (DK == 64) {
+        ss = lanes::sum_of_products(x[0], x[0]);
+      } else {
+        ss = __builtin_fmaf(x[0], x[0], x[1] * x[1]);
+#pragma unroll
+        for (int e = 2; e < DK / 64; ++e) ss = __builtin_fmaf(x[e], x[e], ss);
+        ss = wave_sum(ss);
       }
-      ss = DK == 64 ? lanes::sum_of_products(x[0], x[0]) : wave_sum(ss);
       const float rs = 1.f / sqrtf(ss / (float)a.dim + a.eps);
 #pragma unroll
       for (int e = 0; e < DK / 64; ++e) {
@@ -375,7 +380,7 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
       for (int e = 0; e < DK / 64; ++e) {
         const int i = lane + 64 * e;
         float v = w[i];
-        if (i < a.rot_dims) v = i < half ? w[i] * n.c[e] - w[i + half] * n.s[e] : w[i] * n.c[e] + w[i - half] * n.s[e];
+        if (i < a.rot_dims) v = i < half ? __builtin_fmaf(-w[i + half], n.s[e], w[i] * n.c[e]) : __builtin_fmaf(w[i - half], n.s[e], w[i] * n.c[e]);
         if constexpr (ONE) {
           if (is_q) q_s[u * QS + i] = i < a.dim && i >= a.rot_dims ? f2bf(v * n.nk[e]) : (bf16raw)0;
           else k_cache[crow * KST + i] = f2bf(x[e]);
@@ -479,8 +484,8 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float v = st[r] * a.scale_log2e;
-      if constexpr (ONE) v *= sk[r];
-      if constexpr (REL) v += rc[r] * LOG2E;
+      if constexpr (REL) v = __builtin_fmaf(ONE ? v : st[r], ONE ? sk[r] : a.scale_log2e, rc[r] * LOG2E);
+      else if constexpr (ONE) v *= sk[r];
       sc[r] = ((k0 + r >= first || k0 + r < a.see.keep) && k0 + r <= pos) ? v : -1e30f;
     }
     if constexpr (SETS > 1) {

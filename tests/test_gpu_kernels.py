@@ -908,31 +908,91 @@ def test_fused_decode_attention_sums_any_number_of_slabs(rep, hd, slabs):
     assert out[2].abs().max().item() == 0
 
 
-@pytest.mark.parametrize("waves,shares", [(4, 1), (8, 3)])
-def test_norms_of_heads_of_64_round_a_lanes_own_square_once(C, waves, shares):
-    """A lane has one square of such a head: it meets that of the lane 32 away unrounded, the other sums are fp32.  Keys as decode attention caches them, of
-    tokens on which a square that is rounded first shows: the same bits."""
-    hd, eps = 64, 1e-5
+@pytest.mark.parametrize("dim,rot,rep,waves,shares", [(64, 0, 1, 4, 1), (64, 0, 1, 8, 3), (64, 48, 6, 4, 1), (128, 0, 1, 4, 1), (128, 128, 6, 4, 1), (128, 32, 16, 8, 1), (256, 0, 16, 4, 1), (256, 256, 1, 4, 3)])
+def test_keys_of_decode_attention_round_as_said(C, dim, rot, rep, waves, shares):
+    """Bit by bit, of tokens on which another rounding shows: of a head's first squares the first one is not rounded (a head of 64: a lane's own, not that of the
+    lane 32 away), nor is the second product of a rotation; all else is fp32."""
+    eps, half, f32, f64 = 1e-5, rot // 2, np.float32, np.float64
     gen = torch.Generator().manual_seed(9)
-    raw, bias, gain = torch.randn(1 << 17, hd, generator=gen).bfloat16(), torch.randn(hd, generator=gen), 1 + 0.1 * torch.randn(hd, generator=gen)
-    x, lane = (raw.float() + bias).numpy(), np.arange(hd)
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    raw, bias, gain, angle = rnd(1 << 23).view(-1, dim).bfloat16(), rnd(dim), 1 + 0.1 * rnd(dim), 3 * rnd(half)
+    cos, sin = angle.cos().expand(8, half).contiguous(), angle.sin().expand(8, half).contiguous()
+    x, lane = (raw.float() + bias).numpy(), np.arange(64)
+    part = x.reshape(-1, dim // 64, 64)
 
-    def keys(ss):
+    def keys(first_square, second_turn):
+        if dim == 64:
+            ss = first_square(part[:, 0], part[:, 0][:, lane ^ 32])
+        else:
+            ss = first_square(part[:, 0], part[:, 1])
+            for e in range(2, dim // 64):
+                ss = (part[:, e].astype(f64) ** 2 + ss).astype(f32)  # (the square is exact)
+            ss = ss + ss[:, lane ^ 32]
         for m in (16, 8, 4, 2, 1):
             ss = ss + ss[:, lane ^ m]
-        rs = np.float32(1) / np.sqrt(ss / np.float32(hd) + np.float32(eps))
-        return torch.from_numpy(x * rs * gain.numpy()).bfloat16()
+        w = x * np.tile(f32(1) / np.sqrt(ss / f32(dim) + f32(eps)), dim // 64) * gain.numpy()
+        if rot:
+            c, s = cos[0].numpy(), sin[0].numpy()
+            low, high = w[:, :half].copy(), w[:, half:rot].copy()
+            w[:, :half], w[:, half:rot] = second_turn(low, c, -high, s), second_turn(high, c, low, s)
+        return torch.from_numpy(w).bfloat16()
 
-    want = keys((x.astype(np.float64) ** 2 + (x * x)[:, lane ^ 32]).astype(np.float32))  # (the squares are exact)
-    telling = (want != keys(x * x + (x * x)[:, lane ^ 32])).any(1)
-    assert 4 <= telling.sum() < 64
-    proj, want = raw[telling].to(_dev()).repeat(1, 3), want[telling]
-    t, bias, gain, none = len(want), bias.to(_dev()).repeat(3), gain.to(_dev()), torch.zeros(0, device=_dev())
+    one_rounding = lambda a, b, c, d: (a.astype(f64) * b + c * d).astype(f32)  # noqa: E731  (a b exact, c d rounded)
+    first, other_first = lambda a, b: one_rounding(a, a, b, b), lambda a, b: one_rounding(b, b, a, a)
+    second, other_second = lambda a, b, c, d: one_rounding(c, d, a, b), one_rounding
+    want = keys(first, second)
+    telling = (want != keys(other_first if dim > 64 else lambda a, b: a * a + b * b, second)).any(1)
+    assert telling.sum() >= 4
+    if rot:
+        turns = (want != keys(first, other_second)).any(1)
+        assert turns.sum() >= 4
+        telling |= turns
+    want, k = want[telling], raw[telling].to(_dev())
+    t, none = len(want), torch.zeros(0, device=_dev())
+    proj = torch.cat((k.repeat(1, rep), k, k), 1)
     rows = torch.arange(t, device=_dev(), dtype=torch.int32)
-    kc, vc = (torch.zeros(t, 1, 16, hd, device=_dev(), dtype=torch.bfloat16) for _ in range(2))
-    C.chunk_decode(None, proj, 0, hd, 2 * hd, bias, gain, gain, none, none, 0, eps, kc, vc, rows.view(t, 1), rows, rows, torch.zeros_like(rows), rows * 16, 0, 0, torch.empty_like(proj[:, :hd]), 0, 1, hd, hd,
-                   0, 0, 0, None, None, 0.125, 1.0, waves, shares)
-    assert torch.equal(kc[:, 0, 0].cpu(), want)
+    kc, vc = (torch.zeros(t, 1, 16, dim, device=_dev(), dtype=torch.bfloat16) for _ in range(2))
+    turn = (cos.to(_dev()), sin.to(_dev())) if rot else (none, none)
+    C.chunk_decode(None, proj, 0, rep * dim, (rep + 1) * dim, bias.to(_dev()).repeat(rep + 2), gain.to(_dev()), gain.to(_dev()), *turn, rot, eps, kc, vc, rows.view(t, 1), rows, rows, torch.full_like(rows, 5),
+                   rows * 16 + 5, 0, 0, torch.empty_like(proj[:, : rep * dim]), 0, rep, dim, dim, 0, 0, 0, None, None, 0.125, 1.0, waves, shares)
+    assert torch.equal(kc[:, 0, 5].cpu(), want)
+
+
+@pytest.mark.parametrize("one_row", [False, True])
+@pytest.mark.parametrize("dim,waves,shares", [(64, 4, 1), (128, 8, 3), (256, 4, 1)])
+def test_distance_biases_are_rounded_before_a_score_meets_them(C, dim, waves, shares, one_row):
+    """Scores that a bias cancels but for what its own rounding leaves, of up to half a unit: the weight of an earlier key beside the token's own, whose score is 0.
+    Weights and sums of two keys are bf16 or better: three roundings of at most 2^-8."""
+    nh, scale = 512, 2.0**19
+    gen = torch.Generator().manual_seed(dim)
+    k0 = (1 + torch.rand(nh, generator=gen)).bfloat16()
+    factor = 0.5 + torch.rand(nh, generator=gen) if one_row else torch.ones(nh)
+    log2e = np.float32(1.4426950408889634)
+    st, unit = 8 * k0.float().numpy(), np.float32(scale) * log2e
+    rel = torch.zeros(nh, 2)
+    rel[:, 1] = -torch.from_numpy(st.astype(np.float64) * scale).float() * factor
+    a, b = (st * unit, factor.numpy()) if one_row else (st, unit)
+    bias = rel[:, 1].numpy()
+    score, other = (a.astype(np.float64) * b + bias * log2e), (bias.astype(np.float64) * log2e + a * b)  # (one of the products exact, the other rounded)
+    weight = lambda s: torch.from_numpy(1 / (1 + np.exp2(-s)))  # noqa: E731
+    want, tol = weight(score), 3 * 2.0**-8
+    assert ((want - weight(other)).abs() > 2 * tol).sum() >= nh // 4
+    dev = lambda v: v.to(_dev())  # noqa: E731
+    proj = torch.zeros(1, 3 * nh * dim, dtype=torch.bfloat16)
+    proj[:, : nh * dim : dim] = 1.0  # (normed: the square root of dim; the gain makes it 8)
+    kc = torch.zeros(1, nh, 16, dim, dtype=torch.bfloat16)
+    kc[0, :, 0, 0] = k0
+    if one_row:
+        vc = factor.view(1, nh, 1, 1).expand(1, nh, 16, 1).contiguous()
+    else:
+        vc = torch.zeros_like(kc)
+        vc[0, :, 0, 0] = k0
+    gain, none, i32 = torch.full((dim,), 8 / dim**0.5), torch.zeros(0, device=_dev()), lambda *v: torch.tensor(v, device=_dev(), dtype=torch.int32)  # noqa: E731
+    out = torch.empty(1, nh * dim, device=_dev(), dtype=torch.bfloat16)
+    C.chunk_decode(None, dev(proj), 0, nh * dim, 2 * nh * dim, torch.zeros(3 * nh * dim, device=_dev()), dev(gain), torch.ones(dim, device=_dev()), none, none, 0, 1e-12, dev(kc), dev(vc), i32(0).view(1, 1),
+                   i32(0), i32(0), i32(1), i32(1), 0, 0, out, 0, nh, dim, dim, 0, 0, 0, None, dev(rel), scale, 1.0, waves, shares)
+    got = out.view(nh, dim)[:, 0].double().cpu() / k0.double()
+    assert (got - want).abs().max() <= tol
 
 
 @pytest.mark.parametrize("graphs,custom", [(False, True), (True, True), (False, False), (True, False)])
