@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include "elem.h"
+#include "state_rows.h"
 
 namespace {
 using namespace elem;
@@ -78,7 +79,9 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
   const int kind = a.tok_kind[t], slot = a.tok_seq[t], pos = a.positions[t];
   if (kind != 1) return;  // a padding row
   const int rep = a.heads / a.kv_heads, g = h / rep;
-  const int nc = a.vdim >> 2, nrg = 256 / nc;  // threads across the columns, row groups
+  const StateRows own = state_rows(tid, a.dim, a.vdim);
+  const int nrg = own.groups, rg = own.group, col = own.col;
+  const bool on = own.on();
   float* qs = sm;                       // [dim]
   float* ks = qs + a.dim;               // [dim]
   float* ds = ks + a.dim;               // [dim] decay factors
@@ -113,14 +116,10 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
   const float gain_of = a.o_norm[dv];
   __builtin_amdgcn_sched_barrier(0);
 
-  const int rg = tid / nc, col = (tid - rg * nc) * 4;
-  const bool on = rg < nrg;
-  // rows rg, rg + nrg, ... of the state (behind the last one: the first again, which nothing uses)
-  float* st = a.state + ((long long)slot * a.heads + h) * a.dim * a.vdim + (on && rg < a.dim ? rg * a.vdim + col : 0);
-  const int stride = nrg * a.vdim, mine = on && rg < a.dim ? (a.dim - rg + nrg - 1) / nrg : 0;
+  float* st = a.state + ((long long)slot * a.heads + h) * a.dim * a.vdim;
   float4 s[ROWS];
 #pragma unroll
-  for (int i = 0; i < ROWS; ++i) s[i] = ld4(st + (i < mine ? i * stride : 0));
+  for (int i = 0; i < ROWS; ++i) s[i] = ld4(st + own.at(i));
   __builtin_amdgcn_sched_barrier(0);
 
   float sq = 0.f, sk = 0.f;
@@ -169,7 +168,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
   float4 ak = make_float4(0.f, 0.f, 0.f, 0.f), aq = ak;
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) {
-    if (i < mine) {
+    if (i < own.count) {
       const int r = rg + i * nrg;
       const float dr = ds[r], kv = ks[r] * nk, qv = qs[r] * nq;
       s[i].x *= dr; s[i].y *= dr; s[i].z *= dr; s[i].w *= dr;
@@ -204,10 +203,10 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
     const float4 u = ld4(vs + col);
 #pragma unroll
     for (int i = 0; i < ROWS; ++i) {
-      if (i < mine) {
+      if (i < own.count) {
         const float kv = ks[rg + i * nrg] * nk;
         s[i].x += kv * u.x; s[i].y += kv * u.y; s[i].z += kv * u.z; s[i].w += kv * u.w;
-        st4(st + i * stride, s[i]);
+        st4(st + own.at(i), s[i]);
       }
     }
   }

@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "elem.h"
+#include "state_rows.h"
 
 struct KvrArgs {
   long long ldp; int q_off, k_off, v_off, g_off;
@@ -178,9 +179,9 @@ __global__ __launch_bounds__(256) void retention_step_kernel(const T* __restrict
   if (t < 0) return;  // unused entry
   const int kind = a.tok_kind[t], pos = a.positions[t], slot = a.tok_seq[t];
   if (kind != 1) return;  // a padding row
-  const int nc = a.dvp >> 2, nrg = 256 / nc;
-  const int rg = tid / nc, col = (tid - rg * nc) * 4;
-  const bool on = rg < nrg;
+  const StateRows own = state_rows(tid, a.dimp, a.dvp);
+  const int nrg = own.groups, rg = own.group, col = own.col;
+  const bool on = own.on();
   float* qs = sm;               // [dimp]
   float* ks = qs + a.dimp;      // [dimp]
   float* red = ks + a.dimp;     // [nrg][dvp]
@@ -198,12 +199,10 @@ __global__ __launch_bounds__(256) void retention_step_kernel(const T* __restrict
   const unsigned int gate_of = raw(pr + a.g_off + h * a.vdim + (tid < a.vdim ? tid : 0));
   __builtin_amdgcn_sched_barrier(0);
 
-  // rows rg, rg + nrg, ... of the state (behind the last one: the first again, which nothing uses)
-  float* st = a.state + ((long long)slot * a.heads + h) * a.dimp * a.dvp + (on ? rg * a.dvp + col : 0);
-  const int stride = nrg * a.dvp, mine = on && rg < a.dimp ? (a.dimp - rg + nrg - 1) / nrg : 0;
+  float* st = a.state + ((long long)slot * a.heads + h) * a.dimp * a.dvp;
   float4 m[STEP_ROWS];
 #pragma unroll
-  for (int u = 0; u < STEP_ROWS; ++u) m[u] = ld4(st + (u < mine ? u * stride : 0));
+  for (int u = 0; u < STEP_ROWS; ++u) m[u] = ld4(st + own.at(u));
   __builtin_amdgcn_sched_barrier(0);
 
   if (d0 < a.dimp) {
@@ -230,11 +229,11 @@ __global__ __launch_bounds__(256) void retention_step_kernel(const T* __restrict
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int u = 0; u < STEP_ROWS; ++u) {
-    if (u < mine) {
+    if (u < own.count) {
       const float k = ks[rg + u * nrg], q = qs[rg + u * nrg];
       m[u].x = m[u].x * g + k * v[0]; m[u].y = m[u].y * g + k * v[1]; m[u].z = m[u].z * g + k * v[2]; m[u].w = m[u].w * g + k * v[3];
       o.x += q * m[u].x; o.y += q * m[u].y; o.z += q * m[u].z; o.w += q * m[u].w;
-      st4(st + u * stride, m[u]);
+      st4(st + own.at(u), m[u]);
     }
   }
   if (on) st4(red + rg * a.dvp + col, o);

@@ -24,6 +24,7 @@
 // when a slot changes hands.  Channels are ordered x [heads vdim], b [groups dim], c [groups dim].
 
 #include "attn_tiles.h"
+#include "state_rows.h"
 
 struct KvsArgs {
   long long ldp; int z_off, x_off, dt_off;
@@ -75,9 +76,9 @@ __global__ __launch_bounds__(256) void space_step_kernel(const T* __restrict__ p
   const int kind = a.tok_kind[t], pos = a.positions[t], slot = a.tok_seq[t];
   if (kind != 1) return;  // a padding row
   const int rep = a.heads / a.groups, g = h / rep, inner = a.heads * a.vdim;
-  const int nc = a.dvp >> 2, nrg = 256 / nc;
-  const int rg = tid / nc, col = (tid - rg * nc) * 4;
-  const bool on = rg < nrg;
+  const StateRows own = state_rows(tid, a.dimp, a.dvp);
+  const int nrg = own.groups, rg = own.group, col = own.col;
+  const bool on = own.on();
   float* bs = sm;              // [dimp]: dt b
   float* cs = bs + a.dimp;     // [dimp]
   float* xs = cs + a.dimp;     // [dvp]
@@ -112,14 +113,13 @@ __global__ __launch_bounds__(256) void space_step_kernel(const T* __restrict__ p
   const unsigned int dt_of = raw(proj + t * a.ldp + a.dt_off + h);
   __builtin_amdgcn_sched_barrier(0);
 
-  // rows rg, rg + nrg, ... of the state, U at a time (behind the last one: the first again, which nothing uses)
-  float* st = a.state + ((long long)slot * a.heads + h) * a.dimp * a.dvp + (on && rg < a.dimp ? rg * a.dvp + col : 0);
-  const int stride = nrg * a.dvp, mine = on && rg < a.dimp ? (a.dimp - rg + nrg - 1) / nrg : 0, most = (a.dimp + nrg - 1) / nrg;
+  float* st = a.state + ((long long)slot * a.heads + h) * a.dimp * a.dvp;
+  const int most = (a.dimp + nrg - 1) / nrg;  // rows of a thread, U at a time
   constexpr int U = 8;
   float4 s[U];
   auto fetch = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) s[u] = ld4(st + (i0 + u < mine ? (i0 + u) * stride : 0));
+    for (int u = 0; u < U; ++u) s[u] = ld4(st + own.at(i0 + u));
   };
   fetch(0);
   __builtin_amdgcn_sched_barrier(0);
@@ -159,12 +159,12 @@ __global__ __launch_bounds__(256) void space_step_kernel(const T* __restrict__ p
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (i0 + u < mine) {
+      if (i0 + u < own.count) {
         const int r = rg + (i0 + u) * nrg;
         const float b = bs[r], c = cs[r];
         s[u].x = s[u].x * decay + b * x.x; s[u].y = s[u].y * decay + b * x.y; s[u].z = s[u].z * decay + b * x.z; s[u].w = s[u].w * decay + b * x.w;
         o.x += c * s[u].x; o.y += c * s[u].y; o.z += c * s[u].z; o.w += c * s[u].w;
-        st4(st + (i0 + u) * stride, s[u]);
+        st4(st + own.at(i0 + u), s[u]);
       }
     }
   }

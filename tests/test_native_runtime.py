@@ -55,6 +55,18 @@ def test_ring_buffer_stress_under_sanitizers(tmp_path, flags, env):
     assert "0 bad" in run.stdout and "WARNING: ThreadSanitizer" not in run.stderr and "ERROR: AddressSanitizer" not in run.stderr and "runtime error" not in run.stderr
 
 
+def test_threads_read_their_heads_state_and_nothing_else(tmp_path):
+    """Offsets of the kernels for single tokens (retention, delta rule, state spaces), worked out on the host for every thread: heads of fewer rows than
+    there are row groups, columns that do not fill the threads, the smallest and the largest."""
+    cxx = os.environ.get("CXX", "g++")
+    if shutil.which(cxx) is None:
+        pytest.skip("no C++ compiler")
+    exe = tmp_path / "state_rows"
+    subprocess.run([cxx, "-std=c++17", "-O2", "-D__host__=", "-D__device__=", os.path.join(ROOT, "csrc/tests/state_rows_check.cpp"), "-o", str(exe)], check=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0 and run.stdout.endswith(" 0 bad\n"), run.stdout
+
+
 def test_makefile_has_the_sanitize_target():
     mk = open(os.path.join(ROOT, "Makefile")).read()
     assert "sanitize:" in mk and "-fsanitize=thread" in mk and "-fsanitize=address,undefined" in mk and "ring_stress" in mk
