@@ -48,18 +48,37 @@ __device__ inline int chan_col(const DeltaArgs& a, int c) {
   return c < qk ? a.q_off + c : c < 2 * qk ? a.k_off + c - qk : a.v_off + c - 2 * qk;
 }
 
+// a convolution's sum: the first product is not rounded, the second one is (said here, else it is the compiler's choice at each place)
+template <int TAPS>
+__device__ inline float taps_sum(const float (&w)[TAPS], const float (&x)[TAPS]) {
+  if constexpr (TAPS == 1) return w[0] * x[0];
+  else {
+    float y = __builtin_fmaf(w[0], x[0], w[1] * x[1]);
+#pragma unroll
+    for (int j = 2; j < TAPS; ++j) y = __builtin_fmaf(w[j], x[j], y);
+    return y;
+  }
+}
+
 // silu(convolution) of channel c at row t; `back` = rows of the same portion in front of t.  TAPS: compile-time taps (0: a.taps)
 template <typename T, int TAPS>
 __device__ inline float conv_silu(const DeltaArgs& a, const T* __restrict__ proj, const T* __restrict__ ring, long long t, int pos, int back, int slot, int c) {
   const T* p = proj + t * a.ldp + chan_col(a, c);
   const int taps = TAPS ? TAPS : a.taps;
-  float y = a.conv_w[(taps - 1) * a.channels + c] * ld(p);
-#pragma unroll
-  for (int j = 1; j < taps; ++j) {
+  auto weight = [&](int j) { return a.conv_w[(taps - 1 - j) * a.channels + c]; };
+  auto input = [&](int j) {
     const T* src = j <= back ? p - j * a.ldp : ring + ((long long)slot * taps + (j <= pos ? pos - j : 0) % taps) * a.channels + c;
     const float x = ld(src);
-    y += a.conv_w[(taps - 1 - j) * a.channels + c] * (j <= pos ? x : 0.f);
+    return j <= pos ? x : 0.f;
+  };
+  if constexpr (TAPS > 0) {
+    float w[TAPS], x[TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) { w[j] = weight(j); x[j] = j ? input(j) : ld(p); }
+    return silu(taps_sum<TAPS>(w, x));
   }
+  float y = weight(0) * ld(p);
+  for (int j = 1; j < taps; ++j) y += weight(j) * input(j);
   return silu(y);
 }
 
@@ -135,10 +154,10 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
     if (is_decay(i)) {
       keep(i, fast_exp(-fast_exp(w[e][1]) * softplus(number<T>(x[e][0]) + w[e][0])));
     } else {
-      float y = w[e][0] * number<T>(x[e][0]);
+      float v[SIZE];
 #pragma unroll
-      for (int m = 1; m < TAPS; ++m) y += w[e][m] * (m <= pos ? number<T>(x[e][m]) : 0.f);
-      keep(i, silu(y));
+      for (int m = 0; m < SIZE; ++m) v[m] = m <= pos ? number<T>(x[e][m]) : 0.f;
+      keep(i, silu(taps_sum<SIZE>(w[e], v)));
     }
   }
   for (int i = tid + 256 * EARLY; i < items; i += 256)

@@ -319,6 +319,43 @@ def test_delta_rule_alone(backend, heads, kv, dim, vdim, taps, strong):
         assert bool((state[0] == 7).all()) and bool((state[2] == 7).all()) and bool((ring[0] == 7).all()) and bool((ring[2] == 7).all())
 
 
+def delta_steps(dim, vdim, taps, ty, w, heads, proj, low, steps):
+    """The state that single tokens of four sequences leave: ``proj`` and ``low`` of a step, weights (convolutions [taps][channels], decays, steps)."""
+    mx, n = mixers_of("cuda:0"), 4
+    m = hybrid.DeltaSpec(heads, heads, dim, vdim, taps)
+    qk = heads * dim
+    offs = [0, qk, 2 * qk, 2 * qk + heads * vdim, 0, 0, 0, qk, 0]
+    state = torch.full((n + 1, heads, dim, vdim), 7.0, device="cuda:0")
+    ds = mx.DeltaState(m, hybrid.DeltaWeights(*offs, None, *(x.cuda().contiguous() for x in w), torch.ones(vdim, device="cuda:0")), 1.0, 1e-5, state, torch.full((n + 1, taps, m.channels), 7.0, dtype=ty, device="cuda:0"))
+    for p in range(steps):
+        st = make_step(mx, [(1, p, s + 1) for s in range(n)], "cuda:0", per=1)
+        x, lo = (torch.zeros(st.rows, (y.shape[2] + 7) // 8 * 8, dtype=ty, device="cuda:0") for y in (proj, low))
+        x[:n, : proj.shape[2]], lo[:n, : low.shape[2]] = proj[p].to(ty), low[p].to(ty)
+        ds.run(x, lo, torch.zeros(st.rows, heads * vdim, dtype=ty, device="cuda:0"), st)
+    return state.cpu()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ty", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim,vdim,taps", [(64, 512, 2), (128, 128, 2), (256, 128, 2), (64, 64, 2), (128, 128, 3), (64, 512, 3), (128, 128, 4), (64, 512, 4)])
+def test_convolutions_of_delta_steps_round_the_last_tokens_product_once(ty, dim, vdim, taps):
+    """Values whose last two products cancel: what is left is the rounding of the one before, half of which is the value (silu of a number next to zero).  Old states are wiped,
+    keys are all the same."""
+    heads, first = 2, 30 / math.log(2)
+    gen = torch.Generator().manual_seed(dim + vdim)
+    x, c = torch.randn(4, heads * vdim, generator=gen).to(ty).float(), torch.randn(heads * vdim, generator=gen)
+    conv = torch.zeros(taps, 2 * heads * dim + heads * vdim)
+    conv[taps - 1, : 2 * heads * dim] = 1.0
+    conv[taps - 1, 2 * heads * dim :], conv[taps - 2, 2 * heads * dim :] = c, -c
+    proj = torch.cat((torch.ones(4, 2 * heads * dim), x, torch.full((4, heads), first)), -1).expand(2, -1, -1)
+    low = torch.cat((torch.full((4, heads * dim), 100.0), torch.zeros(4, heads * vdim)), -1).expand(2, -1, -1)
+    state = delta_steps(dim, vdim, taps, ty, (conv, torch.full((heads,), 4.0), torch.zeros(heads * dim)), heads, proj, low, 2)[1:]
+    exact = c.double() * x.double()
+    left = (exact - (c * x).double()).view(4, heads, 1, vdim)
+    assert (left != 0).float().mean() > 0.5
+    assert (state * dim**0.5 - left / 2).abs().max() <= 1e-5 * left.abs().max()
+
+
 @pytest.mark.parametrize("backend", BACKENDS)
 @pytest.mark.parametrize("width", [72, 300, 2048, 4500])
 def test_gated_residual_and_embedding_alone(backend, width):
