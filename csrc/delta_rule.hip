@@ -93,7 +93,7 @@ template <typename T, int ROWS, int TAPS>
 __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__ rows, const T* __restrict__ proj, const T* __restrict__ low, T* __restrict__ ring, T* __restrict__ out, DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const long long t = rows[blockIdx.x];
-  const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (t < 0) return;  // unused entry
   const int kind = a.tok_kind[t], slot = a.tok_seq[t], pos = a.positions[t];
   if (kind != 1) return;  // a padding row
@@ -107,9 +107,23 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
   float* vs = ds + a.dim;               // [vdim]
   float* red = vs + a.vdim;             // [2][nrg][vdim]
   __shared__ float scal[4][4];
-  const int qk = a.kv_heads * a.dim, items = 3 * a.dim + a.vdim;  // what the state meets: queries, keys, decays, values, dealt over the threads
-  auto channel = [&](int i) { return i < 2 * a.dim ? (i < a.dim ? i : i - a.dim + qk) + g * a.dim : 2 * qk + h * a.vdim + i - 3 * a.dim; };
-  auto is_decay = [&](int i) { return i >= 2 * a.dim && i < 3 * a.dim; };
+  const int qk = a.kv_heads * a.dim;
+  // What the state meets: queries, keys, decays, values, dealt over the waves in parts of 64.  Each kind begins with a part (heads of more than 256: with the first
+  // wave's), so that the lanes that add up squares are the same whatever lies in front of them, and a part is of one kind
+  const int section = a.dim <= 256 ? (a.dim + 63) & ~63 : (a.dim + 255) & ~255, parts = (3 * section + a.vdim + 63) >> 6;
+  struct Item { int kind, d; bool there; };  // kind: 0 query, 1 key, 2 decay, 3 value
+  auto item = [&](int part) {
+    Item it;
+    it.kind = (64 * part >= section) + (64 * part >= 2 * section) + (64 * part >= 3 * section);
+    it.d = 64 * part - it.kind * section + lane;
+    it.there = it.d < (it.kind == 3 ? a.vdim : a.dim);
+    it.d = it.there ? it.d : 0;
+    return it;
+  };
+  const int q_channel = g * a.dim, k_channel = qk + q_channel, v_channel = 2 * qk + h * a.vdim;
+  const int q_column = a.q_off + q_channel, k_column = a.k_off + q_channel, v_column = a.v_off + h * a.vdim;  // of the projections
+  auto channel = [&](const Item& it) { return (it.kind == 3 ? v_channel : it.kind == 1 ? k_channel : q_channel) + it.d; };
+  auto column = [&](const Item& it) { return (it.kind == 3 ? v_column : it.kind == 1 ? k_column : q_column) + it.d; };
 
   // the first items of a thread, as loaded: no branches and no conversions, which would wait for them
   constexpr int EARLY = TAPS >= 2 ? 2 : 0, SIZE = TAPS >= 2 ? TAPS : 2;
@@ -117,10 +131,10 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
   float w[2][SIZE];
 #pragma unroll
   for (int e = 0; e < EARLY; ++e) {
-    const int i = tid + 256 * e < items ? tid + 256 * e : items - 1;
-    const bool decay = is_decay(i);
-    const int c = decay ? 0 : channel(i), d = decay ? h * a.dim + i - 2 * a.dim : 0;
-    x[e][0] = raw(decay ? low + t * a.ldl + a.z_off + d : proj + t * a.ldp + chan_col(a, c));
+    const Item it = item(wave + 4 * e);
+    const bool decay = it.kind == 2;
+    const int c = decay ? 0 : channel(it), d = decay ? h * a.dim + it.d : 0;
+    x[e][0] = raw(decay ? low + t * a.ldl + a.z_off + d : proj + t * a.ldp + column(it));
     w[e][0] = *(decay ? a.dt_bias + d : a.conv_w + (TAPS - 1) * a.channels + c);
 #pragma unroll
     for (int m = 1; m < TAPS; ++m) {
@@ -142,36 +156,41 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
   __builtin_amdgcn_sched_barrier(0);
 
   float sq = 0.f, sk = 0.f;
-  auto keep = [&](int i, float y) {
-    sm[i] = y;  // (q, k, decays and v lie one behind another)
-    sq += i < a.dim ? y * y : 0.f;
-    sk += i >= a.dim && i < 2 * a.dim ? y * y : 0.f;
+  auto keep = [&](const Item& it, float y) {
+    if (it.there) sm[it.kind * a.dim + it.d] = y;  // (q, k, decays and v lie one behind another)
+    const float q = it.there && it.kind == 0 ? y : 0.f, k = it.there && it.kind == 1 ? y : 0.f;
+    sq = __builtin_fmaf(q, q, sq);
+    sk = __builtin_fmaf(k, k, sk);
   };
 #pragma unroll
   for (int e = 0; e < EARLY; ++e) {
-    const int i = tid + 256 * e;
-    if (i >= items) continue;
-    if (is_decay(i)) {
-      keep(i, fast_exp(-fast_exp(w[e][1]) * softplus(number<T>(x[e][0]) + w[e][0])));
+    if (wave + 4 * e >= parts) continue;
+    const Item it = item(wave + 4 * e);
+    if (it.kind == 2) {
+      keep(it, fast_exp(-fast_exp(w[e][1]) * softplus(number<T>(x[e][0]) + w[e][0])));
     } else {
       float v[SIZE];
 #pragma unroll
       for (int m = 0; m < SIZE; ++m) v[m] = m <= pos ? number<T>(x[e][m]) : 0.f;
-      keep(i, silu(taps_sum<SIZE>(w[e], v)));
+      keep(it, silu(taps_sum<SIZE>(w[e], v)));
     }
   }
-  for (int i = tid + 256 * EARLY; i < items; i += 256)
-    keep(i, is_decay(i) ? fast_exp(decay_log(a, ld(low + t * a.ldl + a.z_off + h * a.dim + i - 2 * a.dim), h, i - 2 * a.dim)) : conv_silu<T, TAPS>(a, proj, ring, t, pos, 0, slot, channel(i)));
+  for (int part = wave + 4 * EARLY; part < parts; part += 4) {
+    const Item it = item(part);
+    keep(it, it.kind == 2 ? fast_exp(decay_log(a, ld(low + t * a.ldl + a.z_off + h * a.dim + it.d), h, it.d)) : conv_silu<T, TAPS>(a, proj, ring, t, pos, 0, slot, channel(it)));
+  }
   sq = wave_sum(sq);
   sk = wave_sum(sk);
-  if (lane == 0) { scal[0][wave] = sq; scal[1][wave] = sk; }
+  if (lane == 0) { scal[0][wave] = sq; scal[1][(wave - section / 64) & 3] = sk; }  // by their part of 64 of a head
   // the ring entry of this position was last used for position pos - taps, which nobody reads any more
   T* rw = ring + ((long long)slot * a.taps + pos % a.taps) * a.channels;
-  for (int e = 0, i = tid; i < items; ++e, i += 256)
-    if (!is_decay(i) && (i >= 3 * a.dim || h % rep == 0)) {
-      const int c = channel(i);
-      elem::st(rw + c, e < EARLY ? number<T>(x[e & 1][0]) : ld(pr + chan_col(a, c)));
-    }
+  auto pass_on = [&](const Item& it, float v) { elem::st(rw + channel(it), v); };
+  auto passed_on = [&](const Item& it) { return it.there && (it.kind == 3 || (it.kind != 2 && h % rep == 0)); };
+#pragma unroll
+  for (int e = 0; e < EARLY; ++e)
+    if (const Item it = item(wave + 4 * e); passed_on(it)) pass_on(it, number<T>(x[e][0]));
+  for (int part = wave + 4 * EARLY; part < parts; part += 4)
+    if (const Item it = item(part); passed_on(it)) pass_on(it, ld(pr + column(it)));
   __syncthreads();
   const float nq = 1.f / (sqrtf(scal[0][0] + scal[0][1] + scal[0][2] + scal[0][3] + 1e-6f) * sqrtf((float)a.dim));
   const float nk = 1.f / sqrtf(scal[1][0] + scal[1][1] + scal[1][2] + scal[1][3] + 1e-6f);

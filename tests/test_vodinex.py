@@ -337,6 +337,24 @@ def delta_steps(dim, vdim, taps, ty, w, heads, proj, low, steps):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("ty", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim,longer,vdim,taps", [(96, 128, 64, 4), (40, 64, 48, 3), (192, 256, 64, 4), (130, 192, 128, 2), (100, 128, 128, 1), (320, 512, 64, 4), (260, 512, 40, 5)])
+def test_keys_of_delta_steps_are_normed_alike_in_longer_heads(ty, dim, longer, vdim, taps):
+    """Zeros behind a head's keys change none of its state's bits: squares are added up by places in the head, not by what the head's other numbers are."""
+    heads, steps = 3, 5
+    gen = torch.Generator().manual_seed(dim)
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    key, value, beta, z, gate = rnd(steps, 4, heads, dim), rnd(steps, 4, heads * vdim), rnd(steps, 4, heads), rnd(steps, 4, heads, dim), rnd(steps, 4, heads * vdim)
+    ck, cv, a_log, dt = rnd(taps, heads, dim), rnd(taps, heads * vdim), rnd(heads) - 2, rnd(heads, dim)
+    states = []
+    for size in (dim, longer):
+        pad = lambda x: torch.nn.functional.pad(x, (0, size - dim)).flatten(-2)  # noqa: B023, E731
+        w = torch.cat((pad(ck), pad(ck), cv), -1), a_log, pad(dt)
+        states.append(delta_steps(size, vdim, taps, ty, w, heads, torch.cat((pad(key), pad(key), value, beta), -1), torch.cat((pad(z), gate), -1), steps)[1:, :, :dim])
+    assert torch.equal(*states) and states[0].isfinite().all() and states[0].std() > 0.01
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ty", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("dim,vdim,taps", [(64, 512, 2), (128, 128, 2), (256, 128, 2), (64, 64, 2), (128, 128, 3), (64, 512, 3), (128, 128, 4), (64, 512, 4)])
 def test_convolutions_of_delta_steps_round_the_last_tokens_product_once(ty, dim, vdim, taps):
     """Values whose last two products cancel: what is left is the rounding of the one before, half of which is the value (silu of a number next to zero).  Old states are wiped,
