@@ -85,11 +85,11 @@ __device__ inline float conv_silu(const DeltaArgs& a, const T* __restrict__ proj
 __device__ inline float decay_log(const DeltaArgs& a, float z, int h, int d) { return -fast_exp(a.a_log[h]) * softplus(z + a.dt_bias[h * a.dim + d]); }
 
 // ---- decoding ----------------------------------------------------------------------------------------------------
-// grid (listed rows, heads), 256 threads: thread = (row group, 4 columns); ROWS = rows of S per thread.  With many rows the state bounds it (read and written, 5 TB/s);
+// grid (listed rows, heads), 256 threads: thread = (row group, 4 columns); ROWS = rows of S per thread, EARLY = items of a thread that are asked for ahead of S.  With many rows the state bounds it (read and written, 5 TB/s);
 // with few of them a chain of dependent steps does: loads answer in the order they were asked for, so what the convolutions, decays and gates need is asked for ahead
 // of the state, and all of that is worked out while the state is on its way from HBM; nothing is loaded behind it.  Key and query are normed where they are used, so that
 // the sums of their squares and their product cost no barrier of their own.  6 rows of 16 heads of 128 x 128 11.7 -> 9.8 us, 61 of 32 heads 62.9 -> 50.9.
-template <typename T, int ROWS, int TAPS>
+template <typename T, int ROWS, int TAPS, int EARLY>
 __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__ rows, const T* __restrict__ proj, const T* __restrict__ low, T* __restrict__ ring, T* __restrict__ out, DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const long long t = rows[blockIdx.x];
@@ -116,8 +116,9 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
     Item it;
     it.kind = (64 * part >= section) + (64 * part >= 2 * section) + (64 * part >= 3 * section);
     it.d = 64 * part - it.kind * section + lane;
-    it.there = it.d < (it.kind == 3 ? a.vdim : a.dim);
-    it.d = it.there ? it.d : 0;
+    const int size = it.kind == 3 ? a.vdim : a.dim;
+    it.there = it.d < size;
+    it.d = it.d < size - 1 ? it.d : size - 1;  // (behind the last one: that one again)
     return it;
   };
   const int q_channel = g * a.dim, k_channel = qk + q_channel, v_channel = 2 * qk + h * a.vdim;
@@ -125,8 +126,9 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
   auto channel = [&](const Item& it) { return (it.kind == 3 ? v_channel : it.kind == 1 ? k_channel : q_channel) + it.d; };
   auto column = [&](const Item& it) { return (it.kind == 3 ? v_column : it.kind == 1 ? k_column : q_column) + it.d; };
 
-  // the first items of a thread, as loaded: no branches and no conversions, which would wait for them
-  constexpr int EARLY = TAPS >= 2 ? 2 : 0, SIZE = TAPS >= 2 ? TAPS : 2;
+  // the first EARLY items of a thread, as loaded: no branches and no conversions, which would wait for them
+  static_assert(EARLY == 0 || TAPS >= 2, "a convolution of known taps has at least the two words of a decay");
+  constexpr int SIZE = TAPS >= 2 ? TAPS : 2;
   unsigned int x[2][SIZE];
   float w[2][SIZE];
 #pragma unroll
@@ -157,8 +159,9 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const int* __restrict__
 
   float sq = 0.f, sk = 0.f;
   auto keep = [&](const Item& it, float y) {
-    if (it.there) sm[it.kind * a.dim + it.d] = y;  // (q, k, decays and v lie one behind another)
-    const float q = it.there && it.kind == 0 ? y : 0.f, k = it.there && it.kind == 1 ? y : 0.f;
+    sm[it.kind * a.dim + it.d] = y;  // (q, k, decays and v lie one behind another; what several lanes write is the same)
+    y = it.there && it.kind < 2 ? y : 0.f;
+    const float q = it.kind == 0 ? y : 0.f, k = it.kind == 1 ? y : 0.f;
     sq = __builtin_fmaf(q, q, sq);
     sk = __builtin_fmaf(k, k, sk);
   };
@@ -922,8 +925,11 @@ int kvd_step(const KvdArgs* k, const void* proj, const void* low, void* ring, vo
   const DeltaArgs a = args_of(*k);
   const size_t lds = (size_t)(3 * a.dim + a.vdim + 2 * (256 / (a.vdim >> 2)) * a.vdim) * 4;
   const dim3 grid(n_rows, a.heads);
-#define KV_ST1(Tt, R, TP) hipLaunchKernelGGL((delta_step_kernel<Tt, R, TP>), grid, dim3(256), lds, s, row_list, (const Tt*)proj, (const Tt*)low, (Tt*)ring, (Tt*)out, a)
-#define KV_ST(Tt, R) do { if (a.taps == 4) KV_ST1(Tt, R, 4); else if (a.taps == 3) KV_ST1(Tt, R, 3); else if (a.taps == 2) KV_ST1(Tt, R, 2); else KV_ST1(Tt, R, 0); } while (0)
+  // Heads of up to 64 x 64 are one item a thread: asking for a second one, for nothing, made 61 rows of 16 such heads 10.4 us (9.95 without)
+  const bool one_item = a.dim <= 64 && a.vdim <= 64;
+#define KV_ST1(Tt, R, TP, E) hipLaunchKernelGGL((delta_step_kernel<Tt, R, TP, E>), grid, dim3(256), lds, s, row_list, (const Tt*)proj, (const Tt*)low, (Tt*)ring, (Tt*)out, a)
+#define KV_STE(Tt, R, TP) do { if (R == 4 && one_item) KV_ST1(Tt, 4, TP, 1); else KV_ST1(Tt, R, TP, 2); } while (0)
+#define KV_ST(Tt, R) do { if (a.taps == 4) KV_STE(Tt, R, 4); else if (a.taps == 3) KV_STE(Tt, R, 3); else if (a.taps == 2) KV_STE(Tt, R, 2); else KV_ST1(Tt, R, 0, 0); } while (0)
 #define KV_ST2(R) do { if (f32) KV_ST(float, R); else KV_ST(bf16raw, R); } while (0)
   switch (rows) {
     case 4: KV_ST2(4); break;
@@ -933,6 +939,7 @@ int kvd_step(const KvdArgs* k, const void* proj, const void* low, void* ring, vo
   }
 #undef KV_ST2
 #undef KV_ST
+#undef KV_STE
 #undef KV_ST1
   return (int)hipGetLastError();
 }
