@@ -995,6 +995,40 @@ def test_distance_biases_are_rounded_before_a_score_meets_them(C, dim, waves, sh
     assert (got - want).abs().max() <= tol
 
 
+@pytest.mark.parametrize("rank,rot", [(128, 0), (256, 64), (512, 64)])
+def test_latent_rows_joined_of_any_number_of_shares(C, rank, rot):
+    """Rows of few and many keys in 2 to 64 shares (16 of them are joined at a time) against one share: the latents and the outputs are rounded to bf16, 2^-9 of each
+    either way; unused entries and padding rows are left alone."""
+    from kvmini.ops.hip_mixers import FragmentLayout
+
+    nh, dim, vdim, bs, lens = 20, 64, 64, 16, [4100, 1, 0, 700, 64, 2200]
+    t, per, rt = len(lens), 257, 64 if rot else 0
+    gen = torch.Generator(device=_dev()).manual_seed(rank)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device=_dev())  # noqa: E731
+    i32 = lambda v: torch.tensor(v, device=_dev(), dtype=torch.int32)  # noqa: E731
+    bt = torch.randperm(t * per, device=_dev(), generator=gen).view(t, per).int()
+    pos = i32([max(n - 1, 0) for n in lens])
+    slots = i32([int(bt[i, (n - 1) // bs]) * bs + (n - 1) % bs if n else -1 for i, n in enumerate(lens)])
+    cache = rnd(t * per, 1, bs, rank + rt).bfloat16()
+    off = [0, nh * dim, nh * (dim + rt), nh * (dim + rt)]
+    proj = rnd(t, nh * (dim + rt + vdim)).bfloat16()
+    absorb, up = FragmentLayout._pack(0.1 * rnd(nh, rank, dim).bfloat16()), FragmentLayout._pack(rnd(nh, vdim, rank).bfloat16())
+    turn = (torch.zeros(5000, rot // 2, device=_dev()) + 0.6, torch.zeros(5000, rot // 2, device=_dev()) + 0.8) if rot else (None, None)
+
+    def run(shares):
+        out = torch.full((t, nh * vdim), 7.0, device=_dev(), dtype=torch.bfloat16)
+        C.latent_rows(proj, off[0], off[1], 0, 0, off[3], True, absorb, up, None, rank, 1e-5, *turn, cache, False, True, bt, i32([0, 1, 2, 3, -1, 5]), i32(list(range(t))), pos, slots, out, 0, vdim, 0, 0.1, 1.0, shares, 1)
+        return out
+
+    want = run(1).float()
+    assert (want[[2, 4]] == 7).all() and want.isfinite().all()
+    for shares in (2, 15, 16, 17, 32, 33, 40, 64):
+        got = run(shares).float()
+        assert (got[[2, 4]] == 7).all()
+        for i in (0, 1, 3, 5):
+            assert (got[i] - want[i]).norm() <= 4 * 2.0**-9 * want[i].norm(), (shares, i)
+
+
 @pytest.mark.parametrize("graphs,custom", [(False, True), (True, True), (False, False), (True, False)])
 def test_engine_tp_collective_path_on_one_gpu(graphs, custom):
     """The tensor-parallel code path with a one-rank group must reproduce the plain engine's
