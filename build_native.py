@@ -33,9 +33,10 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 # given wrong results on gfx950 in some of their forms: no device code is compiled with them.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # A kernel's first arguments (up to 14 words; pointers and numbers, no structs) arrive in scalar registers with the wave instead of being its first load: 0.1 to 0.2 us
-# of each launch in a captured graph, whose 30 to 60 launches wait for one another.  One row of four 1B layers 220.9 -> 215.4 us, six of a hybrid 318.8 ->
-# 313.3, 20 rows of 8B layers 441 -> 436, prompts of thousands of rows the same.  Launches that are not part of a graph take 0.2 us longer so (MI355X, chains of one small
-# kernel: 2.6 and 2.9 us): what is not captured is built without.
+# of each launch in a captured graph, whose 30 to 60 launches wait for one another.  One row of four 1B layers 220.9 -> 214.1 us, six of a hybrid 318.8 ->
+# 313.3, 20 rows of 8B layers 441 -> 433, prompts of thousands of rows the same.  Launches that are not part of a graph take 0.2 us longer so (MI355X, chains of one small
+# kernel: 2.6 and 2.9 us): what is never captured is built without.  Steps without a graph lose nothing: few rows are bound by the host (one row of 1B layers 279 us without
+# and 279 with), the others gain as in a graph (20 rows of 8B layers 450.6 and 442.8, 16 of zipelix's 1614 and 1604, prompts of 4 x 60 tokens 418.9 and 411.9).
 ARGUMENTS_IN_REGISTERS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 EAGER_SOURCES = {"hist_quantile.hip", "energy_trapz.hip", "sampling.hip", "guided.hip", "xgmi_collectives.hip"}
 
