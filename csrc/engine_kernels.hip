@@ -307,6 +307,7 @@ struct PrefetchPlan {
   int gx, gy, nw, kib;
   long long tile_bytes, split_bytes;
   int wgs;                    // prefetch workgroups in this launch, a multiple of 8
+  int mxfp4;                  // the weights' order goes by it
   unsigned int* sink;         // never written in practice; keeps the loads alive
 };
 
@@ -331,7 +332,7 @@ __device__ inline void prefetch_role(const PrefetchPlan& pf, int j0, int lin, in
     const int g = 8 * ii + x;
     const int by = g / pf.gx, bx = g - by * pf.gx;
     const int units = (int)(pf.tile_bytes >> 10), u0 = by * (int)(pf.split_bytes >> 10);
-    const bool grouped = frag_grouped((long long)pf.gx * pf.nw * 16, units);
+    const bool grouped = frag_grouped((long long)pf.gx * pf.nw * 16, units, pf.mxfp4);
     const uint4* p = reinterpret_cast<const uint4*>(pf.base) + frag_first(bx * pf.nw + w, units, grouped) * 64 + lane;
     for (int k = 0; k < pf.kib && u0 + k < units; ++k) asm volatile("global_load_dwordx4 %0, %1, off" : "+v"(scratch) : "v"(p + frag_behind(u0 + k, grouped) * 64) : "memory");
   }
@@ -2814,14 +2815,14 @@ __global__ __launch_bounds__(256) void swiglu_interleaved_kernel(const unsigned 
 // Host-side check of a prefetch plan against the weight allocation it points into: every range
 // the prefetch workgroups will read must lie inside [base, base + bytes).
 int make_prefetch_plan(const void* base, const long long* v, unsigned int* sink, PrefetchPlan* out) {
-  const long long gx = v[0], gy = v[1], nw = v[2], kib = v[3], tile_bytes = v[4], split_bytes = v[5], wgs = v[6], bytes = v[7];
+  const long long gx = v[0], gy = v[1], nw = v[2], kib = v[3], tile_bytes = v[4], split_bytes = v[5], wgs = v[6], bytes = v[7], mxfp4 = v[8];
   if (gx < 1 || gy < 1 || nw < 1 || kib < 1 || wgs < 8 || (wgs & 7) || wgs > 65536 || gx * gy > (1 << 20)) return -1;
   if (tile_bytes < 1024 || (tile_bytes & 1023) || split_bytes < 1024 || (split_bytes & 1023) || ((uintptr_t)base & 15)) return -1;
   if (kib * 1024 > split_bytes) return -1;
   // the last range starts at ((gx * nw - 1) * tile_bytes + (gy - 1) * split_bytes) and is kib KiB long; tiles lie one behind another or in whole groups,
   // and what a range has past its tile's end is not read
   if ((gx * nw - 1) * tile_bytes + (gy - 1) * split_bytes + kib * 1024 > bytes || gx * nw > bytes / tile_bytes) return -1;
-  *out = PrefetchPlan{(const unsigned char*)base, (int)gx, (int)gy, (int)nw, (int)kib, tile_bytes, split_bytes, (int)wgs, sink};
+  *out = PrefetchPlan{(const unsigned char*)base, (int)gx, (int)gy, (int)nw, (int)kib, tile_bytes, split_bytes, (int)wgs, mxfp4 != 0, sink};
   return 0;
 }
 
@@ -3017,7 +3018,7 @@ __device__ __forceinline__ void dl_gemm(const void* __restrict__ Wp, const DlGem
   bool has = unit < n_units;
   int fg = has ? unit % groups : 0, sp = has ? unit / groups : 0;
   long long tile = (long long)fg * g.nw + wave;
-  const bool grouped = frag_grouped(g.N, ksteps);
+  const bool grouped = frag_grouped(g.N, ksteps, false);
   const dl_raw16* wp = reinterpret_cast<const dl_raw16*>(Wp) + frag_first((int)tile, ksteps, grouped) * 64 + lane;
   int c0 = sp * g.cps, c1 = c0 + g.cps < nchunks ? c0 + g.cps : nchunks;
   if (has) {
@@ -3253,7 +3254,7 @@ int kv_rope_kv_write_slabs(const float* slabs, int n_slabs, long long slab_strid
 // x: bf16 [T, H] (n_slabs == 0) or fp32 slabs [n_slabs][T][H]; residual: bf16 [T, H] in/out
 // (has_residual == 0: treated as zero and only written); ss_part: float [T][ceil(H/512)].
 // pf_base / pf (optional): the packed weights of the GEMM that runs next and its plan
-// {gx, gy, nw, kib, tile_bytes, split_bytes, prefetch workgroups, weight bytes}; see PrefetchPlan.
+// {gx, gy, nw, kib, tile_bytes, split_bytes, prefetch workgroups, weight bytes, whether they are MXFP4}; see PrefetchPlan.
 int kv_residual_reduce(const float* slabs, int n_slabs, long long slab_stride, const void* x, void* residual, int has_residual, float* ss_part, int T, int H,
                        const void* pf_base, const long long* pf, unsigned int* pf_sink, hipStream_t stream) {
   if (T <= 0) return 0;

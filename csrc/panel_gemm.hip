@@ -359,7 +359,7 @@ __device__ __attribute__((always_inline)) inline void dense_panel(const DenseArg
   const int tile_bytes = nks * (Q == MXFP4 ? 512 : 1024);
   const rsrc_t wr = buffer_of(p.w + (long long)panel * (FEATURES / 16) * tile_bytes, (unsigned int)have * tile_bytes);
   static_assert(FEATURES == 16 * FRAG_GROUP, "a panel is a group of tiles, where there are groups: the buffer ends with its last tile's bytes either way");
-  const bool grouped = frag_grouped(p.N, tile_bytes / 1024);
+  const bool grouped = frag_grouped(p.N, tile_bytes / 1024, Q == MXFP4);
   const int next = frag_next(tile_bytes / 1024, grouped) * 1024, w0 = 2 * wave * next + lane * 16, w1 = w0 + next;
   const rsrc_t sr = Q == MXFP4 ? buffer_of(p.scales.blocks + (long long)panel * (FEATURES / 16) * nks * 8, (unsigned int)have * nks * 32) : wr;
   const int s0 = 2 * wave * nks * 32 + (lane & 15) * 4, s1 = s0 + nks * 32;
@@ -523,7 +523,7 @@ __global__ __launch_bounds__(512) void narrow_tiles_kernel(const NarrowArgs p) {
   if (scaled && threadIdx.x < rows) row_scale[threadIdx.x] = MODE == SUMS ? p.scales.x[m0 + (int)threadIdx.x] : scale_of_row<Q>(p, m0 + (int)threadIdx.x);
   const int tile_bytes = nks * (Q == MXFP4 ? 512 : 1024);
   // (a group of tiles is two panels)
-  const bool grouped = frag_grouped(p.N, tile_bytes / 1024);
+  const bool grouped = frag_grouped(p.N, tile_bytes / 1024, Q == MXFP4);
   const int from = grouped ? panel / (FRAG_GROUP * 16 / NARROW_FEATURES) * FRAG_GROUP : panel * (NARROW_FEATURES / 16), have = grouped ? FRAG_GROUP : NARROW_FEATURES / 16;
   const rsrc_t wr = buffer_of(p.w + (long long)from * tile_bytes, (unsigned int)have * tile_bytes);
   const rsrc_t sr = Q == MXFP4 ? buffer_of(p.scales.blocks + (long long)panel * (NARROW_FEATURES / 16) * nks * 8, (unsigned int)(NARROW_FEATURES / 16) * nks * 32) : wr;

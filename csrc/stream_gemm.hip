@@ -102,13 +102,13 @@ __device__ inline frag_ab a_frag4(const raw16 raw, unsigned int sc, int u) {
 // One thread per (16-feature tile, 128-column group, lane): its 16 bytes are four k-steps of 8
 // values; each becomes the lane's 16-byte bf16 fragment of that k-step (1 KiB per wave and store).
 __global__ __launch_bounds__(256) void unpack_mxfp4_kernel(const raw16* __restrict__ wp4, const unsigned int* __restrict__ scales, raw16* __restrict__ wp,
-                                                           long long total, int groups, int grouped4, int grouped) {
+                                                           long long total, int groups, int grouped) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
   const int lane = (int)(i & 63);
   const long long tg = i >> 6;  // tile * groups + group
   const int tile = (int)(tg / groups), g = (int)(tg % groups);
-  const raw16 raw = wp4[(frag_first(tile, groups, grouped4) + frag_behind(g, grouped4)) * 64 + lane];
+  const raw16 raw = wp4[i];
   const unsigned int sc = scales[tg * 16 + (lane & 15)];
   raw16* dst = wp + frag_first(tile, 4 * groups, grouped) * 64 + lane;
 #pragma unroll
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void stream_gemm_kernel(const void* __restrict
   const int c1 = c0 + chunks_per_split < nchunks ? c0 + chunks_per_split : nchunks;
   const long long tile = (long long)blockIdx.x * 4 + wave;  // 16-row tile of W owned by this wave
   const int units = W8 ? ksteps / 2 : ksteps;  // of a tile: a k-step, or two
-  const bool grouped = frag_grouped(N, units);
+  const bool grouped = frag_grouped(N, units, false);
   const raw16* wp = reinterpret_cast<const raw16*>(Wp) + frag_first((int)tile, units, grouped) * 64 + lane;
 
   // x fragment slot s = tid + 256*i  ->  tile f = s/64 (= wave + 4*i), ks = f / MT, j = f % MT
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm3_kernel(const void* __res
   const bool tile_ok = tile_raw + FT <= ntiles;
   const long long tile = tile_ok ? tile_raw : ntiles - FT;  // the wave's first tile
   const int units = ksteps * AL / KS;                                 // of a tile, 1 KiB each
-  const bool grouped = frag_grouped(N, units);
+  const bool grouped = frag_grouped(N, units, W4);
   const long long tile_step = (long long)frag_next(units, grouped) * 64, block_step = (long long)frag_stride(grouped) * 64;
   const raw16* wp = reinterpret_cast<const raw16*>(Wp) + frag_first(__builtin_amdgcn_readfirstlane((int)tile), units, grouped) * 64 + lane;
   const long long sc_units = (long long)(ksteps / 4) * 16;            // scale words of one tile (W4)
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_rowsum_kernel(const void*
   const int ksteps = K >> 5;
   const long long tile = blockIdx.x;
   const int units = ksteps * AL / KS;
-  const bool grouped = frag_grouped(N, units);
+  const bool grouped = frag_grouped(N, units, false);
   const raw16* wp = reinterpret_cast<const raw16*>(Wp) + (frag_first((int)tile, units, grouped) + frag_behind(wave * cpw * AL, grouped)) * 64 + lane;
   const __bf16* xp = x + (long long)r * ldx + (long long)wave * cpw * (KS * 32) + q * 8;
 
@@ -785,7 +785,7 @@ __global__ __launch_bounds__(256) void pack_weight_fp8_kernel(const unsigned cha
   const unsigned char* row = W + (nt * 16 + r) * (long long)K + (long long)p * 64 + q * 8;
   const unsigned long long lo = *reinterpret_cast<const unsigned long long*>(row);
   const unsigned long long hi = *reinterpret_cast<const unsigned long long*>(row + 32);
-  const bool grouped = frag_grouped(N, kpairs);
+  const bool grouped = frag_grouped(N, kpairs, false);
   unsigned long long* dst = reinterpret_cast<unsigned long long*>(Wp + ((frag_first((int)nt, kpairs, grouped) + frag_behind(p, grouped)) * 64 + lane) * 16);
   dst[0] = lo;
   dst[1] = hi;
@@ -805,7 +805,7 @@ __global__ __launch_bounds__(256) void pack_weight_kernel(const unsigned short* 
   const long long nt = tile / ksteps;
   const int r = lane & 15, q = lane >> 4;
   const pk_us4* src = reinterpret_cast<const pk_us4*>(W + (nt * 16 + r) * K + (long long)ks * 32 + q * 8);
-  const bool grouped = !whole_tiles && frag_grouped(N, ksteps);
+  const bool grouped = !whole_tiles && frag_grouped(N, ksteps, false);
   pk_us4* dst = reinterpret_cast<pk_us4*>(Wp + (grouped ? (frag_first((int)nt, ksteps, true) + frag_behind(ks, true)) * 64 + lane : idx) * 8);
   dst[0] = src[0];
   dst[1] = src[1];
@@ -949,8 +949,8 @@ int kv_stream_gemm_rowsum(const void* Wp, const void* x, int M, int N, int K, lo
   return -1;
 }
 
-// MXFP4 packed weights (units [64 lanes][16 B] of a tile's 128 columns in the order of fragments.h + E8M0 scale words
-// [N/16][K/128][16 rows]) -> the bf16 fragments of kv_pack_weight, in that order too,
+// MXFP4 packed weights (pack_mxfp4 order: [N/16][K/128][64 lanes][16 B] + E8M0 scale words
+// [N/16][K/128][16 rows]) -> the bf16 fragments of kv_pack_weight, in their order,
 // exact (e2m1 times a power of two fits in bf16).  Wide steps expand a matrix into a scratch
 // buffer with this and run the bf16 tiled GEMM on it: 0.5 bytes read and 2 written per weight,
 // once per use, instead of one 128-row pass of the streaming kernel per 128 token rows.
@@ -958,7 +958,7 @@ int kv_unpack_mxfp4(const void* Wp4, const void* scales, void* Wp, int N, int K,
   if (N <= 0 || K <= 0 || (N & 15) || (K & 127)) return -1;
   const long long total = (long long)(N >> 4) * (K >> 7) * 64;
   hipLaunchKernelGGL(unpack_mxfp4_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, (const raw16*)Wp4, (const unsigned int*)scales, (raw16*)Wp, total, K >> 7,
-                     frag_grouped(N, K >> 7) ? 1 : 0, frag_grouped(N, K >> 5) ? 1 : 0);
+                     frag_grouped(N, K >> 5, false) ? 1 : 0);
   return (int)hipGetLastError();
 }
 

@@ -257,7 +257,7 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_kernel(const Params p)
   // ---- per-lane LDS-DMA source pointers: of the weights' first stage (the others: stage_bytes), and of stage s0 of x (a stage further = + XROW bytes)
   constexpr int UNITS = A_TILE / 1024;  // of a tile per stage
   const int units = nst * UNITS;        // of a tile
-  const bool grouped = frag_grouped(p.N, units);
+  const bool grouped = frag_grouped(p.N, units, W4);
   const long long block = frag_stride(grouped) * 1024;
   auto stage_bytes = [&](int st) __attribute__((always_inline)) { return UNITS == FRAG_BLOCK ? st * block : (st / FRAG_BLOCK) * block + st % FRAG_BLOCK * 1024; };
   const unsigned char* asrc[PA_W];
@@ -462,7 +462,7 @@ __global__ __launch_bounds__(WM * WN * 64) void wide_gemm_rs_kernel(const Params
 
   // ---- this wave's LDS-DMA pieces: source pointer at its first stage (of x: s0), byte offset inside a ring stage
   constexpr int UNITS = A_TILE / 1024;  // of a tile per stage
-  const bool grouped = frag_grouped(p.N, nst * UNITS);
+  const bool grouped = frag_grouped(p.N, nst * UNITS, WQ == 3);
   const long long block = frag_stride(grouped) * 1024;
   const unsigned char* src[GMAX];
   int doff[GMAX];
@@ -753,8 +753,8 @@ int kv_wide_gemm_fp8a(const void* Wp, const void* x8, void* out, int M, int N, i
   return dispatch_tile<2>(bm, bn, variant, epi, p, stream);
 }
 
-// MXFP4 weights x FP8 activations on the block-scaled MFMA: the weights in the streaming
-// kernels' units [64 lanes][16 B] of 128 columns, in the order of fragments.h, with their E8M0 block scales w_blk (int32 [N/16][K/128][16]) applied by
+// MXFP4 weights x FP8 activations on the block-scaled MFMA: the weights as the streaming kernels
+// read them, [N/16][K/128][64 lanes][16 B], with their E8M0 block scales w_blk (int32 [N/16][K/128][16]) applied by
 // the instruction itself; x8: e4m3 [M][ldx8] in NATURAL k order (kv_quantize_rows_fp8 with permute = 0), a_scale[M].
 // Tiles (256,128), (128,256), (128,128), variants 0 and 2.  K % 128 == 0, N % 64 == 0.
 int kv_wide_gemm_w4a8(const void* Wp4, const int* w_blk, const void* x8, void* out, int M, int N, int K, long long ldx8, long long ldy, int epi, int bm, int bn, int variant,

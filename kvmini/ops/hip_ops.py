@@ -105,8 +105,7 @@ class PackedLinear:
 
 def pack_mxfp4(codes: torch.Tensor, scales: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """MXFP4 codes ``[N, K]`` (0..15) and scale bytes ``[N, K/32]`` in the streaming GEMM's
-    fragment order.  Weights: uint8 ``[N/16, K/128, 64 lanes, 16]`` (where 256 divides N and K, a
-    group of 16 tiles has its 128-column groups in pairs, tile by tile: ``csrc/fragments.h``) — lane ``l`` holds, for each
+    fragment order.  Weights: uint8 ``[N/16, K/128, 64 lanes, 16]`` — lane ``l`` holds, for each
     of the four k-steps ``u`` of a 128-column group, ``W[row l & 15][32 u + 8 (l >> 4) .. + 8)`` as
     4 bytes (low nibble = the even element).  Scales: int32 ``[N/16, K/128, 16 rows]``, byte ``u``
     of a word = the E8M0 scale of k-step ``u``."""
@@ -114,8 +113,6 @@ def pack_mxfp4(codes: torch.Tensor, scales: torch.Tensor) -> Tuple[torch.Tensor,
     c = codes.view(n // 16, 16, k // 128, 4, 4, 4, 2)  # tile, row, group, u, q, byte, half
     c = c.permute(0, 2, 4, 1, 3, 5, 6)                # tile, group, q, row, u, byte, half
     packed = (c[..., 0] | (c[..., 1] << 4)).contiguous().view(n // 16, k // 128, 64, 16)
-    if n % 256 == 0 and k % 256 == 0:
-        packed = packed.view(n // 256, 16, k // 256, 2048).transpose(1, 2).contiguous().view(packed.shape)
     sc = scales.view(n // 16, 16, k // 128, 4).permute(0, 2, 1, 3).contiguous().to(torch.int32)  # tile, group, row, u
     words = sc[..., 0] | (sc[..., 1] << 8) | (sc[..., 2] << 16) | (sc[..., 3] << 24)
     return packed, words.contiguous()
