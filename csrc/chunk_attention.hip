@@ -228,8 +228,11 @@ int launch_prefill(const void* q, const void* kc, const void* vc, const void* ga
 // workgroups.  A wave multiplies a K block, straight from memory as the A operand, with the up to 16 query heads as columns
 // (S^T: a lane owns one head and 4 keys), and the weights, already in the A layout of mfma_f32_16x16x16_bf16, with the V block, which
 // passes through a piece of LDS of the wave's own for the transposed reads.  K / V of the next block (separate keys and values: of two) are in flight meanwhile,
-// the first ones since before the queries were normed.  6 rows of 820 tokens, heads of 64: 11.4 -> 9.8 us; 3 rows of 2000, four layers of a hybrid 325 -> 313; with CUs full
-// of workgroups no difference (61 rows of 8 heads of 128 x 865 tokens 63 us, 3.4 TB/s).
+// the first ones since before the queries were normed.  6 rows of 820 tokens, heads of 64: 11.4 -> 9.8 us; 3 rows of 2000, four layers of a hybrid 325 -> 313.
+// What a wave asks for in vain costs as much as what it needs: 1 KiB an instruction through the CU's 64 bytes a cycle.  So waves without blocks ask for none, and behind a wave's
+// last block the loads are of buffers without bytes.  us a launch, 8 key heads, 4 queries each; nothing ahead, everything ahead whether there or not, and now: 16 rows of 1 token of
+// 128, eight waves 5.9, 7.1 and 5.85, of 200 tokens 8.2, 8.6 and 7.9, of 800 16.9, 15.7 and 14.2; 64 rows of 1 token, four waves 7.3, 8.4 and 7.35, of 200 16.9, 15.6 and 14.7.
+// Of heads of 64, 0.2 to 0.4 are left at up to 60 tokens (16 rows 5.1 and 5.3, 64 rows 6.1 and 6.5), from 200 on it is ahead (64 rows 8.6 and 8.25).
 // FUSED: the kernel also does what norm_rope_write_kernel does for the row (query / key norm, rotation, K / V write).
 // RT >= 0 (one row is key and value): the keys' operands come out of the piece of LDS, too.
 // SPLIT: partial results (maximum, sum, unnormalised output per head) go to a workspace for chunk_decode_combine_kernel.
@@ -287,8 +290,11 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
   const int head_lr = g * rep + h0 + (lr < nhd ? lr : nhd - 1);  // the lane's head
   const float* rel = REL ? a.see.rel + (long long)head_lr * a.see.rel_n : nullptr;
   const int v_row = lane / VCH, v_c = lane % VCH;  // piece `it` of a V block: row v_row + it * (64 / VCH)
+  auto mine = [&](int b) { return b < nb ? b : nb - 1; };  // a block whose page is looked up
+  // A block's operands.  Behind the last block the loads are there all the same, of buffers without bytes: as many are waited for, and nothing is moved
   auto fetch = [&](int b, int set, int page_index) __attribute__((always_inline)) {
-    const int key = block_key(b);
+    const bool there = b < nb;
+    const int key = block_key(mine(b));
     if constexpr (REL) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -299,18 +305,16 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
     }
     const long long page = ((long long)page_index * a.nkv + g) * (bs_mask + 1) + (key & bs_mask);
     if constexpr (!ONE || RW > 0) {
-      const bf16raw* kp = k_cache + (page + lr) * KST + (ONE ? DK : 0) + lq * 8;
+      const __amdgpu_buffer_rsrc_t kb = __builtin_amdgcn_make_buffer_rsrc(k_cache + page * KST, (short)0, there ? 16 * KST * 2 : 0, 0x00027000);
 #pragma unroll
-      for (int ks = 0; ks < KF; ++ks) kn[set][ks] = *reinterpret_cast<const raw16*>(kp + ks * 32);
+      for (int ks = 0; ks < KF; ++ks) kn[set][ks] = __builtin_bit_cast(raw16, __builtin_amdgcn_raw_buffer_load_b128(kb, (lr * KST + (ONE ? DK : 0) + lq * 8) * 2, ks * 64, 0));
     }
     if constexpr (ONE) sn[set] = ld4(a.key_scale + page + 4 * lq);
-    const bf16raw* vp = ONE ? k_cache : v_cache;
+    const __amdgpu_buffer_rsrc_t vb = __builtin_amdgcn_make_buffer_rsrc((ONE ? k_cache : v_cache) + page * VST, (short)0, there ? 16 * VST * 2 : 0, 0x00027000);
 #pragma unroll
-    for (int it = 0; it < VIT; ++it) vn[set][it] = *reinterpret_cast<const raw16*>(vp + (page + v_row + it * (64 / VCH)) * VST + v_c * 8);
+    for (int it = 0; it < VIT; ++it) vn[set][it] = __builtin_bit_cast(raw16, __builtin_amdgcn_raw_buffer_load_b128(vb, (v_row * VST + v_c * 8) * 2, it * (64 / VCH) * VST * 2, 0));
   };
   int first_page[SETS];
-  auto mine = [&](int b) { return b < nb ? b : nb - 1; };  // behind the last block: that one again, whose bytes the caches have
-
 #pragma unroll
   for (int e = 0; e < SETS; ++e) first_page[e] = page_of(mine(me + e * stride));
 
@@ -398,19 +402,32 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
     };
-    const Unit first_unit = load(wave), second_unit = load(wave + NW);
-    __builtin_amdgcn_sched_barrier(0);
+    // (of eight waves few have a second unit, and asking for one that is not there takes 0.2 us)
+    constexpr int AHEAD = NW == 4 ? 2 : 1;
+    Unit units[AHEAD];
 #pragma unroll
-    for (int e = 0; e < SETS; ++e) fetch(mine(me + e * stride), e, first_page[e]);
+    for (int i = 0; i < AHEAD; ++i) units[i] = load(wave + i * NW);
     __builtin_amdgcn_sched_barrier(0);
-    if (wave < n_units) make(wave, first_unit);
-    if (wave + NW < n_units) make(wave + NW, second_unit);
-    for (int u = wave + 2 * NW; u < n_units; u += NW) make(u, load(u));
+    auto make_first = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i)
+        if (wave + i * NW < n_units) make(wave + i * NW, units[i]);
+    };
+    // A wave without blocks has a way of its own (on a common one the units would wait for the blocks as well, which only some waves asked for)
+    if (me < nb) {
+#pragma unroll
+      for (int e = 0; e < SETS; ++e) fetch(me + e * stride, e, first_page[e]);
+      __builtin_amdgcn_sched_barrier(0);
+      make_first();
+    } else {
+      make_first();
+    }
+    for (int u = wave + AHEAD * NW; u < n_units; u += NW) make(u, load(u));
     for (int i = tid; i < (16 - nhd) * KST; i += 64 * NW) q_s[(nhd + i / KST) * QS + i % KST] = 0;
     __threadfence_block();
   } else {
 #pragma unroll
-    for (int e = 0; e < SETS; ++e) fetch(mine(me + e * stride), e, first_page[e]);
+    for (int e = 0; e < SETS; ++e) fetch(me + e * stride, e, first_page[e]);
     for (int i = tid; i < 16 * (KST / 8); i += 64 * NW) {
       const int h = i / (KST / 8), c = i % (KST / 8);
       raw16 v = {0, 0, 0, 0};
@@ -461,7 +478,7 @@ __global__ __launch_bounds__(64 * NW) void chunk_decode_kernel(const bf16raw* __
     // The next block's loads, always as many: what is waited for is counted exactly.  One block at a time: as early as there is room; two: where this one's were, when all
     // of them are used (else they would move from one set of registers to the other, and be waited for there)
     auto next = [&]() __attribute__((always_inline)) {
-      fetch(mine(b + SETS * stride), set, page[set]);
+      fetch(b + SETS * stride, set, page[set]);
       page[set] = page_of(mine(b + 2 * SETS * stride));
     };
     if constexpr (SETS == 1) next();

@@ -995,6 +995,37 @@ def test_distance_biases_are_rounded_before_a_score_meets_them(C, dim, waves, sh
     assert (got - want).abs().max() <= tol
 
 
+@pytest.mark.parametrize("rep,shares", [(4, 1), (8, 1), (12, 1), (4, 3)])
+@pytest.mark.parametrize("dim,waves", [(64, 4), (64, 8), (128, 4), (128, 8)])
+def test_decode_attention_where_waves_have_no_blocks_and_some(C, dim, waves, rep, shares):
+    """Contexts about the 16 keys of a block and the blocks of a workgroup's waves; every key behind a row's last block is NaN.  Queries and keys rounded as the kernel does:
+    what is left are the weights' rounding and the output's, 2^-9 of the largest value each, and as much for the sums."""
+    nkv, scale, lens = 2, 0.05, [1, 15, 16, 17, 64, 65, 128, 129, 200, 256, 257, 400]
+    nh, per, n = nkv * rep, -(-max(lens) // 16) + 2, len(lens)
+    gen = torch.Generator().manual_seed(dim + waves)
+    proj = torch.randn(n, (nh + 2 * nkv) * dim, generator=gen).bfloat16()
+    kv = torch.randn(2, n, per * 16, nkv, dim, generator=gen).bfloat16()
+    normed = lambda x: (x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-5)).bfloat16().double()  # noqa: E731
+    q, k1, v1 = proj.float().split([nh * dim, nkv * dim, nkv * dim], 1)
+    want = torch.empty(n, nh, dim, dtype=torch.float64)
+    cache = torch.full((2, n, per * 16, nkv, dim), float("nan"), dtype=torch.bfloat16)
+    for i, m in enumerate(lens):
+        end = -(-m // 16) * 16
+        cache[:, i, :end] = kv[:, i, :end]
+        keys, values = kv[0, i, :m].double(), kv[1, i, :m].double()
+        keys[-1], values[-1] = normed(k1[i].view(nkv, dim)), v1[i].view(nkv, dim).double()
+        at = normed(q[i].view(nkv, rep, dim))
+        w = torch.softmax(torch.einsum("grd,kgd->grk", at, keys) * scale, -1)
+        want[i] = torch.einsum("grk,kgd->grd", w, values).reshape(nh, dim)
+    kc, vc = (x.view(n * per, 16, nkv, dim).transpose(1, 2).contiguous().to(_dev()) for x in cache)
+    ids, pos = torch.arange(n, device=_dev(), dtype=torch.int32), torch.tensor(lens, device=_dev(), dtype=torch.int32) - 1
+    bt = torch.arange(n * per, device=_dev(), dtype=torch.int32).view(n, per)
+    ones, none, out = torch.ones(dim, device=_dev()), torch.zeros(0, device=_dev()), torch.empty(n, nh * dim, device=_dev(), dtype=torch.bfloat16)
+    C.chunk_decode(None, proj.to(_dev()), 0, nh * dim, (nh + nkv) * dim, torch.zeros((nh + 2 * nkv) * dim, device=_dev()), ones, ones, none, none, 0, 1e-5, kc, vc, bt, ids, ids, pos,
+                   ids * per * 16 + pos, 0, 0, out, 0, nh, dim, dim, 0, 0, 0, None, None, scale, 1.0, waves, shares)
+    assert (out.view(n, nh, dim).double().cpu() - want).abs().max() <= 3 * 2.0**-9 * kv.float().abs().max()
+
+
 @pytest.mark.parametrize("rank,rot", [(128, 0), (256, 64), (512, 64)])
 def test_latent_rows_joined_of_any_number_of_shares(C, rank, rot):
     """Rows of few and many keys in 2 to 64 shares (16 of them are joined at a time) against one share: the latents and the outputs are rounded to bf16, 2^-9 of each
